@@ -6,15 +6,20 @@ There is no fallback: if the library has not been built, loading raises.
 libmarian_hip_int8_tuning.so is the same code built with -DMARIAN_HIP_TUNING
 (include/marian_hip_int8_tuning.h): it adds a process-wide kernel selection override, the kernel
 families only measurements select, and in-kernel clocks.  Tests and measurement scripts reach it
-through `forced_kernel(which)`; nothing else loads it."""
+through `forced_kernel(which)`; nothing else loads it.
+
+_host_calls.so (csrc/host_calls.cpp) is the operators' host path as native code: argument checks, output
+tensors and the call into whichever of the two libraries is in use.  `HostCalls` loads it."""
 import contextlib
 import ctypes
+import importlib.util
 import os
 import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmarian_hip_int8.so")
 TUNING_LIB_PATH = os.path.join(_HERE, "libmarian_hip_int8_tuning.so")
+HOST_PATH = os.path.join(_HERE, "_host_calls.so")
 
 OK, ERR_NULL, ERR_SHAPE, ERR_ALIGN, ERR_WORKSPACE, ERR_HIP, ERR_RANGE, ERR_STATIC_LIMIT, ERR_ALIAS = range(9)
 
@@ -86,6 +91,7 @@ STATIC_MAX_ELEMS = 16 * 1024 * 1024   # MARIAN_HIP_STATIC_MAX_ELEMS
 _lib = None
 _tuning = None
 _active = None   # the tuning build while a forced_kernel() block runs, else None
+_host = None     # the module _host_calls once it is loaded
 
 
 class MarianHipError(RuntimeError):
@@ -97,21 +103,25 @@ class MarianHipError(RuntimeError):
 
 
 def build(verbose=False):
-    """Compile the HIP libraries for gfx950 with hipcc (always recompiles)."""
+    """Compile the HIP libraries for gfx950 with hipcc and the host path with the C++ compiler (always recompiles)."""
     cmd = ["make", "-C", os.path.join(_HERE, "csrc"), "-B", "-j4"]
     out = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if verbose or out.returncode != 0:
         print(out.stdout)
     if out.returncode != 0:
-        raise RuntimeError("hipcc build of libmarian_hip_int8.so failed")
+        raise RuntimeError("build of libmarian_hip_int8.so and _host_calls.so failed")
     return LIB_PATH
 
 
-def _load(path, signatures):
+def _must_exist(path):
     if not os.path.exists(path):
         raise MarianHipError(
             -1, "{} is not built ({}); run __graft_entry__.build() or "
             "`make -C marian-dev_amd/csrc`. There is no CPU fallback.".format(os.path.basename(path), path))
+
+
+def _load(path, signatures):
+    _must_exist(path)
     # torch must load first: it ships its own libamdhip64.so.7 / HSA runtime, and a process
     # can hold only one of them - loading ours first would pull in the system copy and
     # leave torch's runtime without a device (hipErrorNoDevice on the first launch)
@@ -141,20 +151,51 @@ def tuning_lib():
     return _tuning
 
 
+class HostCalls:
+    """The functions of _host_calls.so as attributes, loaded when one is first asked for.  types: called
+    then, returns what its setup() takes."""
+
+    def __init__(self, types):
+        self._types = types
+
+    def __getattr__(self, name):
+        global _host
+        if name.startswith("__"):
+            raise AttributeError(name)
+        if _host is None:
+            _must_exist(HOST_PATH)
+            import torch  # noqa: F401  (its libraries have to be in the process first)
+            spec = importlib.util.spec_from_file_location("_host_calls", HOST_PATH)
+            made = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(made)
+            made.use(lib()._handle)
+            made.setup(*self._types())
+            _host = made
+        fn = getattr(_host, name)
+        setattr(self, name, fn)   # (found without __getattr__ from now on)
+        return fn
+
+
+def _switch(active):
+    global _active
+    _active = active
+    if _host is not None:
+        _host.use(lib()._handle)
+
+
 @contextlib.contextmanager
 def forced_kernel(which):
     """Runs the block on the tuning build with kernel family `which` pinned (0: the tuning build's
     automatic selection); lib() returns the tuning build inside the block."""
-    global _active
     T = tuning_lib()
     outer = _active
-    _active = T
+    _switch(T)
     prev = T.marian_hip_int8_set_kernel(int(which))
     try:
         yield T
     finally:
         T.marian_hip_int8_set_kernel(prev)
-        _active = outer
+        _switch(outer)
 
 
 def check(status, where):

@@ -1,0 +1,775 @@
+// The host path of the operators as native code (Python module _host_calls): argument checks, output
+// tensors and the call into the C ABI for one operator, without Python code in between.
+//
+// What bounds the small calls is the host: a decoding step is some sixty launches whose kernels run
+// 3 - 12 us each, and the same checks and allocations written in Python took 15 - 20 us per call
+// (transformer-big step, beam 4 x batch 32: 990 us of host work for 445 us of kernels).  Here a call
+// costs its output tensors (about half a microsecond each) and the launch itself.
+//
+// Every function takes the arguments of the operator in its normal form - float32 tensors on the GPU,
+// contiguous, quantized weights in prepared order - and returns None when it is handed anything
+// else; the Python mirror (integer.py, ops.py) then checks what is wrong, raises the operator's error
+// or brings the arguments into normal form and calls again.  Nothing is computed here: the kernels
+// are reached through the C ABI of the library that use() was given (the shipped build, or the tuning
+// build inside _lib.forced_kernel()).
+//
+// The interpreter lock is released around every ABI call, as ctypes does.
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+
+#include <cmath>
+#include <map>
+#include <utility>
+#include <vector>
+
+#include "../../include/marian_hip_int16.h"
+#include "../../include/marian_hip_int8.h"
+#include "../../include/marian_hip_ops.h"
+
+namespace {
+
+// ---- the library in use -------------------------------------------------------------------------
+#define MH_FUNCTIONS(F)                                                                                  \
+  F(int8_workspace_bytes) F(int8_prepare_a) F(int8_prepare_b) F(int8_prepare_b_quantized_transposed)     \
+  F(int8_affine_f32) F(int8_affine_f32_chained) F(int8_affine_f32_grouped) F(int8_proj_attention)        \
+  F(int16_prepare_a) F(int16_prepare_b) F(int16_prepare_b_quantized_transposed) F(int16_affine)          \
+  F(layer_norm) F(embed) F(attention_cached) F(attention_ancestors) F(ancestors_advance)                 \
+  F(select_state) F(nbest) F(nbest_beams) F(nbest_beams_workspace_bytes) F(nbest_beams_workspace_init)   \
+  F(logsoftmax_nbest_beams)
+
+struct Library {
+#define F(name) decltype(&marian_hip_##name) name;
+  MH_FUNCTIONS(F)
+#undef F
+};
+Library L{};
+
+// ---- what Python registered ---------------------------------------------------------------------
+PyTypeObject* QTensorType = nullptr;
+PyTypeObject* AbsMaxType = nullptr;
+PyObject *type8 = nullptr, *type16 = nullptr, *raise_status = nullptr, *no_args = nullptr;
+PyObject *s_data, *s_shape, *s_type, *s_prepared;
+
+// A new reference that is dropped at the end of the scope.
+struct Ref {
+  PyObject* p;
+  explicit Ref(PyObject* o = nullptr) : p(o) {}
+  ~Ref() { Py_XDECREF(p); }
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+  Ref(Ref&& o) noexcept : p(o.p) { o.p = nullptr; }
+  PyObject* release() { PyObject* o = p; p = nullptr; return o; }
+  explicit operator bool() const { return p != nullptr; }
+};
+
+struct PyFailed {};   // a Python error is set
+
+PyObject* ok(PyObject* o) {
+  if(!o) throw PyFailed();
+  return o;
+}
+
+inline bool none(PyObject* o) { return o == Py_None; }
+
+// The tensor behind a Python object, or null.
+inline const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// The tensor behind o if it is in normal form: float32, on the GPU, contiguous.
+inline const at::Tensor* f32c(PyObject* o) {
+  const at::Tensor* t = tensor(o);
+  return t && t->scalar_type() == at::kFloat && t->is_cuda() && t->is_contiguous() ? t : nullptr;
+}
+// None, or a tensor in normal form; false when it is neither.
+inline bool f32c_or_none(PyObject* o, const at::Tensor** t) {
+  *t = nullptr;
+  return none(o) || (*t = f32c(o)) != nullptr;
+}
+inline bool ids_type(at::ScalarType s) { return s == at::kInt || s == at::kUInt32; }
+
+inline const float* fptr(const at::Tensor* t) { return t ? static_cast<const float*>(t->const_data_ptr()) : nullptr; }
+inline float* fptr_mut(const at::Tensor& t) { return static_cast<float*>(t.data_ptr()); }
+
+inline at::Tensor empty(at::IntArrayRef size, at::ScalarType type, c10::Device device) {
+  return at::Tensor(at::detail::empty_cuda(size, type, device, std::nullopt));
+}
+inline PyObject* wrap(at::Tensor t) { return ok(THPVariable_Wrap(std::move(t))); }
+
+inline hipStream_t stream_of(c10::Device d) { return c10::hip::getCurrentHIPStream(d.index()).stream(); }
+
+inline double number(PyObject* o) {
+  const double v = PyFloat_AsDouble(o);
+  if(v == -1.0 && PyErr_Occurred()) throw PyFailed();
+  return v;
+}
+inline int64_t whole(PyObject* o) {
+  const long long v = PyLong_AsLongLong(o);
+  if(v == -1 && PyErr_Occurred()) throw PyFailed();
+  return v;
+}
+inline bool truth(PyObject* o) {
+  const int v = PyObject_IsTrue(o);
+  if(v < 0) throw PyFailed();
+  return v != 0;
+}
+
+template <typename F>
+inline void call(const char* where, F f) {
+  PyThreadState* s = PyEval_SaveThread();
+  const int status = f();
+  PyEval_RestoreThread(s);
+  if(status != MARIAN_HIP_OK) {
+    Ref r(PyObject_CallFunction(raise_status, "is", status, where));
+    if(!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, where);
+    throw PyFailed();
+  }
+}
+
+// ---- workspaces: one per device and stream, kept for good (a graph may have recorded one) -------
+struct PerStream {
+  at::Tensor workspace;              // abs-max partials, one-pass exchange
+  std::vector<at::Tensor> nbest;     // the last one the largest
+};
+std::map<std::pair<int, hipStream_t>, PerStream> per_stream;   // (looked up with the interpreter lock held)
+
+at::Tensor& workspace(c10::Device d, hipStream_t st) {
+  PerStream& p = per_stream[{d.index(), st}];
+  if(!p.workspace.defined()) {
+    at::Tensor made = empty({(int64_t)L.int8_workspace_bytes()}, at::kByte, d);
+    if(!p.workspace.defined()) p.workspace = std::move(made);
+  }
+  return p.workspace;
+}
+
+at::Tensor nbest_workspace(int64_t beam, int64_t batch, int64_t vocab, int64_t N, c10::Device d, hipStream_t st) {
+  const int64_t need = (int64_t)L.nbest_beams_workspace_bytes(beam, batch, vocab, N);
+  {
+    std::vector<at::Tensor>& held = per_stream[{d.index(), st}].nbest;
+    if(!held.empty() && held.back().numel() >= need) return held.back();
+  }
+  at::Tensor made = empty({need > 4 ? need : 4}, at::kByte, d);
+  call("getNBestListOfBeams", [&] { return L.nbest_beams_workspace_init(made.data_ptr(), (size_t)made.numel(), st); });
+  per_stream[{d.index(), st}].nbest.push_back(made);
+  return made;
+}
+
+// ---- quantized tensors --------------------------------------------------------------------------
+struct Quantized {
+  Ref data, shape;
+  const at::Tensor* t = nullptr;
+  int64_t rows = 0, cols = 0;
+  int width = 0;
+};
+
+// A matrix in q: Type::intgemm8 or Type::intgemm16, two dimensions.  prepared: 8-bit weights have to be in
+// prepared order (true) or in file order (false).
+bool matrix(PyObject* q, Quantized& m, bool prepared) {
+  if(Py_TYPE(q) != QTensorType) return false;
+  Ref type(ok(PyObject_GetAttr(q, s_type)));
+  m.width = type.p == type8 ? 1 : (type.p == type16 ? 2 : 0);
+  if(m.width == 0) return false;
+  if(m.width == 1 || !prepared) {
+    Ref p(ok(PyObject_GetAttr(q, s_prepared)));
+    if(truth(p.p) != prepared) return false;
+  }
+  Ref shape(ok(PyObject_GetAttr(q, s_shape)));
+  if(!PyTuple_Check(shape.p) || PyTuple_GET_SIZE(shape.p) != 2) return false;
+  m.rows = whole(PyTuple_GET_ITEM(shape.p, 0));
+  m.cols = whole(PyTuple_GET_ITEM(shape.p, 1));
+  Ref data(ok(PyObject_GetAttr(q, s_data)));
+  m.t = tensor(data.p);
+  if(!m.t || !m.t->is_cuda() || m.t->numel() < m.rows * m.cols * m.width + 4) return false;
+  std::swap(m.data.p, data.p);
+  std::swap(m.shape.p, shape.p);
+  return true;
+}
+
+at::Tensor quantized_buffer(int64_t elements, int width, c10::Device d) {
+  return empty({(elements * width + 4 + 255) / 256 * 256}, at::kChar, d);
+}
+
+PyObject* make_quantized(at::Tensor data, PyObject* shape_tuple, PyObject* type, bool prepared) {
+  Ref q(ok(QTensorType->tp_new(QTensorType, no_args, nullptr)));
+  Ref d(wrap(std::move(data)));
+  if(PyObject_SetAttr(q.p, s_data, d.p) || PyObject_SetAttr(q.p, s_shape, shape_tuple) ||
+     PyObject_SetAttr(q.p, s_type, type) || PyObject_SetAttr(q.p, s_prepared, prepared ? Py_True : Py_False))
+    throw PyFailed();
+  return q.release();
+}
+
+PyObject* shape_tuple(at::IntArrayRef s) {
+  Ref t(ok(PyTuple_New((Py_ssize_t)s.size())));
+  for(size_t i = 0; i < s.size(); ++i) PyTuple_SET_ITEM(t.p, (Py_ssize_t)i, ok(PyLong_FromLongLong(s[i])));
+  return t.release();
+}
+
+// ---- abs-max hand-over --------------------------------------------------------------------------
+// None, or the slots of an AbsMax; false when it is neither.
+bool absmax_in(PyObject* o, const float** p) {
+  *p = nullptr;
+  if(none(o)) return true;
+  if(Py_TYPE(o) != AbsMaxType) return false;
+  Ref data(ok(PyObject_GetAttr(o, s_data)));
+  const at::Tensor* t = f32c(data.p);
+  if(!t || t->numel() < MARIAN_HIP_ABSMAX_SLOTS) return false;
+  *p = fptr(t);
+  return true;
+}
+inline at::Tensor absmax_slots(c10::Device d) { return empty({MARIAN_HIP_ABSMAX_SLOTS}, at::kFloat, d); }
+PyObject* make_absmax(at::Tensor slots) {
+  Ref o(ok(AbsMaxType->tp_new(AbsMaxType, no_args, nullptr)));
+  Ref d(wrap(std::move(slots)));
+  if(PyObject_SetAttr(o.p, s_data, d.p)) throw PyFailed();
+  return o.release();
+}
+
+inline at::DimVector with_last(at::IntArrayRef s, int64_t last) {
+  at::DimVector v(s.begin(), s.end());
+  v.back() = last;
+  return v;
+}
+
+#define MH_TRY \
+  HANDLE_TH_ERRORS try {
+#define MH_END                       \
+  }                                  \
+  catch(const PyFailed&) {           \
+    return nullptr;                  \
+  }                                  \
+  END_HANDLE_TH_ERRORS
+#define MH_ARGS(count, name)                                                        \
+  if(nargs != (count)) {                                                            \
+    PyErr_SetString(PyExc_TypeError, name " takes another number of arguments");    \
+    return nullptr;                                                                 \
+  }
+
+// ---- affine -------------------------------------------------------------------------------------
+// prepareA and the multiplication: out and the quantized activations in aq.
+struct Affine {
+  const at::Tensor *a = nullptr, *bias = nullptr, *idx = nullptr;
+  Quantized b;
+  int64_t M = 0, K = 0, n_out = 0;
+};
+
+bool affine_args(PyObject* a, PyObject* bq, PyObject* bias, PyObject* shortlist, Affine& x) {
+  x.a = f32c(a);
+  if(!x.a || x.a->dim() < 1 || !matrix(bq, x.b, true)) return false;
+  x.K = x.a->size(-1);
+  if(x.b.rows != x.K) return false;
+  x.M = x.K ? x.a->numel() / x.K : 0;
+  x.n_out = x.b.cols;
+  if(!f32c_or_none(bias, &x.bias) || (x.bias && x.bias->numel() != x.b.cols)) return false;
+  if(!none(shortlist)) {
+    x.idx = tensor(shortlist);
+    if(!x.idx || x.b.width != 1 || !ids_type(x.idx->scalar_type()) || !x.idx->is_cuda() || !x.idx->is_contiguous()) return false;
+    x.n_out = x.idx->numel();
+  }
+  return true;
+}
+
+// affine_or_dot(a, bQuant, bias, scale, relu, shortlist) -> out
+PyObject* py_affine_or_dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(6, "affine_or_dot");
+  Affine x;
+  if(!affine_args(args[0], args[1], args[2], args[5], x)) Py_RETURN_NONE;
+  const float scale = (float)number(args[3]);
+  const int relu = truth(args[4]);
+  const c10::Device d = x.a->device();
+  at::Tensor out = empty(with_last(x.a->sizes(), x.n_out), at::kFloat, d);
+  const at::Tensor aq = quantized_buffer(x.M * x.K, x.b.width, d);
+  const hipStream_t st = stream_of(d);
+  if(x.b.width == 2) {   // Type::intgemm16: the two nodes one after the other
+    auto* q = static_cast<int16_t*>(aq.data_ptr());
+    call("affineOrDot", [&] {
+      const int s = L.int16_prepare_a(fptr(x.a), q, x.M, x.K, st);
+      return s != MARIAN_HIP_OK ? s
+                                : L.int16_affine(q, static_cast<const int16_t*>(x.b.t->const_data_ptr()), fptr(x.bias), fptr_mut(out),
+                                                 x.M, x.K, x.b.cols, scale, relu, st);
+    });
+    return wrap(std::move(out));
+  }
+  const at::Tensor& ws = workspace(d, st);
+  call("affineOrDot", [&] {
+    return L.int8_affine_f32(fptr(x.a), static_cast<int8_t*>(aq.data_ptr()), static_cast<const int8_t*>(x.b.t->const_data_ptr()),
+                             fptr(x.bias), x.idx ? static_cast<const uint32_t*>(x.idx->const_data_ptr()) : nullptr,
+                             x.idx ? x.n_out : 0, fptr_mut(out), x.M, x.K, x.b.cols, scale, relu, ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  return wrap(std::move(out));
+  MH_END
+}
+
+// affine_f32(a, bQuant, bias, scale, relu, shortlist, absmax, want_absmax) -> (out, aQuant[, absmax of out])
+PyObject* py_affine_f32(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(8, "affine_f32");
+  Affine x;
+  const float* amax = nullptr;
+  if(!affine_args(args[0], args[1], args[2], args[5], x) || x.b.width != 1 || !absmax_in(args[6], &amax)) Py_RETURN_NONE;
+  const float scale = (float)number(args[3]);
+  const int relu = truth(args[4]);
+  const bool want = truth(args[7]);
+  const c10::Device d = x.a->device();
+  at::Tensor out = empty(with_last(x.a->sizes(), x.n_out), at::kFloat, d);
+  at::Tensor aq = quantized_buffer(x.M * x.K, 1, d);
+  at::Tensor omax;
+  if(want) omax = absmax_slots(d);
+  const hipStream_t st = stream_of(d);
+  const at::Tensor& ws = workspace(d, st);
+  call("affineOrDot", [&] {
+    return L.int8_affine_f32_chained(
+        fptr(x.a), static_cast<int8_t*>(aq.data_ptr()), static_cast<const int8_t*>(x.b.t->const_data_ptr()), fptr(x.bias),
+        x.idx ? static_cast<const uint32_t*>(x.idx->const_data_ptr()) : nullptr, x.idx ? x.n_out : 0, fptr_mut(out), x.M, x.K,
+        x.b.cols, scale, relu, amax, want ? fptr_mut(omax) : nullptr, ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  Ref r(ok(PyTuple_New(want ? 3 : 2)));
+  PyTuple_SET_ITEM(r.p, 0, wrap(std::move(out)));
+  Ref shape(shape_tuple(x.a->sizes()));
+  PyTuple_SET_ITEM(r.p, 1, make_quantized(std::move(aq), shape.p, type8, false));
+  if(want) PyTuple_SET_ITEM(r.p, 2, make_absmax(std::move(omax)));
+  return r.release();
+  MH_END
+}
+
+// A list or tuple of (bQuant, bias or None) with K rows each; false when it is anything else.
+constexpr int kMaxMatrices = 4;
+struct Matrices {
+  int n = 0;
+  Quantized b[kMaxMatrices];
+  const int8_t* Bq[kMaxMatrices];
+  const float* bias[kMaxMatrices];
+};
+bool matrices(PyObject* weights, int64_t K, bool bias_checked, Matrices& m) {
+  if(!PyList_Check(weights) && !PyTuple_Check(weights)) return false;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(weights);
+  if(n < 1 || n > kMaxMatrices) return false;
+  m.n = (int)n;
+  for(int g = 0; g < m.n; ++g) {
+    PyObject* w = PySequence_Fast_GET_ITEM(weights, g);
+    if((!PyTuple_Check(w) && !PyList_Check(w)) || PySequence_Fast_GET_SIZE(w) != 2) return false;
+    if(!matrix(PySequence_Fast_GET_ITEM(w, 0), m.b[g], true) || m.b[g].width != 1 || m.b[g].rows != K) return false;
+    const at::Tensor* bias;
+    if(!f32c_or_none(PySequence_Fast_GET_ITEM(w, 1), &bias) || (bias_checked && bias && bias->numel() != m.b[g].cols)) return false;
+    m.Bq[g] = static_cast<const int8_t*>(m.b[g].t->const_data_ptr());
+    m.bias[g] = fptr(bias);
+  }
+  return true;
+}
+
+// affine_f32_grouped(a, weights, scale, relu, absmax) -> ([out, ..], aQuant)
+PyObject* py_affine_f32_grouped(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(5, "affine_f32_grouped");
+  const at::Tensor* a = f32c(args[0]);
+  Matrices w;
+  const float* amax = nullptr;
+  if(!a || a->dim() < 1 || !matrices(args[1], a->size(-1), true, w) || !absmax_in(args[4], &amax)) Py_RETURN_NONE;
+  const float scale = (float)number(args[2]);
+  const int relu = truth(args[3]);
+  const int64_t K = a->size(-1), M = K ? a->numel() / K : 0;
+  const c10::Device d = a->device();
+  at::Tensor aq = quantized_buffer(M * K, 1, d), outs[kMaxMatrices];
+  float* out[kMaxMatrices];
+  int64_t N[kMaxMatrices];
+  for(int g = 0; g < w.n; ++g) {
+    outs[g] = empty(with_last(a->sizes(), w.b[g].cols), at::kFloat, d);
+    out[g] = fptr_mut(outs[g]);
+    N[g] = w.b[g].cols;
+  }
+  const hipStream_t st = stream_of(d);
+  const at::Tensor& ws = workspace(d, st);
+  call("affineOrDot", [&] {
+    return L.int8_affine_f32_grouped(fptr(a), static_cast<int8_t*>(aq.data_ptr()), w.n, w.Bq, w.bias, out, N, M, K, scale, relu, amax,
+                                     ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  Ref list(ok(PyList_New(w.n)));
+  for(int g = 0; g < w.n; ++g) PyList_SET_ITEM(list.p, g, wrap(std::move(outs[g])));
+  Ref shape(shape_tuple(a->sizes()));
+  Ref q(make_quantized(std::move(aq), shape.p, type8, false));
+  return PyTuple_Pack(2, list.p, q.p);
+  MH_END
+}
+
+// ---- quantizers ---------------------------------------------------------------------------------
+// prepare_a(a, width) -> QTensor
+PyObject* py_prepare_a(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(2, "prepare_a");
+  const at::Tensor* a = f32c(args[0]);
+  const int64_t width = whole(args[1]);
+  if(!a || a->dim() < 1 || (width != 1 && width != 2)) Py_RETURN_NONE;
+  const int64_t K = a->size(-1), M = K ? a->numel() / K : 0;
+  const c10::Device d = a->device();
+  at::Tensor out = quantized_buffer(a->numel(), (int)width, d);
+  const hipStream_t st = stream_of(d);
+  const at::Tensor& ws = workspace(d, st);
+  call("prepareA", [&] {
+    return width == 2 ? L.int16_prepare_a(fptr(a), static_cast<int16_t*>(out.data_ptr()), M, K, st)
+                      : L.int8_prepare_a(fptr(a), static_cast<int8_t*>(out.data_ptr()), M, K, ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  Ref shape(shape_tuple(a->sizes()));
+  return make_quantized(std::move(out), shape.p, width == 2 ? type16 : type8, false);
+  MH_END
+}
+
+// prepare_b(w, width) -> QTensor
+PyObject* py_prepare_b(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(2, "prepare_b");
+  const at::Tensor* w = f32c(args[0]);
+  const int64_t width = whole(args[1]);
+  if(!w || w->dim() != 2 || (width != 1 && width != 2)) Py_RETURN_NONE;
+  const int64_t K = w->size(0), N = w->size(1);
+  const c10::Device d = w->device();
+  at::Tensor out = quantized_buffer(K * N, (int)width, d);
+  const hipStream_t st = stream_of(d);
+  const at::Tensor& ws = workspace(d, st);
+  call("prepareB", [&] {
+    return width == 2 ? L.int16_prepare_b(fptr(w), static_cast<int16_t*>(out.data_ptr()), K, N, st)
+                      : L.int8_prepare_b(fptr(w), static_cast<int8_t*>(out.data_ptr()), K, N, ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  Ref shape(shape_tuple(w->sizes()));
+  return make_quantized(std::move(out), shape.p, width == 2 ? type16 : type8, true);
+  MH_END
+}
+
+// prepare_stored(q) -> QTensor in prepared order
+PyObject* py_prepare_stored(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(1, "prepare_stored");
+  Quantized q;
+  if(!matrix(args[0], q, false)) Py_RETURN_NONE;
+  const c10::Device d = q.t->device();
+  at::Tensor out = quantized_buffer(q.rows * q.cols, q.width, d);
+  const hipStream_t st = stream_of(d);
+  call("prepareAndTransposeB", [&] {
+    return q.width == 2 ? L.int16_prepare_b_quantized_transposed(static_cast<const int16_t*>(q.t->const_data_ptr()),
+                                                                 static_cast<int16_t*>(out.data_ptr()), q.rows, q.cols, st)
+                        : L.int8_prepare_b_quantized_transposed(static_cast<const int8_t*>(q.t->const_data_ptr()),
+                                                                static_cast<int8_t*>(out.data_ptr()), q.rows, q.cols, st);
+  });
+  return make_quantized(std::move(out), q.shape.p, q.width == 2 ? type16 : type8, true);
+  MH_END
+}
+
+// ---- float operators ----------------------------------------------------------------------------
+// (out, absmax of out) when it was asked for, else out
+PyObject* with_absmax(at::Tensor out, at::Tensor omax) {
+  if(!omax.defined()) return wrap(std::move(out));
+  Ref o(wrap(std::move(out))), m(make_absmax(std::move(omax)));
+  return PyTuple_Pack(2, o.p, m.p);
+}
+
+// layer_norm(x, gamma, beta, eps, add, want_absmax)
+PyObject* py_layer_norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(6, "layer_norm");
+  const at::Tensor *x = f32c(args[0]), *gamma = f32c(args[1]), *beta, *add;
+  if(!x || x->dim() < 1 || !gamma || !f32c_or_none(args[2], &beta) || !f32c_or_none(args[4], &add)) Py_RETURN_NONE;
+  const int64_t cols = x->size(-1), rows = cols ? x->numel() / cols : 0;
+  if((gamma->numel() != 1 && gamma->numel() != cols) || (beta && beta->numel() != 1 && beta->numel() != cols) ||
+     (add && add->sizes() != x->sizes()))
+    Py_RETURN_NONE;
+  const float eps = (float)number(args[3]);
+  const c10::Device d = x->device();
+  at::Tensor out = empty(x->sizes(), at::kFloat, d), omax;
+  if(truth(args[5])) omax = absmax_slots(d);
+  const hipStream_t st = stream_of(d);
+  call("layerNorm", [&] {
+    return L.layer_norm(fptr(x), fptr(add), fptr(gamma), gamma->numel(), fptr(beta), beta ? beta->numel() : 0, fptr_mut(out), rows,
+                        cols, eps, omax.defined() ? fptr_mut(omax) : nullptr, st);
+  });
+  return with_absmax(std::move(out), std::move(omax));
+  MH_END
+}
+
+// embed(E, ids, scale, signal, rowsPerSignal, want_absmax, out)
+PyObject* py_embed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(7, "embed");
+  const at::Tensor *E = f32c(args[0]), *ids = tensor(args[1]), *signal, *given;
+  if(!E || E->dim() != 2 || !ids || !ids_type(ids->scalar_type()) || !ids->is_contiguous() || ids->device() != E->device() ||
+     !f32c_or_none(args[3], &signal) || !f32c_or_none(args[6], &given))
+    Py_RETURN_NONE;
+  const int64_t vocab = E->size(0), dim = E->size(1), rows = ids->numel();
+  if(signal && (dim == 0 || signal->numel() % dim != 0)) Py_RETURN_NONE;
+  const c10::Device d = E->device();
+  at::Tensor out;
+  if(given) {
+    if(given->device() != d || given->numel() != rows * dim) Py_RETURN_NONE;
+    const float *lo = fptr(given), *table = fptr(E);
+    if(lo < table + E->numel() && table < lo + given->numel()) Py_RETURN_NONE;
+    out = *given;
+  } else {
+    at::DimVector size(ids->sizes().begin(), ids->sizes().end());
+    size.push_back(dim);
+    out = empty(size, at::kFloat, d);
+  }
+  const float scale = (float)number(args[2]);
+  const int64_t per = whole(args[4]);
+  at::Tensor omax;
+  if(truth(args[5])) omax = absmax_slots(d);
+  const hipStream_t st = stream_of(d);
+  call("scaledEmbeddings", [&] {
+    return L.embed(fptr(E), static_cast<const uint32_t*>(ids->const_data_ptr()), rows, vocab, dim, scale, fptr(signal), per,
+                   signal ? signal->numel() / dim : 0, fptr_mut(out), omax.defined() ? fptr_mut(omax) : nullptr, st);
+  });
+  return with_absmax(std::move(out), std::move(omax));
+  MH_END
+}
+
+// select_state(state, ids, out, used)
+PyObject* py_select_state(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(4, "select_state");
+  const at::Tensor *s = f32c(args[0]), *ids = tensor(args[1]), *out = f32c(args[2]);
+  if(!s || !out || s->dim() != 3 || out->dim() != 3 || !ids || !ids_type(ids->scalar_type()) || !ids->is_contiguous() ||
+     ids->device() != s->device() || out->size(0) != ids->numel() || out->size(1) != s->size(1) || out->size(2) != s->size(2))
+    Py_RETURN_NONE;
+  const int64_t used = none(args[3]) ? s->size(2) : whole(args[3]);
+  const hipStream_t st = stream_of(s->device());
+  call("selectState", [&] {
+    return L.select_state(fptr(s), static_cast<const uint32_t*>(ids->const_data_ptr()), ids->numel(), s->size(0), s->size(1), s->size(2),
+                          used, fptr_mut(*out), st);
+  });
+  Py_INCREF(args[2]);
+  return args[2];
+  MH_END
+}
+
+// attention(q, k, v, mask, rowsPerMask, want_absmax, kNew, vNew, kvLen) -> out or (out, absmax)
+PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(9, "attention");
+  const at::Tensor *q = f32c(args[0]), *k = f32c(args[1]), *v = f32c(args[2]), *mask, *kn, *vn;
+  if(!q || !k || !v || q->dim() < 2 || k->dim() < 2 || k->sizes() != v->sizes() || !f32c_or_none(args[3], &mask) ||
+     !f32c_or_none(args[6], &kn) || !f32c_or_none(args[7], &vn))
+    Py_RETURN_NONE;
+  const int64_t dk = q->size(-1), m = q->size(-2), cap = k->size(-2), len = none(args[8]) ? cap : whole(args[8]);
+  if(k->size(-1) != dk || len <= 0 || len > cap || m * dk == 0 || (mask && mask->numel() % len != 0)) Py_RETURN_NONE;
+  const int64_t per = whole(args[4]);
+  const bool want = truth(args[5]);
+  const c10::Device d = q->device();
+  at::Tensor out = empty(q->sizes(), at::kFloat, d), omax;
+  if(want) omax = absmax_slots(d);
+  const hipStream_t st = stream_of(d);
+  call("Attention", [&] {
+    return L.attention_cached(fptr(q), fptr_mut(*k), fptr_mut(*v), fptr(mask), mask ? mask->numel() / len : 0, per, fptr_mut(out),
+                              q->numel() / (m * dk), k->numel() / (cap * dk), m, len, cap, dk, (float)(1.0 / std::pow((double)dk, 0.5)),
+                              want ? fptr_mut(omax) : nullptr, fptr(kn), fptr(vn), st);
+  });
+  return with_absmax(std::move(out), std::move(omax));
+  MH_END
+}
+
+// proj_attention(x, weights, k, v, heads, kvLen, mask, absmax, want_absmax, want_projections)
+//   -> (out, aQuant[, absmax][, projections])
+PyObject* py_proj_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(10, "proj_attention");
+  const at::Tensor *x = f32c(args[0]), *k = f32c(args[2]), *v = f32c(args[3]), *mask;
+  Matrices w;
+  const float* amax = nullptr;
+  if(!x || x->dim() < 1 || !k || !v || k->dim() < 2 || k->size(-1) != 64 || k->sizes() != v->sizes() ||
+     !matrices(args[1], x->size(-1), false, w) || (w.n != 1 && w.n != 3) || !f32c_or_none(args[6], &mask) || !absmax_in(args[7], &amax))
+    Py_RETURN_NONE;
+  const int64_t heads = whole(args[4]), N = heads * 64, K = x->size(-1), M = K ? x->numel() / K : 0;
+  const int64_t cap = k->size(-2), len = none(args[5]) ? cap : whole(args[5]);
+  for(int g = 0; g < w.n; ++g)
+    if(w.b[g].cols != N) Py_RETURN_NONE;
+  if(cap <= 0 || len <= 0 || (mask && mask->numel() % len != 0)) Py_RETURN_NONE;
+  const bool want = truth(args[8]), want_proj = truth(args[9]);
+  const c10::Device d = x->device();
+  const at::DimVector size = with_last(x->sizes(), N);
+  at::Tensor out = empty(size, at::kFloat, d), aq = quantized_buffer(M * K, 1, d), omax, projections[3];
+  float* proj[3] = {nullptr, nullptr, nullptr};
+  if(want) omax = absmax_slots(d);
+  if(want_proj)
+    for(int g = 0; g < w.n; ++g) {
+      projections[g] = empty(size, at::kFloat, d);
+      proj[g] = fptr_mut(projections[g]);
+    }
+  const hipStream_t st = stream_of(d);
+  const at::Tensor& ws = workspace(d, st);
+  call("ProjectedAttention", [&] {
+    return L.int8_proj_attention(fptr(x), static_cast<int8_t*>(aq.data_ptr()), w.n, w.Bq, w.bias, proj, M, K, heads, fptr_mut(*k),
+                                 fptr_mut(*v), k->numel() / (cap * 64), len, cap, fptr(mask), mask ? mask->numel() / len : 0, 1.0f / 8.0f,
+                                 fptr_mut(out), amax, want ? fptr_mut(omax) : nullptr, ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  Ref r(ok(PyTuple_New(2 + (want ? 1 : 0) + (want_proj ? 1 : 0))));
+  PyTuple_SET_ITEM(r.p, 0, wrap(std::move(out)));
+  Ref shape(shape_tuple(x->sizes()));
+  PyTuple_SET_ITEM(r.p, 1, make_quantized(std::move(aq), shape.p, type8, false));
+  if(want) PyTuple_SET_ITEM(r.p, 2, make_absmax(std::move(omax)));
+  if(want_proj) {
+    Ref list(ok(PyList_New(w.n)));
+    for(int g = 0; g < w.n; ++g) PyList_SET_ITEM(list.p, g, wrap(std::move(projections[g])));
+    PyTuple_SET_ITEM(r.p, want ? 3 : 2, list.release());
+  }
+  return r.release();
+  MH_END
+}
+
+// attention_ancestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax) -> out or (out, absmax)
+PyObject* py_attention_ancestors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(8, "attention_ancestors");
+  const at::Tensor *q = f32c(args[0]), *k = f32c(args[1]), *v = f32c(args[2]), *anc = tensor(args[3]), *kn = f32c(args[5]), *vn = f32c(args[6]);
+  if(!q || !k || !v || !kn || !vn || k->dim() != 3 || k->sizes() != v->sizes() || !anc || !ids_type(anc->scalar_type()) ||
+     !anc->is_cuda() || !anc->is_contiguous() || anc->dim() != 2 || anc->size(1) != k->size(1) || anc->size(0) <= 0 ||
+     k->size(0) % anc->size(0) != 0)
+    Py_RETURN_NONE;
+  const int64_t entries = k->size(0), cap = k->size(1), dk = k->size(2), hyps = anc->size(0), len = whole(args[4]);
+  if(q->numel() != entries * dk || kn->numel() != entries * dk || vn->numel() != entries * dk) Py_RETURN_NONE;
+  const c10::Device d = q->device();
+  at::Tensor out = empty(q->sizes(), at::kFloat, d), omax;
+  if(truth(args[7])) omax = absmax_slots(d);
+  const hipStream_t st = stream_of(d);
+  call("AttentionByAncestors", [&] {
+    return L.attention_ancestors(fptr(q), fptr_mut(*k), fptr_mut(*v), fptr_mut(out), hyps, entries / hyps, len, cap, dk,
+                                 (float)(1.0 / std::pow((double)dk, 0.5)), omax.defined() ? fptr_mut(omax) : nullptr, fptr(kn), fptr(vn),
+                                 static_cast<const uint32_t*>(anc->const_data_ptr()), st);
+  });
+  return with_absmax(std::move(out), std::move(omax));
+  MH_END
+}
+
+// ancestors_advance(prev, parents, lenPrev, out)
+PyObject* py_ancestors_advance(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(4, "ancestors_advance");
+  const at::Tensor *prev = tensor(args[0]), *par = tensor(args[1]), *out = tensor(args[3]);
+  if(!prev || !par || !out || prev->scalar_type() != at::kInt || out->scalar_type() != at::kInt || prev->dim() != 2 ||
+     prev->sizes() != out->sizes() || !prev->is_cuda() || !prev->is_contiguous() || !out->is_contiguous() ||
+     !ids_type(par->scalar_type()) || !par->is_contiguous() || par->numel() != prev->size(0))
+    Py_RETURN_NONE;
+  const int64_t len = whole(args[2]);
+  const hipStream_t st = stream_of(prev->device());
+  call("advanceAncestors", [&] {
+    return L.ancestors_advance(static_cast<const uint32_t*>(prev->const_data_ptr()), static_cast<const uint32_t*>(par->const_data_ptr()),
+                               prev->size(0), prev->size(1), len, static_cast<uint32_t*>(out->data_ptr()), st);
+  });
+  Py_INCREF(args[3]);
+  return args[3];
+  MH_END
+}
+
+// ---- n-best -------------------------------------------------------------------------------------
+// nbest(scores, N): scores [dimBatch, ..]
+PyObject* py_nbest(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(2, "nbest");
+  const at::Tensor* s = f32c(args[0]);
+  if(!s || s->dim() < 1) Py_RETURN_NONE;
+  const int64_t N = whole(args[1]), batch = s->size(0), row = batch ? s->numel() / batch : 0;
+  const c10::Device d = s->device();
+  at::Tensor vals = empty({batch * N}, at::kFloat, d), keys = empty({batch * N}, at::kInt, d);
+  const hipStream_t st = stream_of(d);
+  call("getNBestList", [&] {
+    return L.nbest(fptr(s), batch, row, N, fptr_mut(vals), static_cast<uint32_t*>(keys.data_ptr()), st);
+  });
+  Ref a(wrap(std::move(vals))), b(wrap(std::move(keys)));
+  return PyTuple_Pack(2, a.p, b.p);
+  MH_END
+}
+
+// nbest_beams(scores, N): scores [beam, .., vocab]
+PyObject* py_nbest_beams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(2, "nbest_beams");
+  const at::Tensor* s = f32c(args[0]);
+  if(!s || s->dim() < 2) Py_RETURN_NONE;
+  const int64_t N = whole(args[1]), beam = s->size(0), vocab = s->size(-1), batch = beam * vocab != 0 ? s->numel() / (beam * vocab) : 0;
+  const c10::Device d = s->device();
+  at::Tensor vals = empty({batch * N}, at::kFloat, d), keys = empty({batch * N}, at::kInt, d);
+  const hipStream_t st = stream_of(d);
+  const at::Tensor ws = nbest_workspace(beam, batch, vocab, N, d, st);
+  call("getNBestListOfBeams", [&] {
+    return L.nbest_beams(fptr(s), beam, batch, vocab, N, fptr_mut(vals), static_cast<uint32_t*>(keys.data_ptr()), ws.data_ptr(),
+                         (size_t)ws.numel(), st);
+  });
+  Ref a(wrap(std::move(vals))), b(wrap(std::move(keys)));
+  return PyTuple_Pack(2, a.p, b.p);
+  MH_END
+}
+
+// logsoftmax_nbest_beams(logits, N, pathScores, want_logprobs): the sizes of the one-launch form only
+PyObject* py_logsoftmax_nbest_beams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(4, "logsoftmax_nbest_beams");
+  const at::Tensor *s = f32c(args[0]), *add;
+  if(!s || s->dim() < 2 || !f32c_or_none(args[2], &add)) Py_RETURN_NONE;
+  const int64_t N = whole(args[1]), beam = s->size(0), vocab = s->size(-1), batch = beam * vocab != 0 ? s->numel() / (beam * vocab) : 0;
+  if(vocab % 4 != 0 || vocab <= 4096 || vocab > 32768 || reinterpret_cast<uintptr_t>(s->const_data_ptr()) % 16 != 0 ||
+     (add && add->numel() != beam * batch))
+    Py_RETURN_NONE;
+  const c10::Device d = s->device();
+  at::Tensor vals = empty({batch * N}, at::kFloat, d), keys = empty({batch * N}, at::kInt, d), lp;
+  if(truth(args[3])) lp = empty(s->sizes(), at::kFloat, d);
+  const hipStream_t st = stream_of(d);
+  const at::Tensor ws = nbest_workspace(beam, batch, vocab, N, d, st);
+  call("logsoftmaxNBestOfBeams", [&] {
+    return L.logsoftmax_nbest_beams(fptr(s), fptr(add), lp.defined() ? fptr_mut(lp) : nullptr, beam, batch, vocab, N, fptr_mut(vals),
+                                    static_cast<uint32_t*>(keys.data_ptr()), ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  Ref a(wrap(std::move(vals))), b(wrap(std::move(keys)));
+  if(!lp.defined()) return PyTuple_Pack(2, a.p, b.p);
+  Ref c(wrap(std::move(lp)));
+  return PyTuple_Pack(3, a.p, b.p, c.p);
+  MH_END
+}
+
+// ---- module -------------------------------------------------------------------------------------
+// workspace(device index) -> the workspace of that device's current stream
+PyObject* py_workspace(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(1, "workspace");
+  const c10::Device d(c10::kCUDA, (c10::DeviceIndex)whole(args[0]));
+  return wrap(workspace(d, stream_of(d)));
+  MH_END
+}
+
+// use(handle): takes the C ABI's functions from a loaded library (a dlopen handle)
+PyObject* py_use(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(1, "use");
+  void* h = PyLong_AsVoidPtr(args[0]);
+  if(!h && PyErr_Occurred()) return nullptr;
+  Library n{};
+#define F(name)                                                                          \
+  n.name = reinterpret_cast<decltype(&marian_hip_##name)>(dlsym(h, "marian_hip_" #name)); \
+  if(!n.name) {                                                                          \
+    PyErr_SetString(PyExc_ImportError, "marian_hip_" #name " is not in the library");     \
+    return nullptr;                                                                      \
+  }
+  MH_FUNCTIONS(F)
+#undef F
+  L = n;
+  Py_RETURN_NONE;
+  MH_END
+}
+
+// setup(QTensor, AbsMax, Type.intgemm8, Type.intgemm16, check)
+PyObject* py_setup(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(5, "setup");
+  if(!PyType_Check(args[0]) || !PyType_Check(args[1])) {
+    PyErr_SetString(PyExc_TypeError, "setup expects two classes first");
+    return nullptr;
+  }
+  for(int i = 0; i < 5; ++i) Py_INCREF(args[i]);   // (kept for good)
+  QTensorType = reinterpret_cast<PyTypeObject*>(args[0]);
+  AbsMaxType = reinterpret_cast<PyTypeObject*>(args[1]);
+  type8 = args[2];
+  type16 = args[3];
+  raise_status = args[4];
+  Py_RETURN_NONE;
+  MH_END
+}
+
+#define MH_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&py_##name)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
+    MH_METHOD(affine_f32_grouped), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
+    MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors),
+    MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", "host path of the operators", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit__host_calls() {
+  s_data = PyUnicode_InternFromString("data");
+  s_shape = PyUnicode_InternFromString("shape");
+  s_type = PyUnicode_InternFromString("type");
+  s_prepared = PyUnicode_InternFromString("prepared");
+  no_args = PyTuple_New(0);
+  if(!s_data || !s_shape || !s_type || !s_prepared || !no_args) return nullptr;
+  return PyModule_Create(&module);
+}

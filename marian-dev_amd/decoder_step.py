@@ -146,8 +146,7 @@ class DecoderStep:
         tr = self.trace
 
         def rec(kind, **kw):   # clones: later calls overwrite nothing, but the caches are updated in place
-            if tr is not None:
-                tr.append((kind, {k: (v.clone() if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}))
+            tr.append((kind, {k: (v.clone() if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}))
         H, M, d = self.H, self.M, self.d
         dk = d // H
         x, xmax = self.x, None
@@ -155,13 +154,14 @@ class DecoderStep:
         if select and not gemm_only:
             before = self.state
             self.select_states()
-            if not self.by_ancestors:
+            if tr is not None and not self.by_ancestors:
                 rec("select", state=before, rows=self.state_rows, out=self.state, heads=H, used=(self.T - 1) * dk)
         if not gemm_only:
             x = ops.scaledEmbeddings(self.E, self.words, self.emb_scale, self.signal, M, want_absmax=ch)
             if ch:
                 x, xmax = x
-            rec("embed", E=self.E, ids=self.words, scale=self.emb_scale, signal=self.signal, out=x, position=self.T - 1)
+            if tr is not None:
+                rec("embed", E=self.E, ids=self.words, scale=self.emb_scale, signal=self.signal, out=x, position=self.T - 1)
         for li, ly in enumerate(W["layers"]):
             omax = x1max = comax = x2max = f1max = None
             fuse = fused_attention and not gemm_only and not self.by_ancestors and ch
@@ -177,7 +177,6 @@ class DecoderStep:
                         rec("affine", a=x, w=ly[name], out=t, relu=False)
                     rec("self_attention", q=q, k_new=k, v_new=v, k_cache=k_before, v_cache=v_before,
                         k_after=self.Kself[li], v_after=self.Vself[li], out=o, len=self.T)
-                o = o.view(M, d)
             else:
                 if grouped:   # one abs-max, one quantization, one launch for the three projections
                     (q, k, v), _ = integer.affine_f32_grouped(x, [ly["Wq"], ly["Wk"], ly["Wv"]], absmax=xmax)
@@ -185,8 +184,9 @@ class DecoderStep:
                     q, _ = integer.affine_f32(x, *ly["Wq"], absmax=xmax)
                     k, _ = integer.affine_f32(x, *ly["Wk"], absmax=xmax)
                     v, _ = integer.affine_f32(x, *ly["Wv"], absmax=xmax)
-                for name, t in (("Wq", q), ("Wk", k), ("Wv", v)):
-                    rec("affine", a=x, w=ly[name], out=t, relu=False)
+                if tr is not None:
+                    for name, t in (("Wq", q), ("Wk", k), ("Wv", v)):
+                        rec("affine", a=x, w=ly[name], out=t, relu=False)
                 if gemm_only:
                     o = q
                 else:
@@ -195,8 +195,7 @@ class DecoderStep:
                     if tr is not None:
                         k_before, v_before = self.Kself[li].clone(), self.Vself[li].clone()
                     if self.by_ancestors:
-                        o = ops.AttentionByAncestors(q.view(M * H, 1, dk), self.Kself[li], self.Vself[li], self.anc, self.T,
-                                                     k.view(M * H, dk), v.view(M * H, dk), want_absmax=ch)
+                        o = ops.AttentionByAncestors(q, self.Kself[li], self.Vself[li], self.anc, self.T, k, v, want_absmax=ch)
                     else:
                         o = ops.Attention(q.view(M * H, 1, dk), self.Kself[li], self.Vself[li], want_absmax=ch,
                                           kNew=k.view(M * H, dk), vNew=v.view(M * H, dk), kvLen=self.T)
@@ -207,14 +206,16 @@ class DecoderStep:
                             k_after=self.Kself[li], v_after=self.Vself[li], out=o, len=self.T)
                     o = o.view(M, d)
             a, _ = integer.affine_f32(o, *ly["Wo"], absmax=omax)
-            rec("affine", a=o, w=ly["Wo"], out=a, relu=False)
+            if tr is not None:
+                rec("affine", a=o, w=ly["Wo"], out=a, relu=False)
             if gemm_only:
                 x1 = a
             else:
                 x1 = ops.layerNorm(a, *ly["ln1"], eps=1e-6, add=x, want_absmax=ch)
                 if ch:
                     x1, x1max = x1
-                rec("layer_norm", x=a, add=x, gamma=ly["ln1"][0], beta=ly["ln1"][1], out=x1)
+                if tr is not None:
+                    rec("layer_norm", x=a, add=x, gamma=ly["ln1"][0], beta=ly["ln1"][1], out=x1)
             if fused_attention and not gemm_only and ch:   # the context attention's Wq and the attention in one launch
                 res = ops.ProjectedAttention(x1, [ly["cWq"]], self.Kenc[li], self.Venc[li], H, mask=self.mask,
                                              absmax=x1max, want_absmax=True, want_projections=tr is not None)
@@ -223,10 +224,10 @@ class DecoderStep:
                     cq = res[3][0]
                     rec("affine", a=x1, w=ly["cWq"], out=cq, relu=False)
                     rec("context_attention", q=cq, k=self.Kenc[li], v=self.Venc[li], mask=self.mask, out=co)
-                co = co.view(M, d)
             else:
                 cq, _ = integer.affine_f32(x1, *ly["cWq"], absmax=x1max)
-                rec("affine", a=x1, w=ly["cWq"], out=cq, relu=False)
+                if tr is not None:
+                    rec("affine", a=x1, w=ly["cWq"], out=cq, relu=False)
                 if gemm_only:
                     co = cq
                 else:
@@ -234,25 +235,30 @@ class DecoderStep:
                                        rowsPerMask=H, want_absmax=ch)
                     if ch:
                         co, comax = co
-                    rec("context_attention", q=cq, k=self.Kenc[li], v=self.Venc[li], mask=self.mask, out=co)
+                    if tr is not None:
+                        rec("context_attention", q=cq, k=self.Kenc[li], v=self.Venc[li], mask=self.mask, out=co)
                     co = co.view(M, d)
             ca, _ = integer.affine_f32(co, *ly["cWo"], absmax=comax)
-            rec("affine", a=co, w=ly["cWo"], out=ca, relu=False)
+            if tr is not None:
+                rec("affine", a=co, w=ly["cWo"], out=ca, relu=False)
             if gemm_only:
                 x2 = ca
             else:
                 x2 = ops.layerNorm(ca, *ly["ln2"], eps=1e-6, add=x1, want_absmax=ch)
                 if ch:
                     x2, x2max = x2
-                rec("layer_norm", x=ca, add=x1, gamma=ly["ln2"][0], beta=ly["ln2"][1], out=x2)
+                if tr is not None:
+                    rec("layer_norm", x=ca, add=x1, gamma=ly["ln2"][0], beta=ly["ln2"][1], out=x2)
             f1 = integer.affine_f32(x2, *ly["W1"], relu=True, absmax=x2max, want_absmax=ch)
             if ch:
                 f1, _, f1max = f1
             else:
                 f1 = f1[0]
-            rec("affine", a=x2, w=ly["W1"], out=f1, relu=True)
+            if tr is not None:
+                rec("affine", a=x2, w=ly["W1"], out=f1, relu=True)
             f2, _ = integer.affine_f32(f1, *ly["W2"], absmax=f1max)
-            rec("affine", a=f1, w=ly["W2"], out=f2, relu=False)
+            if tr is not None:
+                rec("affine", a=f1, w=ly["W2"], out=f2, relu=False)
             if gemm_only:
                 x = f2
             else:
@@ -260,19 +266,23 @@ class DecoderStep:
                 x = ops.layerNorm(f2, *ly["ln3"], eps=1e-6, add=x2, want_absmax=ch)
                 if ch:
                     x, xmax = x
-                rec("layer_norm", x=f2, add=xin, gamma=ly["ln3"][0], beta=ly["ln3"][1], out=x)
+                if tr is not None:
+                    rec("layer_norm", x=f2, add=xin, gamma=ly["ln3"][0], beta=ly["ln3"][1], out=x)
         logits, _ = integer.affine_f32(x, *W["out"], absmax=xmax)
-        rec("affine", a=x, w=W["out"], out=logits, relu=False)
+        if tr is not None:
+            rec("affine", a=x, w=W["out"], out=logits, relu=False)
         if gemm_only:
             return logits
         if fused_tail:
             vals, keys = ops.logsoftmaxNBestOfBeams(logits.view(self.beam, 1, self.batch, self.V), self.beam)
-            rec("logsoftmax_nbest", logits=logits, vals=vals, keys=keys)
+            if tr is not None:
+                rec("logsoftmax_nbest", logits=logits, vals=vals, keys=keys)
             return vals, keys
         # log-probabilities, then the beam's n-best per sentence over beam x vocabulary
         lp = ops.logsoftmax(logits)
         # (the transposition to [batch, beam * V] of beam_search.cpp:472 happens inside the call)
         vals, keys = ops.getNBestListOfBeams(lp.view(self.beam, 1, self.batch, self.V), self.beam)
-        rec("logsoftmax", x=logits, out=lp)
-        rec("nbest", scores=lp, vals=vals, keys=keys)
+        if tr is not None:
+            rec("logsoftmax", x=logits, out=lp)
+            rec("nbest", scores=lp, vals=vals, keys=keys)
         return lp

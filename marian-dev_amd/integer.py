@@ -105,6 +105,29 @@ def getQuantMult(q):
     return float(q.data[n:n + 4].cpu().numpy().view(np.float32)[0])
 
 
+class AbsMax:
+    """Values whose maximum is max|x| of the tensor they were produced with (2048 floats on the
+    device): handed from the call that writes a tensor to the affine call that reads it, in place
+    of the abs-max pass of prepareA (reference src/tensors/cpu/intgemm_interface.h:23)."""
+
+    def __init__(self, device):
+        self.data = torch.empty(_lib.ABSMAX_SLOTS, dtype=torch.float32, device=device)
+
+    def data_ptr(self):
+        return self.data.data_ptr()
+
+
+# The operators' host path: each function takes arguments in normal form (float32 on the GPU, contiguous,
+# prepared weights) and returns None for anything else, which the functions below then refuse or convert.
+_host = _lib.HostCalls(lambda: (QTensor, AbsMax, Type.intgemm8, Type.intgemm16, _lib.check))
+
+
+def _taken(result, what):
+    """the result of a host call whose arguments have been checked and converted"""
+    _abort_if(result is None, "{}: arguments of another kind than the operator takes", what)
+    return result
+
+
 class Backend:
     """Per-device state the path needs: a stream and the abs-max workspace, the counterpart of
     gpu::Backend (reference src/tensors/gpu/backend.h:23-110) reduced to this path.  The stream is
@@ -117,7 +140,6 @@ class Backend:
     def __init__(self, device):
         self.device = torch.device(device)
         self.workspace_bytes = int(self.lib.marian_hip_int8_workspace_bytes())
-        self._workspaces = {}   # stream handle -> workspace (kept for good: a graph may have recorded it)
         # float32 weights are quantized on first use and remembered when this is Type.intgemm8:
         # the counterpart of getGemmType() (reference src/tensors/backend.h:36-40) with the
         # memoized packing of src/graph/expression_operators.cpp:564-598 (its FBGEMM branch
@@ -132,12 +154,10 @@ class Backend:
     @property
     def workspace(self):
         """The workspace of the current stream (calls on one stream run one after the other and
-        share it; calls on different streams may overlap and must not)."""
-        key = self.stream()
-        ws = self._workspaces.get(key)
-        if ws is None:
-            ws = self._workspaces.setdefault(key, torch.empty(self.workspace_bytes, dtype=torch.uint8, device=self.device))
-        return ws
+        share it; calls on different streams may overlap and must not).  Kept for good: a graph may
+        have recorded its address."""
+        index = self.device.index
+        return _host.workspace(torch.cuda.current_device() if index is None else index)
 
     def setGemmType(self, type_):
         _abort_if(type_ not in (None, Type.intgemm8), "Unsupported type {} for Intgemm type??", type_)
@@ -190,58 +210,47 @@ def _backend_of(t):
     return Backend.get(dev)
 
 
+def _on_gpu(t):
+    _abort_if(t.device.type != "cuda", "the HIP int8 backend needs device tensors, got {}", t.device)
+
+
 def prepareA(a, type_=Type.intgemm8):
     """reference src/tensors/cpu/intgemm_interface.h:17-32 for vtype = intgemm8 (abs-max quantMult)
     or intgemm16 (quantMult 1024, src/tensors/cpu/integer_common.h:174-175)."""
     _abort_if(a.dtype != torch.float32, "Intgemm expects type of A to be float32 not {}", a.dtype)
     _abort_if(type_ not in (Type.intgemm8, Type.intgemm16), "Unsupported type {} for Intgemm type??", type_)
     a = a.contiguous()
-    be = _backend_of(a)
-    out = QTensor.empty(a.shape, type_, a.device)
-    K = cols(a)
-    M = rows(a) if a.numel() else 0
-    if type_ == Type.intgemm16:
-        _lib.check(be.lib.marian_hip_int16_prepare_a(a.data_ptr(), out.data_ptr(), M, K, be.stream()), "prepareA")
-        return out
-    st = be.lib.marian_hip_int8_prepare_a(a.data_ptr(), out.data_ptr(), M, K,
-                                          be.workspace.data_ptr(), be.workspace_bytes, be.stream())
-    _lib.check(st, "prepareA")
-    return out
+    _on_gpu(a)
+    return _taken(_host.prepare_a(a, sizeOf(type_)), "prepareA")
 
 
 def prepareB(w, type_=Type.intgemm8):
     """Offline weight quantizer, reference src/tensors/cpu/expression_graph_packable.h:153-253
-    (intgemm8 branch): fp32 W [K, N] -> Type::intgemm8 tensor of shape [K, N] whose payload is
-    the quantized transpose."""
+    (intgemm8 branch; the 16-bit branch, :203-235, has quantMult 1024): fp32 W [K, N] ->
+    Type::intgemm8 tensor of shape [K, N] whose payload is the quantized transpose."""
+    if type_ is Type.intgemm8:
+        q = _host.prepare_b(w, 1)
+        if q is not None:
+            return q
     _abort_if(type_ not in (Type.intgemm8, Type.intgemm16), "Type {} is not supported", type_)
     _abort_if(w.dtype != torch.float32 or w.dim() != 2, "prepareB expects a float32 matrix, got {}", w.dtype)
     w = w.contiguous()
-    be = _backend_of(w)
-    K, N = w.shape
-    out = QTensor.empty((K, N), type_, w.device, prepared=True)
-    if type_ == Type.intgemm16:   # the 16-bit branch of the packer (:203-235): quantMult 1024
-        _lib.check(be.lib.marian_hip_int16_prepare_b(w.data_ptr(), out.data_ptr(), K, N, be.stream()), "prepareB")
-        return out
-    st = be.lib.marian_hip_int8_prepare_b(w.data_ptr(), out.data_ptr(), K, N,
-                                          be.workspace.data_ptr(), be.workspace_bytes, be.stream())
-    _lib.check(st, "prepareB")
-    return out
+    _on_gpu(w)
+    return _taken(_host.prepare_b(w, sizeOf(type_)), "prepareB")
 
 
 def prepareAndTransposeB(q):
     """A quantized weight item as a model file holds it (plain rows [N, K] + quantMult) -> the
     order the kernels read; reference prepareAndTransposeB, src/tensors/cpu/integer_common.h:189-216
     (there: the tiling of the CPU the process runs on)."""
+    out = _host.prepare_stored(q)
+    if out is not None:
+        return out
     _abort_if(not isinstance(q, QTensor) or not isIntgemm(q.type) or isHardwareSpecific(q.type) or len(q.shape) != 2,
               "prepareAndTransposeB expects a hardware-agnostic intgemm matrix, got {}", getattr(q, "type", type(q)))
     _abort_if(q.prepared, "the weights are prepared already (type {})", q.type)
-    be = _backend_of(q)
-    K, N = q.shape
-    out = QTensor.empty((K, N), q.type, q.data.device, prepared=True)
-    fn = be.lib.marian_hip_int16_prepare_b_quantized_transposed if sizeOf(q.type) == 2 else \
-        be.lib.marian_hip_int8_prepare_b_quantized_transposed
-    _lib.check(fn(q.data_ptr(), out.data_ptr(), K, N, be.stream()), "prepareAndTransposeB")
-    return out
+    _on_gpu(q.data)
+    return _taken(None, "prepareAndTransposeB")
 
 
 def _check_weights(bQuant):
@@ -253,6 +262,24 @@ def _check_weights(bQuant):
               "B of type {} is in file order: it has to go through prepareAndTransposeB first", bQuant.type)
 
 
+def _affine_arguments(a, bQuant, bias, shortlist):
+    """checks the arguments of an affine call; returns a, bias and shortlist in normal form"""
+    _abort_if(not isinstance(a, torch.Tensor) or a.dtype != torch.float32,
+              "Intgemm expects type of A to be float32 not {}", getattr(a, "dtype", type(a)))
+    _check_weights(bQuant)
+    _on_gpu(a)
+    K, N = cols(a), cols(bQuant)
+    _abort_if(rows(bQuant) != K, "Matrix product requires inner dimensions to match: {} vs {}", K, rows(bQuant))
+    if bias is not None:
+        _abort_if(bias.dtype != torch.float32 or bias.numel() != N, "bias must be float32 [1, {}]", N)
+        bias = bias.contiguous()
+    if shortlist is not None:
+        _abort_if(sizeOf(bQuant.type) == 2, "the 16-bit path has no shortlist form (type {})", bQuant.type)
+        _abort_if(shortlist.dtype not in (torch.int32, torch.uint32), "shortlist ids must be uint32, got {}", shortlist.dtype)
+        shortlist = shortlist.contiguous()
+    return a.contiguous(), bias, shortlist
+
+
 def affineOrDot(a, bQuant, bias=None, transA=False, transB=False, scale=1.0, relu=False,
                 shortlist=None):
     """reference src/tensors/cpu/intgemm_interface.h:46-99,102-128.
@@ -260,29 +287,16 @@ def affineOrDot(a, bQuant, bias=None, transA=False, transB=False, scale=1.0, rel
     a: float32 activations; bQuant: QTensor of type intgemm8 with logical shape [K, N].
     transB is ignored like in the reference (:47).  `relu` fuses the in-place ReLU node the
     reference appends (src/graph/expression_operators.cpp:721-731).  `shortlist`: optional
-    uint32 device tensor of sorted unique output ids (multiple of 8 many)."""
-    _abort_if(not isinstance(a, torch.Tensor) or not a.dtype.is_floating_point or a.dtype != torch.float32,
-              "Intgemm expects type of A to be float32 not {}", getattr(a, "dtype", type(a)))
-    _check_weights(bQuant)
-    if transA:
+    uint32 device tensor of sorted unique output ids (multiple of 8 many).  Weights of
+    Type.intgemm16 take the 16-bit path (two nodes one after the other)."""
+    if not transA:
+        out = _host.affine_or_dot(a, bQuant, bias, scale, relu, shortlist)
+        if out is not None:
+            return out
+    elif isinstance(a, torch.Tensor):
         a = a.transpose(-1, -2)
-    if sizeOf(bQuant.type) == 2:   # Type::intgemm16: the two nodes one after the other
-        _abort_if(shortlist is not None, "the 16-bit path has no shortlist form (type {})", bQuant.type)
-        return multiply(prepareA(a, Type.intgemm16), bQuant, bias, scale=scale, relu=relu)
-    out, _ = affine_f32(a, bQuant, bias, scale=scale, relu=relu, shortlist=shortlist)
-    return out
-
-
-class AbsMax:
-    """Values whose maximum is max|x| of the tensor they were produced with (2048 floats on the
-    device): handed from the call that writes a tensor to the affine call that reads it, in place
-    of the abs-max pass of prepareA (reference src/tensors/cpu/intgemm_interface.h:23)."""
-
-    def __init__(self, device):
-        self.data = torch.empty(_lib.ABSMAX_SLOTS, dtype=torch.float32, device=device)
-
-    def data_ptr(self):
-        return self.data.data_ptr()
+    a, bias, shortlist = _affine_arguments(a, bQuant, bias, shortlist)
+    return _taken(_host.affine_or_dot(a, bQuant, bias, scale, relu, shortlist), "affineOrDot")
 
 
 def affine_f32(a, bQuant, bias=None, scale=1.0, relu=False, shortlist=None, absmax=None,
@@ -291,39 +305,11 @@ def affine_f32(a, bQuant, bias=None, scale=1.0, relu=False, shortlist=None, absm
     (one fused kernel for small activations).  Returns (out, aQuant): aQuant is what the
     prepareA node would have produced.  absmax: the AbsMax left by the call that produced `a`;
     want_absmax: also return an AbsMax of `out` as a third value."""
-    _check_weights(bQuant)
-    a = a.contiguous()
-    be = _backend_of(a)
-    aQuant = QTensor.empty(a.shape, Type.intgemm8, a.device)
-    K, N = cols(a), cols(bQuant)
-    _abort_if(rows(bQuant) != K, "Matrix product requires inner dimensions to match: {} vs {}", K, rows(bQuant))
-    M = rows(a) if a.numel() else 0
-    n_out = N if shortlist is None else int(shortlist.numel())
-    out = torch.empty(tuple(a.shape[:-1]) + (n_out,), dtype=torch.float32, device=a.device)
-    bias_ptr = None
-    if bias is not None:
-        _abort_if(bias.dtype != torch.float32 or bias.numel() != N, "bias must be float32 [1, {}]", N)
-        bias = bias.contiguous()
-        bias_ptr = bias.data_ptr()
-    if shortlist is not None:
-        _abort_if(shortlist.dtype not in (torch.int32, torch.uint32), "shortlist ids must be uint32, got {}", shortlist.dtype)
-    idx_ptr = None if shortlist is None else shortlist.data_ptr()
-    n_idx = n_out if shortlist is not None else 0
-    if absmax is None and not want_absmax:
-        st = be.lib.marian_hip_int8_affine_f32(
-            a.data_ptr(), aQuant.data_ptr(), bQuant.data_ptr(), bias_ptr, idx_ptr, n_idx,
-            out.data_ptr(), M, K, N, scale, int(relu), be.workspace.data_ptr(), be.workspace_bytes,
-            be.stream())
-        _lib.check(st, "affineOrDot")
-        return out, aQuant
-    omax = AbsMax(a.device) if want_absmax else None
-    st = be.lib.marian_hip_int8_affine_f32_chained(
-        a.data_ptr(), aQuant.data_ptr(), bQuant.data_ptr(), bias_ptr, idx_ptr, n_idx,
-        out.data_ptr(), M, K, N, scale, int(relu), None if absmax is None else absmax.data_ptr(),
-        None if omax is None else omax.data_ptr(), be.workspace.data_ptr(), be.workspace_bytes,
-        be.stream())
-    _lib.check(st, "affineOrDot")
-    return (out, aQuant, omax) if want_absmax else (out, aQuant)
+    out = _host.affine_f32(a, bQuant, bias, scale, relu, shortlist, absmax, want_absmax)
+    if out is not None:
+        return out
+    a, bias, shortlist = _affine_arguments(a, bQuant, bias, shortlist)
+    return _taken(_host.affine_f32(a, bQuant, bias, scale, relu, shortlist, absmax, want_absmax), "affineOrDot")
 
 
 def affine_f32_grouped(a, weights, scale=1.0, relu=False, absmax=None):
@@ -331,37 +317,16 @@ def affine_f32_grouped(a, weights, scale=1.0, relu=False, absmax=None):
     (marian_hip_int8_affine_f32_grouped): the self-attention projections Wq, Wk, Wv of reference
     src/models/transformer.h:290-325 read the same input.  weights: list of (bQuant, bias or None).
     Returns ([out, ...], aQuant); each out equals affine_f32(a, bQuant, bias)[0] bit for bit."""
-    import ctypes
+    out = _host.affine_f32_grouped(a, weights, scale, relu, absmax)
+    if out is not None:
+        return out
     for bQuant, _ in weights:
         _check_weights(bQuant)
-    a = a.contiguous()
-    be = _backend_of(a)
-    K = cols(a)
-    M = rows(a) if a.numel() else 0
+        _abort_if(sizeOf(bQuant.type) != 1, "Unsupported type {} for Intgemm type??", bQuant.type)
     n = len(weights)
     _abort_if(n < 1 or n > 4, "between one and four weight matrices per call, got {}", n)
-    aQuant = QTensor.empty(a.shape, Type.intgemm8, a.device)
-    outs, keep = [], []
-    Bq_arr, bias_arr, out_arr, N_arr = ((ctypes.c_void_p * n)(), (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)(),
-                                        (ctypes.c_int64 * n)())
-    for g, (bQuant, bias) in enumerate(weights):
-        _check_weights(bQuant)
-        _abort_if(sizeOf(bQuant.type) != 1, "Unsupported type {} for Intgemm type??", bQuant.type)
-        _abort_if(rows(bQuant) != K, "Matrix product requires inner dimensions to match: {} vs {}", K, rows(bQuant))
-        N = cols(bQuant)
-        if bias is not None:
-            _abort_if(bias.dtype != torch.float32 or bias.numel() != N, "bias must be float32 [1, {}]", N)
-            bias = bias.contiguous()
-            keep.append(bias)
-        out = torch.empty(tuple(a.shape[:-1]) + (N,), dtype=torch.float32, device=a.device)
-        outs.append(out)
-        Bq_arr[g], bias_arr[g], out_arr[g], N_arr[g] = (bQuant.data_ptr(), None if bias is None else bias.data_ptr(),
-                                                        out.data_ptr(), N)
-    st = be.lib.marian_hip_int8_affine_f32_grouped(
-        a.data_ptr(), aQuant.data_ptr(), n, Bq_arr, bias_arr, out_arr, N_arr, M, K, scale, int(relu),
-        None if absmax is None else absmax.data_ptr(), be.workspace.data_ptr(), be.workspace_bytes, be.stream())
-    _lib.check(st, "affineOrDot")
-    return outs, aQuant
+    weights = [(bQuant, _affine_arguments(a, bQuant, bias, None)[1]) for bQuant, bias in weights]
+    return _taken(_host.affine_f32_grouped(a.contiguous(), weights, scale, relu, absmax), "affineOrDot")
 
 
 def multiply(aQuant, bQuant, bias=None, scale=1.0, relu=False, shortlist=None):
@@ -436,6 +401,10 @@ def _float_b_unsupported(b):
 
 def dot(a, b, transA=False, transB=False, scale=1.0):
     """reference src/graph/expression_operators.cpp:554-619: isIntgemm(b) selects the int8 path."""
+    if not transA:
+        out = _host.affine_or_dot(a, b, None, scale, False, None)
+        if out is not None:
+            return out
     b = _maybe_quantize_b(a, b)
     if isinstance(b, QTensor) and isIntgemm(b.type):
         return affineOrDot(a, b, None, transA, transB, scale)
@@ -444,6 +413,10 @@ def dot(a, b, transA=False, transB=False, scale=1.0):
 
 def affine(a, b, bias, transA=False, transB=False, scale=1.0):
     """reference src/graph/expression_operators.cpp:647-718."""
+    if not transA:
+        out = _host.affine_or_dot(a, b, bias, scale, False, None)
+        if out is not None:
+            return out
     b = _maybe_quantize_b(a, b)
     if isinstance(b, QTensor) and isIntgemm(b.type):
         return affineOrDot(a, b, bias, transA, transB, scale)
@@ -454,6 +427,9 @@ def affineWithReluDropout(x, W, bias, dropProb=0.0):
     """reference src/graph/expression_operators.cpp:721-731 at inference (dropProb == 0): the
     reference runs affine() and then an in-place ReLU node; here the ReLU is the GEMM epilogue."""
     _abort_if(dropProb != 0.0, "dropout is a training feature; inference path expects dropProb == 0, got {}", dropProb)
+    out = _host.affine_or_dot(x, W, bias, 1.0, True, None)
+    if out is not None:
+        return out
     W = _maybe_quantize_b(x, W)
     if isinstance(W, QTensor) and isIntgemm(W.type):
         return affineOrDot(x, W, bias, False, False, 1.0, relu=True)

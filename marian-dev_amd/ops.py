@@ -17,7 +17,7 @@ step is a call into the C ABI.  There is no CPU fallback.
 import torch
 
 from . import _lib
-from .integer import AbsMax, _abort_if, _backend_of
+from .integer import _abort_if, _backend_of, _host, _on_gpu, _taken
 
 
 def _f32c(x, what):
@@ -29,10 +29,12 @@ def layerNorm(x, gamma, beta=None, eps=1e-9, add=None, want_absmax=False):
     """reference src/graph/expression_operators.cpp:901-913; `add` fuses the skip connection in
     front of it (out = layerNorm(x + add)).  want_absmax: also return the AbsMax of the output
     for the affine calls that read it."""
+    out = _host.layer_norm(x, gamma, beta, eps, add, want_absmax)
+    if out is not None:
+        return out
     x = _f32c(x, "layerNorm")
-    be = _backend_of(x)
+    _on_gpu(x)
     cols = x.shape[-1]
-    rows = x.numel() // cols if x.numel() else 0
     gamma = _f32c(gamma, "layerNorm").reshape(-1)
     _abort_if(gamma.numel() not in (1, cols), "layerNorm: gamma must have {} or 1 values", cols)
     if beta is not None:
@@ -41,14 +43,7 @@ def layerNorm(x, gamma, beta=None, eps=1e-9, add=None, want_absmax=False):
     if add is not None:
         add = _f32c(add, "layerNorm")
         _abort_if(tuple(add.shape) != tuple(x.shape), "layerNorm: skip input shape {} vs {}", tuple(add.shape), tuple(x.shape))
-    out = torch.empty_like(x)
-    omax = AbsMax(x.device) if want_absmax else None
-    st = be.lib.marian_hip_layer_norm(
-        x.data_ptr(), None if add is None else add.data_ptr(), gamma.data_ptr(), gamma.numel(),
-        None if beta is None else beta.data_ptr(), 0 if beta is None else beta.numel(),
-        out.data_ptr(), rows, cols, eps, None if omax is None else omax.data_ptr(), be.stream())
-    _lib.check(st, "layerNorm")
-    return (out, omax) if want_absmax else out
+    return _taken(_host.layer_norm(x, gamma, beta, eps, add, want_absmax), "layerNorm")
 
 
 def scaledEmbeddings(E, ids, scale=1.0, signal=None, rowsPerSignal=1, want_absmax=False, out=None):
@@ -57,33 +52,26 @@ def scaledEmbeddings(E, ids, scale=1.0, signal=None, rowsPerSignal=1, want_absma
     [vocab, dimEmb]; ids: integer tensor on the device, any shape; signal: None or [n, dimEmb],
     output row r taking signal row (r / rowsPerSignal) % n.  Returns [*ids.shape, dimEmb] (`out`
     when given: a contiguous float32 tensor of that many values that does not overlap E)."""
+    res = _host.embed(E, ids, scale, signal, rowsPerSignal, want_absmax, out)
+    if res is not None:
+        return res
     E = _f32c(E, "scaledEmbeddings")
-    be = _backend_of(E)
+    _on_gpu(E)
     _abort_if(E.dim() != 2, "scaledEmbeddings: the table has to be a matrix, got shape {}", tuple(E.shape))
     _abort_if(ids.dtype not in (torch.int32, torch.int64, torch.uint32) or ids.device != E.device,
               "scaledEmbeddings: indices have to be an integer tensor on the table's device")
-    vocab, dimEmb = E.shape
     words = ids.contiguous()
     if words.dtype == torch.int64:   # the reference's IndexType has 32 bits
         words = words.to(torch.int32)
-    n_signals = 0
     if signal is not None:
-        signal = _f32c(signal, "scaledEmbeddings").reshape(-1, dimEmb)
-        n_signals = signal.shape[0]
-    if out is None:
-        out = torch.empty(tuple(ids.shape) + (dimEmb,), dtype=torch.float32, device=E.device)
-    else:
+        signal = _f32c(signal, "scaledEmbeddings").reshape(-1, E.shape[1])
+    if out is not None:
         _abort_if(out.dtype != torch.float32 or not out.is_contiguous() or out.device != E.device or
-                  out.numel() != ids.numel() * dimEmb, "scaledEmbeddings: out has to be a contiguous float32 "
-                  "tensor of {} x {} values on the table's device", ids.numel(), dimEmb)
+                  out.numel() != ids.numel() * E.shape[1], "scaledEmbeddings: out has to be a contiguous float32 "
+                  "tensor of {} x {} values on the table's device", ids.numel(), E.shape[1])
         lo, hi = out.data_ptr(), out.data_ptr() + 4 * out.numel()
         _abort_if(lo < E.data_ptr() + 4 * E.numel() and E.data_ptr() < hi, "scaledEmbeddings: out overlaps the table")
-    omax = AbsMax(E.device) if want_absmax else None
-    st = be.lib.marian_hip_embed(E.data_ptr(), words.data_ptr(), words.numel(), vocab, dimEmb, float(scale),
-                                 None if signal is None else signal.data_ptr(), rowsPerSignal, n_signals,
-                                 out.data_ptr(), None if omax is None else omax.data_ptr(), be.stream())
-    _lib.check(st, "scaledEmbeddings")
-    return (out, omax) if want_absmax else out
+    return _taken(_host.embed(E, words, scale, signal, rowsPerSignal, want_absmax, out), "scaledEmbeddings")
 
 
 def rows(a, indices, out=None):
@@ -98,22 +86,21 @@ def selectState(state, indices, out, used=None):
     src/rnn/types.h:22-42): out[r, s, :used] = state[indices[r], s, :used] for a state [entries,
     segments, capacity] whose segments (the cached positions of a head) are in use up to `used`
     values (None: entirely); out [len(indices), segments, capacity] is a tensor of its own."""
+    res = _host.select_state(state, indices, out, used)
+    if res is not None:
+        return res
     _abort_if(state.dtype != torch.float32 or out.dtype != torch.float32 or state.dim() != 3 or out.dim() != 3 or
               not state.is_contiguous() or not out.is_contiguous(), "selectState expects contiguous float32 "
               "tensors [entries, segments, capacity], got {} and {}", tuple(state.shape), tuple(out.shape))
-    be = _backend_of(state)
-    entries, segments, cap = state.shape
-    _abort_if(tuple(out.shape) != (indices.numel(), segments, cap), "selectState: out has shape {}, not {}",
-              tuple(out.shape), (indices.numel(), segments, cap))
+    _on_gpu(state)
+    _abort_if(tuple(out.shape) != (indices.numel(),) + tuple(state.shape[1:]), "selectState: out has shape {}, not {}",
+              tuple(out.shape), (indices.numel(),) + tuple(state.shape[1:]))
     _abort_if(indices.dtype not in (torch.int32, torch.int64, torch.uint32) or indices.device != state.device,
               "selectState: indices have to be an integer tensor on the state's device")
     ids = indices.contiguous()
     if ids.dtype == torch.int64:
         ids = ids.to(torch.int32)
-    st = be.lib.marian_hip_select_state(state.data_ptr(), ids.data_ptr(), ids.numel(), entries, segments, cap,
-                                        cap if used is None else int(used), out.data_ptr(), be.stream())
-    _lib.check(st, "selectState")
-    return out
+    return _taken(_host.select_state(state, ids, out, used), "selectState")
 
 
 def sinusoidalPositionEmbeddings(dimWords, dimEmb, start=0, device=None):
@@ -215,6 +202,11 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     the cached positions, src/models/transformer.h:683-700).
     kvLen: k and v have room for k.shape[-2] positions per entry, of which the first kvLen are in
     use (caches that stay in place from step to step); None: all of them."""
+    m = q.shape[-2]
+    if m < 8 or kNew is not None or want_absmax or kvLen is not None:
+        out = _host.attention(q, k, v, mask, rowsPerMask, want_absmax, kNew, vNew, kvLen)
+        if out is not None:
+            return out
     q = _f32c(q, "Attention")
     _abort_if(k.dtype != torch.float32 or v.dtype != torch.float32, "Attention expects float32, got {}", k.dtype)
     if kNew is None:
@@ -222,35 +214,23 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     else:
         _abort_if(not (k.is_contiguous() and v.is_contiguous()), "Attention: the key/value cache must be contiguous{}", "")
         kNew, vNew = _f32c(kNew, "Attention"), _f32c(vNew, "Attention")
-    be = _backend_of(q)
-    dk, m, cap = q.shape[-1], q.shape[-2], k.shape[-2]
+    _on_gpu(q)
+    dk, cap = q.shape[-1], k.shape[-2]
     L = cap if kvLen is None else int(kvLen)
     _abort_if(not 0 < L <= cap, "Attention: {} positions in use of {} the cache has room for", L, cap)
     _abort_if(k.shape[-1] != dk or tuple(v.shape) != tuple(k.shape), "Attention: key/value shapes {} {} vs dk {}",
               tuple(k.shape), tuple(v.shape), dk)
-    batchQ = q.numel() // (m * dk)
-    batchKV = k.numel() // (cap * dk)
     if m >= 8 and kNew is None and not want_absmax and L == cap:
         # Many query positions per head (encoder layers, whole target sentences): the one-launch
         # form gives every query row a wave that walks the head's keys and values on its own; the
         # three operators share them through LDS tiles (1024 heads of 64 x 64 x 64: 57 us against 105).
+        batchQ, batchKV = q.numel() // (m * dk), k.numel() // (cap * dk)
         scores = bdot_legacy(q.reshape(batchQ, m, dk), k.reshape(batchKV, L, dk), False, True, 1.0 / float(dk) ** 0.5)
         weights = softmax(scores, mask, rowsPerMask)
         return bdot_legacy(weights, v.reshape(batchKV, L, dk)).reshape(q.shape)
-    n_masks = 0
     if mask is not None:
         mask = _f32c(mask, "Attention").reshape(-1, L)
-        n_masks = mask.shape[0]
-    out = torch.empty_like(q)
-    omax = AbsMax(q.device) if want_absmax else None
-    st = be.lib.marian_hip_attention_cached(q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                            None if mask is None else mask.data_ptr(), n_masks, rowsPerMask,
-                                            out.data_ptr(), batchQ, batchKV, m, L, cap, dk, 1.0 / float(dk) ** 0.5,
-                                            None if omax is None else omax.data_ptr(),
-                                            None if kNew is None else kNew.data_ptr(),
-                                            None if vNew is None else vNew.data_ptr(), be.stream())
-    _lib.check(st, "Attention")
-    return (out, omax) if want_absmax else out
+    return _taken(_host.attention(q, k, v, mask, rowsPerMask, want_absmax, kNew, vNew, L), "Attention")
 
 
 def ProjectedAttention(x, weights, k, v, heads, kvLen=None, mask=None, absmax=None, want_absmax=False,
@@ -266,55 +246,29 @@ def ProjectedAttention(x, weights, k, v, heads, kvLen=None, mask=None, absmax=No
     of x left.  Returns (out [M, heads * 64], aQuant) and, when asked for, the AbsMax of out and
     the projections themselves - bit for bit what affine_f32_grouped / affine_f32 followed by
     Attention give (and faster than those up to 128 rows, level at 256, slower at 512)."""
-    import ctypes
+    res = _host.proj_attention(x, weights, k, v, heads, kvLen, mask, absmax, want_absmax, want_projections)
+    if res is not None:
+        return res
     from . import integer
     x = _f32c(x, "ProjectedAttention")
-    be = _backend_of(x)
+    _on_gpu(x)
     n = len(weights)
     _abort_if(n not in (1, 3), "ProjectedAttention: one projection (q) or three (q, k, v), got {}", n)
-    K = x.shape[-1]
-    M = x.numel() // K if x.numel() else 0
-    N = heads * 64
+    K, N = x.shape[-1], heads * 64
     _abort_if(not (k.is_contiguous() and v.is_contiguous()) or k.dtype != torch.float32 or v.dtype != torch.float32,
               "ProjectedAttention: the key/value caches must be contiguous float32{}", "")
     _abort_if(k.shape[-1] != 64 or tuple(k.shape) != tuple(v.shape), "ProjectedAttention: head size 64, got caches {} {}",
               tuple(k.shape), tuple(v.shape))
-    cap = k.shape[-2]
-    L = cap if kvLen is None else int(kvLen)
-    batchKV = k.numel() // (cap * 64)
-    aQuant = integer.QTensor.empty(x.shape, integer.Type.intgemm8, x.device)
-    Bq_arr, bias_arr, proj_arr = (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)()
-    keep, projections = [], []
-    for g, (bQuant, bias) in enumerate(weights):
+    L = k.shape[-2] if kvLen is None else int(kvLen)
+    for bQuant, _ in weights:
         integer._check_weights(bQuant)
         _abort_if(integer.rows(bQuant) != K or integer.cols(bQuant) != N, "ProjectedAttention: weights {} vs [{}, {}]",
                   tuple(bQuant.shape), K, N)
-        Bq_arr[g] = bQuant.data_ptr()
-        if bias is not None:
-            bias = _f32c(bias, "ProjectedAttention")
-            keep.append(bias)
-        bias_arr[g] = None if bias is None else bias.data_ptr()
-        if want_projections:
-            projections.append(torch.empty(tuple(x.shape[:-1]) + (N,), dtype=torch.float32, device=x.device))
-        proj_arr[g] = projections[g].data_ptr() if want_projections else None
-    n_masks = 0
+    weights = [(bQuant, None if bias is None else _f32c(bias, "ProjectedAttention")) for bQuant, bias in weights]
     if mask is not None:
         mask = _f32c(mask, "ProjectedAttention").reshape(-1, L)
-        n_masks = mask.shape[0]
-    out = torch.empty(tuple(x.shape[:-1]) + (N,), dtype=torch.float32, device=x.device)
-    omax = AbsMax(x.device) if want_absmax else None
-    st = be.lib.marian_hip_int8_proj_attention(
-        x.data_ptr(), aQuant.data_ptr(), n, Bq_arr, bias_arr, proj_arr, M, K, heads, k.data_ptr(), v.data_ptr(), batchKV,
-        L, cap, None if mask is None else mask.data_ptr(), n_masks, 1.0 / 8.0, out.data_ptr(),
-        None if absmax is None else absmax.data_ptr(), None if omax is None else omax.data_ptr(),
-        be.workspace.data_ptr(), be.workspace_bytes, be.stream())
-    _lib.check(st, "ProjectedAttention")
-    res = (out, aQuant)
-    if want_absmax:
-        res += (omax,)
-    if want_projections:
-        res += (projections,)
-    return res
+    return _taken(_host.proj_attention(x, weights, k, v, heads, kvLen, mask, absmax, want_absmax, want_projections),
+                  "ProjectedAttention")
 
 
 def AttentionByAncestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax=False):
@@ -323,8 +277,11 @@ def AttentionByAncestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax=Fals
     position p of hypothesis h is read from the cache entry of hypothesis ancestors[h, p].
     q [hyps * heads, 1, dk]; k, v [hyps * heads, capacity, dk]; ancestors int32 [hyps, capacity];
     kNew, vNew [hyps * heads, dk] become position kvLen - 1 of the hypotheses' own entries."""
+    out = _host.attention_ancestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax)
+    if out is not None:
+        return out
     q, kNew, vNew = _f32c(q, "AttentionByAncestors"), _f32c(kNew, "AttentionByAncestors"), _f32c(vNew, "AttentionByAncestors")
-    be = _backend_of(q)
+    _on_gpu(q)
     _abort_if(k.dtype != torch.float32 or v.dtype != torch.float32 or not (k.is_contiguous() and v.is_contiguous()) or
               k.dim() != 3 or tuple(k.shape) != tuple(v.shape), "AttentionByAncestors: the caches have to be contiguous "
               "float32 tensors [entries, capacity, dk], got {} and {}", tuple(k.shape), tuple(v.shape))
@@ -332,82 +289,50 @@ def AttentionByAncestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax=Fals
     _abort_if(ancestors.dtype not in (torch.int32, torch.uint32) or ancestors.dim() != 2 or ancestors.shape[1] != cap or
               not ancestors.is_contiguous() or entries % ancestors.shape[0] != 0,
               "AttentionByAncestors: ancestors have to be a contiguous int32 tensor [hypotheses, {}]", cap)
-    hyps = ancestors.shape[0]
     _abort_if(q.numel() != entries * dk or kNew.numel() != entries * dk or vNew.numel() != entries * dk,
               "AttentionByAncestors: one query, key and value row of {} values per cache entry", dk)
-    out = torch.empty_like(q)
-    omax = AbsMax(q.device) if want_absmax else None
-    st = be.lib.marian_hip_attention_ancestors(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), hyps,
-                                               entries // hyps, int(kvLen), cap, dk, 1.0 / float(dk) ** 0.5,
-                                               None if omax is None else omax.data_ptr(), kNew.data_ptr(),
-                                               vNew.data_ptr(), ancestors.data_ptr(), be.stream())
-    _lib.check(st, "AttentionByAncestors")
-    return (out, omax) if want_absmax else out
+    return _taken(_host.attention_ancestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax), "AttentionByAncestors")
 
 
 def advanceAncestors(prev, parents, lenPrev, out):
     """the table of ancestors of the next step: out[h, p] = prev[parents[h], p] for p < lenPrev,
     out[h, lenPrev] = h (prev, out: int32 [hypotheses, capacity], two tensors)"""
+    res = _host.ancestors_advance(prev, parents, lenPrev, out)
+    if res is not None:
+        return res
     _abort_if(prev.dtype != torch.int32 or out.dtype != torch.int32 or tuple(prev.shape) != tuple(out.shape) or
               prev.dim() != 2 or not (prev.is_contiguous() and out.is_contiguous()),
               "advanceAncestors expects two contiguous int32 tensors [hypotheses, capacity]{}", "")
-    be = _backend_of(prev)
+    _on_gpu(prev)
     par = parents.contiguous()
     if par.dtype == torch.int64:
         par = par.to(torch.int32)
     _abort_if(par.dtype not in (torch.int32, torch.uint32) or par.numel() != prev.shape[0],
               "advanceAncestors: one int32 back-pointer per hypothesis{}", "")
-    st = be.lib.marian_hip_ancestors_advance(prev.data_ptr(), par.data_ptr(), prev.shape[0], prev.shape[1], int(lenPrev),
-                                             out.data_ptr(), be.stream())
-    _lib.check(st, "advanceAncestors")
-    return out
+    return _taken(_host.ancestors_advance(prev, par, lenPrev, out), "advanceAncestors")
 
 
 def getNBestList(scores, N):
     """reference src/translator/nth_element.cpp:26-67: scores [dimBatch, 1, beam, vocab]; returns
     (pathScores, keys) of dimBatch * N entries, keys = position in the flattened tensor."""
+    out = _host.nbest(scores, N)
+    if out is not None:
+        return out
     scores = _f32c(scores, "getNBestList")
-    be = _backend_of(scores)
-    dimBatch = scores.shape[0]
-    rowLen = scores.numel() // dimBatch if dimBatch else 0
-    vals = torch.empty(dimBatch * N, dtype=torch.float32, device=scores.device)
-    keys = torch.empty(dimBatch * N, dtype=torch.int32, device=scores.device)
-    st = be.lib.marian_hip_nbest(scores.data_ptr(), dimBatch, rowLen, N, vals.data_ptr(), keys.data_ptr(),
-                                 be.stream())
-    _lib.check(st, "getNBestList")
-    return vals, keys
-
-
-# (device, stream) -> list of uint8 tensors, the last one the largest.  The reference's NthElement
-# owns its buffers too (src/translator/nth_element.cu).  A workspace holds arrival counters that
-# every call leaves at zero, so calls on one stream share it; two streams never do.  A workspace
-# that has been handed out is kept for good (a HIP graph may have recorded its address): a larger
-# call gets an additional one.
-_nbest_workspaces = {}
+    _on_gpu(scores)
+    return _taken(_host.nbest(scores, N), "getNBestList")
 
 
 def getNBestListOfBeams(scores, N):
     """reference src/translator/beam_search.cpp:472 + :492: swapAxes(expandedPathScores, 0, 2)
     followed by getNBestList, without the transposed copy.  scores [beam, 1, dimBatch, vocab] (or
     [beam, dimBatch, vocab]); returns what getNBestList returns for the transposed tensor."""
+    out = _host.nbest_beams(scores, N)
+    if out is not None:
+        return out
     scores = _f32c(scores, "getNBestListOfBeams")
-    be = _backend_of(scores)
-    beam, vocab = scores.shape[0], scores.shape[-1]
-    dimBatch = scores.numel() // (beam * vocab) if beam * vocab else 0
-    vals = torch.empty(dimBatch * N, dtype=torch.float32, device=scores.device)
-    keys = torch.empty(dimBatch * N, dtype=torch.int32, device=scores.device)
-    need = be.lib.marian_hip_nbest_beams_workspace_bytes(beam, dimBatch, vocab, N)
-    held = _nbest_workspaces.setdefault((scores.device, be.stream()), [])
-    if not held or held[-1].numel() < need:
-        ws = torch.empty(max(int(need), 4), dtype=torch.uint8, device=scores.device)
-        _lib.check(be.lib.marian_hip_nbest_beams_workspace_init(ws.data_ptr(), ws.numel(), be.stream()),
-                   "getNBestListOfBeams")
-        held.append(ws)
-    ws = held[-1]
-    st = be.lib.marian_hip_nbest_beams(scores.data_ptr(), beam, dimBatch, vocab, N, vals.data_ptr(),
-                                       keys.data_ptr(), ws.data_ptr(), ws.numel(), be.stream())
-    _lib.check(st, "getNBestListOfBeams")
-    return vals, keys
+    _on_gpu(scores)
+    return _taken(_host.nbest_beams(scores, N), "getNBestListOfBeams")
 
 
 def logsoftmaxNBestOfBeams(logits, N, pathScores=None, want_logprobs=False):
@@ -417,8 +342,11 @@ def logsoftmaxNBestOfBeams(logits, N, pathScores=None, want_logprobs=False):
     logits [beam, 1, dimBatch, vocab] (or [beam, dimBatch, vocab]); pathScores: None or one value
     per row [beam, dimBatch]; returns (vals, keys), and the log-probabilities as a third value when
     asked for.  Bit for bit what the separate calls give."""
+    out = _host.logsoftmax_nbest_beams(logits, N, pathScores, want_logprobs)
+    if out is not None:
+        return out
     logits = _f32c(logits, "logsoftmaxNBestOfBeams")
-    be = _backend_of(logits)
+    _on_gpu(logits)
     beam, vocab = logits.shape[0], logits.shape[-1]
     dimBatch = logits.numel() // (beam * vocab) if beam * vocab else 0
     if not (vocab % 4 == 0 and 4096 < vocab <= 32768 and logits.data_ptr() % 16 == 0):
@@ -428,23 +356,7 @@ def logsoftmaxNBestOfBeams(logits, N, pathScores=None, want_logprobs=False):
             (beam,) + (1,) * (logits.dim() - 3) + (dimBatch, 1))
         vals, keys = getNBestListOfBeams(scored, N)
         return (vals, keys, lp) if want_logprobs else (vals, keys)
-    add = None
     if pathScores is not None:
-        add = _f32c(pathScores, "logsoftmaxNBestOfBeams").reshape(-1)
-        _abort_if(add.numel() != beam * dimBatch, "one path score per hypothesis, got {}", add.numel())
-    vals = torch.empty(dimBatch * N, dtype=torch.float32, device=logits.device)
-    keys = torch.empty(dimBatch * N, dtype=torch.int32, device=logits.device)
-    lp = torch.empty_like(logits) if want_logprobs else None
-    need = be.lib.marian_hip_nbest_beams_workspace_bytes(beam, dimBatch, vocab, N)
-    held = _nbest_workspaces.setdefault((logits.device, be.stream()), [])
-    if not held or held[-1].numel() < need:
-        ws = torch.empty(max(int(need), 4), dtype=torch.uint8, device=logits.device)
-        _lib.check(be.lib.marian_hip_nbest_beams_workspace_init(ws.data_ptr(), ws.numel(), be.stream()),
-                   "logsoftmaxNBestOfBeams")
-        held.append(ws)
-    ws = held[-1]
-    st = be.lib.marian_hip_logsoftmax_nbest_beams(
-        logits.data_ptr(), None if add is None else add.data_ptr(), None if lp is None else lp.data_ptr(), beam,
-        dimBatch, vocab, N, vals.data_ptr(), keys.data_ptr(), ws.data_ptr(), ws.numel(), be.stream())
-    _lib.check(st, "logsoftmaxNBestOfBeams")
-    return (vals, keys, lp) if want_logprobs else (vals, keys)
+        pathScores = _f32c(pathScores, "logsoftmaxNBestOfBeams").reshape(-1)
+        _abort_if(pathScores.numel() != beam * dimBatch, "one path score per hypothesis, got {}", pathScores.numel())
+    return _taken(_host.logsoftmax_nbest_beams(logits, N, pathScores, want_logprobs), "logsoftmaxNBestOfBeams")
