@@ -14,10 +14,9 @@
  *                     (src/tensors/cpu/expression_graph_packable.h:203-235,242-250).
  * Shape rules: K % 32 == 0, N % 8 == 0.  Alignment: 16 bytes for matrices, 4 for the bias.
  *
- * gfx950 has no 16-bit integer matrix instruction; the products are taken with v_dot2_i32_i16 on
- * the vector units (two int16 products and the accumulator summed mod 2^32, which is what the
- * CPU's pmaddwd + paddd compute).  The path is exact, not fast: the 8-bit path is the one the
- * matrix cores serve.
+ * gfx950 has no 16-bit integer matrix instruction; a value is taken apart into two bytes and the
+ * products go through the 8-bit matrix instruction, four byte products for one (exact, sums mod
+ * 2^32, which is what the CPU's pmaddwd + paddd compute).
  */
 #ifndef MARIAN_HIP_INT16_H
 #define MARIAN_HIP_INT16_H
@@ -61,6 +60,16 @@ int marian_hip_int16_prepare_b_quantized_transposed(const int16_t* in, int16_t* 
  */
 int marian_hip_int16_affine(const int16_t* Aq, const int16_t* Bq, const float* bias, float* out, int64_t M,
                             int64_t K, int64_t N, float scale, int relu, void* stream);
+
+/*
+ * prepareA and the multiplication in one call on float32 activations A [M x K] (quantized on the way, as
+ * marian_hip_int16_prepare_a does it): what the operator affine / dot needs.  Aq: scratch of
+ * marian_hip_int16_scratch_bytes(M, K, N) bytes, 16-byte aligned, or null; where that is 0, or Aq null,
+ * the call is one launch and Aq is not touched.
+ */
+int marian_hip_int16_affine_f32(const float* A, int16_t* Aq, const int16_t* Bq, const float* bias, float* out, int64_t M,
+                                int64_t K, int64_t N, float scale, int relu, void* stream);
+size_t marian_hip_int16_scratch_bytes(int64_t M, int64_t K, int64_t N);
 
 /* Parity hook: the int32 accumulators (sums mod 2^32) Kernels16::Multiply hands to its callback. */
 int marian_hip_int16_multiply_i32(const int16_t* Aq, const int16_t* Bq, int32_t* acc, int64_t M, int64_t K,

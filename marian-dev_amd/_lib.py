@@ -51,6 +51,8 @@ SIGNATURES = {
     "marian_hip_int16_prepare_b": (_i, [_vp, _vp, _i64, _i64, _vp]),
     "marian_hip_int16_prepare_b_quantized_transposed": (_i, [_vp, _vp, _i64, _i64, _vp]),
     "marian_hip_int16_affine": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _f, _i, _vp]),
+    "marian_hip_int16_affine_f32": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _f, _i, _vp]),
+    "marian_hip_int16_scratch_bytes": (_sz, [_i64, _i64, _i64]),
     "marian_hip_int16_multiply_i32": (_i, [_vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     # include/marian_hip_ops.h
     "marian_hip_layer_norm": (_i, [_vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _f, _vp, _vp]),

@@ -69,30 +69,6 @@ inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_
 
 constexpr int64_t kMaxElems = 2147483647LL;
 
-constexpr int kMaxDevices = 64;
-
-// The current device, as an index into the per-device caches below.
-inline int current_device(int* dev) {
-  MH_HIP(hipGetDevice(dev));
-  if(*dev < 0 || *dev >= kMaxDevices) return MARIAN_HIP_ERR_RANGE;
-  return MARIAN_HIP_OK;
-}
-
-// Raises a kernel's dynamic LDS limit, once per kernel and device (`done`: one bit per device).
-template <typename KernelT>
-int allow_lds(KernelT kernel, int bytes, std::atomic<uint64_t>& done) {
-  if(bytes <= 48 * 1024) return MARIAN_HIP_OK;
-  int dev = 0;
-  int st = current_device(&dev);
-  if(st != MARIAN_HIP_OK) return st;
-  const uint64_t bit = 1ull << dev;
-  if(done.load(std::memory_order_acquire) & bit) return MARIAN_HIP_OK;
-  MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-  done.fetch_or(bit, std::memory_order_release);
-  return MARIAN_HIP_OK;
-}
-
 template <int MT, int NT, int WN, int KW, int PF>
 int launch_stream(const GemmArgs& a, hipStream_t st) {
   using Cfg = StreamCfg<MT, NT, WN, KW, PF>;

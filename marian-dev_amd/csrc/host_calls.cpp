@@ -37,7 +37,8 @@ namespace {
 #define MH_FUNCTIONS(F)                                                                                  \
   F(int8_workspace_bytes) F(int8_prepare_a) F(int8_prepare_b) F(int8_prepare_b_quantized_transposed)     \
   F(int8_affine_f32) F(int8_affine_f32_chained) F(int8_affine_f32_grouped) F(int8_proj_attention)        \
-  F(int16_prepare_a) F(int16_prepare_b) F(int16_prepare_b_quantized_transposed) F(int16_affine)          \
+  F(int16_prepare_a) F(int16_prepare_b) F(int16_prepare_b_quantized_transposed) F(int16_affine_f32)      \
+  F(int16_scratch_bytes)                                                                                 \
   F(layer_norm) F(embed) F(attention_cached) F(attention_ancestors) F(ancestors_advance)                 \
   F(select_state) F(nbest) F(nbest_beams) F(nbest_beams_workspace_bytes) F(nbest_beams_workspace_init)   \
   F(logsoftmax_nbest_beams)
@@ -280,18 +281,18 @@ PyObject* py_affine_or_dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int relu = truth(args[4]);
   const c10::Device d = x.a->device();
   at::Tensor out = empty(with_last(x.a->sizes(), x.n_out), at::kFloat, d);
-  const at::Tensor aq = quantized_buffer(x.M * x.K, x.b.width, d);
   const hipStream_t st = stream_of(d);
-  if(x.b.width == 2) {   // Type::intgemm16: the two nodes one after the other
-    auto* q = static_cast<int16_t*>(aq.data_ptr());
+  if(x.b.width == 2) {   // Type::intgemm16
+    at::Tensor scratch;
+    if(const size_t bytes = L.int16_scratch_bytes(x.M, x.K, x.b.cols)) scratch = empty({(int64_t)bytes}, at::kByte, d);
     call("affineOrDot", [&] {
-      const int s = L.int16_prepare_a(fptr(x.a), q, x.M, x.K, st);
-      return s != MARIAN_HIP_OK ? s
-                                : L.int16_affine(q, static_cast<const int16_t*>(x.b.t->const_data_ptr()), fptr(x.bias), fptr_mut(out),
-                                                 x.M, x.K, x.b.cols, scale, relu, st);
+      return L.int16_affine_f32(fptr(x.a), scratch.defined() ? static_cast<int16_t*>(scratch.data_ptr()) : nullptr,
+                                static_cast<const int16_t*>(x.b.t->const_data_ptr()), fptr(x.bias), fptr_mut(out), x.M, x.K, x.b.cols,
+                                scale, relu, st);
     });
     return wrap(std::move(out));
   }
+  const at::Tensor aq = quantized_buffer(x.M * x.K, x.b.width, d);
   const at::Tensor& ws = workspace(d, st);
   call("affineOrDot", [&] {
     return L.int8_affine_f32(fptr(x.a), static_cast<int8_t*>(aq.data_ptr()), static_cast<const int8_t*>(x.b.t->const_data_ptr()),

@@ -1,8 +1,10 @@
-// The 16-bit intgemm path (Type::intgemm16): quantizers, a dot2-based GEMM and its C ABI.
+// The 16-bit intgemm path (Type::intgemm16): quantizers, GEMMs on the 8-bit matrix instructions and its C ABI.
 // Declarations and the reference call sites each entry point replaces: include/marian_hip_int16.h
 #include "../../include/marian_hip_int16.h"
 
 #include <hip/hip_runtime.h>
+
+#include <atomic>
 
 #include "../../include/marian_hip_int8.h"
 #include "abi_common.h"
@@ -86,82 +88,407 @@ __global__ __launch_bounds__(256) void quantize16_b_transpose_kernel(const float
     *reinterpret_cast<float*>(out + (size_t)K * N) = kQuantMult16;
 }
 
-// C[m, n] = sum_k A[m, k] * B[n, k] over int16 operands, both K-contiguous.  A workgroup of 256
-// threads owns a 64 x 64 tile of the output and walks K in blocks of 64 values (128 bytes per row)
-// staged in LDS as packed pairs, 33 dwords per row (conflict-free for the strided reads); thread
-// (ty, tx) accumulates the 4 x 4 outputs of rows ty + 16 i, columns tx + 16 j with v_dot2_i32_i16:
-// two products and the accumulator, summed mod 2^32.
+// ---- multiplication --------------------------------------------------------------------------
+// C[m, n] = sum_k A[m, k] * B[n, k] mod 2^32 over int16 operands, both K-contiguous, on the 8-bit matrix
+// instructions.  A value is taken apart into bytes, v = 256 h + l + 128 with h = v >> 8 and l = (v & 255) - 128,
+// both in int8, so with v' = v - 128 = 256 h + l
+//     sum a b = sum a' b' + 128 (sum a + sum b) - 16384 K,
+//     sum a' b' = 65536 sum ha hb + 256 sum (ha lb + la hb) + sum la lb :
+// four 16x16x64 byte products per 64 values of k and two row sums.  Every identity holds mod 2^32, so sums
+// that leave int32 wrap as they do on the CPU.  The products with v_dot2_i32_i16 that this replaces had
+// an eighth of the rate (509 x 512 x 2048 and back: 25.2 and 79.8 us).
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+// 16 values of k of one row as two matrix operands (hi and lo bytes), and their sum
+struct Planes {
+  v4i h, l;
+  int sum;
+};
+
+__device__ __forceinline__ void split_words(unsigned d0, unsigned d1, int& h, int& l) {   // four int16 in two words
+  h = (int)__builtin_amdgcn_perm(d1, d0, 0x07050301u);
+  l = (int)(__builtin_amdgcn_perm(d1, d0, 0x06040200u) ^ 0x80808080u);
+}
+
+// The 16 values of a block of 64 k that lane group lk (0 .. 3) supplies: k = 8 lk .. 8 lk + 7 and 32 + 8 lk ..
+// 32 + 8 lk + 7 (the same for both operands, so any order does), which makes the four lanes of a row read
+// 64 contiguous bytes.  Loaded first, taken apart later, so that loads are in flight in between.  Where K ends
+// in half a block (K % 32 == 0) the second run of A is zeros and that of B a copy of other values: the identity
+// above holds for any pair, also with a = 0.
+template <typename T>
+struct Raw;
+template <>
+struct Raw<int16_t> {
+  v4u w[2];
+  __device__ __forceinline__ void load(const int16_t* p, int second) {
+    w[0] = *reinterpret_cast<const v4u*>(p);
+    w[1] = *reinterpret_cast<const v4u*>(p + second);
+  }
+  __device__ __forceinline__ void clear_second() { w[1] = v4u{0, 0, 0, 0}; }
+  __device__ __forceinline__ Planes planes() const {
+    Planes r;
+    r.sum = 0;
+    const unsigned d[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
+    int h[4], l[4];
+#pragma unroll
+    for(int i = 0; i < 4; ++i) split_words(d[2 * i], d[2 * i + 1], h[i], l[i]);
+#pragma unroll
+    for(int i = 0; i < 8; ++i) r.sum = __builtin_amdgcn_sdot2(__builtin_bit_cast(v2s, d[i]), v2s{1, 1}, r.sum, false);
+    r.h = v4i{h[0], h[1], h[2], h[3]};
+    r.l = v4i{l[0], l[1], l[2], l[3]};
+    return r;
+  }
+};
+// float32 activations, quantized on the way.  x * 1024 is exact, so one fused multiply-add with 1.5 * 2^23
+// rounds to nearest-even and leaves the integer in the low bytes of the sum, once x is clamped to int16's
+// range (med3: NaN to the lower end); products of 2^31 and more give -32768 (quantize16_one).
+template <>
+struct Raw<float> {
+  v4f w[4];
+  __device__ __forceinline__ void load(const float* p, int second) {
+    w[0] = reinterpret_cast<const v4f*>(p)[0];
+    w[1] = reinterpret_cast<const v4f*>(p)[1];
+    w[2] = reinterpret_cast<const v4f*>(p + second)[0];
+    w[3] = reinterpret_cast<const v4f*>(p + second)[1];
+  }
+  __device__ __forceinline__ void clear_second() { w[2] = w[3] = v4f{0.0f, 0.0f, 0.0f, 0.0f}; }
+  __device__ __forceinline__ Planes planes() const {
+    constexpr unsigned kMagicBits = 0x4B400000u;
+    float x[16];
+#pragma unroll
+    for(int i = 0; i < 4; ++i) { x[4 * i] = w[i].x; x[4 * i + 1] = w[i].y; x[4 * i + 2] = w[i].z; x[4 * i + 3] = w[i].w; }
+    float top = x[0];
+#pragma unroll
+    for(int i = 1; i < 16; ++i) top = fmaxf(top, x[i]);
+    if(top >= 2097152.0f) {   // (rare: x * 1024 >= 2^31)
+#pragma unroll
+      for(int i = 0; i < 16; ++i) x[i] = x[i] >= 2097152.0f ? -32.0f : x[i];
+    }
+    unsigned b[16], sum = 0;
+#pragma unroll
+    for(int i = 0; i < 16; ++i) {
+      const float c = __builtin_amdgcn_fmed3f(x[i], -32.0f, 32767.0f / 1024.0f);
+      b[i] = __float_as_uint(fmaf(c, kQuantMult16, 12582912.0f));
+      sum += b[i];
+    }
+    Planes r;
+    r.sum = (int)(sum - 16u * kMagicBits);
+    int h[4], l[4];
+#pragma unroll
+    for(int i = 0; i < 4; ++i) {
+      const unsigned p = __builtin_amdgcn_perm(b[4 * i + 1], b[4 * i], 0x05010400u);       // h1 h0 l1 l0
+      const unsigned q = __builtin_amdgcn_perm(b[4 * i + 3], b[4 * i + 2], 0x05010400u);   // h3 h2 l3 l2
+      h[i] = (int)__builtin_amdgcn_perm(q, p, 0x07060302u);
+      l[i] = (int)(__builtin_amdgcn_perm(q, p, 0x05040100u) ^ 0x80808080u);
+    }
+    r.h = v4i{h[0], h[1], h[2], h[3]};
+    r.l = v4i{l[0], l[1], l[2], l[3]};
+    return r;
+  }
+};
+// the three accumulators of one 16 x 16 tile (rows: columns of the output, see mfma_i8_16x16x64)
+struct Acc16 {
+  v4i hh, mid, ll;
+  __device__ __forceinline__ void clear() { hh = mid = ll = v4i{0, 0, 0, 0}; }
+  __device__ __forceinline__ void add(v4i bh, v4i bl, v4i ah, v4i al) {
+    hh = mfma_i8_16x16x64(bh, ah, hh);
+    mid = mfma_i8_16x16x64(bh, al, mid);
+    ll = mfma_i8_16x16x64(bl, al, ll);
+    mid = mfma_i8_16x16x64(bl, ah, mid);
+  }
+  __device__ __forceinline__ v4i sum() const {   // mod 2^32
+    v4i r;
+#pragma unroll
+    for(int e = 0; e < 4; ++e) r[e] = (int)(((unsigned)hh[e] << 16) + ((unsigned)mid[e] << 8) + (unsigned)ll[e]);
+    return r;
+  }
+};
+
+struct Gemm16Args {
+  const void* A;
+  const int16_t* Bq;
+  const float* bias;
+  void* out;
+  int M, K, N;
+  float scale;
+  int relu;
+};
+
+// four neighbouring columns n .. n + 3 of output row m: y = float(acc) * unquant (+ bias); relu: y > 0 ? y : 0;
+// multiply and add round separately
 template <bool DUMP>
-__global__ __launch_bounds__(256) void gemm16_kernel(const int16_t* __restrict__ Aq, const int16_t* __restrict__ Bq,
-                                                     const float* __restrict__ bias, void* __restrict__ out,
-                                                     int M, int K, int N, float scale, int relu) {
-  __shared__ uint32_t As[64][33], Bs[64][33];
-  const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  int acc[4][4];
+__device__ __forceinline__ void store16(const Gemm16Args& g, v4i acc, int m, int n, float unquant) {
+  if(m >= g.M || n >= g.N) return;   // (N % 8 == 0: four columns are inside or outside together)
+  const size_t off = (size_t)m * g.N + n;
+  if(DUMP) {
+    *reinterpret_cast<v4i*>(reinterpret_cast<int32_t*>(g.out) + off) = acc;
+    return;
+  }
+  v4f y;
 #pragma unroll
-  for(int i = 0; i < 4; ++i)
+  for(int e = 0; e < 4; ++e) {
+    float v = (float)acc[e] * unquant;
+    if(g.bias) v = v + g.bias[n + e];
+    if(g.relu) v = v > 0.0f ? v : 0.0f;
+    y[e] = v;
+  }
+  *reinterpret_cast<v4f*>(reinterpret_cast<float*>(g.out) + off) = y;
+}
+
+template <typename AT>
+__device__ __forceinline__ float unquant16(const Gemm16Args& g) {
+  float aqm = kQuantMult16;
+  if constexpr(sizeof(AT) == 2) aqm = *reinterpret_cast<const float*>(reinterpret_cast<const int16_t*>(g.A) + (size_t)g.M * g.K);
+  return unquant_mult(aqm, *reinterpret_cast<const float*>(g.Bq + (size_t)g.K * g.N), g.scale);
+}
+
+// Few tiles: the eight waves of a workgroup split K between them, operands go from memory straight into
+// registers (a lane takes 16 consecutive k of its row, four lanes a 128-byte line) and the partial sums meet
+// in LDS.  A workgroup makes (16 MT) x (16 NT) outputs.  Bound by what a CU can fetch: the activations of
+// 16 MT rows are read again for every 16 NT columns.
+constexpr int kStream16Waves = 8;
+template <typename AT, int MT, int NT, bool DUMP>
+__global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(Gemm16Args g) {
+  constexpr int KW = kStream16Waves, TILES = MT * NT;
+  __shared__ __attribute__((aligned(16))) int part[KW][TILES][64][4];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, lr = lane % 16, lk = lane / 16;
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const AT* arow[MT];
+  const int16_t* brow[NT];
 #pragma unroll
-    for(int j = 0; j < 4; ++j) acc[i][j] = 0;
-  // staging: 64 rows x 128 bytes per operand = 512 pieces of 16 bytes, two per thread and operand
-  const int lr = tid / 8, lc = (tid % 8) * 4;   // row (and row + 32), first dword of the piece
-  for(int kb = 0; kb < K; kb += 64) {
-    const int kv = (K - kb) >= 64 ? 64 : (K - kb);   // K % 32 == 0: a last block of 32 values
-    uint4 ra[2], rb[2];
+  for(int i = 0; i < MT; ++i) arow[i] = reinterpret_cast<const AT*>(g.A) + (size_t)min(m0 + 16 * i + lr, g.M - 1) * g.K;
 #pragma unroll
-    for(int h = 0; h < 2; ++h) {
-      const int r = lr + 32 * h;
-      const int am = min(m0 + r, M - 1), bn = min(n0 + r, N - 1);   // rows past the edge: copies, never stored
-      const bool in_k = lc * 2 < kv;
-      ra[h] = in_k ? *reinterpret_cast<const uint4*>(Aq + (size_t)am * K + kb + lc * 2) : uint4{0, 0, 0, 0};
-      rb[h] = in_k ? *reinterpret_cast<const uint4*>(Bq + (size_t)bn * K + kb + lc * 2) : uint4{0, 0, 0, 0};
+  for(int j = 0; j < NT; ++j) brow[j] = g.Bq + (size_t)min(n0 + 16 * j + lr, g.N - 1) * g.K;
+  Acc16 acc[MT][NT];
+  int asum[MT], bsum[NT], taken = 0;
+#pragma unroll
+  for(int i = 0; i < MT; ++i) {
+    asum[i] = 0;
+#pragma unroll
+    for(int j = 0; j < NT; ++j) acc[i][j].clear();
+  }
+#pragma unroll
+  for(int j = 0; j < NT; ++j) bsum[j] = 0;
+  const int S = (g.K + 63) / 64;
+  const bool half = g.K % 64 != 0;
+  Raw<AT> ra[MT];
+  Raw<int16_t> rb[NT];
+  auto load = [&](int s) __attribute__((always_inline)) {
+    const int k = s * 64 + lk * 8, second = half && s == S - 1 ? 0 : 32;
+#pragma unroll
+    for(int j = 0; j < NT; ++j) rb[j].load(brow[j] + k, second);
+#pragma unroll
+    for(int i = 0; i < MT; ++i) ra[i].load(arow[i] + k, second);
+  };
+  // one step: its operands are taken apart, the next step's loads take their place, then the products
+  auto step = [&](int s, bool more) __attribute__((always_inline)) {
+    Planes a[MT], b[NT];
+    if(!more && half && s == S - 1) {
+#pragma unroll
+      for(int i = 0; i < MT; ++i) ra[i].clear_second();
     }
-    __syncthreads();   // the previous block has been read
 #pragma unroll
-    for(int h = 0; h < 2; ++h) {
-      const int r = lr + 32 * h;
-      As[r][lc] = ra[h].x; As[r][lc + 1] = ra[h].y; As[r][lc + 2] = ra[h].z; As[r][lc + 3] = ra[h].w;
-      Bs[r][lc] = rb[h].x; Bs[r][lc + 1] = rb[h].y; Bs[r][lc + 2] = rb[h].z; Bs[r][lc + 3] = rb[h].w;
+    for(int j = 0; j < NT; ++j) b[j] = rb[j].planes();
+#pragma unroll
+    for(int i = 0; i < MT; ++i) a[i] = ra[i].planes();
+    if(more) load(s + KW);
+#pragma unroll
+    for(int i = 0; i < MT; ++i) {
+      asum[i] += a[i].sum;
+#pragma unroll
+      for(int j = 0; j < NT; ++j) acc[i][j].add(b[j].h, b[j].l, a[i].h, a[i].l);
     }
-    __syncthreads();
-#pragma unroll 8
-    for(int kk = 0; kk < 32; ++kk) {
-      uint32_t a[4], b[4];
 #pragma unroll
-      for(int i = 0; i < 4; ++i) a[i] = As[ty + 16 * i][kk];
+    for(int j = 0; j < NT; ++j) bsum[j] += b[j].sum;
+    taken += 64;
+  };
+  int s = wave;
+  if(s < S) {
+    load(s);
+    // (the load of the next step stands behind no branch: the compiler would wait for it at once)
+    for(; s + KW < S; s += KW) step(s, true);
+    step(s, false);
+  }
+  // row sums over the four lane groups; lane (lr, lk) holds outputs row lr, columns 4 lk .. 4 lk + 3
 #pragma unroll
-      for(int j = 0; j < 4; ++j) b[j] = Bs[tx + 16 * j][kk];
+  for(int i = 0; i < MT; ++i) {
+    asum[i] += __shfl_xor(asum[i], 16);
+    asum[i] += __shfl_xor(asum[i], 32);
+  }
 #pragma unroll
-      for(int i = 0; i < 4; ++i)
+  for(int j = 0; j < NT; ++j) {
+    bsum[j] += __shfl_xor(bsum[j], 16);
+    bsum[j] += __shfl_xor(bsum[j], 32);
+    int bs[4];
 #pragma unroll
-        for(int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_sdot2(__builtin_bit_cast(v2s, a[i]), __builtin_bit_cast(v2s, b[j]), acc[i][j], false);
+    for(int e = 0; e < 4; ++e) bs[e] = __shfl(bsum[j], 4 * lk + e);
+#pragma unroll
+    for(int i = 0; i < MT; ++i) {
+      v4i t = acc[i][j].sum();
+#pragma unroll
+      for(int e = 0; e < 4; ++e) t[e] = (int)((unsigned)t[e] + 128u * (unsigned)(asum[i] + bs[e]) - 16384u * (unsigned)taken);
+      *reinterpret_cast<v4i*>(part[wave][i * NT + j][lane]) = t;
     }
   }
   float unquant = 0.0f;
-  if(!DUMP) {
-    const float aqm = *reinterpret_cast<const float*>(Aq + (size_t)M * K);
-    const float bqm = *reinterpret_cast<const float*>(Bq + (size_t)K * N);
-    unquant = unquant_mult(aqm, bqm, scale);
+  if(!DUMP) unquant = unquant16<AT>(g);
+  __syncthreads();
+  for(int t = threadIdx.x; t < TILES * 64; t += 64 * KW) {
+    const int tile = t / 64, l = t % 64;
+    v4i sum = *reinterpret_cast<const v4i*>(part[0][tile][l]);
+#pragma unroll
+    for(int w = 1; w < KW; ++w) {
+      const v4i p = *reinterpret_cast<const v4i*>(part[w][tile][l]);
+#pragma unroll
+      for(int e = 0; e < 4; ++e) sum[e] = (int)((unsigned)sum[e] + (unsigned)p[e]);
+    }
+    store16<DUMP>(g, sum, m0 + 16 * (tile / NT) + l % 16, n0 + 16 * (tile % NT) + 4 * (l / 16), unquant);
+  }
+}
+
+// Many tiles: a workgroup of eight waves makes a BM x BN tile, both operands of a block of 64 k go through
+// registers (taken apart there, once per workgroup) into LDS, two blocks in turn: while one is multiplied the
+// next is on its way.  LDS rows are 64 bytes,
+// their four pieces permuted by the row number so that reads of neighbouring rows fall on different banks.
+constexpr int kPitch16 = 64, kTile16Depth = 2;
+__device__ __forceinline__ int piece16(int row, int c) { return (c ^ ((row >> 1) & 3)) * 16; }
+template <int BM, int BN>
+constexpr int tile16_lds() { return 2 * 2 * (BM + BN) * kPitch16; }
+template <typename AT, int BM, int BN, int WM, int WN, bool DUMP>
+__global__ __launch_bounds__(64 * WM * WN) void gemm16_tile_kernel(Gemm16Args g, int tiles_n) {
+  constexpr int T = 64 * WM * WN, FM = BM / WM / 16, FN = BN / WN / 16;
+  constexpr int UA = BM * 4 / T, UB = BN * 4 / T;   // pieces of 16 k a thread stages per block
+  static_assert(UA * T == BM * 4 && UB * T == BN * 4 && (T / 4) % 8 == 0, "whole pieces per thread");
+  extern __shared__ __attribute__((aligned(16))) int8_t lds16[];
+  int* const sums = reinterpret_cast<int*>(lds16);   // [BM + BN], at the end
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, lr = lane % 16, lk = lane / 16;
+  const int wm = wave / WN, wn = wave % WN;
+  const int m0 = (int)(blockIdx.x / tiles_n) * BM, n0 = (int)(blockIdx.x % tiles_n) * BN;
+  const int srow = tid / 4, sk = (tid % 4) * 8, spiece = piece16(srow, tid % 4);   // staging: four threads a row, T / 4 rows at a time
+  const AT* asrc[UA];
+  const int16_t* bsrc[UB];
+#pragma unroll
+  for(int u = 0; u < UA; ++u) asrc[u] = reinterpret_cast<const AT*>(g.A) + (size_t)min(m0 + srow + u * (T / 4), g.M - 1) * g.K;
+#pragma unroll
+  for(int u = 0; u < UB; ++u) bsrc[u] = g.Bq + (size_t)min(n0 + srow + u * (T / 4), g.N - 1) * g.K;
+  constexpr int D = kTile16Depth;   // blocks of K on their way
+  Raw<AT> ra[D][UA];
+  Raw<int16_t> rb[D][UB];
+  int asum[UA], bsum[UB];
+#pragma unroll
+  for(int u = 0; u < UA; ++u) asum[u] = 0;
+#pragma unroll
+  for(int u = 0; u < UB; ++u) bsum[u] = 0;
+  Acc16 acc[FM][FN];
+#pragma unroll
+  for(int i = 0; i < FM; ++i)
+#pragma unroll
+    for(int j = 0; j < FN; ++j) acc[i][j].clear();
+  const int blocks = (g.K + 63) / 64;
+  const bool half = g.K % 64 != 0;
+  auto load = [&](int kb, Raw<AT> (&ra)[UA], Raw<int16_t> (&rb)[UB]) __attribute__((always_inline)) {
+    kb = min(kb, blocks - 1);
+    const int k = kb * 64 + sk, second = half && kb == blocks - 1 ? 0 : 32;
+#pragma unroll
+    for(int u = 0; u < UA; ++u) ra[u].load(asrc[u] + k, second);
+#pragma unroll
+    for(int u = 0; u < UB; ++u) rb[u].load(bsrc[u] + k, second);
+  };
+  // planes of stage t: A hi, A lo, B hi, B lo
+  auto plane = [&](int t, int which, int row) {
+    return lds16 + (size_t)t * (2 * (BM + BN) * kPitch16) + (which < 2 ? which * BM : 2 * BM + (which - 2) * BN) * kPitch16 + row * kPitch16;
+  };
+  auto stage = [&](int t, int kb, Raw<AT> (&ra)[UA], Raw<int16_t> (&rb)[UB]) __attribute__((always_inline)) {
+    if(half && kb == blocks - 1) {   // (the same for the whole workgroup)
+#pragma unroll
+      for(int u = 0; u < UA; ++u) ra[u].clear_second();
+    }
+#pragma unroll
+    for(int u = 0; u < UA; ++u) {
+      const Planes p = ra[u].planes();
+      asum[u] += p.sum;
+      *reinterpret_cast<v4i*>(plane(t, 0, srow + u * (T / 4)) + spiece) = p.h;
+      *reinterpret_cast<v4i*>(plane(t, 1, srow + u * (T / 4)) + spiece) = p.l;
+    }
+#pragma unroll
+    for(int u = 0; u < UB; ++u) {
+      const Planes p = rb[u].planes();
+      bsum[u] += p.sum;
+      *reinterpret_cast<v4i*>(plane(t, 2, srow + u * (T / 4)) + spiece) = p.h;
+      *reinterpret_cast<v4i*>(plane(t, 3, srow + u * (T / 4)) + spiece) = p.l;
+    }
+  };
+  auto multiply = [&](int t) __attribute__((always_inline)) {
+    v4i bh[FN], bl[FN];
+#pragma unroll
+    for(int j = 0; j < FN; ++j) {
+      const int row = (wn * FN + j) * 16 + lr;
+      bh[j] = *reinterpret_cast<const v4i*>(plane(t, 2, row) + piece16(row, lk));
+      bl[j] = *reinterpret_cast<const v4i*>(plane(t, 3, row) + piece16(row, lk));
+    }
+#pragma unroll
+    for(int i = 0; i < FM; ++i) {
+      const int row = (wm * FM + i) * 16 + lr;
+      const v4i ah = *reinterpret_cast<const v4i*>(plane(t, 0, row) + piece16(row, lk));
+      const v4i al = *reinterpret_cast<const v4i*>(plane(t, 1, row) + piece16(row, lk));
+#pragma unroll
+      for(int j = 0; j < FN; ++j) acc[i][j].add(bh[j], bl[j], ah, al);
+    }
+  };
+#pragma unroll
+  for(int d = 0; d < D; ++d) load(d, ra[d], rb[d]);
+  stage(0, 0, ra[0], rb[0]);
+  load(D, ra[0], rb[0]);
+  __syncthreads();
+  int kb = 0;
+  // (the loads inside the loop stand behind no branch: the compiler would wait for them at once)
+  for(; kb + 2 * D < blocks; kb += D) {
+#pragma unroll
+    for(int d = 0; d < D; ++d) {
+      const int t = (kb + d) & 1, next = (d + 1) % D;
+      multiply(t);
+      stage(t ^ 1, kb + d + 1, ra[next], rb[next]);   // (the other stage was read before the last barrier)
+      load(kb + d + 1 + D, ra[next], rb[next]);
+      __syncthreads();
+    }
   }
 #pragma unroll
-  for(int i = 0; i < 4; ++i) {
-    const int m = m0 + ty + 16 * i;
-    if(m >= M) continue;
+  for(int d = 0; d < 2 * D; ++d) {
+    if(kb + d < blocks) {   // (the same for the whole workgroup)
+      const int t = (kb + d) & 1, next = (d + 1) % D;
+      multiply(t);
+      if(kb + d + 1 < blocks) stage(t ^ 1, kb + d + 1, ra[next], rb[next]);
+      if(d + 1 < D && kb + d + 1 + D < blocks) load(kb + d + 1 + D, ra[next], rb[next]);
+      __syncthreads();
+    }
+  }
+  // row sums: the four threads of a row sit side by side
 #pragma unroll
-    for(int j = 0; j < 4; ++j) {
-      const int n = n0 + tx + 16 * j;
-      if(n >= N) continue;
-      const size_t off = (size_t)m * N + n;
-      if(DUMP) {
-        reinterpret_cast<int32_t*>(out)[off] = acc[i][j];
-      } else {
-        // y = float(acc) * unquant (+ bias); relu: y > 0 ? y : 0; multiply and add round separately
-        float y = (float)acc[i][j] * unquant;
-        if(bias) y = y + bias[n];
-        if(relu) y = y > 0.0f ? y : 0.0f;
-        reinterpret_cast<float*>(out)[off] = y;
-      }
+  for(int u = 0; u < UA; ++u) {
+    asum[u] += __shfl_xor(asum[u], 1);
+    asum[u] += __shfl_xor(asum[u], 2);
+    if(tid % 4 == 0) sums[srow + u * (T / 4)] = asum[u];
+  }
+#pragma unroll
+  for(int u = 0; u < UB; ++u) {
+    bsum[u] += __shfl_xor(bsum[u], 1);
+    bsum[u] += __shfl_xor(bsum[u], 2);
+    if(tid % 4 == 0) sums[BM + srow + u * (T / 4)] = bsum[u];
+  }
+  float unquant = 0.0f;
+  if(!DUMP) unquant = unquant16<AT>(g);
+  __syncthreads();
+#pragma unroll
+  for(int i = 0; i < FM; ++i) {
+    const int r = (wm * FM + i) * 16 + lr;
+    const int as = sums[r];
+#pragma unroll
+    for(int j = 0; j < FN; ++j) {
+      const int c = (wn * FN + j) * 16 + 4 * lk;
+      v4i v = acc[i][j].sum();
+#pragma unroll
+      for(int e = 0; e < 4; ++e) v[e] = (int)((unsigned)v[e] + 128u * (unsigned)(as + sums[BM + c + e]) - 16384u * 64u * (unsigned)blocks);
+      store16<DUMP>(g, v, m0 + r, n0 + c, unquant);
     }
   }
 }
@@ -175,18 +502,75 @@ int check16(const void* Aq, const void* Bq, const void* out, const float* bias, 
   return MARIAN_HIP_OK;
 }
 
-template <bool DUMP>
-int run16(const int16_t* Aq, const int16_t* Bq, const float* bias, void* out, int64_t M, int64_t K, int64_t N,
-          float scale, int relu, void* stream) {
-  int st = check16(Aq, Bq, out, bias, M, K, N);
-  if(st != MARIAN_HIP_OK) return st;
-  if(M == 0 || N == 0) return MARIAN_HIP_OK;
-  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-  if(grid.y > 65535) return MARIAN_HIP_ERR_RANGE;
-  hipLaunchKernelGGL(gemm16_kernel<DUMP>, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), Aq, Bq, bias, out,
-                     (int)M, (int)K, (int)N, scale, relu ? 1 : 0);
+template <typename AT, int MT, int NT, bool DUMP>
+int launch_stream16(const Gemm16Args& g, hipStream_t st) {
+  const dim3 grid((unsigned)((g.N + 16 * NT - 1) / (16 * NT)), (unsigned)((g.M + 16 * MT - 1) / (16 * MT)));
+  hipLaunchKernelGGL((gemm16_stream_kernel<AT, MT, NT, DUMP>), grid, dim3(64 * kStream16Waves), 0, st, g);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
+}
+
+template <typename AT, int BM, int BN, int WM, int WN, bool DUMP>
+int launch_tile16(const Gemm16Args& g, hipStream_t st) {
+  const int tiles_n = (g.N + BN - 1) / BN, tiles_m = (g.M + BM - 1) / BM;
+  constexpr int lds = tile16_lds<BM, BN>();
+  auto kernel = gemm16_tile_kernel<AT, BM, BN, WM, WN, DUMP>;
+  static std::atomic<uint64_t> lds_done{0};
+  const int lds_status = allow_lds(kernel, lds, lds_done);
+  if(lds_status != MARIAN_HIP_OK) return lds_status;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(64 * WM * WN), lds, st, g, tiles_n);
+  MH_HIP(hipGetLastError());
+  return MARIAN_HIP_OK;
+}
+
+// Which form a call takes.  Per step of k a workgroup loads, converts and multiplies its rows of both operands,
+// about 30 ps a byte (measured, M = 1 .. 4096, whatever the form), so a form costs its workgroups per CU (at
+// least one) times the bytes a workgroup takes in for each k; the 128 x 128 tiles are half again as dear (one
+// workgroup to a CU: products, conversion and LDS traffic overlap less).  Over 25 sizes the form chosen
+// was never more than a tenth behind the best one.  us, int16 activations, in a graph:
+//   1 x 512 x 512 3.1 (stream 16 x 16), 64 x 512 x 2048 4.4 (16 x 32), 509 x 2048 x 512 10.4 (32 x 32), 509 x 512 x 2048
+//   8.7 (64 x 64), 4096 x 4096 x 4096 257 (128 x 128: 535 TOPS of 16-bit products).
+struct Form16 {
+  enum Name { kStream4, kStream8, kStream16, kStream16x32, kStream32x32, kTile64, kTile128 };
+  Name form;
+  double cost;   // bytes per k through the busiest CU
+};
+inline Form16 plan16(int M, int N, int a_bytes) {
+  struct Shape { Form16::Name form; int rows, cols; double factor; };
+  constexpr Shape shapes[] = {{Form16::kStream16, 16, 16, 1.0}, {Form16::kStream16x32, 16, 32, 1.0}, {Form16::kStream32x32, 32, 32, 1.0}, {Form16::kTile64, 64, 64, 1.0},
+                              {Form16::kTile128, 128, 128, 1.5}};
+  Form16 best{Form16::kTile128, 1e30};
+  for(const Shape& s : shapes) {
+    if(s.form < Form16::kTile64 && (M + s.rows - 1) / s.rows > 65535) continue;   // (row tiles are the grid's second dimension)
+    const double workgroups = (double)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols) / 256.0;
+    const double cost = (workgroups > 1.0 ? workgroups : 1.0) * s.factor * (s.rows * a_bytes + s.cols * 2);
+    if(cost < best.cost) best = Form16{s.form, cost};
+  }
+  return best;
+}
+
+// Whether float32 activations are quantized by a launch of their own first: where the bytes that the multiplication
+// then saves take longer than the launch and its pass over memory (3 us and 6 bytes a value at 4 TB/s).
+inline bool quantize_first16(int64_t M, int64_t K, int64_t N) {
+  const double saved = (plan16((int)M, (int)N, 4).cost - plan16((int)M, (int)N, 2).cost) * (double)K * 0.03;   // ns
+  return saved > 3000.0 + (double)M * (double)K * 0.0015;
+}
+
+template <typename AT, bool DUMP>
+int run16(const AT* A, const int16_t* Bq, const float* bias, void* out, int64_t M, int64_t K, int64_t N,
+          float scale, int relu, void* stream) {
+  int status = check16(A, Bq, out, bias, M, K, N);
+  if(status != MARIAN_HIP_OK) return status;
+  if(M == 0 || N == 0) return MARIAN_HIP_OK;
+  Gemm16Args g{A, Bq, bias, out, (int)M, (int)K, (int)N, scale, relu ? 1 : 0};
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  switch(plan16((int)M, (int)N, (int)sizeof(AT)).form) {
+    case Form16::kStream16: return launch_stream16<AT, 1, 1, DUMP>(g, st);
+    case Form16::kStream16x32: return launch_stream16<AT, 1, 2, DUMP>(g, st);
+    case Form16::kStream32x32: return launch_stream16<AT, 2, 2, DUMP>(g, st);
+    case Form16::kTile64: return launch_tile16<AT, 64, 64, 2, 2, DUMP>(g, st);
+    default: return launch_tile16<AT, 128, 128, 2, 4, DUMP>(g, st);
+  }
 }
 
 }  // namespace
@@ -235,12 +619,29 @@ int marian_hip_int16_prepare_b_quantized_transposed(const int16_t* in, int16_t* 
 
 int marian_hip_int16_affine(const int16_t* Aq, const int16_t* Bq, const float* bias, float* out, int64_t M, int64_t K,
                             int64_t N, float scale, int relu, void* stream) {
-  return run16<false>(Aq, Bq, bias, out, M, K, N, scale, relu, stream);
+  return run16<int16_t, false>(Aq, Bq, bias, out, M, K, N, scale, relu, stream);
 }
 
 int marian_hip_int16_multiply_i32(const int16_t* Aq, const int16_t* Bq, int32_t* acc, int64_t M, int64_t K, int64_t N,
                                   void* stream) {
-  return run16<true>(Aq, Bq, nullptr, acc, M, K, N, 1.0f, 0, stream);
+  return run16<int16_t, true>(Aq, Bq, nullptr, acc, M, K, N, 1.0f, 0, stream);
+}
+
+size_t marian_hip_int16_scratch_bytes(int64_t M, int64_t K, int64_t N) {
+  if(M <= 0 || K <= 0 || N <= 0 || M * K > kMaxElems16) return 0;
+  return quantize_first16(M, K, N) ? 2 * (size_t)M * (size_t)K + sizeof(float) : 0;
+}
+
+int marian_hip_int16_affine_f32(const float* A, int16_t* Aq, const int16_t* Bq, const float* bias, float* out, int64_t M, int64_t K,
+                                int64_t N, float scale, int relu, void* stream) {
+  if(Aq && M > 0 && N > 0 && marian_hip_int16_scratch_bytes(M, K, N)) {
+    const int status = check16(A, Bq, out, bias, M, K, N);   // (nothing is launched for a call that is refused)
+    if(status != MARIAN_HIP_OK) return status;
+    const int quantized = marian_hip_int16_prepare_a(A, Aq, M, K, stream);
+    if(quantized != MARIAN_HIP_OK) return quantized;
+    return marian_hip_int16_affine(Aq, Bq, bias, out, M, K, N, scale, relu, stream);
+  }
+  return run16<float, false>(A, Bq, bias, out, M, K, N, scale, relu, stream);
 }
 
 }  // extern "C"

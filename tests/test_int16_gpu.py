@@ -108,6 +108,32 @@ def test_multiply16_wraps_like_the_cpu(integer, o16):
     assert np.array_equal(integer.multiply_i32(Aq, Bq).cpu().numpy(), o16.multiply_i32(Aq_h, Bq_h, M, K, N))
 
 
+# one size or more for every form of the multiplication (16 x 16, 16 x 32 and 32 x 32 outputs by waves that split
+# K; 64 x 64 and 128 x 128 tiles), remainders in every dimension, and activations quantized by a launch of their own
+@pytest.mark.parametrize("M,K,N", [(1, 32, 8), (17, 544, 40), (70, 96, 1048), (257, 1056, 520), (500, 160, 2056),
+                                   (1801, 96, 1800), (700, 4128, 520)])
+def test_affine16_from_float_extremes(integer, o16, synth, M, K, N):
+    """float32 activations with values at and past the ends of int16, NaN and infinities, quantized on the way into
+    the multiplication: bit for bit what prepareA and multiply give on the CPU (whole sums mod 2^32, then two roundings)"""
+    T = load("types")
+    say("affine16 from float32", M, K, N)
+    rng = np.random.default_rng(M + N)
+    A = synth.normal(200 + M, synth.STREAM_A, (M, K), 12.0)
+    special = np.array([np.nan, np.inf, -np.inf, 3e38, -3e38, 2097152.0, 2097151.9, 32.0, -32.0, 31.9995, 1.5 / 1024, -2.5 / 1024], f32)
+    A.flat[rng.integers(0, A.size, 60)] = special[np.arange(60) % special.size]
+    A[-1, -special.size:] = special
+    Bt = rng.integers(-32768, 32768, (N, K), dtype=np.int16)
+    Bt[0, :], Bt[-1, :] = -32768, 32767
+    Bq_h = np.concatenate([Bt.ravel(), np.frombuffer(f32(1024.0).tobytes(), np.int16)])
+    bias = synth.normal(200 + N, synth.STREAM_BIAS, (N,), 1.0)
+    Bq = integer.QTensor.from_numpy(qbytes(Bq_h), (K, N), T.Type.intgemm16, "cuda")
+    Aq_h = o16.prepare_a(A)
+    want, want_acc = o16.affine(Aq_h, Bq_h, bias, M, K, N, 1.0, False)
+    assert np.array_equal(integer.affine(dev(A), Bq, dev(bias)).cpu().numpy(), want)
+    Aq = integer.QTensor.from_numpy(qbytes(Aq_h), (M, K), T.Type.intgemm16, "cuda")
+    assert np.array_equal(integer.multiply_i32(Aq, Bq).cpu().numpy(), want_acc)
+
+
 def test_marian_operator_vectors_through_the_16_bit_path(integer, o16):
     """reference src/tests/units/operator_tests.cpp:618-659 padded to the shape rules (K = 32,
     N = 8): small integers are exact at a multiplier of 1024."""
