@@ -82,10 +82,9 @@ int marian_hip_bdot_legacy(const float* A, const float* B, float* C, int64_t bat
  *   q: [batchQ, m, dk], k and v: [batchKV, len, dk] (entry i uses k, v of i % batchKV: encoder
  *   keys shared by the beam), out: [batchQ, m, dk]; mask as in marian_hip_softmax for score rows
  *   [batchQ * m, len], or NULL.  len <= 4096.
- *   Built for decoding steps (m = 1 or a few query positions per head): every query row gets a
- *   wave that walks the head's keys and values itself.  With eight or more positions per head
- *   (encoder layers) the three separate entry points, which share a head's keys and values
- *   through LDS tiles, are about twice as fast; the host mirror switches over by itself.
+ *   Built for decoding steps (m = 1): every query row gets a wave that walks the head's keys and
+ *   values itself.  For several positions per head (encoder layers) with dk == 64 there is
+ *   marian_hip_attention_rows; the host mirror switches over by itself.
  *   Where several query rows share a cache entry (batchKV < batchQ, m == 1, dk == 64, len <= 96,
  *   16-byte aligned tensors, no k_new) the rows of an entry are taken by one workgroup, which
  *   reads the entry's keys and values once: same bits, 28 instead of 50 us for 512 rows x 16 heads
@@ -101,6 +100,28 @@ int marian_hip_attention(const float* q, float* k, float* v, const float* mask, 
                          int64_t rows_per_mask, float* out, int64_t batchQ, int64_t batchKV,
                          int64_t m, int64_t len, int64_t dk, float scale, float* absmax_out,
                          const float* k_new, const float* v_new, void* stream);
+
+/*
+ * The same attention on heads that may lie side by side in a row, and for several query positions per head
+ * (encoder layers, whole target sentences): q, k, v and out are [batch, heads, positions, dk] with the floats
+ * between two sentences, heads and positions given (three strides each, multiples of four; 16-byte aligned
+ * tensors), so that the output of an affine call is read as it is and SplitHeads / JoinHeads
+ * (src/models/transformer.h:145-170) move nothing.  batchQ, batchKV: entries, sentences times heads; entry i
+ * uses keys and values of entry i % batchKV.  mask as in marian_hip_softmax for score rows [batchQ * m, len], or
+ * NULL.  absmax_out: as for marian_hip_layer_norm (needs batchQ * m <= 2048, or ceil(m / 16) for m where blocks
+ * of rows are taken).
+ *   m >= MARIAN_HIP_ATTENTION_ROWS_MIN: blocks of query rows share keys and values; dk == 64 and len <=
+ *   MARIAN_HIP_ATTENTION_ROWS_MAX_LEN (other sizes: MARIAN_HIP_ERR_SHAPE); bit for bit what
+ *   marian_hip_bdot_legacy, marian_hip_softmax and marian_hip_bdot_legacy give.
+ *   fewer rows: bit for bit marian_hip_attention; len <= 4096.
+ */
+#define MARIAN_HIP_ATTENTION_ROWS_MIN 8
+#define MARIAN_HIP_ATTENTION_ROWS_MAX_LEN 256
+int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const float* k, const int64_t* k_strides,
+                              const float* v, const int64_t* v_strides, const float* mask, int64_t n_masks,
+                              int64_t rows_per_mask, float* out, const int64_t* out_strides, int64_t batchQ,
+                              int64_t batchKV, int64_t heads, int64_t m, int64_t len, int64_t dk, float scale,
+                              float* absmax_out, void* stream);
 
 /*
  * marian_hip_attention on caches that have room to grow: k and v are [batchKV, kv_capacity, dk]

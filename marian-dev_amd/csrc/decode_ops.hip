@@ -15,6 +15,7 @@
 
 #include "../../include/marian_hip_int8.h"
 #include "abi_common.h"
+#include "attention_rows_kernel.h"
 #include "int8_common.h"
 #include "nbest_plan.h"
 #include "quantize_common.h"
@@ -534,7 +535,11 @@ __global__ __launch_bounds__(256) void bdot_tile_kernel(const float* __restrict_
 // of a beam search stay where they were written and the table of ancestors says whose row a
 // position of a hypothesis's history is; the newest position comes from k_new / v_new and goes into
 // the hypothesis's own entry.
-template <bool ANC>
+// STRIDED (no k_new): q, k, v and out have the strides of `hs` instead of lying head by head.
+struct AttentionStrides {
+  HeadStrides q, k, v, out;
+};
+template <bool ANC, bool STRIDED>
 __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict__ Q, float* Kt, float* V,
                                                         const float* __restrict__ k_new,
                                                         const float* __restrict__ v_new,
@@ -543,7 +548,7 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
                                                         float* __restrict__ out, unsigned rows_total,
                                                         unsigned batchKV, int m, int len, int kv_cap, int dk,
                                                         float scale, float* __restrict__ absmax_out,
-                                                        const uint32_t* __restrict__ anc, unsigned heads) {
+                                                        const uint32_t* __restrict__ anc, unsigned heads, AttentionStrides hs) {
   // kv_cap: positions a cache entry has room for (its stride, in rows of dk values); len of them are in use
   // (row counts are below 2^31, checked by the launcher: 32-bit divisions, a tenth of the
   // instructions of 64-bit ones, and this kernel is a chain of short phases)
@@ -561,9 +566,11 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
   // (no division in the usual cases: one position per entry, as many cache entries as entries)
   const unsigned i = m == 1 ? wr : wr / (unsigned)m;
   const unsigned entry = i < batchKV ? i : i % batchKV;
-  const float* q = Q + (size_t)wr * dk;
-  float* kb = Kt + (size_t)entry * kv_cap * dk;
-  float* vb = V + (size_t)entry * kv_cap * dk;
+  const size_t k_row = STRIDED ? (size_t)hs.k.row : (size_t)dk, v_row = STRIDED ? (size_t)hs.v.row : (size_t)dk;
+  const float* q = STRIDED ? Q + hs.q.entry(i, heads) + (size_t)(wr - i * (unsigned)m) * hs.q.row : Q + (size_t)wr * dk;
+  float* kb = Kt + (STRIDED ? hs.k.entry(entry, heads) : (size_t)entry * kv_cap * dk);
+  float* vb = V + (STRIDED ? hs.v.entry(entry, heads) : (size_t)entry * kv_cap * dk);
+  float* y = out + (STRIDED ? hs.out.entry(i, heads) + (size_t)(wr - i * (unsigned)m) * hs.out.row : (size_t)wr * dk);
   // Newest position (m == 1, one wave per cache entry): its key and value rows go into the cache
   // for the following steps; this step reads them from k_new / v_new directly.  Up to 64 values per
   // row they are requested here and stored at the end of the kernel (nothing in this call waits
@@ -580,8 +587,8 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
       vb[(size_t)(len - 1) * dk + d] = v_new[(size_t)wr * dk + d];
     }
   }
-  const float* k_last = k_new ? k_new + (size_t)wr * dk : kb + (size_t)(len - 1) * dk;
-  const float* v_last = v_new ? v_new + (size_t)wr * dk : vb + (size_t)(len - 1) * dk;
+  const float* k_last = k_new ? k_new + (size_t)wr * dk : kb + (size_t)(len - 1) * k_row;
+  const float* v_last = v_new ? v_new + (size_t)wr * dk : vb + (size_t)(len - 1) * v_row;
   unsigned mask_row = 0;
   if(mask) {
     mask_row = rows_per_mask == 1 ? wr : wr / rows_per_mask;
@@ -609,14 +616,14 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
   // floats behind the lane's first row; from group u_last on the lane's position is the last one
   // or past it, and it reads the last row (given separately: it may not be in the cache yet).
   const int u_last = (len + 2 - g) / 4;   // = ceil((len - 1 - g) / 4)
-  auto load_rows = [&](const float* rows, const float* last, int base, v4f (&r)[kAttU]) __attribute__((always_inline)) {
-    const float* first = rows + (size_t)g * dk + 4 * c;
+  auto load_rows = [&](const float* rows, size_t row, const float* last, int base, v4f (&r)[kAttU]) __attribute__((always_inline)) {
+    const float* first = rows + (size_t)g * row + 4 * c;
     const float* last_c = last + 4 * c;
 #pragma unroll
     for(int u = 0; u < kAttU; ++u) {
       if(base + 4 * u < len) {   // (the same for the whole wave)
         const int U = base / 4 + u;
-        const float* p = U >= u_last ? last_c : first + (size_t)U * 4 * dk;
+        const float* p = U >= u_last ? last_c : first + (size_t)U * 4 * row;
         r[u] = *reinterpret_cast<const v4f*>(p);
       } else if(base + 4 * (u & ~3) < len) {   // (read with its group of sixteen positions below)
         r[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -653,11 +660,11 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
   };
   auto load_k = [&](int base, v4f (&r)[kAttU]) __attribute__((always_inline)) {
     if(ANC) load_rows_anc(Kt, k_last, base, r);
-    else load_rows(kb, k_last, base, r);
+    else load_rows(kb, k_row, k_last, base, r);
   };
   auto load_v = [&](int base, v4f (&r)[kAttU]) __attribute__((always_inline)) {
     if(ANC) load_rows_anc(V, v_last, base, r);
-    else load_rows(vb, v_last, base, r);
+    else load_rows(vb, v_row, v_last, base, r);
   };
   if(fast) {
     float mk0 = 0.0f;
@@ -708,7 +715,7 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
   }
   for(int pos = lane; pos < len && !fast; pos += 64) {
     float s = 0.0f;
-    const float* krow = pos == len - 1 ? k_last : kb + (size_t)pos * dk;
+    const float* krow = pos == len - 1 ? k_last : kb + (size_t)pos * k_row;
     if(vec && dk == 64) {   // the usual head size: all sixteen loads of the key row in flight at once
       const v4f* ar = reinterpret_cast<const v4f*>(q);
       const v4f* br = reinterpret_cast<const v4f*>(krow);
@@ -780,7 +787,7 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
     }
     reinterpret_cast<v4f*>(part)[g * 16 + c] = o4;   // partial sums of the positions g, g + 4, ...
     const float o = ((part[lane] + part[64 + lane]) + part[128 + lane]) + part[192 + lane];
-    out[(size_t)wr * dk + lane] = o;
+    y[lane] = o;
     omax = fabsf(o);
   }
   for(int d = lane; d < dk && !fast; d += 64) {
@@ -789,12 +796,12 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
     for(; pos + 8 <= len; pos += 8) {   // eight value loads in flight, same summation order
       float vr[8];
 #pragma unroll
-      for(int u = 0; u < 8; ++u) vr[u] = pos + u == len - 1 ? v_last[d] : vb[(size_t)(pos + u) * dk + d];
+      for(int u = 0; u < 8; ++u) vr[u] = pos + u == len - 1 ? v_last[d] : vb[(size_t)(pos + u) * v_row + d];
 #pragma unroll
       for(int u = 0; u < 8; ++u) o = fmaf(sc[pos + u], vr[u], o);
     }
-    for(; pos < len; ++pos) o = fmaf(sc[pos], pos == len - 1 ? v_last[d] : vb[(size_t)pos * dk + d], o);
-    out[(size_t)wr * dk + d] = 1.0f * o;
+    for(; pos < len; ++pos) o = fmaf(sc[pos], pos == len - 1 ? v_last[d] : vb[(size_t)pos * v_row + d], o);
+    y[d] = 1.0f * o;
     omax = fmaxf(omax, fabsf(1.0f * o));
   }
   if(absmax_out) {   // slot = query row
@@ -2105,6 +2112,65 @@ int marian_hip_attention(const float* q, float* k, float* v, const float* mask, 
                                      scale, absmax_out, k_new, v_new, stream);
 }
 
+int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const float* k, const int64_t* k_strides,
+                              const float* v, const int64_t* v_strides, const float* mask, int64_t n_masks,
+                              int64_t rows_per_mask, float* out, const int64_t* out_strides, int64_t batchQ,
+                              int64_t batchKV, int64_t heads, int64_t m, int64_t len, int64_t dk, float scale,
+                              float* absmax_out, void* stream) {
+  if(batchQ < 0 || batchKV <= 0 || heads <= 0 || m <= 0 || len <= 0 || dk <= 0) return MARIAN_HIP_ERR_SHAPE;
+  if(mask && (n_masks <= 0 || rows_per_mask <= 0)) return MARIAN_HIP_ERR_SHAPE;
+  const bool blocks = dk == 64 && m >= MARIAN_HIP_ATTENTION_ROWS_MIN && len <= MARIAN_HIP_ATTENTION_ROWS_MAX_LEN;
+  if(!blocks && m >= MARIAN_HIP_ATTENTION_ROWS_MIN) return MARIAN_HIP_ERR_SHAPE;
+  if(!q_strides || !k_strides || !v_strides || !out_strides) return MARIAN_HIP_ERR_NULL;
+  if(batchQ == 0) return MARIAN_HIP_OK;
+  if(!q || !k || !v || !out) return MARIAN_HIP_ERR_NULL;
+  if(mask && (n_masks > 2147483647LL || rows_per_mask > 2147483647LL)) return MARIAN_HIP_ERR_RANGE;
+  if(heads > kMaxElemsOps || dk > kMaxElemsOps || m > kMaxElemsOps / dk || len > 4096 || batchQ > kMaxElemsOps / (m * dk) ||
+     batchKV > kMaxElemsOps / (len * dk))
+    return MARIAN_HIP_ERR_RANGE;
+  AttentionStrides hs;
+  HeadStrides* const to[4] = {&hs.q, &hs.k, &hs.v, &hs.out};
+  const int64_t* const given[4] = {q_strides, k_strides, v_strides, out_strides};
+  for(int i = 0; i < 4; ++i) {
+    for(int j = 0; j < 3; ++j)
+      if(given[i][j] < 0 || given[i][j] % 4 != 0) return MARIAN_HIP_ERR_ALIGN;
+    *to[i] = HeadStrides{given[i][0], given[i][1], given[i][2]};
+  }
+  if(!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || (mask && !aligned4(mask)) || (absmax_out && !aligned4(absmax_out)))
+    return MARIAN_HIP_ERR_ALIGN;
+  if(!mask) { n_masks = 1; rows_per_mask = 1; }
+  hipStream_t hst = reinterpret_cast<hipStream_t>(stream);
+  if(!blocks) {   // (a wave per query row)
+    if(absmax_out && batchQ * m > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
+    static std::atomic<uint64_t> lds_done{0};
+    const int lds_status = allow_lds(attention_kernel<false, true>, 72 * 1024, lds_done);
+    if(lds_status != MARIAN_HIP_OK) return lds_status;
+    const size_t lds = (size_t)4 * (size_t)(((len + 3) & ~(int64_t)3) + 256) * sizeof(float);
+    hipLaunchKernelGGL((attention_kernel<false, true>), dim3((unsigned)((batchQ * m + 3) / 4)), dim3(256), lds, hst, q, const_cast<float*>(k),
+                       const_cast<float*>(v), nullptr, nullptr, mask, (unsigned)n_masks, (unsigned)rows_per_mask, out, (unsigned)(batchQ * m),
+                       (unsigned)batchKV, (int)m, (int)len, (int)len, (int)dk, scale, absmax_out, nullptr, (unsigned)heads, hs);
+    MH_HIP(hipGetLastError());
+    return MARIAN_HIP_OK;
+  }
+  // Thirty-two query rows a wave read every key and value half as often as sixteen, and keep the chip busy from
+  // one wave per SIMD on (1024 of them); beyond 128 keys their scores do not fit the registers.
+  const int R = len <= 128 && batchQ * ((m + 31) / 32) >= 1024 ? 2 : 1;
+  if(absmax_out && batchQ * ((m + 16 * R - 1) / (16 * R)) > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
+  AttentionRowsArgs a{q, k, v, mask, out, absmax_out, hs.q, hs.k, hs.v, hs.out, (unsigned)batchQ, (unsigned)batchKV, (unsigned)heads,
+                      (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)((m + 16 * R - 1) / (16 * R)), scale};
+  const dim3 grid((unsigned)((batchQ * a.row_blocks + 3) / 4));
+  const int nb = (int)((len + 63) / 64);
+#define MH_ROWS(R, NB) hipLaunchKernelGGL((attention_rows_kernel<R, NB>), grid, dim3(256), 0, hst, a)
+  if(R == 2) { if(nb == 1) MH_ROWS(2, 1); else MH_ROWS(2, 2); }
+  else if(nb == 1) MH_ROWS(1, 1);
+  else if(nb == 2) MH_ROWS(1, 2);
+  else if(nb == 3) MH_ROWS(1, 3);
+  else MH_ROWS(1, 4);
+#undef MH_ROWS
+  MH_HIP(hipGetLastError());
+  return MARIAN_HIP_OK;
+}
+
 static int attention_impl(const float* q, float* k, float* v, const float* mask, int64_t n_masks,
                           int64_t rows_per_mask, float* out, int64_t batchQ, int64_t batchKV, int64_t m,
                           int64_t len, int64_t kv_capacity, int64_t dk, float scale, float* absmax_out,
@@ -2196,9 +2262,9 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
     MH_HIP(hipGetDevice(&dev));
     if(dev < 0 || dev >= 64) return MARIAN_HIP_ERR_RANGE;
     if(!(lds_done.load(std::memory_order_acquire) & (1ull << dev))) {
-      MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<false>),
+      MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<false, false>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024));
-      MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<true>),
+      MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(attention_kernel<true, false>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024));
       lds_done.fetch_or(1ull << dev, std::memory_order_release);
     }
@@ -2222,15 +2288,15 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
     return MARIAN_HIP_OK;
   }
   if(ancestors)
-    hipLaunchKernelGGL(attention_kernel<true>, dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
+    hipLaunchKernelGGL((attention_kernel<true, false>), dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
                        k_new, v_new, mask, (unsigned)n_masks, (unsigned)rows_per_mask, out, (unsigned)rows_total,
                        (unsigned)batchKV, (int)m, (int)len, (int)kv_capacity, (int)dk, scale, absmax_out, ancestors,
-                       (unsigned)heads);
+                       (unsigned)heads, AttentionStrides());
   else
-    hipLaunchKernelGGL(attention_kernel<false>, dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
+    hipLaunchKernelGGL((attention_kernel<false, false>), dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
                        k_new, v_new, mask, (unsigned)n_masks, (unsigned)rows_per_mask, out, (unsigned)rows_total,
                        (unsigned)batchKV, (int)m, (int)len, (int)kv_capacity, (int)dk, scale, absmax_out, ancestors,
-                       1u);
+                       1u, AttentionStrides());
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }

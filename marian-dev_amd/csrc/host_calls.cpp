@@ -19,6 +19,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/as_strided_native.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 
@@ -39,7 +40,7 @@ namespace {
   F(int8_affine_f32) F(int8_affine_f32_chained) F(int8_affine_f32_grouped) F(int8_proj_attention)        \
   F(int16_prepare_a) F(int16_prepare_b) F(int16_prepare_b_quantized_transposed) F(int16_affine_f32)      \
   F(int16_scratch_bytes)                                                                                 \
-  F(layer_norm) F(embed) F(attention_cached) F(attention_ancestors) F(ancestors_advance)                 \
+  F(layer_norm) F(embed) F(attention_cached) F(attention_rows) F(attention_ancestors) F(ancestors_advance)                 \
   F(select_state) F(nbest) F(nbest_beams) F(nbest_beams_workspace_bytes) F(nbest_beams_workspace_init)   \
   F(logsoftmax_nbest_beams)
 
@@ -557,6 +558,95 @@ PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_END
 }
 
+// ---- heads --------------------------------------------------------------------------------------
+// split_heads(x [beam, batch, steps, model], heads) -> [batch * beam, heads, steps, model / heads], the same memory
+PyObject* py_split_heads(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(2, "split_heads");
+  const at::Tensor* x = f32c(args[0]);
+  const int64_t heads = whole(args[1]);
+  if(!x || x->dim() != 4 || heads <= 0 || x->size(3) % heads != 0) Py_RETURN_NONE;
+  const int64_t entries = x->size(0) * x->size(1), steps = x->size(2), model = x->size(3), depth = model / heads;
+  const int64_t size[4] = {entries, heads, steps, depth};
+  const int64_t stride[4] = {steps * model, steps == 1 ? depth : (heads == 1 ? steps * depth : depth), steps == 1 ? depth : model, 1};
+  return wrap(at::native::as_strided_tensorimpl(*x, size, stride, x->storage_offset()));
+  MH_END
+}
+
+// join_heads(x [batch * beam, heads, steps, depth], beam) -> [beam, batch, steps, heads * depth] where x lies in
+// memory as that tensor does; None otherwise
+PyObject* py_join_heads(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(2, "join_heads");
+  const at::Tensor* x = tensor(args[0]);
+  const int64_t beam = whole(args[1]);
+  if(!x || x->scalar_type() != at::kFloat || !x->is_cuda() || x->dim() != 4 || beam <= 0 || x->size(0) % beam != 0) Py_RETURN_NONE;
+  const int64_t entries = x->size(0), heads = x->size(1), steps = x->size(2), depth = x->size(3), model = heads * depth;
+  if(x->numel() == 0 || x->stride(3) != 1 || (heads > 1 && x->stride(1) != depth) || (steps > 1 && x->stride(2) != model) ||
+     (entries > 1 && x->stride(0) != steps * model))
+    Py_RETURN_NONE;
+  const int64_t size[4] = {beam, entries / beam, steps, model};
+  const int64_t stride[4] = {entries / beam * steps * model, steps * model, model, 1};
+  return wrap(at::native::as_strided_tensorimpl(*x, size, stride, x->storage_offset()));
+  MH_END
+}
+
+// The strides of t as [batch, heads, positions, dk]; false when it has none, or when they are not multiples of
+// sixteen bytes.
+bool head_strides(const at::Tensor& t, int64_t heads, int64_t (&st)[3]) {
+  if(reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 != 0) return false;
+  if(t.is_contiguous()) {   // (heads one behind the other, however they are counted)
+    st[2] = t.size(-1);
+    st[1] = t.size(-2) * st[2];
+    st[0] = heads * st[1];
+  } else {
+    if(t.dim() != 4 || t.size(1) != heads || t.stride(3) != 1) return false;
+    for(int i = 0; i < 3; ++i) st[i] = t.stride(i);
+  }
+  return st[0] >= 0 && st[1] >= 0 && st[2] >= 0 && (st[0] | st[1] | st[2]) % 4 == 0;
+}
+
+// attention_rows(q, k, v, mask, rowsPerMask, kvLen, want_absmax) -> out or (out, absmax): several positions per
+// head, or tensors that are not contiguous.  out lies in memory as q does: head by head, or the heads of a
+// position side by side.
+PyObject* py_attention_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(7, "attention_rows");
+  const at::Tensor *q = tensor(args[0]), *k = tensor(args[1]), *v = tensor(args[2]), *mask;
+  int64_t heads = 1;   // of the tensors that are not contiguous
+  for(const at::Tensor* t : {q, k, v}) {
+    if(!t || t->scalar_type() != at::kFloat || !t->is_cuda() || t->dim() < 3 || t->dim() > 4 || t->numel() == 0) Py_RETURN_NONE;
+    if(t->dim() == 4 && !t->is_contiguous()) heads = t->size(1);
+  }
+  if(k->sizes() != v->sizes() || !f32c_or_none(args[3], &mask)) Py_RETURN_NONE;
+  const int64_t dk = q->size(-1), m = q->size(-2), cap = k->size(-2), len = none(args[5]) ? cap : whole(args[5]), entries = q->numel() / (m * dk);
+  if(k->size(-1) != dk || len <= 0 || len > cap || (mask && mask->numel() % len != 0)) Py_RETURN_NONE;
+  const bool blocks = m >= MARIAN_HIP_ATTENTION_ROWS_MIN, want = truth(args[6]);
+  if(blocks && (dk != 64 || len > MARIAN_HIP_ATTENTION_ROWS_MAX_LEN)) Py_RETURN_NONE;
+  if(want && entries * (blocks ? (m + 15) / 16 : m) > MARIAN_HIP_ABSMAX_SLOTS) Py_RETURN_NONE;
+  const int64_t per = whole(args[4]);
+  int64_t qs[3], ks[3], vs[3], os[3];
+  if(!head_strides(*q, heads, qs) || !head_strides(*k, heads, ks) || !head_strides(*v, heads, vs)) Py_RETURN_NONE;
+  const c10::Device d = q->device();
+  at::Tensor out, omax;
+  if(q->is_contiguous()) {
+    out = empty(q->sizes(), at::kFloat, d);
+    head_strides(out, heads, os);
+  } else {
+    os[0] = m * heads * dk;
+    os[1] = dk;
+    os[2] = heads * dk;
+    const int64_t stride[4] = {os[0], os[1], os[2], 1};
+    out = at::Tensor(at::detail::empty_strided_cuda(q->sizes(), stride, at::kFloat, d));
+  }
+  if(want) omax = absmax_slots(d);
+  const hipStream_t st = stream_of(d);
+  call("Attention", [&] {
+    return L.attention_rows(fptr(q), qs, fptr(k), ks, fptr(v), vs, fptr(mask), mask ? mask->numel() / len : 0, per, fptr_mut(out), os,
+                            entries, k->numel() / (cap * dk), heads, m, len, dk, (float)(1.0 / std::pow((double)dk, 0.5)),
+                            want ? fptr_mut(omax) : nullptr, st);
+  });
+  return with_absmax(std::move(out), std::move(omax));
+  MH_END
+}
+
 // proj_attention(x, weights, k, v, heads, kvLen, mask, absmax, want_absmax, want_projections)
 //   -> (out, aQuant[, absmax][, projections])
 PyObject* py_proj_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -757,7 +847,7 @@ PyObject* py_setup(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyMethodDef methods[] = {
     MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
     MH_METHOD(affine_f32_grouped), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
-    MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors),
+    MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(attention_rows), MH_METHOD(split_heads), MH_METHOD(join_heads), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors),
     MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),
     {nullptr, nullptr, 0, nullptr}};
 

@@ -22,6 +22,10 @@ from .integer import _abort_if, _backend_of, _host, _on_gpu, _taken
 
 def _f32c(x, what):
     _abort_if(x.dtype != torch.float32, "{} expects float32, got {}", what, x.dtype)
+    if not x.is_contiguous() and x.dim() == 4 and x.device.type == "cuda":
+        t = x.transpose(1, 2)   # SplitHeads' view of rows: its copy head by head is the 0213 transpose
+        if t.is_contiguous():
+            return transpose0213(t)
     return x.contiguous()
 
 
@@ -160,13 +164,21 @@ def transpose0213(a):
 
 def SplitHeads(input, dimHeads):
     """reference src/models/transformer.h:145-156: [beam, batch, steps, model] ->
-    [batch * beam, heads, steps, depth]"""
+    [batch * beam, heads, steps, depth].  The result is a view (the heads of a position side by side, as
+    the affine call wrote them): Attention reads it as it is, and what needs it head by head copies."""
+    out = _host.split_heads(input, dimHeads)
+    if out is not None:
+        return out
     dimBeam, dimBatch, dimSteps, dimModel = input.shape
     return transpose0213(input.reshape(dimBatch * dimBeam, dimSteps, dimHeads, dimModel // dimHeads))
 
 
 def JoinHeads(input, dimBeam=1):
-    """reference src/models/transformer.h:158-170"""
+    """reference src/models/transformer.h:158-170; a view where the heads of a position lie side by side (the
+    output of Attention on SplitHeads' views)"""
+    out = _host.join_heads(input, dimBeam)
+    if out is not None:
+        return out
     dimBatchBeam, dimHeads, dimSteps, dimDepth = input.shape
     out = transpose0213(input)
     return out.reshape(dimBeam, dimBatchBeam // dimBeam, dimSteps, dimHeads * dimDepth)
@@ -203,6 +215,10 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     kvLen: k and v have room for k.shape[-2] positions per entry, of which the first kvLen are in
     use (caches that stay in place from step to step); None: all of them."""
     m = q.shape[-2]
+    if kNew is None and (m >= 8 or not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous())):
+        out = _host.attention_rows(q, k, v, mask, rowsPerMask, kvLen, want_absmax)
+        if out is not None:
+            return out
     if m < 8 or kNew is not None or want_absmax or kvLen is not None:
         out = _host.attention(q, k, v, mask, rowsPerMask, want_absmax, kNew, vNew, kvLen)
         if out is not None:
@@ -210,8 +226,13 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     q = _f32c(q, "Attention")
     _abort_if(k.dtype != torch.float32 or v.dtype != torch.float32, "Attention expects float32, got {}", k.dtype)
     if kNew is None:
-        k, v = k.contiguous(), v.contiguous()
+        k, v = _f32c(k, "Attention"), _f32c(v, "Attention")
     else:
+        if not k.is_contiguous() and k.dim() == 4 and k.transpose(1, 2).is_contiguous():   # SplitHeads' view as a cache
+            kc, vc = _f32c(k, "Attention"), _f32c(v, "Attention")
+            out = Attention(q, kc, vc, mask, rowsPerMask, want_absmax, kNew, vNew, kvLen)
+            k.copy_(kc), v.copy_(vc)
+            return out
         _abort_if(not (k.is_contiguous() and v.is_contiguous()), "Attention: the key/value cache must be contiguous{}", "")
         kNew, vNew = _f32c(kNew, "Attention"), _f32c(vNew, "Attention")
     _on_gpu(q)
@@ -221,9 +242,9 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     _abort_if(k.shape[-1] != dk or tuple(v.shape) != tuple(k.shape), "Attention: key/value shapes {} {} vs dk {}",
               tuple(k.shape), tuple(v.shape), dk)
     if m >= 8 and kNew is None and not want_absmax and L == cap:
-        # Many query positions per head (encoder layers, whole target sentences): the one-launch
-        # form gives every query row a wave that walks the head's keys and values on its own; the
-        # three operators share them through LDS tiles (1024 heads of 64 x 64 x 64: 57 us against 105).
+        # Many query positions per head and another head size, or more than 256 keys: the three operators share a head's keys
+        # and values through LDS tiles; the one-launch form gives every query row a wave that walks
+        # them on its own.
         batchQ, batchKV = q.numel() // (m * dk), k.numel() // (cap * dk)
         scores = bdot_legacy(q.reshape(batchQ, m, dk), k.reshape(batchKV, L, dk), False, True, 1.0 / float(dk) ** 0.5)
         weights = softmax(scores, mask, rowsPerMask)
@@ -255,6 +276,13 @@ def ProjectedAttention(x, weights, k, v, heads, kvLen=None, mask=None, absmax=No
     n = len(weights)
     _abort_if(n not in (1, 3), "ProjectedAttention: one projection (q) or three (q, k, v), got {}", n)
     K, N = x.shape[-1], heads * 64
+    if n == 1 and not (k.is_contiguous() and v.is_contiguous()) and k.dim() == 4:
+        # the encoder's keys and values as SplitHeads' views: the two calls, which read them as they are
+        (bQuant, bias), = weights
+        q, aq = integer.affine_f32(x, bQuant, bias, absmax=absmax)
+        o = Attention(q.reshape(-1, 1, 64), k, v, mask, rowsPerMask=heads, want_absmax=want_absmax, kvLen=kvLen)
+        o, omax = o if want_absmax else (o, None)
+        return (o.reshape(q.shape), aq) + ((omax,) if want_absmax else ()) + (([q],) if want_projections else ())
     _abort_if(not (k.is_contiguous() and v.is_contiguous()) or k.dtype != torch.float32 or v.dtype != torch.float32,
               "ProjectedAttention: the key/value caches must be contiguous float32{}", "")
     _abort_if(k.shape[-1] != 64 or tuple(k.shape) != tuple(v.shape), "ProjectedAttention: head size 64, got caches {} {}",

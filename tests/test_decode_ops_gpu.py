@@ -352,6 +352,51 @@ def test_attention_with_many_query_positions(ops, synth, BQ, BKV, m, L, dk, mask
     close(got, want, 4 * REL, 2e-5)
 
 
+@pytest.mark.parametrize("beam,batch,heads,m,L", [(1, 1, 2, 2, 3), (2, 3, 4, 16, 16), (1, 2, 8, 17, 64), (1, 5, 1, 33, 65),
+                                                  (3, 2, 2, 40, 192), (1, 65, 16, 33, 40), (1, 36, 16, 41, 127), (1, 2, 3, 9, 255),
+                                                  (2, 1, 2, 23, 256), (2, 2, 4, 1, 70), (1, 3, 2, 5, 300), (1, 2, 2, 8, 257)])
+@pytest.mark.parametrize("how", ["views", "heads apart", "mask per row", "all masked"])
+def test_attention_on_heads_side_by_side(ops, synth, beam, batch, heads, m, L, how):
+    """SplitHeads' views read as they are (and the same call on copies): blocks of 16 and 32 query rows and of 64
+    keys with their remainders, keys shared by the beam, an -inf mask over whole blocks, a mask for every row.
+    Against the float64 closed form; from 8 rows on also bit for bit what the three operators give."""
+    import torch
+    D, E = heads * 64, beam * batch
+    q = synth.normal(m + L, 0, (1, E, m, D), 1.0)
+    k = synth.normal(m + L, 1, (1, batch, L, D), 1.0)
+    v = synth.normal(m + L, 2, (1, batch, L, D), 1.0)
+    qh, kh, vh = (ops.SplitHeads(dev(t), heads) for t in (q, k, v))
+    rpm, mask = heads * m, np.zeros((batch, L), np.float32)
+    mask[:, max(1, L // 3):] = -np.inf
+    if how == "mask per row":
+        rpm, mask = 1, np.where(synth.normal(m, 5, (E * heads * m, L), 1.0) > 0.5, -99999999.0, 0.0).astype(np.float32)
+        mask[:, L // 2] = 0.0
+    if how == "all masked":
+        mask[0] = -np.inf
+    if how == "heads apart":
+        qh, kh, vh = qh.contiguous(), kh.contiguous(), vh.contiguous()
+    small = E * heads * ((m + 15) // 16) <= 2048 and L <= 256
+    o = ops.Attention(qh, kh, vh, dev(mask), rpm, want_absmax=small)
+    o, omax = o if small else (o, None)
+    assert o.shape == qh.shape
+    got = ops.JoinHeads(o).cpu().numpy().reshape(E, m, heads, 64).transpose(0, 2, 1, 3)
+    split = lambda t: t[0].reshape(t.shape[1], -1, heads, 64).transpose(0, 2, 1, 3).astype(f64)
+    z = np.einsum("bhmd,bhld->bhml", split(q), split(k)[np.arange(E) % batch]) / 8.0
+    rows = (np.arange(E * heads * m) // rpm) % mask.shape[0]
+    z = z + mask.astype(f64)[rows].reshape(E, heads, m, L)
+    with np.errstate(invalid="ignore"):
+        w = np.exp(z - z.max(-1, keepdims=True))
+        want = np.einsum("bhml,bhld->bhmd", w / w.sum(-1, keepdims=True), split(v)[np.arange(E) % batch])
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    close(np.nan_to_num(got), np.nan_to_num(want), 4 * REL, 2e-5)
+    if m >= 8:
+        heads_apart = [t.contiguous().reshape(-1, t.shape[2], 64) for t in (qh, kh, vh)]
+        scores = ops.softmax(ops.bdot_legacy(heads_apart[0], heads_apart[1], False, True, 0.125), dev(mask), rpm)
+        assert np.array_equal(got, ops.bdot_legacy(scores, heads_apart[2]).cpu().numpy().reshape(got.shape), equal_nan=True)
+    if small and not np.isnan(got).any():
+        assert float(omax.data.max()) == float(o.abs().max())
+
+
 def _random_attention_cases(n):
     rng = np.random.default_rng(20261130)
     cases = []
