@@ -108,8 +108,7 @@ int marian_hip_attention(const float* q, float* k, float* v, const float* mask, 
  * tensors), so that the output of an affine call is read as it is and SplitHeads / JoinHeads
  * (src/models/transformer.h:145-170) move nothing.  batchQ, batchKV: entries, sentences times heads; entry i
  * uses keys and values of entry i % batchKV.  mask as in marian_hip_softmax for score rows [batchQ * m, len], or
- * NULL.  absmax_out: as for marian_hip_layer_norm (needs batchQ * m <= 2048, or ceil(m / 16) for m where blocks
- * of rows are taken).
+ * NULL.  absmax_out: as for marian_hip_layer_norm (needs batchQ * m <= 2048).
  *   m >= MARIAN_HIP_ATTENTION_ROWS_MIN: blocks of query rows share keys and values; dk == 64 and len <=
  *   MARIAN_HIP_ATTENTION_ROWS_MAX_LEN (other sizes: MARIAN_HIP_ERR_SHAPE); bit for bit what
  *   marian_hip_bdot_legacy, marian_hip_softmax and marian_hip_bdot_legacy give.

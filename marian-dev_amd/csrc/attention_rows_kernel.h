@@ -20,7 +20,7 @@ struct AttentionRowsArgs {
   float* absmax_out;   // kAbsmaxSlots values whose maximum is max|out| (a slot per wave), or null
   HeadStrides qs, ks, vs, os;
   unsigned batchQ, batchKV, heads, n_masks, rows_per_mask;
-  int m, len, row_blocks;
+  int m, len, row_blocks, row_groups;   // blocks of 16 query rows, and over how many workgroups a head's are dealt out
   float scale;
 };
 
@@ -47,195 +47,182 @@ __device__ __forceinline__ v4f rows_to_registers(v4f m) {
   return v4f{__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(r[2]), __uint_as_float(r[3])};
 }
 
-// A wave makes 16 R query rows of one head over len <= 64 NB keys; waves share nothing, so there is no LDS and no
-// barrier.  Scores come as S^T = K Q^T: lane (c = lane % 16, g = lane / 16) then holds, for query row c, the scores of
-// keys 16 t + 4 g + r (t, r = 0 .. 3) of each block of 64, so a row's maximum and sum need two lane exchanges, and
-// O^T = V^T P^T takes the weights as its second operand, transposed within four lanes.  Every load is sixteen
-// bytes a lane and a wave's lanes cover whole lines: four dimensions of key or query row c (transposed within
-// four lanes as well), four of value row 16 t + 4 r + g.
+// A workgroup of four waves takes one head and every row_groups-th block of 16 query rows, len <= 64 NB keys.
+// Wave w multiplies keys 16 w .. 16 w + 15 of each block of 64 and makes outputs 16 w .. 16 w + 15, so that its share of
+// keys and values (16 NB registers each) is read once for all rows; the scores' maxima, the sums and the weights
+// (4 NB KB) change hands in LDS.
+// Scores come as S^T = K Q^T: lane (c = lane % 16, g = lane / 16) holds, for query row c, the scores of keys 16 w +
+// 4 g + r (r = 0 .. 3) of each block, so a row's maximum and sum need two lane exchanges within the wave, and
+// O^T = V^T P^T takes the weights of row c as its second operand.  Rows of K are loaded four dimensions a lane, whole
+// lines a wave, and transposed within four lanes; rows of Q once for the four waves, through LDS.
 // The results are those of bdot_legacy, softmax and bdot_legacy bit for bit: the matrix instruction adds its four
 // products to the accumulator in order of k, each with one rounding, exactly as a chain of fmaf does (checked
 // over normal and denormal numbers), so with k-steps in ascending order every product sums as bdot_kernel sums;
 // exponentials, their sum (elements 64 apart first, then the tree of wave_sum) and the division are
 // softmax_kernel's.  A rounding that moves here moves an 8-bit quantization further down the network.
-// Bound by the float32 matrix rate (16 x 16 x 4 in 32 clocks: 1024 heads of 64 x 64 take 6.8 us at 2.4 GHz) and, with
-// R = 1, by the loads (keys and values again for every sixteen rows).  The three operators it replaces took 59 us
-// there, and the transpositions to and from heads 32 us.
-template <int R, int NB>
-__global__ __launch_bounds__(256, 2) void attention_rows_kernel(AttentionRowsArgs p) {
-  const unsigned w = blockIdx.x * 4u + threadIdx.x / 64u;
+// Bound by its chains for a few heads, by the float32 matrix rate (16 x 16 x 4 in 32 clocks: 1024 heads of 64 x 64 take
+// 6.8 us at 2.4 GHz) and the traffic (67 MB there) for many.
+// Measured (in a graph, masks included): 8 heads of 23 x 23 4.1 us, 128 of 64 x 64 6.2, 1024 of 64 x 64 23.1, 384 of 128 x 128
+// 29.5.  Before, 1024 heads took three operators of 59 us and four transpositions of 32 us, one sentence 8.7 us with
+// a wave to 16 rows and all keys (no LDS, the same bits).
+template <int NB>
+__global__ __launch_bounds__(256, NB == 1 ? 4 : (NB == 2 ? 3 : 2)) void attention_rows_kernel(AttentionRowsArgs p) {
+  constexpr int kPitch = 64 * NB + 4;   // floats of a weight row
+  __shared__ float top_lds[2][4][16], sum_lds[2][4][16];
+  __shared__ __attribute__((aligned(16))) float weight_lds[2][16][kPitch];
+  __shared__ __attribute__((aligned(16))) float q_lds[2][16][64 + 4];   // d = 16 s + 4 x + y of a row at 16 s + 4 y + x
+  const unsigned entry = blockIdx.x / (unsigned)p.row_groups;
+  const int group = (int)(blockIdx.x % (unsigned)p.row_groups);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, c = lane % 16, g = lane / 16;
   if(p.absmax_out && blockIdx.x == 0)   // slots past the last wave
-    for(unsigned sl = p.batchQ * (unsigned)p.row_blocks + threadIdx.x; sl < (unsigned)kAbsmaxSlots; sl += 256) p.absmax_out[sl] = 0.0f;
-  const unsigned entry = w / (unsigned)p.row_blocks;
-  if(entry >= p.batchQ) return;   // (whole waves)
-  const int row0 = (int)(w % (unsigned)p.row_blocks) * (16 * R);
-  const int lane = threadIdx.x % 64, c = lane % 16, g = lane / 16;
+    for(unsigned sl = gridDim.x * 4u + threadIdx.x; sl < (unsigned)kAbsmaxSlots; sl += 256) p.absmax_out[sl] = 0.0f;
   const unsigned ekv = entry < p.batchKV ? entry : entry % p.batchKV;
-  const float* kb = p.k + p.ks.entry(ekv, p.heads) + 4 * g;
-  const float* vb = p.v + p.vs.entry(ekv, p.heads) + 4 * c;
-  const float* qb = p.q + p.qs.entry(entry, p.heads) + 4 * g;
+  // (offsets within a tensor fit 32 bits: checked by the launcher)
+  const float* kb = p.k + p.ks.entry(ekv, p.heads);
+  const float* vb = p.v + p.vs.entry(ekv, p.heads);
+  const float* qb = p.q + p.qs.entry(entry, p.heads);
+  float* ob = p.out + p.os.entry(entry, p.heads);
+  const int k_row = (int)p.ks.row, v_row = (int)p.vs.row, q_row = (int)p.qs.row, o_row = (int)p.os.row;
 
-  v4f q[R][4];
-  const float* mask[R];
+  v4f k[NB][4], q_next;
+  float v[NB][4][4], mask_next[NB][4];
+  // a block of query rows: sixteen bytes a thread; and the mask values of this lane's scores
+  const int q_in = threadIdx.x / 16, q_at = threadIdx.x % 16;
+  auto load_q = [&](int block) __attribute__((always_inline)) {   // (rows past the end: the last one again, not stored)
+    q_next = *reinterpret_cast<const v4f*>(qb + min(block * 16 + q_in, p.m - 1) * q_row + 4 * q_at);
+    if(p.mask) {
+      unsigned mr = (entry * (unsigned)p.m + (unsigned)min(block * 16 + c, p.m - 1)) / p.rows_per_mask;
+      if(mr >= p.n_masks) mr %= p.n_masks;
+      const float* m = p.mask + (size_t)mr * p.len;
 #pragma unroll
-  for(int rt = 0; rt < R; ++rt) {
-    const int row = min(row0 + 16 * rt + c, p.m - 1);   // (rows past the end: the last one again, not stored)
+      for(int b = 0; b < NB; ++b)
 #pragma unroll
-    for(int s = 0; s < 4; ++s) q[rt][s] = *reinterpret_cast<const v4f*>(qb + (size_t)row * p.qs.row + 16 * s);
-    unsigned mr = (entry * (unsigned)p.m + (unsigned)row) / p.rows_per_mask;
-    if(mr >= p.n_masks) mr %= p.n_masks;
-    mask[rt] = p.mask ? p.mask + (size_t)mr * p.len : nullptr;
-  }
-  v4f k[4][4], v[4][4], z[R][NB][4];
-  auto load_k = [&](int b) __attribute__((always_inline)) {
-#pragma unroll
-    for(int t = 0; t < 4; ++t) {
-      const float* src = kb + (size_t)min(64 * b + 16 * t + c, p.len - 1) * p.ks.row;
-#pragma unroll
-      for(int s = 0; s < 4; ++s) k[t][s] = *reinterpret_cast<const v4f*>(src + 16 * s);
+        for(int r = 0; r < 4; ++r) mask_next[b][r] = m[min(64 * b + 16 * wave + 4 * g + r, p.len - 1)];
     }
   };
-  auto load_v = [&](int b) __attribute__((always_inline)) {
+  auto keep_q = [&](int turn) __attribute__((always_inline)) {
 #pragma unroll
-    for(int t = 0; t < 4; ++t)
-#pragma unroll
-      for(int r = 0; r < 4; ++r) v[t][r] = *reinterpret_cast<const v4f*>(vb + (size_t)min(64 * b + 16 * t + 4 * r + g, p.len - 1) * p.vs.row);
+    for(int y = 0; y < 4; ++y) q_lds[turn][q_in][16 * (q_at / 4) + 4 * y + q_at % 4] = q_next[y];
   };
-  load_k(0);
-#pragma unroll
-  for(int rt = 0; rt < R; ++rt)
-#pragma unroll
-    for(int s = 0; s < 4; ++s) q[rt][s] = rows_to_registers(q[rt][s]);
-
-  // ---- scores ----
+  load_q(group);
 #pragma unroll
   for(int b = 0; b < NB; ++b) {
+    const float* src = kb + min(64 * b + 16 * wave + c, p.len - 1) * k_row + 4 * g;
 #pragma unroll
-    for(int rt = 0; rt < R; ++rt)
+    for(int s = 0; s < 4; ++s) k[b][s] = *reinterpret_cast<const v4f*>(src + 16 * s);
+  }
 #pragma unroll
-      for(int t = 0; t < 4; ++t) z[rt][b][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  for(int b = 0; b < NB; ++b)
 #pragma unroll
     for(int t = 0; t < 4; ++t)
 #pragma unroll
-      for(int s = 0; s < 4; ++s) {
-        const v4f kt = rows_to_registers(k[t][s]);
+      for(int x = 0; x < 4; ++x) v[b][t][x] = vb[min(64 * b + 16 * t + 4 * x + g, p.len - 1) * v_row + 16 * wave + c];
 #pragma unroll
-        for(int x = 0; x < 4; ++x)
+  for(int b = 0; b < NB; ++b)
 #pragma unroll
-          for(int rt = 0; rt < R; ++rt) z[rt][b][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[x], q[rt][s][x], z[rt][b][t], 0, 0, 0);
-      }
-    if(b + 1 < NB) load_k(b + 1);
-    else load_v(0);
+    for(int s = 0; s < 4; ++s) k[b][s] = rows_to_registers(k[b][s]);
+  const int tiles = (p.len + 15) / 16;   // blocks of 16 keys
+  if(p.len % 16 != 0) {   // past the last key: nothing, whatever the last value row holds
+#pragma unroll
+    for(int b = 0; b < NB; ++b)
+#pragma unroll
+      for(int t = 0; t < 4; ++t)
+        if(4 * b + t == tiles - 1) {
+#pragma unroll
+          for(int x = 0; x < 4; ++x)
+            if(64 * b + 16 * t + 4 * x + g >= p.len) v[b][t][x] = 0.0f;
+        }
   }
 
-  // ---- weights ----
+  keep_q(0);
+  __syncthreads();
+  float omax = 0.0f;
+  int turn = 0;   // (a wave may still read one turn's values in LDS while another writes the next's)
+  for(int block = group; block < p.row_blocks; block += p.row_groups, turn ^= 1) {
+    const int row = block * 16 + c;
+    v4f q[4];
 #pragma unroll
-  for(int rt = 0; rt < R; ++rt) {
-    float mx = -__builtin_inff();
+    for(int s = 0; s < 4; ++s) q[s] = *reinterpret_cast<const v4f*>(&q_lds[turn][c][16 * s + 4 * g]);
+    float mask[NB][4];
+#pragma unroll
+    for(int b = 0; b < NB; ++b)
+#pragma unroll
+      for(int r = 0; r < 4; ++r) mask[b][r] = mask_next[b][r];
+    load_q(min(block + p.row_groups, p.row_blocks - 1));
+    // ---- scores ----
+    v4f z[NB];
 #pragma unroll
     for(int b = 0; b < NB; ++b) {
-      const bool whole = b + 1 < NB || 64 * NB == p.len;   // (the same for every wave)
+      z[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+      if(4 * b + wave < tiles) {
 #pragma unroll
-      for(int t = 0; t < 4; ++t) {
-        const int key = 64 * b + 16 * t + 4 * g;
-        v4f mk = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        if(p.mask) {
-          if(whole) mk = *reinterpret_cast<const v4f_any*>(mask[rt] + key);
-          else {
+        for(int s = 0; s < 4; ++s)
 #pragma unroll
-            for(int r = 0; r < 4; ++r) mk[r] = mask[rt][min(key + r, p.len - 1)];
-          }
-        }
-#pragma unroll
-        for(int r = 0; r < 4; ++r) {
-          float x = p.scale * z[rt][b][t][r];
-          if(p.mask) x = x + mk[r];
-          if(!whole && key + r >= p.len) x = -__builtin_inff();
-          z[rt][b][t][r] = x;
-          mx = fmaxf(mx, x);
-        }
+          for(int x = 0; x < 4; ++x) z[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][s][x], q[s][x], z[b], 0, 0, 0);
       }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // (a column past the end of the row adds nothing, also where the whole row is -inf and its sum NaN)
-    float at[4][4];   // the sums of elements 64 apart
+    float mx = -__builtin_inff();
 #pragma unroll
     for(int b = 0; b < NB; ++b)
-#pragma unroll
-      for(int t = 0; t < 4; ++t)
-#pragma unroll
-        for(int r = 0; r < 4; ++r) {
-          float e = expf(z[rt][b][t][r] - mx);
-          if(b + 1 == NB && 64 * b + 16 * t + 4 * g + r >= p.len) e = 0.0f;
-          z[rt][b][t][r] = e;
-          at[t][r] = b == 0 ? e : at[t][r] + e;
-        }
-    float row[4];
-#pragma unroll
-    for(int t = 0; t < 4; ++t) {
-      float s = (at[t][0] + at[t][1]) + (at[t][2] + at[t][3]);
-      s += __shfl_xor(s, 16);
-      row[t] = s + __shfl_xor(s, 32);
-    }
-    const float sum = (row[0] + row[1]) + (row[2] + row[3]);
-#pragma unroll
-    for(int b = 0; b < NB; ++b)
-#pragma unroll
-      for(int t = 0; t < 4; ++t) {
-#pragma unroll
-        for(int r = 0; r < 4; ++r) z[rt][b][t][r] = z[rt][b][t][r] / sum;
-        z[rt][b][t] = rows_to_registers(z[rt][b][t]);   // weight of key 16 t + 4 x + g in register x
-      }
-  }
-
-  // ---- weighted values ----
-  v4f o[R][4];
-#pragma unroll
-  for(int rt = 0; rt < R; ++rt)
-#pragma unroll
-    for(int j = 0; j < 4; ++j) o[rt][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for(int b = 0; b < NB; ++b) {
-    if(b + 1 == NB) {   // past the last key: nothing, whatever the last value row holds
-#pragma unroll
-      for(int t = 0; t < 4; ++t)
-#pragma unroll
-        for(int x = 0; x < 4; ++x)
-          if(64 * b + 16 * t + 4 * x + g >= p.len) {
-            v[t][x] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for(int rt = 0; rt < R; ++rt) z[rt][b][t][x] = 0.0f;
-          }
-    }
-#pragma unroll
-    for(int t = 0; t < 4; ++t)
-#pragma unroll
-      for(int x = 0; x < 4; ++x)
-#pragma unroll
-        for(int j = 0; j < 4; ++j)
-#pragma unroll
-          for(int rt = 0; rt < R; ++rt) o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][x][j], z[rt][b][t][x], o[rt][j], 0, 0, 0);
-    if(b + 1 < NB) load_v(b + 1);
-  }
-  // lane (c, g): row c, d = 16 g + 4 r + j
-  float omax = 0.0f;
-#pragma unroll
-  for(int rt = 0; rt < R; ++rt) {
-    const int row = row0 + 16 * rt + c;
-    if(row < p.m) {
-      float* dst = p.out + p.os.entry(entry, p.heads) + (size_t)row * p.os.row + 16 * g;
 #pragma unroll
       for(int r = 0; r < 4; ++r) {
-        const v4f y = v4f{o[rt][0][r], o[rt][1][r], o[rt][2][r], o[rt][3][r]};
-        *reinterpret_cast<v4f*>(dst + 4 * r) = y;
-        omax = abs4max(y, omax);
+        const int key = 64 * b + 16 * wave + 4 * g + r;
+        float x = p.scale * z[b][r];
+        if(p.mask) x = x + mask[b][r];
+        z[b][r] = key < p.len ? x : -__builtin_inff();
+        mx = fmaxf(mx, z[b][r]);
       }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    if(g == 0) top_lds[turn][wave][c] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(top_lds[turn][0][c], top_lds[turn][1][c]), fmaxf(top_lds[turn][2][c], top_lds[turn][3][c]));
+    // ---- weights ----
+    float at[4];   // the sums of elements 64 apart
+#pragma unroll
+    for(int b = 0; b < NB; ++b)
+#pragma unroll
+      for(int r = 0; r < 4; ++r) {
+        float e = expf(z[b][r] - mx);
+        if(64 * b + 16 * wave + 4 * g + r >= p.len) e = 0.0f;   // (also where the whole row is -inf and its sum NaN)
+        z[b][r] = e;
+        at[r] = b == 0 ? e : at[r] + e;
+      }
+    float part = (at[0] + at[1]) + (at[2] + at[3]);
+    part += __shfl_xor(part, 16);
+    part += __shfl_xor(part, 32);
+    if(g == 0) sum_lds[turn][wave][c] = part;
+    __syncthreads();
+    const float sum = (sum_lds[turn][0][c] + sum_lds[turn][1][c]) + (sum_lds[turn][2][c] + sum_lds[turn][3][c]);
+    // (key 16 t + 4 x + y of a block at 16 t + 4 y + x: what a lane of the next product needs lies together)
+#pragma unroll
+    for(int b = 0; b < NB; ++b)
+#pragma unroll
+      for(int r = 0; r < 4; ++r) {
+        const float w = z[b][r] / sum;
+        weight_lds[turn][c][64 * b + 16 * wave + 4 * r + g] = 64 * b + 16 * wave + 4 * g + r < p.len ? w : 0.0f;
+      }
+    keep_q(turn ^ 1);
+    __syncthreads();
+    // ---- weighted values ----
+    v4f o = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for(int b = 0; b < NB; ++b)
+#pragma unroll
+      for(int t = 0; t < 4; ++t)
+        if(4 * b + t < tiles) {
+          const v4f w = *reinterpret_cast<const v4f*>(&weight_lds[turn][c][64 * b + 16 * t + 4 * g]);
+#pragma unroll
+          for(int x = 0; x < 4; ++x) o = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][t][x], w[x], o, 0, 0, 0);
+        }
+    if(row < p.m) {
+      *reinterpret_cast<v4f*>(ob + row * o_row + 16 * wave + 4 * g) = o;
+      omax = abs4max(o, omax);
     }
   }
   if(p.absmax_out) {
     omax = wave_max(omax);
-    if(lane == 0) p.absmax_out[w] = omax;
+    if(lane == 0) p.absmax_out[blockIdx.x * 4u + wave] = omax;
   }
 }
 

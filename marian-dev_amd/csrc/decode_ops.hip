@@ -2136,6 +2136,9 @@ int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const fl
       if(given[i][j] < 0 || given[i][j] % 4 != 0) return MARIAN_HIP_ERR_ALIGN;
     *to[i] = HeadStrides{given[i][0], given[i][1], given[i][2]};
   }
+  // (positions within a sentence are reached with 32-bit offsets)
+  if(q_strides[2] > kMaxElemsOps / m || out_strides[2] > kMaxElemsOps / m || k_strides[2] > kMaxElemsOps / len || v_strides[2] > kMaxElemsOps / len)
+    return MARIAN_HIP_ERR_RANGE;
   if(!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || (mask && !aligned4(mask)) || (absmax_out && !aligned4(absmax_out)))
     return MARIAN_HIP_ERR_ALIGN;
   if(!mask) { n_masks = 1; rows_per_mask = 1; }
@@ -2152,20 +2155,23 @@ int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const fl
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
   }
-  // Thirty-two query rows a wave read every key and value half as often as sixteen, and keep the chip busy from
-  // one wave per SIMD on (1024 of them); beyond 128 keys their scores do not fit the registers.
-  const int R = len <= 128 && batchQ * ((m + 31) / 32) >= 1024 ? 2 : 1;
-  if(absmax_out && batchQ * ((m + 16 * R - 1) / (16 * R)) > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
+  // One workgroup to a head reads its keys and values once; several where the heads are fewer than CUs, and at most
+  // four blocks of rows to a workgroup, one after the other (128 heads of 64 x 64: 9.0, 6.2, 7.5 us with 1, 2, 4
+  // workgroups a head; 384 of 128 x 128: 36.0, 29.5, 31.6; 1024 of 64 x 64: 23.1, 24.3, 28.9).
+  const int64_t row_blocks = (m + 15) / 16;
+  int64_t groups = batchQ >= 256 ? 1 : (256 + batchQ - 1) / batchQ;
+  if(groups < (row_blocks + 3) / 4) groups = (row_blocks + 3) / 4;
+  if(groups > row_blocks) groups = row_blocks;
+  if(batchQ * groups > kMaxElemsOps / 256) return MARIAN_HIP_ERR_RANGE;
+  if(absmax_out && batchQ * groups * 4 > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
   AttentionRowsArgs a{q, k, v, mask, out, absmax_out, hs.q, hs.k, hs.v, hs.out, (unsigned)batchQ, (unsigned)batchKV, (unsigned)heads,
-                      (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)((m + 16 * R - 1) / (16 * R)), scale};
-  const dim3 grid((unsigned)((batchQ * a.row_blocks + 3) / 4));
-  const int nb = (int)((len + 63) / 64);
-#define MH_ROWS(R, NB) hipLaunchKernelGGL((attention_rows_kernel<R, NB>), grid, dim3(256), 0, hst, a)
-  if(R == 2) { if(nb == 1) MH_ROWS(2, 1); else MH_ROWS(2, 2); }
-  else if(nb == 1) MH_ROWS(1, 1);
-  else if(nb == 2) MH_ROWS(1, 2);
-  else if(nb == 3) MH_ROWS(1, 3);
-  else MH_ROWS(1, 4);
+                      (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)row_blocks, (int)groups, scale};
+  const dim3 grid((unsigned)(batchQ * groups));
+#define MH_ROWS(NB) hipLaunchKernelGGL(attention_rows_kernel<NB>, grid, dim3(256), 0, hst, a)
+  if(len <= 64) MH_ROWS(1);
+  else if(len <= 128) MH_ROWS(2);
+  else if(len <= 192) MH_ROWS(3);
+  else MH_ROWS(4);
 #undef MH_ROWS
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;

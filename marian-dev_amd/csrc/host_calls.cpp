@@ -620,7 +620,7 @@ PyObject* py_attention_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   if(k->size(-1) != dk || len <= 0 || len > cap || (mask && mask->numel() % len != 0)) Py_RETURN_NONE;
   const bool blocks = m >= MARIAN_HIP_ATTENTION_ROWS_MIN, want = truth(args[6]);
   if(blocks && (dk != 64 || len > MARIAN_HIP_ATTENTION_ROWS_MAX_LEN)) Py_RETURN_NONE;
-  if(want && entries * (blocks ? (m + 15) / 16 : m) > MARIAN_HIP_ABSMAX_SLOTS) Py_RETURN_NONE;
+  if(want && entries * m > MARIAN_HIP_ABSMAX_SLOTS) Py_RETURN_NONE;
   const int64_t per = whole(args[4]);
   int64_t qs[3], ks[3], vs[3], os[3];
   if(!head_strides(*q, heads, qs) || !head_strides(*k, heads, ks) || !head_strides(*v, heads, vs)) Py_RETURN_NONE;

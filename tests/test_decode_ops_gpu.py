@@ -375,7 +375,7 @@ def test_attention_on_heads_side_by_side(ops, synth, beam, batch, heads, m, L, h
         mask[0] = -np.inf
     if how == "heads apart":
         qh, kh, vh = qh.contiguous(), kh.contiguous(), vh.contiguous()
-    small = E * heads * ((m + 15) // 16) <= 2048 and L <= 256
+    small = E * heads * m <= 2048 and L <= 256
     o = ops.Attention(qh, kh, vh, dev(mask), rpm, want_absmax=small)
     o, omax = o if small else (o, None)
     assert o.shape == qh.shape
