@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256, NB == 1 ? 4 : (NB == 2 ? 3 : 2)) void attentio
   const int group = (int)(blockIdx.x % (unsigned)p.row_groups);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, c = lane % 16, g = lane / 16;
   if(p.absmax_out && blockIdx.x == 0)   // slots past the last wave
-    for(unsigned sl = gridDim.x * 4u + threadIdx.x; sl < (unsigned)kAbsmaxSlots; sl += 256) p.absmax_out[sl] = 0.0f;
+    for(unsigned sl = p.batchQ * (unsigned)p.row_groups * 4u + threadIdx.x; sl < (unsigned)kAbsmaxSlots; sl += 256) p.absmax_out[sl] = 0.0f;
   const unsigned ekv = entry < p.batchKV ? entry : entry % p.batchKV;
   // (offsets within a tensor fit 32 bits: checked by the launcher)
   const float* kb = p.k + p.ks.entry(ekv, p.heads);

@@ -38,7 +38,7 @@ int marian_hip::launch_absmax_partials(const float* A, unsigned long n, float* p
   if(g < 1) g = 1;
   if(g > (size_t)kMaxPartials) g = kMaxPartials;
   hipLaunchKernelGGL(absmax_partial_kernel, dim3((unsigned)g), dim3(kQuantThreads), 0, reinterpret_cast<hipStream_t>(stream),
-                     A, n4, partials);
+                     A, n4, partials, (int)g);
   const hipError_t e = hipGetLastError();
   if(e != hipSuccess) return marian_hip::record_hip_error((int)e);
   *n_partials = (int)g;
@@ -359,6 +359,8 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
   int blocks = (a.n_out + Cfg::kColsPerBlock - 1) / Cfg::kColsPerBlock;
   int m_tiles = (a.M + ROWS - 1) / ROWS;   // (kFusedAll with full-height tiles: M <= ROWS)
   GemmArgs a2 = a;
+  a2.blocks_x = blocks;
+  a2.blocks_y = m_tiles;
   if constexpr(MODE == kFusedTiled) {
     if(groups) {
       if(groups->cols != Cfg::kColsPerBlock) return MARIAN_HIP_ERR_SHAPE;   // (table built for another kernel)
@@ -368,6 +370,7 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
       if(glds_status != MARIAN_HIP_OK) return glds_status;
       a2.stream_out = 0;
       a2.absmax_out = nullptr;
+      a2.blocks_x = groups->table.block0[groups->table.n];
       hipLaunchKernelGGL(gkernel, dim3(groups->table.block0[groups->table.n], m_tiles), dim3(Cfg::kThreads), lds, st,
                          a2, f.A, f.aq_out, f.partials, f.n_partials, groups->table);
       MH_HIP(hipGetLastError());
@@ -736,14 +739,14 @@ int quantize_with_known_absmax(const float* A, size_t n, const float* absmax_in,
     size_t blocks = sets;
     if(blocks > 4 * (size_t)compute_units()) blocks = 4 * (size_t)compute_units();
     hipLaunchKernelGGL(quantize_a_wide_kernel, dim3((int)blocks), dim3(1024), 0, st, A, (unsigned)(n / 16), absmax_in,
-                       (int)kAbsmaxSlots, Aq);
+                       (int)kAbsmaxSlots, Aq, (unsigned)blocks);
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
   }
   size_t qblocks = (n / 16 + kQuantThreads - 1) / kQuantThreads;
   if(qblocks > 4096) qblocks = 4096;
   hipLaunchKernelGGL(quantize_a_kernel, dim3((int)qblocks), dim3(kQuantThreads), 0, st, A, n / 16, absmax_in,
-                     (int)kAbsmaxSlots, Aq);
+                     (int)kAbsmaxSlots, Aq, (int)qblocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -879,11 +882,11 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
       const unsigned nonce = next_nonce();
       const int spins = ov == 702 ? 0 : kOnePassSpinLimit;
       if(sets == 1)
-        hipLaunchKernelGGL(prepare_a_onepass_kernel<1>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins);
+        hipLaunchKernelGGL(prepare_a_onepass_kernel<1>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
       else if(sets == 2)
-        hipLaunchKernelGGL(prepare_a_onepass_kernel<2>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins);
+        hipLaunchKernelGGL(prepare_a_onepass_kernel<2>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
       else
-        hipLaunchKernelGGL(prepare_a_onepass_kernel<4>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins);
+        hipLaunchKernelGGL(prepare_a_onepass_kernel<4>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
     }
@@ -891,12 +894,12 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
   float* partials = reinterpret_cast<float*>(workspace);
   const int g = absmax_blocks(n / 4);
   hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, A, n / 4,
-                     partials);
+                     partials, g);
   MH_HIP(hipGetLastError());
   size_t qblocks = (n / 16 + kQuantThreads - 1) / kQuantThreads;
   if(qblocks > 4096) qblocks = 4096;
   hipLaunchKernelGGL(quantize_a_kernel, dim3((int)qblocks), dim3(kQuantThreads), 0, st, A, n / 16,
-                     (const float*)partials, g, Aq);
+                     (const float*)partials, g, Aq, (int)qblocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -913,7 +916,7 @@ int marian_hip_int8_prepare_b(const float* W, int8_t* Bq, int64_t K, int64_t N, 
   float* partials = reinterpret_cast<float*>(workspace);
   const int g = absmax_blocks(n / 4);
   hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, W, n / 4,
-                     partials);
+                     partials, g);
   MH_HIP(hipGetLastError());
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)(K / 64));
   hipLaunchKernelGGL(quantize_b_transpose_kernel, grid, dim3(256), 0, st, W, (int)K, (int)N,
@@ -998,7 +1001,7 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
       float* partials = reinterpret_cast<float*>(workspace);
       const int g = absmax_blocks(n / 4);
       hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, hst, A, n / 4,
-                         partials);
+                         partials, g);
       MH_HIP(hipGetLastError());
       f.partials = partials;
       f.n_partials = g;
@@ -1019,8 +1022,8 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
 static int absmax_after(const float* out, int64_t M, int64_t n_out, float* absmax_out, hipStream_t st) {
   const size_t n = (size_t)M * (size_t)n_out;
   const int g = absmax_blocks(n / 4);   // n_out % 8 == 0; g <= 1024 partials
-  hipLaunchKernelGGL(zero_floats_kernel, dim3(2), dim3(kQuantThreads), 0, st, absmax_out + g, kAbsmaxSlots - g);
-  hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, out, n / 4, absmax_out);
+  hipLaunchKernelGGL(zero_floats_kernel, dim3(2), dim3(kQuantThreads), 0, st, absmax_out + g, kAbsmaxSlots - g, 2);
+  hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, out, n / 4, absmax_out, g);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -1111,7 +1114,7 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
       const size_t n = (size_t)M * (size_t)K;
       float* partials = reinterpret_cast<float*>(workspace);
       const int g = absmax_blocks(n / 4);
-      hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, hst, A, n / 4, partials);
+      hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, hst, A, n / 4, partials, g);
       MH_HIP(hipGetLastError());
       f.partials = partials;
       f.n_partials = g;

@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float* in,
                                                          const float* __restrict__ gamma, int gamma_stride,
                                                          const float* __restrict__ beta, int beta_stride,
                                                          float* out, int cols, float eps,
-                                                         float* __restrict__ absmax_out, int absmax_wrap) {
+                                                         float* __restrict__ absmax_out, int absmax_wrap, int rows) {
   __shared__ float red[4];
   float omax = 0.0f;   // max |y| over what this thread writes
   const size_t row = blockIdx.x;
@@ -189,33 +189,44 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float* in,
     } else {
       if(tid == 0) absmax_out[row] = omax;
       if(row == 0)
-        for(int sl = gridDim.x + tid; sl < kAbsmaxSlots; sl += 256) absmax_out[sl] = 0.0f;
+        for(int sl = rows + tid; sl < kAbsmaxSlots; sl += 256) absmax_out[sl] = 0.0f;
     }
   }
 }
 
-// Rows of up to 1024 values: one wave per row and one row per workgroup, four float4 per lane.  The three reductions stay inside the wave, so the kernel has
-// no workgroup barrier and no LDS traffic between its load and its store; scale and shift come as
-// 16-byte loads (gamma_stride / beta_stride 1, 16-byte aligned) or as one broadcast value (0).
-__global__ __launch_bounds__(64) void layer_norm_wave_kernel(const float* in, const float* __restrict__ add,
+// Rows of up to 1024 values: one wave per row and per workgroup, four float4 per lane.  The three reductions stay
+// inside the wave, so the kernel has no workgroup barrier and no LDS traffic between its load and its
+// store; scale and shift come as 16-byte loads (gamma_stride / beta_stride 1, 16-byte aligned) or as one
+// broadcast value (0).
+// MANY: more rows than abs-max slots.  Four waves to a workgroup, each takes every 4 blocks-th row, and the workgroup
+// leaves the maximum of all of them in its slot (one row to a workgroup and shared slots took a launch that clears
+// them and atomic maxima: 4.5 + 10.4 us for 4096 x 1024, now 10.4 us; one wave to a workgroup and two rows to a
+// wave 12.0).
+template <bool MANY>
+__global__ __launch_bounds__(MANY ? 256 : 64) void layer_norm_wave_kernel(const float* in, const float* __restrict__ add,
                                                              const float* __restrict__ gamma, int gamma_stride,
                                                              const float* __restrict__ beta, int beta_stride,
                                                              float* out, int cols, float eps,
-                                                             float* __restrict__ absmax_out, int absmax_wrap) {
-  constexpr int VPL = 4;
-  const size_t row = blockIdx.x;
-  const int lane = threadIdx.x, cols4 = cols / 4;
-  const v4f* x = reinterpret_cast<const v4f*>(in + row * cols);
-  const v4f* a = add ? reinterpret_cast<const v4f*>(add + row * cols) : nullptr;
-  v4f* y = reinterpret_cast<v4f*>(out + row * cols);
+                                                             float* __restrict__ absmax_out, int blocks, int rows) {
+  constexpr int VPL = 4, WAVES = MANY ? 4 : 1;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, cols4 = cols / 4;
   const v4f zero = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   v4f v[VPL], t[VPL], gm[VPL], bt[VPL];
   // all loads at once, positions past the row clamped and dropped afterwards
+  auto load_row = [&](size_t row, v4f (&v)[VPL], v4f (&t)[VPL]) __attribute__((always_inline)) {
+    const v4f* x = reinterpret_cast<const v4f*>(in + row * cols);
+    const v4f* a = add ? reinterpret_cast<const v4f*>(add + row * cols) : nullptr;
+#pragma unroll
+    for(int j = 0; j < VPL; ++j) {
+      const int i = min(j * 64 + lane, cols4 - 1);
+      v[j] = x[i];
+      t[j] = a ? a[i] : zero;
+    }
+  };
+  load_row((size_t)min((int)blockIdx.x * WAVES + wave, rows - 1), v, t);
 #pragma unroll
   for(int j = 0; j < VPL; ++j) {
     const int i = min(j * 64 + lane, cols4 - 1);
-    v[j] = x[i];
-    t[j] = a ? a[i] : zero;
     if(gamma_stride) gm[j] = reinterpret_cast<const v4f*>(gamma)[i];
     if(beta && beta_stride) bt[j] = reinterpret_cast<const v4f*>(beta)[i];
   }
@@ -229,47 +240,58 @@ __global__ __launch_bounds__(64) void layer_norm_wave_kernel(const float* in, co
 #pragma unroll
     for(int j = 0; j < VPL; ++j) bt[j] = v4f{b0, b0, b0, b0};
   }
-  float sum = 0.0f;
-#pragma unroll
-  for(int j = 0; j < VPL; ++j) {
-    if(a) v[j] = v4f{v[j].x + t[j].x, v[j].y + t[j].y, v[j].z + t[j].z, v[j].w + t[j].w};
-    if(j * 64 + lane < cols4) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
-  }
-  const float mean = wave_sum(sum) / (float)cols;
-  float sq = 0.0f;
-#pragma unroll
-  for(int j = 0; j < VPL; ++j) {
-    if(j * 64 + lane < cols4) {
-      const float d0 = v[j].x - mean, d1 = v[j].y - mean, d2 = v[j].z - mean, d3 = v[j].w - mean;
-      sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
-    }
-  }
-  const float sigma = sqrtf(wave_sum(sq) / (float)cols + eps);
   float omax = 0.0f;
+  for(int row = (int)blockIdx.x * WAVES + wave; row < rows; row += blocks * WAVES) {
+    float sum = 0.0f;
 #pragma unroll
-  for(int j = 0; j < VPL; ++j) {
-    const int i = j * 64 + lane;
-    if(i < cols4) {
-      float r[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-      const float g[4] = {gm[j].x, gm[j].y, gm[j].z, gm[j].w}, b[4] = {bt[j].x, bt[j].y, bt[j].z, bt[j].w};
+    for(int j = 0; j < VPL; ++j) {
+      if(add) v[j] = v4f{v[j].x + t[j].x, v[j].y + t[j].y, v[j].z + t[j].z, v[j].w + t[j].w};
+      if(j * 64 + lane < cols4) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
+    }
+    const float mean = wave_sum(sum) / (float)cols;
+    float sq = 0.0f;
 #pragma unroll
-      for(int e = 0; e < 4; ++e) {
-        float o = g[e] * ((r[e] - mean) / sigma);
-        if(beta) o = o + b[e];
-        r[e] = o;
-        omax = fmaxf(omax, fabsf(o));
+    for(int j = 0; j < VPL; ++j) {
+      if(j * 64 + lane < cols4) {
+        const float d0 = v[j].x - mean, d1 = v[j].y - mean, d2 = v[j].z - mean, d3 = v[j].w - mean;
+        sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
       }
-      y[i] = v4f{r[0], r[1], r[2], r[3]};
+    }
+    const float sigma = sqrtf(wave_sum(sq) / (float)cols + eps);
+    v4f* y = reinterpret_cast<v4f*>(out + (size_t)row * cols);
+#pragma unroll
+    for(int j = 0; j < VPL; ++j) {
+      const int i = j * 64 + lane;
+      if(i < cols4) {
+        float r[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+        const float g[4] = {gm[j].x, gm[j].y, gm[j].z, gm[j].w}, b[4] = {bt[j].x, bt[j].y, bt[j].z, bt[j].w};
+#pragma unroll
+        for(int e = 0; e < 4; ++e) {
+          float o = g[e] * ((r[e] - mean) / sigma);
+          if(beta) o = o + b[e];
+          r[e] = o;
+          omax = fmaxf(omax, fabsf(o));
+        }
+        y[i] = v4f{r[0], r[1], r[2], r[3]};
+      }
+    }
+    if constexpr(MANY) {
+      if(row + blocks * WAVES < rows) load_row((size_t)(row + blocks * WAVES), v, t);
+    } else {
+      break;
     }
   }
-  if(absmax_out) {   // slot `row`; the slots past the last row are zeroed by all workgroups together
+  if(absmax_out) {   // a slot per workgroup; the slots past the last one are zeroed by all workgroups together
     omax = wave_maxf(omax);
-    if(absmax_wrap) {   // more rows than slots, see layer_norm_kernel
-      if(lane == 0) atomicMax(reinterpret_cast<int*>(absmax_out) + (int)(row % kAbsmaxSlots), __float_as_int(omax));
-    } else {
-      if(lane == 0) absmax_out[row] = omax;
-      for(int sl = (int)gridDim.x + (int)row * 64 + lane; sl < kAbsmaxSlots; sl += (int)gridDim.x * 64) absmax_out[sl] = 0.0f;
+    if constexpr(MANY) {
+      __shared__ float top[WAVES];
+      if(lane == 0) top[wave] = omax;
+      __syncthreads();
+      omax = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
     }
+    if(threadIdx.x == 0) absmax_out[blockIdx.x] = omax;
+    if(wave == 0)
+      for(int sl = blocks + (int)blockIdx.x * 64 + lane; sl < kAbsmaxSlots; sl += blocks * 64) absmax_out[sl] = 0.0f;
   }
 }
 
@@ -396,8 +418,8 @@ __global__ __launch_bounds__(THREADS) void softmax_wide_kernel(const float* in, 
 template <int VEC>
 __global__ __launch_bounds__(256) void transpose0213_kernel(const float* in,
                                                             float* __restrict__ out, long long total,
-                                                            int d1, int d2, int d3v) {
-  const long long stride = (long long)gridDim.x * 256;
+                                                            int d1, int d2, int d3v, int blocks) {
+  const long long stride = (long long)blocks * 256;
   for(long long o = (long long)blockIdx.x * 256 + threadIdx.x; o < total; o += stride) {
     const int i3 = (int)(o % d3v);
     long long r = o / d3v;
@@ -1152,7 +1174,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
   float amax = 0.0f;
 #pragma unroll
   for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) amax = fmaxf(amax, pm[i]);
-  amax = block_max(amax, red);
+  amax = block_max<kProjThreads / 64>(amax, red);
   // The keys and values are asked for last - a wave's loads complete in the order of their issue,
   // and they are needed last - and only now: in front of the abs-max values they would delay them.
   // No branches around them (positions past the end repeat the last one; the number of loads is
@@ -1647,12 +1669,12 @@ __device__ __forceinline__ void nbest_hand_over(NbestShared& sh, int* is_last, l
 template <int KEEP, bool FENCED = false>
 __global__ __launch_bounds__(1024) void nbest_part_kernel(const float* __restrict__ scores, long long dimBatch,
                                                           long long vocab, int perSeg, long long sliceLen,
-                                                          int N, float* candVal, unsigned* candIdx,
+                                                          int N, int parts, float* candVal, unsigned* candIdx,
                                                           unsigned* counters, float* __restrict__ outScores,
                                                           unsigned* __restrict__ outKeys) {
   __shared__ NbestShared sh;
   __shared__ int is_last;
-  const int part = blockIdx.x, parts = gridDim.x;
+  const int part = blockIdx.x;
   const long long b = blockIdx.y;
   const long long k = part / perSeg, v0 = (long long)(part % perSeg) * sliceLen;
   const long long len = min(sliceLen, vocab - v0);
@@ -1703,14 +1725,14 @@ template <int VPT, int KEEP, bool FENCED = false>
 __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __restrict__ in,
                                                                 const float* __restrict__ rowAdd,
                                                                 float* __restrict__ lpOut, long long dimBatch,
-                                                                int vocab, int N, float* candVal,
+                                                                int vocab, int N, int parts, float* candVal,
                                                                 unsigned* candIdx, unsigned* counters,
                                                                 float* __restrict__ outScores,
                                                                 unsigned* __restrict__ outKeys) {
   __shared__ NbestShared sh;
   __shared__ int is_last;
   __shared__ float red[32];
-  const int k = blockIdx.x, parts = gridDim.x, t = threadIdx.x;
+  const int k = blockIdx.x, t = threadIdx.x;
   const long long b = blockIdx.y;
   const size_t row = (size_t)k * dimBatch + b;
   const int cols4 = vocab / 4;
@@ -1758,8 +1780,8 @@ __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __r
 // bytes before and after it one by one (byte i of the range holds byte i % elem_bytes of the
 // pattern; the middle starts on an element boundary because the range does).
 __global__ __launch_bounds__(256) void fill_kernel(unsigned char* __restrict__ p, long long bytes, long long head,
-                                                   long long vecs, int elem_bytes, unsigned long long pattern) {
-  const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x, nthreads = (long long)gridDim.x * blockDim.x;
+                                                   long long vecs, int elem_bytes, unsigned long long pattern, int blocks) {
+  const long long tid = (long long)blockIdx.x * 256 + threadIdx.x, nthreads = (long long)blocks * 256;
   unsigned long long rep = pattern;
   if(elem_bytes == 1) rep = (pattern & 0xFFull) * 0x0101010101010101ull;
   else if(elem_bytes == 2) rep = (pattern & 0xFFFFull) * 0x0001000100010001ull;
@@ -1786,7 +1808,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const float* __restrict__ E,
                                                     unsigned vocab, int dimEmb, float scale,
                                                     const float* __restrict__ signal, unsigned rows_per_signal,
                                                     unsigned n_signals, float* __restrict__ out,
-                                                    float* __restrict__ absmax_out) {
+                                                    float* __restrict__ absmax_out, unsigned rows, unsigned chunks) {
   __shared__ float red[4];
   const unsigned row = blockIdx.x, chunk = blockIdx.y;
   const int tid = threadIdx.x;
@@ -1826,7 +1848,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const float* __restrict__ E,
     }
   }
   if(absmax_out) {   // a slot per workgroup; the first workgroup zeroes the slots past the last one
-    const unsigned slot = row * gridDim.y + chunk, slots = gridDim.x * gridDim.y;
+    const unsigned slot = row * chunks + chunk, slots = rows * chunks;
     omax = row_reduce<256, true>(omax, red);
     if(tid == 0) absmax_out[slot] = omax;
     if(slot == 0)
@@ -1865,8 +1887,8 @@ __global__ __launch_bounds__(256) void select_state_kernel(const float* __restri
   }
 }
 
-__global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ p, long long n) {
-  for(long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+__global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ p, long long n, int blocks) {
+  for(long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)blocks * 256)
     p[i] = 0u;
 }
 
@@ -1913,24 +1935,32 @@ int marian_hip_layer_norm(const float* in, const float* add, const float* gamma,
   const bool vec = cols % 4 == 0 && aligned16(in) && aligned16(out) && (!add || aligned16(add));
   const bool wave_form = vec && cols <= 1024 && (gs == 0 || aligned16(gamma)) &&
                          (!beta || bs == 0 || aligned16(beta));
-  // more rows than abs-max slots (an encoder's sentence batch): the rows share the slots, which are
-  // cleared first (a kernel, so that the call may sit in a recorded graph)
+  // more rows than abs-max slots (an encoder's sentence batch): the wave form deals the rows out over as many
+  // workgroups as there are slots; the others share the slots, which are cleared first (a kernel, so that
+  // the call may sit in a recorded graph)
   const int wrap = absmax_out && rows > kAbsmaxSlots ? 1 : 0;
+  if(wave_form) {
+    const int blocks = wrap ? (rows + 3 < 4 * (int64_t)kAbsmaxSlots ? (int)((rows + 3) / 4) : kAbsmaxSlots) : (int)rows;
+    if(wrap)
+      hipLaunchKernelGGL(layer_norm_wave_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, blocks, (int)rows);
+    else
+      hipLaunchKernelGGL(layer_norm_wave_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, blocks, (int)rows);
+    MH_HIP(hipGetLastError());
+    return MARIAN_HIP_OK;
+  }
   if(wrap) {
     hipLaunchKernelGGL(zero_words_kernel, dim3(kAbsmaxSlots / 256), dim3(256), 0, st, reinterpret_cast<unsigned*>(absmax_out),
-                       (long long)kAbsmaxSlots);
+                       (long long)kAbsmaxSlots, kAbsmaxSlots / 256);
     MH_HIP(hipGetLastError());
   }
-  if(wave_form)
-    hipLaunchKernelGGL(layer_norm_wave_kernel, dim3((unsigned)rows), dim3(64), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap);
-  else if(vec && cols <= 1024)
-    hipLaunchKernelGGL(layer_norm_kernel<1>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap);
+  if(vec && cols <= 1024)
+    hipLaunchKernelGGL(layer_norm_kernel<1>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   else if(vec && cols <= 4096)
-    hipLaunchKernelGGL(layer_norm_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap);
+    hipLaunchKernelGGL(layer_norm_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   else if(vec && cols <= 8192)
-    hipLaunchKernelGGL(layer_norm_kernel<8>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap);
+    hipLaunchKernelGGL(layer_norm_kernel<8>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   else
-    hipLaunchKernelGGL(layer_norm_kernel<0>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap);
+    hipLaunchKernelGGL(layer_norm_kernel<0>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -1954,10 +1984,10 @@ int marian_hip_embed(const float* E, const uint32_t* ids, int64_t rows, int64_t 
   const unsigned rps = signal ? (unsigned)rows_per_signal : 1u, ns = signal ? (unsigned)n_signals : 1u;
   if(vec)
     hipLaunchKernelGGL(embed_kernel<true>, dim3((unsigned)rows, (unsigned)chunks), dim3(256), 0, st, E, ids,
-                       (unsigned)vocab, (int)dimEmb, scale, signal, rps, ns, out, absmax_out);
+                       (unsigned)vocab, (int)dimEmb, scale, signal, rps, ns, out, absmax_out, (unsigned)rows, (unsigned)chunks);
   else
     hipLaunchKernelGGL(embed_kernel<false>, dim3((unsigned)rows, (unsigned)chunks), dim3(256), 0, st, E, ids,
-                       (unsigned)vocab, (int)dimEmb, scale, signal, rps, ns, out, absmax_out);
+                       (unsigned)vocab, (int)dimEmb, scale, signal, rps, ns, out, absmax_out, (unsigned)rows, (unsigned)chunks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2066,8 +2096,8 @@ int marian_hip_transpose0213(const float* in, float* out, int64_t d0, int64_t d1
   const long long total = d0 * d1 * d2 * (vec ? d3 / 4 : d3);
   long long blocks = (total + 255) / 256;
   if(blocks > 8192) blocks = 8192;
-  if(vec) hipLaunchKernelGGL(transpose0213_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)(d3 / 4));
-  else hipLaunchKernelGGL(transpose0213_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)d3);
+  if(vec) hipLaunchKernelGGL(transpose0213_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)(d3 / 4), (int)blocks);
+  else hipLaunchKernelGGL(transpose0213_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)d3, (int)blocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2448,7 +2478,7 @@ int marian_hip_fill(void* begin, int64_t count, int elem_bytes, uint64_t pattern
   if(blocks > 4096) blocks = 4096;
   hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
                      reinterpret_cast<unsigned char*>(begin), bytes, head, vecs, elem_bytes,
-                     (unsigned long long)pattern);
+                     (unsigned long long)pattern, (int)blocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2467,7 +2497,7 @@ int marian_hip_nbest_beams_workspace_init(void* workspace, size_t workspace_byte
   const long long words = (long long)(workspace_bytes / 4);
   const unsigned blocks = (unsigned)((words + 255) / 256 < 1024 ? (words + 255) / 256 : 1024);
   if(words > 0)
-    hipLaunchKernelGGL(zero_words_kernel, dim3(blocks), dim3(256), 0, st, reinterpret_cast<unsigned*>(workspace), words);
+    hipLaunchKernelGGL(zero_words_kernel, dim3(blocks), dim3(256), 0, st, reinterpret_cast<unsigned*>(workspace), words, (int)blocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2496,7 +2526,7 @@ int marian_hip_nbest_beams(const float* scores, int64_t beam, int64_t dimBatch, 
   const dim3 grid((unsigned)plan.parts, (unsigned)dimBatch);
 #define MH_NBP(KEEP, FENCED)                                                                                   \
   hipLaunchKernelGGL((nbest_part_kernel<KEEP, FENCED>), grid, dim3(1024), 0, st, scores, (long long)dimBatch, \
-                     (long long)vocab, plan.perSeg, plan.sliceLen, (int)N, candVal, candIdx, counters,         \
+                     (long long)vocab, plan.perSeg, plan.sliceLen, (int)N, (int)plan.parts, candVal, candIdx, counters,         \
                      outScores, outKeys)
   if(nbest_fenced()) {
 #ifdef MARIAN_HIP_TUNING
@@ -2537,7 +2567,7 @@ int marian_hip_logsoftmax_nbest_beams(const float* logits, const float* rowAdd, 
   const dim3 grid((unsigned)beam, (unsigned)dimBatch);
 #define MH_LSNB(VPT, KEEP, FENCED)                                                                                   \
   hipLaunchKernelGGL((logsoftmax_nbest_kernel<VPT, KEEP, FENCED>), grid, dim3(1024), 0, st, logits, rowAdd, logProbs, \
-                     (long long)dimBatch, (int)vocab, (int)N, candVal, candIdx, counters, outScores, outKeys)
+                     (long long)dimBatch, (int)vocab, (int)N, (int)beam, candVal, candIdx, counters, outScores, outKeys)
   if(nbest_fenced()) {
 #ifdef MARIAN_HIP_TUNING
     if(N <= 4) MH_LSNB(8, 4, true);

@@ -189,8 +189,9 @@ __device__ __forceinline__ void xcd_tile(int tiles_n, int tiles_m, int block, in
 // workgroup stored (omax: this lane's share), the workgroup of slot 0 zeroes the slots past the
 // `used` ones the launch fills.  red: the LDS ring, free once every wave is past its last fragment
 // read (the first barrier).  All threads of the workgroup call it.
+template <int THREADS>
 __device__ __forceinline__ void publish_tile_absmax(float omax, float* absmax_out, int slot, int used, float* red) {
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, nw = blockDim.x / kWave;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, nw = THREADS / kWave;
   omax = wave_max(omax);
   __syncthreads();
   if(lane == 0) red[wave] = omax;
@@ -201,7 +202,7 @@ __device__ __forceinline__ void publish_tile_absmax(float omax, float* absmax_ou
     absmax_out[slot] = m;
   }
   if(slot == 0)
-    for(int sl = used + tid; sl < kAbsmaxSlots; sl += (int)blockDim.x) absmax_out[sl] = 0.0f;
+    for(int sl = used + tid; sl < kAbsmaxSlots; sl += THREADS) absmax_out[sl] = 0.0f;
 }
 
 // One BM x BN output tile at rows m0 .., columns n0 .. (any multiples of 32; the tile may hang over
@@ -532,7 +533,7 @@ __device__ __forceinline__ void gemm_mfma32_tile(const GemmArgs& args, const int
     }
   }
   if(!(MH_DBG(args, 2)) && AMAX && args.absmax_out && !args.dump)   // (all waves: it has barriers)
-    publish_tile_absmax(omax, args.absmax_out, slot, args.absmax_used, reinterpret_cast<float*>(lds));
+    publish_tile_absmax<(SPLIT ? 2 : 1) * Cfg::kThreads>(omax, args.absmax_out, slot, args.absmax_used, reinterpret_cast<float*>(lds));
   if(MH_PROF(args) && tid == 0) {
     long long* p = MH_PROF(args) + (size_t)slot * 8;
     p[0] = t_start; p[1] = t_prologue; p[2] = t_main; p[3] = MH_CLOCK(); p[6] = w_start; p[7] = MH_WALL();

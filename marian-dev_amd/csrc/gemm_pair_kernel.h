@@ -273,7 +273,7 @@ __device__ __forceinline__ void gemm_pair_tiles(const GemmArgs& args, const int 
     }
   }
   if(AMAX && args.absmax_out)
-    publish_tile_absmax(omax, args.absmax_out, slot, args.absmax_used, reinterpret_cast<float*>(lds));
+    publish_tile_absmax<PairCfg::kThreads>(omax, args.absmax_out, slot, args.absmax_used, reinterpret_cast<float*>(lds));
   if(MH_PROF(args) && tid == 0) {
     long long* p = MH_PROF(args) + (size_t)slot * 8;
     p[0] = t_start; p[1] = t_prologue; p[2] = t_main; p[3] = MH_CLOCK(); p[4] = t_main; p[5] = t_side; p[6] = w_start; p[7] = MH_WALL();

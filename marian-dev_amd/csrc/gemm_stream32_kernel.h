@@ -91,7 +91,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   using Cfg = Stream32Cfg<MT32, WN, KW, PW>;
   constexpr bool GROUPED = std::is_same<GROUPS, GroupTable>::value;
   static_assert(!GROUPED || MODE == kFusedTiled, "several weight matrices: quantize-on-stage form only");
-  int bx = blockIdx.x, gx = gridDim.x;   // column block within this workgroup's matrix, and how many it has
+  int bx = blockIdx.x, gx = args.blocks_x;   // column block within this workgroup's matrix, and how many it has
   if constexpr(GROUPED) {
     int g = 0;
 #pragma unroll
@@ -339,7 +339,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   // ---- activations into LDS, operand order: slot (sub-step, m-tile, lane) of 16 bytes holds
   //      Aq[mt*32 + lane%32][(s0+step)*32 + (lane/32)*16 .. +15]
   if(TILED) {
-    amax = block_max(amax, red);
+    amax = block_max<kStream32Waves>(amax, red);
     aqm = quant_mult_from_maxabs(amax);
     unquant = unquant_mult(aqm, bqm, args.scale);
     finite_t = aqm < __builtin_inff();   // (see the fused form below)
@@ -359,7 +359,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
     // (activation rows between M and the end of the last 32-row tile stay whatever LDS holds: a
     // row only feeds its own output row, integer products cannot trap, and rows past M are never
     // stored)
-    amax = block_max(amax, red);
+    amax = block_max<kStream32Waves>(amax, red);
     if(MH_PROF(args)) tp[1] = MH_CLOCK();
     aqm = quant_mult_from_maxabs(amax);
     unquant = unquant_mult(aqm, bqm, args.scale);
@@ -541,14 +541,14 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   if(args.absmax_out && !args.dump) {
     // slot (workgroup, wave) takes this wave's maximum; workgroup 0 zeroes the slots nobody owns
     // (the launcher made sure that 8 slots per workgroup fit)
-    const int block = blockIdx.y * gx + bx, used = gx * gridDim.y * kStream32Waves;
+    const int block = blockIdx.y * gx + bx, used = gx * args.blocks_y * kStream32Waves;
     omax = wave_max(omax);
     if(lane == 0) args.absmax_out[block * kStream32Waves + wave] = omax;
     if(block == 0)
       for(int sl = used + tid; sl < kAbsmaxSlots; sl += kStream32Threads) args.absmax_out[sl] = 0.0f;
   }
   if(MH_PROF(args) && tid == 0) {
-    long long* p = MH_PROF(args) + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 8;
+    long long* p = MH_PROF(args) + ((size_t)blockIdx.y * args.blocks_x + blockIdx.x) * 8;
     p[0] = tp[0]; p[1] = tp[1]; p[2] = tp[2]; p[3] = tp[3]; p[4] = tp[4]; p[5] = MH_CLOCK();
     p[6] = MH_WALL();
     p[7] = wall0;

@@ -41,11 +41,11 @@ __device__ __forceinline__ uint32_t quantize16_pair(float x0, float x1, float qm
 
 // prepareA: elementwise, eight values (two 16-byte loads, one 16-byte store) per thread and step
 __global__ __launch_bounds__(256) void quantize16_a_kernel(const float* __restrict__ x, size_t n8,
-                                                           int16_t* __restrict__ out) {
+                                                           int16_t* __restrict__ out, int blocks) {
   const v4f* x4 = reinterpret_cast<const v4f*>(x);
   uint4* o = reinterpret_cast<uint4*>(out);
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for(size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += stride) {
+  const size_t stride = (size_t)blocks * 256;
+  for(size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += stride) {
     const v4f a = x4[2 * i], b = x4[2 * i + 1];
     uint4 q;
     q.x = quantize16_pair(a.x, a.y, kQuantMult16);
@@ -586,7 +586,7 @@ int marian_hip_int16_prepare_a(const float* A, int16_t* Aq, int64_t M, int64_t K
   const size_t n8 = (size_t)M * (size_t)K / 8;
   size_t blocks = (n8 + 255) / 256;
   if(blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(quantize16_a_kernel, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), A, n8, Aq);
+  hipLaunchKernelGGL(quantize16_a_kernel, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), A, n8, Aq, (int)blocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }

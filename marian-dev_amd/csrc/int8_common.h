@@ -113,6 +113,7 @@ struct GemmArgs {
   // write the output with non-temporal stores (set by the launchers for outputs of several MB,
   // which would otherwise sit dirty in L2 until the kernel ends and be written back then)
   int stream_out = 0;
+  int blocks_x = 0, blocks_y = 0;   // small-M launches: workgroups of the launch
 };
 
 constexpr int kAbsmaxSlots = 2048;

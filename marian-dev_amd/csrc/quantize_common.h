@@ -104,17 +104,19 @@ __device__ __forceinline__ float wave_max(float m) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), 63));
 }
 
-// Max over the workgroup (whole waves, at most 16 of them); every thread returns the result.
-// red: >= blockDim/64 floats of LDS.
+// Max over the workgroup of WAVES waves (at most 16); every thread returns the result.
+// red: >= WAVES floats of LDS.
+// (The sizes of a launch are template or kernel arguments throughout: a kernel that asks the runtime for them has
+// 256 bytes of hidden arguments, and its launch costs the host 0.35 us more.)
+template <int WAVES>
 __device__ __forceinline__ float block_max(float m, float* red) {
   m = wave_max(m);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int nw = blockDim.x / kWave;
   __syncthreads();
   if(lane == 0) red[wave] = m;
   __syncthreads();
   // every row of 16 lanes reads all the wave maxima, so the rows need no exchange afterwards
-  const float r = (lane % 16 < nw) ? red[lane % 16] : 0.0f;
+  const float r = (lane % 16 < WAVES) ? red[lane % 16] : 0.0f;
   return row16_max(r);
 }
 

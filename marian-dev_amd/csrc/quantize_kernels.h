@@ -8,41 +8,41 @@ namespace marian_hip {
 
 // Pass 1: per-workgroup abs-max of n floats (n % 4 == 0) -> partials[blockIdx.x].
 __global__ __launch_bounds__(kQuantThreads) void absmax_partial_kernel(
-    const float* __restrict__ x, size_t n4, float* __restrict__ partials) {
+    const float* __restrict__ x, size_t n4, float* __restrict__ partials, int blocks) {
   __shared__ float red[kQuantThreads / kWave];
   const v4f* x4 = reinterpret_cast<const v4f*>(x);
   float m = 0.0f;
-  size_t stride = (size_t)gridDim.x * blockDim.x;
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  size_t stride = (size_t)blocks * kQuantThreads;
+  size_t i = (size_t)blockIdx.x * kQuantThreads + threadIdx.x;
   // four independent loads in flight per thread
   for(; i + 3 * stride < n4; i += 4 * stride) {
     v4f a = x4[i], b = x4[i + stride], c = x4[i + 2 * stride], d = x4[i + 3 * stride];
     m = abs4max(a, m); m = abs4max(b, m); m = abs4max(c, m); m = abs4max(d, m);
   }
   for(; i < n4; i += stride) m = abs4max(x4[i], m);
-  m = block_max(m, red);
+  m = block_max<kQuantThreads / kWave>(m, red);
   if(threadIdx.x == 0) partials[blockIdx.x] = m;
 }
 
 // Clears n floats (a kernel rather than a memset node, so callers may capture the call in a graph).
-__global__ __launch_bounds__(kQuantThreads) void zero_floats_kernel(float* __restrict__ p, int n) {
-  for(int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0.0f;
+__global__ __launch_bounds__(kQuantThreads) void zero_floats_kernel(float* __restrict__ p, int n, int blocks) {
+  for(int i = blockIdx.x * kQuantThreads + threadIdx.x; i < n; i += blocks * kQuantThreads) p[i] = 0.0f;
 }
 
 // Pass 2 of prepareA: reduce the partials, quantize 16 values per thread per step, block 0
 // writes the quantMult tail at byte n.
 __global__ __launch_bounds__(kQuantThreads) void quantize_a_kernel(
     const float* __restrict__ x, size_t n16, const float* __restrict__ partials, int n_partials,
-    int8_t* __restrict__ out) {
+    int8_t* __restrict__ out, int blocks) {
   __shared__ float red[kQuantThreads / kWave];
   float m = 0.0f;
-  for(int p = threadIdx.x; p < n_partials; p += blockDim.x) m = fmaxf(m, partials[p]);
-  m = block_max(m, red);
+  for(int p = threadIdx.x; p < n_partials; p += kQuantThreads) m = fmaxf(m, partials[p]);
+  m = block_max<kQuantThreads / kWave>(m, red);
   const float qm = quant_mult_from_maxabs(m);
   const v4f* x4 = reinterpret_cast<const v4f*>(x);
   uint4* o16 = reinterpret_cast<uint4*>(out);
-  size_t stride = (size_t)gridDim.x * blockDim.x;
-  for(size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += stride) {
+  size_t stride = (size_t)blocks * kQuantThreads;
+  for(size_t i = (size_t)blockIdx.x * kQuantThreads + threadIdx.x; i < n16; i += stride) {
     v4f a = x4[4 * i], b = x4[4 * i + 1], c = x4[4 * i + 2], d = x4[4 * i + 3];
     uint4 q;
     q.x = quantize_pack4(a, qm);
@@ -70,10 +70,10 @@ __global__ __launch_bounds__(kSingleBlockThreads) void prepare_a_single_block_ke
 #pragma unroll
     for(int u = 0; u < 8; ++u) m = abs4max(v[u], m);
   }
-  m = block_max(m, red);
+  m = block_max<kSingleBlockThreads / kWave>(m, red);
   const float qm = quant_mult_from_maxabs(m);
   uint4* o16 = reinterpret_cast<uint4*>(out);
-  for(int i = threadIdx.x; i < n16; i += blockDim.x) {
+  for(int i = threadIdx.x; i < n16; i += kSingleBlockThreads) {
     v4f a = x4[4 * i], b = x4[4 * i + 1], c = x4[4 * i + 2], d = x4[4 * i + 3];
     uint4 q;
     q.x = quantize_pack4(a, qm);
@@ -108,13 +108,13 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
                                                                  unsigned long long* slots,
                                                                  unsigned long long* gen_word,
                                                                  unsigned long long* mailboxes,
-                                                                 unsigned nonce, int spin_limit) {
+                                                                 unsigned nonce, int spin_limit, int groups) {
   __shared__ float red[1024 / kWave];
   __shared__ float shared_max;
   __shared__ unsigned shared_tag;
   __shared__ __attribute__((aligned(16))) uint32_t turn[1024 * 4];   // 16 bytes per thread
   const int tid = threadIdx.x, quad = tid / 4, qlane = tid % 4;
-  const int G = gridDim.x, g = blockIdx.x;
+  const int G = groups, g = blockIdx.x;
   // (one thread per workgroup asks for the generation: every access to the word is served by the
   // same memory channel, one after the other)
   unsigned gen = 0;
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
       for(int e = 0; e < 4; ++e) m = abs4max(vals[j][e], m);
     }
   if(tid == 0) shared_tag = (nonce + gen) | 0x80000000u;   // never 0: a cleared word does not match
-  m = block_max(m, red);   // (its barriers also publish shared_tag)
+  m = block_max<1024 / kWave>(m, red);   // (its barriers also publish shared_tag)
   const unsigned tag = shared_tag;
 
   // abs-max over all of x by this workgroup alone (the way out of a wait that ran out)
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
     const size_t n4 = (size_t)n16 * 4;
     float mm = 0.0f;
     for(size_t i = tid; i < n4; i += 1024) mm = abs4max(x4[i], mm);
-    return block_max(mm, red);
+    return block_max<1024 / kWave>(mm, red);
   };
   auto pack = [](unsigned t, float v) { return ((unsigned long long)t << 32) | (unsigned long long)__float_as_uint(v); };
   float amax = m;
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
         }
       }
       const bool all_ok = __syncthreads_and(ok ? 1 : 0) != 0;
-      amax = all_ok ? block_max(mine, red) : scan_all();
+      amax = all_ok ? block_max<1024 / kWave>(mine, red) : scan_all();
       if(tid < kOnePassMailboxes)
         __hip_atomic_store(&mailboxes[tid * 32], pack(tag, amax), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       // the next launch (or replay) expects another tag; every workgroup of this launch has read
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
 // without its exchange.  A set = 256 quads = 64 KB of input per workgroup and step.
 __global__ __launch_bounds__(1024) void quantize_a_wide_kernel(const float* __restrict__ x, unsigned n16,
                                                                const float* __restrict__ partials, int n_partials,
-                                                               int8_t* __restrict__ out) {
+                                                               int8_t* __restrict__ out, unsigned blocks) {
   __shared__ float red[1024 / kWave];
   __shared__ __attribute__((aligned(16))) uint32_t turn[1024 * 4];   // 16 bytes per thread
   const int tid = threadIdx.x, quad = tid / 4, qlane = tid % 4;
@@ -243,14 +243,14 @@ __global__ __launch_bounds__(1024) void quantize_a_wide_kernel(const float* __re
   if(set < n_sets) load_set(set, vals);
   float m = 0.0f;
   for(int p = tid; p < n_partials; p += 1024) m = fmaxf(m, partials[p]);
-  m = block_max(m, red);
+  m = block_max<1024 / kWave>(m, red);
   const float qm = quant_mult_from_maxabs(m);
   const bool finite = qm < __builtin_inff();
-  for(; set < n_sets; set += gridDim.x) {
+  for(; set < n_sets; set += blocks) {
     v4f cur[4];
 #pragma unroll
     for(int e = 0; e < 4; ++e) cur[e] = vals[e];
-    if(set + gridDim.x < n_sets) load_set(set + gridDim.x, vals);
+    if(set + blocks < n_sets) load_set(set + blocks, vals);
     const unsigned q = set * 256u + (unsigned)quad;
     if(4u * q < n16) {
       // (the four lanes of a quad sit in one wave, whose LDS operations execute in order)
@@ -275,8 +275,8 @@ __global__ __launch_bounds__(256) void quantize_b_transpose_kernel(
   // group) hit every bank twice, the minimum for 64 lanes on 32 banks
   __shared__ uint32_t tile[64][17];
   float m = 0.0f;
-  for(int p = threadIdx.x; p < n_partials; p += blockDim.x) m = fmaxf(m, partials[p]);
-  m = block_max(m, red);
+  for(int p = threadIdx.x; p < n_partials; p += 256) m = fmaxf(m, partials[p]);
+  m = block_max<256 / kWave>(m, red);
   const float qm = quant_mult_from_maxabs(m);
 
   const int n0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256) void quantize_b_transpose_kernel(
 __global__ __launch_bounds__(256) void retile_b_kernel(const int8_t* __restrict__ in, int K, int N,
                                                        int8_t* __restrict__ out) {
   const size_t chunks = (size_t)K * (size_t)N / 16;
-  const size_t o = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t o = (size_t)blockIdx.x * 256 + threadIdx.x;
   if(o < chunks) {
     // chunk o of the output: sub-step o / (2 N), then column, half
     const int s = (int)(o / (2 * (size_t)N)), rem = (int)(o % (2 * (size_t)N));
