@@ -221,6 +221,17 @@ int marian_hip_nbest(const float* scores, int64_t dimBatch, int64_t rowLen, int6
                      float* outScores, uint32_t* outKeys, void* stream);
 
 /*
+ * The words a row's best scores stand for, in one launch: the selection of marian_hip_nbest on each of
+ * `rows` rows, with the positions within the row instead of keys, taken through a shortlist's ids where
+ * there is one (Shortlist::reverseMap, reference src/data/shortlist.h:25-29).
+ *   ids: [rowLen] vocabulary ids on the device, or null; outWords: rows * N values, 8-byte aligned.
+ * Positions that no score fills (a row with fewer than N scores that are not NaN) come out as -inf and
+ * -1, or the last of the ids.
+ */
+int marian_hip_nbest_words(const float* scores, int64_t rows, int64_t rowLen, int64_t N, const uint32_t* ids,
+                           float* outScores, int64_t* outWords, void* stream);
+
+/*
  * The transposition and the n-best selection of a beam-search step in one call: reference
  * src/translator/beam_search.cpp:472 (swapAxes(expandedPathScores, 0, 2)) followed by :492
  * (getNBestList).  scores: [beam, dimBatch, vocab], the layout in which the step's scores leave the

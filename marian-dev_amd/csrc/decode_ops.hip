@@ -1334,6 +1334,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
 // massive ties) every thread instead keeps the KEEP >= N best of its elements in registers and
 // the draw pops them one by one.
 constexpr int kNbestMax = 16;
+constexpr int kNbestWaveCols = 2048;   // rows up to this length: a wave each (32 values a lane)
 constexpr long long kNbestMaxBatch = 4096;     // batch entries of the beam-major form
 // Its counters, 256 bytes apart: atomics on one cache line are served one after the other
 // (measured: the 256 arrivals of 32 entries on one line cost 7 us).
@@ -1603,16 +1604,110 @@ __device__ __forceinline__ void nbest_of_row(const float* __restrict__ x, long l
   nbest_core<KEEP>(scan, N, sh, emit);
 }
 
+// Where the winners of a row go: keys = absolute positions (uint32), or words = the positions within the
+// row, taken through ids where a shortlist gave the columns (a filler's position -1 is then the last
+// column, as an index counted from the end).
+struct NbestOut {
+  float* scores;
+  unsigned* keys;        // one of the two is set
+  long long* words;
+  const uint32_t* ids;   // or null
+  __device__ __forceinline__ void put(long long row, long long rowLen, int N, int r, float v, unsigned i) const {
+    scores[row * N + r] = v;
+    if(keys) {
+      keys[row * N + r] = (unsigned)(row * rowLen) + i;
+    } else {
+      const long long at = (int)i == -1 ? -1 : (long long)i;
+      words[row * N + r] = ids ? (long long)(int)ids[at < 0 ? rowLen - 1 : at] : at;
+    }
+  }
+};
+
 template <int KEEP>
-__global__ __launch_bounds__(1024) void nbest_kernel(const float* __restrict__ scores, long long rowLen, int N,
-                                                     float* __restrict__ outScores,
-                                                     unsigned* __restrict__ outKeys) {
+__global__ __launch_bounds__(1024) void nbest_kernel(const float* __restrict__ scores, long long rowLen, int N, NbestOut out) {
   __shared__ NbestShared sh;
   const long long row = blockIdx.x;
-  nbest_of_row<KEEP>(scores + row * rowLen, rowLen, N, sh, [&](int r, float v, unsigned i) {
-    outScores[row * N + r] = v;
-    outKeys[row * N + r] = (unsigned)(row * rowLen) + i;
-  });
+  nbest_of_row<KEEP>(scores + row * rowLen, rowLen, N, sh, [&](int r, float v, unsigned i) { out.put(row, rowLen, N, r, v, i); });
+}
+
+// Short rows (a shortlist's columns): one wave to a row, 64 * VPT elements in registers, no workgroup
+// barrier.  What bounds the launch is its chain - load, bound, collection, draw - and not the bytes.
+// The bound is the N-th largest of the 64 lane maxima (N elements reach it); what reaches it is
+// collected by ballots, normally N to 2 N elements, and ranked one to a lane.  More than 64 (rows of
+// equal or infinite values): drawn one by one, each the best element behind the one before.
+template <int VPT>
+__global__ __launch_bounds__(64) void nbest_wave_kernel(const float* __restrict__ scores, int rowLen, int N, NbestOut out) {
+  __shared__ float cand_val[64];
+  __shared__ unsigned cand_idx[64];
+  const int lane = threadIdx.x;
+  const long long row = blockIdx.x;
+  const float* x = scores + row * rowLen;
+  const float ninf = -__builtin_inff();
+  const unsigned none = 0xFFFFFFFFu;
+  float v[VPT];
+#pragma unroll
+  for(int j = 0; j < VPT; ++j) v[j] = x[min(j * 64 + lane, rowLen - 1)];
+#pragma unroll
+  for(int j = 0; j < VPT; ++j)
+    if(j * 64 + lane >= rowLen) v[j] = __builtin_nanf("");   // (reaches no bound and comes before nothing)
+  float mv = ninf;
+#pragma unroll
+  for(int j = 0; j < VPT; ++j) mv = fmaxf(mv, v[j]);
+  float tv = ninf;
+  for(int r = 0; r < N; ++r) {
+    tv = wave_maxf(mv);
+    const unsigned long long holders = __ballot(mv == tv);
+    if(lane == __ffsll((long long)holders) - 1) mv = ninf;
+  }
+  int count = 0;
+#pragma unroll
+  for(int j = 0; j < VPT; ++j) {
+    const unsigned long long m = __ballot(v[j] >= tv);
+    if(m) {
+      const int at = count + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      if(v[j] >= tv && at < 64) {
+        cand_val[at] = v[j]; cand_idx[at] = (unsigned)(j * 64 + lane);
+      }
+      count += __popcll(m);
+    }
+  }
+  if(count <= 64) {
+    __syncthreads();   // (one wave: orders the LDS accesses)
+    const float cv = lane < count ? cand_val[lane] : ninf;
+    const unsigned ci = lane < count ? cand_idx[lane] : none;
+    int rank = 0;
+    for(int c = 0; c < count; ++c) {
+      const float ov = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cv), c));
+      rank += nbest_before(ov, (unsigned)__builtin_amdgcn_readlane((int)ci, c), cv, ci) ? 1 : 0;
+    }
+    if(lane < count && rank < N) out.put(row, rowLen, N, rank, cv, ci);
+    if(lane >= count && lane < N) out.put(row, rowLen, N, lane, ninf, none);   // (NaN in the row: fewer than N candidates)
+    return;
+  }
+  float pv = __builtin_inff();
+  unsigned pi = 0;
+  for(int r = 0; r < N; ++r) {
+    float bv = ninf;
+    unsigned bi = none;
+#pragma unroll
+    for(int j = 0; j < VPT; ++j) {
+      const unsigned i = (unsigned)(j * 64 + lane);
+      if((r == 0 || nbest_before(pv, pi, v[j], i)) && nbest_before(v[j], i, bv, bi)) {
+        bv = v[j]; bi = i;
+      }
+    }
+#pragma unroll
+    for(int o = 32; o > 0; o >>= 1) {
+      const float ov = __shfl_xor(bv, o, 64);
+      const unsigned oi = (unsigned)__shfl_xor((int)bi, o, 64);
+      if(nbest_before(ov, oi, bv, bi)) {
+        bv = ov; bi = oi;
+      }
+    }
+    if(lane == 0) out.put(row, rowLen, N, r, bv, bi);
+    pv = bv;
+    pi = bi;
+  }
 }
 
 // Hand-over of per-part candidates to the workgroup that finishes an entry last, without fences.
@@ -2444,6 +2539,22 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
   return MARIAN_HIP_OK;
 }
 
+// Rows of up to kNbestWaveCols values: a wave each; longer ones: 1024 threads each.
+static int nbest_rows(const float* scores, int64_t rows, int64_t rowLen, int64_t N, const NbestOut& out, void* stream) {
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+#define MH_NBW(VPT) hipLaunchKernelGGL(nbest_wave_kernel<VPT>, dim3((unsigned)rows), dim3(64), 0, st, scores, (int)rowLen, (int)N, out)
+#define MH_NBK(KEEP) hipLaunchKernelGGL(nbest_kernel<KEEP>, dim3((unsigned)rows), dim3(1024), 0, st, scores, (long long)rowLen, (int)N, out)
+  if(rowLen <= kNbestWaveCols / 2) MH_NBW(kNbestWaveCols / 128);
+  else if(rowLen <= kNbestWaveCols) MH_NBW(kNbestWaveCols / 64);
+  else if(N <= 4) MH_NBK(4);
+  else if(N <= 8) MH_NBK(8);
+  else MH_NBK(16);
+#undef MH_NBW
+#undef MH_NBK
+  MH_HIP(hipGetLastError());
+  return MARIAN_HIP_OK;
+}
+
 int marian_hip_nbest(const float* scores, int64_t dimBatch, int64_t rowLen, int64_t N,
                      float* outScores, uint32_t* outKeys, void* stream) {
   if(dimBatch < 0 || rowLen <= 0 || N <= 0 || N > kNbestMax || N > rowLen) return MARIAN_HIP_ERR_SHAPE;
@@ -2451,15 +2562,18 @@ int marian_hip_nbest(const float* scores, int64_t dimBatch, int64_t rowLen, int6
   if(!scores || !outScores || !outKeys) return MARIAN_HIP_ERR_NULL;
   if(dimBatch * rowLen > 4294967295LL) return MARIAN_HIP_ERR_RANGE;   // keys are uint32
   if(!aligned4(scores) || !aligned4(outScores) || !aligned4(outKeys)) return MARIAN_HIP_ERR_ALIGN;
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if(N <= 4)
-    hipLaunchKernelGGL(nbest_kernel<4>, dim3((unsigned)dimBatch), dim3(1024), 0, st, scores, (long long)rowLen, (int)N, outScores, outKeys);
-  else if(N <= 8)
-    hipLaunchKernelGGL(nbest_kernel<8>, dim3((unsigned)dimBatch), dim3(1024), 0, st, scores, (long long)rowLen, (int)N, outScores, outKeys);
-  else
-    hipLaunchKernelGGL(nbest_kernel<16>, dim3((unsigned)dimBatch), dim3(1024), 0, st, scores, (long long)rowLen, (int)N, outScores, outKeys);
-  MH_HIP(hipGetLastError());
-  return MARIAN_HIP_OK;
+  return nbest_rows(scores, dimBatch, rowLen, N, NbestOut{outScores, outKeys, nullptr, nullptr}, stream);
+}
+
+int marian_hip_nbest_words(const float* scores, int64_t rows, int64_t rowLen, int64_t N, const uint32_t* ids,
+                           float* outScores, int64_t* outWords, void* stream) {
+  if(rows < 0 || rowLen <= 0 || N <= 0 || N > kNbestMax || N > rowLen) return MARIAN_HIP_ERR_SHAPE;
+  if(rows == 0) return MARIAN_HIP_OK;
+  if(!scores || !outScores || !outWords) return MARIAN_HIP_ERR_NULL;
+  if(rows * rowLen > 4294967295LL) return MARIAN_HIP_ERR_RANGE;
+  if(!aligned4(scores) || !aligned4(outScores) || reinterpret_cast<uintptr_t>(outWords) % 8 != 0 || (ids && !aligned4(ids)))
+    return MARIAN_HIP_ERR_ALIGN;
+  return nbest_rows(scores, rows, rowLen, N, NbestOut{outScores, nullptr, reinterpret_cast<long long*>(outWords), ids}, stream);
 }
 
 int marian_hip_fill(void* begin, int64_t count, int elem_bytes, uint64_t pattern, void* stream) {

@@ -41,7 +41,7 @@ namespace {
   F(int16_prepare_a) F(int16_prepare_b) F(int16_prepare_b_quantized_transposed) F(int16_affine_f32)      \
   F(int16_scratch_bytes)                                                                                 \
   F(layer_norm) F(embed) F(attention_cached) F(attention_rows) F(attention_ancestors) F(ancestors_advance)                 \
-  F(select_state) F(nbest) F(nbest_beams) F(nbest_beams_workspace_bytes) F(nbest_beams_workspace_init)   \
+  F(select_state) F(nbest) F(nbest_words) F(nbest_beams) F(nbest_beams_workspace_bytes) F(nbest_beams_workspace_init)   \
   F(logsoftmax_nbest_beams)
 
 struct Library {
@@ -754,6 +754,27 @@ PyObject* py_nbest(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_END
 }
 
+// nbest_words(scores, N, ids): scores [.., cols], ids [cols] or None
+PyObject* py_nbest_words(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(3, "nbest_words");
+  const at::Tensor *s = f32c(args[0]), *ids = nullptr;
+  if(!s || s->dim() < 1) Py_RETURN_NONE;
+  const int64_t N = whole(args[1]), cols = s->size(-1), rows = cols ? s->numel() / cols : 0;
+  if(!none(args[2]) && (!(ids = tensor(args[2])) || !ids_type(ids->scalar_type()) || ids->device() != s->device() ||
+                        !ids->is_contiguous() || ids->numel() != cols))
+    Py_RETURN_NONE;
+  const c10::Device d = s->device();
+  at::Tensor vals = empty({rows, N}, at::kFloat, d), words = empty({rows, N}, at::kLong, d);
+  const hipStream_t st = stream_of(d);
+  call("getNBestList", [&] {   // (no rows: refused)
+    return L.nbest_words(fptr(s), rows, rows ? cols : 0, N, ids ? static_cast<const uint32_t*>(ids->const_data_ptr()) : nullptr,
+                         fptr_mut(vals), static_cast<int64_t*>(words.data_ptr()), st);
+  });
+  Ref a(wrap(std::move(vals))), b(wrap(std::move(words)));
+  return PyTuple_Pack(2, a.p, b.p);
+  MH_END
+}
+
 // nbest_beams(scores, N): scores [beam, .., vocab]
 PyObject* py_nbest_beams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_TRY MH_ARGS(2, "nbest_beams");
@@ -848,7 +869,7 @@ PyMethodDef methods[] = {
     MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
     MH_METHOD(affine_f32_grouped), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
     MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(attention_rows), MH_METHOD(split_heads), MH_METHOD(join_heads), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors),
-    MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),
+    MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_words), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", "host path of the operators", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -351,6 +351,17 @@ def getNBestList(scores, N):
     return _taken(_host.nbest(scores, N), "getNBestList")
 
 
+def getNBestWords(scores, N, ids=None):
+    """the N best of every row of scores [.., cols] and the words they stand for: the positions in the
+    row, or the shortlist's ids [cols] there; returns (scores [rows, N], int64 words [rows, N])"""
+    out = _host.nbest_words(scores, N, ids)
+    if out is not None:
+        return out
+    scores = _f32c(scores, "getNBestWords")
+    _on_gpu(scores)
+    return _taken(_host.nbest_words(scores, N, ids), "getNBestWords")
+
+
 def getNBestListOfBeams(scores, N):
     """reference src/translator/beam_search.cpp:472 + :492: swapAxes(expandedPathScores, 0, 2)
     followed by getNBestList, without the transposed copy.  scores [beam, 1, dimBatch, vocab] (or

@@ -84,3 +84,34 @@ def test_tied_output_layer(integer, orc, synth):
         assert sl.tryForwardMap(int(w)) != out_mod.npos
     layer.clear()
     assert layer.applyAsLogits(torch.from_numpy(x).cuda()).shape[-1] == V
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [1, 5, 63, 64, 65, 1000, 1024, 1025, 2047, 2048, 2049])   # edges of the wave form
+def test_best_words_of_rows(cols):
+    import torch
+    ops = load("ops")
+    g = np.random.default_rng(cols)
+    rows = np.stack([g.standard_normal(cols),                       # ordinary scores
+                     g.integers(0, 3, cols),                        # many equal ones
+                     np.zeros(cols),                                # all equal
+                     np.full(cols, -np.inf),
+                     np.where(g.random(cols) < 0.9, -np.inf, 1.0),
+                     np.arange(cols), -np.arange(cols)]).astype(np.float32)
+    ids = np.sort(g.choice(50000, cols, replace=False)).astype(np.int32)
+    x = torch.from_numpy(rows).cuda()
+    for k in {1, min(4, cols), min(6, cols), min(16, cols)}:
+        order = np.argsort(-rows, axis=1, kind="stable")[:, :k]     # equal scores: the lowest position first
+        for table in (None, ids):
+            scores, words = ops.getNBestWords(x, k, None if table is None else torch.from_numpy(table).cuda())
+            assert words.dtype == torch.int64
+            assert np.array_equal(words.cpu().numpy(), order if table is None else table[order])
+            assert np.array_equal(scores.cpu().numpy(), np.take_along_axis(rows, order, axis=1))
+        vals, keys = ops.getNBestList(x, k)
+        assert np.array_equal(keys.cpu().numpy().reshape(-1, k), order + np.arange(len(rows))[:, None] * cols)
+    bad = np.full((1, cols), np.nan, np.float32)
+    bad[0, cols // 2] = 2.0                                         # one score, the other places unfilled
+    k = min(3, cols)
+    scores, words = ops.getNBestWords(torch.from_numpy(bad).cuda(), k, torch.from_numpy(ids).cuda())
+    assert words.cpu().tolist() == [[int(ids[cols // 2])] + [int(ids[-1])] * (k - 1)]
+    assert scores.cpu().tolist() == [[2.0] + [-np.inf] * (k - 1)]
