@@ -723,30 +723,25 @@ unsigned next_nonce() {
 }
 
 int absmax_blocks(size_t n4) {
-  size_t per_block = (size_t)kQuantThreads * 8;  // eight 16-byte loads per thread
+  size_t per_block = (size_t)kQuantThreads * 4;  // four 16-byte loads per thread, all in flight
   size_t g = (n4 + per_block - 1) / per_block;
   if(g < 1) g = 1;
   if(g > (size_t)kMaxPartials) g = kMaxPartials;
   return (int)g;
 }
 
-// Quantization of n values whose abs-max the producer left in kAbsmaxSlots slots (measurement id
-// 710 keeps the narrow kernel for large inputs).
-int quantize_with_known_absmax(const float* A, size_t n, const float* absmax_in, int8_t* Aq, hipStream_t st) {
-  if(n >= (1u << 20) && n / 16 <= 0xFFFFFFFFull && kernel_override() % 1000 != 710) {
-    // a 64 KB set per workgroup and step; up to four workgroups' worth of sets per CU at a time
-    const size_t sets = (n / 64 + 255) / 256;
-    size_t blocks = sets;
-    if(blocks > 4 * (size_t)compute_units()) blocks = 4 * (size_t)compute_units();
-    hipLaunchKernelGGL(quantize_a_wide_kernel, dim3((int)blocks), dim3(1024), 0, st, A, (unsigned)(n / 16), absmax_in,
-                       (int)kAbsmaxSlots, Aq, (unsigned)blocks);
-    MH_HIP(hipGetLastError());
-    return MARIAN_HIP_OK;
+// Quantization of n values whose abs-max is that of `partials`.  From 1 M values on workgroups of 1024
+// threads, up to four to a CU; below, 256 threads, so that small inputs spread over more CUs.
+int quantize_with_partials(const float* A, size_t n, const float* partials, int n_partials, int8_t* Aq, hipStream_t st) {
+  if(n >= (1u << 20)) {
+    const size_t sets = (n / 64 + 255) / 256, most = 4 * (size_t)compute_units(), blocks = sets < most ? sets : most;
+    hipLaunchKernelGGL(quantize_a_wide_kernel<1024>, dim3((int)blocks), dim3(1024), 0, st, A, (unsigned)(n / 16), partials,
+                       n_partials, Aq, (unsigned)blocks);
+  } else {
+    const size_t blocks = (n / 64 + 63) / 64;
+    hipLaunchKernelGGL(quantize_a_wide_kernel<256>, dim3((int)blocks), dim3(256), 0, st, A, (unsigned)(n / 16), partials,
+                       n_partials, Aq, (unsigned)blocks);
   }
-  size_t qblocks = (n / 16 + kQuantThreads - 1) / kQuantThreads;
-  if(qblocks > 4096) qblocks = 4096;
-  hipLaunchKernelGGL(quantize_a_kernel, dim3((int)qblocks), dim3(kQuantThreads), 0, st, A, n / 16, absmax_in,
-                     (int)kAbsmaxSlots, Aq, (int)qblocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -896,12 +891,7 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
   hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, A, n / 4,
                      partials, g);
   MH_HIP(hipGetLastError());
-  size_t qblocks = (n / 16 + kQuantThreads - 1) / kQuantThreads;
-  if(qblocks > 4096) qblocks = 4096;
-  hipLaunchKernelGGL(quantize_a_kernel, dim3((int)qblocks), dim3(kQuantThreads), 0, st, A, n / 16,
-                     (const float*)partials, g, Aq, (int)qblocks);
-  MH_HIP(hipGetLastError());
-  return MARIAN_HIP_OK;
+  return quantize_with_partials(A, n, partials, g, Aq, st);
 }
 
 int marian_hip_int8_prepare_b(const float* W, int8_t* Bq, int64_t K, int64_t N, void* workspace,
@@ -1009,7 +999,7 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
     return launch_stream32_auto<kFusedTiled>(a, f, hst, want_tiled ? which - 620 : 0);
   }
   if(absmax_in) {   // quantize with the abs-max the producer left, then the GEMM
-    st = quantize_with_known_absmax(A, (size_t)M * (size_t)K, absmax_in, Aq, hst);
+    st = quantize_with_partials(A, (size_t)M * (size_t)K, absmax_in, kAbsmaxSlots, Aq, hst);
     if(st != MARIAN_HIP_OK) return st;
   } else {
     st = marian_hip_int8_prepare_a(A, Aq, M, K, workspace, workspace_bytes, stream);
@@ -1123,7 +1113,7 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
   }
   // Otherwise the activations are quantized once and every matrix gets its own multiplication.
   if(absmax_in) {
-    int st = quantize_with_known_absmax(A, (size_t)M * (size_t)K, absmax_in, Aq, hst);
+    int st = quantize_with_partials(A, (size_t)M * (size_t)K, absmax_in, kAbsmaxSlots, Aq, hst);
     if(st != MARIAN_HIP_OK) return st;
   } else {
     int st = marian_hip_int8_prepare_a(A, Aq, M, K, workspace, workspace_bytes, stream);

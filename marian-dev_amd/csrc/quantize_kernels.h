@@ -29,31 +29,6 @@ __global__ __launch_bounds__(kQuantThreads) void zero_floats_kernel(float* __res
   for(int i = blockIdx.x * kQuantThreads + threadIdx.x; i < n; i += blocks * kQuantThreads) p[i] = 0.0f;
 }
 
-// Pass 2 of prepareA: reduce the partials, quantize 16 values per thread per step, block 0
-// writes the quantMult tail at byte n.
-__global__ __launch_bounds__(kQuantThreads) void quantize_a_kernel(
-    const float* __restrict__ x, size_t n16, const float* __restrict__ partials, int n_partials,
-    int8_t* __restrict__ out, int blocks) {
-  __shared__ float red[kQuantThreads / kWave];
-  float m = 0.0f;
-  for(int p = threadIdx.x; p < n_partials; p += kQuantThreads) m = fmaxf(m, partials[p]);
-  m = block_max<kQuantThreads / kWave>(m, red);
-  const float qm = quant_mult_from_maxabs(m);
-  const v4f* x4 = reinterpret_cast<const v4f*>(x);
-  uint4* o16 = reinterpret_cast<uint4*>(out);
-  size_t stride = (size_t)blocks * kQuantThreads;
-  for(size_t i = (size_t)blockIdx.x * kQuantThreads + threadIdx.x; i < n16; i += stride) {
-    v4f a = x4[4 * i], b = x4[4 * i + 1], c = x4[4 * i + 2], d = x4[4 * i + 3];
-    uint4 q;
-    q.x = quantize_pack4(a, qm);
-    q.y = quantize_pack4(b, qm);
-    q.z = quantize_pack4(c, qm);
-    q.w = quantize_pack4(d, qm);
-    o16[i] = q;
-  }
-  if(blockIdx.x == 0 && threadIdx.x == 0) *reinterpret_cast<float*>(out + n16 * 16) = qm;
-}
-
 // Small activations: one workgroup computes abs-max and quantizes (one launch instead of two).
 __global__ __launch_bounds__(kSingleBlockThreads) void prepare_a_single_block_kernel(
     const float* __restrict__ x, int n16, int8_t* __restrict__ out) {
@@ -218,20 +193,23 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
   if(g == 0 && tid == 0) *reinterpret_cast<float*>(out + (size_t)n16 * 16) = qm;
 }
 
-// Quantization alone for large inputs whose abs-max is known (left in `partials` by the kernel that
+// Pass 2 of prepareA, and quantization alone where the abs-max is known (left in `partials` by the kernel that
 // produced x): the memory access pattern of the one-pass kernel above - a quad of lanes reads 64
 // contiguous bytes per load, four loads in flight per thread (eight while the next set is on its
 // way), the packed bytes take a turn through LDS so that a wave stores 1 KB of contiguous output -
-// without its exchange.  A set = 256 quads = 64 KB of input per workgroup and step.
-__global__ __launch_bounds__(1024) void quantize_a_wide_kernel(const float* __restrict__ x, unsigned n16,
-                                                               const float* __restrict__ partials, int n_partials,
-                                                               int8_t* __restrict__ out, unsigned blocks) {
-  __shared__ float red[1024 / kWave];
-  __shared__ __attribute__((aligned(16))) uint32_t turn[1024 * 4];   // 16 bytes per thread
+// without its exchange.  A set = THREADS / 4 quads = 64 THREADS bytes of input per workgroup and step.
+// n_partials: 1 .. kAbsmaxSlots, all requested at once, behind the first values.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void quantize_a_wide_kernel(const float* __restrict__ x, unsigned n16,
+                                                                  const float* __restrict__ partials, int n_partials,
+                                                                  int8_t* __restrict__ out, unsigned blocks) {
+  __shared__ float red[THREADS / kWave];
+  __shared__ __attribute__((aligned(16))) uint32_t turn[THREADS * 4];   // 16 bytes per thread
   const int tid = threadIdx.x, quad = tid / 4, qlane = tid % 4;
-  const unsigned n_sets = (n16 / 4 + 255) / 256;
+  constexpr unsigned kQuads = THREADS / 4;
+  const unsigned n_sets = (n16 / 4 + kQuads - 1) / kQuads;
   auto load_set = [&](unsigned set, v4f (&v)[4]) {
-    const unsigned q = set * 256u + (unsigned)quad;
+    const unsigned q = set * kQuads + (unsigned)quad;
     const unsigned qc = 4u * q < n16 ? q : 0u;   // (n16 is a multiple of four: whole quads)
     const char* src = reinterpret_cast<const char*>(x) + (size_t)qc * 256 + qlane * 16;
 #pragma unroll
@@ -241,9 +219,12 @@ __global__ __launch_bounds__(1024) void quantize_a_wide_kernel(const float* __re
   unsigned set = blockIdx.x;
   v4f vals[4];
   if(set < n_sets) load_set(set, vals);
-  float m = 0.0f;
-  for(int p = tid; p < n_partials; p += 1024) m = fmaxf(m, partials[p]);
-  m = block_max<1024 / kWave>(m, red);
+  float pm[kAbsmaxSlots / THREADS], m = 0.0f;
+#pragma unroll
+  for(int i = 0; i < kAbsmaxSlots / THREADS; ++i) pm[i] = partials[min(tid + i * THREADS, n_partials - 1)];
+#pragma unroll
+  for(int i = 0; i < kAbsmaxSlots / THREADS; ++i) m = fmaxf(m, pm[i]);
+  m = block_max<THREADS / kWave>(m, red);
   const float qm = quant_mult_from_maxabs(m);
   const bool finite = qm < __builtin_inff();
   for(; set < n_sets; set += blocks) {
@@ -251,7 +232,7 @@ __global__ __launch_bounds__(1024) void quantize_a_wide_kernel(const float* __re
 #pragma unroll
     for(int e = 0; e < 4; ++e) cur[e] = vals[e];
     if(set + blocks < n_sets) load_set(set + blocks, vals);
-    const unsigned q = set * 256u + (unsigned)quad;
+    const unsigned q = set * kQuads + (unsigned)quad;
     if(4u * q < n16) {
       // (the four lanes of a quad sit in one wave, whose LDS operations execute in order)
 #pragma unroll
@@ -274,24 +255,24 @@ __global__ __launch_bounds__(256) void quantize_b_transpose_kernel(
   // [n][k / 4] as packed dwords, 17 dwords per row: the 64 lanes of a wave (consecutive n, one k
   // group) hit every bank twice, the minimum for 64 lanes on 32 banks
   __shared__ uint32_t tile[64][17];
-  float m = 0.0f;
-  for(int p = threadIdx.x; p < n_partials; p += 256) m = fmaxf(m, partials[p]);
-  m = block_max<256 / kWave>(m, red);
-  const float qm = quant_mult_from_maxabs(m);
-
   const int n0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
   const int tn = threadIdx.x % 64, tk = threadIdx.x / 64;  // wave tk takes k rows 16*tk .. 16*tk+15
-  const int n_in = n0 + tn;
+  // the tile and the partials are requested together (K % 64 == 0: the k rows of a tile are all inside;
+  // columns past N read the last one and are not written)
+  const float* w = W + (size_t)(k0 + tk * 16) * N + min(n0 + tn, N - 1);
+  float v[16], pm[kMaxPartials / 256];
 #pragma unroll
-  for(int g = 0; g < 4; ++g) {
-    const int kk = tk * 16 + g * 4;   // four consecutive k of column n: one packed dword
-    v4f v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    if(n_in < N) {   // (K % 64 == 0: the k rows of a tile are all inside)
-      const float* w = W + (size_t)(k0 + kk) * N + n_in;
-      v = v4f{w[0], w[(size_t)N], w[2 * (size_t)N], w[3 * (size_t)N]};
-    }
-    tile[tn][kk / 4] = quantize_pack4(v, qm);
-  }
+  for(int k = 0; k < 16; ++k) v[k] = w[(size_t)k * N];
+#pragma unroll
+  for(int i = 0; i < kMaxPartials / 256; ++i) pm[i] = partials[min((int)threadIdx.x + i * 256, n_partials - 1)];
+  float m = 0.0f;
+#pragma unroll
+  for(int i = 0; i < kMaxPartials / 256; ++i) m = fmaxf(m, pm[i]);
+  m = block_max<256 / kWave>(m, red);
+  const float qm = quant_mult_from_maxabs(m);
+#pragma unroll
+  for(int g = 0; g < 4; ++g)   // four consecutive k of column n: one packed dword
+    tile[tn][tk * 4 + g] = quantize_pack4(v4f{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}, qm);
   __syncthreads();
   // 64 columns (n) x four 16-byte chunks (k): two neighbouring threads write the two halves of a
   // column's sub-step, a wave 32 columns of one sub-step (1 KB of consecutive memory)
