@@ -184,6 +184,31 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
                                        size_t workspace_bytes, void* stream);
 
 /*
+ * The layer norm in front of a multiplication, done by the kernel that multiplies: for the few hypotheses of a
+ * decoding step the launch of the norm costs more than its work.  x = layer norm of (A + add), reference
+ * src/models/transformer.h:184-218 (post-processing "dan": skip connection, then layer norm), and the
+ * multiplications of marian_hip_int8_affine_f32_grouped on x - the bits of the separate calls
+ * (marian_hip_layer_norm, then the chained or grouped call).
+ *   norm: HOST struct, read during the call; add [M x K], gamma [K], beta [K] and out [M x K], which receives x,
+ *     16-byte aligned; out overlaps neither A nor add (MARIAN_HIP_ERR_ALIAS).
+ *   M <= 8, K <= 1024, K % 64 == 0, otherwise MARIAN_HIP_ERR_SHAPE.
+ *   absmax_out: as for marian_hip_int8_affine_f32_chained, with n_groups == 1; or NULL.
+ */
+#define MARIAN_HIP_NORM_MAX_ROWS 8
+#define MARIAN_HIP_NORM_MAX_COLS 1024
+typedef struct marian_hip_norm_input {
+  const float* add;
+  const float* gamma;
+  const float* beta;
+  float* out;
+  float eps;
+} marian_hip_norm_input;
+int marian_hip_int8_affine_f32_normed(const float* A, const marian_hip_norm_input* norm, int64_t n_groups,
+                                      const int8_t* const* Bq, const float* const* bias, float* const* out,
+                                      const int64_t* N, int64_t M, int64_t K, float scale, int relu,
+                                      float* absmax_out, void* stream);
+
+/*
  * The projections in front of an attention and the attention itself, for ONE new target position
  * per query row, in one launch (reference src/models/transformer.h:279-348, MultiHead: q =
  * affine(input, Wq, bq) and, for self-attention, k / v = affine(input, Wk / Wv, ..), the head
@@ -222,6 +247,12 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
                                    int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
                                    float* out, const float* absmax_in, float* absmax_out, void* workspace,
                                    size_t workspace_bytes, void* stream);
+/* The same with the layer norm in front (M <= 8; x goes to norm->out, its quantized form nowhere). */
+int marian_hip_int8_proj_attention_normed(const float* A, const marian_hip_norm_input* norm, int64_t n_proj,
+                                          const int8_t* const* Bq, const float* const* bias, float* const* proj_out,
+                                          int64_t M, int64_t K, int64_t heads, float* k_cache, float* v_cache,
+                                          int64_t batchKV, int64_t len, int64_t kv_capacity, const float* mask,
+                                          int64_t n_masks, float att_scale, float* out, float* absmax_out, void* stream);
 
 /*
  * marian_hip_int8_affine_f32 for callers that cannot allocate and have no workspace to pass: code

@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <initializer_list>
 
 #include "../../include/marian_hip_int8.h"
 
@@ -25,6 +26,21 @@ inline int current_device(int* dev) {
   const hipError_t e = hipGetDevice(dev);
   if(e != hipSuccess) return record_hip_error((int)e);
   if(*dev < 0 || *dev >= kMaxDevices) return MARIAN_HIP_ERR_RANGE;
+  return MARIAN_HIP_OK;
+}
+
+// What the kernels that normalize their input ask of it: few, short rows, whole vectors, an output that no
+// workgroup still reads.  (A: the M x K values the norm starts from.)
+inline int norm_input_check(const marian_hip_norm_input* n, const float* A, int64_t M, int64_t K) {
+  if(M > MARIAN_HIP_NORM_MAX_ROWS || K > MARIAN_HIP_NORM_MAX_COLS || K % 64 != 0) return MARIAN_HIP_ERR_SHAPE;
+  if(!n->add || !n->gamma || !n->beta || !n->out) return MARIAN_HIP_ERR_NULL;
+  for(const float* p : {n->add, n->gamma, n->beta, static_cast<const float*>(n->out)})
+    if(reinterpret_cast<uintptr_t>(p) % 16 != 0) return MARIAN_HIP_ERR_ALIGN;
+  const uintptr_t out = reinterpret_cast<uintptr_t>(n->out), bytes = (uintptr_t)M * (uintptr_t)K * sizeof(float);
+  for(const float* p : {A, n->add}) {
+    const uintptr_t in = reinterpret_cast<uintptr_t>(p);
+    if(in < out + bytes && out < in + bytes) return MARIAN_HIP_ERR_ALIAS;
+  }
   return MARIAN_HIP_OK;
 }
 

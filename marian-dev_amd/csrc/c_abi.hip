@@ -372,7 +372,7 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
       a2.absmax_out = nullptr;
       a2.blocks_x = groups->table.block0[groups->table.n];
       hipLaunchKernelGGL(gkernel, dim3(groups->table.block0[groups->table.n], m_tiles), dim3(Cfg::kThreads), lds, st,
-                         a2, f.A, f.aq_out, f.partials, f.n_partials, groups->table);
+                         a2, f.A, f.aq_out, f.partials, f.n_partials, groups->table, NoNorm());
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
     }
@@ -387,7 +387,35 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
     else a2.absmax_out = nullptr;
   }
   hipLaunchKernelGGL(kernel, dim3(blocks, m_tiles), dim3(Cfg::kThreads), lds, st, a2, f.A,
-                     f.aq_out, f.partials, f.n_partials, NoGroups());
+                     f.aq_out, f.partials, f.n_partials, NoGroups(), NoNorm());
+  MH_HIP(hipGetLastError());
+  return MARIAN_HIP_OK;
+}
+
+// The form that normalizes its input: one or several matrices, 16-row workgroups.
+template <int WN, int KW, int PW>
+int launch_normed(const GemmArgs& a, const float* A, const NormInput& n, const GroupTable* groups, hipStream_t st) {
+  using Cfg = Stream32Cfg<1, WN, KW, PW>;
+  int lds = Cfg::kStageBytes;
+  if(lds < stream32_fused_lds_bytes(1, a.K)) lds = stream32_fused_lds_bytes(1, a.K);
+  if(lds < Cfg::kReduceBytes) lds = Cfg::kReduceBytes;
+  static_assert(Cfg::kReduceBytes <= 48 * 1024 && Cfg::kStageBytes <= 48 * 1024 && 32 * kNormMaxCols <= 48 * 1024, "default LDS limit");
+  GemmArgs a2 = a;
+  a2.blocks_y = 1;
+  a2.blocks_x = groups ? groups->block0[groups->n] : (a.n_out + Cfg::kColsPerBlock - 1) / Cfg::kColsPerBlock;
+  if(groups) {
+    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, GroupTable, NormInput>;
+    hipLaunchKernelGGL(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, a2, A, static_cast<int8_t*>(nullptr),
+                       static_cast<const float*>(nullptr), 0, *groups, n);
+  } else {
+    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, NoGroups, NormInput>;
+    if(a.absmax_out) {   // one slot per wave
+      if((long long)a2.blocks_x * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
+      else a2.absmax_out = nullptr;
+    }
+    hipLaunchKernelGGL(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, a2, A, static_cast<int8_t*>(nullptr),
+                       static_cast<const float*>(nullptr), 0, NoGroups(), n);
+  }
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -1043,6 +1071,73 @@ int marian_hip_int8_affine_f32_chained(const float* A, int8_t* Aq, const int8_t*
 }
 
 
+// The matrices that have columns, and where their column blocks of `cols` columns start.
+static GroupTable group_table(int64_t n_groups, const int8_t* const* Bq, const float* const* bias, float* const* out,
+                              const int64_t* N, int cols) {
+  GroupTable t;
+  t.n = 0;
+  t.block0[0] = 0;
+  for(int64_t g = 0; g < n_groups; ++g) {
+    if(N[g] == 0) continue;
+    const int i = t.n++;
+    t.Bq[i] = Bq[g];
+    t.bias[i] = bias ? bias[g] : nullptr;
+    t.out[i] = out[g];
+    t.N[i] = (int)N[g];
+    t.block0[i + 1] = t.block0[i] + (int)((N[g] + cols - 1) / cols);
+  }
+  for(int i = t.n; i < kMaxGroups; ++i) {   // unused entries: never selected
+    t.Bq[i] = nullptr; t.bias[i] = nullptr; t.out[i] = nullptr; t.N[i] = 0;
+    t.block0[i + 1] = t.block0[t.n];
+  }
+  return t;
+}
+
+int marian_hip_int8_affine_f32_normed(const float* A, const marian_hip_norm_input* norm, int64_t n_groups,
+                                      const int8_t* const* Bq, const float* const* bias, float* const* out,
+                                      const int64_t* N, int64_t M, int64_t K, float scale, int relu,
+                                      float* absmax_out, void* stream) {
+  if(n_groups < 1 || n_groups > kMaxGroups || (absmax_out && n_groups != 1)) return MARIAN_HIP_ERR_SHAPE;
+  if(!norm || !Bq || !out || !N) return MARIAN_HIP_ERR_NULL;
+  int64_t blocks32 = 0;
+  for(int64_t g = 0; g < n_groups; ++g) {
+    // (the multiplication reads no quantized activations: the weights stand in for them in the check)
+    const int st = check_gemm(Bq[g], Bq[g], out[g], bias ? bias[g] : nullptr, nullptr, 0, M, K, N[g]);
+    if(st != MARIAN_HIP_OK) return st;
+    blocks32 += (N[g] + 31) / 32;
+  }
+  if(M == 0) return MARIAN_HIP_OK;
+  if(blocks32 == 0) return MARIAN_HIP_ERR_SHAPE;   // (nobody would write the norm)
+  if(!A) return MARIAN_HIP_ERR_NULL;
+  if(!aligned(A, 16) || (absmax_out && !aligned(absmax_out, 4))) return MARIAN_HIP_ERR_ALIGN;
+  const int nst = norm_input_check(norm, A, M, K);
+  if(nst != MARIAN_HIP_OK) return nst;
+  const NormInput n{norm->add, norm->gamma, norm->beta, norm->out, norm->eps};
+  hipStream_t hst = reinterpret_cast<hipStream_t>(stream);
+  // the widest K split (most loads in flight per weight row) that stays within one workgroup per CU
+  int kw = 8;
+  while(kw > 1 && ((blocks32 * kw + 7) / 8 > compute_units() || K / 32 < kw)) kw >>= 1;
+  const int need = ((int)K / 32 + kw - 1) / kw;
+  const GroupTable table = group_table(n_groups, Bq, bias, out, N, 32 * (8 / kw));
+  const GroupTable* groups = table.n > 1 ? &table : nullptr;
+  GemmArgs a;
+  a.Aq = nullptr; a.Bq = table.Bq[0]; a.bias = table.bias[0]; a.idx = nullptr; a.out = table.out[0];
+  a.M = (int)M; a.K = (int)K; a.N = table.N[0]; a.n_out = table.N[0];
+  a.scale = scale; a.relu = relu ? 1 : 0; a.dump = 0;
+  a.absmax_out = absmax_out;
+#ifdef MARIAN_HIP_TUNING
+  a.prof = g_prof.load(std::memory_order_relaxed);
+#endif
+  t_absmax_written = false;
+  int st;
+  if(kw == 8) st = need <= 2 ? launch_normed<1, 8, 2>(a, A, n, groups, hst) : launch_normed<1, 8, 4>(a, A, n, groups, hst);
+  else if(kw == 4) st = need <= 4 ? launch_normed<2, 4, 4>(a, A, n, groups, hst) : launch_normed<2, 4, 8>(a, A, n, groups, hst);
+  else if(kw == 2) st = launch_normed<4, 2, 8>(a, A, n, groups, hst);
+  else st = launch_normed<8, 1, 8>(a, A, n, groups, hst);
+  if(st != MARIAN_HIP_OK || !absmax_out || t_absmax_written) return st;
+  return absmax_after(out[0], M, N[0], absmax_out, hst);
+}
+
 int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_groups,
                                        const int8_t* const* Bq, const float* const* bias,
                                        float* const* out, const int64_t* N, int64_t M, int64_t K,
@@ -1073,21 +1168,7 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
   if(one_launch) {
     GroupLaunch gl;
     gl.cols = 32 * (8 / plan.kw);
-    gl.table.n = 0;
-    gl.table.block0[0] = 0;
-    for(int64_t g = 0; g < n_groups; ++g) {
-      if(N[g] == 0) continue;
-      const int i = gl.table.n++;
-      gl.table.Bq[i] = Bq[g];
-      gl.table.bias[i] = bias ? bias[g] : nullptr;
-      gl.table.out[i] = out[g];
-      gl.table.N[i] = (int)N[g];
-      gl.table.block0[i + 1] = gl.table.block0[i] + (int)((N[g] + gl.cols - 1) / gl.cols);
-    }
-    for(int i = gl.table.n; i < kMaxGroups; ++i) {   // unused entries: never selected
-      gl.table.Bq[i] = nullptr; gl.table.bias[i] = nullptr; gl.table.out[i] = nullptr; gl.table.N[i] = 0;
-      gl.table.block0[i + 1] = gl.table.block0[gl.table.n];
-    }
+    gl.table = group_table(n_groups, Bq, bias, out, N, gl.cols);
     GemmArgs a;
     a.Aq = Aq; a.Bq = gl.table.Bq[0]; a.bias = gl.table.bias[0]; a.idx = nullptr; a.out = gl.table.out[0];
     a.M = (int)M; a.K = (int)K; a.N = gl.table.N[0]; a.n_out = gl.table.N[0];

@@ -17,6 +17,7 @@
 #include "abi_common.h"
 #include "attention_rows_kernel.h"
 #include "int8_common.h"
+#include "layer_norm_row.h"
 #include "nbest_plan.h"
 #include "quantize_common.h"
 
@@ -26,26 +27,6 @@ namespace {
 
 constexpr int64_t kMaxElemsOps = 2147483647LL;
 
-// Sum over each group of 16 consecutive lanes, left in all 16 of them (four DPP steps: the two
-// lane swaps within a quad, then the mirror within half a row and within the row).
-__device__ __forceinline__ float row16_sum(float v) {
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));  // row_half_mirror
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, false));  // row_mirror
-  return v;
-}
-// Sum over the wave, the same value in all lanes: within the rows of 16 lanes, then across them
-// with the two row-broadcast DPP steps (rows 1 and 3 take in the last lane of the row before them,
-// then rows 2 and 3 the last lane of row 1), which leaves the total in lane 63, read from there as
-// a scalar.  No step goes through the LDS crossbar (a lane exchange there costs ten times a DPP
-// step).  All lanes of the wave must be active.
-__device__ __forceinline__ float wave_sum(float v) {
-  v = row16_sum(v);
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xA, 0xF, false));   // row_bcast:15
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));   // row_bcast:31
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
 // Maximum over the wave, the same value in all lanes (`t > v ? t : v` at every step): the same
 // steps.
 __device__ __forceinline__ float wave_maxf(float v) {
@@ -208,7 +189,7 @@ __global__ __launch_bounds__(MANY ? 256 : 64) void layer_norm_wave_kernel(const 
                                                              const float* __restrict__ beta, int beta_stride,
                                                              float* out, int cols, float eps,
                                                              float* __restrict__ absmax_out, int blocks, int rows) {
-  constexpr int VPL = 4, WAVES = MANY ? 4 : 1;
+  constexpr int VPL = kNormVecs, WAVES = MANY ? 4 : 1;
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, cols4 = cols / 4;
   const v4f zero = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   v4f v[VPL], t[VPL], gm[VPL], bt[VPL];
@@ -242,39 +223,11 @@ __global__ __launch_bounds__(MANY ? 256 : 64) void layer_norm_wave_kernel(const 
   }
   float omax = 0.0f;
   for(int row = (int)blockIdx.x * WAVES + wave; row < rows; row += blocks * WAVES) {
-    float sum = 0.0f;
-#pragma unroll
-    for(int j = 0; j < VPL; ++j) {
-      if(add) v[j] = v4f{v[j].x + t[j].x, v[j].y + t[j].y, v[j].z + t[j].z, v[j].w + t[j].w};
-      if(j * 64 + lane < cols4) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
-    }
-    const float mean = wave_sum(sum) / (float)cols;
-    float sq = 0.0f;
-#pragma unroll
-    for(int j = 0; j < VPL; ++j) {
-      if(j * 64 + lane < cols4) {
-        const float d0 = v[j].x - mean, d1 = v[j].y - mean, d2 = v[j].z - mean, d3 = v[j].w - mean;
-        sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
-      }
-    }
-    const float sigma = sqrtf(wave_sum(sq) / (float)cols + eps);
+    omax = fmaxf(omax, normalize_row(v, t, add != nullptr, gm, bt, beta != nullptr, cols, eps));
     v4f* y = reinterpret_cast<v4f*>(out + (size_t)row * cols);
 #pragma unroll
-    for(int j = 0; j < VPL; ++j) {
-      const int i = j * 64 + lane;
-      if(i < cols4) {
-        float r[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-        const float g[4] = {gm[j].x, gm[j].y, gm[j].z, gm[j].w}, b[4] = {bt[j].x, bt[j].y, bt[j].z, bt[j].w};
-#pragma unroll
-        for(int e = 0; e < 4; ++e) {
-          float o = g[e] * ((r[e] - mean) / sigma);
-          if(beta) o = o + b[e];
-          r[e] = o;
-          omax = fmaxf(omax, fabsf(o));
-        }
-        y[i] = v4f{r[0], r[1], r[2], r[3]};
-      }
-    }
+    for(int j = 0; j < VPL; ++j)
+      if(j * 64 + lane < cols4) y[j * 64 + lane] = v[j];
     if constexpr(MANY) {
       if(row + blocks * WAVES < rows) load_row((size_t)(row + blocks * WAVES), v, t);
     } else {
@@ -909,6 +862,7 @@ struct ProjAttentionArgs {
   // With it (and sentences two or one to a workgroup, len <= kProjStageLen): the keys and values of
   // the workgroup's sentences are read once, into LDS, and every hypothesis' wave takes them from there.
   int stage_kv;
+  NormInput norm;           // (NORM) A is what the layer norm in front of the projections reads
 };
 
 // Entry g of one of the argument arrays, g differing between the threads: selected from the three
@@ -1093,7 +1047,10 @@ __global__ __launch_bounds__(256) void attention_shared_kernel(const float* __re
 // NPROJ: 3 (q, k_new, v_new: self-attention, the new key/value row is appended to the caches) or
 // 1 (q only: attention over caches that are complete, e.g. the encoder's).  R: input rows per
 // workgroup, 8 (a wave per row in the attention).
-template <int NPROJ, int R, int SEGS, int PASSES>
+// NORM: the projections' input is the layer norm of A + norm.add, up to kNormMaxRows rows: every workgroup
+// normalizes all of them, a wave each, while its weights are on their way (a launch of its own for the norm
+// took 3.5 us of GPU and 4 of host time).
+template <int NPROJ, int R, int SEGS, int PASSES, bool NORM = false>
 __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttentionArgs p) {
   static_assert(R == 8, "one wave per row in the attention");
   constexpr bool STAGED = SEGS > 0;
@@ -1120,15 +1077,19 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
   // ---- everything this workgroup will need is requested now, in the order of its use (a wave's
   //      loads complete in the order of their issue): abs-max slots, the input rows, weights, the
   //      mask value, the quantization multipliers of the weights, bias ----
-  float pm[kAbsmaxSlots / kProjThreads];
-#pragma unroll
-  for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) pm[i] = p.partials[min(tid + i * kProjThreads, p.n_partials - 1)];
+  float pm[NORM ? 1 : kAbsmaxSlots / kProjThreads];
   // a quad of lanes takes four consecutive 16-value groups of one row: 64 contiguous bytes per load
   const int grp = (tid / 4) * 4, qlane = tid % 4;
   const int r_in = grp / (2 * S), c16 = grp % (2 * S);
-  const bool has_in = r_in < R;
+  const bool has_in = !NORM && r_in < R;
   v4f in[4];
-  {
+  NormRow nr;
+  if constexpr(NORM) {
+    nr.load(p.A, p.norm, M, K);
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
+#pragma unroll
+    for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) pm[i] = p.partials[min(tid + i * kProjThreads, p.n_partials - 1)];
     const int m = min(row_of(min(r_in, R - 1)), M - 1);
     const float* src = p.A + (size_t)m * (size_t)K + (size_t)c16 * 16 + qlane * 4;
 #pragma unroll
@@ -1154,7 +1115,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
     if(mask_row >= p.n_masks) mask_row %= p.n_masks;
     mk = p.mask + (size_t)mask_row * p.len;
   }
-  const float mk0 = *(mk ? mk + min(lane, p.len - 1) : p.partials);   // (the latter not looked at)
+  const float mk0 = *(mk ? mk + min(lane, p.len - 1) : p.A);   // (the latter not looked at)
   float bqm[NPROJ];
 #pragma unroll
   for(int g = 0; g < NPROJ; ++g) bqm[g] = tail_quant_mult(p.Bq[g], (size_t)K * (size_t)N);
@@ -1172,8 +1133,12 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
 
   // ---- 1, 2: abs-max, quantize into LDS ----
   float amax = 0.0f;
+  if constexpr(NORM) {
+    amax = nr.normalize(p.norm, K);
+  } else {
 #pragma unroll
-  for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) amax = fmaxf(amax, pm[i]);
+    for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) amax = fmaxf(amax, pm[i]);
+  }
   amax = block_max<kProjThreads / 64>(amax, red);
   // The keys and values are asked for last - a wave's loads complete in the order of their issue,
   // and they are needed last - and only now: in front of the abs-max values they would delay them.
@@ -1206,6 +1171,14 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
       *reinterpret_cast<uint32_t*>(a_lds + sw * 16 + qlane * 4) = q[e];
       if(p.aq_out && h == 0 && m < M)
         *reinterpret_cast<uint32_t*>(p.aq_out + (size_t)m * (size_t)K + (size_t)(c16 + e) * 16 + qlane * 4) = q[e];
+    }
+  }
+  if constexpr(NORM) {   // wave w holds row w: quantized where this workgroup multiplies it, written out by one workgroup
+    const int row = __builtin_amdgcn_readfirstlane(wave);
+    if(row < M) {
+      for(int r = 0; r < R; ++r)
+        if(row_of(r) == row) nr.quantize(a_lds, r, K, aqm, proj_row_key);
+      if(h == 0 && blockIdx.y == 0) nr.store(p.norm, row, K);
     }
   }
   if(p.aq_out && h == 0 && blockIdx.y == 0 && tid == 0) *reinterpret_cast<float*>(p.aq_out + (size_t)M * K) = aqm;
@@ -2432,25 +2405,25 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
   return MARIAN_HIP_OK;
 }
 
-int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, const int8_t* const* Bq,
-                                   const float* const* bias, float* const* proj_out, int64_t M, int64_t K,
-                                   int64_t heads, float* k_cache, float* v_cache, int64_t batchKV, int64_t len,
-                                   int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
-                                   float* out, const float* absmax_in, float* absmax_out, void* workspace,
-                                   size_t workspace_bytes, void* stream) {
+static int proj_attention(const float* A, const marian_hip_norm_input* norm, int8_t* Aq, int64_t n_proj, const int8_t* const* Bq,
+                          const float* const* bias, float* const* proj_out, int64_t M, int64_t K,
+                          int64_t heads, float* k_cache, float* v_cache, int64_t batchKV, int64_t len,
+                          int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
+                          float* out, const float* absmax_in, float* absmax_out, void* workspace,
+                          size_t workspace_bytes, void* stream) {
   if(n_proj != 1 && n_proj != 3) return MARIAN_HIP_ERR_SHAPE;
   if(M < 0 || K <= 0 || heads <= 0 || (K % 128) != 0 || K > kProjMaxK) return MARIAN_HIP_ERR_SHAPE;
   if(len <= 0 || len > kProjMaxLen || kv_capacity < len || batchKV <= 0) return MARIAN_HIP_ERR_SHAPE;
   if(mask && n_masks <= 0) return MARIAN_HIP_ERR_SHAPE;
   if(M == 0) return MARIAN_HIP_OK;
-  if(!A || !Aq || !Bq || !k_cache || !v_cache || !out) return MARIAN_HIP_ERR_NULL;
+  if(!A || (!Aq && !norm) || !Bq || !k_cache || !v_cache || !out) return MARIAN_HIP_ERR_NULL;
   if(M * heads > kMaxElemsOps / 64 || batchKV * kv_capacity > kMaxElemsOps / 64 || M * K > kMaxElemsOps ||
      K * heads * 64 > kMaxElemsOps || n_masks > 2147483647LL)
     return MARIAN_HIP_ERR_RANGE;
   // the self-attention form appends to the caches: every query row needs an entry of its own
   if(n_proj == 3 && batchKV != M * heads) return MARIAN_HIP_ERR_SHAPE;
   if(absmax_out && M * heads > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
-  if(!aligned16(A) || !aligned16(Aq) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out))
+  if(!aligned16(A) || (Aq && !aligned16(Aq)) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out))
     return MARIAN_HIP_ERR_ALIGN;
   if((mask && !aligned4(mask)) || (absmax_in && !aligned4(absmax_in)) || (absmax_out && !aligned4(absmax_out)))
     return MARIAN_HIP_ERR_ALIGN;
@@ -2468,7 +2441,15 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   p.A = A; p.aq_out = Aq;
-  if(absmax_in) {
+  p.norm = NormInput{nullptr, nullptr, nullptr, nullptr, 0.0f};
+  p.partials = nullptr;
+  p.n_partials = 0;
+  if(norm) {
+    static_assert(MARIAN_HIP_NORM_MAX_ROWS == kNormMaxRows && MARIAN_HIP_NORM_MAX_COLS == kNormMaxCols, "limits");
+    const int nst = norm_input_check(norm, A, M, K);
+    if(nst != MARIAN_HIP_OK) return nst;
+    p.norm = NormInput{norm->add, norm->gamma, norm->beta, norm->out, norm->eps};
+  } else if(absmax_in) {
     p.partials = absmax_in;
     p.n_partials = kAbsmaxSlots;
   } else {   // nobody left the abs-max of the input: a launch for it
@@ -2500,12 +2481,15 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
       const void* staged[] = {
           reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 1>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 2>),
           reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 3>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 1>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 2>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 3>)};
+          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 2>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 3>),
+          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 1, true>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 2, true>),
+          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 3, true>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 1, true>),
+          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 2, true>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 3, true>)};
       for(const void* f : staged) MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kProjMaxLds));
-      MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0>),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-      MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0>),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
+      const void* unstaged[] = {
+          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0>),
+          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, true>)};
+      for(const void* f : unstaged) MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
       lds_done.fetch_or(1ull << dev, std::memory_order_release);
     }
   }
@@ -2518,8 +2502,11 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
   if(plan.blocks_y > 65535) return MARIAN_HIP_ERR_RANGE;
   if(plan.stage) lds += (size_t)(2 << plan.shift) * (size_t)len * 256;
   const dim3 grid((unsigned)heads, (unsigned)plan.blocks_y);
-#define MH_PA(NP, SEGS, PASSES) \
-  hipLaunchKernelGGL((proj_attention_kernel<NP, R, SEGS, PASSES>), grid, dim3(kProjThreads), lds, st, p)
+#define MH_PA(NP, SEGS, PASSES)                                                                                          \
+  do {                                                                                                                   \
+    if(norm) hipLaunchKernelGGL((proj_attention_kernel<NP, R, SEGS, PASSES, true>), grid, dim3(kProjThreads), lds, st, p); \
+    else hipLaunchKernelGGL((proj_attention_kernel<NP, R, SEGS, PASSES>), grid, dim3(kProjThreads), lds, st, p);           \
+  } while(0)
   if(n_proj == 3) MH_PA(3, 0, 0);
   else if(!p.stage_kv) MH_PA(1, 0, 0);
   else {
@@ -2537,6 +2524,26 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
 #undef MH_PA
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
+}
+
+int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, const int8_t* const* Bq,
+                                   const float* const* bias, float* const* proj_out, int64_t M, int64_t K,
+                                   int64_t heads, float* k_cache, float* v_cache, int64_t batchKV, int64_t len,
+                                   int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
+                                   float* out, const float* absmax_in, float* absmax_out, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
+  return proj_attention(A, nullptr, Aq, n_proj, Bq, bias, proj_out, M, K, heads, k_cache, v_cache, batchKV, len, kv_capacity, mask,
+                        n_masks, att_scale, out, absmax_in, absmax_out, workspace, workspace_bytes, stream);
+}
+
+int marian_hip_int8_proj_attention_normed(const float* A, const marian_hip_norm_input* norm, int64_t n_proj, const int8_t* const* Bq,
+                                          const float* const* bias, float* const* proj_out, int64_t M, int64_t K,
+                                          int64_t heads, float* k_cache, float* v_cache, int64_t batchKV, int64_t len,
+                                          int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
+                                          float* out, float* absmax_out, void* stream) {
+  if(!norm) return MARIAN_HIP_ERR_NULL;
+  return proj_attention(A, norm, nullptr, n_proj, Bq, bias, proj_out, M, K, heads, k_cache, v_cache, batchKV, len, kv_capacity, mask,
+                        n_masks, att_scale, out, nullptr, absmax_out, nullptr, 0, stream);
 }
 
 // Rows of up to kNbestWaveCols values: a wave each; longer ones: 1024 threads each.

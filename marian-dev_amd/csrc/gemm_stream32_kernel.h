@@ -18,11 +18,14 @@
 // MODE kFusedTiled: for activations too large for that.  A separate small kernel leaves per-
 // workgroup abs-max values; this kernel reduces them, and quantizes its own 32 * MT32 rows chunk
 // by chunk on the way into LDS (the workgroups of column 0 also write them out).
+// MODE kFusedNorm: up to eight rows, which are the layer norm of the input (plus a skip connection): a wave
+// normalizes a row in registers, all workgroups all rows, and the quantization goes on from there.
 #pragma once
 
 #include <type_traits>
 
 #include "int8_common.h"
+#include "layer_norm_row.h"
 #include "quantize_kernels.h"
 
 namespace marian_hip {
@@ -30,7 +33,8 @@ namespace marian_hip {
 typedef int v16i_s __attribute__((ext_vector_type(16)));
 
 constexpr int kFusedMaxElems = 32768;   // fp32 activations a workgroup holds in registers
-constexpr int kPrequant = 0, kFusedAll = 1, kFusedTiled = 2;            // MODE
+constexpr int kPrequant = 0, kFusedAll = 1, kFusedTiled = 2, kFusedNorm = 3;            // MODE
+struct NoNorm {};
 
 // The 32 rows of 16-byte chunk c16 of the activations are stored XOR-permuted by this key.  Any key
 // leaves a fragment read (32 consecutive slots, permuted) free of bank conflicts; this one makes
@@ -82,15 +86,17 @@ struct NoGroups {};
 // quantizing per workgroup and twice the workgroups, for calls that would otherwise leave most
 // CUs idle.  With ROWS < M the kFusedAll form still takes the abs-max over all of A in every
 // workgroup and quantizes only its own rows.
-template <int MT32, int WN, int KW, int PW, int MODE, int NG = 4, int ROWS = 32 * MT32, typename GROUPS = NoGroups>
+template <int MT32, int WN, int KW, int PW, int MODE, int NG = 4, int ROWS = 32 * MT32, typename GROUPS = NoGroups, typename NORMED = NoNorm>
 __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs args,
                                                                         const float* A,
                                                                         int8_t* aq_out,
                                                                         const float* partials,
-                                                                        int n_partials, GROUPS groups) {
+                                                                        int n_partials, GROUPS groups, NORMED norm) {
   using Cfg = Stream32Cfg<MT32, WN, KW, PW>;
   constexpr bool GROUPED = std::is_same<GROUPS, GroupTable>::value;
-  static_assert(!GROUPED || MODE == kFusedTiled, "several weight matrices: quantize-on-stage form only");
+  constexpr bool NORM = MODE == kFusedNorm;
+  static_assert(!GROUPED || MODE == kFusedTiled || NORM, "several weight matrices: quantize-on-stage and normalizing forms only");
+  static_assert(!NORM || (Cfg::kWaves == kNormMaxRows && MT32 == 1 && ROWS == 16), "a wave to a row");
   int bx = blockIdx.x, gx = args.blocks_x;   // column block within this workgroup's matrix, and how many it has
   if constexpr(GROUPED) {
     int g = 0;
@@ -110,7 +116,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   static_assert(NG == 2 || NG == 4, "groups per thread");
   static_assert(kFusedMaxElems == 4 * 16 * kWave * 8, "four groups per thread of eight waves hold the largest fused input");
   static_assert(!TILED_ || kAbsmaxSlots % Cfg::kThreads == 0, "the abs-max partials are split evenly over the threads");
-  constexpr bool FUSED = MODE == kFusedAll;
+  constexpr bool FUSED = MODE == kFusedAll || NORM;   // all of A in LDS
   constexpr bool TILED = MODE == kFusedTiled;
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
   __shared__ float red[kStream32Waves];
@@ -183,13 +189,15 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   // the address unit works at) and, after quantization, holds dword i of four 16-byte LDS slots.
   // Quad number qi = j * threads / 4 + tid / 4 covers groups 4 * qi .. 4 * qi + 3; group g is row
   // g / (K/16), 16-byte chunk g % (K/16).
-  v4f vals[FUSED ? kFusedGroups : 1][4];
+  v4f vals[FUSED && !NORM ? kFusedGroups : 1][4];
+  NormRow nrow;
+  if constexpr(NORM) nrow.load(A, norm, M, K);
   const int n16 = M * K / 16;   // groups; a multiple of four
   const int quad = tid / 4, qlane = tid % 4;
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);   // (a scalar for the compiler)
   // does group set j reach into this thread's / this wave's range?  (complete sets: always)
   auto in_range = [&](int j) { return j < kFullGroups || 4 * (j * (kStream32Threads / 4) + quad) < n16; };
-  if(FUSED) {
+  if constexpr(FUSED && !NORM) {
     // a quad's four groups are 256 consecutive bytes; group set j starts 32 KB after set j - 1
     const char* a_quad = reinterpret_cast<const char*>(A) + quad * 256 + qlane * 16;
 #pragma unroll
@@ -220,7 +228,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   // are in flight, not behind the abs-max where the quantization waits for them).
   const unsigned k16n = K / 16;   // 16-byte chunks per activation row (a multiple of four)
   unsigned row = 0, c16 = 0, drow = 0, dc16 = 0;
-  if(FUSED) {
+  if(FUSED && !NORM) {
     row = 4 * quad / k16n;
     c16 = 4 * quad % k16n;
     drow = kStream32Threads / k16n;
@@ -240,7 +248,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   // source; group = row * 2 * CS + 16-byte chunk, a quad of lanes takes four consecutive groups
   // (a wave reads whole rows), quantizes them and finds the operand slots from there.
   constexpr int kStageVecs = Cfg::CS * R * 2 / kStream32Threads;
-  v4i stage[TILED ? 1 : kStageVecs];
+  v4i stage[TILED || FUSED ? 1 : kStageVecs];
   v4f stagef[TILED ? kStageVecs : 1][4];
   auto stage_fetch = [&](int chunk) __attribute__((always_inline)) {
     const int s0 = chunk * Cfg::CS;
@@ -347,7 +355,17 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
     if(aq_out && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0)
       *reinterpret_cast<float*>(aq_out + (size_t)M * K) = aqm;
   }
-  if(FUSED) {
+  if constexpr(NORM) {   // (rows M .. 15 of the operand: see below)
+    amax = block_max<kStream32Waves>(nrow.normalize(norm, K), red);
+    if(MH_PROF(args)) tp[1] = MH_CLOCK();
+    aqm = quant_mult_from_maxabs(amax);
+    unquant = unquant_mult(aqm, bqm, args.scale);
+    if(wave < M) {
+      nrow.quantize(lds, wave, K, aqm, stream32_row_key);
+      if(blockIdx.x == 0) nrow.store(norm, wave, K);
+    }
+    __syncthreads();
+  } else if constexpr(FUSED) {
     // whole A (M*K <= kFusedMaxElems floats) in registers: abs-max, then quantize into LDS
 #pragma unroll
     for(int j = 0; j < kFusedGroups; ++j) {

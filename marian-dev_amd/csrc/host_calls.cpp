@@ -39,7 +39,7 @@ namespace {
   F(int8_workspace_bytes) F(int8_prepare_a) F(int8_prepare_b) F(int8_prepare_b_quantized_transposed)     \
   F(int8_affine_f32) F(int8_affine_f32_chained) F(int8_affine_f32_grouped) F(int8_proj_attention)        \
   F(int16_prepare_a) F(int16_prepare_b) F(int16_prepare_b_quantized_transposed) F(int16_affine_f32)      \
-  F(int16_scratch_bytes)                                                                                 \
+  F(int16_scratch_bytes) F(int8_affine_f32_normed) F(int8_proj_attention_normed)                                                                                 \
   F(layer_norm) F(embed) F(attention_cached) F(attention_rows) F(attention_ancestors) F(ancestors_advance)                 \
   F(select_state) F(nbest) F(nbest_words) F(nbest_beams) F(nbest_beams_workspace_bytes) F(nbest_beams_workspace_init)   \
   F(logsoftmax_nbest_beams)
@@ -393,6 +393,65 @@ PyObject* py_affine_f32_grouped(PyObject*, PyObject* const* args, Py_ssize_t nar
   MH_END
 }
 
+// The layer norm of a + add in front of a multiplication that does it itself; false when the call is not one of
+// those (too many or too long rows, another form): the caller then makes two calls.
+struct Normed {
+  const at::Tensor* a = nullptr;
+  int64_t M = 0, K = 0;
+  at::Tensor x;
+  marian_hip_norm_input n{};
+};
+bool normed(PyObject* a, PyObject* add, PyObject* ln, PyObject* eps, Normed& r) {
+  r.a = f32c(a);
+  const at::Tensor* s = f32c(add);
+  if(!r.a || !s || r.a->dim() < 1 || r.a->sizes() != s->sizes() || !PyTuple_Check(ln) || PyTuple_GET_SIZE(ln) != 2) return false;
+  const at::Tensor *gamma = f32c(PyTuple_GET_ITEM(ln, 0)), *beta = f32c(PyTuple_GET_ITEM(ln, 1));
+  r.K = r.a->size(-1);
+  r.M = r.K ? r.a->numel() / r.K : 0;
+  if(!gamma || !beta || gamma->numel() != r.K || beta->numel() != r.K || r.M < 1 || r.M > MARIAN_HIP_NORM_MAX_ROWS ||
+     r.K > MARIAN_HIP_NORM_MAX_COLS || r.K % 64 != 0)
+    return false;
+  for(const at::Tensor* t : {r.a, s, gamma, beta})
+    if(reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16 != 0) return false;
+  r.x = empty(r.a->sizes(), at::kFloat, r.a->device());
+  r.n = marian_hip_norm_input{fptr(s), fptr(gamma), fptr(beta), fptr_mut(r.x), (float)number(eps)};
+  return true;
+}
+
+// affine_f32_normed(a, add, (gamma, beta), eps, weights, scale, relu, want_absmax) -> (x, [out, ..], absmax or None)
+PyObject* py_affine_f32_normed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(8, "affine_f32_normed");
+  Normed r;
+  Matrices w;
+  if(!normed(args[0], args[1], args[2], args[3], r) || !matrices(args[4], r.K, true, w)) Py_RETURN_NONE;
+  const float scale = (float)number(args[5]);
+  const int relu = truth(args[6]);
+  const bool want = truth(args[7]);
+  if(want && w.n != 1) Py_RETURN_NONE;
+  const c10::Device d = r.a->device();
+  at::Tensor outs[kMaxMatrices], omax;
+  float* out[kMaxMatrices];
+  int64_t N[kMaxMatrices], columns = 0;
+  for(int g = 0; g < w.n; ++g) {
+    outs[g] = empty(with_last(r.a->sizes(), w.b[g].cols), at::kFloat, d);
+    out[g] = fptr_mut(outs[g]);
+    N[g] = w.b[g].cols;
+    columns += N[g];
+  }
+  if(columns == 0) Py_RETURN_NONE;
+  if(want) omax = absmax_slots(d);
+  const hipStream_t st = stream_of(d);
+  call("affineOrDot", [&] {
+    return L.int8_affine_f32_normed(fptr(r.a), &r.n, w.n, w.Bq, w.bias, out, N, r.M, r.K, scale, relu, want ? fptr_mut(omax) : nullptr, st);
+  });
+  Ref x(wrap(std::move(r.x))), list(ok(PyList_New(w.n)));
+  for(int g = 0; g < w.n; ++g) PyList_SET_ITEM(list.p, g, wrap(std::move(outs[g])));
+  if(!want) return PyTuple_Pack(3, x.p, list.p, Py_None);
+  Ref m(make_absmax(std::move(omax)));
+  return PyTuple_Pack(3, x.p, list.p, m.p);
+  MH_END
+}
+
 // ---- quantizers ---------------------------------------------------------------------------------
 // prepare_a(a, width) -> QTensor
 PyObject* py_prepare_a(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -694,6 +753,44 @@ PyObject* py_proj_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   MH_END
 }
 
+// proj_attention_normed(a, add, (gamma, beta), eps, weights, k, v, heads, kvLen, mask, want_projections)
+//   -> (x, out, absmax of out, [projections] or None)
+PyObject* py_proj_attention_normed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(11, "proj_attention_normed");
+  Normed r;
+  const at::Tensor *k = f32c(args[5]), *v = f32c(args[6]), *mask;
+  Matrices w;
+  if(!normed(args[0], args[1], args[2], args[3], r) || r.K % 128 != 0 || !k || !v || k->dim() < 2 || k->size(-1) != 64 ||
+     k->sizes() != v->sizes() || !matrices(args[4], r.K, true, w) || (w.n != 1 && w.n != 3) || !f32c_or_none(args[9], &mask))
+    Py_RETURN_NONE;
+  const int64_t heads = whole(args[7]), N = heads * 64, cap = k->size(-2), len = none(args[8]) ? cap : whole(args[8]);
+  for(int g = 0; g < w.n; ++g)
+    if(w.b[g].cols != N) Py_RETURN_NONE;
+  if(cap <= 0 || len <= 0 || (mask && mask->numel() % len != 0)) Py_RETURN_NONE;
+  const bool want_proj = truth(args[10]);
+  const c10::Device d = r.a->device();
+  const at::DimVector size = with_last(r.a->sizes(), N);
+  at::Tensor out = empty(size, at::kFloat, d), omax = absmax_slots(d), projections[3];
+  float* proj[3] = {nullptr, nullptr, nullptr};
+  if(want_proj)
+    for(int g = 0; g < w.n; ++g) {
+      projections[g] = empty(size, at::kFloat, d);
+      proj[g] = fptr_mut(projections[g]);
+    }
+  const hipStream_t st = stream_of(d);
+  call("ProjectedAttention", [&] {
+    return L.int8_proj_attention_normed(fptr(r.a), &r.n, w.n, w.Bq, w.bias, proj, r.M, r.K, heads, fptr_mut(*k), fptr_mut(*v),
+                                        k->numel() / (cap * 64), len, cap, fptr(mask), mask ? mask->numel() / len : 0, 1.0f / 8.0f,
+                                        fptr_mut(out), fptr_mut(omax), st);
+  });
+  Ref x(wrap(std::move(r.x))), o(wrap(std::move(out))), m(make_absmax(std::move(omax)));
+  if(!want_proj) return PyTuple_Pack(4, x.p, o.p, m.p, Py_None);
+  Ref list(ok(PyList_New(w.n)));
+  for(int g = 0; g < w.n; ++g) PyList_SET_ITEM(list.p, g, wrap(std::move(projections[g])));
+  return PyTuple_Pack(4, x.p, o.p, m.p, list.p);
+  MH_END
+}
+
 // attention_ancestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax) -> out or (out, absmax)
 PyObject* py_attention_ancestors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_TRY MH_ARGS(8, "attention_ancestors");
@@ -867,7 +964,7 @@ PyObject* py_setup(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 #define MH_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&py_##name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
-    MH_METHOD(affine_f32_grouped), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
+    MH_METHOD(affine_f32_grouped), MH_METHOD(affine_f32_normed), MH_METHOD(proj_attention_normed), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
     MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(attention_rows), MH_METHOD(split_heads), MH_METHOD(join_heads), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors),
     MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_words), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),
     {nullptr, nullptr, 0, nullptr}};

@@ -1,0 +1,129 @@
+// Layer normalization of a row of up to 1024 values by one wave, four float4 per lane: the row computation
+// of the layer-norm launch and of the kernels that normalize their input themselves.  The same operations
+// in the same order everywhere, so the results have the same bits.
+#pragma once
+
+#include "int8_common.h"
+#include "quantize_common.h"
+
+namespace marian_hip {
+
+// Sum over each group of 16 consecutive lanes, left in all 16 of them (four DPP steps: the two
+// lane swaps within a quad, then the mirror within half a row and within the row).
+__device__ __forceinline__ float row16_sum(float v) {
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));  // row_half_mirror
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, false));  // row_mirror
+  return v;
+}
+// Sum over the wave, the same value in all lanes: within the rows of 16 lanes, then across them
+// with the two row-broadcast DPP steps (rows 1 and 3 take in the last lane of the row before them,
+// then rows 2 and 3 the last lane of row 1), which leaves the total in lane 63, read from there as
+// a scalar.  No step goes through the LDS crossbar (a lane exchange there costs ten times a DPP
+// step).  All lanes of the wave must be active.
+__device__ __forceinline__ float wave_sum(float v) {
+  v = row16_sum(v);
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xA, 0xF, false));   // row_bcast:15
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));   // row_bcast:31
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+
+constexpr int kNormVecs = 4;   // float4 per lane: rows of up to 1024 values, cols % 4 == 0
+
+// Value j of a lane is float4 number j * 64 + lane of the row; positions past the row are clamped by the
+// loader and dropped here.  v: the row, becomes its normalization (clamped positions: anything); t: what is added to
+// it first (has_add).  Returns the largest magnitude of this lane's values.
+__device__ __forceinline__ float normalize_row(v4f (&v)[kNormVecs], const v4f (&t)[kNormVecs], bool has_add, const v4f (&gm)[kNormVecs],
+                                               const v4f (&bt)[kNormVecs], bool has_beta, int cols, float eps) {
+  const int lane = threadIdx.x % kWave, cols4 = cols / 4;
+  float sum = 0.0f;
+#pragma unroll
+  for(int j = 0; j < kNormVecs; ++j) {
+    if(has_add) v[j] = v4f{v[j].x + t[j].x, v[j].y + t[j].y, v[j].z + t[j].z, v[j].w + t[j].w};
+    if(j * kWave + lane < cols4) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
+  }
+  const float mean = wave_sum(sum) / (float)cols;
+  float sq = 0.0f;
+#pragma unroll
+  for(int j = 0; j < kNormVecs; ++j) {
+    if(j * kWave + lane < cols4) {
+      const float d0 = v[j].x - mean, d1 = v[j].y - mean, d2 = v[j].z - mean, d3 = v[j].w - mean;
+      sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
+    }
+  }
+  const float sigma = sqrtf(wave_sum(sq) / (float)cols + eps);
+  float omax = 0.0f;
+#pragma unroll
+  for(int j = 0; j < kNormVecs; ++j) {
+    if(j * kWave + lane < cols4) {
+      float r[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+      const float g[4] = {gm[j].x, gm[j].y, gm[j].z, gm[j].w}, b[4] = {bt[j].x, bt[j].y, bt[j].z, bt[j].w};
+#pragma unroll
+      for(int e = 0; e < 4; ++e) {
+        float o = g[e] * ((r[e] - mean) / sigma);
+        if(has_beta) o = o + b[e];
+        r[e] = o;
+        omax = fmaxf(omax, fabsf(o));
+      }
+      v[j] = v4f{r[0], r[1], r[2], r[3]};
+    }
+  }
+  return omax;
+}
+
+// A decoding step's few hypotheses: the kernel that multiplies the normalized rows normalizes them itself -
+// every workgroup all of them, a wave to a row - instead of reading what a launch of its own has left.
+constexpr int kNormMaxRows = 8, kNormMaxCols = 256 * kNormVecs;
+struct NormInput {
+  const float* add;     // [M x K]: the skip connection
+  const float* gamma;   // [K]
+  const float* beta;    // [K]
+  float* out;           // [M x K]: the normalized rows, written by one workgroup
+  float eps;
+};
+struct NormRow {
+  v4f v[kNormVecs], t[kNormVecs], gm[kNormVecs], bt[kNormVecs];
+  // Wave w loads row w (rows past M: a copy of the last one).  All loads unconditional, so that waits count them exactly.
+  __device__ __forceinline__ void load(const float* A, const NormInput& n, int M, int K) {
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, cols4 = K / 4;
+    const size_t row = (size_t)min(wave, M - 1) * K;
+#pragma unroll
+    for(int j = 0; j < kNormVecs; ++j) {
+      const int i = min(j * kWave + lane, cols4 - 1);
+      v[j] = reinterpret_cast<const v4f*>(A + row)[i];
+      t[j] = reinterpret_cast<const v4f*>(n.add + row)[i];
+    }
+#pragma unroll
+    for(int j = 0; j < kNormVecs; ++j) {
+      const int i = min(j * kWave + lane, cols4 - 1);
+      gm[j] = reinterpret_cast<const v4f*>(n.gamma)[i];
+      bt[j] = reinterpret_cast<const v4f*>(n.beta)[i];
+    }
+  }
+  __device__ __forceinline__ float normalize(const NormInput& n, int K) {
+    return normalize_row(v, t, true, gm, bt, true, K, n.eps);
+  }
+  // The row's quantized values into LDS in operand order: slot (c16 / 2, c16 % 2, row) of 16 bytes holds 16-byte
+  // chunk c16 of the row, rows XOR-permuted by the key of the chunk.
+  template <typename KEY>
+  __device__ __forceinline__ void quantize(int8_t* lds, int row, int K, float qm, KEY key) const {
+    const int lane = threadIdx.x % kWave;
+    const bool finite = qm < __builtin_inff();
+#pragma unroll
+    for(int j = 0; j < kNormVecs; ++j) {
+      const int i = j * kWave + lane, c16 = i / 4;
+      if(i < K / 4)
+        *reinterpret_cast<uint32_t*>(lds + ((c16 / 2) * 64 + (c16 % 2) * 32 + (row ^ key(c16))) * 16 + (i % 4) * 4) =
+            finite ? quantize_pack4_finite(v[j], qm) : quantize_pack4(v[j], qm);
+    }
+  }
+  __device__ __forceinline__ void store(const NormInput& n, int row, int K) const {
+    const int lane = threadIdx.x % kWave;
+#pragma unroll
+    for(int j = 0; j < kNormVecs; ++j)
+      if(j * kWave + lane < K / 4) reinterpret_cast<v4f*>(n.out + (size_t)row * K)[j * kWave + lane] = v[j];
+  }
+};
+
+}  // namespace marian_hip

@@ -130,6 +130,62 @@ class DecoderStep:
         self.state, self.state_next = self.state_next, self.state
         self._cache_views()
 
+    def _layers_of_few_rows(self, W, x, xmax, rec):
+        """The layers and the output layer for a handful of hypotheses: every layer norm is taken by the
+        launch that multiplies its result (the launches of their own were a fifth of the step for six
+        hypotheses of one sentence).  rec: None, or records the operator calls."""
+        integer, ops, H, M = self.integer, self.ops, self.H, self.M
+        pending = None   # (a, skip, ln): x is still to be taken as the layer norm of a + skip
+        for li, ly in enumerate(W["layers"]):
+            qkv = [ly["Wq"], ly["Wk"], ly["Wv"]]
+            k_cache, v_cache = self.Kself[li], self.Vself[li]
+            if rec:
+                k_before, v_before = k_cache.clone(), v_cache.clone()
+            if self.by_ancestors:
+                if pending:
+                    x, (q, k, v), _ = ops.affineOfLayerNorm(*pending, qkv)
+                else:
+                    (q, k, v), _ = integer.affine_f32_grouped(x, qkv, absmax=xmax)
+                o, omax = ops.AttentionByAncestors(q, k_cache, v_cache, self.anc, self.T, k, v, want_absmax=True)
+                o = o.view(M, self.d)
+            elif pending:
+                x, o, omax, proj = ops.ProjectedAttentionOfLayerNorm(*pending, qkv, k_cache, v_cache, H, kvLen=self.T,
+                                                                     want_projections=bool(rec))
+            else:
+                res = ops.ProjectedAttention(x, qkv, k_cache, v_cache, H, kvLen=self.T, absmax=xmax, want_absmax=True,
+                                             want_projections=bool(rec))
+                o, omax, proj = res[0], res[2], res[3] if rec else None
+            if rec:
+                if not self.by_ancestors:
+                    q, k, v = proj
+                if pending:
+                    rec("layer_norm", x=pending[0], add=pending[1], gamma=pending[2][0], beta=pending[2][1], out=x)
+                for name, t in (("Wq", q), ("Wk", k), ("Wv", v)):
+                    rec("affine", a=x, w=ly[name], out=t, relu=False)
+                rec("self_attention", q=q, k_new=k, v_new=v, k_cache=k_before, v_cache=v_before,
+                    k_after=k_cache, v_after=v_cache, out=o, len=self.T)
+            a, _ = integer.affine_f32(o, *ly["Wo"], absmax=omax)
+            x1, co, comax, proj = ops.ProjectedAttentionOfLayerNorm(a, x, ly["ln1"], [ly["cWq"]], self.Kenc[li], self.Venc[li], H,
+                                                                    mask=self.mask, want_projections=bool(rec))
+            ca, _ = integer.affine_f32(co, *ly["cWo"], absmax=comax)
+            x2, (f1,), f1max = ops.affineOfLayerNorm(ca, x1, ly["ln2"], [ly["W1"]], relu=True, want_absmax=True)
+            f2, _ = integer.affine_f32(f1, *ly["W2"], absmax=f1max)
+            if rec:
+                rec("affine", a=o, w=ly["Wo"], out=a, relu=False)
+                rec("layer_norm", x=a, add=x, gamma=ly["ln1"][0], beta=ly["ln1"][1], out=x1)
+                rec("affine", a=x1, w=ly["cWq"], out=proj[0], relu=False)
+                rec("context_attention", q=proj[0], k=self.Kenc[li], v=self.Venc[li], mask=self.mask, out=co)
+                rec("affine", a=co, w=ly["cWo"], out=ca, relu=False)
+                rec("layer_norm", x=ca, add=x1, gamma=ly["ln2"][0], beta=ly["ln2"][1], out=x2)
+                rec("affine", a=x2, w=ly["W1"], out=f1, relu=True)
+                rec("affine", a=f1, w=ly["W2"], out=f2, relu=False)
+            pending = (f2, x2, ly["ln3"])
+        x, (logits,), _ = ops.affineOfLayerNorm(*pending, [W["out"]])
+        if rec:
+            rec("layer_norm", x=pending[0], add=pending[1], gamma=pending[2][0], beta=pending[2][1], out=x)
+            rec("affine", a=x, w=W["out"], out=logits, relu=False)
+        return logits
+
     def step(self, s, gemm_only=False, chained=True, grouped=True, fused_tail=False, select=False, fused_attention=True):
         """chained: every tensor that feeds an affine call leaves its abs-max where it is
         produced (layer norm, attention, the ReLU GEMM), so those calls skip their abs-max pass.
@@ -162,7 +218,10 @@ class DecoderStep:
                 x, xmax = x
             if tr is not None:
                 rec("embed", E=self.E, ids=self.words, scale=self.emb_scale, signal=self.signal, out=x, position=self.T - 1)
-        for li, ly in enumerate(W["layers"]):
+        few = fused_attention and ch and M <= 8 and bool(W["layers"])   # the rows up to which the layer norms need no launches of their own
+        if few:
+            logits = self._layers_of_few_rows(W, x, xmax, rec if tr is not None else None)
+        for li, ly in enumerate(() if few else W["layers"]):
             omax = x1max = comax = x2max = f1max = None
             fuse = fused_attention and not gemm_only and not self.by_ancestors and ch
             if fuse:   # q, k, v and the self-attention over the cache (the new position appended) in one launch
@@ -268,9 +327,10 @@ class DecoderStep:
                     x, xmax = x
                 if tr is not None:
                     rec("layer_norm", x=f2, add=xin, gamma=ly["ln3"][0], beta=ly["ln3"][1], out=x)
-        logits, _ = integer.affine_f32(x, *W["out"], absmax=xmax)
-        if tr is not None:
-            rec("affine", a=x, w=W["out"], out=logits, relu=False)
+        if not few:
+            logits, _ = integer.affine_f32(x, *W["out"], absmax=xmax)
+            if tr is not None:
+                rec("affine", a=x, w=W["out"], out=logits, relu=False)
         if gemm_only:
             return logits
         if fused_tail:

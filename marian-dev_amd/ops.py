@@ -299,6 +299,35 @@ def ProjectedAttention(x, weights, k, v, heads, kvLen=None, mask=None, absmax=No
                   "ProjectedAttention")
 
 
+def affineOfLayerNorm(a, add, ln, weights, eps=1e-6, relu=False, want_absmax=False):
+    """x = layerNorm(a, *ln, eps, add=add) and x through one or several weight matrices (affine_f32, or
+    affine_f32_grouped for several): one launch for up to eight rows of up to 1024 values
+    (marian_hip_int8_affine_f32_normed), otherwise the separate calls, with the same bits.
+    Returns (x, [out, ..], AbsMax of the only out or None)."""
+    res = _host.affine_f32_normed(a, add, ln, eps, weights, 1.0, relu, want_absmax)
+    if res is not None:
+        return res
+    from . import integer
+    x, xmax = layerNorm(a, *ln, eps=eps, add=add, want_absmax=True)
+    if len(weights) > 1:
+        _abort_if(want_absmax, "affineOfLayerNorm: the abs-max of one output only{}", "")
+        return x, integer.affine_f32_grouped(x, weights, relu=relu, absmax=xmax)[0], None
+    res = integer.affine_f32(x, *weights[0], relu=relu, absmax=xmax, want_absmax=want_absmax)
+    return x, [res[0]], res[2] if want_absmax else None
+
+
+def ProjectedAttentionOfLayerNorm(a, add, ln, weights, k, v, heads, kvLen=None, mask=None, eps=1e-6, want_projections=False):
+    """x = layerNorm(a, *ln, eps, add=add) and ProjectedAttention(x, ..): one launch for up to eight rows
+    (marian_hip_int8_proj_attention_normed), otherwise the two calls, with the same bits.
+    Returns (x, out, AbsMax of out, the projections when asked for or None)."""
+    res = _host.proj_attention_normed(a, add, ln, eps, weights, k, v, heads, kvLen, mask, want_projections)
+    if res is not None:
+        return res
+    x, xmax = layerNorm(a, *ln, eps=eps, add=add, want_absmax=True)
+    res = ProjectedAttention(x, weights, k, v, heads, kvLen, mask, xmax, True, want_projections)
+    return x, res[0], res[2], res[3] if want_projections else None
+
+
 def AttentionByAncestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax=False):
     """Self-attention of a decoding step on caches that are never moved (no counterpart in the
     reference, which copies the surviving hypotheses' states, src/rnn/types.h:22-42): cached

@@ -1,0 +1,103 @@
+"""The calls that take a layer norm with the multiplication behind it, against the separate calls: the same bits."""
+import importlib
+
+import pytest
+
+PKG = "marian-dev_amd"
+
+
+def load(name):
+    return importlib.import_module(PKG + "." + name)
+
+
+pytestmark = pytest.mark.gpu
+
+
+def same(a, b):
+    import torch
+    return a.shape == b.shape and torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+def inputs(M, K, seed, kind="normal"):
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    a, add, gamma, beta = r(M, K), r(M, K), 1 + 0.1 * r(K), 0.1 * r(K)
+    if kind == "constant":     # rows without variance and a zero shift: every output is zero, the quantMult infinite
+        a, add, beta = torch.ones_like(a), torch.ones_like(a), torch.zeros_like(beta)
+    if kind == "infinite":
+        a[0, K // 2] = float("inf")
+    return r, a, add, (gamma, beta)
+
+
+@pytest.mark.parametrize("kind", ["normal", "constant", "infinite"])
+@pytest.mark.parametrize("M,K,N", [
+    (1, 64, [8]), (8, 64, [40]), (3, 128, [32, 8, 200]), (6, 512, [2048]), (6, 512, [512, 512, 512]), (8, 512, [4000]),
+    (2, 576, [576]), (7, 768, [3072]), (8, 1024, [1024, 1024, 1024]), (8, 1024, [4096]), (5, 256, [8192]), (4, 1024, [16384]),
+    (3, 448, [32000]), (1, 512, [40000]), (2, 320, [33000, 40000]),
+    (9, 512, [512]), (4, 1088, [64, 64])])   # (the last two: separate calls)
+def test_affine_of_layer_norm(M, K, N, kind):
+    import torch
+    integer, ops = load("integer"), load("ops")
+    r, a, add, ln = inputs(M, K, 7 * M + K + len(N), kind)
+    weights = [(integer.prepareB(r(K, n) * 0.02), r(n) if i != 1 else None) for i, n in enumerate(N)]
+    relu, want = len(N) == 1, len(N) == 1
+    for eps in (1e-6, 1e-9):
+        x, outs, omax = ops.affineOfLayerNorm(a, add, ln, weights, eps=eps, relu=relu, want_absmax=want)
+        x_s, xmax = ops.layerNorm(a, *ln, eps=eps, add=add, want_absmax=True)
+        assert same(x, x_s)
+        for (w, b), out in zip(weights, outs):
+            assert same(out, integer.affine_f32(x_s, w, b, relu=relu, absmax=xmax)[0])
+        if want:
+            assert omax.data.max().item() == outs[0].abs().max().item() or torch.isnan(outs[0]).any()
+
+
+@pytest.mark.parametrize("hyps,sentences,heads,length", [
+    (1, 1, 2, 1), (6, 1, 8, 23), (1, 8, 4, 33), (4, 2, 16, 96), (2, 3, 8, 64), (8, 1, 12, 97), (3, 2, 16, 5), (5, 2, 8, 9)])
+def test_projected_attention_of_layer_norm(hyps, sentences, heads, length):
+    import torch
+    integer, ops = load("integer"), load("ops")
+    M, K = hyps * sentences, heads * 64
+    r, a, add, ln = inputs(M, K, M + K + length)
+    weights = [(integer.prepareB(r(K, K) * 0.02), r(K)) for _ in range(3)]
+    x_s, xmax = ops.layerNorm(a, *ln, eps=1e-6, add=add, want_absmax=True)
+    # over complete caches, `hyps` hypotheses to a sentence
+    k, v = r(sentences * heads, length, 64), r(sentences * heads, length, 64)
+    mask = -1e8 * (torch.rand(sentences, length, device="cuda") < 0.3).float()
+    mask[:, 0] = 0.0
+    x, out, omax, proj = ops.ProjectedAttentionOfLayerNorm(a, add, ln, weights[:1], k, v, heads, mask=mask, want_projections=True)
+    out_s, _, omax_s, proj_s = ops.ProjectedAttention(x_s, weights[:1], k, v, heads, mask=mask, absmax=xmax, want_absmax=True,
+                                                      want_projections=True)
+    assert same(x, x_s) and same(out, out_s) and same(proj[0], proj_s[0])
+    assert omax.data.max().item() == omax_s.data.max().item()
+    # self-attention: the new key and value are appended
+    k, v = r(M * heads, length + 2, 64), r(M * heads, length + 2, 64)
+    k_s, v_s = k.clone(), v.clone()
+    x, out, omax, proj = ops.ProjectedAttentionOfLayerNorm(a, add, ln, weights, k, v, heads, kvLen=length)
+    out_s, _, omax_s = ops.ProjectedAttention(x_s, weights, k_s, v_s, heads, kvLen=length, absmax=xmax, want_absmax=True)
+    assert same(x, x_s) and same(out, out_s) and same(k, k_s) and same(v, v_s) and proj is None
+    assert omax.data.max().item() == omax_s.data.max().item()
+
+
+def test_refused_arguments():
+    import ctypes
+    import torch
+    lib, L = load("_lib").lib(), load("_lib")
+
+    class Norm(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_void_p) for n in ("add", "gamma", "beta", "out")] + [("eps", ctypes.c_float)]
+    t = torch.zeros(16, 2048, device="cuda")
+    p = t.data_ptr()
+    one = lambda v: (ctypes.c_void_p * 1)(v)
+    n64 = (ctypes.c_int64 * 1)(64)
+
+    def call(norm, M=4, K=64, A=p):
+        return lib.marian_hip_int8_affine_f32_normed(A, ctypes.byref(norm), 1, one(p), None, one(p + 65536), n64, M, K, 1.0, 0, None, None)
+    good = dict(add=p, gamma=p, beta=p, out=p + 32768, eps=1e-6)
+    assert call(Norm(**good), M=9) == L.ERR_SHAPE
+    assert call(Norm(**good), K=1088) == L.ERR_SHAPE
+    assert call(Norm(**{**good, "beta": None})) == L.ERR_NULL
+    assert call(Norm(**{**good, "out": p + 4})) == L.ERR_ALIGN
+    assert call(Norm(**{**good, "out": p + 16})) == L.ERR_ALIAS
+    assert call(Norm(**good), M=0) == L.OK
