@@ -707,6 +707,70 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
   return launch_big<128, 128, 2, 2, 3>(a, st);
 }
 
+// The matrices that have columns, and where their column blocks of `cols` columns start.
+GroupTable group_table(int64_t n_groups, const int8_t* const* Bq, const float* const* bias, float* const* out,
+                              const int64_t* N, int cols) {
+  GroupTable t;
+  t.n = 0;
+  t.block0[0] = 0;
+  for(int64_t g = 0; g < n_groups; ++g) {
+    if(N[g] == 0) continue;
+    const int i = t.n++;
+    t.Bq[i] = Bq[g];
+    t.bias[i] = bias ? bias[g] : nullptr;
+    t.out[i] = out[g];
+    t.N[i] = (int)N[g];
+    t.block0[i + 1] = t.block0[i] + (int)((N[g] + cols - 1) / cols);
+  }
+  for(int i = t.n; i < kMaxGroups; ++i) {   // unused entries: never selected
+    t.Bq[i] = nullptr; t.bias[i] = nullptr; t.out[i] = nullptr; t.N[i] = 0;
+    t.block0[i + 1] = t.block0[t.n];
+  }
+  return t;
+}
+
+// One launch for the matrices behind an input of more rows than the decode forms take (whole K blocks).
+//  - as many 256x256 tiles as the plain launch asks of them, whole ones: tile pairs, one written out
+//    while the next is multiplied (4096 x 1024 x 3072 19.6 us, the next form 22.6, three launches 26.7 - 32);
+//  - a 128x128 tile or more per CU: the eight-wave form, two workgroups to a CU (3000 x 512 x 1536 8.9 us,
+//    1400 x 1024 x 3072 11.6; three launches 14.8 and 16.9);
+//  - fewer: 128x64 tiles in the split form, which CUs that idle leave room for (1000 x 512 x 1536 5.1 us,
+//    600 x 1024 x 3072 6.0; three launches 13.9 and 16.3).
+template <typename CFG, int THREADS, typename KERNEL>
+int launch_grouped_as(KERNEL kernel, const GemmArgs& a, const GroupTable& g, int tiles_m, std::atomic<uint64_t>& lds_done, hipStream_t st) {
+  const int lds_status = allow_lds(kernel, CFG::kLdsBytes, lds_done);
+  if(lds_status != MARIAN_HIP_OK) return lds_status;
+  const int tiles_n = g.block0[g.n];
+  hipLaunchKernelGGL(kernel, dim3(tiles_n * tiles_m), dim3(THREADS), CFG::kLdsBytes, st, a, g, tiles_n, tiles_m);
+  MH_HIP(hipGetLastError());
+  return MARIAN_HIP_OK;
+}
+int launch_big_grouped(const GemmArgs& a, int64_t n_groups, const int8_t* const* Bq, const float* const* bias, float* const* out,
+                       const int64_t* N, hipStream_t st) {
+  long long columns = 0, tiles128 = 0;
+  bool pairs = a.M % PairCfg::BM == 0 && a.K <= 1536 && a.K / PairCfg::BK >= PairCfg::kSideBlocks;
+  for(int64_t g = 0; g < n_groups; ++g) {
+    columns += N[g];
+    tiles128 += (N[g] + 127) / 128;
+    pairs = pairs && N[g] % (2 * PairCfg::BN) == 0 && (!bias || !bias[g] || aligned(bias[g], 16));
+  }
+  tiles128 *= (a.M + 127) / 128;
+  const bool stream_out = (long long)a.M * columns * 4 <= (32ll << 20);   // (as for a single matrix)
+  static std::atomic<uint64_t> lds_done[4];
+  if(pairs && (a.M / 256) * (columns / 256) >= 192)
+    return launch_grouped_as<PairCfg, PairCfg::kThreads>(gemm_pair_group_kernel<true>, a, group_table(n_groups, Bq, bias, out, N, 2 * PairCfg::BN),
+                                                        a.M / PairCfg::BM, lds_done[0], st);
+  if(tiles128 >= compute_units()) {
+    using Cfg = BigCfg<128, 128, 2, 4, 2>;
+    const GroupTable t = group_table(n_groups, Bq, bias, out, N, 128);
+    if(stream_out) return launch_grouped_as<Cfg, Cfg::kThreads>(gemm_mfma32_group_kernel<128, 128, 2, 4, 2, true, false>, a, t, (a.M + 127) / 128, lds_done[1], st);
+    return launch_grouped_as<Cfg, Cfg::kThreads>(gemm_mfma32_group_kernel<128, 128, 2, 4, 2, false, false>, a, t, (a.M + 127) / 128, lds_done[2], st);
+  }
+  using Cfg = BigCfg<128, 64, 2, 2, 3>;
+  return launch_grouped_as<Cfg, 2 * Cfg::kThreads>(gemm_mfma32_group_kernel<128, 64, 2, 2, 3, true, true>, a,
+                                                   group_table(n_groups, Bq, bias, out, N, 64), (a.M + 127) / 128, lds_done[3], st);
+}
+
 int check_gemm(const int8_t* Aq, const int8_t* Bq, const void* out, const float* bias,
                const uint32_t* idx, int64_t n_idx, int64_t M, int64_t K, int64_t N) {
   if(M < 0 || K <= 0 || N < 0 || (K % 64) != 0 || (N % 8) != 0) return MARIAN_HIP_ERR_SHAPE;
@@ -1071,28 +1135,6 @@ int marian_hip_int8_affine_f32_chained(const float* A, int8_t* Aq, const int8_t*
 }
 
 
-// The matrices that have columns, and where their column blocks of `cols` columns start.
-static GroupTable group_table(int64_t n_groups, const int8_t* const* Bq, const float* const* bias, float* const* out,
-                              const int64_t* N, int cols) {
-  GroupTable t;
-  t.n = 0;
-  t.block0[0] = 0;
-  for(int64_t g = 0; g < n_groups; ++g) {
-    if(N[g] == 0) continue;
-    const int i = t.n++;
-    t.Bq[i] = Bq[g];
-    t.bias[i] = bias ? bias[g] : nullptr;
-    t.out[i] = out[g];
-    t.N[i] = (int)N[g];
-    t.block0[i + 1] = t.block0[i] + (int)((N[g] + cols - 1) / cols);
-  }
-  for(int i = t.n; i < kMaxGroups; ++i) {   // unused entries: never selected
-    t.Bq[i] = nullptr; t.bias[i] = nullptr; t.out[i] = nullptr; t.N[i] = 0;
-    t.block0[i + 1] = t.block0[t.n];
-  }
-  return t;
-}
-
 int marian_hip_int8_affine_f32_normed(const float* A, const marian_hip_norm_input* norm, int64_t n_groups,
                                       const int8_t* const* Bq, const float* const* bias, float* const* out,
                                       const int64_t* N, int64_t M, int64_t K, float scale, int relu,
@@ -1199,6 +1241,14 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
   } else {
     int st = marian_hip_int8_prepare_a(A, Aq, M, K, workspace, workspace_bytes, stream);
     if(st != MARIAN_HIP_OK) return st;
+  }
+  if(n_groups > 1 && M > 256 && K % 128 == 0 && kernel_override() % 1000 == 0) {   // (a pinned kernel: the separate launches)
+    if(total_blocks32 == 0) return MARIAN_HIP_OK;
+    GemmArgs a;
+    a.Aq = Aq; a.Bq = nullptr; a.bias = nullptr; a.idx = nullptr; a.out = nullptr;
+    a.M = (int)M; a.K = (int)K; a.N = a.n_out = 0;
+    a.scale = scale; a.relu = relu ? 1 : 0; a.dump = 0;
+    return launch_big_grouped(a, n_groups, Bq, bias, out, N, hst);
   }
   for(int64_t g = 0; g < n_groups; ++g) {
     int st = run_gemm(Aq, Bq[g], bias ? bias[g] : nullptr, nullptr, 0, out[g], M, K, N[g], scale, relu, 0, stream);

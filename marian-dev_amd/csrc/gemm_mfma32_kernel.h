@@ -567,6 +567,19 @@ __global__ __launch_bounds__(2 * WAVES_M * WAVES_N * kWave) void gemm_mfma32_spl
   gemm_mfma32_tile<BM, BN, WAVES_M, WAVES_N, NSTAGE, true, NT, false, AMAX, true>(args, tm * BM, tn * BN, lds, blockIdx.x);
 }
 
+// Several weight matrices behind one input, over their tile columns side by side: at encoder sizes one
+// matrix of a self-attention layer is a tile or less per CU, and three launches are three ramps and
+// three drains (4096 x 1024 x 3 x 1024: 32 us in three launches; see launch_big_grouped for the forms).
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NSTAGE, bool NT, bool SPLIT>
+__global__ __launch_bounds__((SPLIT ? 2 : 1) * WAVES_M * WAVES_N * kWave) void gemm_mfma32_group_kernel(
+    GemmArgs args, GroupTable groups, int tiles_n, int tiles_m) {
+  extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+  int tn, tm;
+  xcd_tile(tiles_n, tiles_m, blockIdx.x, tn, tm);
+  tn = groups.select(args, tn);
+  gemm_mfma32_tile<BM, BN, WAVES_M, WAVES_N, NSTAGE, true, NT, false, false, SPLIT>(args, tm * BM, tn * BN, lds, blockIdx.x);
+}
+
 // A launch whose output is not a whole number of main tiles: `main_tiles` whole BM x BN tiles
 // (the first workgroups, in the XCD-aware order), then small tiles over the rows below them (EBM x
 // EBN tiles: a strip `bottom_tiles_n` tiles wide over all columns, starting at row main_tiles_m * BM)

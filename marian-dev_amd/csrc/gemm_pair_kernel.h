@@ -288,6 +288,16 @@ __global__ __launch_bounds__(PairCfg::kThreads) void gemm_pair_kernel(GemmArgs a
   gemm_pair_tiles<NT, AMAX>(args, tm * PairCfg::BM, tn * 2 * PairCfg::BN, lds, blockIdx.x);
 }
 
+// Several weight matrices behind one input, whole tile pairs each.
+template <bool NT>
+__global__ __launch_bounds__(PairCfg::kThreads) void gemm_pair_group_kernel(GemmArgs args, GroupTable groups, int pairs_n, int tiles_m) {
+  extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+  int tn, tm;
+  xcd_tile(pairs_n, tiles_m, blockIdx.x, tn, tm);
+  tn = groups.select(args, tn);
+  gemm_pair_tiles<NT, false>(args, tm * PairCfg::BM, tn * 2 * PairCfg::BN, lds, blockIdx.x);
+}
+
 // The same for an output that is not a whole number of tile pairs: pairs over the whole 256 x 256
 // blocks, then 64 x 128 tiles over the rows below them and 128 x 64 tiles over the columns to their
 // right (see RaggedPlan; main_tiles_n counts pairs).

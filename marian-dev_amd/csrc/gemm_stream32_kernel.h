@@ -63,18 +63,6 @@ struct Stream32Cfg {
   static_assert(CS % 2 == 0, "a quad of lanes quantizes four 16-byte chunks of one row");
 };
 
-// Several weight matrices behind one activation tensor (kFusedTiled only): the grid's columns are
-// the matrices' column blocks one after the other, and a workgroup takes weights, bias, output and
-// width from the entry its block index falls into (block0[g] <= blockIdx.x < block0[g + 1]).
-constexpr int kMaxGroups = 4;
-struct GroupTable {
-  const int8_t* Bq[kMaxGroups];
-  const float* bias[kMaxGroups];
-  void* out[kMaxGroups];
-  int N[kMaxGroups];
-  int block0[kMaxGroups + 1];
-  int n;
-};
 struct NoGroups {};
 
 // Dynamic LDS: one chunk (kStageBytes), for kFusedAll all of K (32 * MT32 * K bytes) if that is

@@ -118,6 +118,32 @@ struct GemmArgs {
 
 constexpr int kAbsmaxSlots = 2048;
 
+// Several weight matrices behind one activation tensor: the launch's columns are the matrices' column
+// blocks one after the other, and a workgroup takes weights, bias, output and width from the entry its
+// column block falls into (block0[g] <= block < block0[g + 1]).
+constexpr int kMaxGroups = 4;
+struct GroupTable {
+  const int8_t* Bq[kMaxGroups];
+  const float* bias[kMaxGroups];
+  void* out[kMaxGroups];
+  int N[kMaxGroups];
+  int block0[kMaxGroups + 1];
+  int n;
+
+  // Points the arguments to the matrix of column block `block`; returns the block's number within it.
+  __device__ __forceinline__ int select(GemmArgs& a, int block) const {
+    int g = 0;
+#pragma unroll
+    for(int i = 1; i < kMaxGroups; ++i)
+      if(i < n && block >= block0[i]) g = i;
+    a.Bq = Bq[g];
+    a.bias = bias[g];
+    a.out = out[g];
+    a.N = a.n_out = N[g];
+    return block - block0[g];
+  }
+};
+
 // The tuning build (-DMARIAN_HIP_TUNING, libmarian_hip_int8_tuning.so) carries measurement switches
 // and per-workgroup phase clocks in the kernels; the shipped library compiles them out.
 #ifdef MARIAN_HIP_TUNING

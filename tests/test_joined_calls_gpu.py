@@ -1,4 +1,5 @@
-"""The calls that take a layer norm with the multiplication behind it, against the separate calls: the same bits."""
+"""Calls that take several steps in one launch - a layer norm with the multiplication behind it, several matrices behind many
+rows - against the separate calls: the same bits."""
 import importlib
 
 import pytest
@@ -101,3 +102,25 @@ def test_refused_arguments():
     assert call(Norm(**{**good, "out": p + 4})) == L.ERR_ALIGN
     assert call(Norm(**{**good, "out": p + 16})) == L.ERR_ALIAS
     assert call(Norm(**good), M=0) == L.OK
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (4096, 1024, [1024, 1024, 1024]), (2048, 1536, [2048, 1024, 3072, 256]),                   # tile pairs
+    (3000, 512, [512, 512, 512]), (2050, 384, [1000, 8, 2056]), (4096, 1664, [1024, 1024]),     # a 128x128 tile per CU
+    (257, 128, [8, 8]), (600, 1024, [1024, 1024, 1024]), (1000, 512, [512, 0, 72, 200]),        # 128x64 tiles
+    (300, 576, [64, 128])])                                                                     # K not in whole blocks
+@pytest.mark.parametrize("relu", [False, True])
+def test_grouped_matrices_behind_many_rows(M, K, N, relu):
+    import torch
+    integer = load("integer")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + K)
+    x = torch.randn(M, K, device="cuda", generator=g)
+    weights = [(integer.prepareB(torch.randn(K, n, device="cuda", generator=g) * 0.02) if n else
+                integer.QTensor(torch.zeros(256, dtype=torch.int8, device="cuda"), (K, 0), load("types").Type.intgemm8, True),
+                torch.randn(n, device="cuda", generator=g) if i != 1 else None) for i, n in enumerate(N)]
+    outs, _ = integer.affine_f32_grouped(x, weights, relu=relu)
+    for (w, b), out, n in zip(weights, outs, N):
+        assert out.shape == (M, n)
+        if n:
+            assert same(out, integer.affine_f32(x, w, b, relu=relu)[0])
