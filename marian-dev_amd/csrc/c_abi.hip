@@ -425,7 +425,7 @@ int launch_normed(const GemmArgs& a, const float* A, const NormInput& n, const G
 // (MT32 * KW * PW <= 64).  kFusedTiled stages fp32 values in registers: at most 4 per wave (8 when K is not split).
 template <int MT32, int MODE>
 int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int kw, bool half_rows = false,
-                       const GroupLaunch* g = nullptr) {
+                       const GroupLaunch* g = nullptr, bool eight_rows = false) {
   const int need = (a.K / 32 + kw - 1) / kw;   // sub-steps per wave if K is one chunk
   if constexpr(MODE == kFusedTiled) {
     static_assert(MT32 == 1, "tiled fused form: 32 (or 16) rows per workgroup");
@@ -438,6 +438,7 @@ int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int
           return launch_stream32<1, 2, 4, 8, MODE>(a, f, st, g);   // long rows: half as many chunks (measurement id 690 keeps the shorter ones)
         return launch_stream32<1, 2, 4, 4, MODE>(a, f, st, g);
       default:
+        if(eight_rows && need > 4) return launch_stream32<1, 1, 8, 8, MODE, 8>(a, f, st, g);
         if(need > 4 && half_rows && kernel_override() % 1000 != 670)
           return launch_stream32<1, 1, 8, 8, MODE, 16>(a, f, st, g);   // long rows: half as many chunks (measurement id 670 keeps the shorter ones)
         if(need > 2) {
@@ -481,7 +482,8 @@ int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int
 // that work halves and the workgroups double - taken when they still fit one per CU.
 struct TiledPlan {
   int kw;
-  bool half_rows;
+  bool half_rows;    // 16 rows
+  bool eight_rows;   // 8, for long rows
 };
 TiledPlan plan_tiled(int M, int K, int n_out, int kw_override) {
   const int tiles = (n_out + 31) / 32, m_tiles = (M + 31) / 32;
@@ -489,10 +491,12 @@ TiledPlan plan_tiled(int M, int K, int n_out, int kw_override) {
   while(kw > 1 && (long long)((tiles * kw + 7) / 8) * m_tiles > compute_units()) kw >>= 1;
   if(kw_override) kw = kw_override;
   while(kw > 1 && K / 32 < kw) kw >>= 1;
-  const int ov = kernel_override() % 1000;   // 640 / 641: force 32 / 16 rows
+  const int ov = kernel_override() % 1000;   // 640 / 641 / 642: force 32 / 16 / 8 rows
   const long long blocks32 = (long long)((tiles * kw + 7) / 8) * m_tiles;
-  const bool half_rows = kw >= 4 && ov != 640 && (ov == 641 || (M > 16 && 2 * blocks32 <= compute_units()));
-  return TiledPlan{kw, half_rows};
+  const bool half_rows = kw >= 4 && ov != 640 && (ov == 641 || ov == 642 || (M > 16 && 2 * blocks32 <= compute_units()));
+  const bool eight_rows = half_rows && kw == 8 && K > 1024 && ov != 641 &&
+                          (ov == 642 || (long long)tiles * ((M + 7) / 8) <= compute_units());
+  return TiledPlan{kw, half_rows, eight_rows};
 }
 
 // kw_override: 0 = pick the K split from the number of workgroups it gives.
@@ -519,7 +523,7 @@ int launch_stream32_auto(const GemmArgs& a, const FusedSrc& f, hipStream_t st, i
   while(kw > 1 && a.K / 32 < kw) kw >>= 1;
   if constexpr(MODE == kFusedTiled) {
     const TiledPlan plan = plan_tiled(a.M, a.K, a.n_out, kw_override);
-    return launch_stream32_kw<1, MODE>(a, f, st, plan.kw, plan.half_rows);
+    return launch_stream32_kw<1, MODE>(a, f, st, plan.kw, plan.half_rows, nullptr, plan.eight_rows);
   } else {
     if constexpr(MODE == kFusedAll) {
       // The smallest inputs (at most two 16-value groups per thread of four waves): one wave per
@@ -1202,7 +1206,7 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
   // One launch for all matrices where the quantize-on-stage kernel takes the call (the same limits
   // as for a single matrix of the summed width).
   bool one_launch = false;
-  TiledPlan plan{1, false};
+  TiledPlan plan{1, false, false};
   if(total_blocks32 > 0 && (absmax_in || have_ws) && M <= 256 && total_blocks32 * 32 <= 8192) {
     plan = plan_tiled((int)M, (int)K, (int)(total_blocks32 * 32), 0);
     one_launch = K <= 1024 || (K <= 4096 && plan.kw == 8 && (long long)(plan.half_rows ? 16 : 32) * K <= 65536);
@@ -1232,7 +1236,7 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
       f.partials = partials;
       f.n_partials = g;
     }
-    return launch_stream32_kw<1, kFusedTiled>(a, f, hst, plan.kw, plan.half_rows, &gl);
+    return launch_stream32_kw<1, kFusedTiled>(a, f, hst, plan.kw, plan.half_rows, &gl, plan.eight_rows);
   }
   // Otherwise the activations are quantized once and every matrix gets its own multiplication.
   if(absmax_in) {

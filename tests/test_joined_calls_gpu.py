@@ -124,3 +124,21 @@ def test_grouped_matrices_behind_many_rows(M, K, N, relu):
         assert out.shape == (M, n)
         if n:
             assert same(out, integer.affine_f32(x, w, b, relu=relu)[0])
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 2048, 512), (23, 1088, 8), (64, 2048, 512), (57, 3008, 520), (33, 4096, 1000), (25, 1536, 2048)])
+@pytest.mark.parametrize("known", [False, True])
+def test_few_long_rows_equal_the_separate_passes(M, K, N, known):
+    """8-row tiles (rows of more than 1024 values, so few that CUs idle) against the quantizer and the multiplication as two launches"""
+    import torch
+    integer, L = load("integer"), load("_lib")
+    r, x, _, (gamma, _) = inputs(M, K, M + K + N)
+    w, b = integer.prepareB(r(K, N) * 0.02), r(N)
+    xmax = None
+    if known:
+        x, xmax = load("ops").layerNorm(x, gamma, want_absmax=True)
+    with L.forced_kernel(600):
+        want, want_q = integer.affine_f32(x, w, b, relu=True)
+    out, q, omax = integer.affine_f32(x, w, b, relu=True, absmax=xmax, want_absmax=True)
+    assert same(out, want) and torch.equal(q.data[:M * K + 4], want_q.data[:M * K + 4])
+    assert omax.data.max().item() == out.abs().max().item()
