@@ -44,6 +44,19 @@ inline int norm_input_check(const marian_hip_norm_input* n, const float* A, int6
   return MARIAN_HIP_OK;
 }
 
+// Compute units of the current device (looked up once per device; 256 if the query fails).
+inline int compute_units() {
+  static std::atomic<int> cus[kMaxDevices];
+  int dev = 0;
+  if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if(n > 0) return n;
+  if(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+    n = 256;
+  cus[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
+
 // Raises a kernel's dynamic LDS limit, once per kernel and device (`done`: one bit per device).
 template <typename KernelT>
 int allow_lds(KernelT kernel, int bytes, std::atomic<uint64_t>& done) {

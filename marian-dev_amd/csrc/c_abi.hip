@@ -82,19 +82,6 @@ int launch_stream(const GemmArgs& a, hipStream_t st) {
   return MARIAN_HIP_OK;
 }
 
-// Compute units of the current device (looked up once per device; 256 if the query fails).
-int compute_units() {
-  static std::atomic<int> cus[kMaxDevices];
-  int dev = 0;
-  if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if(n > 0) return n;
-  if(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  cus[dev].store(n, std::memory_order_relaxed);
-  return n;
-}
-
 // Whether a large-M launch of `workgroups` workgroups leaves the abs-max of its output itself: one
 // slot per workgroup (not for accumulator dumps).
 inline bool big_leaves_absmax(const GemmArgs& a, long long workgroups) {

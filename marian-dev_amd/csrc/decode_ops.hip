@@ -1046,13 +1046,13 @@ __global__ __launch_bounds__(256) void attention_shared_kernel(const float* __re
 
 // NPROJ: 3 (q, k_new, v_new: self-attention, the new key/value row is appended to the caches) or
 // 1 (q only: attention over caches that are complete, e.g. the encoder's).  R: input rows per
-// workgroup, 8 (a wave per row in the attention).
+// workgroup, 8 (a wave per row in the attention) or 4 (without staging: half of the waves attend).
 // NORM: the projections' input is the layer norm of A + norm.add, up to kNormMaxRows rows: every workgroup
 // normalizes all of them, a wave each, while its weights are on their way (a launch of its own for the norm
 // took 3.5 us of GPU and 4 of host time).
 template <int NPROJ, int R, int SEGS, int PASSES, bool NORM = false>
 __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttentionArgs p) {
-  static_assert(R == 8, "one wave per row in the attention");
+  static_assert(R == 8 || (R == 4 && !(SEGS > 0)), "a wave per row in the attention");
   constexpr bool STAGED = SEGS > 0;
   static_assert(!STAGED || NPROJ == 1, "keys and values are shared only where the caches are complete");
   static_assert(SEGS == 0 || SEGS == 2 || SEGS == 4, "keys and values of one or two sentences");
@@ -2470,8 +2470,12 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, int
   p.att_scale = att_scale; p.out = out; p.absmax_out = absmax_out;
   constexpr int R = 8;
   const int len4 = ((int)len + 3) & ~3;
-  size_t lds = (size_t)32 * (size_t)K + (size_t)n_proj * 8 * R * 128 + (size_t)n_proj * R * 64 * 4 +
-               (size_t)R * (size_t)(len4 + 256) * 4;
+  // Self-attention, every row its own caches: four rows to a workgroup where eight leave half of the CUs idle
+  // (what a workgroup fetches bounds it: 96 KB of weights and 17 KB a row for 65 rows of 8 heads over 34 positions).
+  const bool four = n_proj == 3 && 2 * heads * ((M + 7) / 8) <= compute_units();
+  const int rows = four ? 4 : R;
+  size_t lds = (size_t)32 * (size_t)K + (size_t)n_proj * 8 * rows * 128 + (size_t)n_proj * rows * 64 * 4 +
+               (size_t)rows * (size_t)(len4 + 256) * 4;
   {   // the kernels' dynamic LDS limit, raised once per device (one bit per device)
     static std::atomic<uint64_t> lds_done{0};
     int dev = 0;
@@ -2488,12 +2492,17 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, int
       for(const void* f : staged) MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kProjMaxLds));
       const void* unstaged[] = {
           reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, true>)};
+          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, true>),
+          reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, true>)};
       for(const void* f : unstaged) MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
       lds_done.fetch_or(1ull << dev, std::memory_order_release);
     }
   }
-  const ProjRowPlan plan = proj_row_plan(n_proj, M, heads, batchKV, len, kProjStageLen, lds, (size_t)kProjMaxLds);
+  ProjRowPlan plan = proj_row_plan(n_proj, M, heads, batchKV, len, kProjStageLen, lds, (size_t)kProjMaxLds);
+  if(four) {
+    plan.per_wg = 4;
+    plan.blocks_y = (M + 3) / 4;
+  }
   p.share_shift = plan.shift;
   p.share_nb = plan.sentences;
   p.share_hyps = plan.hyps;
@@ -2502,23 +2511,24 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, int
   if(plan.blocks_y > 65535) return MARIAN_HIP_ERR_RANGE;
   if(plan.stage) lds += (size_t)(2 << plan.shift) * (size_t)len * 256;
   const dim3 grid((unsigned)heads, (unsigned)plan.blocks_y);
-#define MH_PA(NP, SEGS, PASSES)                                                                                          \
-  do {                                                                                                                   \
-    if(norm) hipLaunchKernelGGL((proj_attention_kernel<NP, R, SEGS, PASSES, true>), grid, dim3(kProjThreads), lds, st, p); \
-    else hipLaunchKernelGGL((proj_attention_kernel<NP, R, SEGS, PASSES>), grid, dim3(kProjThreads), lds, st, p);           \
+#define MH_PA(NP, ROWS, SEGS, PASSES)                                                                                       \
+  do {                                                                                                                      \
+    if(norm) hipLaunchKernelGGL((proj_attention_kernel<NP, ROWS, SEGS, PASSES, true>), grid, dim3(kProjThreads), lds, st, p); \
+    else hipLaunchKernelGGL((proj_attention_kernel<NP, ROWS, SEGS, PASSES>), grid, dim3(kProjThreads), lds, st, p);           \
   } while(0)
-  if(n_proj == 3) MH_PA(3, 0, 0);
-  else if(!p.stage_kv) MH_PA(1, 0, 0);
+  if(four) MH_PA(3, 4, 0, 0);
+  else if(n_proj == 3) MH_PA(3, R, 0, 0);
+  else if(!p.stage_kv) MH_PA(1, R, 0, 0);
   else {
     const int passes = ((int)len + 31) / 32;   // 1 .. 3
     if(p.share_shift == 0) {   // one sentence per workgroup
-      if(passes == 1) MH_PA(1, 2, 1);
-      else if(passes == 2) MH_PA(1, 2, 2);
-      else MH_PA(1, 2, 3);
+      if(passes == 1) MH_PA(1, R, 2, 1);
+      else if(passes == 2) MH_PA(1, R, 2, 2);
+      else MH_PA(1, R, 2, 3);
     } else {
-      if(passes == 1) MH_PA(1, 4, 1);
-      else if(passes == 2) MH_PA(1, 4, 2);
-      else MH_PA(1, 4, 3);
+      if(passes == 1) MH_PA(1, R, 4, 1);
+      else if(passes == 2) MH_PA(1, R, 4, 2);
+      else MH_PA(1, R, 4, 3);
     }
   }
 #undef MH_PA

@@ -96,14 +96,14 @@ struct ProjRowPlan {
   int shift;       // log2 of the sentences per workgroup, or -1
   int sentences;
   int hyps;        // hypotheses per sentence
-  int per_wg;      // hypotheses of a sentence a workgroup takes
+  int per_wg;      // hypotheses of a sentence a workgroup takes; shift -1: consecutive rows it takes
   int stage;       // the sentences' keys and values are staged in LDS (shift 0 or 1, len <= stage_len)
   long long blocks_y;   // workgroups per head
 };
 __host__ __device__ __forceinline__ ProjRowPlan proj_row_plan(long long n_proj, long long M, long long heads, long long batchKV,
                                                               long long len, int stage_len, size_t lds_without,
                                                               size_t lds_max) {
-  ProjRowPlan plan = {-1, 0, 0, 0, 0, (M + 7) / 8};
+  ProjRowPlan plan = {-1, 0, 0, 8, 0, (M + 7) / 8};
   if(n_proj != 1 || heads <= 0 || batchKV % heads != 0) return plan;
   const long long nb = batchKV / heads;
   if(nb <= 0 || nb >= M || M % nb != 0 || nb > 2147483647LL) return plan;
@@ -137,7 +137,7 @@ __host__ __device__ __forceinline__ ProjRowPlan proj_row_plan(long long n_proj, 
 }
 // input row r (0 .. 7) of workgroup block_y; rows that do not exist: a value of at least M (= hyps * sentences)
 __host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, int hyps, int per_wg, int block_y, int r) {
-  if(shift < 0) return block_y * 8 + r;
+  if(shift < 0) return block_y * per_wg + r;
   const int groups = sentences >> shift;
   const int j = r >> shift, hyp = (block_y / groups) * per_wg + j;
   if(j >= per_wg || hyp >= hyps) return 0x7fffffff;
