@@ -247,6 +247,15 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
                                    int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
                                    float* out, const float* absmax_in, float* absmax_out, void* workspace,
                                    size_t workspace_bytes, void* stream);
+/* The self-attention form (n_proj = 3) over caches that stay where they were written: position p < len - 1 of
+ * hypothesis m is read from the entry of hypothesis ancestors[m * kv_capacity + p] (see marian_hip_attention_ancestors).
+ * norm: NULL, or the layer norm in front (M <= 8; Aq, absmax_in and workspace are then not used and may be NULL). */
+int marian_hip_int8_proj_attention_ancestors(const float* A, const marian_hip_norm_input* norm, int8_t* Aq,
+                                             const int8_t* const* Bq, const float* const* bias, float* const* proj_out,
+                                             int64_t M, int64_t K, int64_t heads, float* k_cache, float* v_cache,
+                                             int64_t len, int64_t kv_capacity, const uint32_t* ancestors,
+                                             float att_scale, float* out, const float* absmax_in, float* absmax_out,
+                                             void* workspace, size_t workspace_bytes, void* stream);
 /* The same with the layer norm in front (M <= 8; x goes to norm->out, its quantized form nowhere). */
 int marian_hip_int8_proj_attention_normed(const float* A, const marian_hip_norm_input* norm, int64_t n_proj,
                                           const int8_t* const* Bq, const float* const* bias, float* const* proj_out,

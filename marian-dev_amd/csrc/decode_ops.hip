@@ -862,6 +862,7 @@ struct ProjAttentionArgs {
   // With it (and sentences two or one to a workgroup, len <= kProjStageLen): the keys and values of
   // the workgroup's sentences are read once, into LDS, and every hypothesis' wave takes them from there.
   int stage_kv;
+  const uint32_t* anc;      // (ANC) [M, kv_cap]: the hypothesis in whose entry a cached position lies
   NormInput norm;           // (NORM) A is what the layer norm in front of the projections reads
 };
 
@@ -883,11 +884,20 @@ __device__ __forceinline__ int proj_row_key(int c16) { return (c16 ^ (c16 >> 2))
 // same operations in the same order, so the result has the same bits.  q, k_last, v_last may lie
 // in LDS.  sc: len4 floats of this wave, part: 256 floats behind them.  Returns |out| of this lane.
 // LAST_IN_ROWS: k_last and v_last are row len - 1 of kb and vb (one address computation for all rows).
-template <bool LAST_IN_ROWS = false>
+// ANC: kb and vb are the whole caches, and cached position p lies in the entry of hypothesis anc.row[p], as in
+// attention_kernel's form of that name; anc.first: row[min(4 u + lane / 16, len - 1)], requested by the caller.
+constexpr int kAttU = 16;
+struct Ancestors {
+  const uint32_t* row;
+  unsigned n_hyp, heads, head;
+  int kv_cap;
+  unsigned first[kAttU];
+};
+template <bool LAST_IN_ROWS = false, bool ANC = false>
 __device__ __forceinline__ float attention_row64(const float* q, const float* kb, const float* vb, const float* k_last,
                                                  const float* v_last, const float* mk, float mk0, int len, float scale, float* sc,
-                                                 float* part, float* out_row, int lane) {
-  constexpr int kAttU = 16, dk = 64;
+                                                 float* part, float* out_row, int lane, const Ancestors* anc = nullptr) {
+  constexpr int dk = 64;
   const int len4 = (len + 3) & ~3;
   const int g = lane / 16, c = lane % 16;
   const int u_last = (len + 2 - g) / 4;
@@ -899,7 +909,12 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
       if(base + 4 * u < len) {
         const int U = base / 4 + u;
         if constexpr(LAST_IN_ROWS) r[u] = *reinterpret_cast<const v4f*>(rows + (size_t)min(4 * U + g, len - 1) * dk + 4 * c);
-        else if(U >= u_last) r[u] = *reinterpret_cast<const v4f*>(last_c);
+        else if constexpr(ANC) {
+          unsigned from = base == 0 ? anc->first[u] : anc->row[min(4 * U + g, len - 1)];
+          from = min(from, anc->n_hyp - 1u);
+          const float* at = rows + ((size_t)(from * anc->heads + anc->head) * anc->kv_cap + (size_t)(4 * U + g)) * dk + 4 * c;
+          r[u] = *reinterpret_cast<const v4f*>(U >= u_last ? last_c : at);
+        } else if(U >= u_last) r[u] = *reinterpret_cast<const v4f*>(last_c);
         else r[u] = *reinterpret_cast<const v4f*>(first + (size_t)U * 4 * dk);
       } else if(base + 4 * (u & ~3) < len) {
         r[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1050,7 +1065,8 @@ __global__ __launch_bounds__(256) void attention_shared_kernel(const float* __re
 // NORM: the projections' input is the layer norm of A + norm.add, up to kNormMaxRows rows: every workgroup
 // normalizes all of them, a wave each, while its weights are on their way (a launch of its own for the norm
 // took 3.5 us of GPU and 4 of host time).
-template <int NPROJ, int R, int SEGS, int PASSES, bool NORM = false>
+// ANC: the self-attention's cached positions are read through the table of ancestors (attention_kernel's ANC).
+template <int NPROJ, int R, int SEGS, int PASSES, bool NORM = false, bool ANC = false>
 __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttentionArgs p) {
   static_assert(R == 8 || (R == 4 && !(SEGS > 0)), "a wave per row in the attention");
   constexpr bool STAGED = SEGS > 0;
@@ -1116,6 +1132,14 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
     mk = p.mask + (size_t)mask_row * p.len;
   }
   const float mk0 = *(mk ? mk + min(lane, p.len - 1) : p.A);   // (the latter not looked at)
+  Ancestors anc;
+  if constexpr(ANC) {   // (unconditional: waits count)
+    static_assert(NPROJ == 3 && !STAGED, "self-attention");
+    anc.row = p.anc + (size_t)min(m_wave, M - 1) * p.kv_cap;
+    anc.n_hyp = (unsigned)M; anc.heads = (unsigned)p.heads; anc.head = (unsigned)h; anc.kv_cap = p.kv_cap;
+#pragma unroll
+    for(int u = 0; u < kAttU; ++u) anc.first[u] = anc.row[min(4 * u + lane / 16, p.len - 1)];
+  }
   float bqm[NPROJ];
 #pragma unroll
   for(int g = 0; g < NPROJ; ++g) bqm[g] = tail_quant_mult(p.Bq[g], (size_t)K * (size_t)N);
@@ -1282,6 +1306,9 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
       const float* vs = ks + (size_t)p.len * 64;
       omax = attention_row64<true>(q, ks, vs, ks + (size_t)(p.len - 1) * 64, vs + (size_t)(p.len - 1) * 64, mk, mk0, p.len,
                              p.att_scale, sc, sc + len4, p.out + (size_t)wr * 64, lane);
+    } else if constexpr(ANC) {
+      omax = attention_row64<false, true>(q, p.k_cache, p.v_cache, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
+                                          p.out + (size_t)wr * 64, lane, &anc);
     } else {
       omax = attention_row64(q, kb, vb, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
                              p.out + (size_t)wr * 64, lane);
@@ -2405,7 +2432,7 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
   return MARIAN_HIP_OK;
 }
 
-static int proj_attention(const float* A, const marian_hip_norm_input* norm, int8_t* Aq, int64_t n_proj, const int8_t* const* Bq,
+static int proj_attention(const float* A, const marian_hip_norm_input* norm, const uint32_t* anc, int8_t* Aq, int64_t n_proj, const int8_t* const* Bq,
                           const float* const* bias, float* const* proj_out, int64_t M, int64_t K,
                           int64_t heads, float* k_cache, float* v_cache, int64_t batchKV, int64_t len,
                           int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
@@ -2442,6 +2469,7 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, int
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   p.A = A; p.aq_out = Aq;
   p.norm = NormInput{nullptr, nullptr, nullptr, nullptr, 0.0f};
+  p.anc = anc;
   p.partials = nullptr;
   p.n_partials = 0;
   if(norm) {
@@ -2493,7 +2521,9 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, int
       const void* unstaged[] = {
           reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0>),
           reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, true>),
-          reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, true>)};
+          reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, true>),
+          reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, false, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, true, true>),
+          reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, false, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, true, true>)};
       for(const void* f : unstaged) MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
       lds_done.fetch_or(1ull << dev, std::memory_order_release);
     }
@@ -2516,7 +2546,14 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, int
     if(norm) hipLaunchKernelGGL((proj_attention_kernel<NP, ROWS, SEGS, PASSES, true>), grid, dim3(kProjThreads), lds, st, p); \
     else hipLaunchKernelGGL((proj_attention_kernel<NP, ROWS, SEGS, PASSES>), grid, dim3(kProjThreads), lds, st, p);           \
   } while(0)
-  if(four) MH_PA(3, 4, 0, 0);
+#define MH_PAA(ROWS, NORM) \
+  hipLaunchKernelGGL((proj_attention_kernel<3, ROWS, 0, 0, NORM, true>), grid, dim3(kProjThreads), lds, st, p)
+  if(anc) {
+    if(four && norm) MH_PAA(4, true);
+    else if(four) MH_PAA(4, false);
+    else if(norm) MH_PAA(R, true);
+    else MH_PAA(R, false);
+  } else if(four) MH_PA(3, 4, 0, 0);
   else if(n_proj == 3) MH_PA(3, R, 0, 0);
   else if(!p.stage_kv) MH_PA(1, R, 0, 0);
   else {
@@ -2532,6 +2569,7 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, int
     }
   }
 #undef MH_PA
+#undef MH_PAA
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2542,8 +2580,20 @@ int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, c
                                    int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
                                    float* out, const float* absmax_in, float* absmax_out, void* workspace,
                                    size_t workspace_bytes, void* stream) {
-  return proj_attention(A, nullptr, Aq, n_proj, Bq, bias, proj_out, M, K, heads, k_cache, v_cache, batchKV, len, kv_capacity, mask,
+  return proj_attention(A, nullptr, nullptr, Aq, n_proj, Bq, bias, proj_out, M, K, heads, k_cache, v_cache, batchKV, len, kv_capacity, mask,
                         n_masks, att_scale, out, absmax_in, absmax_out, workspace, workspace_bytes, stream);
+}
+
+int marian_hip_int8_proj_attention_ancestors(const float* A, const marian_hip_norm_input* norm, int8_t* Aq, const int8_t* const* Bq,
+                                             const float* const* bias, float* const* proj_out, int64_t M, int64_t K, int64_t heads,
+                                             float* k_cache, float* v_cache, int64_t len, int64_t kv_capacity,
+                                             const uint32_t* ancestors, float att_scale, float* out, const float* absmax_in,
+                                             float* absmax_out, void* workspace, size_t workspace_bytes, void* stream) {
+  if(!ancestors) return MARIAN_HIP_ERR_NULL;
+  if(!aligned4(ancestors)) return MARIAN_HIP_ERR_ALIGN;
+  if(M < 0 || heads <= 0 || M > kMaxElemsOps / heads) return MARIAN_HIP_ERR_SHAPE;
+  return proj_attention(A, norm, ancestors, Aq, 3, Bq, bias, proj_out, M, K, heads, k_cache, v_cache, M ? M * heads : 1, len, kv_capacity,
+                        nullptr, 0, att_scale, out, absmax_in, absmax_out, workspace, workspace_bytes, stream);
 }
 
 int marian_hip_int8_proj_attention_normed(const float* A, const marian_hip_norm_input* norm, int64_t n_proj, const int8_t* const* Bq,
@@ -2552,7 +2602,7 @@ int marian_hip_int8_proj_attention_normed(const float* A, const marian_hip_norm_
                                           int64_t kv_capacity, const float* mask, int64_t n_masks, float att_scale,
                                           float* out, float* absmax_out, void* stream) {
   if(!norm) return MARIAN_HIP_ERR_NULL;
-  return proj_attention(A, norm, nullptr, n_proj, Bq, bias, proj_out, M, K, heads, k_cache, v_cache, batchKV, len, kv_capacity, mask,
+  return proj_attention(A, norm, nullptr, nullptr, n_proj, Bq, bias, proj_out, M, K, heads, k_cache, v_cache, batchKV, len, kv_capacity, mask,
                         n_masks, att_scale, out, nullptr, absmax_out, nullptr, 0, stream);
 }
 

@@ -39,7 +39,7 @@ namespace {
   F(int8_workspace_bytes) F(int8_prepare_a) F(int8_prepare_b) F(int8_prepare_b_quantized_transposed)     \
   F(int8_affine_f32) F(int8_affine_f32_chained) F(int8_affine_f32_grouped) F(int8_proj_attention)        \
   F(int16_prepare_a) F(int16_prepare_b) F(int16_prepare_b_quantized_transposed) F(int16_affine_f32)      \
-  F(int16_scratch_bytes) F(int8_affine_f32_normed) F(int8_proj_attention_normed)                                                                                 \
+  F(int16_scratch_bytes) F(int8_affine_f32_normed) F(int8_proj_attention_normed) F(int8_proj_attention_ancestors)                                                                                 \
   F(layer_norm) F(embed) F(attention_cached) F(attention_rows) F(attention_ancestors) F(ancestors_advance)                 \
   F(select_state) F(nbest) F(nbest_words) F(nbest_beams) F(nbest_beams_workspace_bytes) F(nbest_beams_workspace_init)   \
   F(logsoftmax_nbest_beams)
@@ -791,6 +791,55 @@ PyObject* py_proj_attention_normed(PyObject*, PyObject* const* args, Py_ssize_t 
   MH_END
 }
 
+// proj_attention_ancestors(a, add or None, (gamma, beta), eps, weights, k, v, ancestors, kvLen, absmax, want_projections)
+//   -> (x, out, absmax of out, [projections] or None); add None: x is a itself
+PyObject* py_proj_attention_ancestors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(11, "proj_attention_ancestors");
+  const bool with_norm = !none(args[1]);
+  Normed r;
+  const at::Tensor *k = f32c(args[5]), *v = f32c(args[6]), *anc = tensor(args[7]);
+  const float* amax = nullptr;
+  if(with_norm ? !normed(args[0], args[1], args[2], args[3], r) : !(r.a = f32c(args[0]))) Py_RETURN_NONE;
+  if(r.a->dim() < 1) Py_RETURN_NONE;
+  r.K = r.a->size(-1);
+  r.M = r.K ? r.a->numel() / r.K : 0;
+  Matrices w;
+  const int64_t heads = r.K / 64;
+  if(r.M < 1 || r.K % 128 != 0 || r.K > 1024 || r.M * heads > MARIAN_HIP_ABSMAX_SLOTS || !k || !v || k->dim() != 3 || k->size(-1) != 64 ||
+     k->sizes() != v->sizes() || k->size(0) != r.M * heads || !anc || !ids_type(anc->scalar_type()) || anc->device() != r.a->device() ||
+     !anc->is_contiguous() || anc->dim() != 2 || anc->size(0) != r.M || anc->size(1) != k->size(1) ||
+     !matrices(args[4], r.K, true, w) || w.n != 3 || !absmax_in(args[9], &amax))
+    Py_RETURN_NONE;
+  for(int g = 0; g < 3; ++g)
+    if(w.b[g].cols != r.K) Py_RETURN_NONE;
+  const int64_t len = whole(args[8]), cap = k->size(1);
+  if(len < 1 || len > cap || len > 512) Py_RETURN_NONE;
+  const bool want_proj = truth(args[10]);
+  const c10::Device d = r.a->device();
+  at::Tensor out = empty(r.a->sizes(), at::kFloat, d), omax = absmax_slots(d), projections[3], aq;
+  if(!with_norm) aq = quantized_buffer(r.M * r.K, 1, d);
+  float* proj[3] = {nullptr, nullptr, nullptr};
+  if(want_proj)
+    for(int g = 0; g < 3; ++g) {
+      projections[g] = empty(r.a->sizes(), at::kFloat, d);
+      proj[g] = fptr_mut(projections[g]);
+    }
+  const hipStream_t st = stream_of(d);
+  const at::Tensor& ws = workspace(d, st);
+  call("ProjectedAttention", [&] {
+    return L.int8_proj_attention_ancestors(fptr(r.a), with_norm ? &r.n : nullptr, with_norm ? nullptr : static_cast<int8_t*>(aq.data_ptr()),
+                                           w.Bq, w.bias, proj, r.M, r.K, heads, fptr_mut(*k), fptr_mut(*v), len, cap,
+                                           static_cast<const uint32_t*>(anc->const_data_ptr()), 1.0f / 8.0f, fptr_mut(out), amax,
+                                           fptr_mut(omax), ws.data_ptr(), (size_t)ws.numel(), st);
+  });
+  Ref x(with_norm ? wrap(std::move(r.x)) : (Py_INCREF(args[0]), args[0])), o(wrap(std::move(out))), m(make_absmax(std::move(omax)));
+  if(!want_proj) return PyTuple_Pack(4, x.p, o.p, m.p, Py_None);
+  Ref list(ok(PyList_New(3)));
+  for(int g = 0; g < 3; ++g) PyList_SET_ITEM(list.p, g, wrap(std::move(projections[g])));
+  return PyTuple_Pack(4, x.p, o.p, m.p, list.p);
+  MH_END
+}
+
 // attention_ancestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax) -> out or (out, absmax)
 PyObject* py_attention_ancestors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_TRY MH_ARGS(8, "attention_ancestors");
@@ -964,7 +1013,7 @@ PyObject* py_setup(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 #define MH_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&py_##name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
-    MH_METHOD(affine_f32_grouped), MH_METHOD(affine_f32_normed), MH_METHOD(proj_attention_normed), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
+    MH_METHOD(affine_f32_grouped), MH_METHOD(affine_f32_normed), MH_METHOD(proj_attention_normed), MH_METHOD(proj_attention_ancestors), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
     MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(attention_rows), MH_METHOD(split_heads), MH_METHOD(join_heads), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors),
     MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_words), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),
     {nullptr, nullptr, 0, nullptr}};

@@ -134,7 +134,7 @@ class DecoderStep:
         """The layers and the output layer for a handful of hypotheses: every layer norm is taken by the
         launch that multiplies its result (the launches of their own were a fifth of the step for six
         hypotheses of one sentence).  rec: None, or records the operator calls."""
-        integer, ops, H, M = self.integer, self.ops, self.H, self.M
+        integer, ops, H = self.integer, self.ops, self.H
         pending = None   # (a, skip, ln): x is still to be taken as the layer norm of a + skip
         for li, ly in enumerate(W["layers"]):
             qkv = [ly["Wq"], ly["Wk"], ly["Wv"]]
@@ -142,12 +142,9 @@ class DecoderStep:
             if rec:
                 k_before, v_before = k_cache.clone(), v_cache.clone()
             if self.by_ancestors:
-                if pending:
-                    x, (q, k, v), _ = ops.affineOfLayerNorm(*pending, qkv)
-                else:
-                    (q, k, v), _ = integer.affine_f32_grouped(x, qkv, absmax=xmax)
-                o, omax = ops.AttentionByAncestors(q, k_cache, v_cache, self.anc, self.T, k, v, want_absmax=True)
-                o = o.view(M, self.d)
+                a, add, ln = pending or (x, None, None)
+                x, o, omax, proj = ops.ProjectedAttentionByAncestors(a, qkv, k_cache, v_cache, self.anc, self.T, add, ln, absmax=xmax,
+                                                                     want_projections=bool(rec))
             elif pending:
                 x, o, omax, proj = ops.ProjectedAttentionOfLayerNorm(*pending, qkv, k_cache, v_cache, H, kvLen=self.T,
                                                                      want_projections=bool(rec))
@@ -156,8 +153,7 @@ class DecoderStep:
                                              want_projections=bool(rec))
                 o, omax, proj = res[0], res[2], res[3] if rec else None
             if rec:
-                if not self.by_ancestors:
-                    q, k, v = proj
+                q, k, v = proj
                 if pending:
                     rec("layer_norm", x=pending[0], add=pending[1], gamma=pending[2][0], beta=pending[2][1], out=x)
                 for name, t in (("Wq", q), ("Wk", k), ("Wv", v)):
@@ -232,6 +228,17 @@ class DecoderStep:
                 o, omax = res[0], res[2]
                 if tr is not None:
                     q, k, v = res[3]
+                    for name, t in (("Wq", q), ("Wk", k), ("Wv", v)):
+                        rec("affine", a=x, w=ly[name], out=t, relu=False)
+                    rec("self_attention", q=q, k_new=k, v_new=v, k_cache=k_before, v_cache=v_before,
+                        k_after=self.Kself[li], v_after=self.Vself[li], out=o, len=self.T)
+            elif fused_attention and not gemm_only and ch and grouped:   # the same over the table of ancestors
+                if tr is not None:
+                    k_before, v_before = self.Kself[li].clone(), self.Vself[li].clone()
+                _, o, omax, proj = ops.ProjectedAttentionByAncestors(x, [ly["Wq"], ly["Wk"], ly["Wv"]], self.Kself[li], self.Vself[li],
+                                                                     self.anc, self.T, absmax=xmax, want_projections=tr is not None)
+                if tr is not None:
+                    q, k, v = proj
                     for name, t in (("Wq", q), ("Wk", k), ("Wv", v)):
                         rec("affine", a=x, w=ly[name], out=t, relu=False)
                     rec("self_attention", q=q, k_new=k, v_new=v, k_cache=k_before, v_cache=v_before,

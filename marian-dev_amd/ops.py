@@ -328,6 +328,28 @@ def ProjectedAttentionOfLayerNorm(a, add, ln, weights, k, v, heads, kvLen=None, 
     return x, res[0], res[2], res[3] if want_projections else None
 
 
+def ProjectedAttentionByAncestors(a, weights, k, v, ancestors, kvLen, add=None, ln=None, eps=1e-6, absmax=None, want_projections=False):
+    """Self-attention of one new position per hypothesis over caches that stay where they were written: the
+    projections q, k, v of x and AttentionByAncestors in one launch (up to 256 hypotheses, where it pays, of up to
+    1024 values, 512 positions), otherwise as separate calls, with the same bits.  x is a [M, K], or with `add` and
+    ln = (gamma, beta) layerNorm(a, *ln, eps, add=add).  Returns (x, out [M, K], AbsMax of out, the projections
+    when asked for or None)."""
+    if len(ancestors) <= 256:
+        res = _host.proj_attention_ancestors(a, add, ln, eps, weights, k, v, ancestors, kvLen, absmax, want_projections)
+        if res is not None:
+            return res
+    from . import integer
+    if add is not None:
+        a, absmax = layerNorm(a, *ln, eps=eps, add=add, want_absmax=True)
+        if len(ancestors) <= 256:
+            res = _host.proj_attention_ancestors(a, None, None, eps, weights, k, v, ancestors, kvLen, absmax, want_projections)
+            if res is not None:
+                return res
+    qkv, _ = integer.affine_f32_grouped(a, weights, absmax=absmax)
+    o, omax = AttentionByAncestors(qkv[0], k, v, ancestors, kvLen, qkv[1], qkv[2], want_absmax=True)
+    return a, o.view(a.shape), omax, qkv if want_projections else None
+
+
 def AttentionByAncestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax=False):
     """Self-attention of a decoding step on caches that are never moved (no counterpart in the
     reference, which copies the surviving hypotheses' states, src/rnn/types.h:22-42): cached

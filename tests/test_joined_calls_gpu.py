@@ -142,3 +142,26 @@ def test_few_long_rows_equal_the_separate_passes(M, K, N, known):
     out, q, omax = integer.affine_f32(x, w, b, relu=True, absmax=xmax, want_absmax=True)
     assert same(out, want) and torch.equal(q.data[:M * K + 4], want_q.data[:M * K + 4])
     assert omax.data.max().item() == out.abs().max().item()
+
+
+@pytest.mark.parametrize("M,heads,length,cap", [(1, 2, 1, 1), (6, 8, 12, 12), (8, 16, 65, 70), (37, 4, 33, 40), (128, 16, 21, 30), (64, 2, 130, 130),
+                                                (257, 2, 9, 9), (5, 8, 513, 520)])   # (the last two: separate calls)
+@pytest.mark.parametrize("norm", [False, True])
+def test_projected_attention_by_ancestors(M, heads, length, cap, norm):
+    import torch
+    integer, ops = load("integer"), load("ops")
+    K = heads * 64
+    r, a, add, ln = inputs(M, K, M + K + length)
+    weights = [(integer.prepareB(r(K, K) * 0.02), r(K) if i != 2 else None) for i in range(3)]
+    k, v = r(M * heads, cap, 64), r(M * heads, cap, 64)
+    k_s, v_s = k.clone(), v.clone()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    anc = torch.randint(0, M + 2, (M, cap), device="cuda", generator=g).to(torch.int32)   # (entries past the last hypothesis: clamped)
+    x, xmax = ops.layerNorm(a, *ln, eps=1e-6, add=add, want_absmax=True)
+    args = (a, weights, k, v, anc, length, add, ln) if norm else (x, weights, k, v, anc, length)
+    got_x, out, omax, proj = ops.ProjectedAttentionByAncestors(*args, absmax=None if norm else xmax, want_projections=True)
+    qkv, _ = integer.affine_f32_grouped(x, weights, absmax=xmax)
+    out_s, omax_s = ops.AttentionByAncestors(qkv[0], k_s, v_s, anc, length, qkv[1], qkv[2], want_absmax=True)
+    assert same(got_x, x) and same(out, out_s.view(out.shape)) and same(k, k_s) and same(v, v_s)
+    assert all(same(p, q) for p, q in zip(proj, qkv)) and omax.data.max().item() == omax_s.data.max().item()
