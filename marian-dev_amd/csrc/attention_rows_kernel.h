@@ -22,6 +22,7 @@ struct AttentionRowsArgs {
   unsigned batchQ, batchKV, heads, n_masks, rows_per_mask;
   int m, len, row_blocks, row_groups;   // blocks of 16 query rows, and over how many workgroups a head's are dealt out
   float scale;
+  int head_mask;   // all query rows of a head have the same mask row: it is looked up and loaded once
 };
 
 typedef v4f v4f_any __attribute__((aligned(4)));   // sixteen bytes at any float's address
@@ -62,8 +63,9 @@ __device__ __forceinline__ v4f rows_to_registers(v4f m) {
 // softmax_kernel's.  A rounding that moves here moves an 8-bit quantization further down the network.
 // Bound by its chains for a few heads, by the float32 matrix rate (16 x 16 x 4 in 32 clocks: 1024 heads of 64 x 64 take
 // 6.8 us at 2.4 GHz) and the traffic (67 MB there) for many.
-// Measured (in a graph, masks included): 8 heads of 23 x 23 4.1 us, 128 of 64 x 64 6.2, 1024 of 64 x 64 23.1, 384 of 128 x 128
-// 29.5.  Before, 1024 heads took three operators of 59 us and four transpositions of 32 us, one sentence 8.7 us with
+// Measured (in a graph, masks included): 8 heads of 23 x 23 4.1 us, 128 of 64 x 64 6.2, 1024 of 64 x 64 22.0, 384 of 128 x 128
+// 28.1 (23.1 and 29.4 with a mask row looked up and loaded per block of query rows; fewer resident workgroups or staggered starts
+// change nothing).  Before, 1024 heads took three operators of 59 us and four transpositions of 32 us, one sentence 8.7 us with
 // a wave to 16 rows and all keys (no LDS, the same bits).
 template <int NB>
 __global__ __launch_bounds__(256, NB == 1 ? 4 : (NB == 2 ? 3 : 2)) void attention_rows_kernel(AttentionRowsArgs p) {
@@ -90,21 +92,22 @@ __global__ __launch_bounds__(256, NB == 1 ? 4 : (NB == 2 ? 3 : 2)) void attentio
   const int q_in = threadIdx.x / 16, q_at = threadIdx.x % 16;
   auto load_q = [&](int block) __attribute__((always_inline)) {   // (rows past the end: the last one again, not stored)
     q_next = *reinterpret_cast<const v4f*>(qb + min(block * 16 + q_in, p.m - 1) * q_row + 4 * q_at);
-    if(p.mask) {
-      unsigned mr = (entry * (unsigned)p.m + (unsigned)min(block * 16 + c, p.m - 1)) / p.rows_per_mask;
-      if(mr >= p.n_masks) mr %= p.n_masks;
-      const float* m = p.mask + (size_t)mr * p.len;
+  };
+  auto load_mask = [&](int block) __attribute__((always_inline)) {
+    unsigned mr = (entry * (unsigned)p.m + (unsigned)min(block * 16 + c, p.m - 1)) / p.rows_per_mask;
+    if(mr >= p.n_masks) mr %= p.n_masks;
+    const float* m = p.mask + (size_t)mr * p.len;
 #pragma unroll
-      for(int b = 0; b < NB; ++b)
+    for(int b = 0; b < NB; ++b)
 #pragma unroll
-        for(int r = 0; r < 4; ++r) mask_next[b][r] = m[min(64 * b + 16 * wave + 4 * g + r, p.len - 1)];
-    }
+      for(int r = 0; r < 4; ++r) mask_next[b][r] = m[min(64 * b + 16 * wave + 4 * g + r, p.len - 1)];
   };
   auto keep_q = [&](int turn) __attribute__((always_inline)) {
 #pragma unroll
     for(int y = 0; y < 4; ++y) q_lds[turn][q_in][16 * (q_at / 4) + 4 * y + q_at % 4] = q_next[y];
   };
   load_q(group);
+  if(p.mask) load_mask(group);
 #pragma unroll
   for(int b = 0; b < NB; ++b) {
     const float* src = kb + min(64 * b + 16 * wave + c, p.len - 1) * k_row + 4 * g;
@@ -149,6 +152,7 @@ __global__ __launch_bounds__(256, NB == 1 ? 4 : (NB == 2 ? 3 : 2)) void attentio
 #pragma unroll
       for(int r = 0; r < 4; ++r) mask[b][r] = mask_next[b][r];
     load_q(min(block + p.row_groups, p.row_blocks - 1));
+    if(p.mask && !p.head_mask) load_mask(min(block + p.row_groups, p.row_blocks - 1));
     // ---- scores ----
     v4f z[NB];
 #pragma unroll

@@ -2290,7 +2290,8 @@ int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const fl
   if(batchQ * groups > kMaxElemsOps / 256) return MARIAN_HIP_ERR_RANGE;
   if(absmax_out && batchQ * groups * 4 > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
   AttentionRowsArgs a{q, k, v, mask, out, absmax_out, hs.q, hs.k, hs.v, hs.out, (unsigned)batchQ, (unsigned)batchKV, (unsigned)heads,
-                      (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)row_blocks, (int)groups, scale};
+                      (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)row_blocks, (int)groups, scale,
+                      mask && rows_per_mask % m == 0};
   const dim3 grid((unsigned)(batchQ * groups));
 #define MH_ROWS(NB) hipLaunchKernelGGL(attention_rows_kernel<NB>, grid, dim3(256), 0, hst, a)
   if(len <= 64) MH_ROWS(1);

@@ -947,3 +947,20 @@ def test_advance_ancestors(ops, synth):
     t = dev(prev)
     assert L.lib().marian_hip_ancestors_advance(t.data_ptr(), t.data_ptr(), hyps, cap, 3, t.data_ptr(), None) == L.ERR_ALIAS
     assert L.lib().marian_hip_ancestors_advance(t.data_ptr(), t.data_ptr(), hyps, cap, cap, out.data_ptr(), None) == L.ERR_SHAPE
+
+
+@pytest.mark.parametrize("m,L", [(23, 23), (64, 64), (17, 100), (40, 130)])
+@pytest.mark.parametrize("rows_per_mask", ["row", "odd", "entry", "two entries"])
+def test_attention_over_masks_of_a_row_or_of_a_head(ops, synth, m, L, rows_per_mask):
+    """one mask row for all query rows of a head (looked up once) and several: bit for bit the three operators"""
+    import torch
+    heads, batch = 2, 3
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + L)
+    q, k, v = (torch.randn(batch * heads, n, 64, device="cuda", generator=g) for n in (m, L, L))
+    rpm = {"row": 1, "odd": 7, "entry": m, "two entries": heads * m}[rows_per_mask]
+    mask = -1e8 * (torch.rand((batch * heads * m + rpm - 1) // rpm, L, device="cuda", generator=g) < 0.3).float()
+    mask[:, 0] = 0.0
+    got = ops.Attention(q, k, v, mask, rowsPerMask=rpm)
+    w = ops.softmax(ops.bdot_legacy(q, k, transB=True, scalar=0.125), mask, rowsPerMask=rpm)
+    assert torch.equal(got, ops.bdot_legacy(w, v))
