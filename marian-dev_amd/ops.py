@@ -22,11 +22,14 @@ from .integer import _abort_if, _backend_of, _host, _on_gpu, _taken
 
 def _f32c(x, what):
     _abort_if(x.dtype != torch.float32, "{} expects float32, got {}", what, x.dtype)
-    if not x.is_contiguous() and x.dim() == 4 and x.device.type == "cuda":
-        t = x.transpose(1, 2)   # SplitHeads' view of rows: its copy head by head is the 0213 transpose
-        if t.is_contiguous():
-            return transpose0213(t)
+    if x.device.type == "cuda" and _heads_side_by_side(x):   # its copy head by head is the 0213 transpose
+        return transpose0213(x.transpose(1, 2))
     return x.contiguous()
+
+
+def _heads_side_by_side(t):
+    """SplitHeads' view of rows"""
+    return t.dim() == 4 and not t.is_contiguous() and t.transpose(1, 2).is_contiguous()
 
 
 def layerNorm(x, gamma, beta=None, eps=1e-9, add=None, want_absmax=False):
@@ -165,7 +168,9 @@ def transpose0213(a):
 def SplitHeads(input, dimHeads):
     """reference src/models/transformer.h:145-156: [beam, batch, steps, model] ->
     [batch * beam, heads, steps, depth].  The result is a view (the heads of a position side by side, as
-    the affine call wrote them): Attention reads it as it is, and what needs it head by head copies."""
+    the affine call wrote them): Attention reads it as it is, and what needs it head by head copies.
+    Memory of its own, head by head - for .view(), or for a cache that is appended to while `input` is
+    still needed - is SplitHeads(..).contiguous()."""
     out = _host.split_heads(input, dimHeads)
     if out is not None:
         return out
@@ -174,7 +179,7 @@ def SplitHeads(input, dimHeads):
 
 
 def JoinHeads(input, dimBeam=1):
-    """reference src/models/transformer.h:158-170; a view where the heads of a position lie side by side (the
+    """reference src/models/transformer.h:158-170; a view of `input` where the heads of a position lie side by side (the
     output of Attention on SplitHeads' views)"""
     out = _host.join_heads(input, dimBeam)
     if out is not None:
@@ -211,7 +216,8 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     one launch.  q: [batch*beam, heads, tgt, dk]; k, v: [batch(*beam), heads, len, dk].
     kNew, vNew [batch*beam*heads, dk]: key and value of the newest position of a decoding step;
     they stand for position len - 1 and are also stored there in k and v (the concatenation onto
-    the cached positions, src/models/transformer.h:683-700).
+    the cached positions, src/models/transformer.h:683-700); where k and v are SplitHeads' views, in the
+    tensors they are views of.  The output lies in memory as q does.
     kvLen: k and v have room for k.shape[-2] positions per entry, of which the first kvLen are in
     use (caches that stay in place from step to step); None: all of them."""
     m = q.shape[-2]
@@ -228,13 +234,11 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     if kNew is None:
         k, v = _f32c(k, "Attention"), _f32c(v, "Attention")
     else:
-        if not k.is_contiguous() and k.dim() == 4 and k.transpose(1, 2).is_contiguous():   # SplitHeads' view as a cache
-            kc, vc = _f32c(k, "Attention"), _f32c(v, "Attention")
-            out = Attention(q, kc, vc, mask, rowsPerMask, want_absmax, kNew, vNew, kvLen)
-            k.copy_(kc), v.copy_(vc)
-            return out
-        _abort_if(not (k.is_contiguous() and v.is_contiguous()), "Attention: the key/value cache must be contiguous{}", "")
+        _abort_if(not all(t.is_contiguous() or _heads_side_by_side(t) for t in (k, v)),
+                  "Attention: the key/value cache must be contiguous{}", "")
         kNew, vNew = _f32c(kNew, "Attention"), _f32c(vNew, "Attention")
+        if not (k.is_contiguous() and v.is_contiguous()):
+            return _attention_appending_to_views(q, k, v, mask, rowsPerMask, want_absmax, kNew, vNew, kvLen)
     _on_gpu(q)
     dk, cap = q.shape[-1], k.shape[-2]
     L = cap if kvLen is None else int(kvLen)
@@ -252,6 +256,25 @@ def Attention(q, k, v, mask=None, rowsPerMask=1, want_absmax=False, kNew=None, v
     if mask is not None:
         mask = _f32c(mask, "Attention").reshape(-1, L)
     return _taken(_host.attention(q, k, v, mask, rowsPerMask, want_absmax, kNew, vNew, L), "Attention")
+
+
+def _attention_appending_to_views(q, k, v, mask, rowsPerMask, want_absmax, kNew, vNew, kvLen):
+    """Attention with a new key and value over SplitHeads' views: the one position is written where the views have
+    it, and the attention reads them as they are (with the bits of the call on caches of their own)."""
+    _abort_if(tuple(v.shape) != tuple(k.shape) or q.shape[-1] != k.shape[-1], "Attention: key/value shapes {} {} vs dk {}",
+              tuple(k.shape), tuple(v.shape), q.shape[-1])
+    entries, heads, cap, dk = k.shape
+    L = cap if kvLen is None else int(kvLen)
+    _abort_if(not 0 < L <= min(cap, 4096), "Attention: {} positions in use of {} the cache has room for", L, cap)
+    _abort_if(q.shape[-2] != 1 or any(t.numel() != entries * heads * dk for t in (q, kNew, vNew)),
+              "Attention: one query, new key and new value of {} values per cache entry", dk)
+    _abort_if(want_absmax and entries * heads > _lib.ABSMAX_SLOTS, "Attention: the abs-max of up to {} query rows, got {}",
+              _lib.ABSMAX_SLOTS, entries * heads)
+    if mask is not None:
+        mask = _f32c(mask, "Attention").reshape(-1, L)
+    k[:, :, L - 1].copy_(kNew.view(entries, heads, dk))
+    v[:, :, L - 1].copy_(vNew.view(entries, heads, dk))
+    return Attention(q, k, v, mask, rowsPerMask, want_absmax, kvLen=L)
 
 
 def ProjectedAttention(x, weights, k, v, heads, kvLen=None, mask=None, absmax=None, want_absmax=False,

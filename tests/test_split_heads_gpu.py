@@ -62,3 +62,48 @@ def test_query_projection_over_views_refuses_what_it_refuses_over_copies():
         for caches in ((k, v), (k.contiguous(), v.contiguous())):
             with pytest.raises(RuntimeError):
                 ops.ProjectedAttention(a, w, *caches, heads, kvLen=used, mask=mask[:, :used].contiguous() if used else mask)
+
+
+@pytest.mark.parametrize("sentences,heads,dk,cap,used", [
+    (1, 2, 64, 2, None), (5, 8, 64, 33, 20), (3, 4, 64, 130, 129), (2, 16, 64, 40, 1), (2, 4, 32, 12, 11), (3, 2, 80, 70, None),
+    (2, 3, 6, 9, 5)])   # (6: rows that are not a multiple of 16 bytes)
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_appends_to_views(sentences, heads, dk, cap, used, masked):
+    """the same output as over copies, the new position in the views, nothing else of theirs touched"""
+    import torch
+    ops = load("ops")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(cap + dk)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    keys, values = r(1, sentences, cap, heads * dk), r(1, sentences, cap, heads * dk)
+    k, v = ops.SplitHeads(keys, heads), ops.SplitHeads(values, heads)
+    assert not k.is_contiguous() and k.data_ptr() == keys.data_ptr()
+    kc, vc = k.clone(memory_format=torch.contiguous_format), v.clone(memory_format=torch.contiguous_format)
+    n, L = sentences * heads, used or cap
+    q, kn, vn = r(n, 1, dk), r(n, dk), r(n, dk)
+    mask = r(sentences, L) if masked else None
+    args = dict(mask=mask, rowsPerMask=heads, want_absmax=True, kNew=kn, vNew=vn, kvLen=used)
+    want, wmax = ops.Attention(q, kc, vc, **args)
+    # (the call moves one position of each tensor, not the tensors)
+    before = torch.cuda.memory_stats()["allocated_bytes.all.allocated"]
+    got, gmax = ops.Attention(q, k, v, **args)
+    taken = torch.cuda.memory_stats()["allocated_bytes.all.allocated"] - before
+    assert dk % 4 != 0 or keys.numel() < 30000 or taken < 4 * keys.numel(), taken
+    assert same(got, want) and same(k, kc) and same(v, vc)
+    assert gmax.data.max().item() == wmax.data.max().item()
+
+
+def test_attention_refuses_appends_it_cannot_place():
+    import torch
+    ops = load("ops")
+    keys = torch.zeros(1, 3, 10, 512, device="cuda")
+    k, v = ops.SplitHeads(keys, 8), ops.SplitHeads(keys.clone(), 8)
+    one = lambda *s: torch.ones(*s, device="cuda")
+    good = dict(q=one(24, 1, 64), k=k, v=v, kNew=one(24, 64), vNew=one(24, 64))
+    long = ops.SplitHeads(torch.zeros(1, 1, 4097, 128, device="cuda"), 2)
+    for bad in (dict(q=one(24, 2, 64)), dict(q=one(16, 1, 64)), dict(q=one(24, 1, 32)), dict(kNew=one(23, 64)), dict(vNew=one(24, 32)),
+                dict(kvLen=0), dict(kvLen=11), dict(v=v[:, :, :9]), dict(v=v[..., ::2]), dict(k=k.transpose(2, 3)),
+                dict(k=k.contiguous().view(24, 10, 64)), dict(k=long, v=long, q=one(2, 1, 64), kNew=one(2, 64), vNew=one(2, 64))):
+        with pytest.raises(RuntimeError):
+            ops.Attention(**{**good, **bad})
+    assert not keys.any() and not v.any()   # (nothing was written for a call that is refused)
