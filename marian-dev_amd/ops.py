@@ -299,9 +299,10 @@ def ProjectedAttention(x, weights, k, v, heads, kvLen=None, mask=None, absmax=No
     n = len(weights)
     _abort_if(n not in (1, 3), "ProjectedAttention: one projection (q) or three (q, k, v), got {}", n)
     K, N = x.shape[-1], heads * 64
-    # the encoder's keys and values as SplitHeads' views: the two calls, which read them as they are
-    views = n == 1 and k.dim() == 4 and not (k.is_contiguous() and v.is_contiguous())
-    _abort_if(not (views or (k.is_contiguous() and v.is_contiguous())) or k.dtype != torch.float32 or v.dtype != torch.float32,
+    # caches that are SplitHeads' views: the separate calls, which read them as they are and append where they have the position
+    views = not (k.is_contiguous() and v.is_contiguous())
+    strided = k.dim() == 4 if n == 1 else all(t.is_contiguous() or _heads_side_by_side(t) for t in (k, v))
+    _abort_if((views and not strided) or k.dtype != torch.float32 or v.dtype != torch.float32,
               "ProjectedAttention: the key/value caches must be contiguous float32{}", "")
     _abort_if(k.shape[-1] != 64 or tuple(k.shape) != tuple(v.shape), "ProjectedAttention: head size 64, got caches {} {}",
               tuple(k.shape), tuple(v.shape))
@@ -314,11 +315,12 @@ def ProjectedAttention(x, weights, k, v, heads, kvLen=None, mask=None, absmax=No
         # (the limits of the one-launch form, which refuses them itself)
         _abort_if(K % 128 != 0 or K > 1024 or not 0 < L <= min(k.shape[-2], 512), "ProjectedAttention: rows of {} values over "
                   "{} of {} positions", K, L, k.shape[-2])
-        (bQuant, bias), = weights
-        q, aq = integer.affine_f32(x, bQuant, bias, absmax=absmax)
-        o = Attention(q.reshape(q.numel() // 64, 1, 64), k, v, mask, rowsPerMask=heads, want_absmax=want_absmax, kvLen=L)
+        qkv, aq = integer.affine_f32_grouped(x, weights, absmax=absmax)
+        rows = qkv[0].numel() // 64
+        q, kNew, vNew = [t.view(rows, 64) for t in qkv] if n == 3 else (qkv[0].view(rows, 64), None, None)
+        o = Attention(q.view(rows, 1, 64), k, v, mask, heads, want_absmax, kNew, vNew, L)
         o, omax = o if want_absmax else (o, None)
-        return (o.reshape(q.shape), aq) + ((omax,) if want_absmax else ()) + (([q],) if want_projections else ())
+        return (o.view(qkv[0].shape), aq) + ((omax,) if want_absmax else ()) + ((qkv,) if want_projections else ())
     weights = [(bQuant, None if bias is None else _f32c(bias, "ProjectedAttention")) for bQuant, bias in weights]
     if mask is not None:
         mask = _f32c(mask, "ProjectedAttention").reshape(-1, L)

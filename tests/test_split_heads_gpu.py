@@ -41,7 +41,7 @@ def test_query_projection_over_views(hyps, sentences, heads, length, used):
     assert got[2].data.max().item() == want[2].data.max().item()
 
 
-def test_query_projection_over_views_refuses_what_it_refuses_over_copies():
+def test_projections_over_views_refuse_what_they_refuse_over_copies():
     import torch
     integer, ops = load("integer"), load("ops")
     r, x, weights, mask, keys, values = inputs(2, 3, 8, 20, 5)
@@ -58,10 +58,36 @@ def test_query_projection_over_views_refuses_what_it_refuses_over_copies():
              (x, weights[:1], heads8[0].double(), heads8[1].double(), 8, None),
              (x, weights[:1], *heads8, 8, 21), (x, weights[:1], *heads8, 8, 0),
              (torch.ones(6, 576, device="cuda"), long, *heads8, 8, None)]
+    with pytest.raises(RuntimeError):   # (six rows, the caches of three sentences)
+        ops.ProjectedAttention(x, weights, *heads8, 8)
     for a, w, k, v, heads, used in calls:
         for caches in ((k, v), (k.contiguous(), v.contiguous())):
             with pytest.raises(RuntimeError):
                 ops.ProjectedAttention(a, w, *caches, heads, kvLen=used, mask=mask[:, :used].contiguous() if used else mask)
+
+
+@pytest.mark.parametrize("rows,heads,length,used", [(1, 2, 2, None), (6, 8, 23, 12), (65, 8, 34, 34), (3, 16, 130, 129), (2, 4, 512, 1)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_three_projections_over_views(rows, heads, length, used, masked):
+    """self-attention: the same results as over copies, the new position in the views"""
+    ops = load("ops")
+    r, x, weights, mask, keys, values = inputs(1, rows, heads, length, rows + length)
+    mask = mask[:, :used].contiguous() if masked else None
+    k, v = ops.SplitHeads(keys, heads), ops.SplitHeads(values, heads)
+    kc, vc = k.contiguous(), v.contiguous()
+    args = dict(kvLen=used, mask=mask, want_absmax=True, want_projections=True)
+    want = ops.ProjectedAttention(x, weights, kc, vc, heads, **args)
+    before = r(rows, heads * 64), r(rows, heads * 64)
+    got = ops.ProjectedAttention(x, weights, k, v, heads, **args)
+    assert same(got[0], want[0]) and all(same(p, q) for p, q in zip(got[3], want[3]))
+    assert got[2].data.max().item() == want[2].data.max().item()
+    assert same(k, kc) and same(v, vc)
+    assert (got[1].numpy() == want[1].numpy()).all()
+    # with the layer norm in front, over a cache of which one half is a view
+    (a, add), ln = before, (1 + 0.1 * r(heads * 64), 0.1 * r(heads * 64))
+    want = ops.ProjectedAttentionOfLayerNorm(a, add, ln, weights, kc, vc, heads, kvLen=used, mask=mask)
+    got = ops.ProjectedAttentionOfLayerNorm(a, add, ln, weights, k, v.contiguous(), heads, kvLen=used, mask=mask)
+    assert same(got[0], want[0]) and same(got[1], want[1]) and same(k, kc)
 
 
 @pytest.mark.parametrize("sentences,heads,dk,cap,used", [
