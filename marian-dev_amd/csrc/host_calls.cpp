@@ -335,7 +335,8 @@ PyObject* py_affine_f32(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_END
 }
 
-// A list or tuple of (bQuant, bias or None) with K rows each; false when it is anything else.
+// A list or tuple of (bQuant, bias or None) with K rows each, biases of one value a column (exact_bias: and no more);
+// false when it is anything else.
 constexpr int kMaxMatrices = 4;
 struct Matrices {
   int n = 0;
@@ -343,7 +344,7 @@ struct Matrices {
   const int8_t* Bq[kMaxMatrices];
   const float* bias[kMaxMatrices];
 };
-bool matrices(PyObject* weights, int64_t K, bool bias_checked, Matrices& m) {
+bool matrices(PyObject* weights, int64_t K, bool exact_bias, Matrices& m) {
   if(!PyList_Check(weights) && !PyTuple_Check(weights)) return false;
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(weights);
   if(n < 1 || n > kMaxMatrices) return false;
@@ -353,7 +354,8 @@ bool matrices(PyObject* weights, int64_t K, bool bias_checked, Matrices& m) {
     if((!PyTuple_Check(w) && !PyList_Check(w)) || PySequence_Fast_GET_SIZE(w) != 2) return false;
     if(!matrix(PySequence_Fast_GET_ITEM(w, 0), m.b[g], true) || m.b[g].width != 1 || m.b[g].rows != K) return false;
     const at::Tensor* bias;
-    if(!f32c_or_none(PySequence_Fast_GET_ITEM(w, 1), &bias) || (bias_checked && bias && bias->numel() != m.b[g].cols)) return false;
+    if(!f32c_or_none(PySequence_Fast_GET_ITEM(w, 1), &bias) || (bias && (exact_bias ? bias->numel() != m.b[g].cols : bias->numel() < m.b[g].cols)))
+      return false;
     m.Bq[g] = static_cast<const int8_t*>(m.b[g].t->const_data_ptr());
     m.bias[g] = fptr(bias);
   }
@@ -602,6 +604,8 @@ PyObject* py_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   const int64_t dk = q->size(-1), m = q->size(-2), cap = k->size(-2), len = none(args[8]) ? cap : whole(args[8]);
   if(k->size(-1) != dk || len <= 0 || len > cap || m * dk == 0 || (mask && mask->numel() % len != 0)) Py_RETURN_NONE;
+  for(const at::Tensor* t : {kn, vn})   // (a row for every query row)
+    if(t && t->numel() < q->numel()) Py_RETURN_NONE;
   const int64_t per = whole(args[4]);
   const bool want = truth(args[5]);
   const c10::Device d = q->device();

@@ -104,6 +104,26 @@ def test_refused_arguments():
     assert call(Norm(**good), M=0) == L.OK
 
 
+def test_rows_and_biases_that_are_too_short():
+    """refused before anything is launched: the kernels take their lengths from the other operands"""
+    import torch
+    integer, ops = load("integer"), load("ops")
+    one = lambda *s: torch.ones(*s, device="cuda")
+    q, k, v = one(24, 1, 64), one(24, 10, 64), one(24, 10, 64)
+    for new in ((one(23, 64), one(24, 64)), (one(24, 64), one(1, 64)), (one(24, 32), one(24, 64))):
+        with pytest.raises(RuntimeError):
+            ops.Attention(q, k, v, kNew=new[0], vNew=new[1])
+    w = integer.prepareB(one(512, 512))
+    x, short, k, v = one(3, 512), [(w, one(504))], one(24, 10, 64), one(24, 10, 64)
+    for weights in (short, 3 * short, 2 * [(w, None)] + short):
+        with pytest.raises(RuntimeError):
+            ops.ProjectedAttention(x, weights, k, v, 8)
+        with pytest.raises(RuntimeError):
+            ops.ProjectedAttentionOfLayerNorm(x, x, (one(512), one(512)), weights, k, v, 8)
+    ops.ProjectedAttention(x, [(w, one(1, 512))], k, v, 8)
+    assert (k == 1).all() and (v == 1).all()
+
+
 @pytest.mark.parametrize("M,K,N", [
     (4096, 1024, [1024, 1024, 1024]), (2048, 1536, [2048, 1024, 3072, 256]),                   # tile pairs
     (3000, 512, [512, 512, 512]), (2050, 384, [1000, 8, 2056]), (4096, 1664, [1024, 1024]),     # a 128x128 tile per CU
