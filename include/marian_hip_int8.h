@@ -190,7 +190,9 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
  * multiplications of marian_hip_int8_affine_f32_grouped on x - the bits of the separate calls
  * (marian_hip_layer_norm, then the chained or grouped call).
  *   norm: HOST struct, read during the call; add [M x K], gamma [K], beta [K] and out [M x K], which receives x,
- *     16-byte aligned; out overlaps neither A nor add (MARIAN_HIP_ERR_ALIAS).
+ *     16-byte aligned; out overlaps none of A and the other three.
+ *   out[g] and absmax_out overlap neither A nor any of norm's tensors: every workgroup reads those, while others
+ *     already write (the separate calls may reuse the memory, this one returns MARIAN_HIP_ERR_ALIAS).
  *   M <= 8, K <= 1024, K % 64 == 0, otherwise MARIAN_HIP_ERR_SHAPE.
  *   absmax_out: as for marian_hip_int8_affine_f32_chained, with n_groups == 1; or NULL.
  */
@@ -234,6 +236,9 @@ int marian_hip_int8_affine_f32_normed(const float* A, const marian_hip_norm_inpu
  *     out: [M * heads, 64] = [M x N]; att_scale: the 1 / sqrt(64) of transformer.h:261.
  *   absmax_in / absmax_out / workspace: as for marian_hip_int8_affine_f32_chained (absmax_out
  *     needs M * heads <= 2048; the workspace is only used when absmax_in is NULL).
+ *   What a call writes (out, proj_out, absmax_out, Aq and, with n_proj = 3, the caches) overlaps neither what
+ *     its projections read (A, absmax_in; A, add, gamma, beta and out of the forms with a norm) nor the caches:
+ *     workgroups write while others still read (MARIAN_HIP_ERR_ALIAS; the separate calls may reuse such memory).
  * The result has the bits of the separate calls (marian_hip_int8_affine_f32_grouped, then
  * marian_hip_attention_cached).  When to use it (measured with d = 1024, 16 heads, 21 cached / 60
  * source positions, calls back to back): it is ahead of the two separate calls up to 128 rows

@@ -29,6 +29,24 @@ inline int current_device(int* dev) {
   return MARIAN_HIP_OK;
 }
 
+// A piece of device memory (p null: none).
+struct Span {
+  const void* p;
+  int64_t bytes;
+};
+
+// Every workgroup of a launch that joins several steps reads the inputs of the first one, and the workgroups
+// write the outputs of the last one as they finish: where the two share memory the launch races, though the
+// steps on their own, one after the other on a stream, do not.
+inline int apart(std::initializer_list<Span> written, std::initializer_list<Span> read) {
+  for(const Span& w : written)
+    for(const Span& r : read) {
+      const uintptr_t a = reinterpret_cast<uintptr_t>(w.p), b = reinterpret_cast<uintptr_t>(r.p);
+      if(w.p && r.p && a < b + (uintptr_t)r.bytes && b < a + (uintptr_t)w.bytes) return MARIAN_HIP_ERR_ALIAS;
+    }
+  return MARIAN_HIP_OK;
+}
+
 // What the kernels that normalize their input ask of it: few, short rows, whole vectors, an output that no
 // workgroup still reads.  (A: the M x K values the norm starts from.)
 inline int norm_input_check(const marian_hip_norm_input* n, const float* A, int64_t M, int64_t K) {
@@ -36,12 +54,8 @@ inline int norm_input_check(const marian_hip_norm_input* n, const float* A, int6
   if(!n->add || !n->gamma || !n->beta || !n->out) return MARIAN_HIP_ERR_NULL;
   for(const float* p : {n->add, n->gamma, n->beta, static_cast<const float*>(n->out)})
     if(reinterpret_cast<uintptr_t>(p) % 16 != 0) return MARIAN_HIP_ERR_ALIGN;
-  const uintptr_t out = reinterpret_cast<uintptr_t>(n->out), bytes = (uintptr_t)M * (uintptr_t)K * sizeof(float);
-  for(const float* p : {A, n->add}) {
-    const uintptr_t in = reinterpret_cast<uintptr_t>(p);
-    if(in < out + bytes && out < in + bytes) return MARIAN_HIP_ERR_ALIAS;
-  }
-  return MARIAN_HIP_OK;
+  const int64_t bytes = M * K * (int64_t)sizeof(float), row = K * (int64_t)sizeof(float);
+  return apart({{n->out, bytes}}, {{A, bytes}, {n->add, bytes}, {n->gamma, row}, {n->beta, row}});
 }
 
 // Compute units of the current device (looked up once per device; 256 if the query fails).

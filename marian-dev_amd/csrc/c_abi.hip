@@ -1143,7 +1143,12 @@ int marian_hip_int8_affine_f32_normed(const float* A, const marian_hip_norm_inpu
   if(blocks32 == 0) return MARIAN_HIP_ERR_SHAPE;   // (nobody would write the norm)
   if(!A) return MARIAN_HIP_ERR_NULL;
   if(!aligned(A, 16) || (absmax_out && !aligned(absmax_out, 4))) return MARIAN_HIP_ERR_ALIGN;
-  const int nst = norm_input_check(norm, A, M, K);
+  int nst = norm_input_check(norm, A, M, K);
+  for(int64_t g = 0; g < n_groups && nst == MARIAN_HIP_OK; ++g) {
+    const int64_t bytes = M * K * (int64_t)sizeof(float), row = K * (int64_t)sizeof(float);
+    nst = apart({{out[g], M * N[g] * (int64_t)sizeof(float)}, {absmax_out, kAbsmaxSlots * (int64_t)sizeof(float)}},
+                {{A, bytes}, {norm->add, bytes}, {norm->out, bytes}, {norm->gamma, row}, {norm->beta, row}});
+  }
   if(nst != MARIAN_HIP_OK) return nst;
   const NormInput n{norm->add, norm->gamma, norm->beta, norm->out, norm->eps};
   hipStream_t hst = reinterpret_cast<hipStream_t>(stream);

@@ -2467,6 +2467,16 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, con
     if(!aligned16(p.Bq[g]) || (p.bias[g] && !aligned16(p.bias[g])) || (p.proj_out[g] && !aligned16(p.proj_out[g])))
       return MARIAN_HIP_ERR_ALIGN;
   }
+  {
+    const int64_t f = sizeof(float), values = M * heads * 64 * f, cached = batchKV * kv_capacity * 64 * f, slots = kAbsmaxSlots * f;
+    const Span a{A, M * K * f}, add{norm ? norm->add : nullptr, M * K * f}, x{norm ? norm->out : nullptr, M * K * f};
+    const Span gamma{norm ? norm->gamma : nullptr, K * f}, beta{norm ? norm->beta : nullptr, K * f};
+    const Span known{norm ? nullptr : absmax_in, slots}, k{k_cache, cached}, v{v_cache, cached};
+    int ast = apart({{out, values}, {p.proj_out[0], values}, {p.proj_out[1], values}, {p.proj_out[2], values}, {absmax_out, slots},
+                     {norm ? nullptr : Aq, M * K + f}}, {a, add, x, gamma, beta, known, k, v});
+    if(ast == MARIAN_HIP_OK) ast = apart({k, v}, {a, add, x, gamma, beta, known});   // (appended to, or read beside x)
+    if(ast != MARIAN_HIP_OK) return ast;
+  }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   p.A = A; p.aq_out = Aq;
   p.norm = NormInput{nullptr, nullptr, nullptr, nullptr, 0.0f};

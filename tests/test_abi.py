@@ -147,6 +147,75 @@ def test_argument_validation_returns_codes_not_aborts():
         L.check(L.ERR_SHAPE, "test")
 
 
+class Norm(ctypes.Structure):
+    """marian_hip_norm_input"""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("add", "gamma", "beta", "out")] + [("eps", ctypes.c_float)]
+
+
+MB = 1 << 20
+M, HEADS, K = 6, 8, 512   # of the calls below
+ROWS, ROW, SLOTS = 4 * M * K, 4 * K, 4 * 2048   # bytes of their pieces of memory
+PLACES = {name: (i + 1) * MB for i, name in enumerate(
+    ("A", "add", "gamma", "beta", "x", "Bq", "out", "out1", "out2", "proj", "absmax_in", "absmax_out", "Aq", "k", "v"))}
+pointers = lambda *p: (ctypes.c_void_p * len(p))(*p)
+
+
+def normed(at):
+    lib = load("_lib").lib()
+    norm = Norm(at["add"], at["gamma"], at["beta"], at["x"], 1e-6)
+    return lib.marian_hip_int8_affine_f32_normed(at["A"], ctypes.byref(norm), 3, pointers(*3 * [at["Bq"]]), None,
+                                                 pointers(at["out"], at["out1"], at["out2"]), (ctypes.c_int64 * 3)(K, K, K), M, K,
+                                                 1.0, 0, None, None)
+
+
+def normed_absmax(at):
+    lib = load("_lib").lib()
+    norm = Norm(at["add"], at["gamma"], at["beta"], at["x"], 1e-6)
+    return lib.marian_hip_int8_affine_f32_normed(at["A"], ctypes.byref(norm), 1, pointers(at["Bq"]), None, pointers(at["out"]),
+                                                 (ctypes.c_int64 * 1)(K), M, K, 1.0, 0, at["absmax_out"], None)
+
+
+def projected(at, norm=False, ancestors=False, n=3):
+    lib = load("_lib").lib()
+    Bq, proj = pointers(*n * [at["Bq"]]), pointers(*[at["proj"] + g * ROWS for g in range(n)])
+    made = Norm(at["add"], at["gamma"], at["beta"], at["x"], 1e-6)
+    cache = (at["k"], at["v"])
+    if ancestors:
+        return lib.marian_hip_int8_proj_attention_ancestors(
+            at["A"], ctypes.byref(made) if norm else None, None if norm else at["Aq"], Bq, None, proj, M, K, HEADS, *cache, 4, 5, 64 * MB,
+            0.125, at["out"], None if norm else at["absmax_in"], at["absmax_out"], None, 0, None)
+    if norm:
+        return lib.marian_hip_int8_proj_attention_normed(at["A"], ctypes.byref(made), n, Bq, None, proj, M, K, HEADS, *cache, M * HEADS,
+                                                         4, 5, None, 0, 0.125, at["out"], at["absmax_out"], None)
+    return lib.marian_hip_int8_proj_attention(at["A"], at["Aq"], n, Bq, None, proj, M, K, HEADS, *cache, M * HEADS, 4, 5, None, 0, 0.125,
+                                              at["out"], at["absmax_in"], at["absmax_out"], None, 0, None)
+
+
+CACHE = 4 * M * HEADS * 5 * 64
+SIZES = {"A": ROWS, "add": ROWS, "gamma": ROW, "beta": ROW, "x": ROWS, "out": ROWS, "out1": ROWS, "out2": ROWS, "proj": ROWS,
+         "absmax_in": SLOTS, "absmax_out": SLOTS, "Aq": M * K + 4, "k": CACHE, "v": CACHE}
+norm_reads, caches = ["A", "add", "gamma", "beta"], ["k", "v"]
+
+
+@pytest.mark.parametrize("call,written,read", [
+    (normed, ["x"], norm_reads), (normed, ["out", "out1", "out2"], norm_reads + ["x"]), (normed_absmax, ["absmax_out"], norm_reads + ["x"]),
+    (projected, ["out", "proj", "absmax_out", "Aq"], ["A", "absmax_in"] + caches), (projected, caches, ["A", "absmax_in"]),
+    (lambda at: projected(at, n=1), ["out", "proj", "absmax_out", "Aq"], ["A", "absmax_in"] + caches),
+    (lambda at: projected(at, norm=True), ["x"], norm_reads),
+    (lambda at: projected(at, norm=True), ["out", "proj", "absmax_out"] + caches, norm_reads + ["x"]),
+    (lambda at: projected(at, norm=True, n=1), ["out", "proj", "absmax_out", "x"], norm_reads + caches),
+    (lambda at: projected(at, ancestors=True), ["out", "proj", "absmax_out", "Aq"] + caches, ["A", "absmax_in"]),
+    (lambda at: projected(at, norm=True, ancestors=True), ["out", "proj", "absmax_out"] + caches, norm_reads + ["x"])])
+def test_joined_calls_refuse_to_write_what_other_workgroups_read(call, written, read):
+    """(nothing is dereferenced: the overlap is found before any HIP call)"""
+    alias = load("_lib").ERR_ALIAS
+    for w in written:
+        for r in read:
+            # the same place; the last 16 bytes of what is read; the first 16 of it under the end of what is written
+            for to in (PLACES[r], PLACES[r] + SIZES[r] - 16, PLACES[r] - (SIZES[w] - 4) // 16 * 16):
+                assert call({**PLACES, w: to}) == alias, (w, r, to - PLACES[r])
+
+
 def test_position_signal_made_on_the_host_equals_the_checker():
     """marian_hip_sinusoidal_position_embeddings makes no HIP call: it runs here, and its rows are
     the checker's bit for bit (the same float expressions through the same C library)."""
