@@ -531,7 +531,7 @@ int launch_tile16(const Gemm16Args& g, hipStream_t st) {
 //   1 x 512 x 512 3.1 (stream 16 x 16), 64 x 512 x 2048 4.4 (16 x 32), 509 x 2048 x 512 10.4 (32 x 32), 509 x 512 x 2048
 //   8.7 (64 x 64), 4096 x 4096 x 4096 257 (128 x 128: 535 TOPS of 16-bit products).
 struct Form16 {
-  enum Name { kStream4, kStream8, kStream16, kStream16x32, kStream32x32, kTile64, kTile128 };
+  enum Name { kStream16, kStream16x32, kStream32x32, kTile64, kTile128 };
   Name form;
   double cost;   // bytes per k through the busiest CU
 };
