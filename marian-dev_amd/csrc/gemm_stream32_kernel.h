@@ -85,19 +85,9 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   constexpr bool NORM = MODE == kFusedNorm;
   static_assert(!GROUPED || MODE == kFusedTiled || NORM, "several weight matrices: quantize-on-stage and normalizing forms only");
   static_assert(!NORM || (Cfg::kWaves == kNormMaxRows && MT32 == 1 && ROWS == 16), "a wave to a row");
-  int bx = blockIdx.x, gx = args.blocks_x;   // column block within this workgroup's matrix, and how many it has
-  if constexpr(GROUPED) {
-    int g = 0;
-#pragma unroll
-    for(int i = 1; i < kMaxGroups; ++i)
-      if(i < groups.n && bx >= groups.block0[i]) g = i;
-    args.Bq = groups.Bq[g];
-    args.bias = groups.bias[g];
-    args.out = groups.out[g];
-    args.N = args.n_out = groups.N[g];
-    gx = groups.block0[g + 1] - groups.block0[g];
-    bx -= groups.block0[g];
-  }
+  int bx = blockIdx.x;   // column block within this workgroup's matrix
+  if constexpr(GROUPED) bx = groups.select(args, bx);
+  const int gx = args.blocks_x;   // and how many it has
   constexpr int kStream32Waves = Cfg::kWaves, kStream32Threads = Cfg::kThreads;
   constexpr bool TILED_ = MODE == kFusedTiled;
   constexpr int kFusedGroups = NG, kFullGroups = NG - 2;

@@ -130,7 +130,8 @@ struct GroupTable {
   int block0[kMaxGroups + 1];
   int n;
 
-  // Points the arguments to the matrix of column block `block`; returns the block's number within it.
+  // Points the arguments to the matrix of column block `block` and blocks_x to its number of blocks; returns the
+  // block's number within it.
   __device__ __forceinline__ int select(GemmArgs& a, int block) const {
     int g = 0;
 #pragma unroll
@@ -140,6 +141,7 @@ struct GroupTable {
     a.bias = bias[g];
     a.out = out[g];
     a.N = a.n_out = N[g];
+    a.blocks_x = block0[g + 1] - block0[g];
     return block - block0[g];
   }
 };
