@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <cmath>
 
 #include "../../include/marian_hip_int8.h"
 #include "abi_common.h"
@@ -523,37 +524,49 @@ int launch_tile16(const Gemm16Args& g, hipStream_t st) {
   return MARIAN_HIP_OK;
 }
 
-// Which form a call takes.  Per step of k a workgroup loads, converts and multiplies its rows of both operands,
-// about 30 ps a byte (measured, M = 1 .. 4096, whatever the form), so a form costs its workgroups per CU (at
-// least one) times the bytes a workgroup takes in for each k; the 128 x 128 tiles are half again as dear (one
-// workgroup to a CU: products, conversion and LDS traffic overlap less).  Over 25 sizes the form chosen
-// was never more than a tenth behind the best one.  us, int16 activations, in a graph:
-//   1 x 512 x 512 3.1 (stream 16 x 16), 64 x 512 x 2048 4.4 (16 x 32), 509 x 2048 x 512 10.4 (32 x 32), 509 x 512 x 2048
-//   8.7 (64 x 64), 4096 x 4096 x 4096 257 (128 x 128: 535 TOPS of 16-bit products).
+// Which form a call takes: the one whose busiest CU takes in the fewest bytes per step of k - its workgroups per CU
+// (at least one) times the bytes a workgroup loads, converts and multiplies for each k; the 128 x 128 tiles count half
+// again (one workgroup to a CU: products, conversion and LDS traffic overlap less).  Measured at 99 sizes (K, N = 256 ..
+// 4096, M = 1 .. 4096, launches in a graph), the form taken was never more than 6 % behind the best with int16
+// activations, 10 % with float32 ones (profiles/int16_forms.txt: every form, both kinds).  us, int16 activations:
+//   1 x 512 x 512 3.0 (stream 16 x 16), 64 x 512 x 2048 4.2 (16 x 32), 509 x 2048 x 512 10.4 (32 x 32), 509 x 512 x 2048
+//   8.6 (64 x 64), 4096 x 4096 x 4096 263 (128 x 128: 523 TOPS of 16-bit products).
+// What a call takes is another matter: each form has a start of its own and its own price of a byte (least squares over
+// the same measurements where the form is near the best: -29 .. +19 %); a CU holds one 128 x 128 tile at a time.
 struct Form16 {
   enum Name { kStream16, kStream16x32, kStream32x32, kTile64, kTile128 };
   Name form;
   double cost;   // bytes per k through the busiest CU
+  double ns;     // of the call
 };
-inline Form16 plan16(int M, int N, int a_bytes) {
-  struct Shape { Form16::Name form; int rows, cols; double factor; };
-  constexpr Shape shapes[] = {{Form16::kStream16, 16, 16, 1.0}, {Form16::kStream16x32, 16, 32, 1.0}, {Form16::kStream32x32, 32, 32, 1.0}, {Form16::kTile64, 64, 64, 1.0},
-                              {Form16::kTile128, 128, 128, 1.5}};
-  Form16 best{Form16::kTile128, 1e30};
+inline Form16 plan16(int M, int K, int N, int a_bytes) {
+  struct Shape { Form16::Name form; int rows, cols; double factor, start_ns, a_byte_ns, b_byte_ns; };
+  constexpr Shape shapes[] = {{Form16::kStream16, 16, 16, 1.0, 2600.0, 0.025, 0.033}, {Form16::kStream16x32, 16, 32, 1.0, 2900.0, 0.028, 0.030},
+                              {Form16::kStream32x32, 32, 32, 1.0, 3400.0, 0.033, 0.022}, {Form16::kTile64, 64, 64, 1.0, 5400.0, 0.019, 0.032},
+                              {Form16::kTile128, 128, 128, 1.5, 10000.0, 0.0155, 0.035}};
+  Form16 best{Form16::kTile128, 1e30, 0.0};
   for(const Shape& s : shapes) {
     if(s.form < Form16::kTile64 && (M + s.rows - 1) / s.rows > 65535) continue;   // (row tiles are the grid's second dimension)
     const double workgroups = (double)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols) / 256.0;
-    const double cost = (workgroups > 1.0 ? workgroups : 1.0) * s.factor * (s.rows * a_bytes + s.cols * 2);
-    if(cost < best.cost) best = Form16{s.form, cost};
+    const double per_cu = workgroups > 1.0 ? workgroups : 1.0;
+    const double cost = per_cu * s.factor * (s.rows * a_bytes + s.cols * 2);
+    if(cost >= best.cost) continue;
+    const int rows = M < s.rows ? M : s.rows;   // (rows past the end repeat the last one, which is in the cache)
+    const double tile = K * (s.a_byte_ns * rows * a_bytes + s.b_byte_ns * s.cols * 2);
+    best = Form16{s.form, cost, s.form == Form16::kTile128 ? std::ceil(per_cu) * (s.start_ns + tile) : s.start_ns + per_cu * tile};
   }
   return best;
 }
 
-// Whether float32 activations are quantized by a launch of their own first: where the bytes that the multiplication
-// then saves take longer than the launch and its pass over memory (3 us and 6 bytes a value at 4 TB/s).
+// Whether float32 activations are quantized by a launch of their own first: where the multiplication then saves more
+// than the launch costs: 2 us, and 2.5 ns per thousand values up to 1.2 million and half of one beyond (the pass over
+// them, and the multiplication's wait for values that were just written).  At the 99 sizes the choice is at most 3 %
+// behind the better one but for 256 rows of 512 and of 704 values, which two 32 x 32 workgroups a CU quantize on the way (10
+// and 18 %); with one price for all forms (30 ps a byte) it was 4 .. 18 % behind at nine.
 inline bool quantize_first16(int64_t M, int64_t K, int64_t N) {
-  const double saved = (plan16((int)M, (int)N, 4).cost - plan16((int)M, (int)N, 2).cost) * (double)K * 0.03;   // ns
-  return saved > 3000.0 + (double)M * (double)K * 0.0015;
+  const double saved = plan16((int)M, (int)K, (int)N, 4).ns - plan16((int)M, (int)K, (int)N, 2).ns;
+  const double values = (double)M * (double)K, near = values < 1.2e6 ? values : 1.2e6;
+  return saved > 2000.0 + 0.002 * near + 0.00055 * values;
 }
 
 template <typename AT, bool DUMP>
@@ -564,7 +577,7 @@ int run16(const AT* A, const int16_t* Bq, const float* bias, void* out, int64_t 
   if(M == 0 || N == 0) return MARIAN_HIP_OK;
   Gemm16Args g{A, Bq, bias, out, (int)M, (int)K, (int)N, scale, relu ? 1 : 0};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  switch(plan16((int)M, (int)N, (int)sizeof(AT)).form) {
+  switch(plan16((int)M, (int)K, (int)N, (int)sizeof(AT)).form) {
     case Form16::kStream16: return launch_stream16<AT, 1, 1, DUMP>(g, st);
     case Form16::kStream16x32: return launch_stream16<AT, 1, 2, DUMP>(g, st);
     case Form16::kStream32x32: return launch_stream16<AT, 2, 2, DUMP>(g, st);
