@@ -113,7 +113,7 @@ class MarianHipError(RuntimeError):
 
 def build(verbose=False):
     """Compile the HIP libraries for gfx950 with hipcc and the host path with the C++ compiler (always recompiles)."""
-    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), "-B", "-j4"]
+    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), "-B", "-j4", "python"]
     out = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if verbose or out.returncode != 0:
         print(out.stdout)
@@ -126,7 +126,7 @@ def _must_exist(path):
     if not os.path.exists(path):
         raise MarianHipError(
             -1, "{} is not built ({}); run __graft_entry__.build() or "
-            "`make -C marian-dev_amd/csrc`. There is no CPU fallback.".format(os.path.basename(path), path))
+            "`make -C marian-dev_amd/csrc python`. There is no CPU fallback.".format(os.path.basename(path), path))
 
 
 def _load(path, signatures):
@@ -173,10 +173,14 @@ class HostCalls:
             raise AttributeError(name)
         if _host is None:
             _must_exist(HOST_PATH)
-            import torch  # noqa: F401  (its libraries have to be in the process first)
+            import torch   # (its libraries have to be in the process first)
             spec = importlib.util.spec_from_file_location("_host_calls", HOST_PATH)
-            made = importlib.util.module_from_spec(spec)
-            spec.loader.exec_module(made)
+            try:
+                made = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(made)
+            except ImportError as e:   # (built for another torch: refused by the module, or by the linker)
+                raise MarianHipError(-1, "{} does not fit this torch ({}): {}; run `make -C marian-dev_amd/csrc -B python`".format(
+                    os.path.basename(HOST_PATH), torch.__version__, e)) from e
             made.use(lib()._handle)
             made.setup(*self._types())
             _host = made

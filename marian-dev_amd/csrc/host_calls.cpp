@@ -1026,7 +1026,23 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", "host path of the op
 
 }  // namespace
 
+// This module calls functions of torch's that have no stable binary interface: it works in the torch it was built
+// against and no other.  (Python's own interface only, until that is known.)
+static bool built_for_this_torch() {
+  Ref torch(PyImport_ImportModule("torch"));
+  if(!torch) return false;
+  Ref version(PyObject_GetAttrString(torch.p, "__version__"));
+  if(!version) return false;
+  Ref text(PyObject_Str(version.p));
+  if(!text) return false;
+  if(PyUnicode_CompareWithASCIIString(text.p, MARIAN_BUILT_FOR_TORCH) == 0) return true;
+  PyErr_Format(PyExc_ImportError, "_host_calls.so was built for torch %s and this is torch %U; run make -C marian-dev_amd/csrc -B python",
+               MARIAN_BUILT_FOR_TORCH, text.p);
+  return false;
+}
+
 extern "C" __attribute__((visibility("default"))) PyObject* PyInit__host_calls() {
+  if(!built_for_this_torch()) return nullptr;
   s_data = PyUnicode_InternFromString("data");
   s_shape = PyUnicode_InternFromString("shape");
   s_type = PyUnicode_InternFromString("type");
