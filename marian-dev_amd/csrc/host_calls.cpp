@@ -873,7 +873,8 @@ PyObject* py_ancestors_advance(PyObject*, PyObject* const* args, Py_ssize_t narg
   const at::Tensor *prev = tensor(args[0]), *par = tensor(args[1]), *out = tensor(args[3]);
   if(!prev || !par || !out || prev->scalar_type() != at::kInt || out->scalar_type() != at::kInt || prev->dim() != 2 ||
      prev->sizes() != out->sizes() || !prev->is_cuda() || !prev->is_contiguous() || !out->is_contiguous() ||
-     !ids_type(par->scalar_type()) || !par->is_contiguous() || par->numel() != prev->size(0))
+     !ids_type(par->scalar_type()) || !par->is_contiguous() || par->numel() != prev->size(0) ||
+     par->device() != prev->device() || out->device() != prev->device())
     Py_RETURN_NONE;
   const int64_t len = whole(args[2]);
   const hipStream_t st = stream_of(prev->device());

@@ -124,6 +124,16 @@ def test_rows_and_biases_that_are_too_short():
     assert (k == 1).all() and (v == 1).all()
 
 
+def test_back_pointers_and_tables_on_another_device():
+    import torch
+    ops = load("ops")
+    table, parents = torch.zeros(4, 8, dtype=torch.int32, device="cuda"), torch.zeros(4, dtype=torch.int32, device="cuda")
+    for par, out in ((parents.cpu(), table.clone()), (parents.long().cpu(), table.clone()), (parents, table.cpu())):
+        with pytest.raises(RuntimeError):
+            ops.advanceAncestors(table, par, 3, out)
+    assert ops.advanceAncestors(table, parents.long(), 3, table.clone())[:, 3].tolist() == [0, 1, 2, 3]
+
+
 @pytest.mark.parametrize("M,K,N", [
     (4096, 1024, [1024, 1024, 1024]), (2048, 1536, [2048, 1024, 3072, 256]),                   # tile pairs
     (3000, 512, [512, 512, 512]), (2050, 384, [1000, 8, 2056]), (4096, 1664, [1024, 1024]),     # a 128x128 tile per CU
