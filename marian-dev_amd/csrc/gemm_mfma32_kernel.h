@@ -185,14 +185,6 @@ __device__ __forceinline__ void xcd_tile(int tiles_n, int tiles_m, int block, in
   tm = r / bw;
 }
 
-// A workgroup barrier for what was written to LDS, and only that: __syncthreads() also orders global memory, and the
-// compiler then leaves a wait on vector memory (one that waits for nothing) among the stores of the write-out.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // Abs-max hand-over of a large-M launch: slot `slot` receives the maximum of |y| over the tile this
 // workgroup stored (omax: this lane's share), the workgroup of slot 0 zeroes the slots past the
 // `used` ones the launch fills.  red: the LDS ring, free once every wave is past its last fragment

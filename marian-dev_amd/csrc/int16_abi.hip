@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 
 #include "../../include/marian_hip_int8.h"
 #include "abi_common.h"
@@ -111,6 +112,19 @@ __device__ __forceinline__ void split_words(unsigned d0, unsigned d1, int& h, in
   l = (int)(__builtin_amdgcn_perm(d1, d0, 0x06040200u) ^ 0x80808080u);
 }
 
+__device__ __forceinline__ Planes planes_of_words(const unsigned (&d)[8]) {   // 16 int16
+  Planes r;
+  r.sum = 0;
+  int h[4], l[4];
+#pragma unroll
+  for(int i = 0; i < 4; ++i) split_words(d[2 * i], d[2 * i + 1], h[i], l[i]);
+#pragma unroll
+  for(int i = 0; i < 8; ++i) r.sum = __builtin_amdgcn_sdot2(__builtin_bit_cast(v2s, d[i]), v2s{1, 1}, r.sum, false);
+  r.h = v4i{h[0], h[1], h[2], h[3]};
+  r.l = v4i{l[0], l[1], l[2], l[3]};
+  return r;
+}
+
 // The 16 values of a block of 64 k that lane group lk (0 .. 3) supplies: k = 8 lk .. 8 lk + 7 and 32 + 8 lk ..
 // 32 + 8 lk + 7 (the same for both operands, so any order does), which makes the four lanes of a row read
 // 64 contiguous bytes.  Loaded first, taken apart later, so that loads are in flight in between.  Where K ends
@@ -127,22 +141,15 @@ struct Raw<int16_t> {
   }
   __device__ __forceinline__ void clear_second() { w[1] = v4u{0, 0, 0, 0}; }
   __device__ __forceinline__ Planes planes() const {
-    Planes r;
-    r.sum = 0;
     const unsigned d[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
-    int h[4], l[4];
-#pragma unroll
-    for(int i = 0; i < 4; ++i) split_words(d[2 * i], d[2 * i + 1], h[i], l[i]);
-#pragma unroll
-    for(int i = 0; i < 8; ++i) r.sum = __builtin_amdgcn_sdot2(__builtin_bit_cast(v2s, d[i]), v2s{1, 1}, r.sum, false);
-    r.h = v4i{h[0], h[1], h[2], h[3]};
-    r.l = v4i{l[0], l[1], l[2], l[3]};
-    return r;
+    return planes_of_words(d);
   }
 };
-// float32 activations, quantized on the way.  x * 1024 is exact, so one fused multiply-add with 1.5 * 2^23
-// rounds to nearest-even and leaves the integer in the low bytes of the sum, once x is clamped to int16's
-// range (med3: NaN to the lower end); products of 2^31 and more give -32768 (quantize16_one).
+// float32 activations, quantized on the way.  A sum with 12288 = 1.5 * 2^13 has steps of 1/1024, so the addition rounds x * 1024
+// to nearest-even and leaves the int16 in the low half of the sum, which it writes to where it belongs, as long as it
+// is in range.  A maximum that lets NaN through tells whether all 16 values are; the few that are not are replaced by the
+// value they saturate to (quantize16_one: NaN and products of 2^31 and more give -32768).  2.8 vector instructions a value, where a
+// clamp of every value and sums of the unpacked integers took 5.
 template <>
 struct Raw<float> {
   v4f w[4];
@@ -154,37 +161,26 @@ struct Raw<float> {
   }
   __device__ __forceinline__ void clear_second() { w[2] = w[3] = v4f{0.0f, 0.0f, 0.0f, 0.0f}; }
   __device__ __forceinline__ Planes planes() const {
-    constexpr unsigned kMagicBits = 0x4B400000u;
     float x[16];
 #pragma unroll
     for(int i = 0; i < 4; ++i) { x[4 * i] = w[i].x; x[4 * i + 1] = w[i].y; x[4 * i + 2] = w[i].z; x[4 * i + 3] = w[i].w; }
-    float top = x[0];
+    float top = 0.0f;
 #pragma unroll
-    for(int i = 1; i < 16; ++i) top = fmaxf(top, x[i]);
-    if(top >= 2097152.0f) {   // (rare: x * 1024 >= 2^31)
+    for(int i = 0; i < 16; i += 2)
+      top = __builtin_elementwise_maximum(__builtin_elementwise_maximum(top, __builtin_fabsf(x[i])), __builtin_fabsf(x[i + 1]));
+    if(!(top <= 31.99f)) {   // (rare)
 #pragma unroll
-      for(int i = 0; i < 16; ++i) x[i] = x[i] >= 2097152.0f ? -32.0f : x[i];
+      for(int i = 0; i < 16; ++i)
+        x[i] = x[i] >= 2097152.0f ? -32.0f : __builtin_amdgcn_fmed3f(x[i], -32.0f, 32767.0f / 1024.0f);
     }
-    unsigned b[16], sum = 0;
+    unsigned d[8];
 #pragma unroll
-    for(int i = 0; i < 16; ++i) {
-      const float c = __builtin_amdgcn_fmed3f(x[i], -32.0f, 32767.0f / 1024.0f);
-      b[i] = __float_as_uint(fmaf(c, kQuantMult16, 12582912.0f));
-      sum += b[i];
+    for(int i = 0; i < 8; ++i) {
+      const float magic = 12288.0f;
+      asm("v_add_f32_sdwa %0, %1, %2 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:DWORD" : "=v"(d[i]) : "v"(x[2 * i]), "v"(magic));
+      asm("v_add_f32_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD" : "+v"(d[i]) : "v"(x[2 * i + 1]), "v"(magic));
     }
-    Planes r;
-    r.sum = (int)(sum - 16u * kMagicBits);
-    int h[4], l[4];
-#pragma unroll
-    for(int i = 0; i < 4; ++i) {
-      const unsigned p = __builtin_amdgcn_perm(b[4 * i + 1], b[4 * i], 0x05010400u);       // h1 h0 l1 l0
-      const unsigned q = __builtin_amdgcn_perm(b[4 * i + 3], b[4 * i + 2], 0x05010400u);   // h3 h2 l3 l2
-      h[i] = (int)__builtin_amdgcn_perm(q, p, 0x07060302u);
-      l[i] = (int)(__builtin_amdgcn_perm(q, p, 0x05040100u) ^ 0x80808080u);
-    }
-    r.h = v4i{h[0], h[1], h[2], h[3]};
-    r.l = v4i{l[0], l[1], l[2], l[3]};
-    return r;
+    return planes_of_words(d);
   }
 };
 // the three accumulators of one 16 x 16 tile (rows: columns of the output, see mfma_i8_16x16x64)
@@ -215,12 +211,9 @@ struct Gemm16Args {
   int relu;
 };
 
-// four neighbouring columns n .. n + 3 of output row m: y = float(acc) * unquant (+ bias); relu: y > 0 ? y : 0;
-// multiply and add round separately
+// four neighbouring outputs: y = float(acc) * unquant (+ bias); relu: y > 0 ? y : 0; multiply and add round separately
 template <bool DUMP>
-__device__ __forceinline__ void store16(const Gemm16Args& g, v4i acc, int m, int n, float unquant) {
-  if(m >= g.M || n >= g.N) return;   // (N % 8 == 0: four columns are inside or outside together)
-  const size_t off = (size_t)m * g.N + n;
+__device__ __forceinline__ void store16(const Gemm16Args& g, v4i acc, size_t off, float unquant, const float (&bias)[4]) {
   if(DUMP) {
     *reinterpret_cast<v4i*>(reinterpret_cast<int32_t*>(g.out) + off) = acc;
     return;
@@ -229,7 +222,7 @@ __device__ __forceinline__ void store16(const Gemm16Args& g, v4i acc, int m, int
 #pragma unroll
   for(int e = 0; e < 4; ++e) {
     float v = (float)acc[e] * unquant;
-    if(g.bias) v = v + g.bias[n + e];
+    if(g.bias) v = v + bias[e];
     if(g.relu) v = v > 0.0f ? v : 0.0f;
     y[e] = v;
   }
@@ -243,25 +236,61 @@ __device__ __forceinline__ float unquant16(const Gemm16Args& g) {
   return unquant_mult(aqm, *reinterpret_cast<const float*>(g.Bq + (size_t)g.K * g.N), g.scale);
 }
 
-// Few tiles: the eight waves of a workgroup split K between them, operands go from memory straight into
-// registers (a lane takes 16 consecutive k of its row, four lanes a 128-byte line) and the partial sums meet
-// in LDS.  A workgroup makes (16 MT) x (16 NT) outputs.  Bound by what a CU can fetch: the activations of
-// 16 MT rows are read again for every 16 NT columns.
+// The tile of workgroup `block` of tiles_n x tiles_m: workgroups are dealt out to the eight XCDs in turn, and those of one XCD
+// take neighbouring tiles - bands of eight columns - so that its L2 holds what they share.
+__device__ __forceinline__ void xcd_order16(int tiles_n, int tiles_m, int block, int& tn, int& tm) {
+  const int total = tiles_n * tiles_m, x = block % 8, rest = total % 8;
+  const int t = x * (total / 8) + min(x, rest) + block / 8;
+  const int band = 8, b = t / (band * tiles_m), r = t % (band * tiles_m), width = min(tiles_n - b * band, band);
+  tn = b * band + r % width;
+  tm = r / width;
+}
+
+// Sum over the four lanes of a quad, left in all of them (two DPP lane swaps).
+__device__ __forceinline__ int quad_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
+  return v;
+}
+
+// Few tiles: the eight waves of a workgroup split K between them and the partial sums meet in LDS.  A workgroup
+// makes (16 MT) x (16 NT) outputs.  Operands do not need LDS to be shared, but a matrix instruction wants neighbouring
+// lanes to hold neighbouring rows, and a load of which the four lanes of a quad ask for four lines takes the address unit four
+// times as long: that was the bound (16 bytes a clock and CU).  So a quad loads one row's line, takes its values apart,
+// and the bytes change lanes through the wave's own LDS; two steps of K are on their way.  509 x 2048 x 512 from float32: 14.6 -> 8.8 us,
+// of it 0.4 the order of the tiles over the XCDs; what is left is 384 KB per CU at 64 bytes a clock (2.9 us), beside conversions
+// of about as long, and 3.5 us of launch, first loads and write-out.
 constexpr int kStream16Waves = 8;
-template <typename AT, int MT, int NT, bool DUMP>
-__global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(Gemm16Args g) {
-  constexpr int KW = kStream16Waves, TILES = MT * NT;
-  __shared__ __attribute__((aligned(16))) int part[KW][TILES][64][4];
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, lr = lane % 16, lk = lane / 16;
-  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+template <int MT, int NT>
+constexpr int stream16_lds() { return kStream16Waves * 1024 * (2 * (MT + NT) > MT * NT ? 2 * (MT + NT) : MT * NT); }
+template <typename AT, int MT, int NT, int D, bool DUMP>
+__global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(Gemm16Args g, int tiles_n, int tiles_m) {
+  constexpr int KW = kStream16Waves, TILES = MT * NT, kWaveBytes = stream16_lds<MT, NT>() / KW;
+  extern __shared__ __attribute__((aligned(16))) int8_t lds16[];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int lr = lane % 16, lk = lane / 16;   // the operand row and run of k that a matrix instruction takes from this lane
+  const int qr = lane / 4, qk = lane % 4;     // and those that it loads and takes apart
+  int tn, tm;
+  xcd_order16(tiles_n, tiles_m, blockIdx.x, tn, tm);
+  const int n0 = tn * 16 * NT, m0 = tm * 16 * MT;
+  // what the write-out needs, requested first: the biases of this thread's four columns (without a bias the weights stand in)
+  static_assert(TILES * 64 <= 64 * KW, "a thread finishes four outputs");
+  const int wr_n = n0 + 16 * (threadIdx.x / 64 % NT) + 4 * lk, wr_m = m0 + 16 * (threadIdx.x / 64 / NT) + lr;
+  float bias[4];
+  const float* bias_src = g.bias ? g.bias : reinterpret_cast<const float*>(g.Bq);
+#pragma unroll
+  for(int e = 0; e < 4; ++e) bias[e] = bias_src[min(wr_n, g.N - 4) + e];
+  float unquant = 0.0f;
+  if(!DUMP) unquant = unquant16<AT>(g);
+  int8_t* const mine = lds16 + wave * kWaveBytes;
   const AT* arow[MT];
   const int16_t* brow[NT];
 #pragma unroll
-  for(int i = 0; i < MT; ++i) arow[i] = reinterpret_cast<const AT*>(g.A) + (size_t)min(m0 + 16 * i + lr, g.M - 1) * g.K;
+  for(int i = 0; i < MT; ++i) arow[i] = reinterpret_cast<const AT*>(g.A) + (size_t)min(m0 + 16 * i + qr, g.M - 1) * g.K + qk * 8;
 #pragma unroll
-  for(int j = 0; j < NT; ++j) brow[j] = g.Bq + (size_t)min(n0 + 16 * j + lr, g.N - 1) * g.K;
+  for(int j = 0; j < NT; ++j) brow[j] = g.Bq + (size_t)min(n0 + 16 * j + qr, g.N - 1) * g.K + qk * 8;
   Acc16 acc[MT][NT];
-  int asum[MT], bsum[NT], taken = 0;
+  int asum[MT], bsum[NT];
 #pragma unroll
   for(int i = 0; i < MT; ++i) {
     asum[i] = 0;
@@ -272,114 +301,148 @@ __global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(Gemm
   for(int j = 0; j < NT; ++j) bsum[j] = 0;
   const int S = (g.K + 63) / 64;
   const bool half = g.K % 64 != 0;
-  Raw<AT> ra[MT];
-  Raw<int16_t> rb[NT];
-  auto load = [&](int s) __attribute__((always_inline)) {
-    const int k = s * 64 + lk * 8, second = half && s == S - 1 ? 0 : 32;
-#pragma unroll
-    for(int j = 0; j < NT; ++j) rb[j].load(brow[j] + k, second);
+  const int steps = wave < S ? (S - wave + KW - 1) / KW : 0;   // of this wave: wave, wave + KW, ..
+  Raw<AT> ra[D][MT];
+  Raw<int16_t> rb[D][NT];
+  auto load = [&](int t, Raw<AT> (&ra)[MT], Raw<int16_t> (&rb)[NT]) __attribute__((always_inline)) {
+    const int s = wave + t * KW, k = s * 64, second = half && s == S - 1 ? 0 : 32;
 #pragma unroll
     for(int i = 0; i < MT; ++i) ra[i].load(arow[i] + k, second);
+#pragma unroll
+    for(int j = 0; j < NT; ++j) rb[j].load(brow[j] + k, second);
   };
-  // one step: its operands are taken apart, the next step's loads take their place, then the products
-  auto step = [&](int s, bool more) __attribute__((always_inline)) {
-    Planes a[MT], b[NT];
-    if(!more && half && s == S - 1) {
+  // operands of a step change lanes through the wave's own LDS (a wave's LDS operations keep their order)
+  const int put = (qk * 16 + (qr ^ (2 * qk))) * 16, get = (lk * 16 + (lr ^ (2 * lk))) * 16;
+  auto step = [&](int t, int next, Raw<AT> (&ra)[MT], Raw<int16_t> (&rb)[NT]) __attribute__((always_inline)) {
+    if(half && wave + t * KW == S - 1) {
 #pragma unroll
       for(int i = 0; i < MT; ++i) ra[i].clear_second();
     }
 #pragma unroll
-    for(int j = 0; j < NT; ++j) b[j] = rb[j].planes();
-#pragma unroll
-    for(int i = 0; i < MT; ++i) a[i] = ra[i].planes();
-    if(more) load(s + KW);
-#pragma unroll
     for(int i = 0; i < MT; ++i) {
-      asum[i] += a[i].sum;
-#pragma unroll
-      for(int j = 0; j < NT; ++j) acc[i][j].add(b[j].h, b[j].l, a[i].h, a[i].l);
+      const Planes p = ra[i].planes();
+      asum[i] += p.sum;
+      *reinterpret_cast<v4i*>(mine + (2 * i) * 1024 + put) = p.h;
+      *reinterpret_cast<v4i*>(mine + (2 * i + 1) * 1024 + put) = p.l;
     }
 #pragma unroll
-    for(int j = 0; j < NT; ++j) bsum[j] += b[j].sum;
-    taken += 64;
-  };
-  int s = wave;
-  if(s < S) {
-    load(s);
-    // (the load of the next step stands behind no branch: the compiler would wait for it at once)
-    for(; s + KW < S; s += KW) step(s, true);
-    step(s, false);
-  }
-  // row sums over the four lane groups; lane (lr, lk) holds outputs row lr, columns 4 lk .. 4 lk + 3
+    for(int j = 0; j < NT; ++j) {
+      const Planes p = rb[j].planes();
+      bsum[j] += p.sum;
+      *reinterpret_cast<v4i*>(mine + (2 * MT + 2 * j) * 1024 + put) = p.h;
+      *reinterpret_cast<v4i*>(mine + (2 * MT + 2 * j + 1) * 1024 + put) = p.l;
+    }
+    if(next >= 0) load(next, ra, rb);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    v4i bh[NT], bl[NT];
 #pragma unroll
-  for(int i = 0; i < MT; ++i) {
-    asum[i] += __shfl_xor(asum[i], 16);
-    asum[i] += __shfl_xor(asum[i], 32);
+    for(int j = 0; j < NT; ++j) {
+      bh[j] = *reinterpret_cast<const v4i*>(mine + (2 * MT + 2 * j) * 1024 + get);
+      bl[j] = *reinterpret_cast<const v4i*>(mine + (2 * MT + 2 * j + 1) * 1024 + get);
+    }
+#pragma unroll
+    for(int i = 0; i < MT; ++i) {
+      const v4i ah = *reinterpret_cast<const v4i*>(mine + (2 * i) * 1024 + get);
+      const v4i al = *reinterpret_cast<const v4i*>(mine + (2 * i + 1) * 1024 + get);
+#pragma unroll
+      for(int j = 0; j < NT; ++j) acc[i][j].add(bh[j], bl[j], ah, al);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  // (the loads of later steps stand behind no branch of their own: the compiler would wait for them at once)
+  if(D == 1 || steps < 2) {
+    if(steps > 0) {
+      load(0, ra[0], rb[0]);
+      int t = 0;
+      for(; t + 1 < steps; ++t) step(t, t + 1, ra[0], rb[0]);
+      step(t, -1, ra[0], rb[0]);
+    }
+  } else {
+    load(0, ra[0], rb[0]);
+    load(1, ra[D - 1], rb[D - 1]);
+    int t = 0;
+    for(; t + 3 < steps; t += 2) {
+      step(t, t + 2, ra[0], rb[0]);
+      step(t + 1, t + 3, ra[D - 1], rb[D - 1]);
+    }
+    if(t + 2 < steps) {
+      step(t, t + 2, ra[0], rb[0]);
+      step(t + 1, -1, ra[D - 1], rb[D - 1]);
+      step(t + 2, -1, ra[0], rb[0]);
+    } else {
+      step(t, -1, ra[0], rb[0]);
+      step(t + 1, -1, ra[D - 1], rb[D - 1]);
+    }
   }
+  // row sums over the quads; lane (lr, lk) holds outputs row lr, columns 4 lk .. 4 lk + 3
+#pragma unroll
+  for(int i = 0; i < MT; ++i) asum[i] = __shfl(quad_sum(asum[i]), 4 * lr);
 #pragma unroll
   for(int j = 0; j < NT; ++j) {
-    bsum[j] += __shfl_xor(bsum[j], 16);
-    bsum[j] += __shfl_xor(bsum[j], 32);
+    bsum[j] = quad_sum(bsum[j]);
     int bs[4];
 #pragma unroll
-    for(int e = 0; e < 4; ++e) bs[e] = __shfl(bsum[j], 4 * lk + e);
+    for(int e = 0; e < 4; ++e) bs[e] = __shfl(bsum[j], 16 * lk + 4 * e);
 #pragma unroll
     for(int i = 0; i < MT; ++i) {
       v4i t = acc[i][j].sum();
 #pragma unroll
-      for(int e = 0; e < 4; ++e) t[e] = (int)((unsigned)t[e] + 128u * (unsigned)(asum[i] + bs[e]) - 16384u * (unsigned)taken);
-      *reinterpret_cast<v4i*>(part[wave][i * NT + j][lane]) = t;
+      for(int e = 0; e < 4; ++e)
+        t[e] = (int)((unsigned)t[e] + 128u * (unsigned)(asum[i] + bs[e]) - 16384u * 64u * (unsigned)steps);
+      *reinterpret_cast<v4i*>(mine + (i * NT + j) * 1024 + lane * 16) = t;
     }
   }
-  float unquant = 0.0f;
-  if(!DUMP) unquant = unquant16<AT>(g);
   __syncthreads();
-  for(int t = threadIdx.x; t < TILES * 64; t += 64 * KW) {
-    const int tile = t / 64, l = t % 64;
-    v4i sum = *reinterpret_cast<const v4i*>(part[0][tile][l]);
+  if(wave < TILES && wr_m < g.M && wr_n < g.N) {   // (N % 8 == 0: four columns are inside or outside together)
+    v4i sum = v4i{0, 0, 0, 0};
 #pragma unroll
-    for(int w = 1; w < KW; ++w) {
-      const v4i p = *reinterpret_cast<const v4i*>(part[w][tile][l]);
+    for(int w = 0; w < KW; ++w) {
+      const v4i p = *reinterpret_cast<const v4i*>(lds16 + w * kWaveBytes + wave * 1024 + lane * 16);
 #pragma unroll
       for(int e = 0; e < 4; ++e) sum[e] = (int)((unsigned)sum[e] + (unsigned)p[e]);
     }
-    store16<DUMP>(g, sum, m0 + 16 * (tile / NT) + l % 16, n0 + 16 * (tile % NT) + 4 * (l / 16), unquant);
+    store16<DUMP>(g, sum, (size_t)wr_m * g.N + wr_n, unquant, bias);
   }
 }
 
-// Many tiles: a workgroup of eight waves makes a BM x BN tile, both operands of a block of 64 k go through
-// registers (taken apart there, once per workgroup) into LDS, two blocks in turn: while one is multiplied the
-// next is on its way.  LDS rows are 64 bytes,
-// their four pieces permuted by the row number so that reads of neighbouring rows fall on different banks.
-constexpr int kPitch16 = 64, kTile16Depth = 2;
+// Many tiles: a workgroup of eight waves makes a BM x BN tile; both operands of a block of 64 k go through registers
+// (taken apart there, once per workgroup) into LDS, two stages in turn: while one is multiplied the next is filled.
+// Waves 0 .. 3 stage A, waves 4 .. 7 B - a wave of each kind on every SIMD -, and the first multiply before they stage, the
+// others after, so that one wave's matrix instructions run under the other's vector instructions.
+// LDS rows are 64 bytes, their four pieces permuted by the row number so that reads of neighbouring rows fall on
+// different banks.  The sums leave through LDS as whole rows.  Bound by the vector instructions of the conversion (about 560 clocks per
+// block of 64 k of a 64 x 64 tile, beside 256 of matrix instructions): 509 x 512 x 2048 from float32 10.2 -> 6.8 us, 4096 x 1024 x 4096
+// 106 -> 84 (four waves, or eight that all staged and then all multiplied; a bias load waited for before each store).  32 x 32 x 32
+// instructions are slower here (4096 x 4096 x 1024 82.6 against 74.0 us), and so are four blocks on their way or two blocks to a barrier
+// (more than 128 registers: one workgroup a CU; 2048 x 1024 x 1024 19.7 and 20.5 against 16.6 us).
+constexpr int kPitch16 = 64, kTile16Depth = 2, kTile16Threads = 512;
 __device__ __forceinline__ int piece16(int row, int c) { return (c ^ ((row >> 1) & 3)) * 16; }
 template <int BM, int BN>
-constexpr int tile16_lds() { return 2 * 2 * (BM + BN) * kPitch16; }
+constexpr int tile16_sums() { return 4 * BM * BN > 4 * (BM + BN) * kPitch16 ? 4 * BM * BN : 4 * (BM + BN) * kPitch16; }
+template <int BM, int BN>
+constexpr int tile16_lds() { return tile16_sums<BM, BN>() + 4 * (BM + BN); }
 template <typename AT, int BM, int BN, int WM, int WN, bool DUMP>
-__global__ __launch_bounds__(64 * WM * WN) void gemm16_tile_kernel(Gemm16Args g, int tiles_n) {
-  constexpr int T = 64 * WM * WN, FM = BM / WM / 16, FN = BN / WN / 16;
-  constexpr int UA = BM * 4 / T, UB = BN * 4 / T;   // pieces of 16 k a thread stages per block
-  static_assert(UA * T == BM * 4 && UB * T == BN * 4 && (T / 4) % 8 == 0, "whole pieces per thread");
+__global__ __launch_bounds__(kTile16Threads) void gemm16_tile_kernel(Gemm16Args g, int tiles_n, int tiles_m) {
+  static_assert(WM * WN == 8, "eight waves");
+  constexpr int FM = BM / WM / 16, FN = BN / WN / 16, D = kTile16Depth;   // D: blocks of K on their way
   extern __shared__ __attribute__((aligned(16))) int8_t lds16[];
-  int* const sums = reinterpret_cast<int*>(lds16);   // [BM + BN], at the end
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, lr = lane % 16, lk = lane / 16;
+  int* const sums = reinterpret_cast<int*>(lds16 + tile16_sums<BM, BN>());   // [BM + BN]
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), lr = lane % 16, lk = lane / 16;
   const int wm = wave / WN, wn = wave % WN;
-  const int m0 = (int)(blockIdx.x / tiles_n) * BM, n0 = (int)(blockIdx.x % tiles_n) * BN;
-  const int srow = tid / 4, sk = (tid % 4) * 8, spiece = piece16(srow, tid % 4);   // staging: four threads a row, T / 4 rows at a time
-  const AT* asrc[UA];
-  const int16_t* bsrc[UB];
+  int tn, tm;
+  xcd_order16(tiles_n, tiles_m, blockIdx.x, tn, tm);
+  const int m0 = tm * BM, n0 = tn * BN;
+  // what the write-out needs, requested first: this thread's four columns' biases (without a bias the weights stand in)
+  constexpr int kRowThreads = BN / 4;
+  const int wr_col = 4 * (tid % kRowThreads);
+  float bias[4];
+  const float* bias_src = g.bias ? g.bias : reinterpret_cast<const float*>(g.Bq);
 #pragma unroll
-  for(int u = 0; u < UA; ++u) asrc[u] = reinterpret_cast<const AT*>(g.A) + (size_t)min(m0 + srow + u * (T / 4), g.M - 1) * g.K;
-#pragma unroll
-  for(int u = 0; u < UB; ++u) bsrc[u] = g.Bq + (size_t)min(n0 + srow + u * (T / 4), g.N - 1) * g.K;
-  constexpr int D = kTile16Depth;   // blocks of K on their way
-  Raw<AT> ra[D][UA];
-  Raw<int16_t> rb[D][UB];
-  int asum[UA], bsum[UB];
-#pragma unroll
-  for(int u = 0; u < UA; ++u) asum[u] = 0;
-#pragma unroll
-  for(int u = 0; u < UB; ++u) bsum[u] = 0;
+  for(int e = 0; e < 4; ++e) bias[e] = bias_src[min(n0 + wr_col, g.N - 4) + e];
+  float unquant = 0.0f;
+  if(!DUMP) unquant = unquant16<AT>(g);
   Acc16 acc[FM][FN];
 #pragma unroll
   for(int i = 0; i < FM; ++i)
@@ -387,37 +450,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm16_tile_kernel(Gemm16Args g,
     for(int j = 0; j < FN; ++j) acc[i][j].clear();
   const int blocks = (g.K + 63) / 64;
   const bool half = g.K % 64 != 0;
-  auto load = [&](int kb, Raw<AT> (&ra)[UA], Raw<int16_t> (&rb)[UB]) __attribute__((always_inline)) {
-    kb = min(kb, blocks - 1);
-    const int k = kb * 64 + sk, second = half && kb == blocks - 1 ? 0 : 32;
-#pragma unroll
-    for(int u = 0; u < UA; ++u) ra[u].load(asrc[u] + k, second);
-#pragma unroll
-    for(int u = 0; u < UB; ++u) rb[u].load(bsrc[u] + k, second);
-  };
   // planes of stage t: A hi, A lo, B hi, B lo
   auto plane = [&](int t, int which, int row) {
     return lds16 + (size_t)t * (2 * (BM + BN) * kPitch16) + (which < 2 ? which * BM : 2 * BM + (which - 2) * BN) * kPitch16 + row * kPitch16;
-  };
-  auto stage = [&](int t, int kb, Raw<AT> (&ra)[UA], Raw<int16_t> (&rb)[UB]) __attribute__((always_inline)) {
-    if(half && kb == blocks - 1) {   // (the same for the whole workgroup)
-#pragma unroll
-      for(int u = 0; u < UA; ++u) ra[u].clear_second();
-    }
-#pragma unroll
-    for(int u = 0; u < UA; ++u) {
-      const Planes p = ra[u].planes();
-      asum[u] += p.sum;
-      *reinterpret_cast<v4i*>(plane(t, 0, srow + u * (T / 4)) + spiece) = p.h;
-      *reinterpret_cast<v4i*>(plane(t, 1, srow + u * (T / 4)) + spiece) = p.l;
-    }
-#pragma unroll
-    for(int u = 0; u < UB; ++u) {
-      const Planes p = rb[u].planes();
-      bsum[u] += p.sum;
-      *reinterpret_cast<v4i*>(plane(t, 2, srow + u * (T / 4)) + spiece) = p.h;
-      *reinterpret_cast<v4i*>(plane(t, 3, srow + u * (T / 4)) + spiece) = p.l;
-    }
   };
   auto multiply = [&](int t) __attribute__((always_inline)) {
     v4i bh[FN], bl[FN];
@@ -436,61 +471,101 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm16_tile_kernel(Gemm16Args g,
       for(int j = 0; j < FN; ++j) acc[i][j].add(bh[j], bl[j], ah, al);
     }
   };
+  auto run = [&](auto operand, auto element) __attribute__((always_inline)) {
+    constexpr bool kIsA = decltype(operand)::value;
+    using E = decltype(element);
+    constexpr int ROWS = kIsA ? BM : BN, U = ROWS * 4 / 256;   // pieces of 16 k a thread stages per block
+    static_assert(U * 256 == ROWS * 4, "whole pieces per thread");
+    const int st = tid % 256, srow = st / 4, sk = (st % 4) * 8, spiece = piece16(srow, st % 4);   // four threads a row, 64 rows at a time
+    const E* src[U];
+    int sum[U];
+    Raw<E> raw[D][U];
 #pragma unroll
-  for(int d = 0; d < D; ++d) load(d, ra[d], rb[d]);
-  stage(0, 0, ra[0], rb[0]);
-  load(D, ra[0], rb[0]);
-  __syncthreads();
-  int kb = 0;
-  // (the loads inside the loop stand behind no branch: the compiler would wait for them at once)
-  for(; kb + 2 * D < blocks; kb += D) {
-#pragma unroll
-    for(int d = 0; d < D; ++d) {
-      const int t = (kb + d) & 1, next = (d + 1) % D;
-      multiply(t);
-      stage(t ^ 1, kb + d + 1, ra[next], rb[next]);   // (the other stage was read before the last barrier)
-      load(kb + d + 1 + D, ra[next], rb[next]);
-      __syncthreads();
+    for(int u = 0; u < U; ++u) {
+      const int row = srow + u * 64;
+      if constexpr(kIsA) src[u] = reinterpret_cast<const E*>(g.A) + (size_t)min(m0 + row, g.M - 1) * g.K;
+      else src[u] = g.Bq + (size_t)min(n0 + row, g.N - 1) * g.K;
+      sum[u] = 0;
     }
-  }
+    auto load = [&](int kb, Raw<E> (&r)[U]) __attribute__((always_inline)) {
+      kb = min(kb, blocks - 1);
+      const int k = kb * 64 + sk, second = half && kb == blocks - 1 ? 0 : 32;
 #pragma unroll
-  for(int d = 0; d < 2 * D; ++d) {
-    if(kb + d < blocks) {   // (the same for the whole workgroup)
-      const int t = (kb + d) & 1, next = (d + 1) % D;
-      multiply(t);
-      if(kb + d + 1 < blocks) stage(t ^ 1, kb + d + 1, ra[next], rb[next]);
-      if(d + 1 < D && kb + d + 1 + D < blocks) load(kb + d + 1 + D, ra[next], rb[next]);
-      __syncthreads();
+      for(int u = 0; u < U; ++u) r[u].load(src[u] + k, second);
+    };
+    auto stage = [&](int t, int kb, Raw<E> (&r)[U]) __attribute__((always_inline)) {
+      if(kIsA && half && kb == blocks - 1) {
+#pragma unroll
+        for(int u = 0; u < U; ++u) r[u].clear_second();
+      }
+#pragma unroll
+      for(int u = 0; u < U; ++u) {
+        const Planes p = r[u].planes();
+        sum[u] += p.sum;
+        *reinterpret_cast<v4i*>(plane(t, kIsA ? 0 : 2, srow + u * 64) + spiece) = p.h;
+        *reinterpret_cast<v4i*>(plane(t, kIsA ? 1 : 3, srow + u * 64) + spiece) = p.l;
+      }
+    };
+    // one block: multiplied from stage t while block kb + 1 goes into the other one (which was read before the last barrier)
+    auto block = [&](int kb, Raw<E> (&r)[U], bool fill, bool more) __attribute__((always_inline)) {
+      const int t = kb & 1;
+      if(kIsA) multiply(t);
+      if(fill) stage(t ^ 1, kb + 1, r);
+      if(more) load(kb + 1 + D, r);
+      if(!kIsA) multiply(t);
+      lds_barrier();
+    };
+#pragma unroll
+    for(int d = 0; d < D; ++d) load(d, raw[d]);
+    stage(0, 0, raw[0]);
+    load(D, raw[0]);
+    lds_barrier();
+    int kb = 0;
+    // (the loads inside the loop stand behind no branch: the compiler would wait for them at once)
+    for(; kb + 2 * D < blocks; kb += D) {
+#pragma unroll
+      for(int d = 0; d < D; ++d) block(kb + d, raw[(d + 1) % D], true, true);
     }
-  }
-  // row sums: the four threads of a row sit side by side
 #pragma unroll
-  for(int u = 0; u < UA; ++u) {
-    asum[u] += __shfl_xor(asum[u], 1);
-    asum[u] += __shfl_xor(asum[u], 2);
-    if(tid % 4 == 0) sums[srow + u * (T / 4)] = asum[u];
-  }
+    for(int d = 0; d < 2 * D; ++d) {
+      if(kb + d < blocks) block(kb + d, raw[(d + 1) % D], kb + d + 1 < blocks, d + 1 < D && kb + d + 1 + D < blocks);
+    }
+    // row sums: the four threads of a row sit side by side
 #pragma unroll
-  for(int u = 0; u < UB; ++u) {
-    bsum[u] += __shfl_xor(bsum[u], 1);
-    bsum[u] += __shfl_xor(bsum[u], 2);
-    if(tid % 4 == 0) sums[BM + srow + u * (T / 4)] = bsum[u];
-  }
-  float unquant = 0.0f;
-  if(!DUMP) unquant = unquant16<AT>(g);
-  __syncthreads();
+    for(int u = 0; u < U; ++u) {
+      const int total = quad_sum(sum[u]);
+      if(st % 4 == 0) sums[(kIsA ? 0 : BM) + srow + u * 64] = total;
+    }
+  };
+  if(wave < 4) run(std::true_type(), AT());
+  else run(std::false_type(), int16_t());
+  // (every wave is past its last read of the stages) the sums as rows of BN, their 16-byte pieces permuted by the row number
+  constexpr int kMask = 7;
 #pragma unroll
   for(int i = 0; i < FM; ++i) {
     const int r = (wm * FM + i) * 16 + lr;
-    const int as = sums[r];
 #pragma unroll
     for(int j = 0; j < FN; ++j) {
-      const int c = (wn * FN + j) * 16 + 4 * lk;
-      v4i v = acc[i][j].sum();
-#pragma unroll
-      for(int e = 0; e < 4; ++e) v[e] = (int)((unsigned)v[e] + 128u * (unsigned)(as + sums[BM + c + e]) - 16384u * 64u * (unsigned)blocks);
-      store16<DUMP>(g, v, m0 + r, n0 + c, unquant);
+      const int p = (wn * FN + j) * 4 + lk;
+      *reinterpret_cast<v4i*>(lds16 + (r * (BN / 4) + (p ^ (r & kMask))) * 16) = acc[i][j].sum();
     }
+  }
+  lds_barrier();
+  const int n = n0 + wr_col;
+  unsigned bs[4];
+#pragma unroll
+  for(int e = 0; e < 4; ++e) {
+    bs[e] = 128u * (unsigned)sums[BM + wr_col + e] - 16384u * 64u * (unsigned)blocks;
+    asm volatile("" ::"v"(bias[e]));   // (the wait for the biases stands here, not among the stores)
+  }
+#pragma unroll
+  for(int i = 0; i < BM * kRowThreads / kTile16Threads; ++i) {
+    const int r = i * (kTile16Threads / kRowThreads) + tid / kRowThreads, m = m0 + r;
+    v4i v = *reinterpret_cast<const v4i*>(lds16 + (r * (BN / 4) + ((wr_col / 4) ^ (r & kMask))) * 16);
+    const unsigned as = 128u * (unsigned)sums[r];
+#pragma unroll
+    for(int e = 0; e < 4; ++e) v[e] = (int)((unsigned)v[e] + as + bs[e]);
+    if(m < g.M && n < g.N) store16<DUMP>(g, v, (size_t)m * g.N + n, unquant, bias);
   }
 }
 
@@ -505,8 +580,11 @@ int check16(const void* Aq, const void* Bq, const void* out, const float* bias, 
 
 template <typename AT, int MT, int NT, bool DUMP>
 int launch_stream16(const Gemm16Args& g, hipStream_t st) {
-  const dim3 grid((unsigned)((g.N + 16 * NT - 1) / (16 * NT)), (unsigned)((g.M + 16 * MT - 1) / (16 * MT)));
-  hipLaunchKernelGGL((gemm16_stream_kernel<AT, MT, NT, DUMP>), grid, dim3(64 * kStream16Waves), 0, st, g);
+  const int tiles_n = (g.N + 16 * NT - 1) / (16 * NT), tiles_m = (g.M + 16 * MT - 1) / (16 * MT);
+  constexpr int lds = stream16_lds<MT, NT>();
+  static_assert(lds <= 65536, "no attribute needed");
+  hipLaunchKernelGGL((gemm16_stream_kernel<AT, MT, NT, 2, DUMP>), dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(64 * kStream16Waves), lds, st,
+                     g, tiles_n, tiles_m);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -519,54 +597,50 @@ int launch_tile16(const Gemm16Args& g, hipStream_t st) {
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, lds, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(64 * WM * WN), lds, st, g, tiles_n);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(kTile16Threads), lds, st, g, tiles_n, tiles_m);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
 
-// Which form a call takes: the one whose busiest CU takes in the fewest bytes per step of k - its workgroups per CU
-// (at least one) times the bytes a workgroup loads, converts and multiplies for each k; the 128 x 128 tiles count half
-// again (one workgroup to a CU: products, conversion and LDS traffic overlap less).  Measured at 99 sizes (K, N = 256 ..
-// 4096, M = 1 .. 4096, launches in a graph), the form taken was never more than 6 % behind the best with int16
-// activations, 10 % with float32 ones (profiles/int16_forms.txt: every form, both kinds).  us, int16 activations:
-//   1 x 512 x 512 3.0 (stream 16 x 16), 64 x 512 x 2048 4.2 (16 x 32), 509 x 2048 x 512 10.4 (32 x 32), 509 x 512 x 2048
-//   8.6 (64 x 64), 4096 x 4096 x 4096 263 (128 x 128: 523 TOPS of 16-bit products).
-// What a call takes is another matter: each form has a start of its own and its own price of a byte (least squares over
-// the same measurements where the form is near the best: -29 .. +19 %); a CU holds one 128 x 128 tile at a time.
+// Which form a call takes: the one whose time is the least by a model that has three prices for each form - of a
+// launch, of a further workgroup per CU, and of a byte of either operand that a workgroup takes in (least squares over measurements
+// at 99 sizes where the form is near the best: -26 .. +17 %; K, N = 256 .. 4096, M = 1 .. 4096, launches in a graph; a CU holds one
+// 128 x 128 tile at a time).  The form taken is the best or at most 4 % behind it but for 256 rows of 704 values by 1408
+// (15 %: eleven steps of K over eight waves) and 64 rows of them (7 %; profiles/int16_forms.txt: every form, both kinds).  us, int16
+// and float32 activations:
+//   1 x 512 x 512 2.8 and 3.0 (stream 16 x 16), 64 x 512 x 2048 3.6 and 3.7 (16 x 32), 509 x 2048 x 512 8.1 and 8.8 (32 x 32;
+//   10.4 and 14.6 with lanes that loaded the rows they multiply), 509 x 512 x 2048 6.5 and 6.8 (64 x 64; 8.6 and 10.2 with four
+//   waves that all staged and then all multiplied), 4096 x 4096 x 4096 259 and 270 (128 x 128).
 struct Form16 {
   enum Name { kStream16, kStream16x32, kStream32x32, kTile64, kTile128 };
   Name form;
-  double cost;   // bytes per k through the busiest CU
   double ns;     // of the call
 };
 inline Form16 plan16(int M, int K, int N, int a_bytes) {
-  struct Shape { Form16::Name form; int rows, cols; double factor, start_ns, a_byte_ns, b_byte_ns; };
-  constexpr Shape shapes[] = {{Form16::kStream16, 16, 16, 1.0, 2600.0, 0.025, 0.033}, {Form16::kStream16x32, 16, 32, 1.0, 2900.0, 0.028, 0.030},
-                              {Form16::kStream32x32, 32, 32, 1.0, 3400.0, 0.033, 0.022}, {Form16::kTile64, 64, 64, 1.0, 5400.0, 0.019, 0.032},
-                              {Form16::kTile128, 128, 128, 1.5, 10000.0, 0.0155, 0.035}};
-  Form16 best{Form16::kTile128, 1e30, 0.0};
+  struct Shape { Form16::Name form; int rows, cols; double launch_ns, workgroup_ns, a_byte_ns, b_byte_ns; };
+  constexpr Shape shapes[] = {{Form16::kStream16, 16, 16, 2250.0, 270.0, 0.0057, 0.0257}, {Form16::kStream16x32, 16, 32, 1100.0, 1480.0, 0.0058, 0.0228},
+                              {Form16::kStream32x32, 32, 32, 700.0, 2190.0, 0.0098, 0.0249}, {Form16::kTile64, 64, 64, 2750.0, 530.0, 0.0061, 0.0363},
+                              {Form16::kTile128, 128, 128, 1500.0, 4400.0, 0.0052, 0.0493}};
+  Form16 best{Form16::kTile128, 1e30};
   for(const Shape& s : shapes) {
-    if(s.form < Form16::kTile64 && (M + s.rows - 1) / s.rows > 65535) continue;   // (row tiles are the grid's second dimension)
-    const double workgroups = (double)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols) / 256.0;
-    const double per_cu = workgroups > 1.0 ? workgroups : 1.0;
-    const double cost = per_cu * s.factor * (s.rows * a_bytes + s.cols * 2);
-    if(cost >= best.cost) continue;
+    const double workgroups = (double)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols);
+    if(workgroups * kTile16Threads >= 4294967296.0) continue;   // (a launch has fewer threads than that)
+    double per_cu = workgroups > 256.0 ? workgroups / 256.0 : 1.0;
+    if(s.form == Form16::kTile128) per_cu = std::ceil(per_cu);
     const int rows = M < s.rows ? M : s.rows;   // (rows past the end repeat the last one, which is in the cache)
-    const double tile = K * (s.a_byte_ns * rows * a_bytes + s.b_byte_ns * s.cols * 2);
-    best = Form16{s.form, cost, s.form == Form16::kTile128 ? std::ceil(per_cu) * (s.start_ns + tile) : s.start_ns + per_cu * tile};
+    const double ns = s.launch_ns + per_cu * (s.workgroup_ns + K * (s.a_byte_ns * rows * a_bytes + s.b_byte_ns * s.cols * 2));
+    if(ns < best.ns) best = Form16{s.form, ns};
   }
   return best;
 }
 
 // Whether float32 activations are quantized by a launch of their own first: where the multiplication then saves more
-// than the launch costs: 2 us, and 2.5 ns per thousand values up to 1.2 million and half of one beyond (the pass over
-// them, and the multiplication's wait for values that were just written).  At the 99 sizes the choice is at most 3 %
-// behind the better one but for 256 rows of 512 and of 704 values, which two 32 x 32 workgroups a CU quantize on the way (10
-// and 18 %); with one price for all forms (30 ps a byte) it was 4 .. 18 % behind at nine.
+// than the launch costs, 2 us and 0.75 ns per thousand values (the pass over them, and the multiplication's wait for values
+// that were just written).  Only the 128 x 128 tiles take rows in often enough: the other forms are never more than 1 % behind two
+// launches with one.
 inline bool quantize_first16(int64_t M, int64_t K, int64_t N) {
-  const double saved = plan16((int)M, (int)K, (int)N, 4).ns - plan16((int)M, (int)K, (int)N, 2).ns;
-  const double values = (double)M * (double)K, near = values < 1.2e6 ? values : 1.2e6;
-  return saved > 2000.0 + 0.002 * near + 0.00055 * values;
+  const Form16 one = plan16((int)M, (int)K, (int)N, 4);
+  return one.form == Form16::kTile128 && one.ns - plan16((int)M, (int)K, (int)N, 2).ns > 2000.0 + 0.00075 * (double)M * (double)K;
 }
 
 template <typename AT, bool DUMP>
@@ -581,7 +655,7 @@ int run16(const AT* A, const int16_t* Bq, const float* bias, void* out, int64_t 
     case Form16::kStream16: return launch_stream16<AT, 1, 1, DUMP>(g, st);
     case Form16::kStream16x32: return launch_stream16<AT, 1, 2, DUMP>(g, st);
     case Form16::kStream32x32: return launch_stream16<AT, 2, 2, DUMP>(g, st);
-    case Form16::kTile64: return launch_tile16<AT, 64, 64, 2, 2, DUMP>(g, st);
+    case Form16::kTile64: return launch_tile16<AT, 64, 64, 2, 4, DUMP>(g, st);
     default: return launch_tile16<AT, 128, 128, 2, 4, DUMP>(g, st);
   }
 }

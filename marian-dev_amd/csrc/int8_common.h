@@ -26,6 +26,14 @@ __device__ __forceinline__ v4i load16(const int8_t* p) {
   return *reinterpret_cast<const v4i*>(p);
 }
 
+// A workgroup barrier for what was written to LDS, and only that: __syncthreads() also orders global memory, and the
+// compiler then leaves a wait on vector memory (one that waits for nothing) among the stores of the write-out.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // (the prepared weight order and every operand offset of the kernels: operand_addressing.h)
 
 // quantMult stored behind `elements` int8 values (reference

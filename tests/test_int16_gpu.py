@@ -134,6 +134,27 @@ def test_affine16_from_float_extremes(integer, o16, synth, M, K, N):
     assert np.array_equal(integer.multiply_i32(Aq, Bq).cpu().numpy(), want_acc)
 
 
+# every form (in this order) over the lengths of its pipeline: streams take 1 .. 6 steps of 64 values of k a wave, some
+# waves one fewer, tiles 1 .. 11 blocks of 64; half a block at the end or not
+@pytest.mark.parametrize("M,N,Ks", [(5, 40, (64, 512, 544, 1056, 1568, 2080, 2592)), (70, 1800, (96, 544, 1024, 1600, 2112)),
+                                    (300, 1000, (64, 480, 576, 1184, 1696, 2592)), (520, 1048, (32, 64, 96, 160, 192, 224, 320, 352)),
+                                    (1801, 1800, (512, 544, 608, 672))])
+def test_16_bit_pipelines(integer, o16, M, N, Ks):
+    T = load("types")
+    rng = np.random.default_rng(M)
+    tail = np.frombuffer(f32(1024.0).tobytes(), np.int16)
+    for K in Ks:
+        say("pipeline", M, K, N)
+        A = rng.integers(-32768, 32768, (M, K), dtype=np.int16)
+        Bt = rng.integers(-32768, 32768, (N, K), dtype=np.int16)
+        Aq_h, Bq_h = np.concatenate([A.ravel(), tail]), np.concatenate([Bt.ravel(), tail])
+        Aq = integer.QTensor.from_numpy(qbytes(Aq_h), (M, K), T.Type.intgemm16, "cuda")
+        Bq = integer.QTensor.from_numpy(qbytes(Bq_h), (K, N), T.Type.intgemm16, "cuda")
+        want, want_acc = o16.affine(Aq_h, Bq_h, None, M, K, N, 1.0, False)
+        assert np.array_equal(integer.multiply_i32(Aq, Bq).cpu().numpy(), want_acc), K
+        assert np.array_equal(integer.dot(dev(A.astype(f32) / f32(1024.0)), Bq).cpu().numpy(), want), K
+
+
 def test_marian_operator_vectors_through_the_16_bit_path(integer, o16):
     """reference src/tests/units/operator_tests.cpp:618-659 padded to the shape rules (K = 32,
     N = 8): small integers are exact at a multiplier of 1024."""
