@@ -10,6 +10,7 @@
 #include "abi_common.h"
 #include "gemm_mfma32_kernel.h"
 #include "gemm_pair_kernel.h"
+#include "gemm_rows_kernel.h"
 #include "gemm_stream32_kernel.h"
 #include "gemm_stream_kernel.h"
 #include "quantize_kernels.h"
@@ -407,33 +408,89 @@ int launch_normed(const GemmArgs& a, const float* A, const NormInput& n, const G
   return MARIAN_HIP_OK;
 }
 
+// The tiles of a launch of gx x gy workgroups, dealt out so that the XCDs' L2 caches fetch the fewest bytes (as they come where
+// the tiles don't divide into eight blocks).
+inline RowsTiles rows_tiles(int gx, int gy, long long row_bytes, long long column_bytes) {
+  RowsTiles best{-1, 0, 0};
+  long long least = 0;
+  for(int shift = 0; shift <= 3; ++shift) {
+    const int r = 1 << shift;
+    if(gy % r != 0 || gx % (8 / r) != 0) continue;
+    const RowsTiles t{shift, gy / r, gx / (8 / r)};
+    const long long bytes = t.h * row_bytes + t.w * column_bytes;
+    if(best.shift < 0 || bytes < least) { best = t; least = bytes; }
+  }
+  return best;
+}
+
+// The form that quantizes on the way, every wave for itself: 32 columns and ROWS rows per workgroup, STEPS pairs of K
+// sub-steps to a wave.
+template <int ROWS, int STEPS>
+int launch_rows(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const GroupLaunch* groups) {
+  constexpr int lds = rows_lds_bytes<ROWS>();
+  static_assert(lds <= 48 * 1024, "default LDS limit");
+  GemmArgs a2 = a;
+  a2.blocks_y = (a.M + ROWS - 1) / ROWS;
+  a2.blocks_x = groups ? groups->table.block0[groups->table.n] : (a.n_out + 31) / 32;
+  const RowsTiles tiles = rows_tiles(a2.blocks_x, a2.blocks_y, 4ll * ROWS * a.K, 32ll * a.K);
+  const dim3 grid = tiles.shift < 0 ? dim3(a2.blocks_x, a2.blocks_y) : dim3(8, tiles.h, tiles.w);
+  if(groups) {
+    if(groups->cols != 32) return MARIAN_HIP_ERR_SHAPE;   // (table built for another kernel)
+    a2.stream_out = 0;
+    a2.absmax_out = nullptr;
+    hipLaunchKernelGGL((gemm_rows_kernel<ROWS, STEPS, GroupTable>), grid, dim3(kRowsThreads), lds, st, a2, f.A, f.aq_out, f.partials,
+                       f.n_partials, tiles, groups->table);
+  } else {
+    a2.stream_out = (long long)a.M * a.n_out * 4 >= (4ll << 20) ? 1 : 0;   // (see launch_stream32)
+    if(a.absmax_out) {   // one slot per wave
+      if((long long)a2.blocks_x * a2.blocks_y * kRowsWaves <= kAbsmaxSlots) t_absmax_written = true;
+      else a2.absmax_out = nullptr;
+    }
+    hipLaunchKernelGGL((gemm_rows_kernel<ROWS, STEPS>), grid, dim3(kRowsThreads), lds, st, a2, f.A, f.aq_out, f.partials, f.n_partials,
+                       tiles, NoGroups());
+  }
+  MH_HIP(hipGetLastError());
+  return MARIAN_HIP_OK;
+}
+// The longest K of the form: 8 pairs to a wave, 4 with 32 rows (plan_tiled's calls stay within).
+constexpr int rows_max_k(int rows) { return rows == 32 ? 2048 : 4096; }
+template <int ROWS>
+int launch_rows_steps(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const GroupLaunch* g) {
+  switch((a.K + 511) / 512) {
+    case 1: return launch_rows<ROWS, 1>(a, f, st, g);
+    case 2: return launch_rows<ROWS, 2>(a, f, st, g);
+    case 3: return launch_rows<ROWS, 3>(a, f, st, g);
+    case 4: return launch_rows<ROWS, 4>(a, f, st, g);
+  }
+  if constexpr(ROWS < 32) {
+    switch((a.K + 511) / 512) {
+      case 5: return launch_rows<ROWS, 5>(a, f, st, g);
+      case 6: return launch_rows<ROWS, 6>(a, f, st, g);
+      case 7: return launch_rows<ROWS, 7>(a, f, st, g);
+      case 8: return launch_rows<ROWS, 8>(a, f, st, g);
+    }
+  }
+  return MARIAN_HIP_ERR_SHAPE;
+}
+
 // Picks the number of K sub-steps a wave holds per chunk: the smallest instantiated value that
 // covers K in one chunk, else the largest whose activations fit the 64 KB LDS stage
 // (MT32 * KW * PW <= 64).  kFusedTiled stages fp32 values in registers: at most 4 per wave (8 when K is not split).
 template <int MT32, int MODE>
-int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int kw, bool half_rows = false,
-                       const GroupLaunch* g = nullptr, bool eight_rows = false) {
+int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int kw, int rows = 32, const GroupLaunch* g = nullptr) {
   const int need = (a.K / 32 + kw - 1) / kw;   // sub-steps per wave if K is one chunk
   if constexpr(MODE == kFusedTiled) {
-    static_assert(MT32 == 1, "tiled fused form: 32 (or 16) rows per workgroup");
+    static_assert(MT32 == 1, "tiled fused form: 32 rows per workgroup, or fewer");
     switch(kw) {
       case 1: return launch_stream32<1, 8, 1, 8, MODE>(a, f, st, g);
       case 2: return launch_stream32<1, 4, 2, 4, MODE>(a, f, st, g);
-      case 4:
-        if(half_rows) return launch_stream32<1, 2, 4, 4, MODE, 16>(a, f, st, g);
-        if(need > 4 && kernel_override() % 1000 != 690)
-          return launch_stream32<1, 2, 4, 8, MODE>(a, f, st, g);   // long rows: half as many chunks (measurement id 690 keeps the shorter ones)
+      case 4:   // 64 columns to a workgroup: with one wave's columns 64 wide instead, 128 x 1024 x 4096 takes 7.0 us, not 6.5
+        if(need > 4) return launch_stream32<1, 2, 4, 8, MODE>(a, f, st, g);   // long rows: half as many chunks
         return launch_stream32<1, 2, 4, 4, MODE>(a, f, st, g);
       default:
-        if(eight_rows && need > 4) return launch_stream32<1, 1, 8, 8, MODE, 8>(a, f, st, g);
-        if(need > 4 && half_rows && kernel_override() % 1000 != 670)
-          return launch_stream32<1, 1, 8, 8, MODE, 16>(a, f, st, g);   // long rows: half as many chunks (measurement id 670 keeps the shorter ones)
-        if(need > 2) {
-          if(half_rows) return launch_stream32<1, 1, 8, 4, MODE, 16>(a, f, st, g);
-          return launch_stream32<1, 1, 8, 4, MODE>(a, f, st, g);
-        }
-        if(half_rows) return launch_stream32<1, 1, 8, 2, MODE, 16>(a, f, st, g);
-        return launch_stream32<1, 1, 8, 2, MODE>(a, f, st, g);
+        if(rows == 8) return launch_rows_steps<8>(a, f, st, g);
+        if(rows == 16 || a.K > rows_max_k(32)) return launch_rows_steps<16>(a, f, st, g);   // (more than 2048: a measurement id asked for it)
+        return launch_rows_steps<32>(a, f, st, g);
     }
   } else {
     switch(kw) {
@@ -446,7 +503,7 @@ int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int
         return launch_stream32<MT32, 2, 4, 4, MODE>(a, f, st);
       default:
         if constexpr(MT32 == 1 && MODE == kFusedAll) {
-          if(half_rows) {
+          if(rows == 16) {
             if(need > 4) return launch_stream32<1, 1, 8, 8, MODE, 16>(a, f, st);
             if(need > 2) return launch_stream32<1, 1, 8, 4, MODE, 16>(a, f, st);
             return launch_stream32<1, 1, 8, 2, MODE, 16>(a, f, st);
@@ -465,12 +522,12 @@ int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int
 
 // The K split and the tile height of the tiled fused form for a call.  K split: the widest (most
 // loads in flight per weight row) that stays within one workgroup per CU, the narrowest if none
-// does.  Every workgroup quantizes the activation rows it multiplies; with 16 rows instead of 32
-// that work halves and the workgroups double - taken when they still fit one per CU.
+// does.  Every workgroup quantizes the activation rows it multiplies: as few rows as keep the workgroups one to a CU
+// (8 rows against 16: 64 x 1024 x 1024 3.9 and 4.2 us, 128 x 512 x 512 3.6 and 3.7; 16 against 32: 65 x 512 x 1536 3.7 and 4.1;
+// with a second workgroup on some CUs 128 x 1024 x 1024 8.6 and 4.4, 65 x 512 x 2048 8.2 and 4.1).
 struct TiledPlan {
   int kw;
-  bool half_rows;    // 16 rows
-  bool eight_rows;   // 8, for long rows
+  int rows;   // 32 unless kw is 8
 };
 TiledPlan plan_tiled(int M, int K, int n_out, int kw_override) {
   const int tiles = (n_out + 31) / 32, m_tiles = (M + 31) / 32;
@@ -478,12 +535,12 @@ TiledPlan plan_tiled(int M, int K, int n_out, int kw_override) {
   while(kw > 1 && (long long)((tiles * kw + 7) / 8) * m_tiles > compute_units()) kw >>= 1;
   if(kw_override) kw = kw_override;
   while(kw > 1 && K / 32 < kw) kw >>= 1;
+  if(kw < 8) return TiledPlan{kw, 32};
   const int ov = kernel_override() % 1000;   // 640 / 641 / 642: force 32 / 16 / 8 rows
-  const long long blocks32 = (long long)((tiles * kw + 7) / 8) * m_tiles;
-  const bool half_rows = kw >= 4 && ov != 640 && (ov == 641 || ov == 642 || (M > 16 && 2 * blocks32 <= compute_units()));
-  const bool eight_rows = half_rows && kw == 8 && K > 1024 && ov != 641 &&
-                          (ov == 642 || (long long)tiles * ((M + 7) / 8) <= compute_units());
-  return TiledPlan{kw, half_rows, eight_rows};
+  if(ov >= 640 && ov <= 642) return TiledPlan{kw, 32 >> (ov - 640)};
+  if(M <= 8 || (long long)tiles * ((M + 7) / 8) <= compute_units()) return TiledPlan{kw, 8};
+  if(M <= 16 || (long long)tiles * ((M + 15) / 16) <= compute_units()) return TiledPlan{kw, 16};
+  return TiledPlan{kw, 32};
 }
 
 // kw_override: 0 = pick the K split from the number of workgroups it gives.
@@ -510,7 +567,7 @@ int launch_stream32_auto(const GemmArgs& a, const FusedSrc& f, hipStream_t st, i
   while(kw > 1 && a.K / 32 < kw) kw >>= 1;
   if constexpr(MODE == kFusedTiled) {
     const TiledPlan plan = plan_tiled(a.M, a.K, a.n_out, kw_override);
-    return launch_stream32_kw<1, MODE>(a, f, st, plan.kw, plan.half_rows, nullptr, plan.eight_rows);
+    return launch_stream32_kw<1, MODE>(a, f, st, plan.kw, plan.rows);
   } else {
     if constexpr(MODE == kFusedAll) {
       // The smallest inputs (at most two 16-value groups per thread of four waves): one wave per
@@ -536,7 +593,7 @@ int launch_stream32_auto(const GemmArgs& a, const FusedSrc& f, hipStream_t st, i
       const int ov = kernel_override() % 1000;
       const bool rows16 = a.K / 32 >= 8 && !kw_override && ov != 650 &&
                           (ov == 651 || (a.M > 16 && (long long)tiles * ((a.M + 15) / 16) <= compute_units()));
-      if(rows16) return launch_stream32_kw<1, MODE>(a, f, st, 8, true);
+      if(rows16) return launch_stream32_kw<1, MODE>(a, f, st, 8, 16);
     }
     if(mt == 1) return launch_stream32_kw<1, MODE>(a, f, st, kw);
     if(mt == 2) return launch_stream32_kw<2, MODE>(a, f, st, kw);
@@ -1034,7 +1091,7 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
   if(!aligned(A, 16)) return MARIAN_HIP_ERR_ALIGN;
   // Measurement ids: 600 = separate prepareA and GEMM launches; 611/612/614/618 = one fused
   // kernel with that K split; 620 = abs-max launch + tiled fused kernel, 621/622/624/628 with
-  // that K split.
+  // that K split (8: the form whose waves each quantize for themselves).
   const int which = kernel_override() % 1000;
   hipStream_t hst = reinterpret_cast<hipStream_t>(stream);
   GemmArgs a;
@@ -1047,23 +1104,26 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
   a.absmax_out = absmax_out;
   FusedSrc f;
   f.A = A; f.aq_out = Aq;
-  const bool want_tiled = which >= 620 && which <= 628;
-  if(n_out > 0 && stream32_can_fuse(M, K) && which != 600 && !want_tiled) {
-    int kw = 0;
-    if(which >= 611 && which <= 618) kw = which - 610;
-    return launch_stream32_auto<kFusedAll>(a, f, hst, kw);
-  }
-  // Mid-size activations: every workgroup quantizes its own 16 or 32 rows, so the work is
-  // repeated once per 32..256 output columns; measured to pay (one launch fewer) for short rows
-  // and moderate output widths, and for longer rows when few columns leave room for 16-row
-  // workgroups with an eight-way K split (at most 64 K values per workgroup).
+  const bool want_tiled = which >= 620 && which <= 628 && K <= rows_max_k(16) && M * K <= (1 << 28);
+  // Mid-size activations: every workgroup quantizes its own rows, so the work is repeated for every column tile;
+  // measured to pay (one launch fewer) for short rows and moderate output widths, and for longer rows when few
+  // columns leave room for the eight-way K split.
+  const bool can_fuse = n_out > 0 && stream32_can_fuse(M, K);
   const bool tiled_ok = n_out > 0 && workspace && workspace_bytes >= kWorkspaceBytes &&
                         aligned(workspace, 4);
   bool tiled = want_tiled;
   if(tiled_ok && !tiled && M <= 256 && n_out <= 8192) {
     const TiledPlan plan = plan_tiled((int)M, (int)K, (int)n_out, 0);
-    tiled = K <= 1024 ||
-            (K <= 4096 && plan.kw == 8 && (long long)(plan.half_rows ? 16 : 32) * K <= 65536);
+    const bool rows = plan.kw == 8 && K <= rows_max_k(plan.rows);
+    // Activations that one workgroup can hold whole: where their abs-max is known and there are more than eight rows, a
+    // workgroup that reads its own rows only is ahead (64 x 512 x 512 3.5 against 4.7 us, 23 x 512 x 2048 3.5 and 3.9, 16 x 2048 x
+    // 512 4.7 and 5.9); up to eight rows the two are within 4 % but for long rows (1 x 2048 x 512 4.4 against 4.0).
+    tiled = can_fuse ? rows && absmax_in && M > 8 && which == 0 : K <= 1024 || rows;
+  }
+  if(can_fuse && which != 600 && !tiled) {
+    int kw = 0;
+    if(which >= 611 && which <= 618) kw = which - 610;
+    return launch_stream32_auto<kFusedAll>(a, f, hst, kw);
   }
   if(tiled_ok && which != 600 && tiled) {
     if(absmax_in) {   // the producer of A left its abs-max: no launch for it
@@ -1198,10 +1258,10 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
   // One launch for all matrices where the quantize-on-stage kernel takes the call (the same limits
   // as for a single matrix of the summed width).
   bool one_launch = false;
-  TiledPlan plan{1, false, false};
+  TiledPlan plan{1, 32};
   if(total_blocks32 > 0 && (absmax_in || have_ws) && M <= 256 && total_blocks32 * 32 <= 8192) {
     plan = plan_tiled((int)M, (int)K, (int)(total_blocks32 * 32), 0);
-    one_launch = K <= 1024 || (K <= 4096 && plan.kw == 8 && (long long)(plan.half_rows ? 16 : 32) * K <= 65536);
+    one_launch = K <= 1024 || (plan.kw == 8 && K <= rows_max_k(plan.rows));
   }
   if(one_launch) {
     GroupLaunch gl;
@@ -1228,7 +1288,7 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
       f.partials = partials;
       f.n_partials = g;
     }
-    return launch_stream32_kw<1, kFusedTiled>(a, f, hst, plan.kw, plan.half_rows, &gl, plan.eight_rows);
+    return launch_stream32_kw<1, kFusedTiled>(a, f, hst, plan.kw, plan.rows, &gl);
   }
   // Otherwise the activations are quantized once and every matrix gets its own multiplication.
   if(absmax_in) {

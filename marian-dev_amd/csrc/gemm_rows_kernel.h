@@ -1,0 +1,214 @@
+// Small-M int8 GEMM that quantizes its float32 activations on the way, every wave for itself: an abs-max launch (or the
+// producer of the activations) has left values whose maximum is max|A|.
+//
+// A workgroup makes ROWS x 32 outputs; its eight waves split K into pairs of sub-steps (64 values of k), wave w takes
+// pairs w, w + 8, ..  A wave loads the float32 rows of its pairs itself - sixteen lanes a row, whole 128-byte lines -,
+// quantizes them into LDS of its own in matrix-operand order, multiplies with weights that go from memory straight into
+// operand registers, and keeps D pairs on their way.  No value is quantized twice in a workgroup and nothing but the
+// abs-max and the partial sums at the end changes hands between the waves, so there is no barrier in the loop: one wave's
+// loads are in flight while another quantizes.  (The form before staged a chunk of K for all waves: loads, barrier,
+// quantization, barrier, products, in turn.  Reading alone takes 6.4 us of a 128 x 4096 x 1024 call in 16 x 32 tiles; the staged form
+// took 11.2, this one 8.5; 64 x 1024 x 1024 4.5 and 3.9, 65 x 512 x 1536 4.3 and 3.7, 40 x 3072 x 768 7.7 and 5.7.)
+// ROWS: 32, or 16 or 8 where few tiles would leave most CUs idle (half or a quarter of the float32 bytes and of the
+// quantizing per workgroup, twice or four times the workgroups).
+#pragma once
+
+#include <type_traits>
+
+#include "gemm_stream32_kernel.h"
+
+namespace marian_hip {
+
+constexpr int kRowsWaves = 8, kRowsThreads = kRowsWaves * kWave;
+constexpr int kRawBuffer = 0x00020000;   // a buffer descriptor's last word: 32-bit data, no swizzle
+// LDS of a wave: the four 16-value chunks of a pair, 16 bytes a row; the padding spreads the dwords of four rows over the banks
+template <int ROWS>
+constexpr int rows_chunk_bytes() { return ROWS * 16 + 64; }
+template <int ROWS>
+constexpr int rows_lds_bytes() {   // the staging, or the partial sums
+  return kRowsWaves * (ROWS * 128 > 4 * rows_chunk_bytes<ROWS>() ? ROWS * 128 : 4 * rows_chunk_bytes<ROWS>());
+}
+
+// Which tile a workgroup of gx x gy takes.  Workgroups are dealt out to the eight XCDs in turn; a split of r = 1 << shift (r divides gy,
+// 8 / r divides gx) is launched as 8 x h x w workgroups, h = gy / r, w = gx r / 8, and gives each XCD a block of h x w tiles, so
+// that its L2 fetches fewer operands.  shift < 0: launched as gx x gy.
+struct RowsTiles {
+  int shift, h, w;
+};
+struct RowsTile {
+  int bx, by;
+};
+__host__ __device__ __forceinline__ RowsTile rows_tile(RowsTiles t, int x, int y, int z) {
+  if(t.shift < 0) return RowsTile{x, y};
+  return RowsTile{(x >> t.shift) * t.w + z, (x & ((1 << t.shift) - 1)) * t.h + y};
+}
+
+// pairs of a wave that are on their way at a time, as registers allow
+constexpr int rows_depth(int rows) { return rows == 32 ? 2 : 4; }
+
+// STEPS: pairs that the first waves take, ceil(K / 512); the others take one fewer.
+template <int ROWS, int STEPS, typename GROUPS = NoGroups>
+__global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(GemmArgs args, const float* A, int8_t* aq_out, const float* partials,
+                                                                 int n_partials, RowsTiles tiles, GROUPS groups) {
+  constexpr bool GROUPED = std::is_same<GROUPS, GroupTable>::value;
+  constexpr int CHUNK = rows_chunk_bytes<ROWS>(), LOADS = ROWS / 4;   // of four rows a load
+  extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+  __shared__ float red[kRowsWaves];
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int li = lane % 32, lg = lane / 32;
+  const RowsTile tile = rows_tile(tiles, blockIdx.x, blockIdx.y, blockIdx.z);
+  const bool first_column = tile.bx == 0;
+  int bx = tile.bx;
+  if constexpr(GROUPED) bx = groups.select(args, bx);
+  const int K = args.K, M = args.M, m_base = tile.by * ROWS;
+
+  // The order of the loads: see gemm_stream32_kernel (ids first, then what is needed first, all unconditional).
+  const int n0 = bx * 32;
+  int wsrc = stream32_lane_column(n0, li, args.n_out);
+  const int bias_n = min(n0 + 4 * (lane % 8), args.n_out - 4);   // n_out % 8 == 0: four valid columns
+  uint32_t bias_at[4];
+#pragma unroll
+  for(int e = 0; e < 4; ++e) bias_at[e] = (uint32_t)(bias_n + e);
+  if(args.idx) {
+    if(args.bias) {
+#pragma unroll
+      for(int e = 0; e < 4; ++e) bias_at[e] = args.idx[bias_at[e]];
+    }
+    wsrc = (int)args.idx[wsrc];
+  }
+  asm volatile("" : "+v"(wsrc));
+  const float bqm = tail_quant_mult(args.Bq, (size_t)K * (size_t)args.N);
+  float pm[kAbsmaxSlots / kRowsThreads];
+#pragma unroll
+  for(int i = 0; i < kAbsmaxSlots / kRowsThreads; ++i) pm[i] = partials[min(tid + i * kRowsThreads, n_partials - 1)];
+
+  // lane: value group v (four values) of row 4 j + lane / 16 of load j
+  const int v = lane % 16;
+  unsigned a_off[LOADS];   // bytes from A (M * K <= 2^20 here)
+#pragma unroll
+  for(int j = 0; j < LOADS; ++j) a_off[j] = (unsigned)(min(m_base + 4 * j + lane / 16, M - 1) * K + 4 * v) * 4u;
+  const unsigned w_off = stream32_lane_offset(wsrc, lg);   // bytes from a sub-step's first column
+  const unsigned w_step = 32u * (unsigned)args.N;
+  // (as buffers: a scalar base, a scalar offset along K and a 32-bit lane offset, no vector arithmetic between the loads)
+  const auto a_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(A), 0, (int)(4u * (unsigned)M * (unsigned)K), kRawBuffer);
+  const auto w_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(args.Bq), 0, (int)((unsigned)K * (unsigned)args.N), kRawBuffer);
+  const float* bias_src = args.bias ? args.bias : reinterpret_cast<const float*>(args.Bq);   // (without a bias: dropped in the epilogue)
+  int8_t* const mine = lds + wave * 4 * CHUNK;
+  int8_t* const put = mine + (v / 4) * CHUNK + (lane / 16) * 16 + (v % 4) * 4;
+  const int8_t* const get = mine + lg * CHUNK + (li % ROWS) * 16;   // (rows past ROWS: others again, their outputs are not stored)
+  float bias_s[4], unquant = 0.0f;
+  v16i_s acc;
+  // The whole of a wave's share of K, for T steps: straight-line code, because a load behind a branch would be waited for at
+  // once.  WRITE_AQ: the quantized activations leave as well (rows past M: the last one again, to the same place).
+  auto run = [&](auto steps_tag, auto write_tag) __attribute__((always_inline)) {
+    constexpr int T = decltype(steps_tag)::value, D = T < rows_depth(ROWS) ? T : rows_depth(ROWS);
+    constexpr bool WRITE_AQ = decltype(write_tag)::value;
+    v4f a[D > 0 ? D : 1][LOADS];
+    v4i w[D > 0 ? D : 1][2];
+    auto load = [&](int t, int d) __attribute__((always_inline)) {
+      const unsigned pair = (unsigned)(wave + t * kRowsWaves);
+#pragma unroll
+      for(int j = 0; j < LOADS; ++j) a[d][j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(a_buf, a_off[j], pair * 256u, 0));
+#pragma unroll
+      for(int s = 0; s < 2; ++s) w[d][s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w_buf, w_off, (2u * pair + s) * w_step, 0));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for(int d = 0; d < D; ++d) load(d, d);
+#pragma unroll
+    for(int e = 0; e < 4; ++e) bias_s[e] = bias_src[bias_at[e]];
+    __builtin_amdgcn_sched_barrier(0);
+    float amax = 0.0f;
+#pragma unroll
+    for(int i = 0; i < kAbsmaxSlots / kRowsThreads; ++i) amax = fmaxf(amax, pm[i]);
+    const float aqm = __uint_as_float(__builtin_amdgcn_readfirstlane(
+        __float_as_uint(quant_mult_from_maxabs(block_max<kRowsWaves>(amax, red)))));
+    unquant = unquant_mult(aqm, bqm, args.scale);
+    const bool finite = aqm < __builtin_inff();   // (see gemm_stream32_kernel)
+    if(WRITE_AQ && tile.by == 0 && tid == 0) *reinterpret_cast<float*>(aq_out + (size_t)M * K) = aqm;
+#pragma unroll
+    for(int e = 0; e < 16; ++e) acc[e] = 0;
+#pragma unroll
+    for(int t = 0; t < T; ++t) {
+      const int d = t % D;
+      uint32_t q[LOADS];
+      if(finite) {
+#pragma unroll
+        for(int j = 0; j < LOADS; ++j) q[j] = quantize_pack4_finite(a[d][j], aqm);
+      } else {
+#pragma unroll
+        for(int j = 0; j < LOADS; ++j) q[j] = quantize_pack4(a[d][j], aqm);
+      }
+#pragma unroll
+      for(int j = 0; j < LOADS; ++j) *reinterpret_cast<uint32_t*>(put + j * 64) = q[j];
+      if(WRITE_AQ) {
+#pragma unroll
+        for(int j = 0; j < LOADS; ++j)
+          *reinterpret_cast<uint32_t*>(aq_out + (a_off[j] / 4 + (unsigned)((wave + t * kRowsWaves) * 64))) = q[j];
+      }
+      // (a wave's LDS operations keep their order)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for(int s = 0; s < 2; ++s) {
+        const v4i x = *reinterpret_cast<const v4i*>(get + 2 * s * CHUNK);
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[d][s], x, acc, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if(t + D < T) load(t + D, d);
+    }
+  };
+  const int pairs = K / 64;
+  const bool more = wave < pairs - (STEPS - 1) * kRowsWaves;   // this wave has STEPS pairs
+  if(aq_out && first_column) {
+    if(more) run(std::integral_constant<int, STEPS>(), std::true_type());
+    else run(std::integral_constant<int, STEPS - 1>(), std::true_type());
+  } else {
+    if(more) run(std::integral_constant<int, STEPS>(), std::false_type());
+    else run(std::integral_constant<int, STEPS - 1>(), std::false_type());
+  }
+
+  // ---- partial sums: every wave drops its ROWS x 32 NT tile into LDS (row-major, the 16-byte pieces of a row permuted by
+  //      the row number) and finishes an eighth of the rows, as in gemm_stream32_kernel ----
+  constexpr int kTileBytes = ROWS * 128;
+  __syncthreads();   // (the tiles lie over the staging of other waves)
+  if(li < ROWS) {
+#pragma unroll
+    for(int q = 0; q < 4; ++q)
+      *reinterpret_cast<v4i*>(lds + wave * kTileBytes + li * 128 + ((2 * q + lg) ^ (li & 7)) * 16) =
+          v4i{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  }
+  __syncthreads();
+  float omax = 0.0f;
+  const int n = n0 + 4 * (lane % 8), mrow = wave * (ROWS / kRowsWaves) + lane / 8, m = m_base + mrow;
+  if(lane < ROWS * 8 / kRowsWaves && m < M && n < args.n_out) {
+    const int8_t* src = lds + mrow * 128 + (((lane % 8) ^ (mrow & 7)) * 16);
+    v4i sum = *reinterpret_cast<const v4i*>(src);
+#pragma unroll
+    for(int k = 1; k < kRowsWaves; ++k) sum += *reinterpret_cast<const v4i*>(src + k * kTileBytes);
+    float y[4];
+#pragma unroll
+    for(int e = 0; e < 4; ++e) {   // y = float(acc) * unquant (+ bias); relu: y > 0 ? y : 0; multiply and add round separately
+      y[e] = (float)sum[e] * unquant;
+      if(args.bias) y[e] = y[e] + bias_s[e];
+      if(args.relu) y[e] = y[e] > 0.0f ? y[e] : 0.0f;
+      omax = fmaxf(omax, fabsf(y[e]));
+    }
+    v4f* dst = reinterpret_cast<v4f*>(reinterpret_cast<float*>(args.out) + (size_t)m * (size_t)args.n_out + (size_t)n);
+    const v4f yv = v4f{y[0], y[1], y[2], y[3]};
+    if(args.stream_out) asm volatile("global_store_dwordx4 %0, %1, off nt" : : "v"(dst), "v"(yv) : "memory");
+    else *dst = yv;
+  }
+  if(args.absmax_out) {   // a slot per wave; workgroup 0 zeroes the slots nobody owns
+    const int block = tile.by * args.blocks_x + tile.bx, used = args.blocks_x * args.blocks_y * kRowsWaves;
+    omax = wave_max(omax);
+    if(lane == 0) args.absmax_out[block * kRowsWaves + wave] = omax;
+    if(block == 0)
+      for(int sl = used + tid; sl < kAbsmaxSlots; sl += kRowsThreads) args.absmax_out[sl] = 0.0f;
+  }
+}
+
+}  // namespace marian_hip

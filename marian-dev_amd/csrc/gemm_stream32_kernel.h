@@ -17,7 +17,8 @@
 // and their quantMult to global memory, exactly what prepareA would have produced.
 // MODE kFusedTiled: for activations too large for that.  A separate small kernel leaves per-
 // workgroup abs-max values; this kernel reduces them, and quantizes its own 32 * MT32 rows chunk
-// by chunk on the way into LDS (the workgroups of column 0 also write them out).
+// by chunk on the way into LDS (the workgroups of column 0 also write them out).  For calls of so many columns that a
+// workgroup takes 64 or more; the others: gemm_rows_kernel.h.
 // MODE kFusedNorm: up to eight rows, which are the layer norm of the input (plus a skip connection): a wave
 // normalizes a row in registers, all workgroups all rows, and the quantization goes on from there.
 #pragma once
@@ -70,10 +71,9 @@ struct NoGroups {};
 // NG (kFusedAll): 16-value groups per thread that are compiled in, 2 or 4; all but the last two are
 // complete (the launcher picks NG = 2 for M * K <= 16384), so their loads, abs-max and
 // quantization carry no range checks.
-// ROWS: activation rows a workgroup multiplies, 32 * MT32 or (fused forms, MT32 = 1) 16 or (kFusedTiled) 8: half
-// or a quarter of the quantizing and of the float32 bytes per workgroup and twice or four times the workgroups, for
-// calls that would otherwise leave most CUs idle.  With ROWS < M the kFusedAll form still takes the abs-max over all of A in every
-// workgroup and quantizes only its own rows.
+// ROWS: activation rows a workgroup multiplies, 32 * MT32 or (kFusedAll, MT32 = 1) 16: half of the quantizing per
+// workgroup and twice the workgroups, for calls that would otherwise leave most CUs idle.  With ROWS < M the kFusedAll form
+// still takes the abs-max over all of A in every workgroup and quantizes only its own rows.
 template <int MT32, int WN, int KW, int PW, int MODE, int NG = 4, int ROWS = 32 * MT32, typename GROUPS = NoGroups, typename NORMED = NoNorm>
 __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs args,
                                                                         const float* A,
@@ -112,9 +112,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   const int S = K / 32;                                   // K sub-steps
   const int n_chunks = (S + Cfg::CS - 1) / Cfg::CS;
   constexpr int R = ROWS;   // activation rows of this workgroup
-  static_assert(R == MT32 * 32 || (R == 16 && MT32 == 1 && MODE != kPrequant && (FUSED || Cfg::CS % 16 == 0)) ||
-                    (R == 8 && MT32 == 1 && TILED && Cfg::CS % 32 == 0 && KW <= 8),
-                "half- and quarter-height tiles");
+  static_assert(R == MT32 * 32 || (R == 16 && MT32 == 1 && FUSED), "half-height tiles");
   const int m_base = blockIdx.y * R;
 
   // Loads of a wave return in issue order and the compiler counts them: a value is waited for
