@@ -381,8 +381,8 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
 }
 
 // The form that normalizes its input: one or several matrices, 16-row workgroups.
-template <int WN, int KW, int PW>
-int launch_normed(const GemmArgs& a, const float* A, const NormInput& n, const GroupTable* groups, hipStream_t st) {
+template <int WN, int KW, int PW, int VECS>
+int launch_normed(const GemmArgs& a, const float* A, const NormInputOf<VECS>& n, const GroupTable* groups, hipStream_t st) {
   using Cfg = Stream32Cfg<1, WN, KW, PW>;
   int lds = Cfg::kStageBytes;
   if(lds < stream32_fused_lds_bytes(1, a.K)) lds = stream32_fused_lds_bytes(1, a.K);
@@ -392,11 +392,11 @@ int launch_normed(const GemmArgs& a, const float* A, const NormInput& n, const G
   a2.blocks_y = 1;
   a2.blocks_x = groups ? groups->block0[groups->n] : (a.n_out + Cfg::kColsPerBlock - 1) / Cfg::kColsPerBlock;
   if(groups) {
-    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, GroupTable, NormInput>;
+    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, GroupTable, NormInputOf<VECS>>;
     hipLaunchKernelGGL(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, a2, A, static_cast<int8_t*>(nullptr),
                        static_cast<const float*>(nullptr), 0, *groups, n);
   } else {
-    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, NoGroups, NormInput>;
+    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, NoGroups, NormInputOf<VECS>>;
     if(a.absmax_out) {   // one slot per wave
       if((long long)a2.blocks_x * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
       else a2.absmax_out = nullptr;
@@ -1210,12 +1210,10 @@ int marian_hip_int8_affine_f32_normed(const float* A, const marian_hip_norm_inpu
                 {{A, bytes}, {norm->add, bytes}, {norm->out, bytes}, {norm->gamma, row}, {norm->beta, row}});
   }
   if(nst != MARIAN_HIP_OK) return nst;
-  const NormInput n{norm->add, norm->gamma, norm->beta, norm->out, norm->eps};
   hipStream_t hst = reinterpret_cast<hipStream_t>(stream);
   // the widest K split (most loads in flight per weight row) that stays within one workgroup per CU
   int kw = 8;
   while(kw > 1 && ((blocks32 * kw + 7) / 8 > compute_units() || K / 32 < kw)) kw >>= 1;
-  const int need = ((int)K / 32 + kw - 1) / kw;
   const GroupTable table = group_table(n_groups, Bq, bias, out, N, 32 * (8 / kw));
   const GroupTable* groups = table.n > 1 ? &table : nullptr;
   GemmArgs a;
@@ -1227,11 +1225,21 @@ int marian_hip_int8_affine_f32_normed(const float* A, const marian_hip_norm_inpu
   a.prof = g_prof.load(std::memory_order_relaxed);
 #endif
   t_absmax_written = false;
-  int st;
-  if(kw == 8) st = need <= 2 ? launch_normed<1, 8, 2>(a, A, n, groups, hst) : launch_normed<1, 8, 4>(a, A, n, groups, hst);
-  else if(kw == 4) st = need <= 4 ? launch_normed<2, 4, 4>(a, A, n, groups, hst) : launch_normed<2, 4, 8>(a, A, n, groups, hst);
-  else if(kw == 2) st = launch_normed<4, 2, 8>(a, A, n, groups, hst);
-  else st = launch_normed<8, 1, 8>(a, A, n, groups, hst);
+  auto launch = [&](auto n) {
+    constexpr int V = decltype(n)::kVecs;
+    n.add = norm->add; n.gamma = norm->gamma; n.beta = norm->beta; n.out = norm->out; n.eps = norm->eps;
+    if(kw == 8) {
+      if constexpr(V == kNormVecs / 2) return launch_normed<1, 8, 2, V>(a, A, n, groups, hst);   // (K <= 512: two sub-steps a wave)
+      else return launch_normed<1, 8, 4, V>(a, A, n, groups, hst);
+    }
+    if(kw == 4) {
+      if constexpr(V == kNormVecs / 2) return launch_normed<2, 4, 4, V>(a, A, n, groups, hst);
+      else return launch_normed<2, 4, 8, V>(a, A, n, groups, hst);
+    }
+    if(kw == 2) return launch_normed<4, 2, 8, V>(a, A, n, groups, hst);
+    return launch_normed<8, 1, 8, V>(a, A, n, groups, hst);
+  };
+  const int st = K <= kNormMaxCols / 2 ? launch(NormInputOf<kNormVecs / 2>()) : launch(NormInputOf<kNormVecs>());
   if(st != MARIAN_HIP_OK || !absmax_out || t_absmax_written) return st;
   return absmax_after(out[0], M, N[0], absmax_out, hst);
 }

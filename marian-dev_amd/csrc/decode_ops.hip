@@ -12,6 +12,7 @@
 
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 
 #include "../../include/marian_hip_int8.h"
 #include "abi_common.h"
@@ -820,18 +821,16 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
 // Measured (transformer-big step, 128 rows, 16 heads): 13.5 us against 8.2 + 8.4 us for q, k, v and
 // the self-attention over 21 positions, 13.9 against 5.3 + 8.4 us for Wq and the context attention over
 // 60 positions with every wave reading its own keys and values; staging the shared ones takes the
-// whole step from 0.437 to 0.425 ms.  Clocks read inside the kernel (weights and caches of 24
-// layers in rotation, so that they come from HBM): the launch is bound by what a CU can fetch,
-// about 15 bytes per clock when most of it misses L2 - the self-attention form's 310 KB per
-// workgroup (192 KB of weights, 32 KB of input, 86 KB of keys and values) in 26 000 clocks, the
-// context form's 156 KB (staged) in 17 700.  Tried and dropped, each without a gain in the step:
-// asking for a row's keys and values at kernel start (loads into a scratch word of LDS, by the
-// multiplying waves or by two more waves), or into registers once the abs-max is known in the
-// self-attention form - the attention then waits less and the quantization more, for the same
-// bytes; barriers that put every wave's small requests in front of any wave's large ones; the
+// whole step from 0.437 to 0.425 ms.  The self-attention form is bound by what a CU can fetch: 310 KB per workgroup
+// (192 KB of weights, 32 KB of input, 86 KB of keys and values), the latter from HBM.  Clocks inside the kernel: the
+// cached rows came only when the projections were there, 10 800 of 26 100; asked for behind the weights into registers (HELD)
+// the attention takes 3 400, the wait for the abs-max 4 400 more (a wave's requests are accepted as fast as the CU fetches),
+// and the whole 24 100.  In the smaller forms K = 512 asks for the sub-steps it has (PW: eight with repeats before), and rows are worked
+// out without a division (the launch has a dimension for sentence groups and one for hypothesis chunks): 6 rows x 8 heads over 12
+// positions 19 800 -> 15 600 clocks, their context over 23 positions 18 100 -> 14 100; 65 rows over 34 positions 19 300 -> 17 900.
+// Tried and dropped: barriers that put every wave's small requests in front of any wave's large ones; the
 // workgroups of a head starting at different sub-steps of K, so that they would not all miss L2 on
 // the same lines of the weights at the same time (+5 us per step).
-constexpr int kProjThreads = 512, kProjMaxK = 1024, kProjMaxLen = 512;
 // keys and values shared by the rows of a workgroup are staged in LDS up to this many positions
 constexpr int kProjStageLen = 96;
 constexpr int kProjMaxLds = 160 * 1024 - 256;   // dynamic LDS of a workgroup (a few bytes are static)
@@ -893,10 +892,19 @@ struct Ancestors {
   int kv_cap;
   unsigned first[kAttU];
 };
-template <bool LAST_IN_ROWS = false, bool ANC = false>
+// HELD: the rows of positions up to 4 HELD (len at most that) are in `held` already, position 4 u + lane / 16 in k[u] and
+// v[u] but for the newest, which k_last and v_last have.
+template <int HELD>
+struct HeldRows {
+  v4f k[HELD], v[HELD];
+};
+template <>
+struct HeldRows<0> {};
+template <bool LAST_IN_ROWS = false, bool ANC = false, int HELD = 0>
 __device__ __forceinline__ float attention_row64(const float* q, const float* kb, const float* vb, const float* k_last,
                                                  const float* v_last, const float* mk, float mk0, int len, float scale, float* sc,
-                                                 float* part, float* out_row, int lane, const Ancestors* anc = nullptr) {
+                                                 float* part, float* out_row, int lane, const Ancestors* anc = nullptr,
+                                                 const HeldRows<HELD>* held = nullptr) {
   constexpr int dk = 64;
   const int len4 = (len + 3) & ~3;
   const int g = lane / 16, c = lane % 16;
@@ -923,11 +931,22 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
   };
   const v4f q4 = reinterpret_cast<const v4f*>(q)[c];
   v4f kr[kAttU], vr[kAttU];
-  load_rows(kb, k_last, 0, kr);
-  load_rows(vb, v_last, 0, vr);
+  if constexpr(HELD > 0) {
+    const v4f k_new = reinterpret_cast<const v4f*>(k_last)[c], v_new = reinterpret_cast<const v4f*>(v_last)[c];
+#pragma unroll
+    for(int u = 0; u < HELD; ++u) {   // (positions past the last one: it again, dropped below)
+      const bool newest = 4 * u + g >= len - 1;
+      kr[u] = newest ? k_new : held->k[u];
+      vr[u] = newest ? v_new : held->v[u];
+    }
+  } else {
+    load_rows(kb, k_last, 0, kr);
+    load_rows(vb, v_last, 0, vr);
+  }
+  constexpr int kFirst = HELD > 0 ? HELD : kAttU;   // positions of the first pass, in fours
   for(int base = 0;;) {
 #pragma unroll
-    for(int u0 = 0; u0 < kAttU; u0 += 4) {
+    for(int u0 = 0; u0 < kFirst; u0 += 4) {
       if(base + 4 * u0 < len) {
         float s[4];
 #pragma unroll
@@ -947,7 +966,7 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
       }
     }
     base += 4 * kAttU;
-    if(base >= len) break;
+    if(HELD > 0 || base >= len) break;
     load_rows(kb, k_last, base, kr);
   }
   float mx = -__builtin_inff();
@@ -970,10 +989,10 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
   sum = wave_sum(sum);
   for(int pos = lane; pos < len; pos += 64) sc[pos] = (pos == lane ? e_first : expf(sc[pos] - mx)) / sum;
   v4f o4 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-  for(int base = 0; base < len; base += 4 * kAttU) {
-    if(base > 0) load_rows(vb, v_last, base, vr);
+  for(int base = 0; base < len; base += 4 * kAttU) {   // (rows in hand: once)
+    if(HELD == 0 && base > 0) load_rows(vb, v_last, base, vr);
 #pragma unroll
-    for(int u0 = 0; u0 < kAttU; u0 += 4) {
+    for(int u0 = 0; u0 < kFirst; u0 += 4) {
       if(base + 4 * u0 < len) {
         float w[4];
 #pragma unroll
@@ -1066,8 +1085,12 @@ __global__ __launch_bounds__(256) void attention_shared_kernel(const float* __re
 // normalizes all of them, a wave each, while its weights are on their way (a launch of its own for the norm
 // took 3.5 us of GPU and 4 of host time).
 // ANC: the self-attention's cached positions are read through the table of ancestors (attention_kernel's ANC).
-template <int NPROJ, int R, int SEGS, int PASSES, bool NORM = false, bool ANC = false>
+// PW: K sub-steps of 32 a wave loads, K / 128 rounded up to 4 or 8.
+// HELD: (self-attention) cached keys and values of up to 4 HELD positions are asked for behind the weights, so that they arrive
+// during quantization and products; 0: longer histories, asked for when the projections are there.
+template <int NPROJ, int R, int SEGS, int PASSES, int PW, int HELD, bool NORM = false, bool ANC = false>
 __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttentionArgs p) {
+  static_assert(HELD == 0 || NPROJ == 3, "the newest key and value come from the projections");
   static_assert(R == 8 || (R == 4 && !(SEGS > 0)), "a wave per row in the attention");
   constexpr bool STAGED = SEGS > 0;
   static_assert(!STAGED || NPROJ == 1, "keys and values are shared only where the caches are complete");
@@ -1076,19 +1099,36 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
   typedef int v16i_p __attribute__((ext_vector_type(16)));
   extern __shared__ __attribute__((aligned(16))) int8_t plds[];
   __shared__ float red[kProjThreads / 64];
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;   // (a scalar: what follows from it is too)
   const int wn = wave % 2, kw = wave / 2, li = lane % 32, lg = lane / 32;
   const int h = blockIdx.x;
   // input row r of this workgroup (rows past the end: M or more)
-  const int sent_base = p.share_shift < 0 ? 0 : proj_first_sentence(p.share_shift, p.share_nb, (int)blockIdx.y);
-  auto row_of = [&](int r) -> int { return proj_row_of(p.share_shift, p.share_nb, p.share_hyps, p.share_per, (int)blockIdx.y, r); };
-  const int K = p.K, M = p.M, S = K / 32, PW = S / 4, N = p.heads * 64;
+  const int sent_base = p.share_shift < 0 ? 0 : (int)blockIdx.y << p.share_shift;
+  auto row_of = [&](int r) -> int {
+    return proj_row_at(p.share_shift, p.share_nb, p.share_hyps, p.share_per, (int)blockIdx.y, (int)blockIdx.z, r);
+  };
+  const bool first_rows = blockIdx.y == 0 && blockIdx.z == 0;
+  const int K = p.K, M = p.M, S = K / 32, steps = S / 4, N = p.heads * 64;   // steps: sub-steps of a wave, at most PW
   int8_t* a_lds = plds;                                   // 32 rows x K bytes, operand order
   int8_t* part_lds = a_lds + 32 * K;                      // NPROJ x 2 x 4 partial tiles of R rows x 128 bytes
   float* proj_lds = reinterpret_cast<float*>(part_lds + NPROJ * 8 * R * 128);   // [NPROJ][R][64]
   float* att_lds = proj_lds + NPROJ * R * 64;             // per wave: scores + 256 partial outputs
   const int len4s = (p.len + 3) & ~3;
   float* kv_lds = att_lds + R * (len4s + 256);            // staged keys and values: [sentence][k, v][len][64]
+
+  const int m_wave = row_of(min(wave, R - 1));   // the row this wave attends for
+  Ancestors anc;
+  auto load_ancestors = [&]() __attribute__((always_inline)) {   // (unconditional: waits count)
+    static_assert(!ANC || (NPROJ == 3 && !STAGED), "self-attention");
+    anc.row = p.anc + (size_t)min(m_wave, M - 1) * p.kv_cap;
+    anc.n_hyp = (unsigned)M; anc.heads = (unsigned)p.heads; anc.head = (unsigned)h; anc.kv_cap = p.kv_cap;
+#pragma unroll
+    for(int u = 0; u < (HELD > 0 ? HELD : kAttU); ++u) anc.first[u] = anc.row[min(4 * u + lane / 16, p.len - 1)];
+  };
+  if constexpr(ANC && HELD > 0) {   // (they are addresses)
+    load_ancestors();
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // ---- everything this workgroup will need is requested now, in the order of its use (a wave's
   //      loads complete in the order of their issue): abs-max slots, the input rows, weights, the
@@ -1099,7 +1139,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
   const int r_in = grp / (2 * S), c16 = grp % (2 * S);
   const bool has_in = !NORM && r_in < R;
   v4f in[4];
-  NormRow nr;
+  NormRow<PW == 4 ? kNormVecs / 2 : kNormVecs> nr;
   if constexpr(NORM) {
     nr.load(p.A, p.norm, M, K);
     __builtin_amdgcn_sched_barrier(0);
@@ -1111,12 +1151,12 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
 #pragma unroll
     for(int e = 0; e < 4; ++e) in[e] = *reinterpret_cast<const v4f*>(src + e * 16);
   }
-  v4i w[NPROJ][8];
+  v4i w[NPROJ][PW];
   const int ncol = h * 64 + wn * 32 + li;
   // (asked for in the order the multiplication takes them: sub-step by sub-step, all projections)
 #pragma unroll
-  for(int pp = 0; pp < 8; ++pp) {
-    const size_t at = stream32_lane_offset(ncol, lg) + (size_t)stream32_clamped_substep(kw * PW + pp, S) * 32u * (size_t)N;
+  for(int pp = 0; pp < PW; ++pp) {
+    const size_t at = stream32_lane_offset(ncol, lg) + (size_t)stream32_clamped_substep(kw * steps + pp, S) * 32u * (size_t)N;
 #pragma unroll
     for(int g = 0; g < NPROJ; ++g) w[g][pp] = load16(p.Bq[g] + at);
   }
@@ -1124,7 +1164,6 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
   constexpr int kStageSegs = STAGED ? SEGS : 1, kStagePasses = STAGED ? PASSES : 1;
   v4f stage[kStageSegs][kStagePasses];
   // the mask value of this wave's row for position `lane`
-  const int m_wave = row_of(min(wave, R - 1));
   const float* mk = nullptr;
   if(p.mask && m_wave < M) {
     unsigned mask_row = (unsigned)m_wave;
@@ -1132,14 +1171,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
     mk = p.mask + (size_t)mask_row * p.len;
   }
   const float mk0 = *(mk ? mk + min(lane, p.len - 1) : p.A);   // (the latter not looked at)
-  Ancestors anc;
-  if constexpr(ANC) {   // (unconditional: waits count)
-    static_assert(NPROJ == 3 && !STAGED, "self-attention");
-    anc.row = p.anc + (size_t)min(m_wave, M - 1) * p.kv_cap;
-    anc.n_hyp = (unsigned)M; anc.heads = (unsigned)p.heads; anc.head = (unsigned)h; anc.kv_cap = p.kv_cap;
-#pragma unroll
-    for(int u = 0; u < kAttU; ++u) anc.first[u] = anc.row[min(4 * u + lane / 16, p.len - 1)];
-  }
+  if constexpr(ANC && HELD == 0) load_ancestors();
   float bqm[NPROJ];
 #pragma unroll
   for(int g = 0; g < NPROJ; ++g) bqm[g] = tail_quant_mult(p.Bq[g], (size_t)K * (size_t)N);
@@ -1153,6 +1185,29 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
     const float* b = pick3(p.bias, tg / 2);
     // (no bias: sixteen bytes of the weights instead, not looked at)
     bias4[it] = *reinterpret_cast<const v4f*>(b ? b + h * 64 + (tg % 2) * 32 + pc * 4 : reinterpret_cast<const float*>(p.Bq[0]));
+  }
+
+  HeldRows<HELD> held;
+  if constexpr(HELD > 0) {   // (as buffers: a wave without a row asks for nothing, and the waits still count)
+    __builtin_amdgcn_sched_barrier(0);
+    const bool mine = wave < R && m_wave < M;
+    const size_t entry = ANC ? 0 : (size_t)min(m_wave, M - 1) * p.heads + h;
+    const unsigned bytes = mine ? (ANC ? (unsigned)M * (unsigned)p.heads : 1u) * (unsigned)p.kv_cap * 256u : 0u;
+    const auto k_buf = __builtin_amdgcn_make_buffer_rsrc(p.k_cache + entry * p.kv_cap * 64, 0, (int)bytes, kRawBuffer);
+    const auto v_buf = __builtin_amdgcn_make_buffer_rsrc(p.v_cache + entry * p.kv_cap * 64, 0, (int)bytes, kRawBuffer);
+    unsigned at[HELD];
+#pragma unroll
+    for(int u = 0; u < HELD; ++u) {
+      const unsigned pos = (unsigned)(4 * u + lane / 16);
+      at[u] = pos * 256u + (lane % 16) * 16u;
+      if(ANC) at[u] += (min(anc.first[u], anc.n_hyp - 1u) * (unsigned)p.heads + (unsigned)h) * (unsigned)p.kv_cap * 256u;
+      if((int)pos >= p.len - 1) at[u] = 0xFFFFFFF0u;   // (past the cached ones: past the buffer, nothing is fetched)
+    }
+#pragma unroll
+    for(int u = 0; u < HELD; ++u) held.k[u] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(k_buf, at[u], 0, 0));
+#pragma unroll
+    for(int u = 0; u < HELD; ++u) held.v[u] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(v_buf, at[u], 0, 0));
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   // ---- 1, 2: abs-max, quantize into LDS ----
@@ -1198,14 +1253,14 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
     }
   }
   if constexpr(NORM) {   // wave w holds row w: quantized where this workgroup multiplies it, written out by one workgroup
-    const int row = __builtin_amdgcn_readfirstlane(wave);
+    const int row = wave;
     if(row < M) {
       for(int r = 0; r < R; ++r)
         if(row_of(r) == row) nr.quantize(a_lds, r, K, aqm, proj_row_key);
-      if(h == 0 && blockIdx.y == 0) nr.store(p.norm, row, K);
+      if(h == 0 && first_rows) nr.store(p.norm, row, K);
     }
   }
-  if(p.aq_out && h == 0 && blockIdx.y == 0 && tid == 0) *reinterpret_cast<float*>(p.aq_out + (size_t)M * K) = aqm;
+  if(p.aq_out && h == 0 && first_rows && tid == 0) *reinterpret_cast<float*>(p.aq_out + (size_t)M * K) = aqm;
   __syncthreads();
 
   // ---- 3: multiply (rows R .. 31 of the operand are whatever LDS held: they only feed output rows
@@ -1216,9 +1271,9 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
 #pragma unroll
     for(int v = 0; v < 16; ++v) acc[g][v] = 0;
 #pragma unroll
-  for(int pp = 0; pp < 8; ++pp) {
-    if(pp < PW) {   // (the same for the whole workgroup)
-      const int s = kw * PW + pp;
+  for(int pp = 0; pp < PW; ++pp) {
+    if(pp < steps) {   // (the same for the whole workgroup)
+      const int s = kw * steps + pp;
       const v4i a = *reinterpret_cast<const v4i*>(a_lds + s * 1024 + (lg * 32 + (li ^ proj_row_key(2 * s + lg))) * 16);
 #pragma unroll
       for(int g = 0; g < NPROJ; ++g) acc[g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[g][pp], a, acc[g], 0, 0, 0);
@@ -1287,7 +1342,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
 
   // ---- 5: the attention of row `wave` ----
   const int rows_total = M * p.heads;
-  if(p.absmax_out && blockIdx.x == 0 && blockIdx.y == 0)   // slots past the last query row
+  if(p.absmax_out && h == 0 && first_rows)   // slots past the last query row
     for(int sl = rows_total + tid; sl < kAbsmaxSlots; sl += kProjThreads) p.absmax_out[sl] = 0.0f;
   const int m = m_wave;
   if(wave < R && m < M) {   // (whole waves)
@@ -1306,6 +1361,9 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
       const float* vs = ks + (size_t)p.len * 64;
       omax = attention_row64<true>(q, ks, vs, ks + (size_t)(p.len - 1) * 64, vs + (size_t)(p.len - 1) * 64, mk, mk0, p.len,
                              p.att_scale, sc, sc + len4, p.out + (size_t)wr * 64, lane);
+    } else if constexpr(HELD > 0) {
+      omax = attention_row64<false, false, HELD>(q, kb, vb, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
+                                                 p.out + (size_t)wr * 64, lane, nullptr, &held);
     } else if constexpr(ANC) {
       omax = attention_row64<false, true>(q, p.k_cache, p.v_cache, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
                                           p.out + (size_t)wr * 64, lane, &anc);
@@ -2433,6 +2491,19 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
   return MARIAN_HIP_OK;
 }
 
+}  // extern "C"
+template <int NPROJ, int R, int SEGS, int PASSES, int PW, int HELD, bool NORM, bool ANC>
+static int launch_proj(const ProjAttentionArgs& p, dim3 grid, size_t lds, hipStream_t st) {
+  auto kernel = proj_attention_kernel<NPROJ, R, SEGS, PASSES, PW, HELD, NORM, ANC>;
+  static std::atomic<uint64_t> lds_done{0};
+  const int lst = allow_lds(kernel, SEGS > 0 ? kProjMaxLds : 96 * 1024, lds_done);
+  if(lst != MARIAN_HIP_OK) return lst;
+  hipLaunchKernelGGL(kernel, grid, dim3(kProjThreads), lds, st, p);
+  MH_HIP(hipGetLastError());
+  return MARIAN_HIP_OK;
+}
+
+extern "C" {
 static int proj_attention(const float* A, const marian_hip_norm_input* norm, const uint32_t* anc, int8_t* Aq, int64_t n_proj, const int8_t* const* Bq,
                           const float* const* bias, float* const* proj_out, int64_t M, int64_t K,
                           int64_t heads, float* k_cache, float* v_cache, int64_t batchKV, int64_t len,
@@ -2515,30 +2586,6 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, con
   const int rows = four ? 4 : R;
   size_t lds = (size_t)32 * (size_t)K + (size_t)n_proj * 8 * rows * 128 + (size_t)n_proj * rows * 64 * 4 +
                (size_t)rows * (size_t)(len4 + 256) * 4;
-  {   // the kernels' dynamic LDS limit, raised once per device (one bit per device)
-    static std::atomic<uint64_t> lds_done{0};
-    int dev = 0;
-    MH_HIP(hipGetDevice(&dev));
-    if(dev < 0 || dev >= 64) return MARIAN_HIP_ERR_RANGE;
-    if(!(lds_done.load(std::memory_order_acquire) & (1ull << dev))) {
-      const void* staged[] = {
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 1>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 2>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 3>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 1>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 2>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 3>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 1, true>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 2, true>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 2, 3, true>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 1, true>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 2, true>), reinterpret_cast<const void*>(proj_attention_kernel<1, R, 4, 3, true>)};
-      for(const void* f : staged) MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kProjMaxLds));
-      const void* unstaged[] = {
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0>),
-          reinterpret_cast<const void*>(proj_attention_kernel<1, R, 0, 0, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, true>),
-          reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0>), reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, true>),
-          reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, false, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, R, 0, 0, true, true>),
-          reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, false, true>), reinterpret_cast<const void*>(proj_attention_kernel<3, 4, 0, 0, true, true>)};
-      for(const void* f : unstaged) MH_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-      lds_done.fetch_or(1ull << dev, std::memory_order_release);
-    }
-  }
   ProjRowPlan plan = proj_row_plan(n_proj, M, heads, batchKV, len, kProjStageLen, lds, (size_t)kProjMaxLds);
   if(four) {
     plan.per_wg = 4;
@@ -2551,38 +2598,46 @@ static int proj_attention(const float* A, const marian_hip_norm_input* norm, con
   p.stage_kv = plan.stage;
   if(plan.blocks_y > 65535) return MARIAN_HIP_ERR_RANGE;
   if(plan.stage) lds += (size_t)(2 << plan.shift) * (size_t)len * 256;
-  const dim3 grid((unsigned)heads, (unsigned)plan.blocks_y);
-#define MH_PA(NP, ROWS, SEGS, PASSES)                                                                                       \
-  do {                                                                                                                      \
-    if(norm) hipLaunchKernelGGL((proj_attention_kernel<NP, ROWS, SEGS, PASSES, true>), grid, dim3(kProjThreads), lds, st, p); \
-    else hipLaunchKernelGGL((proj_attention_kernel<NP, ROWS, SEGS, PASSES>), grid, dim3(kProjThreads), lds, st, p);           \
-  } while(0)
-#define MH_PAA(ROWS, NORM) \
-  hipLaunchKernelGGL((proj_attention_kernel<3, ROWS, 0, 0, NORM, true>), grid, dim3(kProjThreads), lds, st, p)
-  if(anc) {
-    if(four && norm) MH_PAA(4, true);
-    else if(four) MH_PAA(4, false);
-    else if(norm) MH_PAA(R, true);
-    else MH_PAA(R, false);
-  } else if(four) MH_PA(3, 4, 0, 0);
-  else if(n_proj == 3) MH_PA(3, R, 0, 0);
-  else if(!p.stage_kv) MH_PA(1, R, 0, 0);
-  else {
-    const int passes = ((int)len + 31) / 32;   // 1 .. 3
-    if(p.share_shift == 0) {   // one sentence per workgroup
-      if(passes == 1) MH_PA(1, R, 2, 1);
-      else if(passes == 2) MH_PA(1, R, 2, 2);
-      else MH_PA(1, R, 2, 3);
-    } else {
-      if(passes == 1) MH_PA(1, R, 4, 1);
-      else if(passes == 2) MH_PA(1, R, 4, 2);
-      else MH_PA(1, R, 4, 3);
-    }
-  }
-#undef MH_PA
-#undef MH_PAA
-  MH_HIP(hipGetLastError());
-  return MARIAN_HIP_OK;
+  const unsigned groups = plan.shift < 0 ? (unsigned)plan.blocks_y : (unsigned)proj_groups(plan.shift, plan.sentences);
+  const dim3 grid((unsigned)heads, groups, (unsigned)plan.blocks_y / groups);
+  // The cached rows are asked for behind the weights where they and the weights fit the registers: 64 positions beside 4 sub-steps of
+  // three matrices, 32 beside 8 (an ancestor's row by a 32-bit offset into the caches).
+  const int most_held = K <= 512 ? 16 : 8;
+  const int held = n_proj != 3 || len > 4 * most_held || (anc && M * heads * kv_capacity >= (1 << 24)) || kv_capacity >= (1 << 24)
+                       ? 0 : (len <= 32 ? 8 : 16);
+  const int passes = ((int)len + 31) / 32;   // of the staged context's positions, 1 .. 3
+  auto launch = [&](auto pw) {
+    constexpr int PW = decltype(pw)::value;
+    auto rows_held = [&](auto rows, auto held_tag) {
+      constexpr int ROWS = decltype(rows)::value, HELD = decltype(held_tag)::value;
+      if(anc && norm) return launch_proj<3, ROWS, 0, 0, PW, HELD, true, true>(p, grid, lds, st);
+      if(anc) return launch_proj<3, ROWS, 0, 0, PW, HELD, false, true>(p, grid, lds, st);
+      if(norm) return launch_proj<3, ROWS, 0, 0, PW, HELD, true, false>(p, grid, lds, st);
+      return launch_proj<3, ROWS, 0, 0, PW, HELD, false, false>(p, grid, lds, st);
+    };
+    auto self = [&](auto rows) {
+      if constexpr(PW == 4) {
+        if(held == 16) return rows_held(rows, std::integral_constant<int, 16>());
+      }
+      if(held == 8) return rows_held(rows, std::integral_constant<int, 8>());
+      return rows_held(rows, std::integral_constant<int, 0>());
+    };
+    auto context = [&](auto segs, auto pass) {
+      constexpr int SEGS = decltype(segs)::value, PASSES = decltype(pass)::value;
+      if(norm) return launch_proj<1, R, SEGS, PASSES, PW, 0, true, false>(p, grid, lds, st);
+      return launch_proj<1, R, SEGS, PASSES, PW, 0, false, false>(p, grid, lds, st);
+    };
+    auto staged = [&](auto segs) {
+      if(passes == 1) return context(segs, std::integral_constant<int, 1>());
+      if(passes == 2) return context(segs, std::integral_constant<int, 2>());
+      return context(segs, std::integral_constant<int, 3>());
+    };
+    if(four) return self(std::integral_constant<int, 4>());
+    if(n_proj == 3) return self(std::integral_constant<int, R>());
+    if(!p.stage_kv) return context(std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
+    return p.share_shift == 0 ? staged(std::integral_constant<int, 2>()) : staged(std::integral_constant<int, 4>());   // one sentence or two
+  };
+  return K <= 512 ? launch(std::integral_constant<int, 4>()) : launch(std::integral_constant<int, 8>());
 }
 
 int marian_hip_int8_proj_attention(const float* A, int8_t* Aq, int64_t n_proj, const int8_t* const* Bq,

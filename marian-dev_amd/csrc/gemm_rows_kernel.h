@@ -20,7 +20,6 @@
 namespace marian_hip {
 
 constexpr int kRowsWaves = 8, kRowsThreads = kRowsWaves * kWave;
-constexpr int kRawBuffer = 0x00020000;   // a buffer descriptor's last word: 32-bit data, no swizzle
 // LDS of a wave: the four 16-value chunks of a pair, 16 bytes a row; the padding spreads the dwords of four rows over the banks
 template <int ROWS>
 constexpr int rows_chunk_bytes() { return ROWS * 16 + 64; }

@@ -35,7 +35,9 @@ typedef int v16i_s __attribute__((ext_vector_type(16)));
 
 constexpr int kFusedMaxElems = 32768;   // fp32 activations a workgroup holds in registers
 constexpr int kPrequant = 0, kFusedAll = 1, kFusedTiled = 2, kFusedNorm = 3;            // MODE
-struct NoNorm {};
+struct NoNorm {
+  static constexpr int kVecs = kNormVecs;
+};
 
 // The 32 rows of 16-byte chunk c16 of the activations are stored XOR-permuted by this key.  Any key
 // leaves a fragment read (32 consecutive slots, permuted) free of bank conflicts; this one makes
@@ -167,7 +169,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   // Quad number qi = j * threads / 4 + tid / 4 covers groups 4 * qi .. 4 * qi + 3; group g is row
   // g / (K/16), 16-byte chunk g % (K/16).
   v4f vals[FUSED && !NORM ? kFusedGroups : 1][4];
-  NormRow nrow;
+  NormRow<NORMED::kVecs> nrow;
   if constexpr(NORM) nrow.load(A, norm, M, K);
   const int n16 = M * K / 16;   // groups; a multiple of four
   const int quad = tid / 4, qlane = tid % 4;

@@ -12,6 +12,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64;        // CDNA wavefront
+constexpr int kRawBuffer = 0x00020000;   // a buffer descriptor's last word: 32-bit data, no swizzle
 constexpr int kFragBytes = 1024; // one MFMA 16x16x64 i8 operand: 64 lanes x 16 bytes
 
 // D[i][j] += sum_k A[i][k] * B[j][k] over 64 values of k.  Lane l supplies 16 consecutive

@@ -29,24 +29,25 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
-constexpr int kNormVecs = 4;   // float4 per lane: rows of up to 1024 values, cols % 4 == 0
+constexpr int kNormVecs = 4;   // float4 per lane: rows of up to 1024 values, cols % 4 == 0 (half as many: up to 512)
 
 // Value j of a lane is float4 number j * 64 + lane of the row; positions past the row are clamped by the
 // loader and dropped here.  v: the row, becomes its normalization (clamped positions: anything); t: what is added to
 // it first (has_add).  Returns the largest magnitude of this lane's values.
-__device__ __forceinline__ float normalize_row(v4f (&v)[kNormVecs], const v4f (&t)[kNormVecs], bool has_add, const v4f (&gm)[kNormVecs],
-                                               const v4f (&bt)[kNormVecs], bool has_beta, int cols, float eps) {
+template <int VECS>
+__device__ __forceinline__ float normalize_row(v4f (&v)[VECS], const v4f (&t)[VECS], bool has_add, const v4f (&gm)[VECS],
+                                               const v4f (&bt)[VECS], bool has_beta, int cols, float eps) {
   const int lane = threadIdx.x % kWave, cols4 = cols / 4;
   float sum = 0.0f;
 #pragma unroll
-  for(int j = 0; j < kNormVecs; ++j) {
+  for(int j = 0; j < VECS; ++j) {
     if(has_add) v[j] = v4f{v[j].x + t[j].x, v[j].y + t[j].y, v[j].z + t[j].z, v[j].w + t[j].w};
     if(j * kWave + lane < cols4) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
   }
   const float mean = wave_sum(sum) / (float)cols;
   float sq = 0.0f;
 #pragma unroll
-  for(int j = 0; j < kNormVecs; ++j) {
+  for(int j = 0; j < VECS; ++j) {
     if(j * kWave + lane < cols4) {
       const float d0 = v[j].x - mean, d1 = v[j].y - mean, d2 = v[j].z - mean, d3 = v[j].w - mean;
       sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
@@ -55,7 +56,7 @@ __device__ __forceinline__ float normalize_row(v4f (&v)[kNormVecs], const v4f (&
   const float sigma = sqrtf(wave_sum(sq) / (float)cols + eps);
   float omax = 0.0f;
 #pragma unroll
-  for(int j = 0; j < kNormVecs; ++j) {
+  for(int j = 0; j < VECS; ++j) {
     if(j * kWave + lane < cols4) {
       float r[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
       const float g[4] = {gm[j].x, gm[j].y, gm[j].z, gm[j].w}, b[4] = {bt[j].x, bt[j].y, bt[j].z, bt[j].w};
@@ -82,20 +83,26 @@ struct NormInput {
   float* out;           // [M x K]: the normalized rows, written by one workgroup
   float eps;
 };
+// The same with the vectors a lane takes of a row, as a kernel argument.
+template <int VECS>
+struct NormInputOf : NormInput {
+  static constexpr int kVecs = VECS;
+};
+template <int VECS>
 struct NormRow {
-  v4f v[kNormVecs], t[kNormVecs], gm[kNormVecs], bt[kNormVecs];
+  v4f v[VECS], t[VECS], gm[VECS], bt[VECS];
   // Wave w loads row w (rows past M: a copy of the last one).  All loads unconditional, so that waits count them exactly.
   __device__ __forceinline__ void load(const float* A, const NormInput& n, int M, int K) {
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, cols4 = K / 4;
     const size_t row = (size_t)min(wave, M - 1) * K;
 #pragma unroll
-    for(int j = 0; j < kNormVecs; ++j) {
+    for(int j = 0; j < VECS; ++j) {
       const int i = min(j * kWave + lane, cols4 - 1);
       v[j] = reinterpret_cast<const v4f*>(A + row)[i];
       t[j] = reinterpret_cast<const v4f*>(n.add + row)[i];
     }
 #pragma unroll
-    for(int j = 0; j < kNormVecs; ++j) {
+    for(int j = 0; j < VECS; ++j) {
       const int i = min(j * kWave + lane, cols4 - 1);
       gm[j] = reinterpret_cast<const v4f*>(n.gamma)[i];
       bt[j] = reinterpret_cast<const v4f*>(n.beta)[i];
@@ -111,7 +118,7 @@ struct NormRow {
     const int lane = threadIdx.x % kWave;
     const bool finite = qm < __builtin_inff();
 #pragma unroll
-    for(int j = 0; j < kNormVecs; ++j) {
+    for(int j = 0; j < VECS; ++j) {
       const int i = j * kWave + lane, c16 = i / 4;
       if(i < K / 4)
         *reinterpret_cast<uint32_t*>(lds + ((c16 / 2) * 64 + (c16 % 2) * 32 + (row ^ key(c16))) * 16 + (i % 4) * 4) =
@@ -121,7 +128,7 @@ struct NormRow {
   __device__ __forceinline__ void store(const NormInput& n, int row, int K) const {
     const int lane = threadIdx.x % kWave;
 #pragma unroll
-    for(int j = 0; j < kNormVecs; ++j)
+    for(int j = 0; j < VECS; ++j)
       if(j * kWave + lane < K / 4) reinterpret_cast<v4f*>(n.out + (size_t)row * K)[j * kWave + lane] = v[j];
   }
 };

@@ -135,17 +135,25 @@ __host__ __device__ __forceinline__ ProjRowPlan proj_row_plan(long long n_proj, 
   plan.stage = best_shift <= 1 && len <= stage_len && lds_without + kv_bytes <= lds_max;
   return plan;
 }
-// input row r (0 .. 7) of workgroup block_y; rows that do not exist: a value of at least M (= hyps * sentences)
-__host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, int hyps, int per_wg, int block_y, int r) {
-  if(shift < 0) return block_y * per_wg + r;
-  const int groups = sentences >> shift;
-  const int j = r >> shift, hyp = (block_y / groups) * per_wg + j;
+// Input row r (0 .. 7) of the workgroup of sentence group `group` and hypothesis chunk `chunk` (shift < 0: of rows number
+// `group`); rows that do not exist: a value of at least M (= hyps * sentences).  The launch has a dimension for either, so
+// that no workgroup divides.
+__host__ __device__ __forceinline__ int proj_row_at(int shift, int sentences, int hyps, int per_wg, int group, int chunk, int r) {
+  if(shift < 0) return group * per_wg + r;
+  const int j = r >> shift, hyp = chunk * per_wg + j;
   if(j >= per_wg || hyp >= hyps) return 0x7fffffff;
-  return hyp * sentences + ((block_y % groups) << shift) + (r & ((1 << shift) - 1));
+  return hyp * sentences + (group << shift) + (r & ((1 << shift) - 1));
+}
+// sentence groups of a launch (shift >= 0), and the tile of workgroup block_y of its groups x chunks
+__host__ __device__ __forceinline__ int proj_groups(int shift, int sentences) { return sentences >> shift; }
+__host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, int hyps, int per_wg, int block_y, int r) {
+  if(shift < 0) return proj_row_at(shift, sentences, hyps, per_wg, block_y, 0, r);
+  const int groups = proj_groups(shift, sentences);
+  return proj_row_at(shift, sentences, hyps, per_wg, block_y % groups, block_y / groups, r);
 }
 // first sentence of workgroup block_y (shift >= 0)
 __host__ __device__ __forceinline__ int proj_first_sentence(int shift, int sentences, int block_y) {
-  return (block_y % (sentences >> shift)) << shift;
+  return (block_y % proj_groups(shift, sentences)) << shift;
 }
 
 }  // namespace marian_hip

@@ -185,3 +185,41 @@ def test_proj_attention_argument_checks(integer):
     assert call(3, 8, 128, 2, 16, 5, 4) == L.ERR_SHAPE        # capacity < len
     assert call(3, 8, 128, 2, 8, 1, 1) == L.ERR_SHAPE         # self-attention: an entry per query row
     assert call(3, 0, 128, 2, 16, 1, 1) == L.OK               # empty batch
+
+
+@pytest.mark.parametrize("K", [128, 512, 640, 1024])
+@pytest.mark.parametrize("M", [3, 9, 40])
+def test_cached_rows_asked_for_early(integer, M, K):
+    """histories at the edges of what is asked for behind the weights (32 and 64 positions, by K), rows of the caches that
+    hold nothing yet (NaN), caches of the rows' own and over a table of ancestors: the separate calls' bits"""
+    import torch
+    ops = load("ops")
+    heads = K // 64
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + K)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    ws = [(integer.prepareB(r(K, K) * 0.02), r(K) * 0.01) for _ in range(3)]
+    x = r(M, K)
+    xmax = integer.AbsMax(x.device)
+    xmax.data.zero_()
+    xmax.data[1] = x.abs().max()
+    (q, k, v), _ = integer.affine_f32_grouped(x, ws, absmax=xmax)
+    for T in (1, 2, 4, 5, 29, 31, 32, 33, 36, 61, 64, 65, 70):
+        say("early rows", M, K, T)
+        cap = T + 3
+        kc, vc = r(M * heads, cap, 64), r(M * heads, cap, 64)
+        kc[:, T - 1:], vc[:, T - 1:] = float("nan"), float("nan")
+        kc2, vc2 = kc.clone(), vc.clone()
+        want = ops.Attention(q.view(M * heads, 1, 64), kc, vc, kNew=k.view(M * heads, 64), vNew=v.view(M * heads, 64), kvLen=T)
+        got = ops.ProjectedAttention(x, ws, kc2, vc2, heads, kvLen=T, absmax=xmax)[0]
+        assert torch.equal(got.view(-1), want.view(-1)), T
+        assert torch.equal(kc2[:, :T], kc[:, :T]) and torch.equal(vc2[:, :T], vc[:, :T]), T
+        # the same histories scattered over the hypotheses' entries
+        anc = torch.randint(0, M, (M, cap), device="cuda", generator=g, dtype=torch.int32)
+        kc, vc = r(M * heads, cap, 64), r(M * heads, cap, 64)
+        own, at = torch.arange(cap, device="cuda")[None, None, :], anc.long()[:, None, :]
+        pick = lambda c: c.view(M, heads, cap, 64)[at, torch.arange(heads, device="cuda")[None, :, None], own].reshape(M * heads, cap, 64).clone()
+        ks, vs = pick(kc), pick(vc)
+        want = ops.Attention(q.view(M * heads, 1, 64), ks, vs, kNew=k.view(M * heads, 64), vNew=v.view(M * heads, 64), kvLen=T)
+        got = ops.ProjectedAttentionByAncestors(x, ws, kc, vc, anc, T, absmax=xmax)[1]
+        assert torch.equal(got.view(-1), want.view(-1)), T
