@@ -831,6 +831,7 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
 // Tried and dropped: barriers that put every wave's small requests in front of any wave's large ones; the
 // workgroups of a head starting at different sub-steps of K, so that they would not all miss L2 on
 // the same lines of the weights at the same time (+5 us per step).
+constexpr int kProjThreads = 512, kProjMaxK = 1024, kProjMaxLen = 512;
 // keys and values shared by the rows of a workgroup are staged in LDS up to this many positions
 constexpr int kProjStageLen = 96;
 constexpr int kProjMaxLds = 160 * 1024 - 256;   // dynamic LDS of a workgroup (a few bytes are static)
@@ -1103,9 +1104,9 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
   const int wn = wave % 2, kw = wave / 2, li = lane % 32, lg = lane / 32;
   const int h = blockIdx.x;
   // input row r of this workgroup (rows past the end: M or more)
-  const int sent_base = p.share_shift < 0 ? 0 : (int)blockIdx.y << p.share_shift;
+  const int sent_base = p.share_shift < 0 ? 0 : proj_first_sentence(p.share_shift, (int)blockIdx.y);
   auto row_of = [&](int r) -> int {
-    return proj_row_at(p.share_shift, p.share_nb, p.share_hyps, p.share_per, (int)blockIdx.y, (int)blockIdx.z, r);
+    return proj_row_of(p.share_shift, p.share_nb, p.share_hyps, p.share_per, (int)blockIdx.y, (int)blockIdx.z, r);
   };
   const bool first_rows = blockIdx.y == 0 && blockIdx.z == 0;
   const int K = p.K, M = p.M, S = K / 32, steps = S / 4, N = p.heads * 64;   // steps: sub-steps of a wave, at most PW

@@ -138,7 +138,7 @@ __host__ __device__ __forceinline__ ProjRowPlan proj_row_plan(long long n_proj, 
 // Input row r (0 .. 7) of the workgroup of sentence group `group` and hypothesis chunk `chunk` (shift < 0: of rows number
 // `group`); rows that do not exist: a value of at least M (= hyps * sentences).  The launch has a dimension for either, so
 // that no workgroup divides.
-__host__ __device__ __forceinline__ int proj_row_at(int shift, int sentences, int hyps, int per_wg, int group, int chunk, int r) {
+__host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, int hyps, int per_wg, int group, int chunk, int r) {
   if(shift < 0) return group * per_wg + r;
   const int j = r >> shift, hyp = chunk * per_wg + j;
   if(j >= per_wg || hyp >= hyps) return 0x7fffffff;
@@ -147,13 +147,14 @@ __host__ __device__ __forceinline__ int proj_row_at(int shift, int sentences, in
 // sentence groups of a launch (shift >= 0), and the tile of workgroup block_y of its groups x chunks
 __host__ __device__ __forceinline__ int proj_groups(int shift, int sentences) { return sentences >> shift; }
 __host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, int hyps, int per_wg, int block_y, int r) {
-  if(shift < 0) return proj_row_at(shift, sentences, hyps, per_wg, block_y, 0, r);
+  if(shift < 0) return proj_row_of(shift, sentences, hyps, per_wg, block_y, 0, r);
   const int groups = proj_groups(shift, sentences);
-  return proj_row_at(shift, sentences, hyps, per_wg, block_y % groups, block_y / groups, r);
+  return proj_row_of(shift, sentences, hyps, per_wg, block_y % groups, block_y / groups, r);
 }
-// first sentence of workgroup block_y (shift >= 0)
+// first sentence of a group, and of workgroup block_y (shift >= 0)
+__host__ __device__ __forceinline__ int proj_first_sentence(int shift, int group) { return group << shift; }
 __host__ __device__ __forceinline__ int proj_first_sentence(int shift, int sentences, int block_y) {
-  return (block_y % proj_groups(shift, sentences)) << shift;
+  return proj_first_sentence(shift, block_y % proj_groups(shift, sentences));
 }
 
 }  // namespace marian_hip
