@@ -38,7 +38,7 @@ int marian_hip::launch_absmax_partials(const float* A, unsigned long n, float* p
   size_t g = (n4 + per_block - 1) / per_block;
   if(g < 1) g = 1;
   if(g > (size_t)kMaxPartials) g = kMaxPartials;
-  hipLaunchKernelGGL(absmax_partial_kernel, dim3((unsigned)g), dim3(kQuantThreads), 0, reinterpret_cast<hipStream_t>(stream),
+  MH_LAUNCH(absmax_partial_kernel, dim3((unsigned)g), dim3(kQuantThreads), 0, reinterpret_cast<hipStream_t>(stream),
                      A, n4, partials, (int)g);
   const hipError_t e = hipGetLastError();
   if(e != hipSuccess) return marian_hip::record_hip_error((int)e);
@@ -78,7 +78,7 @@ int launch_stream(const GemmArgs& a, hipStream_t st) {
   const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
   int blocks = (a.n_out + Cfg::kColsPerBlock - 1) / Cfg::kColsPerBlock;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a);
+  MH_LAUNCH(kernel, dim3(blocks), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -103,7 +103,7 @@ int launch_big_split(const GemmArgs& a, hipStream_t st) {
     const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done[1]);
     if(lds_status != MARIAN_HIP_OK) return lds_status;
     a2.absmax_used = tiles_n * tiles_m;
-    hipLaunchKernelGGL(kernel, dim3(tiles_n * tiles_m), dim3(2 * Cfg::kThreads), Cfg::kLdsBytes, st, a2, tiles_n, tiles_m);
+    MH_LAUNCH(kernel, dim3(tiles_n * tiles_m), dim3(2 * Cfg::kThreads), Cfg::kLdsBytes, st, a2, tiles_n, tiles_m);
     MH_HIP(hipGetLastError());
     t_absmax_written = true;
     return MARIAN_HIP_OK;
@@ -111,7 +111,7 @@ int launch_big_split(const GemmArgs& a, hipStream_t st) {
   auto kernel = gemm_mfma32_split_kernel<BM, BN, WM, WN, NSTAGE, NT, false>;
   const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done[0]);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
-  hipLaunchKernelGGL(kernel, dim3(tiles_n * tiles_m), dim3(2 * Cfg::kThreads), Cfg::kLdsBytes, st, a2, tiles_n, tiles_m);
+  MH_LAUNCH(kernel, dim3(tiles_n * tiles_m), dim3(2 * Cfg::kThreads), Cfg::kLdsBytes, st, a2, tiles_n, tiles_m);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -132,7 +132,7 @@ int launch_big(const GemmArgs& a, hipStream_t st) {
       static std::atomic<uint64_t> half_lds_done{0};
       const int half_lds_status = allow_lds(half, Cfg::kLdsBytes, half_lds_done);
       if(half_lds_status != MARIAN_HIP_OK) return half_lds_status;
-      hipLaunchKernelGGL(half, dim3(tiles_n * tiles_m), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a,
+      MH_LAUNCH(half, dim3(tiles_n * tiles_m), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a,
                          tiles_n, tiles_m);
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
@@ -146,7 +146,7 @@ int launch_big(const GemmArgs& a, hipStream_t st) {
       if(lds_status != MARIAN_HIP_OK) return lds_status;
       GemmArgs a2 = a;
       a2.absmax_used = tiles_n * tiles_m;
-      hipLaunchKernelGGL(kernel, dim3(tiles_n * tiles_m), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a2, tiles_n, tiles_m);
+      MH_LAUNCH(kernel, dim3(tiles_n * tiles_m), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a2, tiles_n, tiles_m);
       MH_HIP(hipGetLastError());
       t_absmax_written = true;
       return MARIAN_HIP_OK;
@@ -156,7 +156,7 @@ int launch_big(const GemmArgs& a, hipStream_t st) {
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
-  hipLaunchKernelGGL(kernel, dim3(tiles_n * tiles_m), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a,
+  MH_LAUNCH(kernel, dim3(tiles_n * tiles_m), dim3(Cfg::kThreads), Cfg::kLdsBytes, st, a,
                      tiles_n, tiles_m);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -227,7 +227,7 @@ int launch_big_ragged_as(const GemmArgs& a, const Ragged& r, hipStream_t st) {
   if(lds_status != MARIAN_HIP_OK) return lds_status;
   GemmArgs a2 = a;
   a2.absmax_used = r.workgroups;
-  hipLaunchKernelGGL(kernel, dim3(r.workgroups), dim3(Cfg::kThreads), lds, st, a2, r.plan);
+  MH_LAUNCH(kernel, dim3(r.workgroups), dim3(Cfg::kThreads), lds, st, a2, r.plan);
   MH_HIP(hipGetLastError());
   if(AMAX) t_absmax_written = true;
   return MARIAN_HIP_OK;
@@ -261,7 +261,7 @@ int launch_pair_as(const GemmArgs& a, hipStream_t st) {
   int tiles_m = a.M / PairCfg::BM;
   GemmArgs a2 = a;
   a2.absmax_used = pairs_n * tiles_m;
-  hipLaunchKernelGGL(kernel, dim3(pairs_n * tiles_m), dim3(PairCfg::kThreads), PairCfg::kLdsBytes, st, a2,
+  MH_LAUNCH(kernel, dim3(pairs_n * tiles_m), dim3(PairCfg::kThreads), PairCfg::kLdsBytes, st, a2,
                      pairs_n, tiles_m);
   MH_HIP(hipGetLastError());
   if(AMAX) t_absmax_written = true;
@@ -298,7 +298,7 @@ int launch_pair_ragged_as(const GemmArgs& a, const Ragged& r, hipStream_t st) {
   if(AMAX && workgroups > kAbsmaxSlots) return launch_pair_ragged_as<NT, false>(a, r, st);   // (one slot per workgroup)
   GemmArgs a2 = a;
   a2.absmax_used = workgroups;
-  hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(PairCfg::kThreads), lds, st, a2, plan);
+  MH_LAUNCH(kernel, dim3(workgroups), dim3(PairCfg::kThreads), lds, st, a2, plan);
   MH_HIP(hipGetLastError());
   if(AMAX) t_absmax_written = true;
   return MARIAN_HIP_OK;
@@ -359,8 +359,9 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
       a2.stream_out = 0;
       a2.absmax_out = nullptr;
       a2.blocks_x = groups->table.block0[groups->table.n];
-      hipLaunchKernelGGL(gkernel, dim3(groups->table.block0[groups->table.n], m_tiles), dim3(Cfg::kThreads), lds, st,
-                         a2, f.A, f.aq_out, f.partials, f.n_partials, groups->table, NoNorm());
+      MH_LAUNCH(gkernel, dim3(groups->table.block0[groups->table.n], m_tiles), dim3(Cfg::kThreads), lds, st,
+                         f.A, a2.Bq, a2.Aq, f.partials, a2.M, a2.K, a2.N, a2.n_out, f.n_partials, a2.idx ? 1 : 0, a2, f.aq_out,
+                         groups->table, NoNorm());
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
     }
@@ -374,8 +375,8 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
     if((long long)blocks * m_tiles * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
     else a2.absmax_out = nullptr;
   }
-  hipLaunchKernelGGL(kernel, dim3(blocks, m_tiles), dim3(Cfg::kThreads), lds, st, a2, f.A,
-                     f.aq_out, f.partials, f.n_partials, NoGroups(), NoNorm());
+  MH_LAUNCH(kernel, dim3(blocks, m_tiles), dim3(Cfg::kThreads), lds, st, f.A, a2.Bq, a2.Aq, f.partials, a2.M, a2.K,
+                     a2.N, a2.n_out, f.n_partials, a2.idx ? 1 : 0, a2, f.aq_out, NoGroups(), NoNorm());
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -393,16 +394,16 @@ int launch_normed(const GemmArgs& a, const float* A, const NormInputOf<VECS>& n,
   a2.blocks_x = groups ? groups->block0[groups->n] : (a.n_out + Cfg::kColsPerBlock - 1) / Cfg::kColsPerBlock;
   if(groups) {
     auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, GroupTable, NormInputOf<VECS>>;
-    hipLaunchKernelGGL(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, a2, A, static_cast<int8_t*>(nullptr),
-                       static_cast<const float*>(nullptr), 0, *groups, n);
+    MH_LAUNCH(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, A, a2.Bq, a2.Aq, n.add, a2.M, a2.K, a2.N, a2.n_out, 0, 0, a2,
+                       static_cast<int8_t*>(nullptr), *groups, n);
   } else {
     auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, NoGroups, NormInputOf<VECS>>;
     if(a.absmax_out) {   // one slot per wave
       if((long long)a2.blocks_x * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
       else a2.absmax_out = nullptr;
     }
-    hipLaunchKernelGGL(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, a2, A, static_cast<int8_t*>(nullptr),
-                       static_cast<const float*>(nullptr), 0, NoGroups(), n);
+    MH_LAUNCH(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, A, a2.Bq, a2.Aq, n.add, a2.M, a2.K, a2.N, a2.n_out, 0, 0, a2,
+                       static_cast<int8_t*>(nullptr), NoGroups(), n);
   }
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -434,20 +435,23 @@ int launch_rows(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const Grou
   a2.blocks_x = groups ? groups->table.block0[groups->table.n] : (a.n_out + 31) / 32;
   const RowsTiles tiles = rows_tiles(a2.blocks_x, a2.blocks_y, 4ll * ROWS * a.K, 32ll * a.K);
   const dim3 grid = tiles.shift < 0 ? dim3(a2.blocks_x, a2.blocks_y) : dim3(8, tiles.h, tiles.w);
+  if(tiles.h > 0xFFFF || tiles.w > 0xFFFF) return MARIAN_HIP_ERR_RANGE;   // (plan_tiled's calls are far below)
+  const unsigned tile_block = (unsigned)tiles.h | (unsigned)tiles.w << 16;
+  const int flags = (a.idx ? 1 : 0) + 2 * (tiles.shift + 1);
   if(groups) {
     if(groups->cols != 32) return MARIAN_HIP_ERR_SHAPE;   // (table built for another kernel)
     a2.stream_out = 0;
     a2.absmax_out = nullptr;
-    hipLaunchKernelGGL((gemm_rows_kernel<ROWS, STEPS, GroupTable>), grid, dim3(kRowsThreads), lds, st, a2, f.A, f.aq_out, f.partials,
-                       f.n_partials, tiles, groups->table);
+    MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS, GroupTable>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, a2.M, a2.K,
+                       a2.N, a2.n_out, f.n_partials, tile_block, flags, a2, f.aq_out, groups->table);
   } else {
     a2.stream_out = (long long)a.M * a.n_out * 4 >= (4ll << 20) ? 1 : 0;   // (see launch_stream32)
     if(a.absmax_out) {   // one slot per wave
       if((long long)a2.blocks_x * a2.blocks_y * kRowsWaves <= kAbsmaxSlots) t_absmax_written = true;
       else a2.absmax_out = nullptr;
     }
-    hipLaunchKernelGGL((gemm_rows_kernel<ROWS, STEPS>), grid, dim3(kRowsThreads), lds, st, a2, f.A, f.aq_out, f.partials, f.n_partials,
-                       tiles, NoGroups());
+    MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, a2.M, a2.K, a2.N, a2.n_out,
+                       f.n_partials, tile_block, flags, a2, f.aq_out, NoGroups());
   }
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -789,7 +793,7 @@ int launch_grouped_as(KERNEL kernel, const GemmArgs& a, const GroupTable& g, int
   const int lds_status = allow_lds(kernel, CFG::kLdsBytes, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
   const int tiles_n = g.block0[g.n];
-  hipLaunchKernelGGL(kernel, dim3(tiles_n * tiles_m), dim3(THREADS), CFG::kLdsBytes, st, a, g, tiles_n, tiles_m);
+  MH_LAUNCH(kernel, dim3(tiles_n * tiles_m), dim3(THREADS), CFG::kLdsBytes, st, a, g, tiles_n, tiles_m);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -875,11 +879,11 @@ int absmax_blocks(size_t n4) {
 int quantize_with_partials(const float* A, size_t n, const float* partials, int n_partials, int8_t* Aq, hipStream_t st) {
   if(n >= (1u << 20)) {
     const size_t sets = (n / 64 + 255) / 256, most = 4 * (size_t)compute_units(), blocks = sets < most ? sets : most;
-    hipLaunchKernelGGL(quantize_a_wide_kernel<1024>, dim3((int)blocks), dim3(1024), 0, st, A, (unsigned)(n / 16), partials,
+    MH_LAUNCH(quantize_a_wide_kernel<1024>, dim3((int)blocks), dim3(1024), 0, st, A, (unsigned)(n / 16), partials,
                        n_partials, Aq, (unsigned)blocks);
   } else {
     const size_t blocks = (n / 64 + 63) / 64;
-    hipLaunchKernelGGL(quantize_a_wide_kernel<256>, dim3((int)blocks), dim3(256), 0, st, A, (unsigned)(n / 16), partials,
+    MH_LAUNCH(quantize_a_wide_kernel<256>, dim3((int)blocks), dim3(256), 0, st, A, (unsigned)(n / 16), partials,
                        n_partials, Aq, (unsigned)blocks);
   }
   MH_HIP(hipGetLastError());
@@ -989,7 +993,7 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const size_t n = (size_t)M * (size_t)K;
   if(n <= (size_t)kSingleBlockMaxElems) {
-    hipLaunchKernelGGL(prepare_a_single_block_kernel, dim3(1), dim3(kSingleBlockThreads), 0, st,
+    MH_LAUNCH(prepare_a_single_block_kernel, dim3(1), dim3(kSingleBlockThreads), 0, st,
                        A, (int)(n / 16), Aq);
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
@@ -1017,18 +1021,18 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
       const unsigned nonce = next_nonce();
       const int spins = ov == 702 ? 0 : kOnePassSpinLimit;
       if(sets == 1)
-        hipLaunchKernelGGL(prepare_a_onepass_kernel<1>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
+        MH_LAUNCH(prepare_a_onepass_kernel<1>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
       else if(sets == 2)
-        hipLaunchKernelGGL(prepare_a_onepass_kernel<2>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
+        MH_LAUNCH(prepare_a_onepass_kernel<2>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
       else
-        hipLaunchKernelGGL(prepare_a_onepass_kernel<4>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
+        MH_LAUNCH(prepare_a_onepass_kernel<4>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
     }
   }
   float* partials = reinterpret_cast<float*>(workspace);
   const int g = absmax_blocks(n / 4);
-  hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, A, n / 4,
+  MH_LAUNCH(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, A, n / 4,
                      partials, g);
   MH_HIP(hipGetLastError());
   return quantize_with_partials(A, n, partials, g, Aq, st);
@@ -1045,11 +1049,11 @@ int marian_hip_int8_prepare_b(const float* W, int8_t* Bq, int64_t K, int64_t N, 
   const size_t n = (size_t)K * (size_t)N;
   float* partials = reinterpret_cast<float*>(workspace);
   const int g = absmax_blocks(n / 4);
-  hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, W, n / 4,
+  MH_LAUNCH(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, W, n / 4,
                      partials, g);
   MH_HIP(hipGetLastError());
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)(K / 64));
-  hipLaunchKernelGGL(quantize_b_transpose_kernel, grid, dim3(256), 0, st, W, (int)K, (int)N,
+  MH_LAUNCH(quantize_b_transpose_kernel, grid, dim3(256), 0, st, W, (int)K, (int)N,
                      (const float*)partials, g, Bq);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -1067,7 +1071,7 @@ int marian_hip_int8_prepare_b_quantized_transposed(const int8_t* in, int8_t* out
   const uintptr_t bytes = (uintptr_t)K * (uintptr_t)N + sizeof(float);
   if(a0 < b0 + bytes && b0 < a0 + bytes) return MARIAN_HIP_ERR_ALIAS;
   const size_t chunks = (size_t)K * (size_t)N / 16;
-  hipLaunchKernelGGL(retile_b_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0,
+  MH_LAUNCH(retile_b_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), in, (int)K, (int)N, out);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -1133,7 +1137,7 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
       const size_t n = (size_t)M * (size_t)K;
       float* partials = reinterpret_cast<float*>(workspace);
       const int g = absmax_blocks(n / 4);
-      hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, hst, A, n / 4,
+      MH_LAUNCH(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, hst, A, n / 4,
                          partials, g);
       MH_HIP(hipGetLastError());
       f.partials = partials;
@@ -1155,8 +1159,8 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
 static int absmax_after(const float* out, int64_t M, int64_t n_out, float* absmax_out, hipStream_t st) {
   const size_t n = (size_t)M * (size_t)n_out;
   const int g = absmax_blocks(n / 4);   // n_out % 8 == 0; g <= 1024 partials
-  hipLaunchKernelGGL(zero_floats_kernel, dim3(2), dim3(kQuantThreads), 0, st, absmax_out + g, kAbsmaxSlots - g, 2);
-  hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, out, n / 4, absmax_out, g);
+  MH_LAUNCH(zero_floats_kernel, dim3(2), dim3(kQuantThreads), 0, st, absmax_out + g, kAbsmaxSlots - g, 2);
+  MH_LAUNCH(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, out, n / 4, absmax_out, g);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -1291,7 +1295,7 @@ int marian_hip_int8_affine_f32_grouped(const float* A, int8_t* Aq, int64_t n_gro
       const size_t n = (size_t)M * (size_t)K;
       float* partials = reinterpret_cast<float*>(workspace);
       const int g = absmax_blocks(n / 4);
-      hipLaunchKernelGGL(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, hst, A, n / 4, partials, g);
+      MH_LAUNCH(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, hst, A, n / 4, partials, g);
       MH_HIP(hipGetLastError());
       f.partials = partials;
       f.n_partials = g;

@@ -1086,11 +1086,16 @@ __global__ __launch_bounds__(256) void attention_shared_kernel(const float* __re
 // normalizes all of them, a wave each, while its weights are on their way (a launch of its own for the norm
 // took 3.5 us of GPU and 4 of host time).
 // ANC: the self-attention's cached positions are read through the table of ancestors (attention_kernel's ANC).
+// aux: the abs-max partials, or (NORM) what is added to A.
 // PW: K sub-steps of 32 a wave loads, K / 128 rounded up to 4 or 8.
 // HELD: (self-attention) cached keys and values of up to 4 HELD positions are asked for behind the weights, so that they arrive
 // during quantization and products; 0: longer histories, asked for when the projections are there.
 template <int NPROJ, int R, int SEGS, int PASSES, int PW, int HELD, bool NORM = false, bool ANC = false>
-__global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttentionArgs p) {
+__global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const float* A, const float* aux, const int8_t* Bq0, const int8_t* Bq1,
+                                                                      const int8_t* Bq2, int M, int K, int heads, int n_partials,
+                                                                      ProjAttentionArgs p) {
+  p.A = A; p.Bq[0] = Bq0; p.Bq[1] = Bq1; p.Bq[2] = Bq2;   // (what is needed first comes in registers, see the Makefile)
+  p.M = M; p.K = K; p.heads = heads; p.n_partials = n_partials; p.partials = aux;
   static_assert(HELD == 0 || NPROJ == 3, "the newest key and value come from the projections");
   static_assert(R == 8 || (R == 4 && !(SEGS > 0)), "a wave per row in the attention");
   constexpr bool STAGED = SEGS > 0;
@@ -1109,7 +1114,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
     return proj_row_of(p.share_shift, p.share_nb, p.share_hyps, p.share_per, (int)blockIdx.y, (int)blockIdx.z, r);
   };
   const bool first_rows = blockIdx.y == 0 && blockIdx.z == 0;
-  const int K = p.K, M = p.M, S = K / 32, steps = S / 4, N = p.heads * 64;   // steps: sub-steps of a wave, at most PW
+  const int S = K / 32, steps = S / 4, N = p.heads * 64;   // steps: sub-steps of a wave, at most PW
   int8_t* a_lds = plds;                                   // 32 rows x K bytes, operand order
   int8_t* part_lds = a_lds + 32 * K;                      // NPROJ x 2 x 4 partial tiles of R rows x 128 bytes
   float* proj_lds = reinterpret_cast<float*>(part_lds + NPROJ * 8 * R * 128);   // [NPROJ][R][64]
@@ -1142,7 +1147,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(ProjAttent
   v4f in[4];
   NormRow<PW == 4 ? kNormVecs / 2 : kNormVecs> nr;
   if constexpr(NORM) {
-    nr.load(p.A, p.norm, M, K);
+    nr.load(p.A, aux, p.norm, M, K);
     __builtin_amdgcn_sched_barrier(0);
   } else {
 #pragma unroll
@@ -2096,25 +2101,25 @@ int marian_hip_layer_norm(const float* in, const float* add, const float* gamma,
   if(wave_form) {
     const int blocks = wrap ? (rows + 3 < 4 * (int64_t)kAbsmaxSlots ? (int)((rows + 3) / 4) : kAbsmaxSlots) : (int)rows;
     if(wrap)
-      hipLaunchKernelGGL(layer_norm_wave_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, blocks, (int)rows);
+      MH_LAUNCH(layer_norm_wave_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, blocks, (int)rows);
     else
-      hipLaunchKernelGGL(layer_norm_wave_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, blocks, (int)rows);
+      MH_LAUNCH(layer_norm_wave_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, blocks, (int)rows);
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
   }
   if(wrap) {
-    hipLaunchKernelGGL(zero_words_kernel, dim3(kAbsmaxSlots / 256), dim3(256), 0, st, reinterpret_cast<unsigned*>(absmax_out),
+    MH_LAUNCH(zero_words_kernel, dim3(kAbsmaxSlots / 256), dim3(256), 0, st, reinterpret_cast<unsigned*>(absmax_out),
                        (long long)kAbsmaxSlots, kAbsmaxSlots / 256);
     MH_HIP(hipGetLastError());
   }
   if(vec && cols <= 1024)
-    hipLaunchKernelGGL(layer_norm_kernel<1>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
+    MH_LAUNCH(layer_norm_kernel<1>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   else if(vec && cols <= 4096)
-    hipLaunchKernelGGL(layer_norm_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
+    MH_LAUNCH(layer_norm_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   else if(vec && cols <= 8192)
-    hipLaunchKernelGGL(layer_norm_kernel<8>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
+    MH_LAUNCH(layer_norm_kernel<8>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   else
-    hipLaunchKernelGGL(layer_norm_kernel<0>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
+    MH_LAUNCH(layer_norm_kernel<0>, dim3((unsigned)rows), dim3(256), 0, st, in, add, gamma, gs, beta, bs, out, (int)cols, eps, absmax_out, wrap, (int)rows);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2137,10 +2142,10 @@ int marian_hip_embed(const float* E, const uint32_t* ids, int64_t rows, int64_t 
   const bool vec = dimEmb % 4 == 0 && aligned16(E) && aligned16(out) && (!signal || aligned16(signal));
   const unsigned rps = signal ? (unsigned)rows_per_signal : 1u, ns = signal ? (unsigned)n_signals : 1u;
   if(vec)
-    hipLaunchKernelGGL(embed_kernel<true>, dim3((unsigned)rows, (unsigned)chunks), dim3(256), 0, st, E, ids,
+    MH_LAUNCH(embed_kernel<true>, dim3((unsigned)rows, (unsigned)chunks), dim3(256), 0, st, E, ids,
                        (unsigned)vocab, (int)dimEmb, scale, signal, rps, ns, out, absmax_out, (unsigned)rows, (unsigned)chunks);
   else
-    hipLaunchKernelGGL(embed_kernel<false>, dim3((unsigned)rows, (unsigned)chunks), dim3(256), 0, st, E, ids,
+    MH_LAUNCH(embed_kernel<false>, dim3((unsigned)rows, (unsigned)chunks), dim3(256), 0, st, E, ids,
                        (unsigned)vocab, (int)dimEmb, scale, signal, rps, ns, out, absmax_out, (unsigned)rows, (unsigned)chunks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -2166,10 +2171,10 @@ int marian_hip_select_state(const float* state, const uint32_t* ids, int64_t row
   const bool vec = seg_len % 4 == 0 && seg_capacity % 4 == 0 && aligned16(state) && aligned16(out);
   const dim3 grid((unsigned)(rows * segments), (unsigned)chunks);
   if(vec)
-    hipLaunchKernelGGL(select_state_kernel<true>, grid, dim3(256), 0, st, state, ids, (unsigned)entries, (unsigned)segments,
+    MH_LAUNCH(select_state_kernel<true>, grid, dim3(256), 0, st, state, ids, (unsigned)entries, (unsigned)segments,
                        (long long)seg_capacity, (int)seg_len, out);
   else
-    hipLaunchKernelGGL(select_state_kernel<false>, grid, dim3(256), 0, st, state, ids, (unsigned)entries, (unsigned)segments,
+    MH_LAUNCH(select_state_kernel<false>, grid, dim3(256), 0, st, state, ids, (unsigned)entries, (unsigned)segments,
                        (long long)seg_capacity, (int)seg_len, out);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -2209,20 +2214,20 @@ static int softmax_common(const float* in, const float* mask, int64_t n_masks, i
   const bool wide_ok = cols % 4 == 0 && cols <= 65536 && aligned16(in) && aligned16(out) && (!mask || aligned16(mask));
   if(cols <= 2048 && !(wide_ok && cols > 256)) {
     const unsigned blocks = (unsigned)((rows + 3) / 4);
-    if(log) hipLaunchKernelGGL((softmax_kernel<64, true>), dim3(blocks), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
-    else hipLaunchKernelGGL((softmax_kernel<64, false>), dim3(blocks), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
+    if(log) MH_LAUNCH((softmax_kernel<64, true>), dim3(blocks), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
+    else MH_LAUNCH((softmax_kernel<64, false>), dim3(blocks), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
   } else if(wide_ok && cols <= 4096) {
-    if(log) hipLaunchKernelGGL((softmax_wide_kernel<true, 256, 4>), dim3((unsigned)rows), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
-    else hipLaunchKernelGGL((softmax_wide_kernel<false, 256, 4>), dim3((unsigned)rows), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
+    if(log) MH_LAUNCH((softmax_wide_kernel<true, 256, 4>), dim3((unsigned)rows), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
+    else MH_LAUNCH((softmax_wide_kernel<false, 256, 4>), dim3((unsigned)rows), dim3(256), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
   } else if(wide_ok && cols <= 32768) {
-    if(log) hipLaunchKernelGGL((softmax_wide_kernel<true, 1024, 8>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
-    else hipLaunchKernelGGL((softmax_wide_kernel<false, 1024, 8>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
+    if(log) MH_LAUNCH((softmax_wide_kernel<true, 1024, 8>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
+    else MH_LAUNCH((softmax_wide_kernel<false, 1024, 8>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
   } else if(wide_ok) {
-    if(log) hipLaunchKernelGGL((softmax_wide_kernel<true, 1024, 16>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
-    else hipLaunchKernelGGL((softmax_wide_kernel<false, 1024, 16>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
+    if(log) MH_LAUNCH((softmax_wide_kernel<true, 1024, 16>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
+    else MH_LAUNCH((softmax_wide_kernel<false, 1024, 16>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (int)cols);
   } else {
-    if(log) hipLaunchKernelGGL((softmax_kernel<1024, true>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
-    else hipLaunchKernelGGL((softmax_kernel<1024, false>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
+    if(log) MH_LAUNCH((softmax_kernel<1024, true>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
+    else MH_LAUNCH((softmax_kernel<1024, false>), dim3((unsigned)rows), dim3(1024), 0, st, in, mask, (long long)n_masks, (long long)rows_per_mask, out, (long long)rows, (int)cols);
   }
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -2250,8 +2255,8 @@ int marian_hip_transpose0213(const float* in, float* out, int64_t d0, int64_t d1
   const long long total = d0 * d1 * d2 * (vec ? d3 / 4 : d3);
   long long blocks = (total + 255) / 256;
   if(blocks > 8192) blocks = 8192;
-  if(vec) hipLaunchKernelGGL(transpose0213_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)(d3 / 4), (int)blocks);
-  else hipLaunchKernelGGL(transpose0213_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)d3, (int)blocks);
+  if(vec) MH_LAUNCH(transpose0213_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)(d3 / 4), (int)blocks);
+  else MH_LAUNCH(transpose0213_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, st, in, out, total, (int)d1, (int)d2, (int)d3, (int)blocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2273,15 +2278,15 @@ int marian_hip_bdot_legacy(const float* A, const float* B, float* C, int64_t bat
   if(tile_ok) {
     const dim3 grid((unsigned)((n + 63) / 64), (unsigned)((m + 63) / 64), (unsigned)batchC);
     if(transB)
-      hipLaunchKernelGGL(bdot_tile_kernel<true>, grid, dim3(256), 0, st, A, B, C, (long long)batchA,
+      MH_LAUNCH(bdot_tile_kernel<true>, grid, dim3(256), 0, st, A, B, C, (long long)batchA,
                          (long long)batchB, (int)m, (int)n, (int)k, scalar);
     else
-      hipLaunchKernelGGL(bdot_tile_kernel<false>, grid, dim3(256), 0, st, A, B, C, (long long)batchA,
+      MH_LAUNCH(bdot_tile_kernel<false>, grid, dim3(256), 0, st, A, B, C, (long long)batchA,
                          (long long)batchB, (int)m, (int)n, (int)k, scalar);
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
   }
-  hipLaunchKernelGGL(bdot_kernel, dim3((unsigned)((rows_total + 3) / 4)), dim3(256), 0, st, A, B, C,
+  MH_LAUNCH(bdot_kernel, dim3((unsigned)((rows_total + 3) / 4)), dim3(256), 0, st, A, B, C,
                      (long long)batchA, (long long)batchB, rows_total, (int)m, (int)n, (int)k,
                      transA ? 1 : 0, transB ? 1 : 0, scalar);
   MH_HIP(hipGetLastError());
@@ -2333,7 +2338,7 @@ int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const fl
     const int lds_status = allow_lds(attention_kernel<false, true>, 72 * 1024, lds_done);
     if(lds_status != MARIAN_HIP_OK) return lds_status;
     const size_t lds = (size_t)4 * (size_t)(((len + 3) & ~(int64_t)3) + 256) * sizeof(float);
-    hipLaunchKernelGGL((attention_kernel<false, true>), dim3((unsigned)((batchQ * m + 3) / 4)), dim3(256), lds, hst, q, const_cast<float*>(k),
+    MH_LAUNCH((attention_kernel<false, true>), dim3((unsigned)((batchQ * m + 3) / 4)), dim3(256), lds, hst, q, const_cast<float*>(k),
                        const_cast<float*>(v), nullptr, nullptr, mask, (unsigned)n_masks, (unsigned)rows_per_mask, out, (unsigned)(batchQ * m),
                        (unsigned)batchKV, (int)m, (int)len, (int)len, (int)dk, scale, absmax_out, nullptr, (unsigned)heads, hs);
     MH_HIP(hipGetLastError());
@@ -2352,7 +2357,7 @@ int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const fl
                       (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)row_blocks, (int)groups, scale,
                       mask && rows_per_mask % m == 0};
   const dim3 grid((unsigned)(batchQ * groups));
-#define MH_ROWS(NB) hipLaunchKernelGGL(attention_rows_kernel<NB>, grid, dim3(256), 0, hst, a)
+#define MH_ROWS(NB) MH_LAUNCH(attention_rows_kernel<NB>, grid, dim3(256), 0, hst, a)
   if(len <= 64) MH_ROWS(1);
   else if(len <= 128) MH_ROWS(2);
   else if(len <= 192) MH_ROWS(3);
@@ -2415,7 +2420,7 @@ int marian_hip_ancestors_advance(const uint32_t* prev, const uint32_t* parents, 
   const uintptr_t bytes = (uintptr_t)(n_hyp * kv_capacity) * 4;
   if(a0 < b0 + bytes && b0 < a0 + bytes) return MARIAN_HIP_ERR_ALIAS;   // (a row may be read after the row of the same number has been written)
   const int64_t n = n_hyp * (len_prev + 1);
-  hipLaunchKernelGGL(ancestors_advance_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+  MH_LAUNCH(ancestors_advance_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), prev, parents, (unsigned)n_hyp, (unsigned)kv_capacity,
                      (unsigned)len_prev, next);
   MH_HIP(hipGetLastError());
@@ -2468,7 +2473,7 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
     const dim3 grid((unsigned)batchKV, (unsigned)((hyps + 3) / 4));
     const size_t slds = (size_t)2 * (size_t)len * 256 + lds;
 #define MH_SATT(PASSES) \
-    hipLaunchKernelGGL(attention_shared_kernel<PASSES>, grid, dim3(256), slds, st, q, k, v, mask, (unsigned)n_masks, \
+    MH_LAUNCH(attention_shared_kernel<PASSES>, grid, dim3(256), slds, st, q, k, v, mask, (unsigned)n_masks, \
                        (unsigned)rows_per_mask, out, (unsigned)rows_total, (unsigned)batchKV, (int)len, (int)kv_capacity, \
                        scale, absmax_out)
     if(len <= 32) MH_SATT(2);
@@ -2479,12 +2484,12 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
     return MARIAN_HIP_OK;
   }
   if(ancestors)
-    hipLaunchKernelGGL((attention_kernel<true, false>), dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
+    MH_LAUNCH((attention_kernel<true, false>), dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
                        k_new, v_new, mask, (unsigned)n_masks, (unsigned)rows_per_mask, out, (unsigned)rows_total,
                        (unsigned)batchKV, (int)m, (int)len, (int)kv_capacity, (int)dk, scale, absmax_out, ancestors,
                        (unsigned)heads, AttentionStrides());
   else
-    hipLaunchKernelGGL((attention_kernel<false, false>), dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
+    MH_LAUNCH((attention_kernel<false, false>), dim3((unsigned)((rows_total + 3) / 4)), dim3(256), lds, st, q, k, v,
                        k_new, v_new, mask, (unsigned)n_masks, (unsigned)rows_per_mask, out, (unsigned)rows_total,
                        (unsigned)batchKV, (int)m, (int)len, (int)kv_capacity, (int)dk, scale, absmax_out, ancestors,
                        1u, AttentionStrides());
@@ -2499,7 +2504,8 @@ static int launch_proj(const ProjAttentionArgs& p, dim3 grid, size_t lds, hipStr
   static std::atomic<uint64_t> lds_done{0};
   const int lst = allow_lds(kernel, SEGS > 0 ? kProjMaxLds : 96 * 1024, lds_done);
   if(lst != MARIAN_HIP_OK) return lst;
-  hipLaunchKernelGGL(kernel, grid, dim3(kProjThreads), lds, st, p);
+  MH_LAUNCH(kernel, grid, dim3(kProjThreads), lds, st, p.A, NORM ? p.norm.add : p.partials, p.Bq[0], p.Bq[1], p.Bq[2], p.M, p.K, p.heads,
+                     p.n_partials, p);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2676,8 +2682,8 @@ int marian_hip_int8_proj_attention_normed(const float* A, const marian_hip_norm_
 // Rows of up to kNbestWaveCols values: a wave each; longer ones: 1024 threads each.
 static int nbest_rows(const float* scores, int64_t rows, int64_t rowLen, int64_t N, const NbestOut& out, void* stream) {
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-#define MH_NBW(VPT) hipLaunchKernelGGL(nbest_wave_kernel<VPT>, dim3((unsigned)rows), dim3(64), 0, st, scores, (int)rowLen, (int)N, out)
-#define MH_NBK(KEEP) hipLaunchKernelGGL(nbest_kernel<KEEP>, dim3((unsigned)rows), dim3(1024), 0, st, scores, (long long)rowLen, (int)N, out)
+#define MH_NBW(VPT) MH_LAUNCH(nbest_wave_kernel<VPT>, dim3((unsigned)rows), dim3(64), 0, st, scores, (int)rowLen, (int)N, out)
+#define MH_NBK(KEEP) MH_LAUNCH(nbest_kernel<KEEP>, dim3((unsigned)rows), dim3(1024), 0, st, scores, (long long)rowLen, (int)N, out)
   if(rowLen <= kNbestWaveCols / 2) MH_NBW(kNbestWaveCols / 128);
   else if(rowLen <= kNbestWaveCols) MH_NBW(kNbestWaveCols / 64);
   else if(N <= 4) MH_NBK(4);
@@ -2724,7 +2730,7 @@ int marian_hip_fill(void* begin, int64_t count, int elem_bytes, uint64_t pattern
   long long blocks = (vecs + 255) / 256;
   if(blocks < 1) blocks = 1;
   if(blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+  MH_LAUNCH(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
                      reinterpret_cast<unsigned char*>(begin), bytes, head, vecs, elem_bytes,
                      (unsigned long long)pattern, (int)blocks);
   MH_HIP(hipGetLastError());
@@ -2745,7 +2751,7 @@ int marian_hip_nbest_beams_workspace_init(void* workspace, size_t workspace_byte
   const long long words = (long long)(workspace_bytes / 4);
   const unsigned blocks = (unsigned)((words + 255) / 256 < 1024 ? (words + 255) / 256 : 1024);
   if(words > 0)
-    hipLaunchKernelGGL(zero_words_kernel, dim3(blocks), dim3(256), 0, st, reinterpret_cast<unsigned*>(workspace), words, (int)blocks);
+    MH_LAUNCH(zero_words_kernel, dim3(blocks), dim3(256), 0, st, reinterpret_cast<unsigned*>(workspace), words, (int)blocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -2773,7 +2779,7 @@ int marian_hip_nbest_beams(const float* scores, int64_t beam, int64_t dimBatch, 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)plan.parts, (unsigned)dimBatch);
 #define MH_NBP(KEEP, FENCED)                                                                                   \
-  hipLaunchKernelGGL((nbest_part_kernel<KEEP, FENCED>), grid, dim3(1024), 0, st, scores, (long long)dimBatch, \
+  MH_LAUNCH((nbest_part_kernel<KEEP, FENCED>), grid, dim3(1024), 0, st, scores, (long long)dimBatch, \
                      (long long)vocab, plan.perSeg, plan.sliceLen, (int)N, (int)plan.parts, candVal, candIdx, counters,         \
                      outScores, outKeys)
   if(nbest_fenced()) {
@@ -2814,7 +2820,7 @@ int marian_hip_logsoftmax_nbest_beams(const float* logits, const float* rowAdd, 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)beam, (unsigned)dimBatch);
 #define MH_LSNB(VPT, KEEP, FENCED)                                                                                   \
-  hipLaunchKernelGGL((logsoftmax_nbest_kernel<VPT, KEEP, FENCED>), grid, dim3(1024), 0, st, logits, rowAdd, logProbs, \
+  MH_LAUNCH((logsoftmax_nbest_kernel<VPT, KEEP, FENCED>), grid, dim3(1024), 0, st, logits, rowAdd, logProbs, \
                      (long long)dimBatch, (int)vocab, (int)N, (int)beam, candVal, candIdx, counters, outScores, outKeys)
   if(nbest_fenced()) {
 #ifdef MARIAN_HIP_TUNING

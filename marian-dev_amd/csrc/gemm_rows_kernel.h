@@ -45,10 +45,13 @@ __host__ __device__ __forceinline__ RowsTile rows_tile(RowsTiles t, int x, int y
 // pairs of a wave that are on their way at a time, as registers allow
 constexpr int rows_depth(int rows) { return rows == 32 ? 2 : 4; }
 
-// STEPS: pairs that the first waves take, ceil(K / 512); the others take one fewer.
+// STEPS: pairs that the first waves take, ceil(K / 512); the others take one fewer.  tile_block: h | w << 16; flags: 1 with a shortlist,
+// plus 2 (shift + 1).  (The fields of args that are arguments of their own as well are those.)
 template <int ROWS, int STEPS, typename GROUPS = NoGroups>
-__global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(GemmArgs args, const float* A, int8_t* aq_out, const float* partials,
-                                                                 int n_partials, RowsTiles tiles, GROUPS groups) {
+__global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A, const int8_t* Bq, const float* partials, int M, int K, int N,
+                                                                 int n_out, int n_partials, unsigned tile_block, int flags, GemmArgs args,
+                                                                 int8_t* aq_out, GROUPS groups) {
+  args.Bq = Bq; args.M = M; args.K = K; args.N = N; args.n_out = n_out;   // (what is needed first comes in registers, see the Makefile)
   constexpr bool GROUPED = std::is_same<GROUPS, GroupTable>::value;
   constexpr int CHUNK = rows_chunk_bytes<ROWS>(), LOADS = ROWS / 4;   // of four rows a load
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
@@ -56,11 +59,11 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(GemmArgs args, 
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int li = lane % 32, lg = lane / 32;
-  const RowsTile tile = rows_tile(tiles, blockIdx.x, blockIdx.y, blockIdx.z);
+  const RowsTile tile = rows_tile(RowsTiles{(flags >> 1) - 1, (int)(tile_block & 0xFFFFu), (int)(tile_block >> 16)}, blockIdx.x, blockIdx.y, blockIdx.z);
   const bool first_column = tile.bx == 0;
   int bx = tile.bx;
   if constexpr(GROUPED) bx = groups.select(args, bx);
-  const int K = args.K, M = args.M, m_base = tile.by * ROWS;
+  const int m_base = tile.by * ROWS;
 
   // The order of the loads: see gemm_stream32_kernel (ids first, then what is needed first, all unconditional).
   const int n0 = bx * 32;
@@ -69,7 +72,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(GemmArgs args, 
   uint32_t bias_at[4];
 #pragma unroll
   for(int e = 0; e < 4; ++e) bias_at[e] = (uint32_t)(bias_n + e);
-  if(args.idx) {
+  if(flags & 1) {   // through a shortlist
     if(args.bias) {
 #pragma unroll
       for(int e = 0; e < 4; ++e) bias_at[e] = args.idx[bias_at[e]];

@@ -69,7 +69,8 @@ struct Stream32Cfg {
 struct NoGroups {};
 
 // Dynamic LDS: one chunk (kStageBytes), for kFusedAll all of K (32 * MT32 * K bytes) if that is
-// more; at least kReduceBytes.  partials: n_partials (1..2048) abs-max values (kFusedTiled only).
+// more; at least kReduceBytes.  aux: n_partials (1..2048) abs-max values (kFusedTiled), what is added to A (kFusedNorm).  The fields of args
+// that are arguments of their own as well are those; shortlist: whether there is one.
 // NG (kFusedAll): 16-value groups per thread that are compiled in, 2 or 4; all but the last two are
 // complete (the launcher picks NG = 2 for M * K <= 16384), so their loads, abs-max and
 // quantization carry no range checks.
@@ -77,11 +78,12 @@ struct NoGroups {};
 // workgroup and twice the workgroups, for calls that would otherwise leave most CUs idle.  With ROWS < M the kFusedAll form
 // still takes the abs-max over all of A in every workgroup and quantizes only its own rows.
 template <int MT32, int WN, int KW, int PW, int MODE, int NG = 4, int ROWS = 32 * MT32, typename GROUPS = NoGroups, typename NORMED = NoNorm>
-__global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs args,
-                                                                        const float* A,
-                                                                        int8_t* aq_out,
-                                                                        const float* partials,
-                                                                        int n_partials, GROUPS groups, NORMED norm) {
+__global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const float* A, const int8_t* Bq, const int8_t* Aq,
+                                                                        const float* aux, int M, int K, int N, int n_out,
+                                                                        int n_partials, int shortlist, GemmArgs args,
+                                                                        int8_t* aq_out, GROUPS groups, NORMED norm) {
+  args.Bq = Bq; args.Aq = Aq; args.M = M; args.K = K; args.N = N; args.n_out = n_out;   // (what is needed first comes in registers, see the Makefile)
+  const float* const partials = aux;
   using Cfg = Stream32Cfg<MT32, WN, KW, PW>;
   constexpr bool GROUPED = std::is_same<GROUPS, GroupTable>::value;
   constexpr bool NORM = MODE == kFusedNorm;
@@ -110,7 +112,6 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   const int wave = tid / kWave, lane = tid % kWave;
   const int wn = wave % WN, kw = wave / WN;
   const int li = lane % 32, lg = lane / 32;
-  const int K = args.K, M = args.M;
   const int S = K / 32;                                   // K sub-steps
   const int n_chunks = (S + Cfg::CS - 1) / Cfg::CS;
   constexpr int R = ROWS;   // activation rows of this workgroup
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   uint32_t bias_at[4];
 #pragma unroll
   for(int e = 0; e < 4; ++e) bias_at[e] = (uint32_t)(bias_n + e);
-  if(args.idx) {
+  if(shortlist) {
     if(args.bias) {
 #pragma unroll
       for(int e = 0; e < 4; ++e) bias_at[e] = args.idx[bias_at[e]];
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(GemmArgs
   // g / (K/16), 16-byte chunk g % (K/16).
   v4f vals[FUSED && !NORM ? kFusedGroups : 1][4];
   NormRow<NORMED::kVecs> nrow;
-  if constexpr(NORM) nrow.load(A, norm, M, K);
+  if constexpr(NORM) nrow.load(A, aux, norm, M, K);
   const int n16 = M * K / 16;   // groups; a multiple of four
   const int quad = tid / 4, qlane = tid % 4;
   const int wave_s = __builtin_amdgcn_readfirstlane(wave);   // (a scalar for the compiler)

@@ -264,7 +264,9 @@ constexpr int kStream16Waves = 8;
 template <int MT, int NT>
 constexpr int stream16_lds() { return kStream16Waves * 1024 * (2 * (MT + NT) > MT * NT ? 2 * (MT + NT) : MT * NT); }
 template <typename AT, int MT, int NT, int D, bool DUMP>
-__global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(Gemm16Args g, int tiles_n, int tiles_m) {
+__global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(const void* A, const int16_t* Bq, const float* bias_in, int M, int K, int N,
+                                                                              int tiles_n, int tiles_m, Gemm16Args g) {
+  g.A = A; g.Bq = Bq; g.bias = bias_in; g.M = M; g.K = K; g.N = N;   // (what is needed first comes in registers, see the Makefile)
   constexpr int KW = kStream16Waves, TILES = MT * NT, kWaveBytes = stream16_lds<MT, NT>() / KW;
   extern __shared__ __attribute__((aligned(16))) int8_t lds16[];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -424,7 +426,9 @@ constexpr int tile16_sums() { return 4 * BM * BN > 4 * (BM + BN) * kPitch16 ? 4 
 template <int BM, int BN>
 constexpr int tile16_lds() { return tile16_sums<BM, BN>() + 4 * (BM + BN); }
 template <typename AT, int BM, int BN, int WM, int WN, bool DUMP>
-__global__ __launch_bounds__(kTile16Threads) void gemm16_tile_kernel(Gemm16Args g, int tiles_n, int tiles_m) {
+__global__ __launch_bounds__(kTile16Threads) void gemm16_tile_kernel(const void* A, const int16_t* Bq, const float* bias_in, int M, int K, int N,
+                                                                     int tiles_n, int tiles_m, Gemm16Args g) {
+  g.A = A; g.Bq = Bq; g.bias = bias_in; g.M = M; g.K = K; g.N = N;   // (see gemm16_stream_kernel)
   static_assert(WM * WN == 8, "eight waves");
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16, D = kTile16Depth;   // D: blocks of K on their way
   extern __shared__ __attribute__((aligned(16))) int8_t lds16[];
@@ -583,8 +587,8 @@ int launch_stream16(const Gemm16Args& g, hipStream_t st) {
   const int tiles_n = (g.N + 16 * NT - 1) / (16 * NT), tiles_m = (g.M + 16 * MT - 1) / (16 * MT);
   constexpr int lds = stream16_lds<MT, NT>();
   static_assert(lds <= 65536, "no attribute needed");
-  hipLaunchKernelGGL((gemm16_stream_kernel<AT, MT, NT, 2, DUMP>), dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(64 * kStream16Waves), lds, st,
-                     g, tiles_n, tiles_m);
+  MH_LAUNCH((gemm16_stream_kernel<AT, MT, NT, 2, DUMP>), dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(64 * kStream16Waves), lds, st,
+                     g.A, g.Bq, g.bias, g.M, g.K, g.N, tiles_n, tiles_m, g);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -597,7 +601,8 @@ int launch_tile16(const Gemm16Args& g, hipStream_t st) {
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, lds, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(kTile16Threads), lds, st, g, tiles_n, tiles_m);
+  MH_LAUNCH(kernel, dim3((unsigned)tiles_n * (unsigned)tiles_m), dim3(kTile16Threads), lds, st, g.A, g.Bq, g.bias, g.M, g.K, g.N,
+                     tiles_n, tiles_m, g);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -673,7 +678,7 @@ int marian_hip_int16_prepare_a(const float* A, int16_t* Aq, int64_t M, int64_t K
   const size_t n8 = (size_t)M * (size_t)K / 8;
   size_t blocks = (n8 + 255) / 256;
   if(blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(quantize16_a_kernel, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), A, n8, Aq, (int)blocks);
+  MH_LAUNCH(quantize16_a_kernel, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), A, n8, Aq, (int)blocks);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -685,7 +690,7 @@ int marian_hip_int16_prepare_b(const float* W, int16_t* Bq, int64_t K, int64_t N
   if(!aligned(W, 4) || !aligned(Bq, 16)) return MARIAN_HIP_ERR_ALIGN;
   const dim3 grid((unsigned)((N + 63) / 64), (unsigned)(K / 32));
   if(grid.y > 65535) return MARIAN_HIP_ERR_RANGE;
-  hipLaunchKernelGGL(quantize16_b_transpose_kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), W, (int)K, (int)N, Bq);
+  MH_LAUNCH(quantize16_b_transpose_kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), W, (int)K, (int)N, Bq);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }

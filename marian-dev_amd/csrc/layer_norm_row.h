@@ -92,14 +92,14 @@ template <int VECS>
 struct NormRow {
   v4f v[VECS], t[VECS], gm[VECS], bt[VECS];
   // Wave w loads row w (rows past M: a copy of the last one).  All loads unconditional, so that waits count them exactly.
-  __device__ __forceinline__ void load(const float* A, const NormInput& n, int M, int K) {
+  __device__ __forceinline__ void load(const float* A, const float* add, const NormInput& n, int M, int K) {
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, cols4 = K / 4;
     const size_t row = (size_t)min(wave, M - 1) * K;
 #pragma unroll
     for(int j = 0; j < VECS; ++j) {
       const int i = min(j * kWave + lane, cols4 - 1);
       v[j] = reinterpret_cast<const v4f*>(A + row)[i];
-      t[j] = reinterpret_cast<const v4f*>(n.add + row)[i];
+      t[j] = reinterpret_cast<const v4f*>(add + row)[i];
     }
 #pragma unroll
     for(int j = 0; j < VECS; ++j) {
