@@ -23,6 +23,7 @@
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <utility>
@@ -119,12 +120,14 @@ inline bool truth(PyObject* o) {
   return v != 0;
 }
 
+// Calls f without the interpreter lock; a status is raised as an error of `where`, or of what f left in *which.
 template <typename F>
-inline void call(const char* where, F f) {
+inline void call(const char* where, F f, const char** which = nullptr) {
   PyThreadState* s = PyEval_SaveThread();
   const int status = f();
   PyEval_RestoreThread(s);
   if(status != MARIAN_HIP_OK) {
+    if(which && **which) where = *which;
     Ref r(PyObject_CallFunction(raise_status, "is", status, where));
     if(!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, where);
     throw PyFailed();
@@ -844,6 +847,208 @@ PyObject* py_proj_attention_ancestors(PyObject*, PyObject* const* args, Py_ssize
   MH_END
 }
 
+// ---- the layers of a decoding step ---------------------------------------------------------------
+// The calls of a decoding step's layers, one after the other, as decoder_step.py makes them one by one: the same entry
+// points of the library on the same values.  Made from Python, each cost 5.5 us of host time (arguments, three tensors, two
+// objects, the launch), more than the kernels of a small step take; here everything is looked at first, what lies between the
+// layers is one allocation, and the launches follow each other without the interpreter lock.
+struct DecoderMatrix {
+  Quantized b;
+  at::Tensor bias;
+  const int8_t* weights() const { return static_cast<const int8_t*>(b.t->const_data_ptr()); }
+  const float* shift() const { return bias.defined() ? static_cast<const float*>(bias.const_data_ptr()) : nullptr; }
+};
+struct DecoderNorm {
+  at::Tensor gamma, beta;
+};
+struct DecoderLayer {
+  DecoderMatrix qkv[3], o, cq, co, w1, w2;
+  DecoderNorm ln1, ln2, ln3;
+  at::Tensor k, v, kc, vc;   // caches of the target positions, and the source's
+};
+
+// Whether a layer's vector can be read as the kernels do: n values on device d, from an address of whole vectors.
+inline bool decoder_vector(const at::Tensor* t, int64_t n, c10::Device d) {
+  return t && t->numel() == n && t->device() == d && reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16 == 0;
+}
+// A (bQuant, bias or None) with K rows and N columns (0: any number), the bias of one value a column.
+bool decoder_matrix(PyObject* w, int64_t K, int64_t N, c10::Device d, DecoderMatrix& m) {
+  if(!w || !PyTuple_Check(w) || PyTuple_GET_SIZE(w) != 2) return false;
+  const at::Tensor* bias;
+  if(!matrix(PyTuple_GET_ITEM(w, 0), m.b, true) || m.b.width != 1 || m.b.rows != K || (N && m.b.cols != N) ||
+     m.b.t->device() != d || !f32c_or_none(PyTuple_GET_ITEM(w, 1), &bias) || (bias && !decoder_vector(bias, m.b.cols, d)))
+    return false;
+  if(bias) m.bias = *bias;
+  return true;
+}
+bool decoder_norm(PyObject* ln, int64_t n, c10::Device d, DecoderNorm& out) {
+  if(!ln || !PyTuple_Check(ln) || PyTuple_GET_SIZE(ln) != 2) return false;
+  const at::Tensor *gamma = f32c(PyTuple_GET_ITEM(ln, 0)), *beta = f32c(PyTuple_GET_ITEM(ln, 1));
+  if(!decoder_vector(gamma, n, d) || !decoder_vector(beta, n, d)) return false;
+  out.gamma = *gamma;
+  out.beta = *beta;
+  return true;
+}
+// A cache of `entries` entries of [.., 64] (all of one size) at place i of a list.
+bool decoder_cache(PyObject* list, Py_ssize_t i, int64_t entries, c10::Device d, int64_t& capacity, at::Tensor& out) {
+  const at::Tensor* t = f32c(PyList_GET_ITEM(list, i));
+  if(!t || t->device() != d || t->dim() != 3 || t->size(2) != 64 || (entries && t->size(0) != entries) || (capacity && t->size(1) != capacity)) return false;
+  capacity = t->size(1);
+  out = *t;
+  return true;
+}
+
+// decoder_layers(x, absmax of x, layers, Kself, Vself, Kenc, Venc, mask, ancestors or None, heads, kvLen, eps, (output matrix, bias))
+//   -> scores [M, vocabulary]; layers: dicts of Wq, Wk, Wv, Wo, cWq, cWo, W1, W2 (bQuant, bias) and ln1, ln2, ln3 (gamma, beta)
+PyObject* py_decoder_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(13, "decoder_layers");
+  const at::Tensor *x = f32c(args[0]), *mask, *anc = nullptr;
+  const float* amax = nullptr;
+  for(int i : {2, 3, 4, 5, 6})
+    if(!PyList_Check(args[i]) || PyList_GET_SIZE(args[i]) != PyList_GET_SIZE(args[2])) Py_RETURN_NONE;
+  const Py_ssize_t n = PyList_GET_SIZE(args[2]);
+  if(!x || x->dim() != 2 || n < 1 || !absmax_in(args[1], &amax) || !amax || !f32c_or_none(args[7], &mask)) Py_RETURN_NONE;
+  const int64_t M = x->size(0), d = x->size(1), heads = whole(args[9]), len = whole(args[10]);
+  const float eps = (float)number(args[11]);
+  if(M < 1 || d % 128 != 0 || d > 1024 || d != heads * 64 || M * heads > MARIAN_HIP_ABSMAX_SLOTS || len < 1 || len > 512 ||
+     reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16 != 0)
+    Py_RETURN_NONE;
+  if(!none(args[8])) {
+    anc = tensor(args[8]);
+    if(M > 256 || !anc || !ids_type(anc->scalar_type()) || anc->device() != x->device() || !anc->is_contiguous() || anc->dim() != 2 || anc->size(0) != M)
+      Py_RETURN_NONE;
+  }
+  const c10::Device dev = x->device();
+  if(mask && mask->device() != dev) Py_RETURN_NONE;
+  const bool few = M <= MARIAN_HIP_NORM_MAX_ROWS;   // the layer norms need no launches of their own
+  int64_t cap = anc ? anc->size(1) : 0, source = 0, widest = d;
+  std::vector<DecoderLayer> layers((size_t)n);
+  for(Py_ssize_t i = 0; i < n; ++i) {
+    DecoderLayer& l = layers[(size_t)i];
+    PyObject* dict = PyList_GET_ITEM(args[2], i);
+    if(!PyDict_Check(dict)) Py_RETURN_NONE;
+    auto item = [&](const char* name) { return PyDict_GetItemString(dict, name); };
+    int64_t source_cap = source;
+    if(!decoder_matrix(item("Wq"), d, d, dev, l.qkv[0]) || !decoder_matrix(item("Wk"), d, d, dev, l.qkv[1]) || !decoder_matrix(item("Wv"), d, d, dev, l.qkv[2]) ||
+       !decoder_matrix(item("Wo"), d, d, dev, l.o) || !decoder_matrix(item("cWq"), d, d, dev, l.cq) || !decoder_matrix(item("cWo"), d, d, dev, l.co) ||
+       !decoder_matrix(item("W1"), d, 0, dev, l.w1) || !decoder_matrix(item("W2"), l.w1.b.cols, d, dev, l.w2) ||
+       !decoder_norm(item("ln1"), d, dev, l.ln1) || !decoder_norm(item("ln2"), d, dev, l.ln2) || !decoder_norm(item("ln3"), d, dev, l.ln3) ||
+       !decoder_cache(args[3], i, M * heads, dev, cap, l.k) || !decoder_cache(args[4], i, M * heads, dev, cap, l.v) ||
+       !decoder_cache(args[5], i, i ? layers[0].kc.size(0) : 0, dev, source_cap, l.kc) || !decoder_cache(args[6], i, l.kc.size(0), dev, source_cap, l.vc))
+      Py_RETURN_NONE;
+    source = source_cap;
+    widest = std::max(widest, l.w1.b.cols);
+  }
+  DecoderMatrix last;
+  if(!decoder_matrix(args[12], d, 0, dev, last) || len > cap || source < 1 || source > 512 || widest % 64 != 0 || last.b.cols < 1 ||
+     layers[0].kc.size(0) < 1 || (mask && (mask->numel() < 1 || mask->numel() % source != 0)))
+    Py_RETURN_NONE;
+  const int64_t entries = layers[0].kc.size(0), masks = mask ? mask->numel() / source : 0;
+  // what lies between the calls: rows of d (x twice, for one layer's and the next's), of the widest, slots, quantized activations
+  enum { kO, kA, kX1, kCo, kCa, kX2, kF2, kXa, kXb, kRows };
+  const int64_t row_bytes = (M * d * 4 + 255) / 256 * 256, wide_bytes = (M * widest * 4 + 255) / 256 * 256;
+  const int64_t slot_bytes = MARIAN_HIP_ABSMAX_SLOTS * 4;
+  enum { kOMax, kX1Max, kCoMax, kX2Max, kF1Max, kXMax, kSlots };
+  at::Tensor arena = empty({kRows * row_bytes + wide_bytes + kSlots * slot_bytes + M * widest + 256}, at::kByte, dev);
+  char* const base = static_cast<char*>(arena.data_ptr());
+  auto rows = [&](int i) { return reinterpret_cast<float*>(base + i * row_bytes); };
+  auto slots = [&](int i) { return reinterpret_cast<float*>(base + kRows * row_bytes + wide_bytes + i * slot_bytes); };
+  float* const f1 = reinterpret_cast<float*>(base + kRows * row_bytes);
+  int8_t* const aq = reinterpret_cast<int8_t*>(base + kRows * row_bytes + wide_bytes + kSlots * slot_bytes);
+  at::Tensor scores = empty({M, last.b.cols}, at::kFloat, dev);
+  float* const out = fptr_mut(scores);
+  const hipStream_t st = stream_of(dev);
+  const at::Tensor& ws = workspace(dev, st);
+  void* const wp = ws.data_ptr();
+  const size_t wn = (size_t)ws.numel();
+  const uint32_t* const table = anc ? static_cast<const uint32_t*>(anc->const_data_ptr()) : nullptr;
+  const char* where = "";
+  call("decoder step", [&] {
+    auto affine = [&](const float* a, const DecoderMatrix& w, float* to, int relu, const float* in_max, float* out_max) {
+      return L.int8_affine_f32_chained(a, aq, w.weights(), w.shift(), nullptr, 0, to, M, w.b.rows, w.b.cols, 1.0f, relu, in_max, out_max, wp, wn, st);
+    };
+    auto norm = [&](const float* a, const float* add, const DecoderNorm& ln, float* to, float* out_max) {
+      return L.layer_norm(a, add, fptr(&ln.gamma), d, fptr(&ln.beta), d, to, M, d, eps, out_max, st);
+    };
+    auto normed = [&](const float* add, const DecoderNorm& ln, float* to) {
+      return marian_hip_norm_input{add, fptr(&ln.gamma), fptr(&ln.beta), to, eps};
+    };
+    auto affine_of_norm = [&](const float* a, const marian_hip_norm_input& ln, const DecoderMatrix& w, float* to, int relu, float* out_max) {
+      const int8_t* Bq = w.weights();
+      const float* bias = w.shift();
+      const int64_t N = w.b.cols;
+      return L.int8_affine_f32_normed(a, &ln, 1, &Bq, &bias, &to, &N, M, d, 1.0f, relu, out_max, st);
+    };
+    const float* now = fptr(x);
+    const float* now_max = amax;
+    float* none_out[3] = {nullptr, nullptr, nullptr};
+    int status = MARIAN_HIP_OK;
+#define MH_STEP(name, expr)                      \
+  do {                                           \
+    status = (expr);                             \
+    if(status != MARIAN_HIP_OK) {                \
+      where = name;                              \
+      return status;                             \
+    }                                            \
+  } while(0)
+    for(size_t i = 0; i < layers.size(); ++i) {
+      const DecoderLayer& l = layers[i];
+      const int8_t* Bq[3] = {l.qkv[0].weights(), l.qkv[1].weights(), l.qkv[2].weights()};
+      const float* bias[3] = {l.qkv[0].shift(), l.qkv[1].shift(), l.qkv[2].shift()};
+      float *k = fptr_mut(l.k), *v = fptr_mut(l.v), *next = rows(i % 2 ? kXb : kXa);
+      // self-attention; behind a layer of few rows its input is that layer's last norm, taken on the way
+      const bool pending = few && i > 0;
+      const marian_hip_norm_input last_norm = pending ? normed(rows(kX2), layers[i - 1].ln3, next) : marian_hip_norm_input{};
+      const float* in = pending ? rows(kF2) : now;
+      if(anc)
+        MH_STEP("ProjectedAttention", L.int8_proj_attention_ancestors(in, pending ? &last_norm : nullptr, pending ? nullptr : aq, Bq, bias, none_out, M, d,
+                                                                     heads, k, v, len, cap, table, 1.0f / 8.0f, rows(kO), pending ? nullptr : now_max,
+                                                                     slots(kOMax), wp, wn, st));
+      else if(pending)
+        MH_STEP("ProjectedAttention", L.int8_proj_attention_normed(in, &last_norm, 3, Bq, bias, none_out, M, d, heads, k, v, M * heads, len, cap, nullptr,
+                                                                  0, 1.0f / 8.0f, rows(kO), slots(kOMax), st));
+      else
+        MH_STEP("ProjectedAttention", L.int8_proj_attention(in, aq, 3, Bq, bias, none_out, M, d, heads, k, v, M * heads, len, cap, nullptr, 0,
+                                                           1.0f / 8.0f, rows(kO), now_max, slots(kOMax), wp, wn, st));
+      if(pending) now = next;
+      MH_STEP("affineOrDot", affine(rows(kO), l.o, rows(kA), 0, slots(kOMax), nullptr));
+      // attention over the source
+      const int8_t* cBq = l.cq.weights();
+      const float* cbias = l.cq.shift();
+      float *kc = fptr_mut(l.kc), *vc = fptr_mut(l.vc);
+      if(few) {
+        const marian_hip_norm_input ln = normed(now, l.ln1, rows(kX1));
+        MH_STEP("ProjectedAttention", L.int8_proj_attention_normed(rows(kA), &ln, 1, &cBq, &cbias, none_out, M, d, heads, kc, vc, entries, source, source,
+                                                                  fptr(mask), masks, 1.0f / 8.0f, rows(kCo), slots(kCoMax), st));
+      } else {
+        MH_STEP("layerNorm", norm(rows(kA), now, l.ln1, rows(kX1), slots(kX1Max)));
+        MH_STEP("ProjectedAttention", L.int8_proj_attention(rows(kX1), aq, 1, &cBq, &cbias, none_out, M, d, heads, kc, vc, entries, source, source,
+                                                           fptr(mask), masks, 1.0f / 8.0f, rows(kCo), slots(kX1Max), slots(kCoMax), wp, wn, st));
+      }
+      MH_STEP("affineOrDot", affine(rows(kCo), l.co, rows(kCa), 0, slots(kCoMax), nullptr));
+      // feed-forward block
+      if(few) {
+        MH_STEP("affineOrDot", affine_of_norm(rows(kCa), normed(rows(kX1), l.ln2, rows(kX2)), l.w1, f1, 1, slots(kF1Max)));
+      } else {
+        MH_STEP("layerNorm", norm(rows(kCa), rows(kX1), l.ln2, rows(kX2), slots(kX2Max)));
+        MH_STEP("affineOrDot", affine(rows(kX2), l.w1, f1, 1, slots(kX2Max), slots(kF1Max)));
+      }
+      MH_STEP("affineOrDot", affine(f1, l.w2, rows(kF2), 0, slots(kF1Max), nullptr));
+      if(!few) {
+        MH_STEP("layerNorm", norm(rows(kF2), rows(kX2), l.ln3, next, slots(kXMax)));
+        now = next;
+        now_max = slots(kXMax);
+      }
+    }
+    if(few) MH_STEP("affineOrDot", affine_of_norm(rows(kF2), normed(rows(kX2), layers.back().ln3, rows(layers.size() % 2 ? kXb : kXa)), last, out, 0, nullptr));
+    else MH_STEP("affineOrDot", affine(now, last, out, 0, now_max, nullptr));
+#undef MH_STEP
+    return status;
+  }, &where);
+  return wrap(std::move(scores));
+  MH_END
+}
+
 // attention_ancestors(q, k, v, ancestors, kvLen, kNew, vNew, want_absmax) -> out or (out, absmax)
 PyObject* py_attention_ancestors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_TRY MH_ARGS(8, "attention_ancestors");
@@ -1019,7 +1224,7 @@ PyObject* py_setup(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyMethodDef methods[] = {
     MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
     MH_METHOD(affine_f32_grouped), MH_METHOD(affine_f32_normed), MH_METHOD(proj_attention_normed), MH_METHOD(proj_attention_ancestors), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
-    MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(attention_rows), MH_METHOD(split_heads), MH_METHOD(join_heads), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors),
+    MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(attention_rows), MH_METHOD(split_heads), MH_METHOD(join_heads), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors), MH_METHOD(decoder_layers),
     MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_words), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),
     {nullptr, nullptr, 0, nullptr}};
 

@@ -130,6 +130,13 @@ class DecoderStep:
         self.state, self.state_next = self.state_next, self.state
         self._cache_views()
 
+    def _layers_native(self, W, x, xmax):
+        """The calls that _layers_of_few_rows and step() make for the layers and the output layer, made by one native function
+        (_host_calls: decoder_layers): the same launches, bit for bit, without Python in between.  None where it does not
+        take the step (sizes or forms that the one-launch attentions refuse)."""
+        return integer._host.decoder_layers(x, xmax, W["layers"], self.Kself, self.Vself, self.Kenc, self.Venc, self.mask,
+                                            self.anc if self.by_ancestors else None, self.H, self.T, 1e-6, W["out"])
+
     def _layers_of_few_rows(self, W, x, xmax, rec):
         """The layers and the output layer for a handful of hypotheses: every layer norm is taken by the
         launch that multiplies its result (the launches of their own were a fifth of the step for six
@@ -214,10 +221,14 @@ class DecoderStep:
                 x, xmax = x
             if tr is not None:
                 rec("embed", E=self.E, ids=self.words, scale=self.emb_scale, signal=self.signal, out=x, position=self.T - 1)
-        few = fused_attention and ch and M <= 8 and bool(W["layers"])   # the rows up to which the layer norms need no launches of their own
-        if few:
-            logits = self._layers_of_few_rows(W, x, xmax, rec if tr is not None else None)
-        for li, ly in enumerate(() if few else W["layers"]):
+        logits = None
+        if fused_attention and ch and W["layers"]:
+            if tr is None and (grouped or not self.by_ancestors):   # all calls of the layers from native code, where it knows their form
+                logits = self._layers_native(W, x, xmax)
+            if logits is None and M <= 8:   # the rows up to which the layer norms need no launches of their own
+                logits = self._layers_of_few_rows(W, x, xmax, rec if tr is not None else None)
+        done = logits is not None
+        for li, ly in enumerate(() if done else W["layers"]):
             omax = x1max = comax = x2max = f1max = None
             fuse = fused_attention and not gemm_only and not self.by_ancestors and ch
             if fuse:   # q, k, v and the self-attention over the cache (the new position appended) in one launch
@@ -334,7 +345,7 @@ class DecoderStep:
                     x, xmax = x
                 if tr is not None:
                     rec("layer_norm", x=f2, add=xin, gamma=ly["ln3"][0], beta=ly["ln3"][1], out=x)
-        if not few:
+        if not done:
             logits, _ = integer.affine_f32(x, *W["out"], absmax=xmax)
             if tr is not None:
                 rec("affine", a=x, w=W["out"], out=logits, relu=False)

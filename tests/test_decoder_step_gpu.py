@@ -230,3 +230,31 @@ def test_ancestor_table_at_benchmark_size():
             words = torch.randint(0, copied.V, (copied.M,), device="cuda", generator=g)
             copied.advance(words, parents.reshape(-1))
             lazy.advance(words, parents.reshape(-1))
+
+
+@pytest.mark.parametrize("ancestors", [False, True])
+@pytest.mark.parametrize("beam,batch,d,layers,ffn,src,cap", [(1, 1, 128, 1, 192, 1, 3), (4, 2, 256, 2, 1024, 9, 8),
+                                                             (3, 3, 256, 3, 832, 65, None), (6, 20, 512, 2, 2048, 60, 24)])
+def test_layers_from_native_code(ancestors, beam, batch, d, layers, ffn, src, cap):
+    """The step whose layers one native function calls (8 rows: the last that take the layer norms in other launches, 9: the
+    first behind them) against the same calls made one by one: scores and caches bit for bit; forms that it does not know are left."""
+    import torch
+    D = load("decoder_step")
+    step = D.DecoderStep(sets=1, d=d, ffn=ffn, heads=d // 64, vocab=1000, layers=layers, beam=beam, batch=batch, t_past=2,
+                         src_len=src, min_src_len=1, seed=61, t_capacity=cap, ancestors=ancestors)
+    native, taken = step._layers_native, []
+    caches = step.state.clone()
+
+    def counted(*args):
+        taken.append(native(*args))
+        return taken[-1]
+
+    step._layers_native = counted
+    got = step.step(0)
+    after, _ = step.state.clone(), step.state.copy_(caches)
+    assert len(taken) == 1 and taken[0] is not None
+    step._layers_native = lambda *args: None
+    assert torch.equal(step.step(0), got) and torch.equal(step.state, after)
+    step.mask = step.mask.double()   # a type the native function leaves to the single calls
+    x, xmax = step.ops.scaledEmbeddings(step.E, step.words, step.emb_scale, step.signal, step.M, want_absmax=True)
+    assert native(step.sets[0], x, xmax) is None
