@@ -866,6 +866,18 @@ unsigned next_nonce() {
   return nonce.fetch_add(0x9E3779B1u, std::memory_order_relaxed);
 }
 
+// The words of a workspace through which the workgroups of a one-pass launch exchange their abs-max.
+struct OnePass {
+  unsigned long long *slots, *gen, *mail;
+  unsigned nonce;
+  int spins;
+};
+OnePass onepass_words(void* workspace, bool no_patience) {
+  unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
+  return {reinterpret_cast<unsigned long long*>(ws + kOnePassSlotsOffset), reinterpret_cast<unsigned long long*>(ws + kOnePassGenOffset),
+          reinterpret_cast<unsigned long long*>(ws + kOnePassMailOffset), next_nonce(), no_patience ? 0 : kOnePassSpinLimit};
+}
+
 int absmax_blocks(size_t n4) {
   size_t per_block = (size_t)kQuantThreads * 4;  // four 16-byte loads per thread, all in flight
   size_t g = (n4 + per_block - 1) / per_block;
@@ -1014,18 +1026,13 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
     const size_t groups = (n16 + 1024 * (size_t)sets - 1) / (1024 * (size_t)sets);
     const bool fits = groups <= (size_t)cus;
     if(fits && ov != 700 && (n >= kOnePassMinElems || ov == 701 || ov == 702)) {
-      unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
-      unsigned long long* slots = reinterpret_cast<unsigned long long*>(ws + kOnePassSlotsOffset);
-      unsigned long long* gen = reinterpret_cast<unsigned long long*>(ws + kOnePassGenOffset);
-      unsigned long long* mail = reinterpret_cast<unsigned long long*>(ws + kOnePassMailOffset);
-      const unsigned nonce = next_nonce();
-      const int spins = ov == 702 ? 0 : kOnePassSpinLimit;
+      const OnePass o = onepass_words(workspace, ov == 702);
       if(sets == 1)
-        MH_LAUNCH(prepare_a_onepass_kernel<1>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
+        MH_LAUNCH(prepare_a_onepass_kernel<1>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.mail, o.nonce, o.spins, (int)groups);
       else if(sets == 2)
-        MH_LAUNCH(prepare_a_onepass_kernel<2>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
+        MH_LAUNCH(prepare_a_onepass_kernel<2>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.mail, o.nonce, o.spins, (int)groups);
       else
-        MH_LAUNCH(prepare_a_onepass_kernel<4>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, slots, gen, mail, nonce, spins, (int)groups);
+        MH_LAUNCH(prepare_a_onepass_kernel<4>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.mail, o.nonce, o.spins, (int)groups);
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
     }
@@ -1047,6 +1054,22 @@ int marian_hip_int8_prepare_b(const float* W, int8_t* Bq, int64_t K, int64_t N, 
   if(workspace_bytes < kWorkspaceBytes) return MARIAN_HIP_ERR_WORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const size_t n = (size_t)K * (size_t)N;
+  // One launch where every CU can hold its tiles (measurement ids 700 / 702: two passes / one pass with no patience).
+  const int ov = kernel_override() % 1000;
+  const long long tiles_n = (N + 63) / 64, tiles = tiles_n * (K / 64);
+  const long long cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
+  if(tiles <= 4 * cus && ov != 700 && aligned(workspace, 8)) {
+    const OnePass o = onepass_words(workspace, ov == 702);
+    const int per = tiles <= cus ? 1 : tiles <= 2 * cus ? 2 : 4, groups = (int)((tiles + per - 1) / per);
+    if(per == 1)
+      MH_LAUNCH(prepare_b_onepass_kernel<1>, dim3(groups), dim3(256), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.mail, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+    else if(per == 2)
+      MH_LAUNCH(prepare_b_onepass_kernel<2>, dim3(groups), dim3(512), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.mail, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+    else
+      MH_LAUNCH(prepare_b_onepass_kernel<4>, dim3(groups), dim3(1024), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.mail, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+    MH_HIP(hipGetLastError());
+    return MARIAN_HIP_OK;
+  }
   float* partials = reinterpret_cast<float*>(workspace);
   const int g = absmax_blocks(n / 4);
   MH_LAUNCH(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, W, n / 4,

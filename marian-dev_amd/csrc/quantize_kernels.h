@@ -77,6 +77,71 @@ __global__ __launch_bounds__(kSingleBlockThreads) void prepare_a_single_block_ke
 // first use.  Every wait is bounded: a workgroup that runs out of patience (the device was shared
 // and not all workgroups were resident) takes the abs-max over the whole input itself - the
 // result is the same - clears its slot, and the launch still ends.
+__device__ __forceinline__ unsigned long long onepass_word(unsigned tag, float v) {
+  return ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v);
+}
+// m: abs-max of this workgroup's values (in every thread), tag: this launch's, G <= THREADS workgroups.  scan: the abs-max of
+// the whole input, by this workgroup alone.
+template <int THREADS, class Scan>
+__device__ __forceinline__ float onepass_exchange(float m, unsigned gen, unsigned tag, unsigned long long* slots,
+                                                  unsigned long long* gen_word, unsigned long long* mailboxes, int spin_limit,
+                                                  int G, float* red, float* shared_max, Scan scan) {
+  const int tid = threadIdx.x, g = blockIdx.x;
+  if(tid == 0) __hip_atomic_store(&slots[g * kOnePassStride], onepass_word(tag, m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  bool ok = true;
+  if(g == 0) {
+    float mine = 0.0f;
+    if(tid < G) {
+      ok = false;
+      for(int spin = 0; spin < spin_limit; ++spin) {
+        const unsigned long long w = __hip_atomic_load(&slots[tid * kOnePassStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if((unsigned)(w >> 32) == tag) {
+          mine = __uint_as_float((unsigned)w);
+          ok = true;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(4);
+      }
+    }
+    const bool all_ok = __syncthreads_and(ok ? 1 : 0) != 0;
+    const float amax = all_ok ? block_max<THREADS / kWave>(mine, red) : scan();
+    if(tid < kOnePassMailboxes)
+      __hip_atomic_store(&mailboxes[tid * 32], onepass_word(tag, amax), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the next launch (or replay) expects another tag; every workgroup of this launch has read
+    // the generation by now, or will find its words unanswered and help itself
+    if(tid == 0) {
+      __hip_atomic_store(gen_word, (unsigned long long)(gen + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&slots[0], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return amax;
+  }
+  if(tid == 0) {
+    ok = false;
+    const unsigned long long* box = &mailboxes[(g % kOnePassMailboxes) * 32];
+    for(int spin = 0; spin < spin_limit; ++spin) {
+      const unsigned long long w = __hip_atomic_load(box, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if((unsigned)(w >> 32) == tag) {
+        *shared_max = __uint_as_float((unsigned)w);
+        ok = true;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(8);
+    }
+    // answered or not, this launch is done with the slot
+    __hip_atomic_store(&slots[g * kOnePassStride], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const bool answered = __syncthreads_and(ok ? 1 : 0) != 0;
+  return answered ? *shared_max : scan();
+}
+// Abs-max of n4 vectors by one workgroup (the way out of a wait that ran out).
+template <int THREADS>
+__device__ __forceinline__ float onepass_scan(const float* x, size_t n4, float* red) {
+  const v4f* x4 = reinterpret_cast<const v4f*>(x);
+  float m = 0.0f;
+  for(size_t i = threadIdx.x; i < n4; i += THREADS) m = abs4max(x4[i], m);
+  return block_max<THREADS / kWave>(m, red);
+}
+
 template <int SETS>
 __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __restrict__ x, unsigned n16,
                                                                  int8_t* __restrict__ out,
@@ -118,63 +183,10 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
   m = block_max<1024 / kWave>(m, red);   // (its barriers also publish shared_tag)
   const unsigned tag = shared_tag;
 
-  // abs-max over all of x by this workgroup alone (the way out of a wait that ran out)
-  auto scan_all = [&]() {
-    const v4f* x4 = reinterpret_cast<const v4f*>(x);
-    const size_t n4 = (size_t)n16 * 4;
-    float mm = 0.0f;
-    for(size_t i = tid; i < n4; i += 1024) mm = abs4max(x4[i], mm);
-    return block_max<1024 / kWave>(mm, red);
-  };
-  auto pack = [](unsigned t, float v) { return ((unsigned long long)t << 32) | (unsigned long long)__float_as_uint(v); };
   float amax = m;
-  if(G > 1) {
-    if(tid == 0) __hip_atomic_store(&slots[g * kOnePassStride], pack(tag, m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    bool ok = true;
-    if(g == 0) {
-      float mine = 0.0f;
-      if(tid < G) {
-        ok = false;
-        for(int spin = 0; spin < spin_limit; ++spin) {
-          const unsigned long long w = __hip_atomic_load(&slots[tid * kOnePassStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if((unsigned)(w >> 32) == tag) {
-            mine = __uint_as_float((unsigned)w);
-            ok = true;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(4);
-        }
-      }
-      const bool all_ok = __syncthreads_and(ok ? 1 : 0) != 0;
-      amax = all_ok ? block_max<1024 / kWave>(mine, red) : scan_all();
-      if(tid < kOnePassMailboxes)
-        __hip_atomic_store(&mailboxes[tid * 32], pack(tag, amax), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      // the next launch (or replay) expects another tag; every workgroup of this launch has read
-      // the generation by now, or will find its words unanswered and help itself
-      if(tid == 0) {
-        __hip_atomic_store(gen_word, (unsigned long long)(gen + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&slots[0], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    } else {
-      if(tid == 0) {
-        ok = false;
-        const unsigned long long* box = &mailboxes[(g % kOnePassMailboxes) * 32];
-        for(int spin = 0; spin < spin_limit; ++spin) {
-          const unsigned long long w = __hip_atomic_load(box, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if((unsigned)(w >> 32) == tag) {
-            shared_max = __uint_as_float((unsigned)w);
-            ok = true;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(8);
-        }
-        // answered or not, this launch is done with the slot
-        __hip_atomic_store(&slots[g * kOnePassStride], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      const bool answered = __syncthreads_and(ok ? 1 : 0) != 0;
-      amax = answered ? shared_max : scan_all();
-    }
-  }
+  if(G > 1)
+    amax = onepass_exchange<1024>(m, gen, tag, slots, gen_word, mailboxes, spin_limit, G, red, &shared_max,
+                                  [&] { return onepass_scan<1024>(x, (size_t)n16 * 4, red); });
   const float qm = quant_mult_from_maxabs(amax);
   const bool finite = qm < __builtin_inff();
 #pragma unroll
@@ -245,24 +257,47 @@ __global__ __launch_bounds__(THREADS) void quantize_a_wide_kernel(const float* _
   if(blockIdx.x == 0 && tid == 0) *reinterpret_cast<float*>(out + (size_t)n16 * 16) = qm;
 }
 
-// Pass 2 of prepareB: W fp32 [K x N] -> K-blocked int8 payload of the quantized transpose + tail.
-// A workgroup transposes a 64(k) x 64(n) tile through LDS: reads are coalesced along n, writes are
-// 16-byte chunks of K values, the columns of a K sub-step side by side.
+// prepareB: W fp32 [K x N] -> K-blocked int8 payload of the quantized transpose + tail, in two parts that the kernels below
+// share.  256 threads transpose a 64(k) x 64(n) tile through LDS: reads are coalesced along n, writes are 16-byte chunks of K
+// values, the columns of a K sub-step side by side.  thread: 0 .. 255 of them.
+__device__ __forceinline__ void load_b_tile(const float* __restrict__ W, int K, int N, int n0, int k0, int thread, float (&v)[16]) {
+  // wave tk takes k rows 16*tk .. 16*tk+15 (K % 64 == 0: the k rows of a tile are all inside; columns past N read the last
+  // one and are not written)
+  const int tn = thread % 64, tk = thread / 64;
+  const float* w = W + (size_t)(k0 + tk * 16) * N + min(n0 + tn, N - 1);
+#pragma unroll
+  for(int k = 0; k < 16; ++k) v[k] = w[(size_t)k * N];
+}
+// tile: [n][k / 4] as packed dwords, 17 dwords per row: the 64 lanes of a wave (consecutive n, one k group) hit every bank
+// twice, the minimum for 64 lanes on 32 banks.  Holds a barrier: every thread of the workgroup calls it.
+__device__ __forceinline__ void store_b_tile(const float (&v)[16], float qm, uint32_t (*tile)[17], int K, int N, int n0, int k0,
+                                             int thread, bool live, int8_t* __restrict__ out) {
+  const int tn = thread % 64, tk = thread / 64;
+#pragma unroll
+  for(int g = 0; g < 4; ++g)   // four consecutive k of column n: one packed dword
+    tile[tn][tk * 4 + g] = quantize_pack4(v4f{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}, qm);
+  __syncthreads();
+  // 64 columns (n) x four 16-byte chunks (k): two neighbouring threads write the two halves of a
+  // column's sub-step, a wave 32 columns of one sub-step (1 KB of consecutive memory)
+  const int rn = (thread / 2) % 64, ck = (thread / 128) * 32 + (thread % 2) * 16;
+  const int n = n0 + rn, k = k0 + ck;
+  if(live && n < N) {
+    uint4 q;
+    q.x = tile[rn][ck / 4]; q.y = tile[rn][ck / 4 + 1]; q.z = tile[rn][ck / 4 + 2]; q.w = tile[rn][ck / 4 + 3];
+    *reinterpret_cast<uint4*>(out + b_chunk_offset(n, k / 16, N)) = q;
+  }
+}
+
+// Pass 2 of prepareB (the abs-max is that of `partials`), one tile to a workgroup.
 __global__ __launch_bounds__(256) void quantize_b_transpose_kernel(
     const float* __restrict__ W, int K, int N, const float* __restrict__ partials,
     int n_partials, int8_t* __restrict__ out) {
   __shared__ float red[256 / kWave];
-  // [n][k / 4] as packed dwords, 17 dwords per row: the 64 lanes of a wave (consecutive n, one k
-  // group) hit every bank twice, the minimum for 64 lanes on 32 banks
   __shared__ uint32_t tile[64][17];
   const int n0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
-  const int tn = threadIdx.x % 64, tk = threadIdx.x / 64;  // wave tk takes k rows 16*tk .. 16*tk+15
-  // the tile and the partials are requested together (K % 64 == 0: the k rows of a tile are all inside;
-  // columns past N read the last one and are not written)
-  const float* w = W + (size_t)(k0 + tk * 16) * N + min(n0 + tn, N - 1);
+  // the tile and the partials are requested together
   float v[16], pm[kMaxPartials / 256];
-#pragma unroll
-  for(int k = 0; k < 16; ++k) v[k] = w[(size_t)k * N];
+  load_b_tile(W, K, N, n0, k0, threadIdx.x, v);
 #pragma unroll
   for(int i = 0; i < kMaxPartials / 256; ++i) pm[i] = partials[min((int)threadIdx.x + i * 256, n_partials - 1)];
   float m = 0.0f;
@@ -270,21 +305,44 @@ __global__ __launch_bounds__(256) void quantize_b_transpose_kernel(
   for(int i = 0; i < kMaxPartials / 256; ++i) m = fmaxf(m, pm[i]);
   m = block_max<256 / kWave>(m, red);
   const float qm = quant_mult_from_maxabs(m);
-#pragma unroll
-  for(int g = 0; g < 4; ++g)   // four consecutive k of column n: one packed dword
-    tile[tn][tk * 4 + g] = quantize_pack4(v4f{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}, qm);
-  __syncthreads();
-  // 64 columns (n) x four 16-byte chunks (k): two neighbouring threads write the two halves of a
-  // column's sub-step, a wave 32 columns of one sub-step (1 KB of consecutive memory)
-  const int rn = (threadIdx.x / 2) % 64, ck = (threadIdx.x / 128) * 32 + (threadIdx.x % 2) * 16;
-  int n = n0 + rn, k = k0 + ck;
-  if(n < N && k < K) {  // K % 64 == 0, so a 16-byte run is inside or outside as a whole
-    uint4 v;
-    v.x = tile[rn][ck / 4]; v.y = tile[rn][ck / 4 + 1]; v.z = tile[rn][ck / 4 + 2]; v.w = tile[rn][ck / 4 + 3];
-    *reinterpret_cast<uint4*>(out + b_chunk_offset(n, k / 16, N)) = v;
-  }
+  store_b_tile(v, qm, tile, K, N, n0, k0, threadIdx.x, true, out);
   if(blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)
     *reinterpret_cast<float*>(out + (size_t)K * N) = qm;
+}
+
+// prepareB in one launch, for matrices of up to four tiles a CU: TILES tiles to a workgroup of TILES x 256 threads, held in
+// registers while the workgroups exchange their abs-max (as the one-pass form of prepareA).  The call is bound by its launches
+// on the host: 1024 x 1024 in two of them 7.9 us, in one 6.3.
+template <int TILES>
+__global__ __launch_bounds__(TILES * 256) void prepare_b_onepass_kernel(const float* __restrict__ W, int K, int N,
+                                                                        int8_t* __restrict__ out, unsigned long long* slots,
+                                                                        unsigned long long* gen_word,
+                                                                        unsigned long long* mailboxes, unsigned nonce,
+                                                                        int spin_limit, int groups, int tiles_n, int tiles) {
+  __shared__ float red[TILES * 256 / kWave];
+  __shared__ float shared_max;
+  __shared__ unsigned shared_tag;
+  __shared__ uint32_t turn[TILES][64][17];
+  const int tid = threadIdx.x, sub = tid / 256, thread = tid % 256;
+  unsigned gen = 0;
+  if(tid == 0 && groups > 1) gen = (unsigned)__hip_atomic_load(gen_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int wanted = __builtin_amdgcn_readfirstlane((int)blockIdx.x * TILES + sub);
+  const bool live = wanted < tiles;
+  const int t = live ? wanted : 0;   // (read again and not written: a repeated value does not change a maximum)
+  const int n0 = (t % tiles_n) * 64, k0 = (t / tiles_n) * 64;
+  float v[16], m = 0.0f;
+  load_b_tile(W, K, N, n0, k0, thread, v);
+#pragma unroll
+  for(int k = 0; k < 16; ++k) m = fmaxf(m, fabsf(v[k]));
+  if(tid == 0) shared_tag = (nonce + gen) | 0x80000000u;   // never 0: a cleared word does not match
+  m = block_max<TILES * 256 / kWave>(m, red);   // (its barriers also publish shared_tag)
+  float amax = m;
+  if(groups > 1)
+    amax = onepass_exchange<TILES * 256>(m, gen, shared_tag, slots, gen_word, mailboxes, spin_limit, groups, red, &shared_max,
+                                         [&] { return onepass_scan<TILES * 256>(W, (size_t)K * N / 4, red); });
+  const float qm = quant_mult_from_maxabs(amax);
+  store_b_tile(v, qm, turn[sub], K, N, n0, k0, thread, live, out);
+  if(blockIdx.x == 0 && tid == 0) *reinterpret_cast<float*>(out + (size_t)K * N) = qm;
 }
 
 // prepareBQuantizedTransposed: int8 W^T as plain rows [N x K] (the payload of a model file) -> the

@@ -125,6 +125,25 @@ def test_prepare_b_bit_exact(integer, orc, synth, K, N):
     assert np.array_equal(upload_b(integer, want, (K, N)).numpy(), q.numpy())
 
 
+@pytest.mark.parametrize("kernel", [0, 700, 702])
+@pytest.mark.parametrize("K,N", [(64, 64), (64, 72), (128, 4096), (1024, 1024), (1088, 1024), (512, 4040), (4096, 968), (1024, 4096),
+                                 (1024, 4104)])
+def test_prepare_b_one_launch_and_two(integer, orc, synth, K, N, kernel):
+    """prepareB with the abs-max exchanged between the workgroups (the automatic choice up to 1024 tiles of 64 x 64: one, two and
+    four tiles to a workgroup, a last one with tiles left over; 1024 x 4104 is the first beyond), in two launches (700), and with
+    workgroups that scan the whole matrix themselves (702); called twice, since a call leaves words for the next."""
+    if kernel == 702 and K * N > (1 << 20):
+        pytest.skip("every workgroup scanning 4 M values: correct, and slow on purpose")
+    say("prepare_b launches", K, N, kernel)
+    W = synth.normal(260 + N, synth.STREAM_W, (K, N), 0.02)
+    W.flat[(K * 37 + 5 * N + 3) % W.size] = np.float32(-0.75)   # the extreme sits in one workgroup's share
+    want = orc.prepare_b(W)
+    with forced(kernel):
+        first, second = integer.prepareB(dev(W)).file_bytes(), integer.prepareB(dev(W * np.float32(0.5))).file_bytes()
+    assert np.array_equal(first, want)
+    assert np.array_equal(second, orc.prepare_b(W * np.float32(0.5)))
+
+
 def _random_prepare_cases(n):
     rng = np.random.default_rng(20261131)
     return [(i, int(rng.choice([1, 2, 5, 31, 64, 100, 511, 512, 513, 1500, 4099])), 64 * int(rng.integers(1, 65)),
