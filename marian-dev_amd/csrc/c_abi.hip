@@ -855,12 +855,11 @@ int run_gemm(const int8_t* Aq, const int8_t* Bq, const float* bias, const uint32
   return launch_gemm(a, reinterpret_cast<hipStream_t>(stream));
 }
 
-// One-pass prepareA: from this many values on (below, two launches are as fast or faster), how long a
-// workgroup polls before it helps itself (each poll is a memory round trip of about a microsecond),
-// and the nonce that starts its tags (random per process, so that words left in recycled device
+// One-pass forms: how long a workgroup polls before it helps itself (each poll is a memory round trip of about half a
+// microsecond: 2 ms, where a launch that has the chip waits for 2 us and one that shares it with other streams may find that
+// its last workgroups have to wait for theirs), and the nonce that starts their tags (random per process, so that words left in recycled device
 // memory by another process do not match).
-constexpr size_t kOnePassMinElems = 4u << 20;   // (measured: 8 MB of input - no gain; 16.8 MB: 10.3 -> 9.4 us; 67 MB: 30.4 -> 21.1 us)
-constexpr int kOnePassSpinLimit = 20000;
+constexpr int kOnePassSpinLimit = 4000;
 unsigned next_nonce() {
   static std::atomic<unsigned> nonce{(unsigned)std::random_device{}() | 1u};
   return nonce.fetch_add(0x9E3779B1u, std::memory_order_relaxed);
@@ -868,14 +867,14 @@ unsigned next_nonce() {
 
 // The words of a workspace through which the workgroups of a one-pass launch exchange their abs-max.
 struct OnePass {
-  unsigned long long *slots, *gen, *mail;
+  unsigned long long *slots, *gen, *boards;
   unsigned nonce;
   int spins;
 };
 OnePass onepass_words(void* workspace, bool no_patience) {
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
   return {reinterpret_cast<unsigned long long*>(ws + kOnePassSlotsOffset), reinterpret_cast<unsigned long long*>(ws + kOnePassGenOffset),
-          reinterpret_cast<unsigned long long*>(ws + kOnePassMailOffset), next_nonce(), no_patience ? 0 : kOnePassSpinLimit};
+          reinterpret_cast<unsigned long long*>(ws + kOnePassBoardOffset), next_nonce(), no_patience ? 0 : kOnePassSpinLimit};
 }
 
 int absmax_blocks(size_t n4) {
@@ -1013,26 +1012,30 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
   if(!workspace) return MARIAN_HIP_ERR_NULL;
   if(workspace_bytes < kWorkspaceBytes) return MARIAN_HIP_ERR_WORKSPACE;
   if(!aligned(workspace, 8)) return MARIAN_HIP_ERR_ALIGN;
-  // One pass over the input where it fits the register files of the chip's CUs (one workgroup per
-  // CU: 16.7 M values on 256 CUs) and is large enough for the second read to cost more than the
-  // exchange of the abs-max between the workgroups (measurement ids 700 / 701 force two passes /
-  // one pass; 702: one pass with no patience, every workgroup scans the whole input itself).
+  // One pass over the input where it fits the register files of the chip's CUs (one workgroup per CU: 16.7 M values on 256
+  // CUs), back to back in a graph against two passes: 64 x 1024 values 4.1 and 4.3 us, 1024 x 1024 4.4 and 5.0, 4096 x 1024
+  // 6.0 and 7.9, 2050 x 4096 8.6 and 14.2, 4096 x 4096 17.2 and 24.7, and one launch fewer on a stream.  (Measurement
+  // ids: 700 two passes; 702 one pass with no patience, every workgroup scans the whole input itself.)
   {
     const int ov = kernel_override() % 1000;
     const int cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
     const size_t n16 = n / 16;
     int sets = 1;
-    while(sets < 4 && (n16 + 1024 * (size_t)sets - 1) / (1024 * (size_t)sets) > (size_t)cus) sets *= 2;
+    while(sets < 4 && (n16 + 1024 * (size_t)sets - 1) / (1024 * (size_t)sets) > (size_t)cus) ++sets;
     const size_t groups = (n16 + 1024 * (size_t)sets - 1) / (1024 * (size_t)sets);
     const bool fits = groups <= (size_t)cus;
-    if(fits && ov != 700 && (n >= kOnePassMinElems || ov == 701 || ov == 702)) {
+    if(fits && ov != 700) {
       const OnePass o = onepass_words(workspace, ov == 702);
-      if(sets == 1)
-        MH_LAUNCH(prepare_a_onepass_kernel<1>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.mail, o.nonce, o.spins, (int)groups);
-      else if(sets == 2)
-        MH_LAUNCH(prepare_a_onepass_kernel<2>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.mail, o.nonce, o.spins, (int)groups);
-      else
-        MH_LAUNCH(prepare_a_onepass_kernel<4>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.mail, o.nonce, o.spins, (int)groups);
+#define MH_ONEPASS(SETS)                                                                                                       \
+  MH_LAUNCH(prepare_a_onepass_kernel<SETS>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.boards, \
+            o.nonce, o.spins, (int)groups)
+      switch(sets) {
+        case 1: MH_ONEPASS(1); break;
+        case 2: MH_ONEPASS(2); break;
+        case 3: MH_ONEPASS(3); break;
+        default: MH_ONEPASS(4); break;
+      }
+#undef MH_ONEPASS
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
     }
@@ -1062,11 +1065,11 @@ int marian_hip_int8_prepare_b(const float* W, int8_t* Bq, int64_t K, int64_t N, 
     const OnePass o = onepass_words(workspace, ov == 702);
     const int per = tiles <= cus ? 1 : tiles <= 2 * cus ? 2 : 4, groups = (int)((tiles + per - 1) / per);
     if(per == 1)
-      MH_LAUNCH(prepare_b_onepass_kernel<1>, dim3(groups), dim3(256), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.mail, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<1>, dim3(groups), dim3(256), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
     else if(per == 2)
-      MH_LAUNCH(prepare_b_onepass_kernel<2>, dim3(groups), dim3(512), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.mail, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<2>, dim3(groups), dim3(512), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
     else
-      MH_LAUNCH(prepare_b_onepass_kernel<4>, dim3(groups), dim3(1024), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.mail, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<4>, dim3(groups), dim3(1024), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
   }
@@ -1393,8 +1396,8 @@ int marian_hip_int8_affine_f32_static(const float* A, const int8_t* Bq, const fl
   int8_t* Aq = reinterpret_cast<int8_t*>(base);
   void* workspace = base + kStaticAqBytes;
   // The quantized activations and the abs-max partials are written earlier in the same call than
-  // they are read.  The hand-over area of the one-pass prepareA (M * K >= 4 Mi: arrival slots,
-  // generation word, mailboxes) is different: its words persist from call to call and are matched
+  // they are read.  The hand-over area of the one-pass prepareA (more than 32 Ki values: arrival slots,
+  // generation word, boards) is different: its words persist from call to call and are matched
   // by tag (a per-process nonce plus the generation word, top bit always set), so a word left by
   // an earlier call - or the zeros the array starts with - never passes for a fresh one.  Nothing
   // has to be cleared between calls.

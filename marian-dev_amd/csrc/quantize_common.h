@@ -9,16 +9,16 @@ namespace marian_hip {
 constexpr int kQuantThreads = 256;
 constexpr int kMaxPartials = 1024;                  // floats of workspace used by the two-pass forms
 // Workspace layout: [0, 4 KB) abs-max partials of the two-pass forms; then the hand-over area of the
-// one-pass prepareA: 256 arrival slots of 8 bytes (a cache line each made no difference: 23.8 us
-// either way for 4096 x 4096), one generation word, and 16 mailboxes 256 bytes apart.
+// one-pass forms: 256 arrival slots of 8 bytes, one generation word, and 16 boards of 16 words,
+// 256 bytes apart.
 constexpr int kOnePassMaxGroups = 256;              // workgroups of the one-pass form (one per CU)
-constexpr int kOnePassMailboxes = 16;
-constexpr int kOnePassStride = 1;                   // 8-byte words between two slots
+constexpr int kOnePassBoards = 16;                  // workgroups of a group, and boards that its maximum is published on
+constexpr int kOnePassBoardWords = 32;              // 8-byte words between two boards (16 of them a group's)
 constexpr size_t kOnePassSlotsOffset = kMaxPartials * sizeof(float);
-constexpr size_t kOnePassGenOffset = kOnePassSlotsOffset + kOnePassMaxGroups * kOnePassStride * 8;
-constexpr size_t kOnePassMailOffset = 8192;
-constexpr size_t kWorkspaceBytes = kOnePassMailOffset + kOnePassMailboxes * 256;   // 12 KB
-static_assert(kOnePassGenOffset + 8 <= kOnePassMailOffset, "workspace layout");
+constexpr size_t kOnePassGenOffset = kOnePassSlotsOffset + kOnePassMaxGroups * 8;
+constexpr size_t kOnePassBoardOffset = 8192;
+constexpr size_t kWorkspaceBytes = kOnePassBoardOffset + kOnePassBoards * kOnePassBoardWords * 8;   // 12 KB
+static_assert(kOnePassGenOffset + 8 <= kOnePassBoardOffset, "workspace layout");
 constexpr int kSingleBlockThreads = 1024;
 constexpr int kSingleBlockMaxElems = 32 * 1024;     // one workgroup does abs-max and quantize (beyond: 8.6 us against 6.4 us for two launches)
 
