@@ -319,6 +319,7 @@ struct FusedSrc {   // what the fused modes read and write besides GemmArgs
   int8_t* aq_out = nullptr;
   const float* partials = nullptr;
   int n_partials = 0;
+  const AbsMaxExchange* exchange = nullptr;   // in place of partials (gemm_rows_kernel)
 };
 
 // Several weight matrices behind one activation tensor: the table the kernel reads, built for
@@ -443,15 +444,19 @@ int launch_rows(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const Grou
     a2.stream_out = 0;
     a2.absmax_out = nullptr;
     MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS, GroupTable>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, a2.M, a2.K,
-                       a2.N, a2.n_out, f.n_partials, tile_block, flags, a2, f.aq_out, groups->table);
+                       a2.N, a2.n_out, f.n_partials, tile_block, flags, a2, f.aq_out, groups->table, AbsMaxSlots());
   } else {
     a2.stream_out = (long long)a.M * a.n_out * 4 >= (4ll << 20) ? 1 : 0;   // (see launch_stream32)
     if(a.absmax_out) {   // one slot per wave
       if((long long)a2.blocks_x * a2.blocks_y * kRowsWaves <= kAbsmaxSlots) t_absmax_written = true;
       else a2.absmax_out = nullptr;
     }
-    MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, a2.M, a2.K, a2.N, a2.n_out,
-                       f.n_partials, tile_block, flags, a2, f.aq_out, NoGroups());
+    if(f.exchange)
+      MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS, NoGroups, AbsMaxExchange>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, nullptr, a2.M, a2.K,
+                         a2.N, a2.n_out, 0, tile_block, flags, a2, f.aq_out, NoGroups(), *f.exchange);
+    else
+      MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, a2.M, a2.K, a2.N, a2.n_out,
+                         f.n_partials, tile_block, flags, a2, f.aq_out, NoGroups(), AbsMaxSlots());
   }
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -865,12 +870,18 @@ unsigned next_nonce() {
   return nonce.fetch_add(0x9E3779B1u, std::memory_order_relaxed);
 }
 
+// Whether the workgroups of gemm_rows_kernel take the abs-max of the activations themselves: one to a CU, a share of the
+// activations that a thread holds in a few registers, and rows of up to 2048 values (100 x 4096 x 1024 9.5 us that way, with a
+// launch in front 9.1; 40 x 3072 x 768 7.3 and 7.0).  (Measurement ids: 630 the launch in front; 702 no patience.)
+bool rows_can_exchange(int M, int K, int n_out, int kw_override) {
+  const TiledPlan plan = plan_tiled(M, K, n_out, kw_override);
+  const long long groups = ((n_out + 31) / 32) * (long long)((M + plan.rows - 1) / plan.rows);
+  const int cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
+  return plan.kw == 8 && K <= 2048 && groups <= cus && (long long)M * K <= groups * kRowsShare;
+}
+
 // The words of a workspace through which the workgroups of a one-pass launch exchange their abs-max.
-struct OnePass {
-  unsigned long long *slots, *gen, *boards;
-  unsigned nonce;
-  int spins;
-};
+using OnePass = AbsMaxExchange;
 OnePass onepass_words(void* workspace, bool no_patience) {
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
   return {reinterpret_cast<unsigned long long*>(ws + kOnePassSlotsOffset), reinterpret_cast<unsigned long long*>(ws + kOnePassGenOffset),
@@ -1159,6 +1170,10 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
     if(absmax_in) {   // the producer of A left its abs-max: no launch for it
       f.partials = absmax_in;
       f.n_partials = kAbsmaxSlots;
+    } else if(which != 630 && rows_can_exchange((int)M, (int)K, (int)n_out, want_tiled ? which - 620 : 0) && aligned(workspace, 8)) {
+      const OnePass o = onepass_words(workspace, which == 702);
+      f.exchange = &o;
+      return launch_stream32_auto<kFusedTiled>(a, f, hst, want_tiled ? which - 620 : 0);
     } else {
       const size_t n = (size_t)M * (size_t)K;
       float* partials = reinterpret_cast<float*>(workspace);

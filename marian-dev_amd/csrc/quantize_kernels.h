@@ -2,6 +2,7 @@
 #pragma once
 
 #include "int8_common.h"
+#include "onepass_exchange.h"
 #include "quantize_common.h"
 
 namespace marian_hip {
@@ -65,83 +66,7 @@ __global__ __launch_bounds__(kSingleBlockThreads) void prepare_a_single_block_ke
 // second read costs as much as the first (67 MB: 14 us each, the memory-side cache does not help).
 // Here the input stays in registers between the two steps: at most one workgroup of 1024 threads
 // per CU, each thread holding SETS x 16 values, so 256 CUs hold up to 16.7 M values (4096 x 4096).
-// In between, the workgroups exchange their abs-max through the workspace, in groups of 16:
-//   * every workgroup stores (tag, abs-max bits) into its arrival slot - one 8-byte store at device
-//     scope, so tag and value arrive together;
-//   * the first workgroup of a group polls its group's slots (one line), takes the maximum and publishes (tag, max) to its
-//     word of every one of 16 boards (a line each);
-//   * every workgroup polls the words of all groups on one board (16 pollers a board) and takes their maximum;
-//   * nothing but these 8-byte words is handed over, so no fence is needed.
-// (One workgroup that polls all slots and answers all made the launch 0.9 us longer: 4096 x 1024 8.1 against 7.25 us.)
-// The tag is a host nonce plus a generation word that lives in the workspace and that workgroup 0
-// advances at the end of every launch: words left by an earlier launch - or by an earlier replay of
-// a recorded graph, which repeats the nonce - never match, whatever the workspace held before its
-// first use.  Every wait is bounded: a workgroup that runs out of patience (the device was shared
-// and not all workgroups were resident) takes the abs-max over the whole input itself - the
-// result is the same - clears its slot, and the launch still ends.
-__device__ __forceinline__ unsigned long long onepass_word(unsigned tag, float v) {
-  return ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v);
-}
-// m: abs-max of this workgroup's values (in every thread), tag: this launch's, G <= THREADS workgroups.  scan: the abs-max of
-// the whole input, by this workgroup alone.
-template <int THREADS, class Scan>
-__device__ __forceinline__ float onepass_exchange(float m, unsigned gen, unsigned tag, unsigned long long* slots,
-                                                  unsigned long long* gen_word, unsigned long long* boards, int spin_limit,
-                                                  int G, float* red, float* shared_max, Scan scan) {
-  const int tid = threadIdx.x, g = blockIdx.x;
-  static_assert(kOnePassMaxGroups == kOnePassBoards * kOnePassBoards, "a group's slots and a board's words are polled by the same lanes");
-  // n words from p with this launch's tag, polled by the first lanes of wave 0: their maximum, in *found whether all came
-  auto collect = [&](const unsigned long long* p, int n, bool* found) {
-    float v = 0.0f;
-    *found = false;
-    for(int spin = 0; spin < spin_limit; ++spin) {
-      const unsigned long long w = __hip_atomic_load(p + min(tid, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      v = __uint_as_float((unsigned)w);
-      *found = __all((unsigned)(w >> 32) == tag);
-      if(*found) break;
-      __builtin_amdgcn_s_sleep(1);
-    }
-    return wave_max(v);
-  };
-  if(tid < kWave) {
-    bool found = true;
-    if(tid == 0) __hip_atomic_store(&slots[g], onepass_word(tag, m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool leads = g % kOnePassBoards == 0;
-    if(leads) {
-      const float v = collect(slots + g, min(kOnePassBoards, G - g), &found);
-      if(found && tid < kOnePassBoards)
-        __hip_atomic_store(&boards[tid * kOnePassBoardWords + g / kOnePassBoards], onepass_word(tag, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    float v = 0.0f;
-    if(found) {
-      v = collect(boards + (g % kOnePassBoards) * kOnePassBoardWords, (G + kOnePassBoards - 1) / kOnePassBoards, &found);
-      // A group's words that went out behind the generation's end (below) carry the next launch's tag; the words of
-      // workgroup 0's group then never match, so they are taken back here.
-      if(leads && !found && tid < kOnePassBoards)
-        __hip_atomic_store(&boards[tid * kOnePassBoardWords + g / kOnePassBoards], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if(tid == 0) {
-      // answered or not, this launch is done with the slot
-      __hip_atomic_store(&slots[g], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      // the next launch (or replay) expects another tag; every workgroup of this launch has read
-      // the generation by now, or will find its words unanswered and help itself
-      if(g == 0) __hip_atomic_store(gen_word, (unsigned long long)(gen + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *shared_max = found ? v : -1.0f;
-    }
-  }
-  __syncthreads();
-  const float all = *shared_max;
-  return all >= 0.0f ? all : scan();
-}
-// Abs-max of n4 vectors by one workgroup (the way out of a wait that ran out).
-template <int THREADS>
-__device__ __forceinline__ float onepass_scan(const float* x, size_t n4, float* red) {
-  const v4f* x4 = reinterpret_cast<const v4f*>(x);
-  float m = 0.0f;
-  for(size_t i = threadIdx.x; i < n4; i += THREADS) m = abs4max(x4[i], m);
-  return block_max<THREADS / kWave>(m, red);
-}
-
+// In between, the workgroups exchange their abs-max (onepass_exchange.h).
 template <int SETS>
 __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __restrict__ x, unsigned n16,
                                                                  int8_t* __restrict__ out,
@@ -185,7 +110,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
 
   float amax = m;
   if(G > 1)
-    amax = onepass_exchange<1024>(m, gen, tag, slots, gen_word, boards, spin_limit, G, red, &shared_max,
+    amax = onepass_exchange<1024>((int)blockIdx.x, m, gen, tag, slots, gen_word, boards, spin_limit, G, red, &shared_max,
                                   [&] { return onepass_scan<1024>(x, (size_t)n16 * 4, red); });
   const float qm = quant_mult_from_maxabs(amax);
   const bool finite = qm < __builtin_inff();
@@ -338,7 +263,7 @@ __global__ __launch_bounds__(TILES * 256) void prepare_b_onepass_kernel(const fl
   m = block_max<TILES * 256 / kWave>(m, red);   // (its barriers also publish shared_tag)
   float amax = m;
   if(groups > 1)
-    amax = onepass_exchange<TILES * 256>(m, gen, shared_tag, slots, gen_word, boards, spin_limit, groups, red, &shared_max,
+    amax = onepass_exchange<TILES * 256>((int)blockIdx.x, m, gen, shared_tag, slots, gen_word, boards, spin_limit, groups, red, &shared_max,
                                          [&] { return onepass_scan<TILES * 256>(W, (size_t)K * N / 4, red); });
   const float qm = quant_mult_from_maxabs(amax);
   store_b_tile(v, qm, turn[sub], K, N, n0, k0, thread, live, out);

@@ -58,6 +58,25 @@ def test_affine_with_known_absmax(integer, orc, synth, M, K, N, kind):
             assert np.array_equal(short.cpu().numpy(), want[:, idx])
 
 
+@pytest.mark.parametrize("kernel", [0, 630, 702])
+@pytest.mark.parametrize("M,K,N", [(64, 2048, 8), (128, 576, 264), (64, 1024, 1024), (9, 1984, 2056), (30, 2048, 512), (128, 1088, 1000),
+                                   (113, 2048, 1024), (255, 960, 1024), (200, 2048, 1048), (250, 1216, 1000)])
+def test_affine_that_takes_its_absmax(integer, orc, synth, M, K, N, kernel):
+    """The abs-max taken by the launch that multiplies (id 630: by a launch in front; 702: every workgroup scans all activations
+    itself), at one to 256 workgroups, the largest value in the last workgroup's share; twice, since a call leaves words for the next."""
+    import contextlib
+    W, bias = synth.normal(940 + N, synth.STREAM_W, (K, N), 0.02), synth.normal(940 + N, synth.STREAM_BIAS, (N,), 0.01)
+    Bq_h, Bq = orc.prepare_b(W), integer.prepareB(upload(W))
+    with load("_lib").forced_kernel(kernel) if kernel else contextlib.nullcontext():
+        for turn in range(2):
+            A = synth.normal(940 + M + K + turn, synth.STREAM_A, (M, K), 1.0 + turn)
+            A.flat[A.size - 1 - 3 * turn] = -9.5 - turn
+            Aq_h = orc.prepare_a(A)
+            out, Aq = integer.affine_f32(upload(A), Bq, upload(bias))
+            assert np.array_equal(Aq.numpy(), Aq_h)
+            assert np.array_equal(out.cpu().numpy(), orc.affine(Aq_h, Bq_h, bias, M, K, N, 1.0, False)[0])
+
+
 @pytest.mark.parametrize("gx,gy", [(32, 8), (64, 4), (16, 5), (3, 7), (8, 1), (1, 8), (24, 3), (48, 2), (100, 2)])
 def test_tiles_are_each_taken_once(integer, synth, orc, gx, gy):
     """every split of the tiles over the XCDs: 16 (8 and 32) rows by 32 columns, one output wrong per tile missed"""
