@@ -361,8 +361,8 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
       a2.absmax_out = nullptr;
       a2.blocks_x = groups->table.block0[groups->table.n];
       MH_LAUNCH(gkernel, dim3(groups->table.block0[groups->table.n], m_tiles), dim3(Cfg::kThreads), lds, st,
-                         f.A, a2.Bq, a2.Aq, f.partials, a2.M, a2.K, a2.N, a2.n_out, f.n_partials, a2.idx ? 1 : 0, a2, f.aq_out,
-                         groups->table, NoNorm());
+                         f.A, a2.Bq, a2.Aq, f.partials, int_pair(a2.M, a2.K), int_pair(a2.N, a2.n_out),
+                         int_pair(f.n_partials, a2.idx ? 1 : 0), Stream32Rest<GroupTable, NoNorm>{a2, f.aq_out, groups->table, NoNorm()});
       MH_HIP(hipGetLastError());
       return MARIAN_HIP_OK;
     }
@@ -376,8 +376,8 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
     if((long long)blocks * m_tiles * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
     else a2.absmax_out = nullptr;
   }
-  MH_LAUNCH(kernel, dim3(blocks, m_tiles), dim3(Cfg::kThreads), lds, st, f.A, a2.Bq, a2.Aq, f.partials, a2.M, a2.K,
-                     a2.N, a2.n_out, f.n_partials, a2.idx ? 1 : 0, a2, f.aq_out, NoGroups(), NoNorm());
+  MH_LAUNCH(kernel, dim3(blocks, m_tiles), dim3(Cfg::kThreads), lds, st, f.A, a2.Bq, a2.Aq, f.partials, int_pair(a2.M, a2.K),
+            int_pair(a2.N, a2.n_out), int_pair(f.n_partials, a2.idx ? 1 : 0), Stream32Rest<NoGroups, NoNorm>{a2, f.aq_out, NoGroups(), NoNorm()});
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -395,16 +395,16 @@ int launch_normed(const GemmArgs& a, const float* A, const NormInputOf<VECS>& n,
   a2.blocks_x = groups ? groups->block0[groups->n] : (a.n_out + Cfg::kColsPerBlock - 1) / Cfg::kColsPerBlock;
   if(groups) {
     auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, GroupTable, NormInputOf<VECS>>;
-    MH_LAUNCH(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, A, a2.Bq, a2.Aq, n.add, a2.M, a2.K, a2.N, a2.n_out, 0, 0, a2,
-                       static_cast<int8_t*>(nullptr), *groups, n);
+    MH_LAUNCH(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, A, a2.Bq, a2.Aq, n.add, int_pair(a2.M, a2.K), int_pair(a2.N, a2.n_out),
+              int_pair(0, 0), Stream32Rest<GroupTable, NormInputOf<VECS>>{a2, nullptr, *groups, n});
   } else {
     auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, NoGroups, NormInputOf<VECS>>;
     if(a.absmax_out) {   // one slot per wave
       if((long long)a2.blocks_x * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
       else a2.absmax_out = nullptr;
     }
-    MH_LAUNCH(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, A, a2.Bq, a2.Aq, n.add, a2.M, a2.K, a2.N, a2.n_out, 0, 0, a2,
-                       static_cast<int8_t*>(nullptr), NoGroups(), n);
+    MH_LAUNCH(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, A, a2.Bq, a2.Aq, n.add, int_pair(a2.M, a2.K), int_pair(a2.N, a2.n_out),
+              int_pair(0, 0), Stream32Rest<NoGroups, NormInputOf<VECS>>{a2, nullptr, NoGroups(), n});
   }
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
@@ -443,8 +443,9 @@ int launch_rows(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const Grou
     if(groups->cols != 32) return MARIAN_HIP_ERR_SHAPE;   // (table built for another kernel)
     a2.stream_out = 0;
     a2.absmax_out = nullptr;
-    MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS, GroupTable>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, a2.M, a2.K,
-                       a2.N, a2.n_out, f.n_partials, tile_block, flags, a2, f.aq_out, groups->table, AbsMaxSlots());
+    MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS, GroupTable>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, int_pair(a2.M, a2.K),
+              int_pair(a2.N, a2.n_out), int_pair(f.n_partials, flags), tile_block,
+              RowsRest<GroupTable, AbsMaxSlots>{a2, f.aq_out, groups->table, AbsMaxSlots()});
   } else {
     a2.stream_out = (long long)a.M * a.n_out * 4 >= (4ll << 20) ? 1 : 0;   // (see launch_stream32)
     if(a.absmax_out) {   // one slot per wave
@@ -452,11 +453,13 @@ int launch_rows(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const Grou
       else a2.absmax_out = nullptr;
     }
     if(f.exchange)
-      MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS, NoGroups, AbsMaxExchange>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, nullptr, a2.M, a2.K,
-                         a2.N, a2.n_out, 0, tile_block, flags, a2, f.aq_out, NoGroups(), *f.exchange);
+      MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS, NoGroups, AbsMaxExchange>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, nullptr,
+                int_pair(a2.M, a2.K), int_pair(a2.N, a2.n_out), int_pair(0, flags), tile_block,
+                RowsRest<NoGroups, AbsMaxExchange>{a2, f.aq_out, NoGroups(), *f.exchange});
     else
-      MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, a2.M, a2.K, a2.N, a2.n_out,
-                         f.n_partials, tile_block, flags, a2, f.aq_out, NoGroups(), AbsMaxSlots());
+      MH_LAUNCH((gemm_rows_kernel<ROWS, STEPS>), grid, dim3(kRowsThreads), lds, st, f.A, a2.Bq, f.partials, int_pair(a2.M, a2.K),
+                int_pair(a2.N, a2.n_out), int_pair(f.n_partials, flags), tile_block,
+                RowsRest<NoGroups, AbsMaxSlots>{a2, f.aq_out, NoGroups(), AbsMaxSlots()});
   }
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;

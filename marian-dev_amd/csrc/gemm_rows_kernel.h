@@ -60,12 +60,27 @@ struct AbsMaxExchange {
 constexpr int kRowsShareVecs = 4;   // of four values, of a thread
 constexpr int kRowsShare = kRowsThreads * kRowsShareVecs * 4;
 
+// Arguments behind those that come in registers.
+template <typename GROUPS, typename ABSMAX>
+struct RowsRest {
+  GemmArgs args;
+  int8_t* aq_out;
+  GROUPS groups;
+  ABSMAX absmax;
+};
+
 // STEPS: pairs that the first waves take, ceil(K / 512); the others take one fewer.  tile_block: h | w << 16; flags: 1 with a shortlist,
 // plus 2 (shift + 1).  (The fields of args that are arguments of their own as well are those.)
 template <int ROWS, int STEPS, typename GROUPS = NoGroups, typename ABSMAX = AbsMaxSlots>
-__global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A, const int8_t* Bq, const float* partials, int M, int K, int N,
-                                                                 int n_out, int n_partials, unsigned tile_block, int flags, GemmArgs args,
-                                                                 int8_t* aq_out, GROUPS groups, ABSMAX absmax) {
+__global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A, const int8_t* Bq, const float* partials, unsigned long long M_K,
+                                                                 unsigned long long N_n_out, unsigned long long n_partials_flags,
+                                                                 unsigned tile_block, RowsRest<GROUPS, ABSMAX> rest) {
+  const int M = int_pair(M_K).first, K = int_pair(M_K).second, N = int_pair(N_n_out).first, n_out = int_pair(N_n_out).second;
+  const int n_partials = int_pair(n_partials_flags).first, flags = int_pair(n_partials_flags).second;
+  GemmArgs args = rest.args;
+  int8_t* const aq_out = rest.aq_out;
+  const GROUPS& groups = rest.groups;
+  const ABSMAX& absmax = rest.absmax;
   args.Bq = Bq; args.M = M; args.K = K; args.N = N; args.n_out = n_out;   // (what is needed first comes in registers, see the Makefile)
   constexpr bool GROUPED = std::is_same<GROUPS, GroupTable>::value, EXCHANGE = std::is_same<ABSMAX, AbsMaxExchange>::value;
   constexpr int CHUNK = rows_chunk_bytes<ROWS>(), LOADS = ROWS / 4;   // of four rows a load

@@ -67,6 +67,14 @@ struct Stream32Cfg {
 };
 
 struct NoGroups {};
+// Arguments behind those that come in registers.
+template <typename GROUPS, typename NORMED>
+struct Stream32Rest {
+  GemmArgs args;
+  int8_t* aq_out;
+  GROUPS groups;
+  NORMED norm;
+};
 
 // Dynamic LDS: one chunk (kStageBytes), for kFusedAll all of K (32 * MT32 * K bytes) if that is
 // more; at least kReduceBytes.  aux: n_partials (1..2048) abs-max values (kFusedTiled), what is added to A (kFusedNorm).  The fields of args
@@ -79,9 +87,15 @@ struct NoGroups {};
 // still takes the abs-max over all of A in every workgroup and quantizes only its own rows.
 template <int MT32, int WN, int KW, int PW, int MODE, int NG = 4, int ROWS = 32 * MT32, typename GROUPS = NoGroups, typename NORMED = NoNorm>
 __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const float* A, const int8_t* Bq, const int8_t* Aq,
-                                                                        const float* aux, int M, int K, int N, int n_out,
-                                                                        int n_partials, int shortlist, GemmArgs args,
-                                                                        int8_t* aq_out, GROUPS groups, NORMED norm) {
+                                                                        const float* aux, unsigned long long M_K, unsigned long long N_n_out,
+                                                                        unsigned long long n_partials_shortlist,
+                                                                        Stream32Rest<GROUPS, NORMED> rest) {
+  const int M = int_pair(M_K).first, K = int_pair(M_K).second, N = int_pair(N_n_out).first, n_out = int_pair(N_n_out).second;
+  const int n_partials = int_pair(n_partials_shortlist).first, shortlist = int_pair(n_partials_shortlist).second;
+  GemmArgs args = rest.args;
+  int8_t* const aq_out = rest.aq_out;
+  const GROUPS& groups = rest.groups;
+  const NORMED& norm = rest.norm;
   args.Bq = Bq; args.Aq = Aq; args.M = M; args.K = K; args.N = N; args.n_out = n_out;   // (what is needed first comes in registers, see the Makefile)
   const float* const partials = aux;
   using Cfg = Stream32Cfg<MT32, WN, KW, PW>;
