@@ -36,7 +36,7 @@
  * may overlap on the device.  What may be shared between overlapping calls and what may not:
  *   - weights, bias, shortlist ids, any input: read only, share freely;
  *   - the workspace (marian_hip_int8_workspace_bytes()): ONE PER STREAM.  It holds the abs-max
- *     partials of the call in flight and the words the workgroups of a one-pass prepareA exchange;
+ *     partials of the call in flight and the words that workgroups exchange within a launch;
  *     calls on one stream run one after the other and share it, calls on different streams must
  *     each bring their own (a backend object per worker, as in the reference, does that);
  *   - the n-best workspace of marian_hip_nbest_beams / marian_hip_logsoftmax_nbest_beams
@@ -46,8 +46,9 @@
  *   - outputs and Aq: whatever the caller's graph guarantees, the library keeps no pointer.
  * The library's own process-wide state is limited to caches that are written once per device
  * (kernel attributes, the number of compute units, the address of the static scratch) and a
- * counter for tags, all atomics; the last HIP error is kept per thread.  A one-pass prepareA
- * puts a workgroup on every compute unit; while another stream keeps compute units busy its
+ * counter for tags, all atomics; the last HIP error is kept per thread.  The launches
+ * that take an abs-max and use it (prepareA, prepareB, an affine call of 9 to 256 rows) have up to
+ * one workgroup on every compute unit; while another stream keeps compute units busy their
  * workgroups may not all be resident, their waits for one another are bounded, and the call then
  * finishes by the slower route with the same result.
  *
@@ -276,7 +277,7 @@ int marian_hip_int8_proj_attention_normed(const float* A, const marian_hip_norm_
  * (M*K + 4 bytes) and the abs-max partials live in an array of
  * MARIAN_HIP_STATIC_MAX_ELEMS + 256 + marian_hip_int8_workspace_bytes() bytes that the library
  * holds on every GPU it runs on until the process ends (16 MiB + 256 B + the 12 KB workspace).
- * The words workgroups exchange through the workspace (one-pass prepareA, M * K >= 4 Mi) persist
+ * The words workgroups exchange through the workspace (launches that take an abs-max and use it) persist
  * between calls and are told apart by tags; nothing in the array is ever cleared.  The call makes
  * no hipMalloc / hipFree and no allocating library call.  `out` is what marian_hip_int8_affine_f32 writes, bit for bit.
  *   M * K > MARIAN_HIP_STATIC_MAX_ELEMS returns MARIAN_HIP_ERR_STATIC_LIMIT (checked first).
