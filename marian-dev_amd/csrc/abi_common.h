@@ -32,19 +32,23 @@ inline int current_device(int* dev) {
   return MARIAN_HIP_OK;
 }
 
-// Launches one kernel: its function on the stream's device is looked up once and kept, which spares the host a fifth of
+// Launches KERNEL: its function on the stream's device is looked up once and kept, which spares the host a fifth of
 // a microsecond of 2.4 a launch (the runtime's table of kernels, and the launch configuration that <<<>>> hands over by a stack).
-class Launcher {
+// What is kept belongs to the kernel itself, so that no place can find the function of another one.
+template <auto KERNEL>
+class Launcher;
+template <typename... P, void (*KERNEL)(P...)>
+class Launcher<KERNEL> {
  public:
-  template <typename... P, typename... A>
-  int operator()(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, const A&... given) {
+  template <typename... A>
+  static int launch(dim3 grid, dim3 block, size_t lds, hipStream_t st, const A&... given) {
     int dev = 0;
     hipError_t e = st ? hipStreamGetDevice(st, &dev) : hipGetDevice(&dev);
     if(e != hipSuccess) return record_hip_error((int)e);
     if(dev < 0 || dev >= kMaxDevices) return MARIAN_HIP_ERR_RANGE;
     hipFunction_t f = function_[dev].load(std::memory_order_acquire);
     if(!f) {
-      e = hipGetFuncBySymbol(&f, reinterpret_cast<const void*>(kernel));
+      e = hipGetFuncBySymbol(&f, reinterpret_cast<const void*>(KERNEL));
       if(e != hipSuccess) return record_hip_error((int)e);
       function_[dev].store(f, std::memory_order_release);   // (every thread finds the same function)
     }
@@ -59,14 +63,13 @@ class Launcher {
     const hipError_t e = hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block.x, block.y, block.z, (unsigned)lds, st, arguments, nullptr);
     return e == hipSuccess ? MARIAN_HIP_OK : record_hip_error((int)e);
   }
-  std::array<std::atomic<hipFunction_t>, kMaxDevices> function_{};
+  inline static std::array<std::atomic<hipFunction_t>, kMaxDevices> function_{};
 };
-// One kernel at each place (in a template: in each instantiation); leaves the calling function with the status of a launch that failed.
-#define MH_LAUNCH(...)                                       \
-  do {                                                       \
-    static Launcher launcher_;                               \
-    const int launch_status_ = launcher_(__VA_ARGS__);       \
-    if(launch_status_ != MARIAN_HIP_OK) return launch_status_; \
+// Leaves the calling function with the status of a launch that failed.  (KERNEL: a constant; of several template arguments: in parentheses)
+#define MH_LAUNCH(KERNEL, ...)                                                       \
+  do {                                                                               \
+    const int launch_status_ = marian_hip::Launcher<KERNEL>::launch(__VA_ARGS__);    \
+    if(launch_status_ != MARIAN_HIP_OK) return launch_status_;                       \
   } while(0)
 
 // A piece of device memory (p null: none).

@@ -73,7 +73,7 @@ constexpr int64_t kMaxElems = 2147483647LL;
 template <int MT, int NT, int WN, int KW, int PF>
 int launch_stream(const GemmArgs& a, hipStream_t st) {
   using Cfg = StreamCfg<MT, NT, WN, KW, PF>;
-  auto kernel = gemm_stream_kernel<MT, NT, WN, KW, PF>;
+  constexpr auto kernel = gemm_stream_kernel<MT, NT, WN, KW, PF>;
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
@@ -99,7 +99,7 @@ int launch_big_split(const GemmArgs& a, hipStream_t st) {
   static std::atomic<uint64_t> lds_done[2];
   GemmArgs a2 = a;
   if(big_leaves_absmax(a, (long long)tiles_n * tiles_m)) {
-    auto kernel = gemm_mfma32_split_kernel<BM, BN, WM, WN, NSTAGE, NT, true>;
+    constexpr auto kernel = gemm_mfma32_split_kernel<BM, BN, WM, WN, NSTAGE, NT, true>;
     const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done[1]);
     if(lds_status != MARIAN_HIP_OK) return lds_status;
     a2.absmax_used = tiles_n * tiles_m;
@@ -108,7 +108,7 @@ int launch_big_split(const GemmArgs& a, hipStream_t st) {
     t_absmax_written = true;
     return MARIAN_HIP_OK;
   }
-  auto kernel = gemm_mfma32_split_kernel<BM, BN, WM, WN, NSTAGE, NT, false>;
+  constexpr auto kernel = gemm_mfma32_split_kernel<BM, BN, WM, WN, NSTAGE, NT, false>;
   const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done[0]);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
   MH_LAUNCH(kernel, dim3(tiles_n * tiles_m), dim3(2 * Cfg::kThreads), Cfg::kLdsBytes, st, a2, tiles_n, tiles_m);
@@ -128,7 +128,7 @@ int launch_big(const GemmArgs& a, hipStream_t st) {
     if constexpr(!Cfg::kHalfTailOk || !PAIRED) {
       return launch_big<128, 128, 2, 4, 2, true, NT>(a, st);
     } else {
-      auto half = gemm_mfma32_kernel<BM, BN, WM, WN, NSTAGE, true, NT, true>;
+      constexpr auto half = gemm_mfma32_kernel<BM, BN, WM, WN, NSTAGE, true, NT, true>;
       static std::atomic<uint64_t> half_lds_done{0};
       const int half_lds_status = allow_lds(half, Cfg::kLdsBytes, half_lds_done);
       if(half_lds_status != MARIAN_HIP_OK) return half_lds_status;
@@ -140,7 +140,7 @@ int launch_big(const GemmArgs& a, hipStream_t st) {
   }
   if constexpr(PAIRED) {
     if(big_leaves_absmax(a, (long long)tiles_n * tiles_m)) {
-      auto kernel = gemm_mfma32_kernel<BM, BN, WM, WN, NSTAGE, true, NT, false, true>;
+      constexpr auto kernel = gemm_mfma32_kernel<BM, BN, WM, WN, NSTAGE, true, NT, false, true>;
       static std::atomic<uint64_t> amax_lds_done{0};
       const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, amax_lds_done);
       if(lds_status != MARIAN_HIP_OK) return lds_status;
@@ -152,7 +152,7 @@ int launch_big(const GemmArgs& a, hipStream_t st) {
       return MARIAN_HIP_OK;
     }
   }
-  auto kernel = gemm_mfma32_kernel<BM, BN, WM, WN, NSTAGE, PAIRED, NT>;
+  constexpr auto kernel = gemm_mfma32_kernel<BM, BN, WM, WN, NSTAGE, PAIRED, NT>;
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, Cfg::kLdsBytes, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
@@ -221,7 +221,7 @@ int launch_big_ragged_as(const GemmArgs& a, const Ragged& r, hipStream_t st) {
   using RCfg = BigCfg<128, 64, RWM, RWN, RS>;
   constexpr int lds = Cfg::kLdsBytes > ECfg::kLdsBytes ? (Cfg::kLdsBytes > RCfg::kLdsBytes ? Cfg::kLdsBytes : RCfg::kLdsBytes)
                                                        : (ECfg::kLdsBytes > RCfg::kLdsBytes ? ECfg::kLdsBytes : RCfg::kLdsBytes);
-  auto kernel = gemm_mfma32_ragged_kernel<BM, BN, WM, WN, NSTAGE, 64, 128, EWM, EWN, ES, 128, 64, RWM, RWN, RS, NT, AMAX>;
+  constexpr auto kernel = gemm_mfma32_ragged_kernel<BM, BN, WM, WN, NSTAGE, 64, 128, EWM, EWN, ES, 128, 64, RWM, RWN, RS, NT, AMAX>;
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, lds, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
@@ -253,7 +253,7 @@ inline bool pair_kernel_fits(const GemmArgs& a) {
 
 template <bool NT, bool AMAX>
 int launch_pair_as(const GemmArgs& a, hipStream_t st) {
-  auto kernel = gemm_pair_kernel<NT, AMAX>;
+  constexpr auto kernel = gemm_pair_kernel<NT, AMAX>;
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, PairCfg::kLdsBytes, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
@@ -281,7 +281,7 @@ int launch_pair_ragged_as(const GemmArgs& a, const Ragged& r, hipStream_t st) {
   using RCfg = BigCfg<128, 64, 2, 2, 3>;
   constexpr int lds = PairCfg::kLdsBytes > ECfg::kLdsBytes ? (PairCfg::kLdsBytes > RCfg::kLdsBytes ? PairCfg::kLdsBytes : RCfg::kLdsBytes)
                                                            : (ECfg::kLdsBytes > RCfg::kLdsBytes ? ECfg::kLdsBytes : RCfg::kLdsBytes);
-  auto kernel = gemm_pair_ragged_kernel<NT, AMAX>;
+  constexpr auto kernel = gemm_pair_ragged_kernel<NT, AMAX>;
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, lds, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
@@ -336,7 +336,7 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
       return launch_stream32<MT32, WN, KW, PW, MODE, ROWS, 2>(a, f, st);
   }
   using Cfg = Stream32Cfg<MT32, WN, KW, PW>;
-  auto kernel = gemm_stream32_kernel<MT32, WN, KW, PW, MODE, NG, ROWS>;
+  constexpr auto kernel = gemm_stream32_kernel<MT32, WN, KW, PW, MODE, NG, ROWS>;
   constexpr int kMaxLds = 64 * 1024 > Cfg::kLdsBytes ? 64 * 1024 : Cfg::kLdsBytes;
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, kMaxLds, lds_done);
@@ -353,7 +353,7 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
   if constexpr(MODE == kFusedTiled) {
     if(groups) {
       if(groups->cols != Cfg::kColsPerBlock) return MARIAN_HIP_ERR_SHAPE;   // (table built for another kernel)
-      auto gkernel = gemm_stream32_kernel<MT32, WN, KW, PW, MODE, NG, ROWS, GroupTable>;
+      constexpr auto gkernel = gemm_stream32_kernel<MT32, WN, KW, PW, MODE, NG, ROWS, GroupTable>;
       static std::atomic<uint64_t> glds_done{0};
       const int glds_status = allow_lds(gkernel, kMaxLds, glds_done);
       if(glds_status != MARIAN_HIP_OK) return glds_status;
@@ -394,11 +394,11 @@ int launch_normed(const GemmArgs& a, const float* A, const NormInputOf<VECS>& n,
   a2.blocks_y = 1;
   a2.blocks_x = groups ? groups->block0[groups->n] : (a.n_out + Cfg::kColsPerBlock - 1) / Cfg::kColsPerBlock;
   if(groups) {
-    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, GroupTable, NormInputOf<VECS>>;
+    constexpr auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, GroupTable, NormInputOf<VECS>>;
     MH_LAUNCH(kernel, dim3(a2.blocks_x), dim3(Cfg::kThreads), lds, st, A, a2.Bq, a2.Aq, n.add, int_pair(a2.M, a2.K), int_pair(a2.N, a2.n_out),
               int_pair(0, 0), Stream32Rest<GroupTable, NormInputOf<VECS>>{a2, nullptr, *groups, n});
   } else {
-    auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, NoGroups, NormInputOf<VECS>>;
+    constexpr auto kernel = gemm_stream32_kernel<1, WN, KW, PW, kFusedNorm, 4, 16, NoGroups, NormInputOf<VECS>>;
     if(a.absmax_out) {   // one slot per wave
       if((long long)a2.blocks_x * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
       else a2.absmax_out = nullptr;
@@ -796,12 +796,13 @@ GroupTable group_table(int64_t n_groups, const int8_t* const* Bq, const float* c
 //    1400 x 1024 x 3072 11.6; three launches 14.8 and 16.9);
 //  - fewer: 128x64 tiles in the split form, which CUs that idle leave room for (1000 x 512 x 1536 5.1 us,
 //    600 x 1024 x 3072 6.0; three launches 13.9 and 16.3).
-template <typename CFG, int THREADS, typename KERNEL>
-int launch_grouped_as(KERNEL kernel, const GemmArgs& a, const GroupTable& g, int tiles_m, std::atomic<uint64_t>& lds_done, hipStream_t st) {
-  const int lds_status = allow_lds(kernel, CFG::kLdsBytes, lds_done);
+template <typename CFG, int THREADS, auto KERNEL>
+int launch_grouped_as(const GemmArgs& a, const GroupTable& g, int tiles_m, hipStream_t st) {
+  static std::atomic<uint64_t> lds_done{0};
+  const int lds_status = allow_lds(KERNEL, CFG::kLdsBytes, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
   const int tiles_n = g.block0[g.n];
-  MH_LAUNCH(kernel, dim3(tiles_n * tiles_m), dim3(THREADS), CFG::kLdsBytes, st, a, g, tiles_n, tiles_m);
+  MH_LAUNCH(KERNEL, dim3(tiles_n * tiles_m), dim3(THREADS), CFG::kLdsBytes, st, a, g, tiles_n, tiles_m);
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }
@@ -816,19 +817,18 @@ int launch_big_grouped(const GemmArgs& a, int64_t n_groups, const int8_t* const*
   }
   tiles128 *= (a.M + 127) / 128;
   const bool stream_out = (long long)a.M * columns * 4 <= (32ll << 20);   // (as for a single matrix)
-  static std::atomic<uint64_t> lds_done[4];
   if(pairs && (a.M / 256) * (columns / 256) >= 192)
-    return launch_grouped_as<PairCfg, PairCfg::kThreads>(gemm_pair_group_kernel<true>, a, group_table(n_groups, Bq, bias, out, N, 2 * PairCfg::BN),
-                                                        a.M / PairCfg::BM, lds_done[0], st);
+    return launch_grouped_as<PairCfg, PairCfg::kThreads, gemm_pair_group_kernel<true>>(
+        a, group_table(n_groups, Bq, bias, out, N, 2 * PairCfg::BN), a.M / PairCfg::BM, st);
   if(tiles128 >= compute_units()) {
     using Cfg = BigCfg<128, 128, 2, 4, 2>;
     const GroupTable t = group_table(n_groups, Bq, bias, out, N, 128);
-    if(stream_out) return launch_grouped_as<Cfg, Cfg::kThreads>(gemm_mfma32_group_kernel<128, 128, 2, 4, 2, true, false>, a, t, (a.M + 127) / 128, lds_done[1], st);
-    return launch_grouped_as<Cfg, Cfg::kThreads>(gemm_mfma32_group_kernel<128, 128, 2, 4, 2, false, false>, a, t, (a.M + 127) / 128, lds_done[2], st);
+    if(stream_out) return launch_grouped_as<Cfg, Cfg::kThreads, gemm_mfma32_group_kernel<128, 128, 2, 4, 2, true, false>>(a, t, (a.M + 127) / 128, st);
+    return launch_grouped_as<Cfg, Cfg::kThreads, gemm_mfma32_group_kernel<128, 128, 2, 4, 2, false, false>>(a, t, (a.M + 127) / 128, st);
   }
   using Cfg = BigCfg<128, 64, 2, 2, 3>;
-  return launch_grouped_as<Cfg, 2 * Cfg::kThreads>(gemm_mfma32_group_kernel<128, 64, 2, 2, 3, true, true>, a,
-                                                   group_table(n_groups, Bq, bias, out, N, 64), (a.M + 127) / 128, lds_done[3], st);
+  return launch_grouped_as<Cfg, 2 * Cfg::kThreads, gemm_mfma32_group_kernel<128, 64, 2, 2, 3, true, true>>(
+      a, group_table(n_groups, Bq, bias, out, N, 64), (a.M + 127) / 128, st);
 }
 
 int check_gemm(const int8_t* Aq, const int8_t* Bq, const void* out, const float* bias,

@@ -2500,7 +2500,7 @@ static int attention_impl(const float* q, float* k, float* v, const float* mask,
 }  // extern "C"
 template <int NPROJ, int R, int SEGS, int PASSES, int PW, int HELD, bool NORM, bool ANC>
 static int launch_proj(const ProjAttentionArgs& p, dim3 grid, size_t lds, hipStream_t st) {
-  auto kernel = proj_attention_kernel<NPROJ, R, SEGS, PASSES, PW, HELD, NORM, ANC>;
+  constexpr auto kernel = proj_attention_kernel<NPROJ, R, SEGS, PASSES, PW, HELD, NORM, ANC>;
   static std::atomic<uint64_t> lds_done{0};
   const int lst = allow_lds(kernel, SEGS > 0 ? kProjMaxLds : 96 * 1024, lds_done);
   if(lst != MARIAN_HIP_OK) return lst;

@@ -597,7 +597,7 @@ template <typename AT, int BM, int BN, int WM, int WN, bool DUMP>
 int launch_tile16(const Gemm16Args& g, hipStream_t st) {
   const int tiles_n = (g.N + BN - 1) / BN, tiles_m = (g.M + BM - 1) / BM;
   constexpr int lds = tile16_lds<BM, BN>();
-  auto kernel = gemm16_tile_kernel<AT, BM, BN, WM, WN, DUMP>;
+  constexpr auto kernel = gemm16_tile_kernel<AT, BM, BN, WM, WN, DUMP>;
   static std::atomic<uint64_t> lds_done{0};
   const int lds_status = allow_lds(kernel, lds, lds_done);
   if(lds_status != MARIAN_HIP_OK) return lds_status;
