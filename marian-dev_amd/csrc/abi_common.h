@@ -32,6 +32,50 @@ inline int current_device(int* dev) {
   return MARIAN_HIP_OK;
 }
 
+// Whether there is only one device: then nobody has to be asked which one a stream is of, or is current.
+inline bool one_device() {
+  static std::atomic<int> devices{0};
+  int n = devices.load(std::memory_order_relaxed);
+  if(n == 0 && hipGetDeviceCount(&n) == hipSuccess) devices.store(n, std::memory_order_relaxed);
+  return n == 1;
+}
+
+// The device that work on `stream` runs on: of the default streams the current one.
+inline int stream_device(hipStream_t stream, int* dev) {
+  if(one_device()) {
+    *dev = 0;
+    return MARIAN_HIP_OK;
+  }
+  if(!stream || stream == hipStreamLegacy || stream == hipStreamPerThread) return current_device(dev);
+  hipDevice_t d = 0;
+  const hipError_t e = hipStreamGetDevice(stream, &d);
+  if(e != hipSuccess) return record_hip_error((int)e);
+  if(d < 0 || d >= kMaxDevices) return MARIAN_HIP_ERR_RANGE;
+  *dev = d;
+  return MARIAN_HIP_OK;
+}
+
+// Makes `dev` the thread's device until the end of the scope, if it is another one.
+class OnDevice {
+ public:
+  explicit OnDevice(int dev) : status(MARIAN_HIP_OK) {
+    if(one_device()) return;
+    status = current_device(&before_);
+    if(status != MARIAN_HIP_OK || before_ == dev) return;
+    const hipError_t e = hipSetDevice(dev);
+    if(e != hipSuccess) status = record_hip_error((int)e);
+    else moved_ = true;
+  }
+  ~OnDevice() { if(moved_) (void)hipSetDevice(before_); }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+  int status;
+
+ private:
+  int before_ = 0;
+  bool moved_ = false;
+};
+
 // Launches KERNEL: its function on the stream's device is looked up once and kept, which spares the host a fifth of
 // a microsecond of 2.4 a launch (the runtime's table of kernels, and the launch configuration that <<<>>> hands over by a stack).
 // What is kept belongs to the kernel itself, so that no place can find the function of another one.
@@ -43,12 +87,13 @@ class Launcher<KERNEL> {
   template <typename... A>
   static int launch(dim3 grid, dim3 block, size_t lds, hipStream_t st, const A&... given) {
     int dev = 0;
-    hipError_t e = st ? hipStreamGetDevice(st, &dev) : hipGetDevice(&dev);
-    if(e != hipSuccess) return record_hip_error((int)e);
-    if(dev < 0 || dev >= kMaxDevices) return MARIAN_HIP_ERR_RANGE;
+    const int status = stream_device(st, &dev);
+    if(status != MARIAN_HIP_OK) return status;
+    const OnDevice on(dev);   // (a symbol's function is that of the thread's device)
+    if(on.status != MARIAN_HIP_OK) return on.status;
     hipFunction_t f = function_[dev].load(std::memory_order_acquire);
     if(!f) {
-      e = hipGetFuncBySymbol(&f, reinterpret_cast<const void*>(KERNEL));
+      const hipError_t e = hipGetFuncBySymbol(&f, reinterpret_cast<const void*>(KERNEL));
       if(e != hipSuccess) return record_hip_error((int)e);
       function_[dev].store(f, std::memory_order_release);   // (every thread finds the same function)
     }
