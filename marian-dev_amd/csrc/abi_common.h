@@ -76,6 +76,12 @@ class OnDevice {
   bool moved_ = false;
 };
 
+// The status of a launch that the runtime refused: the error is this call's, and not left for the next one that asks for the last.
+inline int refused_launch(hipError_t e) {
+  (void)hipGetLastError();
+  return record_hip_error((int)e);
+}
+
 // Launches KERNEL: its function on the stream's device is looked up once and kept, which spares the host a fifth of
 // a microsecond of 2.4 a launch (the runtime's table of kernels, and the launch configuration that <<<>>> hands over by a stack).
 // What is kept belongs to the kernel itself, so that no place can find the function of another one.
@@ -94,7 +100,7 @@ class Launcher<KERNEL> {
     hipFunction_t f = function_[dev].load(std::memory_order_acquire);
     if(!f) {
       const hipError_t e = hipGetFuncBySymbol(&f, reinterpret_cast<const void*>(KERNEL));
-      if(e != hipSuccess) return record_hip_error((int)e);
+      if(e != hipSuccess) return refused_launch(e);
       function_[dev].store(f, std::memory_order_release);   // (every thread finds the same function)
     }
     std::tuple<P...> values(static_cast<P>(given)...);
@@ -106,7 +112,7 @@ class Launcher<KERNEL> {
   static int launch(hipFunction_t f, dim3 grid, dim3 block, size_t lds, hipStream_t st, Values& values, std::index_sequence<I...>) {
     void* arguments[] = {&std::get<I>(values)...};
     const hipError_t e = hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block.x, block.y, block.z, (unsigned)lds, st, arguments, nullptr);
-    return e == hipSuccess ? MARIAN_HIP_OK : record_hip_error((int)e);
+    return e == hipSuccess ? MARIAN_HIP_OK : refused_launch(e);
   }
   inline static std::array<std::atomic<hipFunction_t>, kMaxDevices> function_{};
 };

@@ -16,7 +16,8 @@ struct Launch {
   const Function* function;
   int argument, current;   // current: the device the launch was made on
 };
-int g_current = 0, g_devices = 2;
+int g_current = 0, g_devices = 2, g_recorded = 0;
+hipError_t g_refuse = hipSuccess, g_last = hipSuccess;
 const hipStream_t kStreamOfOne = reinterpret_cast<hipStream_t>(0x1000);   // a stream of device 1 (the others: of device 0)
 std::vector<Function*> g_functions;
 std::vector<Launch> g_launches;
@@ -47,16 +48,27 @@ hipError_t hipGetFuncBySymbol(hipFunction_t* f, const void* symbol) {
 }
 hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, hipStream_t,
                                  void** arguments, void**) {
+  if(g_refuse != hipSuccess) {
+    g_last = g_refuse;
+    return g_refuse;
+  }
   g_launches.push_back(Launch{reinterpret_cast<Function*>(f), *static_cast<int*>(arguments[0]), g_current});
   return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {   // the last error since it was asked for
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
 hipError_t hipDeviceGetAttribute(int*, hipDeviceAttribute_t, int) { return hipSuccess; }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
 }
 
 namespace marian_hip {
-int record_hip_error(int) { return MARIAN_HIP_ERR_HIP; }
+int record_hip_error(int e) {
+  g_recorded = e;
+  return MARIAN_HIP_ERR_HIP;
+}
 }
 
 namespace {
@@ -114,12 +126,24 @@ void device_of_the_stream(int first_current) {
     }
   g_current = 0;
 }
+
+// A launch that the runtime refuses is reported by its own call, and by no later one.
+template <int N>
+void third(int) { g_failures += N; }
+void refused_once() {
+  g_refuse = hipErrorInvalidConfiguration;
+  expect(launch_one<third<3>>(0, nullptr) == MARIAN_HIP_ERR_HIP && g_recorded == hipErrorInvalidConfiguration, "a refused launch is reported");
+  g_refuse = hipSuccess;
+  expect(launch_one<third<3>>(0, nullptr) == MARIAN_HIP_OK, "the next launch");
+  expect(hipGetLastError() == hipSuccess, "no error left for the next call");
+}
 }  // namespace
 
 int main() {
   each_kernel_its_own();
   device_of_the_stream<1>(0);
   device_of_the_stream<2>(1);
+  refused_once();
   if(g_failures) return 1;
   std::printf("ok\n");
   return 0;
