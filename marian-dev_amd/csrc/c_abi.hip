@@ -863,11 +863,8 @@ int run_gemm(const int8_t* Aq, const int8_t* Bq, const float* bias, const uint32
   return launch_gemm(a, reinterpret_cast<hipStream_t>(stream));
 }
 
-// One-pass forms: how long a workgroup polls before it helps itself (each poll is a memory round trip of about half a
-// microsecond: 2 ms, where a launch that has the chip waits for 2 us and one that shares it with other streams may find that
-// its last workgroups have to wait for theirs), and the nonce that starts their tags (random per process, so that words left in recycled device
-// memory by another process do not match).
-constexpr int kOnePassSpinLimit = 4000;
+// The nonce that starts the tags of a one-pass launch (random per process, so that words left in recycled device memory by another
+// process do not match).
 unsigned next_nonce() {
   static std::atomic<unsigned> nonce{(unsigned)std::random_device{}() | 1u};
   return nonce.fetch_add(0x9E3779B1u, std::memory_order_relaxed);
@@ -883,12 +880,12 @@ bool rows_can_exchange(int M, int K, int n_out, int kw_override) {
   return plan.kw == 8 && K <= 2048 && groups <= cus && (long long)M * K <= groups * kRowsShare;
 }
 
-// The words of a workspace through which the workgroups of a one-pass launch exchange their abs-max.
+// The words of a workspace through which the workgroups of a one-pass launch exchange the abs-max of so many values.
 using OnePass = AbsMaxExchange;
-OnePass onepass_words(void* workspace, bool no_patience) {
+OnePass onepass_words(void* workspace, size_t values, bool no_patience) {
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
   return {reinterpret_cast<unsigned long long*>(ws + kOnePassSlotsOffset), reinterpret_cast<unsigned long long*>(ws + kOnePassGenOffset),
-          reinterpret_cast<unsigned long long*>(ws + kOnePassBoardOffset), next_nonce(), no_patience ? 0 : kOnePassSpinLimit};
+          reinterpret_cast<unsigned long long*>(ws + kOnePassBoardOffset), next_nonce(), no_patience ? 0 : onepass_polls(values)};
 }
 
 int absmax_blocks(size_t n4) {
@@ -1039,10 +1036,10 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
     const size_t groups = (n16 + 1024 * (size_t)sets - 1) / (1024 * (size_t)sets);
     const bool fits = groups <= (size_t)cus;
     if(fits && ov != 700) {
-      const OnePass o = onepass_words(workspace, ov == 702);
+      const OnePass o = onepass_words(workspace, n, ov == 702);
 #define MH_ONEPASS(SETS)                                                                                                       \
   MH_LAUNCH(prepare_a_onepass_kernel<SETS>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.boards, \
-            o.nonce, o.spins, (int)groups)
+            o.nonce, o.polls, (int)groups)
       switch(sets) {
         case 1: MH_ONEPASS(1); break;
         case 2: MH_ONEPASS(2); break;
@@ -1076,14 +1073,14 @@ int marian_hip_int8_prepare_b(const float* W, int8_t* Bq, int64_t K, int64_t N, 
   const long long tiles_n = (N + 63) / 64, tiles = tiles_n * (K / 64);
   const long long cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
   if(tiles <= 4 * cus && ov != 700 && aligned(workspace, 8)) {
-    const OnePass o = onepass_words(workspace, ov == 702);
+    const OnePass o = onepass_words(workspace, n, ov == 702);
     const int per = tiles <= cus ? 1 : tiles <= 2 * cus ? 2 : 4, groups = (int)((tiles + per - 1) / per);
     if(per == 1)
-      MH_LAUNCH(prepare_b_onepass_kernel<1>, dim3(groups), dim3(256), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<1>, dim3(groups), dim3(256), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
     else if(per == 2)
-      MH_LAUNCH(prepare_b_onepass_kernel<2>, dim3(groups), dim3(512), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<2>, dim3(groups), dim3(512), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
     else
-      MH_LAUNCH(prepare_b_onepass_kernel<4>, dim3(groups), dim3(1024), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.spins, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<4>, dim3(groups), dim3(1024), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
   }
@@ -1174,7 +1171,7 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
       f.partials = absmax_in;
       f.n_partials = kAbsmaxSlots;
     } else if(which != 630 && rows_can_exchange((int)M, (int)K, (int)n_out, want_tiled ? which - 620 : 0) && aligned(workspace, 8)) {
-      const OnePass o = onepass_words(workspace, which == 702);
+      const OnePass o = onepass_words(workspace, (size_t)M * (size_t)K, which == 702);
       f.exchange = &o;
       return launch_stream32_auto<kFusedTiled>(a, f, hst, want_tiled ? which - 620 : 0);
     } else {

@@ -55,7 +55,7 @@ struct AbsMaxSlots {};
 struct AbsMaxExchange {
   unsigned long long *slots, *gen, *boards;
   unsigned nonce;
-  int spins;
+  int polls;
 };
 constexpr int kRowsShareVecs = 4;   // of four values, of a thread
 constexpr int kRowsShare = kRowsThreads * kRowsShareVecs * 4;
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
       amax = block_max<kRowsWaves>(amax, red);
       if(blocks > 1)
         amax = onepass_exchange<kRowsThreads>(block, amax, gen, (absmax.nonce + gen) | 0x80000000u, absmax.slots, absmax.gen, absmax.boards,
-                                              absmax.spins, blocks, red, &red[kRowsWaves],
+                                              absmax.polls, blocks, red, &red[kRowsWaves],
                                               [&] { return onepass_scan<kRowsThreads>(A, (size_t)M * K / 4, red); });
     } else {
 #pragma unroll

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "int8_common.h"
+#include "onepass_patience.h"
 #include "quantize_common.h"
 
 namespace marian_hip {
@@ -17,8 +18,8 @@ namespace marian_hip {
 // The tag is a host nonce plus a generation word that lives in the workspace and that workgroup 0
 // advances at the end of every launch: words left by an earlier launch - or by an earlier replay of
 // a recorded graph, which repeats the nonce - never match, whatever the workspace held before its
-// first use.  Every wait is bounded: a workgroup that runs out of patience (the device was shared
-// and not all workgroups were resident) takes the abs-max over the whole input itself - the
+// first use.  Every wait is bounded, and a workgroup's waits together are (onepass_patience.h): one that runs out of patience (the
+// device was shared and not all workgroups were resident) takes the abs-max over the whole input itself - the
 // result is the same - clears its slot, and the launch still ends.
 __device__ __forceinline__ unsigned long long onepass_word(unsigned tag, float v) {
   return ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v);
@@ -27,21 +28,21 @@ __device__ __forceinline__ unsigned long long onepass_word(unsigned tag, float v
 // word as it was (in thread 0).  scan: the abs-max of the whole input, by this workgroup alone.
 template <int THREADS, class Scan>
 __device__ __forceinline__ float onepass_exchange(int g, float m, unsigned gen, unsigned tag, unsigned long long* slots,
-                                                  unsigned long long* gen_word, unsigned long long* boards, int spin_limit,
+                                                  unsigned long long* gen_word, unsigned long long* boards, int polls,
                                                   int G, float* red, float* shared_max, Scan scan) {
   const int tid = threadIdx.x;
   static_assert(kOnePassMaxGroups == kOnePassBoards * kOnePassBoards, "a group's slots and a board's words are polled by the same lanes");
+  int polls_left = polls;   // (of the whole workgroup: only its first wave waits)
   // n words from p with this launch's tag, polled by the first lanes of wave 0: their maximum, in *found whether all came
   auto collect = [&](const unsigned long long* p, int n, bool* found) {
     float v = 0.0f;
-    *found = false;
-    for(int spin = 0; spin < spin_limit; ++spin) {
+    *found = onepass_wait(polls_left, [&] {
       const unsigned long long w = __hip_atomic_load(p + min(tid, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       v = __uint_as_float((unsigned)w);
-      *found = __all((unsigned)(w >> 32) == tag);
-      if(*found) break;
-      __builtin_amdgcn_s_sleep(1);
-    }
+      const bool all = __all((unsigned)(w >> 32) == tag);
+      if(!all) __builtin_amdgcn_s_sleep(1);
+      return all;
+    });
     return wave_max(v);
   };
   if(tid < kWave) {

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
                                                                  unsigned long long* slots,
                                                                  unsigned long long* gen_word,
                                                                  unsigned long long* boards,
-                                                                 unsigned nonce, int spin_limit, int groups) {
+                                                                 unsigned nonce, int polls, int groups) {
   __shared__ float red[1024 / kWave];
   __shared__ float shared_max;
   __shared__ unsigned shared_tag;
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
 
   float amax = m;
   if(G > 1)
-    amax = onepass_exchange<1024>((int)blockIdx.x, m, gen, tag, slots, gen_word, boards, spin_limit, G, red, &shared_max,
+    amax = onepass_exchange<1024>((int)blockIdx.x, m, gen, tag, slots, gen_word, boards, polls, G, red, &shared_max,
                                   [&] { return onepass_scan<1024>(x, (size_t)n16 * 4, red); });
   const float qm = quant_mult_from_maxabs(amax);
   const bool finite = qm < __builtin_inff();
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(TILES * 256) void prepare_b_onepass_kernel(const fl
                                                                         int8_t* __restrict__ out, unsigned long long* slots,
                                                                         unsigned long long* gen_word,
                                                                         unsigned long long* boards, unsigned nonce,
-                                                                        int spin_limit, int groups, int tiles_n, int tiles) {
+                                                                        int polls, int groups, int tiles_n, int tiles) {
   __shared__ float red[TILES * 256 / kWave];
   __shared__ float shared_max;
   __shared__ unsigned shared_tag;
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(TILES * 256) void prepare_b_onepass_kernel(const fl
   m = block_max<TILES * 256 / kWave>(m, red);   // (its barriers also publish shared_tag)
   float amax = m;
   if(groups > 1)
-    amax = onepass_exchange<TILES * 256>((int)blockIdx.x, m, gen, shared_tag, slots, gen_word, boards, spin_limit, groups, red, &shared_max,
+    amax = onepass_exchange<TILES * 256>((int)blockIdx.x, m, gen, shared_tag, slots, gen_word, boards, polls, groups, red, &shared_max,
                                          [&] { return onepass_scan<TILES * 256>(W, (size_t)K * N / 4, red); });
   const float qm = quant_mult_from_maxabs(amax);
   store_b_tile(v, qm, turn[sub], K, N, n0, k0, thread, live, out);
