@@ -872,12 +872,24 @@ unsigned next_nonce() {
 
 // Whether the workgroups of gemm_rows_kernel take the abs-max of the activations themselves: one to a CU, a share of the
 // activations that a thread holds in a few registers, and rows of up to 2048 values (100 x 4096 x 1024 9.5 us that way, with a
-// launch in front 9.1; 40 x 3072 x 768 7.3 and 7.0).  (Measurement ids: 630 the launch in front; 702 no patience.)
+// launch in front 9.1; 40 x 3072 x 768 7.3 and 7.0).  The exchange takes the GPU longer than a launch in front - 64 x 1024 x 1024 in a
+// graph 5.92 and 5.42 us, 256 x 512 x 512 6.14 and 5.36, 256 x 1024 x 1000 7.44 and 6.87, at 26 of 48 sizes 4 % or more, at four 2 - 5 %
+// less (32 x 2048 x 512 5.91 and 6.20) - and spares the host a launch of 2.2: launched one by one from C++ the same calls take 5.84 and 7.38,
+// 6.40 and 7.24, 7.46 and 7.42 (at worst 128 x 1088 x 640 7.06 and 6.84), from Python more of that or less with the host.  So calls
+// that are being recorded have the launch in front.  (Measurement ids: 630 the launch in front; 702 no patience.)
 bool rows_can_exchange(int M, int K, int n_out, int kw_override) {
   const TiledPlan plan = plan_tiled(M, K, n_out, kw_override);
   const long long groups = ((n_out + 31) / 32) * (long long)((M + plan.rows - 1) / plan.rows);
   const int cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
   return plan.kw == 8 && K <= 2048 && groups <= cus && (long long)M * K <= groups * kRowsShare;
+}
+
+// Whether calls on the stream are recorded into a graph instead of being launched.
+bool recorded(hipStream_t st) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if(hipStreamIsCapturing(st, &status) == hipSuccess) return status == hipStreamCaptureStatusActive;
+  (void)hipGetLastError();   // (the launch will tell)
+  return false;
 }
 
 // The words of a workspace through which the workgroups of a one-pass launch exchange the abs-max of so many values.
@@ -1170,7 +1182,8 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
     if(absmax_in) {   // the producer of A left its abs-max: no launch for it
       f.partials = absmax_in;
       f.n_partials = kAbsmaxSlots;
-    } else if(which != 630 && rows_can_exchange((int)M, (int)K, (int)n_out, want_tiled ? which - 620 : 0) && aligned(workspace, 8)) {
+    } else if(which != 630 && rows_can_exchange((int)M, (int)K, (int)n_out, want_tiled ? which - 620 : 0) && aligned(workspace, 8) &&
+              !recorded(hst)) {
       const OnePass o = onepass_words(workspace, (size_t)M * (size_t)K, which == 702);
       f.exchange = &o;
       return launch_stream32_auto<kFusedTiled>(a, f, hst, want_tiled ? which - 620 : 0);
