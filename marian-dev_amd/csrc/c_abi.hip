@@ -410,21 +410,6 @@ int launch_normed(const GemmArgs& a, const float* A, const NormInputOf<VECS>& n,
   return MARIAN_HIP_OK;
 }
 
-// The tiles of a launch of gx x gy workgroups, dealt out so that the XCDs' L2 caches fetch the fewest bytes (as they come where
-// the tiles don't divide into eight blocks).
-inline RowsTiles rows_tiles(int gx, int gy, long long row_bytes, long long column_bytes) {
-  RowsTiles best{-1, 0, 0};
-  long long least = 0;
-  for(int shift = 0; shift <= 3; ++shift) {
-    const int r = 1 << shift;
-    if(gy % r != 0 || gx % (8 / r) != 0) continue;
-    const RowsTiles t{shift, gy / r, gx / (8 / r)};
-    const long long bytes = t.h * row_bytes + t.w * column_bytes;
-    if(best.shift < 0 || bytes < least) { best = t; least = bytes; }
-  }
-  return best;
-}
-
 // The form that quantizes on the way, every wave for itself: 32 columns and ROWS rows per workgroup, STEPS pairs of K
 // sub-steps to a wave.
 template <int ROWS, int STEPS>

@@ -20,27 +20,13 @@
 
 namespace marian_hip {
 
-constexpr int kRowsWaves = 8, kRowsThreads = kRowsWaves * kWave;
+constexpr int kRowsThreads = kRowsWaves * kWave;
 // LDS of a wave: the four 16-value chunks of a pair, 16 bytes a row; the padding spreads the dwords of four rows over the banks
 template <int ROWS>
 constexpr int rows_chunk_bytes() { return ROWS * 16 + 64; }
 template <int ROWS>
 constexpr int rows_lds_bytes() {   // the staging, or the partial sums
   return kRowsWaves * (ROWS * 128 > 4 * rows_chunk_bytes<ROWS>() ? ROWS * 128 : 4 * rows_chunk_bytes<ROWS>());
-}
-
-// Which tile a workgroup of gx x gy takes.  Workgroups are dealt out to the eight XCDs in turn; a split of r = 1 << shift (r divides gy,
-// 8 / r divides gx) is launched as 8 x h x w workgroups, h = gy / r, w = gx r / 8, and gives each XCD a block of h x w tiles, so
-// that its L2 fetches fewer operands.  shift < 0: launched as gx x gy.
-struct RowsTiles {
-  int shift, h, w;
-};
-struct RowsTile {
-  int bx, by;
-};
-__host__ __device__ __forceinline__ RowsTile rows_tile(RowsTiles t, int x, int y, int z) {
-  if(t.shift < 0) return RowsTile{x, y};
-  return RowsTile{(x >> t.shift) * t.w + z, (x & ((1 << t.shift) - 1)) * t.h + y};
 }
 
 // pairs of a wave that are on their way at a time, as registers allow
@@ -119,7 +105,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     if(wave == 0) gen = (unsigned)__hip_atomic_load(absmax.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int n4 = M * K / 4, each = (n4 + blocks - 1) / blocks;   // (past the share: the tensor's last values, again)
 #pragma unroll
-    for(int i = 0; i < kRowsShareVecs; ++i) share[i] = reinterpret_cast<const v4f*>(A)[min(block * each + min(tid + i * kRowsThreads, each - 1), n4 - 1)];
+    for(int i = 0; i < kRowsShareVecs; ++i) share[i] = reinterpret_cast<const v4f*>(A)[rows_share_vec(block, each, i, tid, kRowsThreads, n4)];
   } else {
 #pragma unroll
     for(int i = 0; i < kAbsmaxSlots / kRowsThreads; ++i) pm[i] = partials[min(tid + i * kRowsThreads, n_partials - 1)];
@@ -127,9 +113,9 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
 
   // lane: value group v (four values) of row 4 j + lane / 16 of load j
   const int v = lane % 16;
-  unsigned a_off[LOADS];   // bytes from A (M * K <= 2^20 here)
+  unsigned a_off[LOADS];   // bytes from A (M * K <= 2^20, 2^28 where a measurement id asks for the form)
 #pragma unroll
-  for(int j = 0; j < LOADS; ++j) a_off[j] = (unsigned)(min(m_base + 4 * j + lane / 16, M - 1) * K + 4 * v) * 4u;
+  for(int j = 0; j < LOADS; ++j) a_off[j] = rows_a_offset(m_base, j, lane, v, M, K);
   const unsigned w_off = stream32_lane_offset(wsrc, lg);   // bytes from a sub-step's first column
   const unsigned w_step = 32u * (unsigned)args.N;
   // (as buffers: a scalar base, a scalar offset along K and a 32-bit lane offset, no vector arithmetic between the loads)
@@ -149,9 +135,9 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     v4f a[D > 0 ? D : 1][LOADS];
     v4i w[D > 0 ? D : 1][2];
     auto load = [&](int t, int d) __attribute__((always_inline)) {
-      const unsigned pair = (unsigned)(wave + t * kRowsWaves);
+      const unsigned pair = (unsigned)rows_pair(wave, t);
 #pragma unroll
-      for(int j = 0; j < LOADS; ++j) a[d][j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(a_buf, a_off[j], pair * 256u, 0));
+      for(int j = 0; j < LOADS; ++j) a[d][j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(a_buf, a_off[j], pair * kRowsPairBytes, 0));
 #pragma unroll
       for(int s = 0; s < 2; ++s) w[d][s] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w_buf, w_off, (2u * pair + s) * w_step, 0));
       __builtin_amdgcn_sched_barrier(0);
@@ -184,7 +170,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     for(int e = 0; e < 16; ++e) acc[e] = 0;
 #pragma unroll
     for(int t = 0; t < T; ++t) {
-      const int d = t % D;
+      const int d = t % (D > 0 ? D : 1);
       uint32_t q[LOADS];
       if(finite) {
 #pragma unroll
@@ -198,7 +184,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
       if(WRITE_AQ) {
 #pragma unroll
         for(int j = 0; j < LOADS; ++j)
-          *reinterpret_cast<uint32_t*>(aq_out + (a_off[j] / 4 + (unsigned)((wave + t * kRowsWaves) * 64))) = q[j];
+          *reinterpret_cast<uint32_t*>(aq_out + (a_off[j] / 4 + (unsigned)(rows_pair(wave, t) * 64))) = q[j];
       }
       // (a wave's LDS operations keep their order)
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -213,8 +199,9 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
       if(t + D < T) load(t + D, d);
     }
   };
-  const int pairs = K / 64;
-  const bool more = wave < pairs - (STEPS - 1) * kRowsWaves;   // this wave has STEPS pairs
+  // The waves of a workgroup run different instances of this code, and meet at its barriers all the same: the hardware counts
+  // the waves that have come to a barrier, whichever instruction they came by, and every instance has the same barriers in the same order.
+  const bool more = rows_has_all_steps(K, STEPS, wave);
   if(aq_out && first_column) {
     if(more) run(std::integral_constant<int, STEPS>(), std::true_type());
     else run(std::integral_constant<int, STEPS - 1>(), std::true_type());

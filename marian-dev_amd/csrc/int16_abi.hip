@@ -248,16 +248,6 @@ __device__ __forceinline__ float unquant16(const Gemm16Args& g) {
   return unquant_mult(aqm, *reinterpret_cast<const float*>(g.Bq + (size_t)g.K * g.N), g.scale);
 }
 
-// The tile of workgroup `block` of tiles_n x tiles_m: workgroups are dealt out to the eight XCDs in turn, and those of one XCD
-// take neighbouring tiles - bands of eight columns - so that its L2 holds what they share.
-__device__ __forceinline__ void xcd_order16(int tiles_n, int tiles_m, int block, int& tn, int& tm) {
-  const int total = tiles_n * tiles_m, x = block % 8, rest = total % 8;
-  const int t = x * (total / 8) + min(x, rest) + block / 8;
-  const int band = 8, b = t / (band * tiles_m), r = t % (band * tiles_m), width = min(tiles_n - b * band, band);
-  tn = b * band + r % width;
-  tm = r / width;
-}
-
 // Sum over the four lanes of a quad, left in all of them (two DPP lane swaps).
 __device__ __forceinline__ int quad_sum(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
@@ -301,9 +291,9 @@ __global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(cons
   const AT* arow[MT];
   const int16_t* brow[NT];
 #pragma unroll
-  for(int i = 0; i < MT; ++i) arow[i] = reinterpret_cast<const AT*>(g.A) + (size_t)min(m0 + 16 * i + qr, g.M - 1) * g.K + qk * 8;
+  for(int i = 0; i < MT; ++i) arow[i] = reinterpret_cast<const AT*>(g.A) + row16_offset(m0 + 16 * i + qr, g.M, g.K) + piece16_offset(qk);
 #pragma unroll
-  for(int j = 0; j < NT; ++j) brow[j] = g.Bq + (size_t)min(n0 + 16 * j + qr, g.N - 1) * g.K + qk * 8;
+  for(int j = 0; j < NT; ++j) brow[j] = g.Bq + row16_offset(n0 + 16 * j + qr, g.N, g.K) + piece16_offset(qk);
   Acc16 acc[MT][NT];
   int asum[MT], bsum[NT];
 #pragma unroll
@@ -320,7 +310,7 @@ __global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(cons
   Raw<AT> ra[D][MT];
   Raw<int16_t> rb[D][NT];
   auto load = [&](int t, Raw<AT> (&ra)[MT], Raw<int16_t> (&rb)[NT]) __attribute__((always_inline)) {
-    const int s = wave + t * KW, k = s * 64, second = half && s == S - 1 ? 0 : 32;
+    const int s = wave + t * KW, k = s * kStep16, second = half && s == S - 1 ? 0 : 32;
 #pragma unroll
     for(int i = 0; i < MT; ++i) ra[i].load(arow[i] + k, second);
 #pragma unroll
@@ -494,20 +484,20 @@ __global__ __launch_bounds__(kTile16Threads) void gemm16_tile_kernel(const void*
     using E = decltype(element);
     constexpr int ROWS = kIsA ? BM : BN, U = ROWS * 4 / 256;   // pieces of 16 k a thread stages per block
     static_assert(U * 256 == ROWS * 4, "whole pieces per thread");
-    const int st = tid % 256, srow = st / 4, sk = (st % 4) * 8, spiece = piece16(srow, st % 4);   // four threads a row, 64 rows at a time
+    const int st = tid % 256, srow = st / 4, sk = piece16_offset(st % 4), spiece = piece16(srow, st % 4);   // four threads a row, 64 rows at a time
     const E* src[U];
     int sum[U];
     Raw<E> raw[D][U];
 #pragma unroll
     for(int u = 0; u < U; ++u) {
       const int row = srow + u * 64;
-      if constexpr(kIsA) src[u] = reinterpret_cast<const E*>(g.A) + (size_t)min(m0 + row, g.M - 1) * g.K;
-      else src[u] = g.Bq + (size_t)min(n0 + row, g.N - 1) * g.K;
+      if constexpr(kIsA) src[u] = reinterpret_cast<const E*>(g.A) + row16_offset(m0 + row, g.M, g.K);
+      else src[u] = g.Bq + row16_offset(n0 + row, g.N, g.K);
       sum[u] = 0;
     }
     auto load = [&](int kb, Raw<E> (&r)[U]) __attribute__((always_inline)) {
       kb = min(kb, blocks - 1);
-      const int k = kb * 64 + sk, second = half && kb == blocks - 1 ? 0 : 32;
+      const int k = kb * kStep16 + sk, second = half && kb == blocks - 1 ? 0 : 32;
 #pragma unroll
       for(int u = 0; u < U; ++u) r[u].load(src[u] + k, second);
     };
@@ -555,6 +545,7 @@ __global__ __launch_bounds__(kTile16Threads) void gemm16_tile_kernel(const void*
       if(st % 4 == 0) sums[(kIsA ? 0 : BM) + srow + u * 64] = total;
     }
   };
+  // (waves of a workgroup meet at the barriers of different instances: see gemm_rows_kernel)
   if(wave < 4) run(std::true_type(), AT());
   else run(std::false_type(), int16_t());
   // (every wave is past its last read of the stages) the sums as rows of BN, their 16-byte pieces permuted by the row number

@@ -144,17 +144,67 @@ __host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, in
   if(j >= per_wg || hyp >= hyps) return 0x7fffffff;
   return hyp * sentences + (group << shift) + (r & ((1 << shift) - 1));
 }
-// sentence groups of a launch (shift >= 0), and the tile of workgroup block_y of its groups x chunks
+// sentence groups of a launch (shift >= 0), and the first sentence of one
 __host__ __device__ __forceinline__ int proj_groups(int shift, int sentences) { return sentences >> shift; }
-__host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, int hyps, int per_wg, int block_y, int r) {
-  if(shift < 0) return proj_row_of(shift, sentences, hyps, per_wg, block_y, 0, r);
-  const int groups = proj_groups(shift, sentences);
-  return proj_row_of(shift, sentences, hyps, per_wg, block_y % groups, block_y / groups, r);
-}
-// first sentence of a group, and of workgroup block_y (shift >= 0)
 __host__ __device__ __forceinline__ int proj_first_sentence(int shift, int group) { return group << shift; }
-__host__ __device__ __forceinline__ int proj_first_sentence(int shift, int sentences, int block_y) {
-  return proj_first_sentence(shift, block_y % proj_groups(shift, sentences));
+
+// ---- gemm_rows_kernel: tiles of rows x 32 columns, every wave its own share of K ----
+constexpr int kRowsWaves = 8;
+// Which tile a workgroup of gx x gy takes.  Workgroups are dealt out to the eight XCDs in turn; a split of r = 1 << shift (r divides gy,
+// 8 / r divides gx) is launched as 8 x h x w workgroups, h = gy / r, w = gx r / 8, and gives each XCD a block of h x w tiles, so
+// that its L2 fetches fewer operands.  shift < 0: launched as gx x gy.
+struct RowsTiles {
+  int shift, h, w;
+};
+struct RowsTile {
+  int bx, by;
+};
+__host__ __device__ __forceinline__ RowsTile rows_tile(RowsTiles t, int x, int y, int z) {
+  if(t.shift < 0) return RowsTile{x, y};
+  return RowsTile{(x >> t.shift) * t.w + z, (x & ((1 << t.shift) - 1)) * t.h + y};
+}
+// The split of gx x gy tiles with which the XCDs' L2 caches fetch the fewest bytes (as they come where the tiles don't divide into eight blocks).
+__host__ __device__ __forceinline__ RowsTiles rows_tiles(int gx, int gy, long long row_bytes, long long column_bytes) {
+  RowsTiles best{-1, 0, 0};
+  long long least = 0;
+  for(int shift = 0; shift <= 3; ++shift) {
+    const int r = 1 << shift;
+    if(gy % r != 0 || gx % (8 / r) != 0) continue;
+    const RowsTiles t{shift, gy / r, gx / (8 / r)};
+    const long long bytes = t.h * row_bytes + t.w * column_bytes;
+    if(best.shift < 0 || bytes < least) { best = t; least = bytes; }
+  }
+  return best;
+}
+// K is taken in pairs of sub-steps (64 values of k): pair number t of a wave, and whether the wave has `steps` of them, ceil(K / 512), or one fewer
+__host__ __device__ __forceinline__ int rows_pair(int wave, int t) { return wave + t * kRowsWaves; }
+__host__ __device__ __forceinline__ bool rows_has_all_steps(int K, int steps, int wave) { return wave < K / 64 - (steps - 1) * kRowsWaves; }
+// Load j of a pair brings rows 4 j .. 4 j + 3 of the tile, sixteen lanes a row: byte offset of the four float32 values of a lane at
+// pair 0, v = lane % 16 (M * K <= 2^28); a pair is kRowsPairBytes of a row
+constexpr unsigned kRowsPairBytes = 256;
+__host__ __device__ __forceinline__ unsigned rows_a_offset(int m_base, int j, int lane, int v, int M, int K) {
+  return (unsigned)(addr_min(m_base + 4 * j + lane / 16, M - 1) * K + 4 * v) * 4u;
+}
+// Vector i of a thread's share of the activations, of workgroup `block` with `each` vectors (past the share or the tensor: the last ones again)
+__host__ __device__ __forceinline__ int rows_share_vec(int block, int each, int i, int tid, int threads, int n4) {
+  return addr_min(block * each + addr_min(tid + i * threads, each - 1), n4 - 1);
+}
+
+// ---- 16-bit kernels (rows of K values, K % 32 == 0, taken in steps of 64) ----
+// The four lanes of a quad take a row's step: piece q eight values from piece16_offset(q) and eight from 32 behind (where K % 64 != 0 the last
+// step has only the former: it reads them twice, and the kernels drop the second).  Index of a row's first value (rows past the end: the last one);
+// a step is kStep16 values.
+constexpr int kStep16 = 64;
+__host__ __device__ __forceinline__ size_t row16_offset(int row, int rows, int K) { return (size_t)addr_min(row, rows - 1) * K; }
+__host__ __device__ __forceinline__ int piece16_offset(int piece) { return piece * 8; }
+// The tile of workgroup `block` of tiles_n x tiles_m: workgroups are dealt out to the eight XCDs in turn, and those of one XCD
+// take neighbouring tiles - bands of eight columns - so that its L2 holds what they share.
+__host__ __device__ __forceinline__ void xcd_order16(int tiles_n, int tiles_m, int block, int& tn, int& tm) {
+  const int total = tiles_n * tiles_m, x = block % 8, rest = total % 8;
+  const int t = x * (total / 8) + addr_min(x, rest) + block / 8;
+  const int band = 8, b = t / (band * tiles_m), r = t % (band * tiles_m), width = addr_min(tiles_n - b * band, band);
+  tn = b * band + r % width;
+  tm = r / width;
 }
 
 }  // namespace marian_hip

@@ -153,6 +153,106 @@ static void staged(int BM, int BN, int waves, int M, int K, int N, const std::ve
     }
 }
 
+// ---- gemm_rows_kernel<ROWS, STEPS>: float32 rows and weights, every wave its own pairs of K sub-steps ----
+static void rows_form(int ROWS, int M, int K, int N, const std::vector<uint32_t>* idx) {
+  char where[160];
+  const int n_out = idx ? (int)idx->size() : N, steps = (K + 511) / 512;
+  const int gx = (n_out + 31) / 32, gy = (M + ROWS - 1) / ROWS, S = K / 32;
+  const long long a_bytes = 4LL * M * K, b_bytes = (long long)K * N;
+  const RowsTiles tiles = rows_tiles(gx, gy, 4LL * ROWS * K, 32LL * K);
+  std::snprintf(where, sizeof where, "rows ROWS=%d M=%d K=%d N=%d n_out=%d shift=%d", ROWS, M, K, N, n_out, tiles.shift);
+  const int X = tiles.shift < 0 ? gx : 8, Y = tiles.shift < 0 ? gy : tiles.h, Z = tiles.shift < 0 ? 1 : tiles.w;
+  if(X * Y * Z != gx * gy) fail("workgroups", X * Y * Z, gx * gy, where);
+  std::vector<int> taken((size_t)gx * gy, 0);
+  for(int x = 0; x < X; ++x)
+    for(int y = 0; y < Y; ++y)
+      for(int z = 0; z < Z; ++z) {
+        const RowsTile t = rows_tile(tiles, x, y, z);
+        ++g_checked;
+        if(t.bx < 0 || t.bx >= gx || t.by < 0 || t.by >= gy) { fail("tile outside", t.bx, t.by, where); continue; }
+        ++taken[(size_t)t.by * gx + t.bx];
+      }
+  for(size_t i = 0; i < taken.size(); ++i)
+    if(taken[i] != 1) { fail("tile coverage", (long long)i, taken[i], where); break; }
+  std::vector<int> seen_a((size_t)M * (K / 4), 0), seen_b((size_t)n_out * 2 * S, 0);   // (row, four values), (column, 16-byte chunk)
+  for(int wave = 0; wave < kRowsWaves; ++wave)
+    for(int t = 0; t < (rows_has_all_steps(K, steps, wave) ? steps : steps - 1); ++t) {
+      const int pair = rows_pair(wave, t);
+      for(int lane = 0; lane < 64; ++lane) {
+        for(int by = 0; by < gy; ++by)
+          for(int j = 0; j < ROWS / 4; ++j) {
+            const long long off = (long long)rows_a_offset(by * ROWS, j, lane, lane % 16, M, K) + (long long)pair * kRowsPairBytes;
+            inside(off, a_bytes, "activations", where);
+            const int row = by * ROWS + 4 * j + lane / 16;
+            if(off / (4LL * K) != addr_min(row, M - 1)) fail("activation load leaves its row", off, row, where);
+            if(row < M) ++seen_a[(size_t)row * (K / 4) + (size_t)(off % (4LL * K)) / 16];
+          }
+        const int li = lane % 32, lg = lane / 32;
+        for(int bx = 0; bx < gx; ++bx)
+          for(int s = 0; s < 2; ++s) {
+            const int col = stream32_lane_column(bx * 32, li, n_out), src = idx ? (int)(*idx)[col] : col;
+            inside((long long)stream32_lane_offset(src, lg) + (2LL * pair + s) * 32 * N, b_bytes, "weights", where);
+            if(bx * 32 + li < n_out) ++seen_b[((size_t)(bx * 32 + li) * S + 2 * pair + s) * 2 + lg];
+          }
+      }
+    }
+  for(size_t i = 0; i < seen_a.size(); ++i)
+    if(seen_a[i] != 1) { fail("activation coverage", (long long)i, seen_a[i], where); break; }
+  for(size_t i = 0; i < seen_b.size(); ++i)
+    if(seen_b[i] != 1) { fail("weight coverage", (long long)i, seen_b[i], where); break; }
+  // the shares of the abs-max that is exchanged: four vectors a thread
+  const int blocks = gx * gy, n4 = M * K / 4, each = (n4 + blocks - 1) / blocks;
+  if(each > 4 * 512) return;   // (not a call that exchanges)
+  std::vector<char> shared((size_t)n4, 0);
+  for(int block = 0; block < blocks; ++block)
+    for(int tid = 0; tid < 512; ++tid)
+      for(int i = 0; i < 4; ++i) {
+        const int v = rows_share_vec(block, each, i, tid, 512, n4);
+        ++g_checked;
+        if(v < 0 || v >= n4) { fail("share outside", v, n4, where); return; }
+        shared[(size_t)v] = 1;
+      }
+  for(int v = 0; v < n4; ++v)
+    if(!shared[(size_t)v]) { fail("share coverage", v, n4, where); break; }
+}
+
+// ---- 16-bit kernels: one operand of `rows` rows in tiles of `tile` rows, by the quads of a workgroup's lanes ----
+static void steps16(int tile, int rows, int K) {
+  char where[160];
+  std::snprintf(where, sizeof where, "16-bit tile of %d rows, %d rows, K=%d", tile, rows, K);
+  const int steps = (K + 63) / 64;
+  const bool half = K % 64 != 0;
+  std::vector<int> seen((size_t)rows * (K / 8), 0);   // (row, eight values)
+  for(int base = 0; base < rows; base += tile)
+    for(int r = 0; r < tile; ++r)
+      for(int piece = 0; piece < 4; ++piece)
+        for(int s = 0; s < steps; ++s) {
+          const long long first = (long long)row16_offset(base + r, rows, K) + piece16_offset(piece) + (long long)s * kStep16;
+          for(int part = 0; part < 2; ++part) {
+            const bool dropped = part && half && s == steps - 1;   // (the kernels' own condition)
+            const long long at = first + (part && !dropped ? 32 : 0);
+            ++g_checked;
+            if(at < 0 || at + 8 > (long long)rows * K) { fail("16-bit load", at, (long long)rows * K, where); continue; }
+            if(at / K != addr_min(base + r, rows - 1) || at % K + 8 > K) fail("16-bit load leaves its row", at, base + r, where);
+            if(base + r < rows && !dropped) ++seen[(size_t)(base + r) * (K / 8) + (size_t)(at % K) / 8];
+          }
+        }
+  for(size_t i = 0; i < seen.size(); ++i)
+    if(seen[i] != 1) { fail("16-bit coverage", (long long)i, seen[i], where); break; }
+}
+static void tiles16(int tiles_n, int tiles_m) {
+  std::vector<int> taken((size_t)tiles_n * tiles_m, 0);
+  for(int block = 0; block < tiles_n * tiles_m; ++block) {
+    int tn = -1, tm = -1;
+    xcd_order16(tiles_n, tiles_m, block, tn, tm);
+    ++g_checked;
+    if(tn < 0 || tn >= tiles_n || tm < 0 || tm >= tiles_m) { fail("16-bit tile outside", tn, tm, "xcd_order16"); continue; }
+    ++taken[(size_t)tm * tiles_n + tn];
+  }
+  for(size_t i = 0; i < taken.size(); ++i)
+    if(taken[i] != 1) { fail("16-bit tile coverage", tiles_n, tiles_m, "xcd_order16"); break; }
+}
+
 // The rows the workgroups of the one-launch projections + attention take: every row exactly once,
 // the rows of a workgroup that share a sentence slot attend to that sentence, and every staged
 // key/value load (and LDS slot) lies inside the caches (the staging area).
@@ -165,21 +265,24 @@ static void proj_rows(long long hyps, long long sentences, long long heads, long
   char where[160];
   std::snprintf(where, sizeof(where), "proj rows hyps %lld sentences %lld len %lld shift %d per %d stage %d", hyps, sentences,
                 len, plan.shift, plan.per_wg, plan.stage);
-  const int blocks = (int)plan.blocks_y;
+  // the launch: a dimension for groups of sentences (plain form: of rows) and one for chunks of hypotheses
+  const int groups = plan.shift < 0 ? (int)plan.blocks_y : proj_groups(plan.shift, plan.sentences), chunks = (int)plan.blocks_y / groups;
+  if((long long)groups * chunks != plan.blocks_y) fail("workgroups of the launch", groups, chunks, where);
   if(plan.shift < 0 && plan.blocks_y != (M + 7) / 8) fail("workgroups of the plain form", plan.blocks_y, (M + 7) / 8, where);
   if(plan.shift >= 0 && ((plan.per_wg << plan.shift) > 8 || (plan.per_wg << plan.shift) < 4 || plan.hyps != hyps))
     fail("hypotheses per workgroup", plan.per_wg, plan.shift, where);
   std::vector<int> seen((size_t)M, 0);
-  for(int by = 0; by < blocks; ++by)
+  for(int by = 0; by < groups * chunks; ++by)
     for(int r = 0; r < 8; ++r) {
-      const int m = proj_row_of(plan.shift, plan.sentences, plan.hyps, plan.per_wg, by, r);
+      const int group = by % groups, chunk = by / groups;
+      const int m = proj_row_of(plan.shift, plan.sentences, plan.hyps, plan.per_wg, group, chunk, r);
       ++g_checked;
       if(m < 0) { fail("negative row", by, r, where); continue; }
       if(m >= M) continue;   // rows past the end are skipped by the kernel
       ++seen[(size_t)m];
       if(plan.shift >= 0) {
         const int slot = r & ((1 << plan.shift) - 1);
-        const int sentence = proj_first_sentence(plan.shift, plan.sentences, by) + slot;
+        const int sentence = proj_first_sentence(plan.shift, group) + slot;
         if(sentence >= sentences || m % sentences != sentence) fail("row outside its sentence", by, r, where);
         if(plan.stage) {   // the loads of segment 2 * slot (keys) and 2 * slot + 1 (values)
           const long long entry = (long long)sentence * heads + (heads - 1);
@@ -231,6 +334,27 @@ int main() {
             for(auto& sl : shortlists(N, 8)) staged(c[0], c[1], c[2], M, K, N, &sl);
         }
   std::printf("staged: %lld loads checked\n", g_checked - before);
+  before = g_checked;
+  for(int ROWS : {8, 16, 32})
+    for(int K : {256, 320, 512, 576, 1088, 2048, 4096}) {
+      if(ROWS == 32 && K > 2048) continue;
+      for(int M : {1, 9, 31, 32, 65})
+        for(int N : {8, 24, 264, 1000}) {
+          rows_form(ROWS, M, K, N, nullptr);
+          if(N >= 264)
+            for(auto& sl : shortlists(N, 40)) rows_form(ROWS, M, K, N, &sl);
+        }
+    }
+  for(int shift_x : {1, 2, 3, 5, 8, 16, 24, 48, 100})   // every split of the tiles
+    for(int gy : {1, 2, 3, 4, 5, 8, 13, 32}) rows_form(8, 8 * gy, 256, 32 * shift_x, nullptr);
+  std::printf("rows: %lld loads checked\n", g_checked - before);
+  before = g_checked;
+  for(int tile : {16, 32, 64, 128})
+    for(int rows : {1, 8, 15, 16, 33, 64, 129, 200})
+      for(int K : {32, 64, 96, 128, 160, 544, 1056}) steps16(tile, rows, K);
+  for(int tn = 1; tn <= 40; ++tn)
+    for(int tm = 1; tm <= 40; ++tm) tiles16(tn, tm);
+  std::printf("16-bit: %lld loads and tiles checked\n", g_checked - before);
   before = g_checked;
   for(long long hyps : {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 16, 17})
     for(long long sentences : {1, 2, 3, 4, 5, 8, 10, 32, 33})

@@ -3,7 +3,7 @@ the GEMM kernels compile for their operand offsets (marian-dev_amd/csrc/operand_
 columns and their clamps, sub-step clamps, the LDS staging offsets of the large-M tiles, the
 detours of a 64-column last K block, shortlist gathers) and walks every lane, wave, tile and K
 step of edge shapes - N = 8 / 24 / 1000 / 1032, K = 64 / 192 / 576 / 1088 / 1024, M = 129 ... 300,
-shortlists of 8 - through it: every 16-byte load inside its operand, every multiplied chunk
+shortlists of 8; few rows of up to 4096 values, the 16-bit kernels' steps and tiles - through it: every 16-byte load inside its operand, every multiplied chunk
 fetched exactly once.  Built with the host sanitizers."""
 import os
 import subprocess
@@ -29,7 +29,10 @@ def test_kernels_use_the_checked_helpers():
         "gemm_stream_kernel.h": ["stream16_lane_offset("],
         "gemm_mfma32_kernel.h": ["stage_a_offset(", "stage_b_column(", "stage_b_offset(", "stage_a_tail_adjust(", "stage_b_goes_back("],
         "gemm_pair_kernel.h": ["stage_a_row(", "stage_a_chunk(", "stage_b_offset("],
-        "decode_ops.hip": ["stream32_lane_offset(", "stream32_clamped_substep(", "proj_row_plan(", "proj_row_of(", "proj_first_sentence("],
+        "gemm_rows_kernel.h": ["rows_tile(", "rows_pair(", "rows_has_all_steps(", "rows_a_offset(", "kRowsPairBytes", "rows_share_vec(", "stream32_lane_column(", "stream32_lane_offset("],
+        "c_abi.hip": ["rows_tiles("],
+        "int16_abi.hip": ["row16_offset(", "piece16_offset(", "kStep16", "xcd_order16("],
+        "decode_ops.hip": ["stream32_lane_offset(", "stream32_clamped_substep(", "proj_row_plan(", "proj_groups(", "proj_row_of(", "proj_first_sentence("],
     }
     for name, calls in uses.items():
         text = open(os.path.join(CSRC, name)).read()
