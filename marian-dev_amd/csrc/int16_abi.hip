@@ -269,7 +269,7 @@ template <typename AT, int MT, int NT, int D, bool DUMP>
 __global__ __launch_bounds__(64 * kStream16Waves) void gemm16_stream_kernel(const void* A, const int16_t* Bq, const float* bias_in,
                                                                               unsigned long long M_K, int N, Gemm16Rest rest) {
   const Gemm16Args g = gemm16_args(A, Bq, bias_in, M_K, N, rest);
-  const int tiles_n = (g.N + 16 * NT - 1) / (16 * NT), tiles_m = (g.M + 16 * MT - 1) / (16 * MT);
+  const int tiles_n = (int)((unsigned)(g.N + 16 * NT - 1) / (16 * NT)), tiles_m = (int)((unsigned)(g.M + 16 * MT - 1) / (16 * MT));
   constexpr int KW = kStream16Waves, TILES = MT * NT, kWaveBytes = stream16_lds<MT, NT>() / KW;
   extern __shared__ __attribute__((aligned(16))) int8_t lds16[];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -432,7 +432,7 @@ template <typename AT, int BM, int BN, int WM, int WN, bool DUMP>
 __global__ __launch_bounds__(kTile16Threads) void gemm16_tile_kernel(const void* A, const int16_t* Bq, const float* bias_in,
                                                                      unsigned long long M_K, int N, Gemm16Rest rest) {
   const Gemm16Args g = gemm16_args(A, Bq, bias_in, M_K, N, rest);
-  const int tiles_n = (g.N + BN - 1) / BN, tiles_m = (g.M + BM - 1) / BM;
+  const int tiles_n = (int)((unsigned)(g.N + BN - 1) / BN), tiles_m = (int)((unsigned)(g.M + BM - 1) / BM);
   static_assert(WM * WN == 8, "eight waves");
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16, D = kTile16Depth;   // D: blocks of K on their way
   extern __shared__ __attribute__((aligned(16))) int8_t lds16[];
