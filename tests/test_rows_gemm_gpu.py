@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 f32 = np.float32
 
 SIZES = [
-    # 8 rows
-    (9, 64, 8), (17, 448, 24), (23, 512, 512), (40, 576, 264), (64, 1024, 1024), (12, 1600, 72), (30, 2048, 512), (20, 2624, 96),
+    # 8 rows (K = 64: fewer sub-steps than waves, another form)
+    (9, 64, 8), (9, 256, 8), (17, 448, 24), (23, 512, 512), (40, 576, 264), (64, 1024, 1024), (12, 1600, 72), (30, 2048, 512), (20, 2624, 96),
     (33, 3136, 128), (9, 4032, 40), (31, 4096, 40),
     # 16 rows
     (127, 512, 1024), (128, 1088, 1000), (16, 1536, 4096), (100, 4096, 1000), (128, 3520, 1024), (113, 2560, 1024), (128, 2880, 1000),
@@ -77,10 +77,38 @@ def test_affine_that_takes_its_absmax(integer, orc, synth, M, K, N, kernel):
             assert np.array_equal(out.cpu().numpy(), orc.affine(Aq_h, Bq_h, bias, M, K, N, 1.0, False)[0])
 
 
-@pytest.mark.parametrize("gx,gy", [(32, 8), (64, 4), (16, 5), (3, 7), (8, 1), (1, 8), (24, 3), (48, 2), (100, 2)])
+@pytest.mark.parametrize("kind", ["zero", "infinite", "nan", "tiny"])
+@pytest.mark.parametrize("kernel", [0, 702])
+@pytest.mark.parametrize("M,K,N", [(64, 1024, 1024), (128, 1088, 1000), (250, 1216, 1000)])
+def test_absmax_that_is_none_of_the_usual(integer, orc, synth, M, K, N, kernel, kind):
+    """What is exchanged is a zero, an infinity, a maximum beside NaNs (which count for nothing) or a denormal number: the bytes and
+    outputs of the checker, with the values in the share of the last workgroup."""
+    import contextlib
+    A = synth.normal(980 + M, synth.STREAM_A, (M, K), 1.0)
+    if kind == "zero":
+        A[:] = 0.0
+    elif kind == "infinite":
+        A[-1, -2] = -np.inf
+    elif kind == "nan":
+        A[-1, -2:], A[0, 0] = np.nan, np.nan
+        A[-1, -5] = 7.25
+    else:
+        A *= f32(1e-41)
+    W, bias = synth.normal(980 + N, synth.STREAM_W, (K, N), 0.02), synth.normal(980 + N, synth.STREAM_BIAS, (N,), 0.01)
+    Aq_h, Bq_h = orc.prepare_a(A), orc.prepare_b(W)
+    want = orc.affine(Aq_h, Bq_h, bias, M, K, N, 1.0, False)[0]
+    Bq = integer.prepareB(upload(W))
+    with load("_lib").forced_kernel(kernel) if kernel else contextlib.nullcontext():
+        out, Aq = integer.affine_f32(upload(A), Bq, upload(bias))
+    assert np.array_equal(Aq.numpy(), Aq_h)
+    assert np.array_equal(out.cpu().numpy(), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("gx,gy", [(32, 8), (64, 4), (16, 5), (3, 7), (8, 1), (1, 8), (24, 3), (48, 2), (100, 2), (16, 16), (5, 32), (2, 13)])
 def test_tiles_are_each_taken_once(integer, synth, orc, gx, gy):
-    """every split of the tiles over the XCDs: 16 (8 and 32) rows by 32 columns, one output wrong per tile missed"""
-    M, K, N = 16 * gy, 128, 32 * gx
+    """every split of the tiles over the XCDs: 8, 16 or 32 rows by 32 columns, one output wrong per tile missed (K = 512: the form
+    whose waves split K in eight, where the columns leave room for it)"""
+    M, K, N = 16 * gy, 512, 32 * gx
     A, W = synth.normal(gx, synth.STREAM_A, (M, K), 1.0), synth.normal(gy, synth.STREAM_W, (K, N), 0.02)
     want, _ = orc.affine(orc.prepare_a(A), orc.prepare_b(W), None, M, K, N, 1.0, False)
     x = upload(A)

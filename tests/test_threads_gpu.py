@@ -2,7 +2,7 @@
 call (reference src/translator/translator.h:158-164: one graph and backend per worker thread,
 several workers may share a device).  Each thread runs 200 mixed calls on a stream and workspace
 of its own - fused small-M, grouped, the one-pass prepareA at 4096 x 1024, a large-M GEMM, a
-shortlisted output layer, log-softmax + n-best - while the other does the same, and every result
+shortlisted output layer, one-launch prepareB, log-softmax + n-best - while the other does the same, and every result
 is compared with the CPU checker's (n-best: with the separate calls' result taken beforehand);
 the run stops at the first mismatch."""
 import sys
@@ -62,6 +62,19 @@ def build_cases(integer, ops, orc, synth, torch, seed):
     cases.append(("prepareA 4096x1024",
                   (lambda dA=dA: [integer.prepareA(dA).data[: 4096 * 1024 + 4]]),
                   [orc.prepare_a(A).view(np.int8)]))
+    # prepareB in one launch (one and four tiles to a workgroup), and a multiplication that exchanges its abs-max
+    for s, K, N in ((seed + 84, 512, 520), (seed + 85, 1024, 4096)):
+        W = synth.normal(s, synth.STREAM_W, (K, N), 0.02)
+        dW = dev(W)
+        cases.append(("prepareB %dx%d" % (K, N), (lambda dW=dW: [integer.prepareB(dW).data[: dW.numel() + 4]]),
+                      [load("layout").to_prepared(orc.prepare_b(W), K, N).view(np.int8)]))
+    M, K, N = 64, 1024, 1000
+    A = synth.normal(seed + 86, synth.STREAM_A, (M, K), 1.0)
+    Bh, Bq = weights(seed + 87, K, N)
+    want, _ = orc.affine(orc.prepare_a(A), Bh, None, M, K, N, 1.0, False)
+    dA = dev(A)
+    cases.append(("affine_f32 64x1024x1000 without a bias", (lambda dA=dA, Bq=Bq: [integer.affine_f32(dA, Bq, None)[0]]),
+                  [np.asarray(want, dtype=f32).reshape(M, N)]))
     # a large-M GEMM from float32 input (prepareA + tile kernel), ragged on both sides
     M, K, N = 1100, 1024, 1032
     A = synth.normal(seed + 91, synth.STREAM_A, (M, K), 1.0)
