@@ -36,13 +36,14 @@ __device__ __forceinline__ float onepass_exchange(int g, float m, unsigned gen, 
   // n words from p with this launch's tag, polled by the first lanes of wave 0: their maximum, in *found whether all came
   auto collect = [&](const unsigned long long* p, int n, bool* found) {
     float v = 0.0f;
-    *found = onepass_wait(polls_left, [&] {
+    *found = false;
+    for(; onepass_patience(polls_left); onepass_polled(polls_left)) {
       const unsigned long long w = __hip_atomic_load(p + min(tid, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       v = __uint_as_float((unsigned)w);
-      const bool all = __all((unsigned)(w >> 32) == tag);
-      if(!all) __builtin_amdgcn_s_sleep(1);
-      return all;
-    });
+      *found = __all((unsigned)(w >> 32) == tag);
+      if(*found) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
     return wave_max(v);
   };
   if(tid < kWave) {

@@ -11,15 +11,9 @@
 
 namespace marian_hip {
 
-// Polls until poll() finds what it waits for; every wait of a workgroup draws on the same budget.
-template <class Poll>
-__host__ __device__ __forceinline__ bool onepass_wait(int& polls_left, Poll poll) {
-  while(polls_left > 0) {
-    --polls_left;
-    if(poll()) return true;
-  }
-  return false;
-}
+// A workgroup's waits draw on one budget of polls.
+__host__ __device__ __forceinline__ bool onepass_patience(int polls_left) { return polls_left > 0; }
+__host__ __device__ __forceinline__ void onepass_polled(int& polls_left) { --polls_left; }
 
 // Polls of a workgroup before it helps itself, each a memory round trip of about half a microsecond.  A launch that has the chip
 // waits for 2 us.  Where its last workgroups have to wait for compute units that work on another stream holds - which may itself

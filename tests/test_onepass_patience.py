@@ -16,10 +16,13 @@ int main() {
   for(int budget : {0, 1, 5, 64})
     for(int first : {0, 1, 3, 64, 100}) {   // the poll that finds the first words; 0: none does
       int left = budget, polls = 0;
-      const bool found = onepass_wait(left, [&] { return ++polls == first; });
+      bool found = false;
+      for(; onepass_patience(left); onepass_polled(left))
+        if((found = ++polls == first)) break;
       if(found != (first > 0 && first <= budget)) { std::printf("found at poll %d of %d\n", first, budget); return 1; }
-      if(found) onepass_wait(left, [&] { ++polls; return false; });
-      if(polls > budget || left < 0) { std::printf("%d polls of %d\n", polls, budget); return 1; }
+      if(found)
+        for(; onepass_patience(left); onepass_polled(left)) ++polls;
+      if(polls > budget + 1 || left < 0) { std::printf("%d polls of %d\n", polls, budget); return 1; }   // (the poll that finds costs none)
     }
   for(size_t n : {33ul << 10, 64ul << 10, 1ul << 20, 4ul << 20, 16ul << 20}) std::printf("%zu %d\n", n, onepass_polls(n));
   return 0;
@@ -41,4 +44,5 @@ def test_waits_are_bounded(tmp_path):
             us, way_out = 0.5 * polls, 256 * 4 * n / 6e12 * 1e6
             assert 20 <= us <= 40 + way_out, (n, us, way_out)
     used = open(os.path.join(CSRC, "onepass_exchange.h")).read()
-    assert used.count("onepass_wait(") == 1 and "for(int spin" not in used   # (the kernels wait nowhere else)
+    assert used.count("for(; onepass_patience(polls_left); onepass_polled(polls_left))") == 1   # (the kernels wait nowhere else)
+    assert used.count("int polls_left = polls;") == 1 and used.count("while(") == 0 and used.count("for(") == 2
