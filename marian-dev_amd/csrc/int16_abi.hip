@@ -616,7 +616,8 @@ int launch_tile16(const Gemm16Args& g, hipStream_t st) {
 // launch, of a further workgroup per CU, and of a byte of either operand that a workgroup takes in (least squares over measurements
 // at 99 sizes where the form is near the best: -26 .. +17 %; K, N = 256 .. 4096, M = 1 .. 4096, launches in a graph; a CU holds one
 // 128 x 128 tile at a time).  The form taken is the best or at most 4 % behind it but for 256 rows of 704 values by 1408
-// (15 %: eleven steps of K over eight waves) and 64 rows of them (7 %; profiles/int16_forms.txt: every form, both kinds).  us, int16
+// (14 and 17 %, int16 and float32 activations: eleven steps of K over eight waves) and 64 float32 rows of them (7 %;
+// profiles/int16_forms.txt: every form, both kinds).  us, int16
 // and float32 activations:
 //   1 x 512 x 512 2.8 and 3.0 (stream 16 x 16), 64 x 512 x 2048 3.6 and 3.7 (16 x 32), 509 x 2048 x 512 8.1 and 8.8 (32 x 32;
 //   10.4 and 14.6 with lanes that loaded the rows they multiply), 509 x 512 x 2048 6.5 and 6.8 (64 x 64; 8.6 and 10.2 with four
