@@ -376,8 +376,8 @@ int launch_stream32(const GemmArgs& a, const FusedSrc& f, hipStream_t st, const 
     if((long long)blocks * m_tiles * Cfg::kWaves <= kAbsmaxSlots) t_absmax_written = true;
     else a2.absmax_out = nullptr;
   }
-  MH_LAUNCH(kernel, dim3(blocks, m_tiles), dim3(Cfg::kThreads), lds, st, f.A, a2.Bq, a2.Aq, f.partials, int_pair(a2.M, a2.K),
-            int_pair(a2.N, a2.n_out), int_pair(f.n_partials, a2.idx ? 1 : 0), Stream32Rest<NoGroups, NoNorm>{a2, f.aq_out, NoGroups(), NoNorm()});
+  MH_LAUNCH(kernel, dim3(blocks, m_tiles), dim3(Cfg::kThreads), lds, st, f.A, a2.Bq, a2.Aq, MODE == kFusedAll ? a2.bias : f.partials,
+            int_pair(a2.M, a2.K), int_pair(a2.N, a2.n_out), int_pair(f.n_partials, a2.idx ? 1 : 0), Stream32Rest<NoGroups, NoNorm>{a2, f.aq_out, NoGroups(), NoNorm()});
   MH_HIP(hipGetLastError());
   return MARIAN_HIP_OK;
 }

@@ -77,8 +77,10 @@ struct Stream32Rest {
 };
 
 // Dynamic LDS: one chunk (kStageBytes), for kFusedAll all of K (32 * MT32 * K bytes) if that is
-// more; at least kReduceBytes.  aux: n_partials (1..2048) abs-max values (kFusedTiled), what is added to A (kFusedNorm).  The fields of args
-// that are arguments of their own as well are those; shortlist: whether there is one.
+// more; at least kReduceBytes.  aux: n_partials (1..2048) abs-max values (kFusedTiled), what is added to A (kFusedNorm), the
+// bias (kFusedAll: one address fewer to wait for ahead of the weights; in a graph 4 x 1024 x 2360 3.38 us with it in args and 3.32 now,
+// 2 x 256 x 3000 2.93 and 2.87, 1 x 512 x 512 2.92 and 2.87).  The fields of args that are
+// arguments of their own as well are those; shortlist: whether there is one.
 // NG (kFusedAll): 16-value groups per thread that are compiled in, 2 or 4; all but the last two are
 // complete (the launcher picks NG = 2 for M * K <= 16384), so their loads, abs-max and
 // quantization carry no range checks.
@@ -98,6 +100,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
   const NORMED& norm = rest.norm;
   args.Bq = Bq; args.Aq = Aq; args.M = M; args.K = K; args.N = N; args.n_out = n_out;   // (what is needed first comes in registers, see the Makefile)
   const float* const partials = aux;
+  if constexpr(MODE == kFusedAll) args.bias = aux;
   using Cfg = Stream32Cfg<MT32, WN, KW, PW>;
   constexpr bool GROUPED = std::is_same<GROUPS, GroupTable>::value;
   constexpr bool NORM = MODE == kFusedNorm;
