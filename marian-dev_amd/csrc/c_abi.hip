@@ -855,18 +855,16 @@ unsigned next_nonce() {
   return nonce.fetch_add(0x9E3779B1u, std::memory_order_relaxed);
 }
 
-// Whether the workgroups of gemm_rows_kernel take the abs-max of the activations themselves: one to a CU, a share of the
-// activations that a thread holds in a few registers, and rows of up to 2048 values (100 x 4096 x 1024 9.5 us that way, with a
-// launch in front 9.1; 40 x 3072 x 768 7.3 and 7.0).  The exchange takes the GPU longer than a launch in front - 64 x 1024 x 1024 in a
-// graph 5.92 and 5.42 us, 256 x 512 x 512 6.14 and 5.36, 256 x 1024 x 1000 7.44 and 6.87, at 26 of 48 sizes 4 % or more, at four 2 - 5 %
-// less (32 x 2048 x 512 5.91 and 6.20) - and spares the host a launch of 2.2: launched one by one from C++ the same calls take 5.84 and 7.38,
-// 6.40 and 7.24, 7.46 and 7.42 (at worst 128 x 1088 x 640 7.06 and 6.84), from Python more of that or less with the host.  So calls
-// that are being recorded have the launch in front.  (Measurement ids: 630 the launch in front; 702 no patience.)
+// Whether the workgroups of gemm_rows_kernel take the abs-max of the activations themselves: one to a CU, and a share of the
+// activations that a thread holds in a few registers.  Launched one by one, with a launch in front and so: 64 x 1024 x 1024 7.4 and 5.3 us,
+// 256 x 1024 x 1000 7.4 and 6.5, 128 x 4096 x 1024 10.3 and 9.4, 40 x 3072 x 768 7.8 and 6.9, 64 x 4096 x 512 8.8 and 8.1.
+// Calls that are being recorded have the launch in front, which costs the host nothing there.  (Measurement ids: 630 the launch in
+// front; 702 no patience.)
 bool rows_can_exchange(int M, int K, int n_out, int kw_override) {
   const TiledPlan plan = plan_tiled(M, K, n_out, kw_override);
   const long long groups = ((n_out + 31) / 32) * (long long)((M + plan.rows - 1) / plan.rows);
   const int cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
-  return plan.kw == 8 && K <= 2048 && groups <= cus && (long long)M * K <= groups * kRowsShare;
+  return plan.kw == 8 && K <= rows_max_k(plan.rows) && groups <= cus && (long long)M * K <= groups * kRowsShare;
 }
 
 // Whether calls on the stream are recorded into a graph instead of being launched.
@@ -878,11 +876,13 @@ bool recorded(hipStream_t st) {
 }
 
 // The words of a workspace through which the workgroups of a one-pass launch exchange the abs-max of so many values.
-using OnePass = AbsMaxExchange;
-OnePass onepass_words(void* workspace, size_t values, bool no_patience) {
-  unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
-  return {reinterpret_cast<unsigned long long*>(ws + kOnePassSlotsOffset), reinterpret_cast<unsigned long long*>(ws + kOnePassGenOffset),
-          reinterpret_cast<unsigned long long*>(ws + kOnePassBoardOffset), next_nonce(), no_patience ? 0 : onepass_polls(values)};
+AbsMaxExchange onepass_words(void* workspace, size_t values, bool no_patience) {
+  return {reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(workspace) + kOnePassWordsOffset), next_nonce(),
+          no_patience ? 0 : onepass_polls(values)};
+}
+// The generation word of launches that are recorded into a graph, whose replays repeat their nonce; else null.
+unsigned long long* onepass_generation(void* workspace, hipStream_t st) {
+  return recorded(st) ? reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(workspace) + kOnePassGenOffset) : nullptr;
 }
 
 int absmax_blocks(size_t n4) {
@@ -1033,9 +1033,10 @@ int marian_hip_int8_prepare_a(const float* A, int8_t* Aq, int64_t M, int64_t K, 
     const size_t groups = (n16 + 1024 * (size_t)sets - 1) / (1024 * (size_t)sets);
     const bool fits = groups <= (size_t)cus;
     if(fits && ov != 700) {
-      const OnePass o = onepass_words(workspace, n, ov == 702);
+      const AbsMaxExchange o = onepass_words(workspace, n, ov == 702);
+      unsigned long long* const gen = onepass_generation(workspace, st);
 #define MH_ONEPASS(SETS)                                                                                                       \
-  MH_LAUNCH(prepare_a_onepass_kernel<SETS>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.slots, o.gen, o.boards, \
+  MH_LAUNCH(prepare_a_onepass_kernel<SETS>, dim3((int)groups), dim3(1024), 0, st, A, (unsigned)n16, Aq, o.words, gen, \
             o.nonce, o.polls, (int)groups)
       switch(sets) {
         case 1: MH_ONEPASS(1); break;
@@ -1070,14 +1071,15 @@ int marian_hip_int8_prepare_b(const float* W, int8_t* Bq, int64_t K, int64_t N, 
   const long long tiles_n = (N + 63) / 64, tiles = tiles_n * (K / 64);
   const long long cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
   if(tiles <= 4 * cus && ov != 700 && aligned(workspace, 8)) {
-    const OnePass o = onepass_words(workspace, n, ov == 702);
+    const AbsMaxExchange o = onepass_words(workspace, n, ov == 702);
+    unsigned long long* const gen = onepass_generation(workspace, st);
     const int per = tiles <= cus ? 1 : tiles <= 2 * cus ? 2 : 4, groups = (int)((tiles + per - 1) / per);
     if(per == 1)
-      MH_LAUNCH(prepare_b_onepass_kernel<1>, dim3(groups), dim3(256), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<1>, dim3(groups), dim3(256), 0, st, W, (int)K, (int)N, Bq, o.words, gen, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
     else if(per == 2)
-      MH_LAUNCH(prepare_b_onepass_kernel<2>, dim3(groups), dim3(512), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<2>, dim3(groups), dim3(512), 0, st, W, (int)K, (int)N, Bq, o.words, gen, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
     else
-      MH_LAUNCH(prepare_b_onepass_kernel<4>, dim3(groups), dim3(1024), 0, st, W, (int)K, (int)N, Bq, o.slots, o.gen, o.boards, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
+      MH_LAUNCH(prepare_b_onepass_kernel<4>, dim3(groups), dim3(1024), 0, st, W, (int)K, (int)N, Bq, o.words, gen, o.nonce, o.polls, groups, (int)tiles_n, (int)tiles);
     MH_HIP(hipGetLastError());
     return MARIAN_HIP_OK;
   }
@@ -1169,7 +1171,7 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
       f.n_partials = kAbsmaxSlots;
     } else if(which != 630 && rows_can_exchange((int)M, (int)K, (int)n_out, want_tiled ? which - 620 : 0) && aligned(workspace, 8) &&
               !recorded(hst)) {
-      const OnePass o = onepass_words(workspace, (size_t)M * (size_t)K, which == 702);
+      const AbsMaxExchange o = onepass_words(workspace, (size_t)M * (size_t)K, which == 702);
       f.exchange = &o;
       return launch_stream32_auto<kFusedTiled>(a, f, hst, want_tiled ? which - 620 : 0);
     } else {
@@ -1409,9 +1411,9 @@ int marian_hip_int8_affine_f32_static(const float* A, const int8_t* Bq, const fl
   int8_t* Aq = reinterpret_cast<int8_t*>(base);
   void* workspace = base + kStaticAqBytes;
   // The quantized activations and the abs-max partials are written earlier in the same call than
-  // they are read.  The hand-over area of the one-pass prepareA (more than 32 Ki values: arrival slots,
-  // generation word, boards) is different: its words persist from call to call and are matched
-  // by tag (a per-process nonce plus the generation word, top bit always set), so a word left by
+  // they are read.  The hand-over area of the one-pass prepareA (more than 32 Ki values: words
+  // and a generation) is different: its words persist from call to call and are matched
+  // by tag (a nonce of the call, plus the generation in a graph, top bit always set), so a word left by
   // an earlier call - or the zeros the array starts with - never passes for a fresh one.  Nothing
   // has to be cleared between calls.
   return affine_f32_impl(A, Aq, Bq, bias, idx, n_idx, out, M, K, N, scale, relu, nullptr, nullptr,

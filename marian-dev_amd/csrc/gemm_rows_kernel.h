@@ -35,11 +35,10 @@ constexpr int rows_depth(int rows) { return rows == 32 ? 2 : 4; }
 // Where the abs-max of the activations comes from.  AbsMaxSlots: n_partials values at `partials`, whose maximum it is.
 // AbsMaxExchange: nobody has taken it.  Every workgroup takes that of its share of the activations (kRowsShare values at most, read
 // ahead of its operands) and they exchange it while their first operands are on their way, instead of a launch in front: calls on a stream
-// 64 x 1024 x 1024 6.6 -> 6.2 us, 32 x 2048 x 512 6.7 -> 6.1, 256 x 512 x 512 6.7 -> 5.7, 256 x 1024 x 1000 7.2 and 7.45, and 2.2 us
-// less of the host's time each (a feed-forward block of 64 x 512 -> 2048 from Python 12.9 -> 11.6).
+// 64 x 1024 x 1024 7.4 -> 5.3 us, 256 x 512 x 512 6.7 -> 5.3, 256 x 1024 x 1000 7.4 -> 6.5, and 2.2 us less of the host's time each.
 struct AbsMaxSlots {};
 struct AbsMaxExchange {
-  unsigned long long *slots, *gen, *boards;
+  unsigned long long* words;
   unsigned nonce;
   int polls;
 };
@@ -99,10 +98,8 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
   const float bqm = tail_quant_mult(args.Bq, (size_t)K * (size_t)args.N);
   float pm[kAbsmaxSlots / kRowsThreads];
   v4f share[kRowsShareVecs];
-  unsigned gen = 0;
   const int block = tile.by * args.blocks_x + tile.bx, blocks = args.blocks_x * args.blocks_y;
   if constexpr(EXCHANGE) {
-    if(wave == 0) gen = (unsigned)__hip_atomic_load(absmax.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int n4 = M * K / 4, each = (n4 + blocks - 1) / blocks;   // (past the share: the tensor's last values, again)
 #pragma unroll
     for(int i = 0; i < kRowsShareVecs; ++i) share[i] = reinterpret_cast<const v4f*>(A)[rows_share_vec(block, each, i, tid, kRowsThreads, n4)];
@@ -154,9 +151,8 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
       for(int i = 0; i < kRowsShareVecs; ++i) amax = abs4max(share[i], amax);
       amax = block_max<kRowsWaves>(amax, red);
       if(blocks > 1)
-        amax = onepass_exchange<kRowsThreads>(block, amax, gen, (absmax.nonce + gen) | 0x80000000u, absmax.slots, absmax.gen, absmax.boards,
-                                              absmax.polls, blocks, red, &red[kRowsWaves],
-                                              [&] { return onepass_scan<kRowsThreads>(A, (size_t)M * K / 4, red); });
+        amax = onepass_exchange(block, amax, absmax.nonce, 0u, absmax.words, nullptr, absmax.polls, blocks, &red[kRowsWaves],
+                                [&] { return onepass_scan<kRowsThreads>(A, (size_t)M * K / 4, red); });
     } else {
 #pragma unroll
       for(int i = 0; i < kAbsmaxSlots / kRowsThreads; ++i) amax = fmaxf(amax, pm[i]);

@@ -7,70 +7,68 @@
 
 namespace marian_hip {
 
-// The workgroups of a launch exchange their abs-max through the workspace, in groups of 16:
-//   * every workgroup stores (tag, abs-max bits) into its arrival slot - one 8-byte store at device
-//     scope, so tag and value arrive together;
-//   * the first workgroup of a group polls its group's slots (one line), takes the maximum and publishes (tag, max) to its
-//     word of every one of 16 boards (a line each);
-//   * every workgroup polls the words of all groups on one board (16 pollers a board) and takes their maximum;
+// The workgroups of a launch exchange their abs-max through the workspace, in one step:
+//   * every workgroup stores (tag, abs-max bits) into its word of each of four copies - one instruction, 8 bytes at device
+//     scope a lane, so tag and value arrive together;
+//   * every workgroup polls all words of one copy (2 KB for 256 workgroups, four loads in flight a lane) and takes their maximum;
+//     workgroups that start together have their words in different lines (0.1 us);
 //   * nothing but these 8-byte words is handed over, so no fence is needed.
-// (One workgroup that polls all slots and answers all made the launch 0.9 us longer: 4096 x 1024 8.1 against 7.25 us.)
-// The tag is a host nonce plus a generation word that lives in the workspace and that workgroup 0
-// advances at the end of every launch: words left by an earlier launch - or by an earlier replay of
-// a recorded graph, which repeats the nonce - never match, whatever the workspace held before its
-// first use.  Every wait is bounded, and a workgroup's waits together are (onepass_patience.h): one that runs out of patience (the
+// Bound by trips to the memory side, the store's and a poll's, 1.2 us.  The first poll waits for a quarter of that: one that comes back
+// unanswered costs a trip, and the 4096 lines that 256 workgroups ask for are in the way of the words and of the loads still under way
+// (without the pause, with 512, 1024, 1536 and 2048 clocks of it: 64 x 1024 x 1024 through gemm_rows_kernel 5.7, 5.7, 5.4, 5.6, 5.7 us,
+// 256 x 1024 x 1000 7.1, 6.9, 6.5, 6.8, 7.0, prepareA of 4096 x 1024 7.2, 7.0, 6.3, 6.2, 6.4; a wave of its own for the polls, without
+// loads in front of them, is no better).  The form before had four trips, groups of 16 whose first workgroup answered for them: 6.6, 7.8 and
+// 7.5 us.  Copies, a launch that does nothing else, without the pause: 1, 2, 4, 8 and 16 of them 3.8, 3.6, 3.4, 3.4 and 3.5 us, 4.5 in four trips.
+// The tag is a host nonce, another for every launch; words left by an earlier launch never match, whatever the workspace
+// held before its first use.  A launch that is recorded into a graph repeats its nonce with every replay, so there a generation word that
+// lives in the workspace and that workgroup 0 advances at the end of every replay is added to it (0.2 us: gen_word is null elsewhere).
+// Every wait is bounded, and a workgroup's waits together are (onepass_patience.h): one that runs out of patience (the
 // device was shared and not all workgroups were resident) takes the abs-max over the whole input itself - the
-// result is the same - clears its slot, and the launch still ends.
+// result is the same -, and the launch still ends.
 __device__ __forceinline__ unsigned long long onepass_word(unsigned tag, float v) {
   return ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v);
 }
-// g: this workgroup of G <= 256, m: the abs-max of its values (in every thread), tag: this launch's (in wave 0), gen: the generation
-// word as it was (in thread 0).  scan: the abs-max of the whole input, by this workgroup alone.
-template <int THREADS, class Scan>
-__device__ __forceinline__ float onepass_exchange(int g, float m, unsigned gen, unsigned tag, unsigned long long* slots,
-                                                  unsigned long long* gen_word, unsigned long long* boards, int polls,
-                                                  int G, float* red, float* shared_max, Scan scan) {
+// g: this workgroup of G <= 256, m: the abs-max of its values (in every thread), nonce: this launch's; gen: the generation
+// word as it was (0 without one).  scan: the abs-max of the whole input, by this workgroup alone.
+template <class Scan>
+__device__ __forceinline__ float onepass_exchange(int g, float m, unsigned nonce, unsigned gen, unsigned long long* words,
+                                                  unsigned long long* gen_word, int polls, int G, float* shared_max, Scan scan) {
   const int tid = threadIdx.x;
-  static_assert(kOnePassMaxGroups == kOnePassBoards * kOnePassBoards, "a group's slots and a board's words are polled by the same lanes");
+  static_assert(kOnePassMaxGroups == 4 * kWave, "four words a lane");
   int polls_left = polls;   // (of the whole workgroup: only its first wave waits)
-  // n words from p with this launch's tag, polled by the first lanes of wave 0: their maximum, in *found whether all came
-  auto collect = [&](const unsigned long long* p, int n, bool* found) {
+  if(tid < kWave) {
+    const unsigned tag = (nonce + gen) | 0x80000000u;   // never 0: a cleared word does not match
+    const unsigned long long own = onepass_word(tag, m);
+    const int shift = G > 16 ? 28 - __builtin_clz(G - 1) : 0;   // 1 << shift lines of 16 words: the fewest that hold G
+    unsigned long long* const put = words + (tid % kOnePassCopies) * kOnePassMaxGroups + ((g & ((1 << shift) - 1)) * 16 + (g >> shift));
+    const unsigned long long* const get = words + (g % kOnePassCopies) * kOnePassMaxGroups;
+    if(tid < kOnePassCopies) __hip_atomic_store(put, own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    auto word = [&](int i) __attribute__((always_inline)) {
+      const int at = i * kWave + tid, from = (at % 16 << shift) + at / 16;   // (lanes past the words: one of theirs again)
+      return i * kWave < 16 << shift ? __hip_atomic_load(get + (from < G && at < 16 << shift ? at : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : own;
+    };
+    auto tag_of = [](unsigned long long w) { return (unsigned)(w >> 32); };
+    auto value_of = [](unsigned long long w) { return __uint_as_float((unsigned)w); };
     float v = 0.0f;
-    *found = false;
+    bool found = false;
+    __builtin_amdgcn_s_sleep(16);   // (1024 clocks, see above)
     for(; onepass_patience(polls_left); onepass_polled(polls_left)) {
-      const unsigned long long w = __hip_atomic_load(p + min(tid, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      v = __uint_as_float((unsigned)w);
-      *found = __all((unsigned)(w >> 32) == tag);
-      if(*found) break;
+      const unsigned long long w0 = word(0), w1 = word(1), w2 = word(2), w3 = word(3);
+      v = fmaxf(fmaxf(value_of(w0), value_of(w1)), fmaxf(value_of(w2), value_of(w3)));
+      found = __all(tag_of(w0) == tag && tag_of(w1) == tag && tag_of(w2) == tag && tag_of(w3) == tag);
+      if(found) break;
       __builtin_amdgcn_s_sleep(1);
     }
-    return wave_max(v);
-  };
-  if(tid < kWave) {
-    bool found = true;
-    if(tid == 0) __hip_atomic_store(&slots[g], onepass_word(tag, m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool leads = g % kOnePassBoards == 0;
-    if(leads) {
-      const float v = collect(slots + g, min(kOnePassBoards, G - g), &found);
-      if(found && tid < kOnePassBoards)
-        __hip_atomic_store(&boards[tid * kOnePassBoardWords + g / kOnePassBoards], onepass_word(tag, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = wave_max(v);
+    if(gen_word) {
+      // Words that went out behind the generation's end carry the next replay's tag.  Their workgroup never finds those of
+      // workgroup 0, which ended before it read the generation, so it comes here without an answer and takes them back.
+      if(!found && tid < kOnePassCopies) __hip_atomic_store(put, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // the next replay expects another tag; every workgroup of this one has read the generation by now, or will find its
+      // words unanswered and help itself
+      if(g == 0 && tid == 0) __hip_atomic_store(gen_word, (unsigned long long)(gen + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    float v = 0.0f;
-    if(found) {
-      v = collect(boards + (g % kOnePassBoards) * kOnePassBoardWords, (G + kOnePassBoards - 1) / kOnePassBoards, &found);
-      // A group's words that went out behind the generation's end (below) carry the next launch's tag; the words of
-      // workgroup 0's group then never match, so they are taken back here.
-      if(leads && !found && tid < kOnePassBoards)
-        __hip_atomic_store(&boards[tid * kOnePassBoardWords + g / kOnePassBoards], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if(tid == 0) {
-      // answered or not, this launch is done with the slot
-      __hip_atomic_store(&slots[g], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      // the next launch (or replay) expects another tag; every workgroup of this launch has read
-      // the generation by now, or will find its words unanswered and help itself
-      if(g == 0) __hip_atomic_store(gen_word, (unsigned long long)(gen + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *shared_max = found ? v : -1.0f;
-    }
+    if(tid == 0) *shared_max = found ? v : -1.0f;
   }
   __syncthreads();
   const float all = *shared_max;

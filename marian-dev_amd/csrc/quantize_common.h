@@ -8,17 +8,16 @@ namespace marian_hip {
 
 constexpr int kQuantThreads = 256;
 constexpr int kMaxPartials = 1024;                  // floats of workspace used by the two-pass forms
-// Workspace layout: [0, 4 KB) abs-max partials of the two-pass forms; then the hand-over area of the
-// one-pass forms: 256 arrival slots of 8 bytes, one generation word, and 16 boards of 16 words,
-// 256 bytes apart.
-constexpr int kOnePassMaxGroups = 256;              // workgroups of the one-pass form (one per CU)
-constexpr int kOnePassBoards = 16;                  // workgroups of a group, and boards that its maximum is published on
-constexpr int kOnePassBoardWords = 32;              // 8-byte words between two boards (16 of them a group's)
-constexpr size_t kOnePassSlotsOffset = kMaxPartials * sizeof(float);
-constexpr size_t kOnePassGenOffset = kOnePassSlotsOffset + kOnePassMaxGroups * 8;
-constexpr size_t kOnePassBoardOffset = 8192;
-constexpr size_t kWorkspaceBytes = kOnePassBoardOffset + kOnePassBoards * kOnePassBoardWords * 8;   // 12 KB
-static_assert(kOnePassGenOffset + 8 <= kOnePassBoardOffset, "workspace layout");
+// Workspace layout: [0, 4 KB) abs-max partials of the two-pass forms; [2, 10 KB) four copies of the words that workgroups
+// exchange within a launch, 256 of 8 bytes each; then a generation word.  The first copy lies over partials: a launch uses
+// either, and what one leaves means nothing to the other (a word that counts has its top bit set, where a partial, which is not
+// negative, has none; partials are written before they are read).
+constexpr int kOnePassMaxGroups = 256;              // workgroups of the one-pass forms (one per CU)
+constexpr int kOnePassCopies = 4;
+constexpr size_t kOnePassWordsOffset = 2048;
+constexpr size_t kOnePassGenOffset = kOnePassWordsOffset + kOnePassCopies * kOnePassMaxGroups * 8;
+constexpr size_t kWorkspaceBytes = 12288;
+static_assert(kOnePassGenOffset + 8 <= kWorkspaceBytes && kOnePassGenOffset >= kMaxPartials * sizeof(float), "workspace layout");
 constexpr int kSingleBlockThreads = 1024;
 constexpr int kSingleBlockMaxElems = 32 * 1024;     // one workgroup does abs-max and quantize (beyond: 8.6 us against 6.4 us for two launches)
 

@@ -70,20 +70,18 @@ __global__ __launch_bounds__(kSingleBlockThreads) void prepare_a_single_block_ke
 template <int SETS>
 __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __restrict__ x, unsigned n16,
                                                                  int8_t* __restrict__ out,
-                                                                 unsigned long long* slots,
+                                                                 unsigned long long* words,
                                                                  unsigned long long* gen_word,
-                                                                 unsigned long long* boards,
                                                                  unsigned nonce, int polls, int groups) {
   __shared__ float red[1024 / kWave];
   __shared__ float shared_max;
-  __shared__ unsigned shared_tag;
   __shared__ __attribute__((aligned(16))) uint32_t turn[1024 * 4];   // 16 bytes per thread
   const int tid = threadIdx.x, quad = tid / 4, qlane = tid % 4;
   const int G = groups, g = blockIdx.x;
-  // (one thread per workgroup asks for the generation: every access to the word is served by the
+  // (one wave per workgroup asks for the generation: every access to the word is served by the
   // same memory channel, one after the other)
   unsigned gen = 0;
-  if(tid == 0 && G > 1) gen = (unsigned)__hip_atomic_load(gen_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if(tid < kWave && gen_word) gen = (unsigned)__hip_atomic_load(gen_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // set j of this workgroup: quads (g * SETS + j) * 256 .. + 255, a quad = four consecutive 16-value
   // groups (256 contiguous bytes); load e brings lane i of the quad the i-th four values of group e
   v4f vals[SETS][4];
@@ -104,13 +102,10 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
 #pragma unroll
       for(int e = 0; e < 4; ++e) m = abs4max(vals[j][e], m);
     }
-  if(tid == 0) shared_tag = (nonce + gen) | 0x80000000u;   // never 0: a cleared word does not match
-  m = block_max<1024 / kWave>(m, red);   // (its barriers also publish shared_tag)
-  const unsigned tag = shared_tag;
-
+  m = block_max<1024 / kWave>(m, red);
   float amax = m;
   if(G > 1)
-    amax = onepass_exchange<1024>((int)blockIdx.x, m, gen, tag, slots, gen_word, boards, polls, G, red, &shared_max,
+    amax = onepass_exchange((int)blockIdx.x, m, nonce, gen, words, gen_word, polls, G, &shared_max,
                                   [&] { return onepass_scan<1024>(x, (size_t)n16 * 4, red); });
   const float qm = quant_mult_from_maxabs(amax);
   const bool finite = qm < __builtin_inff();
@@ -240,17 +235,15 @@ __global__ __launch_bounds__(256) void quantize_b_transpose_kernel(
 // on the host: 1024 x 1024 in two of them 7.9 us, in one 5.7.
 template <int TILES>
 __global__ __launch_bounds__(TILES * 256) void prepare_b_onepass_kernel(const float* __restrict__ W, int K, int N,
-                                                                        int8_t* __restrict__ out, unsigned long long* slots,
-                                                                        unsigned long long* gen_word,
-                                                                        unsigned long long* boards, unsigned nonce,
+                                                                        int8_t* __restrict__ out, unsigned long long* words,
+                                                                        unsigned long long* gen_word, unsigned nonce,
                                                                         int polls, int groups, int tiles_n, int tiles) {
   __shared__ float red[TILES * 256 / kWave];
   __shared__ float shared_max;
-  __shared__ unsigned shared_tag;
   __shared__ uint32_t turn[TILES][64][17];
   const int tid = threadIdx.x, sub = tid / 256, thread = tid % 256;
   unsigned gen = 0;
-  if(tid == 0 && groups > 1) gen = (unsigned)__hip_atomic_load(gen_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if(tid < kWave && gen_word) gen = (unsigned)__hip_atomic_load(gen_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const int wanted = __builtin_amdgcn_readfirstlane((int)blockIdx.x * TILES + sub);
   const bool live = wanted < tiles;
   const int t = live ? wanted : 0;   // (read again and not written: a repeated value does not change a maximum)
@@ -259,12 +252,11 @@ __global__ __launch_bounds__(TILES * 256) void prepare_b_onepass_kernel(const fl
   load_b_tile(W, K, N, n0, k0, thread, v);
 #pragma unroll
   for(int k = 0; k < 16; ++k) m = fmaxf(m, fabsf(v[k]));
-  if(tid == 0) shared_tag = (nonce + gen) | 0x80000000u;   // never 0: a cleared word does not match
-  m = block_max<TILES * 256 / kWave>(m, red);   // (its barriers also publish shared_tag)
+  m = block_max<TILES * 256 / kWave>(m, red);
   float amax = m;
   if(groups > 1)
-    amax = onepass_exchange<TILES * 256>((int)blockIdx.x, m, gen, shared_tag, slots, gen_word, boards, polls, groups, red, &shared_max,
-                                         [&] { return onepass_scan<TILES * 256>(W, (size_t)K * N / 4, red); });
+    amax = onepass_exchange((int)blockIdx.x, m, nonce, gen, words, gen_word, polls, groups, &shared_max,
+                            [&] { return onepass_scan<TILES * 256>(W, (size_t)K * N / 4, red); });
   const float qm = quant_mult_from_maxabs(amax);
   store_b_tile(v, qm, turn[sub], K, N, n0, k0, thread, live, out);
   if(blockIdx.x == 0 && tid == 0) *reinterpret_cast<float*>(out + (size_t)K * N) = qm;
