@@ -617,6 +617,23 @@ int launch_stream_auto(const GemmArgs& a, hipStream_t st, int force_wide) {
   return launch_stream_mt<8>(a, st, wide);
 }
 
+// Small tiles where larger ones would leave CUs idle.  A CU takes in (rows + columns) x K bytes of its tile, so a long K asks
+// for the smallest tiles that still find a CU each (300 x 4096 x 1024: 128x64 tiles 10.6 us, 64x64 8.3, 32x64 7.6; 1000 x 4096 x 1024
+// 11.1, 9.1, 10.7 - two of the last to a CU; 1300 x 2048 x 512 6.9, 5.9, 6.5; 1000 x 512 x 512 4.7, 4.0, 3.7; against
+// gemm_stream32_kernel 256 x 3072 x 768 8.4 and 6.4, 200 x 4096 x 4096 10.8 and 8.9, but 256 x 1024 x 1024 3.94 and 3.95).
+// t64x64_shared: short rows, several tiles to a CU, one of which is loaded while another is multiplied or written out
+// (1000 x 512 x 2048 5.2 -> 4.8 us, 1500 x 512 x 2048 6.5 -> 5.4, 1000 x 768 x 3072 7.1 -> 6.5, but 2050 x 512 x 2048 7.9 -> 8.3,
+// 1200 x 768 x 3072 7.0 -> 7.4, 2050 x 1024 x 1024 6.6 -> 7.4).  (Measurement id 340: none of them.)
+enum class SmallTiles { none, t32x64, t64x64, t64x64_shared };
+SmallTiles small_tiles(const GemmArgs& a, long long columns) {   // columns: of 64, each a tile column
+  if(a.K % 128 != 0 || a.dump || kernel_override() % 1000 == 340) return SmallTiles::none;
+  const long long cus = compute_units(), t64 = columns * ((a.M + 63) / 64);
+  if(columns * ((a.M + 31) / 32) <= cus) return SmallTiles::t32x64;
+  if(t64 <= cus) return SmallTiles::t64x64;
+  if(a.K < 1024 && t64 <= (a.K <= 512 ? 4 : 3) * cus) return SmallTiles::t64x64_shared;
+  return SmallTiles::none;
+}
+
 int launch_gemm(const GemmArgs& a, hipStream_t st) {
 #ifdef MARIAN_HIP_TUNING
   const int which = kernel_override() % 1000;
@@ -665,6 +682,10 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
     case 376: if(a.K % 128 == 0) return launch_big_split<128, 64, 2, 2, 4, true>(a, st); break;
     case 377: if(a.K % 128 == 0) return launch_big_split<128, 64, 2, 2, 4, false>(a, st); break;
     case 374: if(a.K % 128 == 0) return launch_big_split<128, 128, 2, 2, 4, false>(a, st); break;
+    // 379, 380: the split form in small tiles; 381: 64x64 tiles without loading waves
+    case 379: if(a.K % 128 == 0) return launch_big_split<32, 64, 1, 2, 4, true>(a, st); break;
+    case 380: if(a.K % 128 == 0) return launch_big_split<64, 64, 2, 2, 4, true>(a, st); break;
+    case 381: return launch_big<64, 64, 2, 2, 2, true, true>(a, st);
     case 364: return launch_big_auto<128, 128, 2, 2, 3, false>(a, st, 1);
     case 368: return launch_big_auto<128, 128, 2, 2, 3, true>(a, st, 1);
     case 501: return launch_stream32_auto<kPrequant>(a, FusedSrc(), st, 0);
@@ -683,11 +704,18 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
   //  - otherwise the 32x32x32 MFMA kernel, which also tiles M (shortlisted output layer, M = 256)
   const int tiles32 = (a.n_out + 31) / 32;
   if(a.M <= 8 || (a.M <= 16 && tiles32 < 512)) return launch_stream_auto(a, st, 2);
-  //    (few columns, M up to 512; beyond 256 rows with K >= 2048 and 1024 or more columns the
-  //    128x64-tile kernel below is 20 % faster)
-  if(a.M <= 128 || (a.M <= 512 && tiles32 < 128 &&
-                    (a.M <= 256 || a.K < 2048 || tiles32 < 32)))
+  //    (few columns, M up to 512; beyond 256 rows with K >= 2048 and 1024 or more columns larger tiles
+  //    are 20 % faster), but for what small tiles do better: more than 256 rows, or long rows
+  const SmallTiles small = small_tiles(a, (a.n_out + 63) / 64);
+  if((a.M <= 128 || (a.M <= 512 && tiles32 < 128 && (a.M <= 256 || a.K < 2048 || tiles32 < 32))) &&
+     (small == SmallTiles::none || a.idx || a.M <= 64 || (a.M <= 256 && a.K < 2048)))
     return launch_stream32_auto<kPrequant>(a, FusedSrc(), st, 0);
+  switch(small) {
+    case SmallTiles::t32x64: return launch_big_split<32, 64, 1, 2, 4, true>(a, st);
+    case SmallTiles::t64x64: return launch_big_split<64, 64, 2, 2, 4, true>(a, st);
+    case SmallTiles::t64x64_shared: return launch_big<64, 64, 2, 2, 2, true, true>(a, st);
+    case SmallTiles::none: break;
+  }
   // large outputs: 256x256 tiles (one per CU keeps operand traffic lowest); otherwise 128x128
   // tiles with a three-deep LDS ring so that enough loads are in flight per CU
   const long long tiles256 = ((a.M + 255) / 256) * (long long)((a.n_out + 255) / 256);
@@ -747,6 +775,12 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
                   : launch_big_ragged_as<128, 128, 2, 4, 2, false, false>(a, r, st);
     }
   }
+  // More than one tile to a CU, fewer than two: the eight-wave form again, two workgroups to a CU, instead of two rounds of the
+  // four-wave form (1500 x 1024 x 4096 15.9 -> 10.9 us, 3000 x 2048 x 2048 23.7 -> 17.4, 2500 x 4096 x 2048 35.9 -> 27.8).
+  if(tiles128 > compute_units() && kernel_override() % 1000 != 340) {
+    if(stream_out) return launch_big<128, 128, 2, 4, 2, true, true>(a, st);
+    return launch_big<128, 128, 2, 4, 2>(a, st);
+  }
   if(split) return stream_out ? launch_big_split<128, 128, 2, 2, 3, true>(a, st) : launch_big_split<128, 128, 2, 2, 3, false>(a, st);
   if(stream_out) return launch_big<128, 128, 2, 2, 3, true, true>(a, st);
   return launch_big<128, 128, 2, 2, 3>(a, st);
@@ -779,6 +813,7 @@ GroupTable group_table(int64_t n_groups, const int8_t* const* Bq, const float* c
 //    while the next is multiplied (4096 x 1024 x 3072 19.6 us, the next form 22.6, three launches 26.7 - 32);
 //  - a 128x128 tile or more per CU: the eight-wave form, two workgroups to a CU (3000 x 512 x 1536 8.9 us,
 //    1400 x 1024 x 3072 11.6; three launches 14.8 and 16.9);
+//  - small tiles as for a single matrix (small_tiles);
 //  - fewer: 128x64 tiles in the split form, which CUs that idle leave room for (1000 x 512 x 1536 5.1 us,
 //    600 x 1024 x 3072 6.0; three launches 13.9 and 16.3).
 template <typename CFG, int THREADS, auto KERNEL>
@@ -793,10 +828,11 @@ int launch_grouped_as(const GemmArgs& a, const GroupTable& g, int tiles_m, hipSt
 }
 int launch_big_grouped(const GemmArgs& a, int64_t n_groups, const int8_t* const* Bq, const float* const* bias, float* const* out,
                        const int64_t* N, hipStream_t st) {
-  long long columns = 0, tiles128 = 0;
+  long long columns = 0, columns64 = 0, tiles128 = 0;
   bool pairs = a.M % PairCfg::BM == 0 && a.K <= 1536 && a.K / PairCfg::BK >= PairCfg::kSideBlocks;
   for(int64_t g = 0; g < n_groups; ++g) {
     columns += N[g];
+    columns64 += (N[g] + 63) / 64;
     tiles128 += (N[g] + 127) / 128;
     pairs = pairs && N[g] % (2 * PairCfg::BN) == 0 && (!bias || !bias[g] || aligned(bias[g], 16));
   }
@@ -805,6 +841,24 @@ int launch_big_grouped(const GemmArgs& a, int64_t n_groups, const int8_t* const*
   if(pairs && (a.M / 256) * (columns / 256) >= 192)
     return launch_grouped_as<PairCfg, PairCfg::kThreads, gemm_pair_group_kernel<true>>(
         a, group_table(n_groups, Bq, bias, out, N, 2 * PairCfg::BN), a.M / PairCfg::BM, st);
+  switch(small_tiles(a, columns64)) {
+    case SmallTiles::t32x64: {
+      using Cfg = BigCfg<32, 64, 1, 2, 4>;
+      return launch_grouped_as<Cfg, 2 * Cfg::kThreads, gemm_mfma32_group_kernel<32, 64, 1, 2, 4, true, true>>(
+          a, group_table(n_groups, Bq, bias, out, N, 64), (a.M + 31) / 32, st);
+    }
+    case SmallTiles::t64x64: {
+      using Cfg = BigCfg<64, 64, 2, 2, 4>;
+      return launch_grouped_as<Cfg, 2 * Cfg::kThreads, gemm_mfma32_group_kernel<64, 64, 2, 2, 4, true, true>>(
+          a, group_table(n_groups, Bq, bias, out, N, 64), (a.M + 63) / 64, st);
+    }
+    case SmallTiles::t64x64_shared: {
+      using Cfg = BigCfg<64, 64, 2, 2, 2>;
+      return launch_grouped_as<Cfg, Cfg::kThreads, gemm_mfma32_group_kernel<64, 64, 2, 2, 2, true, false>>(
+          a, group_table(n_groups, Bq, bias, out, N, 64), (a.M + 63) / 64, st);
+    }
+    case SmallTiles::none: break;
+  }
   if(tiles128 >= compute_units()) {
     using Cfg = BigCfg<128, 128, 2, 4, 2>;
     const GroupTable t = group_table(n_groups, Bq, bias, out, N, 128);

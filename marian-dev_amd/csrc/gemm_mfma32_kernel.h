@@ -174,9 +174,8 @@ __device__ __forceinline__ void store_tile32_any(const v16i& acc, char* out, siz
 // take a compact block of tiles - 4 tiles along n by a run along m - so that the XCD's L2 holds
 // few weight panels and few activation panels at a time.
 __device__ __forceinline__ void xcd_tile(int tiles_n, int tiles_m, int block, int& tn, int& tm) {
-  const int total = tiles_n * tiles_m;
-  int t = block;
-  if(total % 8 == 0) t = (block % 8) * (total / 8) + block / 8;
+  const int total = tiles_n * tiles_m, xcd = block % 8;
+  const int t = xcd * (total / 8) + min(xcd, total % 8) + block / 8;   // (the first total % 8 of them have one more)
   const int band = 4;
   const int b = t / (band * tiles_m);
   const int r = t % (band * tiles_m);
