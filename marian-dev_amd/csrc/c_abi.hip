@@ -634,6 +634,12 @@ SmallTiles small_tiles(const GemmArgs& a, long long columns) {   // columns: of 
   return SmallTiles::none;
 }
 
+// Whether an output is written with non-temporal stores, which leave nothing dirty in the L2 caches for the end of the launch: up
+// to 56 MB (2050 x 1024 x 4096 19.7 -> 18.1 us, 3000 x 1024 x 4096 22.9 -> 21.6, but 4096 x 1024 x 4096 26.3 and 27.2), and where rows
+// begin between lines, which such stores then write in parts, up to 14 MB (1500 x 1024 x 2056 9.34 and 9.30 us, 1500 x 1024 x 3000 10.9 and
+// 11.5, 2200 x 1024 x 3000 12.5 and 15.2).
+bool streams_out(long long M, long long n_out) { return M * n_out * 4 <= (n_out % 32 == 0 ? 56ll << 20 : 14ll << 20); }
+
 int launch_gemm(const GemmArgs& a, hipStream_t st) {
 #ifdef MARIAN_HIP_TUNING
   const int which = kernel_override() % 1000;
@@ -719,8 +725,7 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
   // large outputs: 256x256 tiles (one per CU keeps operand traffic lowest); otherwise 128x128
   // tiles with a three-deep LDS ring so that enough loads are in flight per CU
   const long long tiles256 = ((a.M + 255) / 256) * (long long)((a.n_out + 255) / 256);
-  // an output that would fit the L2 caches (8 x 4 MB) is streamed out with non-temporal stores
-  const bool stream_out = (long long)a.M * a.n_out * 4 <= (32ll << 20) && !a.dump;
+  const bool stream_out = streams_out(a.M, a.n_out) && !a.dump;
   if(tiles256 >= 192) {
     // short K: the fp32 output is most of the bytes; write one tile out while the next is multiplied
     if(a.K <= 1536 && kernel_override() % 1000 != 332) {
@@ -737,10 +742,16 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
     if(stream_out) return launch_big_auto<256, 256, 2, 4, 2, true>(a, st, 1);
     return launch_big_auto<256, 256, 2, 4, 2, false>(a, st, 1);
   }
-  // two or more 128x128 tiles per CU: eight waves and two LDS stages, so that two workgroups share
-  // a CU and one multiplies while the other writes its tile out; otherwise four waves, three stages
+  // two or more 128x128 tiles per CU: 256x256 tiles again, on half of the CUs and more, which take in half the operands
+  // (2300 x 1024 x 4096 20.5 -> 18.3 us, 2500 x 4096 x 4096 53.8 -> 45.9, 3000 x 768 x 3072 16.8 -> 14.6); where K is 64 modulo 128, and
+  // rows are short, eight waves and two LDS stages, so that two workgroups share a CU and one multiplies while the other writes its tile
+  // out (2500 x 512 x 4096 13.1 and 13.5 us); otherwise four waves, three stages
   const long long tiles128 = ((a.M + 127) / 128) * (long long)((a.n_out + 127) / 128);
   if(tiles128 >= 2 * compute_units()) {
+    if(a.K > 512 && a.K % 128 == 0) {
+      if(stream_out) return launch_big_auto<256, 256, 2, 4, 2, true>(a, st, 1);
+      return launch_big_auto<256, 256, 2, 4, 2, false>(a, st, 1);
+    }
     if(stream_out) return launch_big_auto<128, 128, 2, 4, 2, true>(a, st, 2);
     return launch_big_auto<128, 128, 2, 4, 2, false>(a, st, 2);
   }
@@ -837,7 +848,8 @@ int launch_big_grouped(const GemmArgs& a, int64_t n_groups, const int8_t* const*
     pairs = pairs && N[g] % (2 * PairCfg::BN) == 0 && (!bias || !bias[g] || aligned(bias[g], 16));
   }
   tiles128 *= (a.M + 127) / 128;
-  const bool stream_out = (long long)a.M * columns * 4 <= (32ll << 20);   // (as for a single matrix)
+  bool stream_out = true;   // (as for a single matrix)
+  for(int64_t g = 0; g < n_groups; ++g) stream_out = stream_out && (N[g] == 0 || streams_out((long long)a.M * columns / N[g], N[g]));
   if(pairs && (a.M / 256) * (columns / 256) >= 192)
     return launch_grouped_as<PairCfg, PairCfg::kThreads, gemm_pair_group_kernel<true>>(
         a, group_table(n_groups, Bq, bias, out, N, 2 * PairCfg::BN), a.M / PairCfg::BM, st);
