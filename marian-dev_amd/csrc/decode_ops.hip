@@ -1193,6 +1193,27 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     bias4[it] = *reinterpret_cast<const v4f*>(b ? b + h * 64 + (tg % 2) * 32 + pc * 4 : reinterpret_cast<const float*>(p.Bq[0]));
   }
 
+  // The keys and values are asked for last - a wave's loads complete in the order of their issue, and they are needed
+  // last.  No branches around them (positions past the end repeat the last one; the number of loads is the kernel's), so that the
+  // waits in front of the earlier loads' uses count exactly.  Behind a layer norm, whose reductions they would come in
+  // between, only when the abs-max is there: a step of 65 x 512 over 47 source positions 317.0 -> 315.5 us with them here, one of 6 x 512
+  // over 23, with layer norms, 209.7 and 210.3.
+  auto load_stage = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for(int seg = 0; seg < SEGS; ++seg) {
+      const unsigned entry = (unsigned)(sent_base + (seg >> 1)) * (unsigned)p.heads + (unsigned)h;
+      const float* src = ((seg & 1) ? p.v_cache : p.k_cache) + (size_t)entry * p.kv_cap * 64 + (tid % 16) * 4;
+#pragma unroll
+      for(int j = 0; j < PASSES; ++j)
+        stage[seg][j] = *reinterpret_cast<const v4f*>(src + (size_t)min(tid / 16 + 32 * j, p.len - 1) * 64);
+    }
+  };
+  if constexpr(STAGED && !NORM) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_stage();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   HeldRows<HELD> held;
   if constexpr(HELD > 0) {   // (as buffers: a wave without a row asks for nothing, and the waits still count)
     __builtin_amdgcn_sched_barrier(0);
@@ -1225,20 +1246,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) amax = fmaxf(amax, pm[i]);
   }
   amax = block_max<kProjThreads / 64>(amax, red);
-  // The keys and values are asked for last - a wave's loads complete in the order of their issue,
-  // and they are needed last - and only now: in front of the abs-max values they would delay them.
-  // No branches around them (positions past the end repeat the last one; the number of loads is
-  // the kernel's), so that the waits in front of the earlier loads' uses count exactly.
-  if constexpr(STAGED) {
-#pragma unroll
-    for(int seg = 0; seg < SEGS; ++seg) {
-      const unsigned entry = (unsigned)(sent_base + (seg >> 1)) * (unsigned)p.heads + (unsigned)h;
-      const float* src = ((seg & 1) ? p.v_cache : p.k_cache) + (size_t)entry * p.kv_cap * 64 + (tid % 16) * 4;
-#pragma unroll
-      for(int j = 0; j < PASSES; ++j)
-        stage[seg][j] = *reinterpret_cast<const v4f*>(src + (size_t)min(tid / 16 + 32 * j, p.len - 1) * 64);
-    }
-  }
+  if constexpr(STAGED && NORM) load_stage();
   const float aqm = quant_mult_from_maxabs(amax);
   const bool finite = aqm < __builtin_inff();
   float unquant[NPROJ];
