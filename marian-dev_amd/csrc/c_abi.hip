@@ -711,10 +711,26 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
   const int tiles32 = (a.n_out + 31) / 32;
   if(a.M <= 8 || (a.M <= 16 && tiles32 < 512)) return launch_stream_auto(a, st, 2);
   //    (few columns, M up to 512; beyond 256 rows with K >= 2048 and 1024 or more columns larger tiles
-  //    are 20 % faster), but for what small tiles do better: more than 256 rows, or long rows
+  //    are 20 % faster), but for what small tiles do better: more than 64 rows - 128 x 768 x 3072 4.6 and 3.9 us, 200 x 768 x 2048 4.6 and
+  //    4.2, 128 x 1280 x 4096 7.1 and 5.3, 256 x 1792 x 3072 10.0 and 6.8, weights from memory -, except where the
+  //    stream form's K split comes out even (129 x 512 x 1024 3.2 and 3.7, 70 x 1024 x 4096 4.3 and 4.6; but 160 x 1024 x 2048 4.3 and 4.2)
   const SmallTiles small = small_tiles(a, (a.n_out + 63) / 64);
+  const bool even = small == SmallTiles::t32x64 && ((a.K == 512 && a.M <= 256) || (a.K == 1024 && a.M <= 128));
+  const bool tiles_fit = small == SmallTiles::t32x64 || small == SmallTiles::t64x64;
+  // Wide outputs of 65 .. 128 rows (scores over a vocabulary), of which the tiles above do not get a CU each: tiles as high as the rows,
+  // 128x64 in the split form up to half a 128x128 tile a CU and for long rows, else 128x128, two workgroups to a CU.  Weights from memory
+  // (their copies in turn), 128 rows, the stream form and now: x 512 x 12000 7.3 and 5.5 us (64x64 tiles 5.8), x 1024 x 8200 10.8 and 7.4 (8.1),
+  // x 1024 x 32000 16.1 and 11.9 (128x64 13.6, 64x64 16.1), x 512 x 32000 10.5 and 8.3, x 1024 x 50000 21.5 and 18.8, x 2048 x 12000 17.6 and
+  // 10.6, 65 x 512 x 32000 8.6 and 7.8; at 256 rows 64x64 tiles are behind the forms below (x 1024 x 12000 11.1 and 9.1).
+  if(!a.idx && !a.dump && a.M > 64 && a.M <= 128 && a.K % 128 == 0 && !tiles_fit && kernel_override() % 1000 != 340) {
+    const long long cus = compute_units(), cols64 = (a.n_out + 63) / 64, cols128 = (a.n_out + 127) / 128;
+    if(!streams_out(a.M, a.n_out)) return launch_big<128, 128, 2, 4, 2>(a, st);
+    if(a.K > 1024 && cols64 <= cus) return launch_big_split<128, 64, 2, 2, 4, true>(a, st);
+    if(a.K > 1024 ? cols128 <= cus : 2 * cols128 <= cus) return launch_big_split<128, 64, 2, 2, 3, true>(a, st);
+    return launch_big<128, 128, 2, 4, 2, true, true>(a, st);
+  }
   if((a.M <= 128 || (a.M <= 512 && tiles32 < 128 && (a.M <= 256 || a.K < 2048 || tiles32 < 32))) &&
-     (small == SmallTiles::none || a.idx || a.M <= 64 || (a.M <= 256 && a.K < 2048)))
+     (small == SmallTiles::none || a.idx || a.M <= 64 || even))
     return launch_stream32_auto<kPrequant>(a, FusedSrc(), st, 0);
   switch(small) {
     case SmallTiles::t32x64: return launch_big_split<32, 64, 1, 2, 4, true>(a, st);
@@ -775,8 +791,10 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
   // A few rows or columns more than one 128x128 tile per CU: whole tiles plus small ones, by the
   // eight-wave form, two of whose workgroups share a CU - the small tiles then run beside the whole
   // ones from the start (measured: 2050 x 1024 x 2056 11.7 instead of 15.4 us with the four-wave form,
-  // whose 96 KB of LDS leave no room for a second workgroup, and 17.3 us with 289 tiles alike).
-  {
+  // whose 96 KB of LDS leave no room for a second workgroup, and 17.3 us with 289 tiles alike).  Not for two whole
+  // rows of tiles, where the small ones are many columns (weights from memory: 256 x 512 x 20000 12.7 us, with 128x128 tiles alone 11.0,
+  // 256 x 1024 x 32000 18.4 and 17.1; but 220 x 1024 x 20000 13.3 and 14.9).
+  if(a.M != 256 || kernel_override() % 1000 == 340) {
     const Ragged r = plan_ragged(a, 128, 128, 64, 128, 128, 64, 1);
     if(r.use) {
       const bool amax = big_leaves_absmax(a, r.workgroups);
