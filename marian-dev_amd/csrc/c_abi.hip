@@ -969,11 +969,11 @@ unsigned long long* onepass_generation(void* workspace, hipStream_t st) {
   return recorded(st) ? reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(workspace) + kOnePassGenOffset) : nullptr;
 }
 
-int absmax_blocks(size_t n4) {
+int absmax_blocks(size_t n4, int most = kMaxPartials) {   // most: partials that there is room for
   size_t per_block = (size_t)kQuantThreads * 4;  // four 16-byte loads per thread, all in flight
   size_t g = (n4 + per_block - 1) / per_block;
   if(g < 1) g = 1;
-  if(g > (size_t)kMaxPartials) g = kMaxPartials;
+  if(g > (size_t)most) g = (size_t)most;
   return (int)g;
 }
 
@@ -1283,7 +1283,7 @@ static int affine_f32_impl(const float* A, int8_t* Aq, const int8_t* Bq, const f
 // abs-max of a finished output for the next call, when the kernel that wrote it did not leave it
 static int absmax_after(const float* out, int64_t M, int64_t n_out, float* absmax_out, hipStream_t st) {
   const size_t n = (size_t)M * (size_t)n_out;
-  const int g = absmax_blocks(n / 4);   // n_out % 8 == 0; g <= 1024 partials
+  const int g = absmax_blocks(n / 4, 1024);   // n_out % 8 == 0; four workgroups to a CU
   MH_LAUNCH(zero_floats_kernel, dim3(2), dim3(kQuantThreads), 0, st, absmax_out + g, kAbsmaxSlots - g, 2);
   MH_LAUNCH(absmax_partial_kernel, dim3(g), dim3(kQuantThreads), 0, st, out, n / 4, absmax_out, g);
   MH_HIP(hipGetLastError());

@@ -7,17 +7,16 @@
 namespace marian_hip {
 
 constexpr int kQuantThreads = 256;
-constexpr int kMaxPartials = 1024;                  // floats of workspace used by the two-pass forms
-// Workspace layout: [0, 4 KB) abs-max partials of the two-pass forms; [2, 10 KB) four copies of the words that workgroups
-// exchange within a launch, 256 of 8 bytes each; then a generation word.  The first copy lies over partials: a launch uses
-// either, and what one leaves means nothing to the other (a word that counts has its top bit set, where a partial, which is not
-// negative, has none; partials are written before they are read).
+// Workspace layout, 12 KB: 31 lines of abs-max partials of the two-pass forms, a line with a generation word, four copies of the words that
+// workgroups exchange within a launch, 256 of 8 bytes each.  No two of them overlap: partials are written by one launch
+// and read by the next, and a launch that exchanges words may come in between.
+constexpr int kMaxPartials = 31 * 32;
 constexpr int kOnePassMaxGroups = 256;              // workgroups of the one-pass forms (one per CU)
 constexpr int kOnePassCopies = 4;
-constexpr size_t kOnePassWordsOffset = 2048;
-constexpr size_t kOnePassGenOffset = kOnePassWordsOffset + kOnePassCopies * kOnePassMaxGroups * 8;
-constexpr size_t kWorkspaceBytes = 12288;
-static_assert(kOnePassGenOffset + 8 <= kWorkspaceBytes && kOnePassGenOffset >= kMaxPartials * sizeof(float), "workspace layout");
+constexpr size_t kOnePassGenOffset = kMaxPartials * sizeof(float);
+constexpr size_t kOnePassWordsOffset = 4096;
+constexpr size_t kWorkspaceBytes = kOnePassWordsOffset + kOnePassCopies * kOnePassMaxGroups * 8;
+static_assert(kOnePassGenOffset + 128 == kOnePassWordsOffset && kWorkspaceBytes == 12288, "workspace layout");
 constexpr int kSingleBlockThreads = 1024;
 constexpr int kSingleBlockMaxElems = 32 * 1024;     // one workgroup does abs-max and quantize (beyond: 8.6 us against 6.4 us for two launches)
 

@@ -216,13 +216,13 @@ __global__ __launch_bounds__(256) void quantize_b_transpose_kernel(
   __shared__ uint32_t tile[64][17];
   const int n0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
   // the tile and the partials are requested together
-  float v[16], pm[kMaxPartials / 256];
+  float v[16], pm[(kMaxPartials + 255) / 256];
   load_b_tile(W, K, N, n0, k0, threadIdx.x, v);
 #pragma unroll
-  for(int i = 0; i < kMaxPartials / 256; ++i) pm[i] = partials[min((int)threadIdx.x + i * 256, n_partials - 1)];
+  for(int i = 0; i < (kMaxPartials + 255) / 256; ++i) pm[i] = partials[min((int)threadIdx.x + i * 256, n_partials - 1)];
   float m = 0.0f;
 #pragma unroll
-  for(int i = 0; i < kMaxPartials / 256; ++i) m = fmaxf(m, pm[i]);
+  for(int i = 0; i < (kMaxPartials + 255) / 256; ++i) m = fmaxf(m, pm[i]);
   m = block_max<256 / kWave>(m, red);
   const float qm = quant_mult_from_maxabs(m);
   store_b_tile(v, qm, tile, K, N, n0, k0, threadIdx.x, true, out);
