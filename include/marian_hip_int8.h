@@ -38,7 +38,9 @@
  *   - the workspace (marian_hip_int8_workspace_bytes()): ONE PER STREAM.  It holds the abs-max
  *     partials of the call in flight and the words that workgroups exchange within a launch;
  *     calls on one stream run one after the other and share it, calls on different streams must
- *     each bring their own (a backend object per worker, as in the reference, does that);
+ *     each bring their own (a backend object per worker, as in the reference, does that).  A call
+ *     may be two launches, the second of which reads what the first left there: threads that share
+ *     a stream and its workspace make their calls one at a time (the Python operators see to that);
  *   - the n-best workspace of marian_hip_nbest_beams / marian_hip_logsoftmax_nbest_beams
  *     (include/marian_hip_ops.h): one per stream, for the same reason (arrival counters);
  *   - the static scratch behind marian_hip_int8_affine_f32_static: one per device, so those calls

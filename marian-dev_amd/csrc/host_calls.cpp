@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cmath>
 #include <map>
+#include <mutex>
 #include <optional>
 #include <utility>
 #include <vector>
@@ -121,12 +122,20 @@ inline bool truth(PyObject* o) {
   return v != 0;
 }
 
-// Calls f without the interpreter lock; a status is raised as an error of `where`, or of what f left in *which.
+// Calls f without the interpreter lock, and with `turn` if it is given; a status is raised as an error of `where`, or of what f
+// left in *which.
 template <typename F>
-inline void call(const char* where, F f, const char** which = nullptr) {
-  PyThreadState* s = PyEval_SaveThread();
-  const int status = f();
-  PyEval_RestoreThread(s);
+inline void call(const char* where, F f, const char** which = nullptr, std::mutex* turn = nullptr) {
+  int status;
+  {
+    struct Unlocked {
+      PyThreadState* s = PyEval_SaveThread();
+      ~Unlocked() { PyEval_RestoreThread(s); }
+    } unlocked;
+    std::unique_lock<std::mutex> held;
+    if(turn) held = std::unique_lock<std::mutex>(*turn);
+    status = f();
+  }
   if(status != MARIAN_HIP_OK) {
     if(which && **which) where = *which;
     Ref r(PyObject_CallFunction(raise_status, "is", status, where));
@@ -138,18 +147,28 @@ inline void call(const char* where, F f, const char** which = nullptr) {
 // ---- workspaces: one per device and stream, kept for good (a graph may have recorded one) -------
 struct PerStream {
   at::Tensor workspace;              // abs-max partials, one-pass exchange
+  std::mutex turn;                   // held while a call makes its launches over the workspace
   std::vector<at::Tensor> nbest;     // the last one the largest
   std::vector<at::Tensor> scratch;   // not lent at the moment
 };
 std::map<std::pair<int, hipStream_t>, PerStream> per_stream;   // (looked up with the interpreter lock held)
 
-at::Tensor& workspace(c10::Device d, hipStream_t st) {
+PerStream& with_workspace(c10::Device d, hipStream_t st) {
   PerStream& p = per_stream[{d.index(), st}];
   if(!p.workspace.defined()) {
     at::Tensor made = empty({(int64_t)L.int8_workspace_bytes()}, at::kByte, d);
     if(!p.workspace.defined()) p.workspace = std::move(made);
   }
-  return p.workspace;
+  return p;
+}
+
+// A call whose launches hand each other something in the workspace of its stream.  They follow each other on the stream: where threads
+// share one, the launches of another thread's call would otherwise come in between and write over it.
+template <typename F>
+inline void call_over(PerStream& p, const char* where, F f, const char** which = nullptr) {
+  void* const ws = p.workspace.data_ptr();
+  const size_t bytes = (size_t)p.workspace.numel();
+  call(where, [&] { return f(ws, bytes); }, which, &p.turn);
 }
 
 // Memory of one call that nobody sees afterwards: what a stream's earlier calls gave back, which spares the call an allocation
@@ -333,11 +352,11 @@ PyObject* py_affine_or_dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return wrap(std::move(out));
   }
   const Scratch aq(x.M * x.K + 4, d, st);
-  const at::Tensor& ws = workspace(d, st);
-  call("affineOrDot", [&] {
+  PerStream& ps = with_workspace(d, st);
+  call_over(ps, "affineOrDot", [&](void* ws, size_t ws_bytes) {
     return L.int8_affine_f32(fptr(x.a), static_cast<int8_t*>(aq.data()), static_cast<const int8_t*>(x.b.t->const_data_ptr()),
                              fptr(x.bias), x.idx ? static_cast<const uint32_t*>(x.idx->const_data_ptr()) : nullptr,
-                             x.idx ? x.n_out : 0, fptr_mut(out), x.M, x.K, x.b.cols, scale, relu, ws.data_ptr(), (size_t)ws.numel(), st);
+                             x.idx ? x.n_out : 0, fptr_mut(out), x.M, x.K, x.b.cols, scale, relu, ws, ws_bytes, st);
   });
   return wrap(std::move(out));
   MH_END
@@ -358,12 +377,12 @@ PyObject* py_affine_f32(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   at::Tensor omax;
   if(want) omax = absmax_slots(d);
   const hipStream_t st = stream_of(d);
-  const at::Tensor& ws = workspace(d, st);
-  call("affineOrDot", [&] {
+  PerStream& ps = with_workspace(d, st);
+  call_over(ps, "affineOrDot", [&](void* ws, size_t ws_bytes) {
     return L.int8_affine_f32_chained(
         fptr(x.a), static_cast<int8_t*>(aq.data_ptr()), static_cast<const int8_t*>(x.b.t->const_data_ptr()), fptr(x.bias),
         x.idx ? static_cast<const uint32_t*>(x.idx->const_data_ptr()) : nullptr, x.idx ? x.n_out : 0, fptr_mut(out), x.M, x.K,
-        x.b.cols, scale, relu, amax, want ? fptr_mut(omax) : nullptr, ws.data_ptr(), (size_t)ws.numel(), st);
+        x.b.cols, scale, relu, amax, want ? fptr_mut(omax) : nullptr, ws, ws_bytes, st);
   });
   Ref r(ok(PyTuple_New(want ? 3 : 2)));
   PyTuple_SET_ITEM(r.p, 0, wrap(std::move(out)));
@@ -421,10 +440,10 @@ PyObject* py_affine_f32_grouped(PyObject*, PyObject* const* args, Py_ssize_t nar
     N[g] = w.b[g].cols;
   }
   const hipStream_t st = stream_of(d);
-  const at::Tensor& ws = workspace(d, st);
-  call("affineOrDot", [&] {
+  PerStream& ps = with_workspace(d, st);
+  call_over(ps, "affineOrDot", [&](void* ws, size_t ws_bytes) {
     return L.int8_affine_f32_grouped(fptr(a), static_cast<int8_t*>(aq.data_ptr()), w.n, w.Bq, w.bias, out, N, M, K, scale, relu, amax,
-                                     ws.data_ptr(), (size_t)ws.numel(), st);
+                                     ws, ws_bytes, st);
   });
   Ref list(ok(PyList_New(w.n)));
   for(int g = 0; g < w.n; ++g) PyList_SET_ITEM(list.p, g, wrap(std::move(outs[g])));
@@ -504,10 +523,10 @@ PyObject* py_prepare_a(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const c10::Device d = a->device();
   at::Tensor out = quantized_buffer(a->numel(), (int)width, d);
   const hipStream_t st = stream_of(d);
-  const at::Tensor& ws = workspace(d, st);
-  call("prepareA", [&] {
+  PerStream& ps = with_workspace(d, st);
+  call_over(ps, "prepareA", [&](void* ws, size_t ws_bytes) {
     return width == 2 ? L.int16_prepare_a(fptr(a), static_cast<int16_t*>(out.data_ptr()), M, K, st)
-                      : L.int8_prepare_a(fptr(a), static_cast<int8_t*>(out.data_ptr()), M, K, ws.data_ptr(), (size_t)ws.numel(), st);
+                      : L.int8_prepare_a(fptr(a), static_cast<int8_t*>(out.data_ptr()), M, K, ws, ws_bytes, st);
   });
   Ref shape(shape_tuple(a->sizes()));
   return make_quantized(std::move(out), shape.p, width == 2 ? type16 : type8, false);
@@ -524,10 +543,10 @@ PyObject* py_prepare_b(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const c10::Device d = w->device();
   at::Tensor out = quantized_buffer(K * N, (int)width, d);
   const hipStream_t st = stream_of(d);
-  const at::Tensor& ws = workspace(d, st);
-  call("prepareB", [&] {
+  PerStream& ps = with_workspace(d, st);
+  call_over(ps, "prepareB", [&](void* ws, size_t ws_bytes) {
     return width == 2 ? L.int16_prepare_b(fptr(w), static_cast<int16_t*>(out.data_ptr()), K, N, st)
-                      : L.int8_prepare_b(fptr(w), static_cast<int8_t*>(out.data_ptr()), K, N, ws.data_ptr(), (size_t)ws.numel(), st);
+                      : L.int8_prepare_b(fptr(w), static_cast<int8_t*>(out.data_ptr()), K, N, ws, ws_bytes, st);
   });
   Ref shape(shape_tuple(w->sizes()));
   return make_quantized(std::move(out), shape.p, width == 2 ? type16 : type8, true);
@@ -776,11 +795,11 @@ PyObject* py_proj_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
       proj[g] = fptr_mut(projections[g]);
     }
   const hipStream_t st = stream_of(d);
-  const at::Tensor& ws = workspace(d, st);
-  call("ProjectedAttention", [&] {
+  PerStream& ps = with_workspace(d, st);
+  call_over(ps, "ProjectedAttention", [&](void* ws, size_t ws_bytes) {
     return L.int8_proj_attention(fptr(x), static_cast<int8_t*>(aq.data_ptr()), w.n, w.Bq, w.bias, proj, M, K, heads, fptr_mut(*k),
                                  fptr_mut(*v), k->numel() / (cap * 64), len, cap, fptr(mask), mask ? mask->numel() / len : 0, 1.0f / 8.0f,
-                                 fptr_mut(out), amax, want ? fptr_mut(omax) : nullptr, ws.data_ptr(), (size_t)ws.numel(), st);
+                                 fptr_mut(out), amax, want ? fptr_mut(omax) : nullptr, ws, ws_bytes, st);
   });
   Ref r(ok(PyTuple_New(2 + (want ? 1 : 0) + (want_proj ? 1 : 0))));
   PyTuple_SET_ITEM(r.p, 0, wrap(std::move(out)));
@@ -868,12 +887,12 @@ PyObject* py_proj_attention_ancestors(PyObject*, PyObject* const* args, Py_ssize
       proj[g] = fptr_mut(projections[g]);
     }
   const hipStream_t st = stream_of(d);
-  const at::Tensor& ws = workspace(d, st);
-  call("ProjectedAttention", [&] {
+  PerStream& ps = with_workspace(d, st);
+  call_over(ps, "ProjectedAttention", [&](void* ws, size_t ws_bytes) {
     return L.int8_proj_attention_ancestors(fptr(r.a), with_norm ? &r.n : nullptr, with_norm ? nullptr : static_cast<int8_t*>(aq.data_ptr()),
                                            w.Bq, w.bias, proj, r.M, r.K, heads, fptr_mut(*k), fptr_mut(*v), len, cap,
                                            static_cast<const uint32_t*>(anc->const_data_ptr()), 1.0f / 8.0f, fptr_mut(out), amax,
-                                           fptr_mut(omax), ws.data_ptr(), (size_t)ws.numel(), st);
+                                           fptr_mut(omax), ws, ws_bytes, st);
   });
   Ref x(with_norm ? wrap(std::move(r.x)) : (Py_INCREF(args[0]), args[0])), o(wrap(std::move(out))), m(make_absmax(std::move(omax)));
   if(!want_proj) return PyTuple_Pack(4, x.p, o.p, m.p, Py_None);
@@ -994,12 +1013,10 @@ PyObject* py_decoder_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   at::Tensor scores = empty({M, last.b.cols}, at::kFloat, dev);
   float* const out = fptr_mut(scores);
   const hipStream_t st = stream_of(dev);
-  const at::Tensor& ws = workspace(dev, st);
-  void* const wp = ws.data_ptr();
-  const size_t wn = (size_t)ws.numel();
+  PerStream& ps = with_workspace(dev, st);
   const uint32_t* const table = anc ? static_cast<const uint32_t*>(anc->const_data_ptr()) : nullptr;
   const char* where = "";
-  call("decoder step", [&] {
+  call_over(ps, "decoder step", [&](void* wp, size_t wn) {
     auto affine = [&](const float* a, const DecoderMatrix& w, float* to, int relu, const float* in_max, float* out_max) {
       return L.int8_affine_f32_chained(a, aq, w.weights(), w.shift(), nullptr, 0, to, M, w.b.rows, w.b.cols, 1.0f, relu, in_max, out_max, wp, wn, st);
     };
@@ -1216,7 +1233,7 @@ PyObject* py_logsoftmax_nbest_beams(PyObject*, PyObject* const* args, Py_ssize_t
 PyObject* py_workspace(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_TRY MH_ARGS(1, "workspace");
   const c10::Device d(c10::kCUDA, (c10::DeviceIndex)whole(args[0]));
-  return wrap(workspace(d, stream_of(d)));
+  return wrap(with_workspace(d, stream_of(d)).workspace);
   MH_END
 }
 

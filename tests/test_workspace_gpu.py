@@ -67,3 +67,37 @@ def test_quantizer_of_as_many_partials_as_there_are(orc, synth):
         big = W.copy()
         big.flat[at] = np.float32(0.75)
         assert np.array_equal(integer.prepareB(torch.from_numpy(big).cuda()).file_bytes(), orc.prepare_b(big)), at
+
+
+def test_threads_that_share_a_stream_and_its_partials():
+    """Calls of two launches, the first of which leaves partials for the second, made by threads at once."""
+    import threading
+
+    import torch
+    integer = load("integer")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+
+    def normal(*shape, scale=1.0):
+        return torch.randn(*shape, device="cuda", generator=g) * scale
+
+    def work(scale):
+        w, x = normal(1024, 8192, scale=scale), normal(64, 1024, scale=scale)
+        three = [(integer.prepareB(normal(1024, 1024, scale=0.02)), None) for _ in range(3)]
+        return lambda: [integer.prepareB(w).data[:w.numel() + 4], *integer.affine_f32_grouped(x, three)[0]]
+    work = [work(scale) for scale in (1.0, 0.25, 4.0, 0.02)]
+    want = [w() for w in work]
+    torch.cuda.synchronize()
+    bad, start = [], threading.Barrier(len(work))
+
+    def run(i):
+        start.wait()
+        for n in range(40):
+            if not all(torch.equal(a, b) for a, b in zip(work[i](), want[i])):
+                bad.append((i, n))
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(len(work))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
