@@ -14,6 +14,7 @@
 #include "gemm_stream32_kernel.h"
 #include "gemm_stream_kernel.h"
 #include "quantize_kernels.h"
+#include "stream_recorded.h"
 #ifdef MARIAN_HIP_TUNING
 // kernel families that only measurements select, and the switches that select them
 #include "../../include/marian_hip_int8_tuning.h"
@@ -949,14 +950,6 @@ bool rows_can_exchange(int M, int K, int n_out, int kw_override) {
   const long long groups = ((n_out + 31) / 32) * (long long)((M + plan.rows - 1) / plan.rows);
   const int cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
   return plan.kw == 8 && K <= rows_max_k(plan.rows) && groups <= cus && (long long)M * K <= groups * kRowsShare;
-}
-
-// Whether calls on the stream are recorded into a graph instead of being launched.
-bool recorded(hipStream_t st) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if(hipStreamIsCapturing(st, &status) == hipSuccess) return status == hipStreamCaptureStatusActive;
-  (void)hipGetLastError();   // (the launch will tell)
-  return false;
 }
 
 // The words of a workspace through which the workgroups of a one-pass launch exchange the abs-max of so many values.

@@ -34,6 +34,7 @@
 #include "../../include/marian_hip_int16.h"
 #include "../../include/marian_hip_int8.h"
 #include "../../include/marian_hip_ops.h"
+#include "stream_recorded.h"
 
 namespace {
 
@@ -181,8 +182,7 @@ constexpr size_t kScratchPieces = 4;
 class Scratch {   // (made and dropped with the interpreter lock held)
  public:
   Scratch(int64_t bytes, c10::Device d, hipStream_t st) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if(bytes <= kScratchBytes && hipStreamIsCapturing(st, &status) == hipSuccess && status == hipStreamCaptureStatusNone) {
+    if(bytes <= kScratchBytes && !marian_hip::recorded(st)) {
       home_ = &per_stream[{d.index(), st}].scratch;
       home_->reserve(kScratchPieces);
     }
