@@ -145,12 +145,12 @@ inline void call(const char* where, F f, const char** which = nullptr, std::mute
   }
 }
 
-// ---- workspaces: one per device and stream, kept for good (a graph may have recorded one) -------
+// ---- what stays with a stream: workspaces, for good (a graph may have recorded one), and scratch ---------
 struct PerStream {
   at::Tensor workspace;              // abs-max partials, one-pass exchange
   std::mutex turn;                   // held while a call makes its launches over the workspace
   std::vector<at::Tensor> nbest;     // the last one the largest
-  std::vector<at::Tensor> scratch;   // not lent at the moment
+  at::Tensor scratch;                // of the calls, not lent at the moment
 };
 std::map<std::pair<int, hipStream_t>, PerStream> per_stream;   // (looked up with the interpreter lock held)
 
@@ -172,36 +172,41 @@ inline void call_over(PerStream& p, const char* where, F f, const char** which =
   call(where, [&] { return f(ws, bytes); }, which, &p.turn);
 }
 
-// Memory of one call that nobody sees afterwards: what a stream's earlier calls gave back, which spares the call an allocation
-// (0.45 us of a small call's 4.7), or new where it is large.  Calls of one stream run one after the other, so the next may have it as soon as
-// the launches are made; a call that another thread makes meanwhile finds another piece.  At most kScratchPieces of
-// kScratchBytes stay with a stream, for good as the workspaces do.  A call that is recorded has memory of its own: its graph may be replayed
-// on another stream.
+// Memory of one call that nobody sees afterwards: what the stream's last call gave back if that is large enough, which spares the call
+// an allocation (0.45 us of a small call's 4.7), or new.  Calls of one stream run one after the other, so the next may have it as soon
+// as the launches are made; a call that another thread makes meanwhile finds none and takes new memory.  A stream keeps
+// one piece, the largest of up to kScratchBytes, kScratchStreams of them do, and release_scratch gives all back.
+// A call that is recorded has memory of its own: its graph may be replayed on another stream.
 constexpr int64_t kScratchBytes = 1 << 20;
-constexpr size_t kScratchPieces = 4;
+constexpr int kScratchStreams = 16;
+int scratch_kept = 0;
 class Scratch {   // (made and dropped with the interpreter lock held)
  public:
   Scratch(int64_t bytes, c10::Device d, hipStream_t st) {
+    int64_t size = bytes;
     if(bytes <= kScratchBytes && !marian_hip::recorded(st)) {
-      home_ = &per_stream[{d.index(), st}].scratch;
-      home_->reserve(kScratchPieces);
+      home_ = &per_stream[{d.index(), st}];
+      if(home_->scratch.defined()) {
+        t_ = std::move(home_->scratch);
+        --scratch_kept;
+      }
+      for(size = 4096; size < bytes;) size *= 2;
     }
-    if(home_ && !home_->empty()) {
-      t_ = std::move(home_->back());
-      home_->pop_back();
-    } else {
-      t_ = empty({home_ ? kScratchBytes : bytes}, at::kByte, d);
-    }
+    if(!t_.defined() || t_.numel() < bytes) t_ = empty({size}, at::kByte, d);
   }
   ~Scratch() {
-    if(home_ && home_->size() < kScratchPieces) home_->push_back(std::move(t_));
+    if(!home_) return;
+    at::Tensor& kept = home_->scratch;
+    if(kept.defined() ? kept.numel() >= t_.numel() : scratch_kept >= kScratchStreams) return;
+    scratch_kept += !kept.defined();
+    kept = std::move(t_);
   }
   Scratch(const Scratch&) = delete;
   Scratch& operator=(const Scratch&) = delete;
   void* data() const { return t_.data_ptr(); }
 
  private:
-  std::vector<at::Tensor>* home_ = nullptr;
+  PerStream* home_ = nullptr;
   at::Tensor t_;
 };
 
@@ -1237,6 +1242,15 @@ PyObject* py_workspace(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_END
 }
 
+// release_scratch(): the scratch of all streams goes back to torch's allocator
+PyObject* py_release_scratch(PyObject*, PyObject* const*, Py_ssize_t nargs) {
+  MH_TRY MH_ARGS(0, "release_scratch");
+  for(auto& p : per_stream) p.second.scratch = at::Tensor();
+  scratch_kept = 0;
+  Py_RETURN_NONE;
+  MH_END
+}
+
 // use(handle): takes the C ABI's functions from a loaded library (a dlopen handle)
 PyObject* py_use(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   MH_TRY MH_ARGS(1, "use");
@@ -1275,7 +1289,7 @@ PyObject* py_setup(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 #define MH_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&py_##name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
+    MH_METHOD(setup), MH_METHOD(use), MH_METHOD(workspace), MH_METHOD(release_scratch), MH_METHOD(affine_or_dot), MH_METHOD(affine_f32),
     MH_METHOD(affine_f32_grouped), MH_METHOD(affine_f32_normed), MH_METHOD(proj_attention_normed), MH_METHOD(proj_attention_ancestors), MH_METHOD(prepare_a), MH_METHOD(prepare_b), MH_METHOD(prepare_stored), MH_METHOD(layer_norm),
     MH_METHOD(embed), MH_METHOD(select_state), MH_METHOD(attention), MH_METHOD(attention_rows), MH_METHOD(split_heads), MH_METHOD(join_heads), MH_METHOD(proj_attention), MH_METHOD(attention_ancestors), MH_METHOD(decoder_layers),
     MH_METHOD(ancestors_advance), MH_METHOD(nbest), MH_METHOD(nbest_words), MH_METHOD(nbest_beams), MH_METHOD(logsoftmax_nbest_beams),

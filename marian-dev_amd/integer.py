@@ -159,6 +159,12 @@ class Backend:
         index = self.device.index
         return _host.workspace(torch.cuda.current_device() if index is None else index)
 
+    @staticmethod
+    def releaseScratch():
+        """Gives the memory that small calls keep between them (one piece of up to 1 MB a stream, of up to
+        16 streams) back to torch's allocator, from where torch.cuda.empty_cache() gives it to the device."""
+        _host.release_scratch()
+
     def setGemmType(self, type_):
         _abort_if(type_ not in (None, Type.intgemm8), "Unsupported type {} for Intgemm type??", type_)
         self.gemmType = type_

@@ -56,3 +56,42 @@ def test_recorded_calls_share_nothing():
             assert all(torch.equal(a, b) for a, b in zip(got, w))
             for t in got:
                 t.zero_()
+
+
+def test_scratch_is_bounded_and_given_back():
+    """A piece of the size that is asked for, a stream at a time, of a bounded number of streams, until it is asked back."""
+    import torch
+    integer = load("integer")
+    release = integer.Backend.releaseScratch
+    w = integer.prepareB(torch.randn(512, 512, device="cuda") * 0.02)
+    streams = [torch.cuda.Stream() for _ in range(24)]
+    xs = {m: torch.randn(m, 512, device="cuda") for m in (1, 300, 64)}
+
+    def grown(m, over):
+        """bytes that stay after calls of m rows"""
+        for s in over:
+            with torch.cuda.stream(s):
+                out = integer.dot(xs[m], w)
+            s.synchronize()
+            del out
+        return torch.cuda.memory_allocated() - before
+    for s in streams:   # workspaces, which are kept for good
+        with torch.cuda.stream(s):
+            integer.affine_f32(xs[1], w)
+        s.synchronize()
+    release()
+    before = torch.cuda.memory_allocated()
+    assert 0 < grown(1, streams[:1]) <= 4096
+    assert 4096 < grown(300, streams[:1]) <= 256 << 10          # a larger piece takes its place
+    assert grown(64, streams[:1]) <= 256 << 10                  # and serves smaller calls
+    assert grown(1, streams) <= (256 << 10) + 15 * 4096          # sixteen streams at the most
+    release()
+    assert torch.cuda.memory_allocated() == before
+    assert 0 < grown(1, streams[-1:]) <= 4096                   # and again
+    big = torch.randn(2300, 512, device="cuda")                  # more than a piece: never kept
+    release()
+    before = torch.cuda.memory_allocated()
+    out = integer.dot(big, w)
+    torch.cuda.synchronize()
+    del out
+    assert torch.cuda.memory_allocated() == before
