@@ -759,13 +759,14 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
     if(stream_out) return launch_big_auto<256, 256, 2, 4, 2, true>(a, st, 1);
     return launch_big_auto<256, 256, 2, 4, 2, false>(a, st, 1);
   }
-  // two or more 128x128 tiles per CU: 256x256 tiles again, on half of the CUs and more, which take in half the operands
-  // (2300 x 1024 x 4096 20.5 -> 18.3 us, 2500 x 4096 x 4096 53.8 -> 45.9, 3000 x 768 x 3072 16.8 -> 14.6); where K is 64 modulo 128, and
-  // rows are short, eight waves and two LDS stages, so that two workgroups share a CU and one multiplies while the other writes its tile
-  // out (2500 x 512 x 4096 13.1 and 13.5 us); otherwise four waves, three stages
+  // Two 128x128 tiles to a CU: eight waves and two LDS stages, so that two workgroups share a CU and one multiplies while the other writes
+  // its tile out (2048 x 1024 x 4096 14.4 us, with 128 tiles of 256x256 18.2; 1000 x 2048 x 8192 24.0 and 27.5).  A few more than
+  // two would be a second round: 256x256 tiles again, on half of the CUs and more, which take in half the operands
+  // (2050 x 1024 x 4096 20.4 -> 18.4 us, 2500 x 4096 x 4096 53.8 -> 45.9, 3000 x 768 x 3072 18.4 -> 16.2); not for short rows,
+  // where the output is most of the bytes (2500 x 512 x 4096 13.1 and 13.5 us; 700 x 640 x 16000 20.3 and 16.9), nor where K is 64 modulo 128.
   const long long tiles128 = ((a.M + 127) / 128) * (long long)((a.n_out + 127) / 128);
   if(tiles128 >= 2 * compute_units()) {
-    if(a.K > 512 && a.K % 128 == 0) {
+    if(tiles128 > 2 * compute_units() && a.K > 512 && a.K % 128 == 0) {
       if(stream_out) return launch_big_auto<256, 256, 2, 4, 2, true>(a, st, 1);
       return launch_big_auto<256, 256, 2, 4, 2, false>(a, st, 1);
     }
