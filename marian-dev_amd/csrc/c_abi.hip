@@ -518,9 +518,17 @@ int launch_stream32_kw(const GemmArgs& a, const FusedSrc& f, hipStream_t st, int
   }
 }
 
-// The K split and the tile height of the tiled fused form for a call.  K split: the widest (most
-// loads in flight per weight row) that stays within one workgroup per CU, the narrowest if none
-// does.  Every workgroup quantizes the activation rows it multiplies: as few rows as keep the workgroups one to a CU
+// The waves that share a row of weights: the widest K split (most loads in flight per weight row) that stays within one workgroup per
+// CU, the narrowest if none does; at most a sub-step of 32 values to a wave.
+int stream32_k_split(int tiles, int m_tiles, int K, int kw_override = 0) {
+  int kw = 8;
+  while(kw > 1 && (long long)((tiles * kw + 7) / 8) * m_tiles > compute_units()) kw >>= 1;
+  if(kw_override) kw = kw_override;
+  while(kw > 1 && K / 32 < kw) kw >>= 1;
+  return kw;
+}
+
+// The K split and the tile height of the tiled fused form for a call.  Every workgroup quantizes the activation rows it multiplies: as few rows as keep the workgroups one to a CU
 // (8 rows against 16: 64 x 1024 x 1024 3.9 and 4.2 us, 128 x 512 x 512 3.6 and 3.7; 16 against 32: 65 x 512 x 1536 3.7 and 4.1;
 // with a second workgroup on some CUs 128 x 1024 x 1024 8.6 and 4.4, 65 x 512 x 2048 8.2 and 4.1).
 struct TiledPlan {
@@ -529,10 +537,7 @@ struct TiledPlan {
 };
 TiledPlan plan_tiled(int M, int K, int n_out, int kw_override) {
   const int tiles = (n_out + 31) / 32, m_tiles = (M + 31) / 32;
-  int kw = 8;
-  while(kw > 1 && (long long)((tiles * kw + 7) / 8) * m_tiles > compute_units()) kw >>= 1;
-  if(kw_override) kw = kw_override;
-  while(kw > 1 && K / 32 < kw) kw >>= 1;
+  const int kw = stream32_k_split(tiles, m_tiles, K, kw_override);
   if(kw < 8) return TiledPlan{kw, 32};
   const int ov = kernel_override() % 1000;   // 640 / 641 / 642: force 32 / 16 / 8 rows
   if(ov >= 640 && ov <= 642) return TiledPlan{kw, 32 >> (ov - 640)};
@@ -557,12 +562,7 @@ int launch_stream32_auto(const GemmArgs& a, const FusedSrc& f, hipStream_t st, i
   }
   if(MODE == kFusedTiled) mt = 1;
   const int m_tiles = MODE == kFusedAll ? 1 : (a.M + mt * 32 - 1) / (mt * 32);
-  // the widest K split (most loads in flight per weight row) that stays within one workgroup
-  // per CU; the narrowest if none does
-  int kw = 8;
-  while(kw > 1 && (long long)((tiles * kw + 7) / 8) * m_tiles > compute_units()) kw >>= 1;
-  if(kw_override) kw = kw_override;
-  while(kw > 1 && a.K / 32 < kw) kw >>= 1;
+  const int kw = stream32_k_split(tiles, m_tiles, a.K, kw_override);
   if constexpr(MODE == kFusedTiled) {
     const TiledPlan plan = plan_tiled(a.M, a.K, a.n_out, kw_override);
     return launch_stream32_kw<1, MODE>(a, f, st, plan.kw, plan.rows);
@@ -620,8 +620,7 @@ int launch_stream_auto(const GemmArgs& a, hipStream_t st, int force_wide) {
 
 // Small tiles where larger ones would leave CUs idle.  A CU takes in (rows + columns) x K bytes of its tile, so a long K asks
 // for the smallest tiles that still find a CU each (300 x 4096 x 1024: 128x64 tiles 10.6 us, 64x64 8.3, 32x64 7.6; 1000 x 4096 x 1024
-// 11.1, 9.1, 10.7 - two of the last to a CU; 1300 x 2048 x 512 6.9, 5.9, 6.5; 1000 x 512 x 512 4.7, 4.0, 3.7; against
-// gemm_stream32_kernel 256 x 3072 x 768 8.4 and 6.4, 200 x 4096 x 4096 10.8 and 8.9, but 256 x 1024 x 1024 3.94 and 3.95).
+// 11.1, 9.1, 10.7 - two of the last to a CU; 1300 x 2048 x 512 6.9, 5.9, 6.5; 1000 x 512 x 512 4.7, 4.0, 3.7).
 // t64x64_shared: short rows, several tiles to a CU, one of which is loaded while another is multiplied or written out
 // (1000 x 512 x 2048 5.2 -> 4.8 us, 1500 x 512 x 2048 6.5 -> 5.4, 1000 x 768 x 3072 7.1 -> 6.5, but 2050 x 512 x 2048 7.9 -> 8.3,
 // 1200 x 768 x 3072 7.0 -> 7.4, 2050 x 1024 x 1024 6.6 -> 7.4).  (Measurement id 340: none of them.)
@@ -633,6 +632,20 @@ SmallTiles small_tiles(const GemmArgs& a, long long columns) {   // columns: of 
   if(t64 <= cus) return SmallTiles::t64x64;
   if(a.K < 1024 && t64 <= (a.K <= 512 ? 4 : 3) * cus) return SmallTiles::t64x64_shared;
   return SmallTiles::none;
+}
+
+// Whether gemm_stream32_kernel, of up to 512 rows, is ahead of small tiles that find a CU each.  A wave's share of K is what decides: it holds 2, 4 or
+// 8 sub-steps of 32 values at a time and reads twos and fours well, eight only when they are full; a share of several eights pays where
+// eight waves split K.  Stream form and tiles, weights from the memory-side cache: 65 x 384 x 512 3.0 and 3.5 us, 129 x 512 x 1536 3.2 and 3.8, 200 x 1024 x
+// 1024 3.8 and 4.3, 100 x 2048 x 1536 5.2 and 6.4, 300 x 512 x 1024 3.2 and 3.8; but 100 x 1280 x 1032 (five to a wave) 5.3 and 4.7, 128 x 3072 x 512 (two
+// rounds) 9.0 and 6.8, 160 x 768 x 3072 (six) 4.9 and 4.3.  64x64 tiles: 200 x 512 x 3000 (full) 4.0 and 4.4, 200 x 384 x 3072 4.1 and 3.8,
+// 128 x 512 x 8192, whose stream form takes 128 rows to a workgroup, 5.9 and 4.5.
+bool stream32_ahead(const GemmArgs& a, SmallTiles small) {
+  const int tiles32 = (a.n_out + 31) / 32;
+  if(tiles32 >= 256) return false;   // (launch_stream32_auto)
+  const int kw = stream32_k_split(tiles32, (a.M + 31) / 32, a.K), share = (a.K / 32 + kw - 1) / kw;
+  if(small == SmallTiles::t64x64) return share == 8;
+  return share <= 4 || (share % 8 == 0 && share <= 2 * kw);
 }
 
 // Whether an output is written with non-temporal stores, which leave nothing dirty in the L2 caches for the end of the launch: up
@@ -712,11 +725,8 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
   const int tiles32 = (a.n_out + 31) / 32;
   if(a.M <= 8 || (a.M <= 16 && tiles32 < 512)) return launch_stream_auto(a, st, 2);
   //    (few columns, M up to 512; beyond 256 rows with K >= 2048 and 1024 or more columns larger tiles
-  //    are 20 % faster), but for what small tiles do better: more than 64 rows - 128 x 768 x 3072 4.6 and 3.9 us, 200 x 768 x 2048 4.6 and
-  //    4.2, 128 x 1280 x 4096 7.1 and 5.3, 256 x 1792 x 3072 10.0 and 6.8, weights from memory -, except where the
-  //    stream form's K split comes out even (129 x 512 x 1024 3.2 and 3.7, 70 x 1024 x 4096 4.3 and 4.6; but 160 x 1024 x 2048 4.3 and 4.2)
+  //    are 20 % faster), but for what small tiles do better (stream32_ahead)
   const SmallTiles small = small_tiles(a, (a.n_out + 63) / 64);
-  const bool even = small == SmallTiles::t32x64 && ((a.K == 512 && a.M <= 256) || (a.K == 1024 && a.M <= 128));
   const bool tiles_fit = small == SmallTiles::t32x64 || small == SmallTiles::t64x64;
   // Wide outputs of 65 .. 128 rows (scores over a vocabulary), of which the tiles above do not get a CU each: tiles as high as the rows,
   // 128x64 in the split form up to half a 128x128 tile a CU and for long rows, else 128x128, two workgroups to a CU.  Weights from memory
@@ -731,7 +741,7 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
     return launch_big<128, 128, 2, 4, 2, true, true>(a, st);
   }
   if((a.M <= 128 || (a.M <= 512 && tiles32 < 128 && (a.M <= 256 || a.K < 2048 || tiles32 < 32))) &&
-     (small == SmallTiles::none || a.idx || a.M <= 64 || even))
+     (small == SmallTiles::none || a.idx || a.M <= 64 || (tiles_fit && stream32_ahead(a, small))))
     return launch_stream32_auto<kPrequant>(a, FusedSrc(), st, 0);
   switch(small) {
     case SmallTiles::t32x64: return launch_big_split<32, 64, 1, 2, 4, true>(a, st);

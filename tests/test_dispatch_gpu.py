@@ -31,3 +31,31 @@ def workgroups(M, K, N):
 ])
 def test_two_tiles_to_a_cu(M, K, N, tiles):
     assert workgroups(M, K, N) == tiles
+
+
+# rows, K, columns, and the rows and columns of a tile (None: the stream form, whose waves leave a value each, eight to a workgroup)
+@pytest.mark.parametrize("M,K,N,tile", [
+    (65, 384, 512, None),       # eight waves, two sub-steps each
+    (200, 1024, 1024, None),    # four
+    (129, 2048, 1536, None),    # eight
+    (300, 512, 1024, None),     # four waves, four
+    (100, 4096, 768, None),     # eight waves, two rounds of eight
+    (65, 256, 3000, None),      # four waves, two
+    (200, 512, 3000, None),     # two waves, eight
+    (100, 1280, 1032, (32, 64)),    # eight waves, five
+    (128, 3072, 512, (32, 64)),     # twelve
+    (129, 1536, 1032, (32, 64)),    # six
+    (160, 768, 3072, (32, 64)),     # four waves, six
+    (160, 2048, 2048, (32, 64)),    # two rounds of eight
+    (200, 384, 3072, (64, 64)),     # two waves, six
+    (128, 512, 8192, (64, 64)),     # 128 rows to a workgroup in the stream form
+])
+def test_stream_form_or_small_tiles(M, K, N, tile):
+    lib = load("_lib")
+    with lib.forced_kernel(600):   # (quantized first: affine_f32 of so few rows may quantize on the way instead)
+        found = workgroups(M, K, N)
+    tiles = lambda rows, columns: -(-M // rows) * -(-N // columns)
+    if tile:
+        assert found == tiles(*tile)
+    else:
+        assert found > 2 * tiles(32, 64)

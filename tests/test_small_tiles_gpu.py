@@ -10,8 +10,10 @@ pytestmark = pytest.mark.gpu
 
 # (workgroups of 32x64 and of 64x64 tiles on a chip of 256 CUs: the form)
 SHAPES = [
-    (257, 128, 8),        # 9: 32x64, one K block
-    (288, 1024, 1024),    # 144: 32x64, whole tiles
+    (257, 128, 8),        # the stream form: one sub-step to a wave
+    (520, 128, 8),        # 17: 32x64, one K block
+    (288, 1024, 1024),    # the stream form: eight sub-steps to a wave
+    (288, 1280, 1024),    # 144: 32x64, whole tiles
     (511, 2048, 1024),    # 256: 32x64, the last size, a row short
     (513, 2048, 1024),    # 272, 144: 64x64, a row more
     (1024, 384, 1024),    # 64x64, whole tiles, the last size, fewer blocks than stages
@@ -20,7 +22,7 @@ SHAPES = [
     (700, 768, 2056),     # 363: K = 768
     (65, 2048, 520),      # few rows, long ones: 32x64
     (200, 4096, 4104),    # 260: no small tiles
-    (129, 2048, 3000),    # 32x64 tiles over 235 of 64x64
+    (129, 2048, 3000),    # 32x64, 235
     (300, 576, 512),      # K no whole number of blocks: no small tiles
 ]
 

@@ -9,14 +9,17 @@ pytestmark = pytest.mark.gpu
 # (on a chip of 256 CUs)
 SHAPES = [
     (64, 768, 2048),      # the stream form
-    (65, 512, 2048),      # the stream form: an even split
+    (65, 512, 2048),      # the stream form: two sub-steps to a wave
     (65, 512, 8200),      # 128x64, three stages
     (128, 1024, 4096),    # the stream form, its last width
     (128, 1024, 4104),    # 64x64
-    (129, 1024, 1032),    # 32x64
+    (129, 1024, 1032),    # the stream form: four sub-steps to a wave
+    (129, 1280, 1032),    # 32x64: five
     (256, 512, 2048),     # the stream form
-    (257, 512, 2048),     # 64x64, several to a CU
-    (65, 768, 776),       # 32x64
+    (257, 512, 2048),     # the stream form: two waves, eight sub-steps each
+    (257, 384, 2048),     # 64x64: six
+    (65, 768, 776),       # the stream form: three sub-steps to a wave
+    (65, 1536, 776),      # 32x64: six
     (128, 640, 16384),    # 128x64, its last width
     (128, 640, 16392),    # 128x128
     (100, 1024, 32776),   # 128x128, ragged rows short of 14 MB
