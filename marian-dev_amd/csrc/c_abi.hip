@@ -622,15 +622,25 @@ int launch_stream_auto(const GemmArgs& a, hipStream_t st, int force_wide) {
 // for the smallest tiles that still find a CU each (300 x 4096 x 1024: 128x64 tiles 10.6 us, 64x64 8.3, 32x64 7.6; 1000 x 4096 x 1024
 // 11.1, 9.1, 10.7 - two of the last to a CU; 1300 x 2048 x 512 6.9, 5.9, 6.5; 1000 x 512 x 512 4.7, 4.0, 3.7).
 // t64x64_shared: short rows, several tiles to a CU, one of which is loaded while another is multiplied or written out
-// (1000 x 512 x 2048 5.2 -> 4.8 us, 1500 x 512 x 2048 6.5 -> 5.4, 1000 x 768 x 3072 7.1 -> 6.5, but 2050 x 512 x 2048 7.9 -> 8.3,
-// 1200 x 768 x 3072 7.0 -> 7.4, 2050 x 1024 x 1024 6.6 -> 7.4).  (Measurement id 340: none of them.)
-enum class SmallTiles { none, t32x64, t64x64, t64x64_shared };
+// (1000 x 512 x 2048 5.2 -> 4.8 us, 1500 x 512 x 2048 6.5 -> 5.4, but 2050 x 512 x 2048 7.9 -> 8.3, 1200 x 768 x 3072 7.0 -> 7.4,
+// 2050 x 1024 x 1024 6.6 -> 7.4).  They hold two blocks ahead: from K = 640 on 128x64 tiles with four are ahead wherever a CU gets one
+// (512 x 768 x 4096 5.9 us, shared 6.9; 300 x 768 x 4096 5.7 and 6.6, 2048 x 768 x 768 5.1 and 5.6, but 1500 x 768 x 1536, where some would get two,
+// 7.1 and 6.4), and where the weights are most of what comes in at K = 512 too (160 x 512 x 8192 5.2 and 5.7, but 1500 x 512 x 1024 5.4 and
+// 4.9).  Such wide outputs take four to a CU only where 128x128 tiles do not find a CU each (512 x 512 x 8192 7.4 and 8.4 us, 300 x 384 x 12000 7.5
+// and 6.7), with K over 512 nine quarters (250 x 640 x 10240, ten, 8.0 and 8.9; 340 x 640 x 6144, nine, 7.5 and 6.6).
+// (Measurement id 340: none of them.)
+enum class SmallTiles { none, t32x64, t64x64, t64x64_shared, t128x64 };
 SmallTiles small_tiles(const GemmArgs& a, long long columns) {   // columns: of 64, each a tile column
   if(a.K % 128 != 0 || a.dump || kernel_override() % 1000 == 340) return SmallTiles::none;
   const long long cus = compute_units(), t64 = columns * ((a.M + 63) / 64);
   if(columns * ((a.M + 31) / 32) <= cus) return SmallTiles::t32x64;
   if(t64 <= cus) return SmallTiles::t64x64;
-  if(a.K < 1024 && t64 <= (a.K <= 512 ? 4 : 3) * cus) return SmallTiles::t64x64_shared;
+  if(a.K >= 1024) return SmallTiles::none;
+  const bool wide = columns * 64 >= 16ll * a.M;
+  if((a.K > 512 || (a.K > 384 && wide)) && columns * ((a.M + 127) / 128) <= cus) return SmallTiles::t128x64;
+  const bool four = !wide || a.K <= 256 || ((a.M + 127) / 128) * ((columns + 1) / 2) > cus;
+  const long long quarters = a.K > 512 ? (wide ? 9 : 12) : (four ? 16 : 12);   // of a tile to a CU
+  if(4 * t64 <= quarters * cus) return SmallTiles::t64x64_shared;
   return SmallTiles::none;
 }
 
@@ -747,6 +757,7 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
     case SmallTiles::t32x64: return launch_big_split<32, 64, 1, 2, 4, true>(a, st);
     case SmallTiles::t64x64: return launch_big_split<64, 64, 2, 2, 4, true>(a, st);
     case SmallTiles::t64x64_shared: return launch_big<64, 64, 2, 2, 2, true, true>(a, st);
+    case SmallTiles::t128x64: return launch_big_split<128, 64, 2, 2, 4, true>(a, st);
     case SmallTiles::none: break;
   }
   // large outputs: 256x256 tiles (one per CU keeps operand traffic lowest); otherwise 128x128
@@ -899,6 +910,7 @@ int launch_big_grouped(const GemmArgs& a, int64_t n_groups, const int8_t* const*
       return launch_grouped_as<Cfg, Cfg::kThreads, gemm_mfma32_group_kernel<64, 64, 2, 2, 2, true, false>>(
           a, group_table(n_groups, Bq, bias, out, N, 64), (a.M + 63) / 64, st);
     }
+    case SmallTiles::t128x64:   // (below)
     case SmallTiles::none: break;
   }
   if(tiles128 >= compute_units()) {

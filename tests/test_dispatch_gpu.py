@@ -59,3 +59,21 @@ def test_stream_form_or_small_tiles(M, K, N, tile):
         assert found == tiles(*tile)
     else:
         assert found > 2 * tiles(32, 64)
+
+
+@pytest.mark.parametrize("M,K,N,tile", [
+    (512, 768, 4096, (128, 64)),    # one to a CU
+    (2048, 768, 768, (128, 64)),
+    (600, 640, 3072, (128, 64)),
+    (1500, 768, 1536, (64, 64)),    # 128x64 would be 288
+    (1500, 512, 1024, (64, 64)),    # shorter rows
+    (160, 512, 8192, (128, 64)),    # mostly weights
+    (192, 384, 8192, (64, 64)),
+    (512, 512, 8192, (128, 128)),   # four of 64x64 to a CU
+    (300, 384, 12000, (64, 64)),    # 128x128 would be 282
+    (1000, 512, 4096, (64, 64)),    # fewer of them weights
+    (340, 640, 6144, (64, 64)),     # longer rows, nine to four CUs
+])
+def test_small_tiles_several_to_a_cu_or_taller_ones(M, K, N, tile):
+    with load("_lib").forced_kernel(600):
+        assert workgroups(M, K, N) == -(-M // tile[0]) * -(-N // tile[1])
