@@ -865,7 +865,9 @@ GroupTable group_table(int64_t n_groups, const int8_t* const* Bq, const float* c
 //    while the next is multiplied (4096 x 1024 x 3072 19.6 us, the next form 22.6, three launches 26.7 - 32);
 //  - a 128x128 tile or more per CU: the eight-wave form, two workgroups to a CU (3000 x 512 x 1536 8.9 us,
 //    1400 x 1024 x 3072 11.6; three launches 14.8 and 16.9);
-//  - small tiles as for a single matrix (small_tiles);
+//  - small tiles as for a single matrix (small_tiles), several to a CU fewer than three each and, from K = 384 on, only where 128x64 tiles do not
+//    find a CU each (with the quantization in front 300 x 768 x 6144 10.2 -> 9.1 us, 1500 x 512 x 1536 9.8 -> 9.2, 600 x 768 x 4608 10.7 -> 10.1; but
+//    1024 x 512 x 3000, three each, 10.2 and 11.2, 768 x 768 x 2304, where 128x64 tiles fit, 8.8 and 9.5);
 //  - fewer: 128x64 tiles in the split form, which CUs that idle leave room for (1000 x 512 x 1536 5.1 us,
 //    600 x 1024 x 3072 6.0; three launches 13.9 and 16.3).
 template <typename CFG, int THREADS, auto KERNEL>
@@ -894,7 +896,11 @@ int launch_big_grouped(const GemmArgs& a, int64_t n_groups, const int8_t* const*
   if(pairs && (a.M / 256) * (columns / 256) >= 192)
     return launch_grouped_as<PairCfg, PairCfg::kThreads, gemm_pair_group_kernel<true>>(
         a, group_table(n_groups, Bq, bias, out, N, 2 * PairCfg::BN), a.M / PairCfg::BM, st);
-  switch(small_tiles(a, columns64)) {
+  SmallTiles small = small_tiles(a, columns64);
+  if(small == SmallTiles::t64x64_shared && ((a.K > 256 && columns64 * ((a.M + 127) / 128) <= compute_units()) ||
+                                            columns64 * ((a.M + 63) / 64) >= 3 * compute_units()))
+    small = SmallTiles::none;
+  switch(small) {
     case SmallTiles::t32x64: {
       using Cfg = BigCfg<32, 64, 1, 2, 4>;
       return launch_grouped_as<Cfg, 2 * Cfg::kThreads, gemm_mfma32_group_kernel<32, 64, 1, 2, 4, true, true>>(

@@ -1,5 +1,7 @@
 """Which form a multiplication takes (csrc/c_abi.hip, launch_gemm), where a rule's line lies: told by the number of workgroups that leave an
 abs-max, on a chip of 256 CUs.  The sizes beside each were measured on both sides of the line."""
+import ctypes
+
 import pytest
 
 from conftest import load
@@ -77,3 +79,49 @@ def test_stream_form_or_small_tiles(M, K, N, tile):
 def test_small_tiles_several_to_a_cu_or_taller_ones(M, K, N, tile):
     with load("_lib").forced_kernel(600):
         assert workgroups(M, K, N) == -(-M // tile[0]) * -(-N // tile[1])
+
+
+class KernelNode(ctypes.Structure):
+    """hipKernelNodeParams"""
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
+                ("params", ctypes.c_void_p), ("lds", ctypes.c_uint)]
+
+
+def launches(call):
+    """the workgroups of the launches that a call makes, recorded"""
+    import torch
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64.so" in line))
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    raw, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    found = []
+    for node in nodes:
+        p = KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        found.append(p.grid[0] * p.grid[1] * p.grid[2])
+    return found
+
+
+@pytest.mark.parametrize("M,K,Ns,tile", [
+    (300, 768, (2048, 2048, 2048), (64, 64)),   # 128x64 would be 288; 480 of these
+    (1500, 512, (512, 512, 512), (64, 64)),     # 576
+    (600, 768, (1536, 1536, 1536), (64, 64)),   # 720
+    (1024, 512, (1000, 1000, 1000), (128, 64)),  # 768: three to a CU
+    (768, 768, (768, 768, 768), (128, 64)),     # 216 of 128x64
+    (768, 256, (768, 768, 768), (64, 64)),      # short rows
+    (600, 512, (512, 512), (64, 64)),           # one to a CU
+])
+def test_matrices_side_by_side(M, K, Ns, tile):
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the numbers are those of 256 CUs")
+    integer = load("integer")
+    x = torch.randn(M, K, device="cuda")
+    weights = [(integer.prepareB(torch.randn(K, n, device="cuda") * 0.02), None) for n in Ns]
+    assert launches(lambda: integer.affine_f32_grouped(x, weights))[-1] == -(-M // tile[0]) * sum(-(-n // tile[1]) for n in Ns)
