@@ -814,10 +814,9 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
   // A few rows or columns more than one 128x128 tile per CU: whole tiles plus small ones, by the
   // eight-wave form, two of whose workgroups share a CU - the small tiles then run beside the whole
   // ones from the start (measured: 2050 x 1024 x 2056 11.7 instead of 15.4 us with the four-wave form,
-  // whose 96 KB of LDS leave no room for a second workgroup, and 17.3 us with 289 tiles alike).  Not for two whole
-  // rows of tiles, where the small ones are many columns (weights from memory: 256 x 512 x 20000 12.7 us, with 128x128 tiles alone 11.0,
-  // 256 x 1024 x 32000 18.4 and 17.1; but 220 x 1024 x 20000 13.3 and 14.9).
-  if(a.M != 256 || kernel_override() % 1000 == 340) {
+  // whose 96 KB of LDS leave no room for a second workgroup, and 17.3 us with 289 tiles alike; weights from memory, 256 x 1024 x 16448
+  // 11.0 us and with 128x128 tiles two to a CU 11.6, 220 x 1024 x 20000 13.3 and 14.9).
+  {
     const Ragged r = plan_ragged(a, 128, 128, 64, 128, 128, 64, 1);
     if(r.use) {
       const bool amax = big_leaves_absmax(a, r.workgroups);
@@ -828,7 +827,8 @@ int launch_gemm(const GemmArgs& a, hipStream_t st) {
     }
   }
   // More than one tile to a CU, fewer than two: the eight-wave form again, two workgroups to a CU, instead of two rounds of the
-  // four-wave form (1500 x 1024 x 4096 15.9 -> 10.9 us, 3000 x 2048 x 2048 23.7 -> 17.4, 2500 x 4096 x 2048 35.9 -> 27.8).
+  // four-wave form (1500 x 1024 x 4096 15.9 -> 10.9 us, 3000 x 2048 x 2048 23.7 -> 17.4, 2500 x 4096 x 2048 35.9 -> 27.8; weights from memory,
+  // 256 x 1024 x 32000 18.4 -> 17.1, 256 x 512 x 20000 12.7 -> 11.0).
   if(tiles128 > compute_units() && kernel_override() % 1000 != 340) {
     if(stream_out) return launch_big<128, 128, 2, 4, 2, true, true>(a, st);
     return launch_big<128, 128, 2, 4, 2>(a, st);

@@ -81,6 +81,17 @@ def test_small_tiles_several_to_a_cu_or_taller_ones(M, K, N, tile):
         assert workgroups(M, K, N) == -(-M // tile[0]) * -(-N // tile[1])
 
 
+@pytest.mark.parametrize("M,K,N,tiles", [
+    (256, 1024, 16448, 256 + 2),        # two rows of 128 whole 128x128 tiles, and one of 128x64 each for the last columns
+    (256, 512, 16504, 256 + 4),
+    (384, 1024, 10928, 255 + 3),
+    (256, 1024, 20000, 2 * 157),        # two rounds either way: 128x128 alone
+])
+def test_a_little_more_than_a_tile_to_a_cu(M, K, N, tiles):
+    with load("_lib").forced_kernel(600):
+        assert workgroups(M, K, N) == tiles
+
+
 class KernelNode(ctypes.Structure):
     """hipKernelNodeParams"""
     _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),

@@ -28,7 +28,8 @@ SHAPES = [
     (77, 1152, 16392),    # 128x64, three stages, two to a CU
     (80, 1152, 32776),    # 128x128, more than one to a CU
     (129, 1024, 8200),    # the forms of more rows
-    (256, 1024, 16392),   # 128x128 alone, no small tiles beside them
+    (256, 1024, 16392),   # 128x128, and 128x64 for the last columns
+    (256, 1024, 20000),   # 128x128 alone
     (200, 1152, 8200),    # long rows
     (130, 576, 8200),     # K no whole number of blocks
 ]
