@@ -659,10 +659,12 @@ bool stream32_ahead(const GemmArgs& a, SmallTiles small) {
 }
 
 // Whether an output is written with non-temporal stores, which leave nothing dirty in the L2 caches for the end of the launch: up
-// to 56 MB (2050 x 1024 x 4096 19.7 -> 18.1 us, 3000 x 1024 x 4096 22.9 -> 21.6, but 4096 x 1024 x 4096 26.3 and 27.2), and where rows
-// begin between lines, which such stores then write in parts, up to 14 MB (1500 x 1024 x 2056 9.34 and 9.30 us, 1500 x 1024 x 3000 10.9 and
-// 11.5, 2200 x 1024 x 3000 12.5 and 15.2).
-bool streams_out(long long M, long long n_out) { return M * n_out * 4 <= (n_out % 32 == 0 ? 56ll << 20 : 14ll << 20); }
+// to 32 MB, what those hold.  Beyond, the launch that reads the output pays what such stores gain (2050 x 1024 x 4096 with prepareA behind it
+// 33.2 us, with plain stores 32.9, 2300 x 1024 x 4096 35.6 and 34.8, 2500 x 512 x 4096 39.9 and 38.8; the first alone 24.0 and 24.7), and where
+// what other launches wrote fills the memory-side cache it waits for the writes (prepareA of that output behind 1 GB of them 17.0 and
+// 9.9 us).  Where rows begin between lines, which such stores then write in parts, up to 14 MB (1500 x 1024 x 2056 9.34 and 9.30 us,
+// 1500 x 1024 x 3000 10.9 and 11.5, 2200 x 1024 x 3000 12.5 and 15.2).
+bool streams_out(long long M, long long n_out) { return M * n_out * 4 <= (n_out % 32 == 0 ? 32ll << 20 : 14ll << 20); }
 
 int launch_gemm(const GemmArgs& a, hipStream_t st) {
 #ifdef MARIAN_HIP_TUNING

@@ -98,8 +98,8 @@ class KernelNode(ctypes.Structure):
                 ("params", ctypes.c_void_p), ("lds", ctypes.c_uint)]
 
 
-def launches(call):
-    """the workgroups of the launches that a call makes, recorded"""
+def launches(call, kernels=False):
+    """the workgroups of the launches that a call makes, recorded, or their kernels"""
     import torch
     hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64.so" in line))
     call()
@@ -115,7 +115,7 @@ def launches(call):
     for node in nodes:
         p = KernelNode()
         assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
-        found.append(p.grid[0] * p.grid[1] * p.grid[2])
+        found.append(p.func if kernels else p.grid[0] * p.grid[1] * p.grid[2])
     return found
 
 
@@ -136,3 +136,21 @@ def test_matrices_side_by_side(M, K, Ns, tile):
     x = torch.randn(M, K, device="cuda")
     weights = [(integer.prepareB(torch.randn(K, n, device="cuda") * 0.02), None) for n in Ns]
     assert launches(lambda: integer.affine_f32_grouped(x, weights))[-1] == -(-M // tile[0]) * sum(-(-n // tile[1]) for n in Ns)
+
+
+@pytest.mark.parametrize("M,N,streamed", [
+    (2100, 3968, True),    # 31.8 MB
+    (2050, 4096, False),   # 32.03 MB: what reads the output would pay for the stores
+    (2500, 4096, False),
+])
+def test_stores_of_large_outputs(M, N, streamed):
+    """256x256 tiles with edges, and the same kernel as an output of 64 MB, or another"""
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the form is that of 256 CUs")
+    integer = load("integer")
+
+    def kernel(m, k, n):
+        Aq, w = integer.prepareA(torch.randn(m, k, device="cuda")), integer.prepareB(torch.randn(k, n, device="cuda") * 0.02)
+        return launches(lambda: integer.multiply(Aq, w), kernels=True)[-1]
+    assert (kernel(M, 2048, N) != kernel(4090, 2048, 4096)) == streamed
