@@ -973,14 +973,17 @@ unsigned next_nonce() {
 
 // Whether the workgroups of gemm_rows_kernel take the abs-max of the activations themselves: one to a CU, and a share of the
 // activations that a thread holds in a few registers.  Launched one by one, with a launch in front and so: 64 x 1024 x 1024 7.4 and 5.3 us,
-// 256 x 1024 x 1000 7.4 and 6.5, 128 x 4096 x 1024 10.3 and 9.4, 40 x 3072 x 768 7.8 and 6.9, 64 x 4096 x 512 8.8 and 8.1.
+// 256 x 1024 x 1000 7.4 and 6.5, 40 x 3072 x 768 7.8 and 6.9, 64 x 4096 x 512 8.8 and 8.1.  Long rows only with a workgroup to two CUs: the exchange gains
+// little there (128 x 4096 x 1024 10.3 and 9.4), and workgroups that fill their CU's LDS and wait for each other keep a second stream's
+// launch out (two streams, us a call of both: 128 x 4096 x 1024 13.2 and 20.5, 100 x 4096 x 1024 12.8 and 20.9, but 64 x 4096 x 512, 128 workgroups, 8.8
+// and 7.4, 256 x 1024 x 1000 14.4 and 12.7; on a stream that has half of the CUs 100 x 4096 x 1024 14.5 and 72).
 // Calls that are being recorded have the launch in front, which costs the host nothing there.  (Measurement ids: 630 the launch in
 // front; 702 no patience.)
 bool rows_can_exchange(int M, int K, int n_out, int kw_override) {
   const TiledPlan plan = plan_tiled(M, K, n_out, kw_override);
   const long long groups = ((n_out + 31) / 32) * (long long)((M + plan.rows - 1) / plan.rows);
   const int cus = compute_units() < kOnePassMaxGroups ? compute_units() : kOnePassMaxGroups;
-  return plan.kw == 8 && K <= rows_max_k(plan.rows) && groups <= cus && (long long)M * K <= groups * kRowsShare;
+  return plan.kw == 8 && K <= rows_max_k(plan.rows) && groups <= (K > 2048 ? cus / 2 : cus) && (long long)M * K <= groups * kRowsShare;
 }
 
 // The words of a workspace through which the workgroups of a one-pass launch exchange the abs-max of so many values.
