@@ -974,8 +974,8 @@ unsigned next_nonce() {
 // Whether the workgroups of gemm_rows_kernel take the abs-max of the activations themselves: one to a CU, and a share of the
 // activations that a thread holds in a few registers.  Launched one by one, with a launch in front and so: 64 x 1024 x 1024 7.4 and 5.3 us,
 // 256 x 1024 x 1000 7.4 and 6.5, 40 x 3072 x 768 7.8 and 6.9, 64 x 4096 x 512 8.8 and 8.1.  Long rows only with a workgroup to two CUs: the exchange gains
-// little there (128 x 4096 x 1024 10.3 and 9.4), and workgroups that fill their CU's LDS and wait for each other keep a second stream's
-// launch out (two streams, us a call of both: 128 x 4096 x 1024 13.2 and 20.5, 100 x 4096 x 1024 12.8 and 20.9, but 64 x 4096 x 512, 128 workgroups, 8.8
+// little there (128 x 4096 x 1024 10.3 and 9.4), and workgroups that wait for each other and leave their CU no registers for another (16 rows:
+// 165 a lane and more) keep a second stream's launch out (two streams, us a call of both: 128 x 4096 x 1024 13.2 and 20.5, 100 x 4096 x 1024 12.8 and 20.9, but 64 x 4096 x 512, 128 workgroups, 8.8
 // and 7.4, 256 x 1024 x 1000 14.4 and 12.7; on a stream that has half of the CUs 100 x 4096 x 1024 14.5 and 72).
 // Calls that are being recorded have the launch in front, which costs the host nothing there.  (Measurement ids: 630 the launch in
 // front; 702 no patience.)

@@ -12,7 +12,7 @@ PROGRAM = r"""
 #include "onepass_patience.h"
 using namespace marian_hip;
 int main() {
-  // a workgroup that waits twice (the first of a group: for its group, then for the others) has one budget for both
+  // one budget for a workgroup's waits, however many there are
   for(int budget : {0, 1, 5, 64})
     for(int first : {0, 1, 3, 64, 100}) {   // the poll that finds the first words; 0: none does
       int left = budget, polls = 0;
@@ -32,7 +32,7 @@ int main() {
 
 def test_waits_are_bounded(tmp_path):
     """One budget for all waits of a workgroup, and a budget of the order of what the wait spares: ten times the usual wait of
-    2 us at the least, tens of microseconds more than it takes 256 workgroups to read the whole input each at the most."""
+    1.2 us and more at the least, tens of microseconds more than it takes 256 workgroups to read the whole input each at the most."""
     (tmp_path / "p.cpp").write_text(PROGRAM)
     exe = str(tmp_path / "p")
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, "-o", exe, str(tmp_path / "p.cpp")])

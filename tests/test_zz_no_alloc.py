@@ -35,8 +35,8 @@ CASES = [
     ((128, 1024, 1024, True, False, 0), (64, 512, 2048, False, True, 0)),   # abs-max launch + quantize-on-stage, then fused
     ((1024, 2048, 1024, True, True, 0), (256, 1024, 32000, True, False, 1000)),   # large-M kernel, then shortlisted output layer
     # 4 Mi values and more: the one-pass prepareA, whose workgroups exchange their abs-max through
-    # words of the static workspace that persist from call to call (arrival slots, generation word,
-    # mailboxes) - twice in a row on different inputs, a two-set input, then a small call
+    # words of the static workspace that persist from call to call (four copies, and a generation
+    # word) - twice in a row on different inputs, a two-set input, then a small call
     ((4096, 1024, 256, True, True, 0), (4096, 1024, 264, True, False, 0), (2048, 4096, 128, False, True, 0),
      (64, 512, 512, True, False, 0)),
 ]
