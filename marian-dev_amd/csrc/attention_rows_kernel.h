@@ -230,4 +230,193 @@ __global__ __launch_bounds__(256, NB == 1 ? 4 : (NB == 2 ? 3 : 2)) void attentio
   }
 }
 
+// Max and sum over the four rows of sixteen lanes, in all of them: two swaps of register halves, nothing through LDS.
+typedef unsigned v2u_rows __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float rows4_max(float v) {
+  v2u_rows s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+  s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+}
+__device__ __forceinline__ float rows4_sum(float v) {
+  v2u_rows s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(s.x) + __uint_as_float(s.y);
+  s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(s.x) + __uint_as_float(s.y);
+}
+
+// As attention_rows_kernel, for heads that fill the chip: a wave takes 16 query rows and all keys, so nothing changes hands
+// between the waves but the keys and values, which they lay out in LDS in matrix-operand order once.  The weights of a row
+// stay in registers (a transposition over the rows of sixteen lanes makes them operands).
+// Bound by the float32 pipes: a float32 matrix instruction holds up the SIMD's other float32 instructions, of other waves
+// too (32 of them and 128 fmaf take 0.45 and 0.23 us by themselves, 0.67 together), so the 128 products of 32 clocks and some 450
+// vector instructions of a wave of 64 keys add up; the form above has 890 of the latter, a division and three barriers of
+// four waves to every 16 x 64 scores.  Loads run past the ends into nothing (buffers) instead of having their rows clamped, divisions share
+// their divisor's reciprocal.
+// Measured (masks included, the form above and this): 1024 heads of 64 x 64 21.8 -> 18.8 us, 256 of them 9.2 -> 7.1; 1024 of 23 x 23 10.0 -> 7.6;
+// 512 of 48 x 48 9.6 -> 8.6; 512 of 70 x 70 23.0 -> 20.0; 384 of 128 x 128 28.5 -> 26.0.  The least number of blocks
+// of keys is a kernel of its own: four for 37 keys 14.8 us, three 12.7.
+// TILES: blocks of 16 keys; WAVES: 16-row blocks of queries of a workgroup.
+template <int TILES, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 4) void attention_heads_kernel(AttentionRowsArgs p) {
+  constexpr int kTiles = TILES, kWaves = WAVES, kStage = (TILES + WAVES - 1) / WAVES;
+  __shared__ v4f k_lds[kTiles][4][kWave], v_lds[kTiles][4][kWave];
+  const unsigned entry = blockIdx.x / (unsigned)p.row_groups;
+  const int group = (int)(blockIdx.x % (unsigned)p.row_groups);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, c = lane % 16, g = lane / 16;
+  if(p.absmax_out && blockIdx.x == 0)   // slots past the last wave
+    for(unsigned sl = p.batchQ * (unsigned)p.row_groups * kWaves + threadIdx.x; sl < (unsigned)kAbsmaxSlots; sl += 64 * kWaves) p.absmax_out[sl] = 0.0f;
+  const unsigned ekv = entry < p.batchKV ? entry : entry % p.batchKV;
+  const unsigned k_row = (unsigned)p.ks.row * 4u, v_row = (unsigned)p.vs.row * 4u, q_row = (unsigned)p.qs.row * 4u;   // bytes
+  const int row0 = (group * kWaves + wave) * 16, row = row0 + c;
+  // (as buffers that end behind their last row: rows past it read as zeros, without a check)
+  const auto k_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.k + p.ks.entry(ekv, p.heads)), 0, (int)((unsigned)(p.len - 1) * k_row + 256u), kRawBuffer);
+  const auto v_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.v + p.vs.entry(ekv, p.heads)), 0, (int)((unsigned)(p.len - 1) * v_row + 256u), kRawBuffer);
+  const auto q_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.q + p.qs.entry(entry, p.heads)), 0, (int)((unsigned)(p.m - 1) * q_row + 256u), kRawBuffer);
+  auto load = [](auto buf, unsigned lane_at, unsigned at) __attribute__((always_inline)) { return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(buf, lane_at, at, 0)); };
+
+  // ---- keys and values of the wave's block of sixteen, its query rows, their mask values ----
+  v4f kr[kStage][4], vr[kStage][4], q[4], mask[kTiles];
+  const unsigned k_at = (unsigned)(16 * wave + c) * k_row + 16u * g, v_at = (unsigned)(16 * wave + g) * v_row + 16u * c, q_at = (unsigned)row * q_row + 16u * g;
+#pragma unroll
+  for(int i = 0; i < kStage; ++i)
+#pragma unroll
+    for(int s = 0; s < 4; ++s) kr[i][s] = load(k_buf, k_at, 16u * kWaves * i * k_row + 64u * s);
+#pragma unroll
+  for(int i = 0; i < kStage; ++i)
+#pragma unroll
+    for(int x = 0; x < 4; ++x) vr[i][x] = load(v_buf, v_at, (16u * kWaves * i + 4u * x) * v_row);
+#pragma unroll
+  for(int s = 0; s < 4; ++s) q[s] = load(q_buf, q_at, 64u * s);
+  if(p.mask) {   // (values past a mask row's end: of the next row or none, not looked at)
+    unsigned mr = entry * (unsigned)p.m;
+    if(p.head_mask) {
+      mr /= p.rows_per_mask;
+      if(mr >= p.n_masks) mr %= p.n_masks;
+    } else {
+      mr = (mr + (unsigned)min(row, p.m - 1)) / p.rows_per_mask;
+      if(mr >= p.n_masks) mr %= p.n_masks;
+    }
+    const auto m_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.mask), 0, (int)(p.n_masks * (unsigned)p.len * 4u), kRawBuffer);
+    const unsigned m_at = mr * (unsigned)p.len * 4u + 16u * g;
+#pragma unroll
+    for(int t = 0; t < kTiles; ++t) mask[t] = load(m_buf, m_at, 64u * t);
+  }
+#pragma unroll
+  for(int i = 0; i < kStage; ++i) {
+    const int t = wave + kWaves * i;
+    if(kTiles % kWaves == 0 || t < kTiles) {
+#pragma unroll
+      for(int s = 0; s < 4; ++s) k_lds[t][s][lane] = rows_to_registers(kr[i][s]);
+#pragma unroll
+      for(int e = 0; e < 4; ++e) v_lds[t][c / 4][16 * g + 4 * (c % 4) + e] = v4f{vr[i][0][e], vr[i][1][e], vr[i][2][e], vr[i][3][e]};
+    }
+  }
+  __syncthreads();
+  [[maybe_unused]] const int tiles = (p.len + 15) / 16;
+  float omax = 0.0f;
+  if(row0 < p.m) {   // (whole waves)
+#pragma unroll
+    for(int s = 0; s < 4; ++s) q[s] = rows_to_registers(q[s]);
+    // ---- scores ----
+    v4f z[kTiles];
+#pragma unroll
+    for(int t = 0; t < kTiles; ++t) z[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for(int t = 0; t < kTiles; t += 2) {   // (two at a time: a product waits for the one before it into the same scores)
+#pragma unroll
+      for(int s = 0; s < 4; ++s) {
+        const v4f k0 = k_lds[t][s][lane], k1 = k_lds[t + 1 < kTiles ? t + 1 : t][s][lane];
+#pragma unroll
+        for(int x = 0; x < 4; ++x) {
+          z[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k0[x], q[s][x], z[t], 0, 0, 0);
+          if(t + 1 < kTiles) z[t + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k1[x], q[s][x], z[t + 1], 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for(int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for(int r = 0; r < 4; ++r) z[t][r] = p.scale * z[t][r];
+    if(p.mask) {
+#pragma unroll
+      for(int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for(int r = 0; r < 4; ++r) z[t][r] = z[t][r] + mask[t][r];
+    }
+    if(p.len < 16 * kTiles) {
+#pragma unroll
+      for(int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for(int r = 0; r < 4; ++r) z[t][r] = 16 * t + 4 * g + r < p.len ? z[t][r] : -__builtin_inff();
+    }
+    float mx = -__builtin_inff();
+#pragma unroll
+    for(int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for(int r = 0; r < 4; ++r) mx = fmaxf(mx, z[t][r]);
+    mx = rows4_max(mx);
+    // ---- weights (past the last key: exp(-inf) = 0, or NaN in a row whose sum is NaN anyway) ----
+    v4f part;
+    unsigned least = ~0u;
+#pragma unroll
+    for(int t = 0; t < 4; ++t) {
+      float at[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // the sums of elements 64 apart
+#pragma unroll
+      for(int b = t; b < kTiles; b += 4)
+#pragma unroll
+        for(int r = 0; r < 4; ++r) {
+          const float e = expf(z[b][r] - mx);
+          z[b][r] = e;
+          least = min(least, __float_as_uint(e) - 1u);   // (zeros pass)
+          at[r] = b == t ? e : at[r] + e;
+        }
+      part[t] = (at[0] + at[1]) + (at[2] + at[3]);
+    }
+    part = rows_to_registers(part);   // row t: block t's four rows
+    const float sum = rows4_sum((part.x + part.y) + (part.z + part.w));   // (1 .. 16 TILES, or NaN)
+    if(__all(least >= __float_as_uint(kQuotientLeast) - 1u)) {
+      const float r1 = 1.0f / sum;
+#pragma unroll
+      for(int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for(int r = 0; r < 4; ++r) z[t][r] = shared_quotient(z[t][r], sum, r1);
+    } else {
+#pragma unroll
+      for(int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for(int r = 0; r < 4; ++r) z[t][r] = z[t][r] / sum;
+    }
+#pragma unroll
+    for(int t = 0; t < kTiles; ++t) z[t] = rows_to_registers(z[t]);
+    // ---- weighted values ----
+    v4f o[4];
+#pragma unroll
+    for(int j = 0; j < 4; ++j) o[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for(int t = 0; t < kTiles; ++t)
+      if(TILES < 7 || t < tiles) {
+        v4f v[4];
+#pragma unroll
+        for(int j = 0; j < 4; ++j) v[j] = v_lds[t][j][lane];
+#pragma unroll
+        for(int x = 0; x < 4; ++x)
+#pragma unroll
+          for(int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j][x], z[t][x], o[j], 0, 0, 0);
+      }
+    if(row < p.m) {
+      float* ob = p.out + p.os.entry(entry, p.heads) + (unsigned)row * (unsigned)p.os.row + 4 * g;
+#pragma unroll
+      for(int j = 0; j < 4; ++j) {
+        *reinterpret_cast<v4f*>(ob + 16 * j) = o[j];
+        omax = abs4max(o[j], omax);
+      }
+    }
+  }
+  if(p.absmax_out) {
+    omax = wave_max(omax);
+    if(lane == 0) p.absmax_out[blockIdx.x * (unsigned)kWaves + wave] = omax;
+  }
+}
+
 }  // namespace marian_hip

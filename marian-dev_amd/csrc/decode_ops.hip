@@ -2382,6 +2382,33 @@ int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const fl
   if(groups > row_blocks) groups = row_blocks;
   if(batchQ * groups > kMaxElemsOps / 256) return MARIAN_HIP_ERR_RANGE;
   if(absmax_out && batchQ * groups * 4 > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
+  // A wave to 16 query rows where that deal leaves some CUs two workgroups: 144 heads of 64 x 64 7.7 -> 6.8 us, of 23 x 23 5.2 -> 4.6,
+  // of 80 x 80 13.1 -> 11.2; 128 of 64 x 64 stay at 6.2 (6.7), 64 of 128 x 128 at 8.8 (10.4).  Not where its workgroups have one block
+  // each (80 heads of 64 x 64 5.6, 6.7 us) unless a head has two blocks at the most.
+  if(batchQ * groups > 256 && (groups < row_blocks || row_blocks <= 2) && len <= 128) {
+    const int tiles = len <= 32 ? 2 : len <= 48 ? 3 : len <= 64 ? 4 : len <= 80 ? 5 : len <= 96 ? 6 : 8;
+    const int waves = tiles == 2 ? 2 : tiles % 4 == 0 ? 4 : 3;
+    const int64_t wgs = (row_blocks + waves - 1) / waves;   // of a head
+    // (its buffers hold a head each, offsets past the last row included, and end behind the last row of 64 values)
+    auto fits = [](int64_t row, int64_t positions) { return row <= (1 << 29) / (positions + 128); };
+    if(fits(q_strides[2], m) && fits(k_strides[2], len) && fits(v_strides[2], len) && fits(out_strides[2], m) && k_strides[2] >= 64 && v_strides[2] >= 64 &&
+       (!mask || n_masks <= (1 << 29) / (len + 128)) && (!absmax_out || batchQ * wgs * waves <= kAbsmaxSlots)) {
+      AttentionRowsArgs a{q, k, v, mask, out, absmax_out, hs.q, hs.k, hs.v, hs.out, (unsigned)batchQ, (unsigned)batchKV, (unsigned)heads,
+                          (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)row_blocks, (int)wgs, scale,
+                          mask && rows_per_mask % m == 0};
+      const dim3 grid((unsigned)(batchQ * wgs)), block((unsigned)waves * 64);
+#define MH_HEADS(TILES, WAVES) MH_LAUNCH((attention_heads_kernel<TILES, WAVES>), grid, block, 0, hst, a)
+      if(tiles == 2) MH_HEADS(2, 2);
+      else if(tiles == 3) MH_HEADS(3, 3);
+      else if(tiles == 4) MH_HEADS(4, 4);
+      else if(tiles == 5) MH_HEADS(5, 3);
+      else if(tiles == 6) MH_HEADS(6, 3);
+      else MH_HEADS(8, 4);
+#undef MH_HEADS
+      MH_HIP(hipGetLastError());
+      return MARIAN_HIP_OK;
+    }
+  }
   AttentionRowsArgs a{q, k, v, mask, out, absmax_out, hs.q, hs.k, hs.v, hs.out, (unsigned)batchQ, (unsigned)batchKV, (unsigned)heads,
                       (unsigned)n_masks, (unsigned)rows_per_mask, (int)m, (int)len, (int)row_blocks, (int)groups, scale,
                       mask && rows_per_mask % m == 0};

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "int8_common.h"
+#include "shared_quotient.h"
 
 namespace marian_hip {
 
