@@ -883,7 +883,6 @@ __device__ __forceinline__ int proj_row_key(int c16) { return (c16 ^ (c16 >> 2))
 // cover a key or value row, four consecutive positions per load, up to 64 positions in flight), the
 // same operations in the same order, so the result has the same bits.  q, k_last, v_last may lie
 // in LDS.  sc: len4 floats of this wave, part: 256 floats behind them.  Returns |out| of this lane.
-// LAST_IN_ROWS: k_last and v_last are row len - 1 of kb and vb (one address computation for all rows).
 // ANC: kb and vb are the whole caches, and cached position p lies in the entry of hypothesis anc.row[p], as in
 // attention_kernel's form of that name; anc.first: row[min(4 u + lane / 16, len - 1)], requested by the caller.
 constexpr int kAttU = 16;
@@ -893,19 +892,17 @@ struct Ancestors {
   int kv_cap;
   unsigned first[kAttU];
 };
-// HELD: the rows of positions up to 4 HELD (len at most that) are in `held` already, position 4 u + lane / 16 in k[u] and
-// v[u] but for the newest, which k_last and v_last have.
+// The cached rows of up to 4 HELD positions in registers: position 4 u + lane / 16 in k[u] and v[u] but for the newest.
 template <int HELD>
 struct HeldRows {
   v4f k[HELD], v[HELD];
 };
 template <>
 struct HeldRows<0> {};
-template <bool LAST_IN_ROWS = false, bool ANC = false, int HELD = 0>
+template <bool ANC = false>
 __device__ __forceinline__ float attention_row64(const float* q, const float* kb, const float* vb, const float* k_last,
                                                  const float* v_last, const float* mk, float mk0, int len, float scale, float* sc,
-                                                 float* part, float* out_row, int lane, const Ancestors* anc = nullptr,
-                                                 const HeldRows<HELD>* held = nullptr) {
+                                                 float* part, float* out_row, int lane, const Ancestors* anc = nullptr) {
   constexpr int dk = 64;
   const int len4 = (len + 3) & ~3;
   const int g = lane / 16, c = lane % 16;
@@ -917,8 +914,7 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
     for(int u = 0; u < kAttU; ++u) {
       if(base + 4 * u < len) {
         const int U = base / 4 + u;
-        if constexpr(LAST_IN_ROWS) r[u] = *reinterpret_cast<const v4f*>(rows + (size_t)min(4 * U + g, len - 1) * dk + 4 * c);
-        else if constexpr(ANC) {
+        if constexpr(ANC) {
           unsigned from = base == 0 ? anc->first[u] : anc->row[min(4 * U + g, len - 1)];
           from = min(from, anc->n_hyp - 1u);
           const float* at = rows + ((size_t)(from * anc->heads + anc->head) * anc->kv_cap + (size_t)(4 * U + g)) * dk + 4 * c;
@@ -932,22 +928,11 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
   };
   const v4f q4 = reinterpret_cast<const v4f*>(q)[c];
   v4f kr[kAttU], vr[kAttU];
-  if constexpr(HELD > 0) {
-    const v4f k_new = reinterpret_cast<const v4f*>(k_last)[c], v_new = reinterpret_cast<const v4f*>(v_last)[c];
-#pragma unroll
-    for(int u = 0; u < HELD; ++u) {   // (positions past the last one: it again, dropped below)
-      const bool newest = 4 * u + g >= len - 1;
-      kr[u] = newest ? k_new : held->k[u];
-      vr[u] = newest ? v_new : held->v[u];
-    }
-  } else {
-    load_rows(kb, k_last, 0, kr);
-    load_rows(vb, v_last, 0, vr);
-  }
-  constexpr int kFirst = HELD > 0 ? HELD : kAttU;   // positions of the first pass, in fours
+  load_rows(kb, k_last, 0, kr);
+  load_rows(vb, v_last, 0, vr);
   for(int base = 0;;) {
 #pragma unroll
-    for(int u0 = 0; u0 < kFirst; u0 += 4) {
+    for(int u0 = 0; u0 < kAttU; u0 += 4) {
       if(base + 4 * u0 < len) {
         float s[4];
 #pragma unroll
@@ -967,7 +952,7 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
       }
     }
     base += 4 * kAttU;
-    if(HELD > 0 || base >= len) break;
+    if(base >= len) break;
     load_rows(kb, k_last, base, kr);
   }
   float mx = -__builtin_inff();
@@ -991,9 +976,9 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
   for(int pos = lane; pos < len; pos += 64) sc[pos] = (pos == lane ? e_first : expf(sc[pos] - mx)) / sum;
   v4f o4 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   for(int base = 0; base < len; base += 4 * kAttU) {   // (rows in hand: once)
-    if(HELD == 0 && base > 0) load_rows(vb, v_last, base, vr);
+    if(base > 0) load_rows(vb, v_last, base, vr);
 #pragma unroll
-    for(int u0 = 0; u0 < kFirst; u0 += 4) {
+    for(int u0 = 0; u0 < kAttU; u0 += 4) {
       if(base + 4 * u0 < len) {
         float w[4];
 #pragma unroll
@@ -1014,6 +999,102 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
   out_row[lane] = o;
   return fabsf(o);
 }
+
+// attention_row64 where all rows are at hand, in LDS or in registers, and no more than 16 BLOCKS: no pass after another, no
+// address of its own for every row and no loop over positions - 64 of them are the lanes of the wave.  The same operations in the same
+// order.  Bound by its own instructions, one wave to a row and two to a SIMD: the general form took 5200 - 6500 clocks of a launch's 15 000 - 20 000
+// with staged rows (a branch around every LDS load, 2200 of them), 3000 - 4600 with held ones.  Steps of 6 layers, with it, weights asked for
+// without vector arithmetic and one copy of the quantization instead of eight: 6 x 512 over 12 and 23 positions 208.7 -> 196.8 us, 65 x 512 over
+// 34 and 47 315.9 -> 307.7, 128 x 1024 over 21 and 60 392.0 -> 378.4.
+// keys(r), values(r): rows 4 u + lane / 16 (those past the last one: it again), four values from 4 (lane % 16) on.
+// Positions past len within four weigh nothing, fours past it are not added.
+template <int BLOCKS, class Keys, class Values>
+__device__ __forceinline__ float attention_row64_short(const float* q, Keys keys, Values values, const float* mk, float mk0, int len,
+                                                       float scale, float* sc, float* part, float* out_row, int lane) {
+  static_assert(BLOCKS <= 8, "two positions a lane");
+  const int g = lane / 16, c = lane % 16;
+  const v4f q4 = reinterpret_cast<const v4f*>(q)[c];
+  v4f r[4 * BLOCKS];
+  keys(r);
+  [[maybe_unused]] float mk1 = 0.0f;
+  if constexpr(BLOCKS > 4) {
+    if(mk) mk1 = mk[min(64 + lane, len - 1)];
+  }
+#pragma unroll
+  for(int b = 0; b < BLOCKS; ++b) {
+    if(b == 0 || 16 * b < len) {
+      float s[4];
+#pragma unroll
+      for(int u = 0; u < 4; ++u) {
+        float t = q4.x * r[4 * b + u].x;
+        t = fmaf(q4.y, r[4 * b + u].y, t);
+        t = fmaf(q4.z, r[4 * b + u].z, t);
+        s[u] = fmaf(q4.w, r[4 * b + u].w, t);
+      }
+#pragma unroll
+      for(int u = 0; u < 4; ++u) s[u] = row16_sum(s[u]);
+      if(c == 0) {   // (past len: not looked at)
+#pragma unroll
+        for(int u = 0; u < 4; ++u) sc[16 * b + 4 * u + g] = scale * s[u];
+      }
+    }
+  }
+  values(r);
+  const bool here = lane < len;
+  [[maybe_unused]] const bool here1 = 64 + lane < len;
+  [[maybe_unused]] float z1 = 0.0f, e1 = 0.0f;
+  float z = sc[lane];
+  if(mk) z = z + mk0;
+  float mx = here ? fmaxf(-__builtin_inff(), z) : -__builtin_inff();
+  if constexpr(BLOCKS > 4) {
+    z1 = sc[64 + lane];
+    if(mk) z1 = z1 + mk1;
+    mx = here1 ? fmaxf(mx, z1) : mx;
+  }
+  mx = wave_maxf(mx);
+  const float e = here ? expf(z - mx) : 0.0f;
+  float sum = 0.0f + e;
+  if constexpr(BLOCKS > 4) {
+    e1 = here1 ? expf(z1 - mx) : 0.0f;
+    sum += e1;
+  }
+  sum = wave_sum(sum);
+  sc[lane] = here ? e / sum : 0.0f;
+  if constexpr(BLOCKS > 4) sc[64 + lane] = here1 ? e1 / sum : 0.0f;
+  float w[4 * BLOCKS];
+#pragma unroll
+  for(int u = 0; u < 4 * BLOCKS; ++u) w[u] = sc[4 * u + g];
+  v4f o4 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for(int b = 0; b < BLOCKS; ++b) {
+    if(b == 0 || 16 * b < len) {
+#pragma unroll
+      for(int u = 4 * b; u < 4 * b + 4; ++u) {
+        const bool there = u % 4 == 0 || 4 * u < len;   // (rows that are not there may be infinite)
+        o4.x = fmaf(w[u], there ? r[u].x : 0.0f, o4.x);
+        o4.y = fmaf(w[u], there ? r[u].y : 0.0f, o4.y);
+        o4.z = fmaf(w[u], there ? r[u].z : 0.0f, o4.z);
+        o4.w = fmaf(w[u], there ? r[u].w : 0.0f, o4.w);
+      }
+    }
+  }
+  reinterpret_cast<v4f*>(part)[g * 16 + c] = o4;   // partial sums of the positions g, g + 4, ...
+  const float o = ((part[lane] + part[64 + lane]) + part[128 + lane]) + part[192 + lane];
+  out_row[lane] = o;
+  return fabsf(o);
+}
+// Rows of 64 values one after the other in LDS.
+template <int BLOCKS>
+struct StagedRows {
+  const float* rows;
+  int len, lane;
+  __device__ __forceinline__ void operator()(v4f (&r)[4 * BLOCKS]) const {
+    const unsigned first = (unsigned)(lane / 16) * 256u, last = (unsigned)(len - 1) * 256u;
+#pragma unroll
+    for(int u = 0; u < 4 * BLOCKS; ++u)
+      r[u] = *reinterpret_cast<const v4f*>(reinterpret_cast<const char*>(rows) + min(first + 1024u * u, last) + (lane % 16) * 16);
+  }
+};
 
 // Attention over caches that several query rows share (the encoder's keys and values: query row
 // r reads cache entry r % batchKV, so rows e, e + batchKV, e + 2 batchKV, .. - the hypotheses of a
@@ -1070,8 +1151,8 @@ __global__ __launch_bounds__(256) void attention_shared_kernel(const float* __re
   }
   __syncthreads();
   if(valid) {   // (whole waves)
-    float omax = attention_row64<true>(Q + (size_t)wr * 64, ks, vs, ks + (size_t)(len - 1) * 64, vs + (size_t)(len - 1) * 64, mk,
-                                       mk0, len, scale, sc, sc + len4, out + (size_t)wr * 64, lane);
+    float omax = attention_row64_short<PASSES>(Q + (size_t)wr * 64, StagedRows<PASSES>{ks, len, lane}, StagedRows<PASSES>{vs, len, lane}, mk,
+                                               mk0, len, scale, sc, sc + len4, out + (size_t)wr * 64, lane);
     if(absmax_out) {
       omax = wave_maxf(omax);
       if(lane == 0) absmax_out[wr] = omax;
@@ -1158,13 +1239,16 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     for(int e = 0; e < 4; ++e) in[e] = *reinterpret_cast<const v4f*>(src + e * 16);
   }
   v4i w[NPROJ][PW];
-  const int ncol = h * 64 + wn * 32 + li;
-  // (asked for in the order the multiplication takes them: sub-step by sub-step, all projections)
+  const unsigned w_off = stream32_lane_offset(h * 64 + wn * 32 + li, lg), w_step = 32u * (unsigned)N;
+  // (asked for in the order the multiplication takes them: sub-step by sub-step, all projections; as buffers: no vector arithmetic)
 #pragma unroll
   for(int pp = 0; pp < PW; ++pp) {
-    const size_t at = stream32_lane_offset(ncol, lg) + (size_t)stream32_clamped_substep(kw * steps + pp, S) * 32u * (size_t)N;
+    const unsigned at = (unsigned)stream32_clamped_substep(kw * steps + pp, S) * w_step;
 #pragma unroll
-    for(int g = 0; g < NPROJ; ++g) w[g][pp] = load16(p.Bq[g] + at);
+    for(int g = 0; g < NPROJ; ++g) {
+      const auto w_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.Bq[g]), 0, (int)((unsigned)K * (unsigned)N), kRawBuffer);
+      w[g][pp] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w_buf, w_off, at, 0));
+    }
   }
   // keys and values of the workgroup's sentences: sixteen threads per position, 32 positions per pass
   constexpr int kStageSegs = STAGED ? SEGS : 1, kStagePasses = STAGED ? PASSES : 1;
@@ -1248,9 +1332,6 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
   if constexpr(STAGED && NORM) load_stage();
   const float aqm = quant_mult_from_maxabs(amax);
   const bool finite = aqm < __builtin_inff();
-  float unquant[NPROJ];
-#pragma unroll
-  for(int g = 0; g < NPROJ; ++g) unquant[g] = unquant_mult(aqm, bqm[g], 1.0f);
   if(has_in) {
     uint32_t q[4];
 #pragma unroll
@@ -1268,8 +1349,11 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
   if constexpr(NORM) {   // wave w holds row w: quantized where this workgroup multiplies it, written out by one workgroup
     const int row = wave;
     if(row < M) {
+      int at = -1;   // (scalar: the quantization stands here once)
+#pragma unroll
       for(int r = 0; r < R; ++r)
-        if(row_of(r) == row) nr.quantize(a_lds, r, K, aqm, proj_row_key);
+        if(row_of(r) == row) at = r;
+      if(at >= 0) nr.quantize(a_lds, at, K, aqm, proj_row_key);
       if(h == 0 && first_rows) nr.store(p.norm, row, K);
     }
   }
@@ -1292,6 +1376,9 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
       for(int g = 0; g < NPROJ; ++g) acc[g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[g][pp], a, acc[g], 0, 0, 0);
     }
   }
+  float unquant[NPROJ];   // (while the products are made)
+#pragma unroll
+  for(int g = 0; g < NPROJ; ++g) unquant[g] = unquant_mult(aqm, bqm[g], 1.0f);
   // accumulator value v of lane (li, lg): input row li, column 8 * (v / 4) + 4 * lg + v % 4 of the
   // wave's 32; a tile row is 128 bytes, its eight 16-byte pieces XOR-permuted by the row number
   if(li < R) {
@@ -1372,13 +1459,25 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     if constexpr(STAGED) {
       const float* ks = kv_lds + (size_t)(2 * (wave & ((1 << p.share_shift) - 1))) * p.len * 64;
       const float* vs = ks + (size_t)p.len * 64;
-      omax = attention_row64<true>(q, ks, vs, ks + (size_t)(p.len - 1) * 64, vs + (size_t)(p.len - 1) * 64, mk, mk0, p.len,
-                             p.att_scale, sc, sc + len4, p.out + (size_t)wr * 64, lane);
+      using Rows = StagedRows<2 * PASSES>;
+      omax = attention_row64_short<2 * PASSES>(q, Rows{ks, p.len, lane}, Rows{vs, p.len, lane}, mk, mk0, p.len, p.att_scale, sc, sc + len4,
+                                               p.out + (size_t)wr * 64, lane);
     } else if constexpr(HELD > 0) {
-      omax = attention_row64<false, false, HELD>(q, kb, vb, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
-                                                 p.out + (size_t)wr * 64, lane, nullptr, &held);
+      // (positions past the last one: it again, dropped by their weight)
+      struct WithNewest {
+        const v4f (&rows)[HELD];
+        const float* newest;
+        int len, lane;
+        __device__ __forceinline__ void operator()(v4f (&r)[HELD]) const {
+          const v4f last = reinterpret_cast<const v4f*>(newest)[lane % 16];
+#pragma unroll
+          for(int u = 0; u < HELD; ++u) r[u] = 4 * u + lane / 16 >= len - 1 ? last : rows[u];
+        }
+      };
+      omax = attention_row64_short<HELD / 4>(q, WithNewest{held.k, k_last, p.len, lane}, WithNewest{held.v, v_last, p.len, lane}, mk, mk0, p.len, p.att_scale, sc,
+                                             sc + len4, p.out + (size_t)wr * 64, lane);
     } else if constexpr(ANC) {
-      omax = attention_row64<false, true>(q, p.k_cache, p.v_cache, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
+      omax = attention_row64<true>(q, p.k_cache, p.v_cache, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
                                           p.out + (size_t)wr * 64, lane, &anc);
     } else {
       omax = attention_row64(q, kb, vb, k_last, v_last, mk, mk0, p.len, p.att_scale, sc, sc + len4,
