@@ -1277,6 +1277,13 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     bias4[it] = *reinterpret_cast<const v4f*>(b ? b + h * 64 + (tg % 2) * 32 + pc * 4 : reinterpret_cast<const float*>(p.Bq[0]));
   }
 
+  // NORM: as which row this workgroup multiplies the one that this wave normalizes (found while the loads are under way)
+  [[maybe_unused]] int norm_at = -1;
+  if constexpr(NORM) {
+    norm_at = __builtin_amdgcn_readfirstlane(proj_place_of(p.share_shift, p.share_nb, p.share_hyps, p.share_per, (int)blockIdx.y, (int)blockIdx.z, wave));
+    if(norm_at >= R) norm_at = -1;
+  }
+
   // The keys and values are asked for last - a wave's loads complete in the order of their issue, and they are needed
   // last.  No branches around them (positions past the end repeat the last one; the number of loads is the kernel's), so that the
   // waits in front of the earlier loads' uses count exactly.  Behind a layer norm, whose reductions they would come in
@@ -1349,11 +1356,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
   if constexpr(NORM) {   // wave w holds row w: quantized where this workgroup multiplies it, written out by one workgroup
     const int row = wave;
     if(row < M) {
-      int at = -1;   // (scalar: the quantization stands here once)
-#pragma unroll
-      for(int r = 0; r < R; ++r)
-        if(row_of(r) == row) at = r;
-      if(at >= 0) nr.quantize(a_lds, at, K, aqm, proj_row_key);
+      if(norm_at >= 0) nr.quantize(a_lds, norm_at, K, aqm, proj_row_key);
       if(h == 0 && first_rows) nr.store(p.norm, row, K);
     }
   }

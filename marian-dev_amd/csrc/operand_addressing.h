@@ -144,6 +144,15 @@ __host__ __device__ __forceinline__ int proj_row_of(int shift, int sentences, in
   if(j >= per_wg || hyp >= hyps) return 0x7fffffff;
   return hyp * sentences + (group << shift) + (r & ((1 << shift) - 1));
 }
+// The other way round: as which row the workgroup takes input row `row` (below M), or -1.
+__host__ __device__ __forceinline__ int proj_place_of(int shift, int sentences, int hyps, int per_wg, int group, int chunk, int row) {
+  if(shift < 0) {
+    const int r = row - group * per_wg;
+    return r >= 0 && r < per_wg ? r : -1;
+  }
+  const int hyp = (int)((unsigned)row / (unsigned)sentences), j = hyp - chunk * per_wg, s = row - hyp * sentences - (group << shift);
+  return s >= 0 && s < 1 << shift && j >= 0 && j < per_wg && hyp < hyps ? (j << shift) + s : -1;
+}
 // sentence groups of a launch (shift >= 0), and the first sentence of one
 __host__ __device__ __forceinline__ int proj_groups(int shift, int sentences) { return sentences >> shift; }
 __host__ __device__ __forceinline__ int proj_first_sentence(int shift, int group) { return group << shift; }

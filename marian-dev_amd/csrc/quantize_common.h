@@ -82,14 +82,18 @@ __device__ __forceinline__ float abs4max(v4f x, float m) {
 
 // Max over each row of 16 lanes, left in all 16 of them: four DPP steps (the two lane swaps within
 // a quad, the mirror within half a row and within the row).  All lanes of the wave must be active.
-// (fmaxf passes over NaN operands whatever the order, so the result does not depend on the order.)
-__device__ __forceinline__ float row16_max(float m) {
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0xB1, 0xF, 0xF, false)));   // quad_perm [1,0,3,2]
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x4E, 0xF, 0xF, false)));   // quad_perm [2,3,0,1]
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x141, 0xF, 0xF, false)));  // row_half_mirror
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x140, 0xF, 0xF, false)));  // row_mirror
-  return m;
+// The magnitudes that are reduced here are zero or positive and never NaN (fmaxf passes over NaN operands), so their bits order as
+// unsigned numbers do, and a step is one instruction: a float maximum has its operands made quiet first, four more
+// (ten steps stand between the arrival of a row and its quantization; a block of 64 x 512 x 2048 and back 10.43 -> 10.27 us).
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ unsigned max_step(unsigned m) {
+  const unsigned t = (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, CTRL, ROWS, 0xF, false);
+  return t > m ? t : m;
 }
+__device__ __forceinline__ unsigned row16_max_bits(unsigned m) {
+  return max_step<0x140>(max_step<0x141>(max_step<0x4E>(max_step<0xB1>(m))));   // quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror, row_mirror
+}
+__device__ __forceinline__ float row16_max(float m) { return __uint_as_float(row16_max_bits(__float_as_uint(m))); }
 // Max over the wave, in all lanes: within the rows, then across them with the two row-broadcast
 // DPP steps (rows 1 and 3 take in the last lane of the row before them, then rows 2 and 3 the last
 // lane of row 1), which leaves the result in lane 63, read from there as a scalar.  No step goes
@@ -97,10 +101,8 @@ __device__ __forceinline__ float row16_max(float m) {
 // sit between the arrival of the activations and their quantization in every fused call).  All
 // lanes of the wave must be active.
 __device__ __forceinline__ float wave_max(float m) {
-  m = row16_max(m);
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, m), __builtin_bit_cast(int, m), 0x142, 0xA, 0xF, false)));   // row_bcast:15
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, m), __builtin_bit_cast(int, m), 0x143, 0xC, 0xF, false)));   // row_bcast:31
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), 63));
+  const unsigned r = max_step<0x143, 0xC>(max_step<0x142, 0xA>(row16_max_bits(__float_as_uint(m))));   // row_bcast:15, row_bcast:31
+  return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)r, 63));
 }
 
 // Max over the workgroup of WAVES waves (at most 16); every thread returns the result.
