@@ -1209,8 +1209,10 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     static_assert(!ANC || (NPROJ == 3 && !STAGED), "self-attention");
     anc.row = p.anc + (size_t)min(m_wave, M - 1) * p.kv_cap;
     anc.n_hyp = (unsigned)M; anc.heads = (unsigned)p.heads; anc.head = (unsigned)h; anc.kv_cap = p.kv_cap;
+    const auto row_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(anc.row), 0, p.len * 4, kRawBuffer);
 #pragma unroll
-    for(int u = 0; u < (HELD > 0 ? HELD : kAttU); ++u) anc.first[u] = anc.row[min(4 * u + lane / 16, p.len - 1)];
+    for(int u = 0; u < (HELD > 0 ? HELD : kAttU); ++u)   // (past the end: hypothesis 0, not looked at)
+      anc.first[u] = __builtin_amdgcn_raw_buffer_load_b32(row_buf, (unsigned)lane / 16 * 4u, 16u * u, 0);
   };
   if constexpr(ANC && HELD > 0) {   // (they are addresses)
     load_ancestors();
@@ -1313,11 +1315,13 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     const auto k_buf = __builtin_amdgcn_make_buffer_rsrc(p.k_cache + entry * p.kv_cap * 64, 0, (int)bytes, kRawBuffer);
     const auto v_buf = __builtin_amdgcn_make_buffer_rsrc(p.v_cache + entry * p.kv_cap * 64, 0, (int)bytes, kRawBuffer);
     unsigned at[HELD];
+    const unsigned rows_of_one = (unsigned)p.heads * (unsigned)p.kv_cap, first = (unsigned)h * (unsigned)p.kv_cap + (unsigned)lane / 16;
 #pragma unroll
     for(int u = 0; u < HELD; ++u) {
       const unsigned pos = (unsigned)(4 * u + lane / 16);
-      at[u] = pos * 256u + (lane % 16) * 16u;
-      if(ANC) at[u] += (min(anc.first[u], anc.n_hyp - 1u) * (unsigned)p.heads + (unsigned)h) * (unsigned)p.kv_cap * 256u;
+      // (both below 2^24, see the launcher: a full-rate multiplication)
+      if(ANC) at[u] = (__umul24(min(anc.first[u], anc.n_hyp - 1u), rows_of_one) + (first + 4u * u)) * 256u + (lane % 16) * 16u;
+      else at[u] = pos * 256u + (lane % 16) * 16u;
       if((int)pos >= p.len - 1) at[u] = 0xFFFFFFF0u;   // (past the cached ones: past the buffer, nothing is fetched)
     }
 #pragma unroll
@@ -1338,11 +1342,11 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
   amax = block_max<kProjThreads / 64>(amax, red);
   if constexpr(STAGED && NORM) load_stage();
   const float aqm = quant_mult_from_maxabs(amax);
-  const bool finite = aqm < __builtin_inff();
+  const float by = quantizer(aqm);
   if(has_in) {
     uint32_t q[4];
 #pragma unroll
-    for(int e = 0; e < 4; ++e) q[e] = finite ? quantize_pack4_finite(in[e], aqm) : quantize_pack4(in[e], aqm);
+    for(int e = 0; e < 4; ++e) q[e] = quantize_pack4(in[e], by);
     const int slot0 = (c16 / 2) * 64, x = r_in ^ proj_row_key(c16);
     const int m = row_of(min(r_in, R - 1));
 #pragma unroll

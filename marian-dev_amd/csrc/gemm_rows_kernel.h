@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     }
     const float aqm = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(quant_mult_from_maxabs(amax))));
     unquant = unquant_mult(aqm, bqm, args.scale);
-    const bool finite = aqm < __builtin_inff();   // (see gemm_stream32_kernel)
+    const float by = quantizer(aqm);
     if(WRITE_AQ && tile.by == 0 && tid == 0) *reinterpret_cast<float*>(aq_out + (size_t)M * K) = aqm;
 #pragma unroll
     for(int e = 0; e < 16; ++e) acc[e] = 0;
@@ -168,13 +168,8 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     for(int t = 0; t < T; ++t) {
       const int d = t % (D > 0 ? D : 1);
       uint32_t q[LOADS];
-      if(finite) {
 #pragma unroll
-        for(int j = 0; j < LOADS; ++j) q[j] = quantize_pack4_finite(a[d][j], aqm);
-      } else {
-#pragma unroll
-        for(int j = 0; j < LOADS; ++j) q[j] = quantize_pack4(a[d][j], aqm);
-      }
+      for(int j = 0; j < LOADS; ++j) q[j] = quantize_pack4(a[d][j], by);
 #pragma unroll
       for(int j = 0; j < LOADS; ++j) *reinterpret_cast<uint32_t*>(put + j * 64) = q[j];
       if(WRITE_AQ) {

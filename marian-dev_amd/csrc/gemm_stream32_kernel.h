@@ -234,7 +234,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
   }
 
   float aqm = 0.0f;        // quantMult of the activations (fused modes)
-  bool finite_t = false;   // kFusedTiled: the quantMult is finite
+  float by = 0.0f;   // the multiplier of the quantizing (kFusedTiled, kFusedAll)
   // The multiplier of the epilogue (a division through double precision) is worked out as soon as
   // the quantMult of the activations is known, under the matrix instructions.
   float unquant = 0.0f;
@@ -279,13 +279,8 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
         const int g = (slot / 4) * 4, r = g / (2 * Cfg::CS), c16 = g % (2 * Cfg::CS);
         const int m = m_base + r;
         uint32_t q[4];
-        if(finite_t) {
 #pragma unroll
-          for(int e = 0; e < 4; ++e) q[e] = quantize_pack4_finite(stagef[j][e], aqm);
-        } else {
-#pragma unroll
-          for(int e = 0; e < 4; ++e) q[e] = quantize_pack4(stagef[j][e], aqm);
-        }
+        for(int e = 0; e < 4; ++e) q[e] = quantize_pack4(stagef[j][e], by);
         const int slot0 = ((c16 / 2) * MT32 + r / 32) * 64, x = (r % 32) ^ stream32_row_key(c16);
 #pragma unroll
         for(int e = 0; e < 4; ++e) {
@@ -347,7 +342,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
     amax = block_max<kStream32Waves>(amax, red);
     aqm = quant_mult_from_maxabs(amax);
     unquant = unquant_mult(aqm, bqm, args.scale);
-    finite_t = aqm < __builtin_inff();   // (see the fused form below)
+    by = quantizer(aqm);
     if(MH_PROF(args)) tp[1] = MH_CLOCK();
     if(aq_out && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0)
       *reinterpret_cast<float*>(aq_out + (size_t)M * K) = aqm;
@@ -378,23 +373,14 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
     if(MH_PROF(args)) tp[1] = MH_CLOCK();
     aqm = quant_mult_from_maxabs(amax);
     unquant = unquant_mult(aqm, bqm, args.scale);
-    // With a finite quantMult no product can leave [-127.0001, 127.0001]: finite values are at
-    // most the abs-max in magnitude, and an infinite value makes the quantMult 0 and its product
-    // NaN.  (An abs-max of zero, or one below 127 / FLT_MAX, gives an infinite quantMult, and then
-    // infinite products, which the conversion of the CPU path turns into -127, not +127.)
-    const bool finite = aqm < __builtin_inff();
+    by = quantizer(aqm);
     uint32_t q[kFusedGroups][4];
 #pragma unroll
     for(int j = 0; j < kFusedGroups; ++j) {
       const unsigned rr = row - m_base;   // row within this workgroup's tile
       if(in_range(j) && rr < (unsigned)R) {
-        if(finite) {
 #pragma unroll
-          for(int e = 0; e < 4; ++e) q[j][e] = quantize_pack4_finite(vals[j][e], aqm);
-        } else {
-#pragma unroll
-          for(int e = 0; e < 4; ++e) q[j][e] = quantize_pack4(vals[j][e], aqm);
-        }
+        for(int e = 0; e < 4; ++e) q[j][e] = quantize_pack4(vals[j][e], by);
         // slot of group e: chunk c16 + e, i.e. sub-step (c16 + e) / 2, half (c16 + e) % 2, and
         // the row permuted by the key of chunk c16 + e, which is the key of c16 (c16 % 4 == 0) ^ e
         const unsigned slot0 = ((c16 >> 1) * MT32 + (rr >> 5)) * 64, x = (rr & 31) ^ stream32_row_key(c16);

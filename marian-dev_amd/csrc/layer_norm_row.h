@@ -116,19 +116,12 @@ struct NormRow {
   template <typename KEY>
   __device__ __forceinline__ void quantize(int8_t* lds, int row, int K, float qm, KEY key) const {
     const int lane = threadIdx.x % kWave;
-    uint32_t q[VECS];
-    if(qm < __builtin_inff()) {
-#pragma unroll
-      for(int j = 0; j < VECS; ++j) q[j] = quantize_pack4_finite(v[j], qm);
-    } else {
-#pragma unroll
-      for(int j = 0; j < VECS; ++j) q[j] = quantize_pack4(v[j], qm);
-    }
+    const float by = quantizer(qm);
 #pragma unroll
     for(int j = 0; j < VECS; ++j) {
       const int i = j * kWave + lane, c16 = i / 4;
       if(i < K / 4)
-        *reinterpret_cast<uint32_t*>(lds + ((c16 / 2) * 64 + (c16 % 2) * 32 + (row ^ key(c16))) * 16 + (i % 4) * 4) = q[j];
+        *reinterpret_cast<uint32_t*>(lds + ((c16 / 2) * 64 + (c16 % 2) * 32 + (row ^ key(c16))) * 16 + (i % 4) * 4) = quantize_pack4(v[j], by);
     }
   }
   __device__ __forceinline__ void store(const NormInput& n, int row, int K) const {

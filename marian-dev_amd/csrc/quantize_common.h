@@ -21,25 +21,6 @@ static_assert(kOnePassGenOffset + 128 == kOnePassWordsOffset && kWorkspaceBytes 
 constexpr int kSingleBlockThreads = 1024;
 constexpr int kSingleBlockMaxElems = 32 * 1024;     // one workgroup does abs-max and quantize (beyond: 8.6 us against 6.4 us for two launches)
 
-// q = clamp(rne(fl32(x * qm)), -127, 127); products that are NaN or outside int32 give -127
-// (x86 cvtps2dq integer-indefinite followed by saturating packs and max(-127)).
-__device__ __forceinline__ int quantize_one(float x, float qm) {
-  float v = x * qm;
-  float r = __builtin_rintf(v);
-  r = fminf(fmaxf(r, -127.0f), 127.0f);
-  int q = (int)r;
-  return (fabsf(v) < 2147483648.0f) ? q : -127;
-}
-
-// The value whose rounding to nearest-even is quantize_one(x, qm): clamping to [-127, 127] first
-// commutes with rounding (the bounds are integers; med3 returns -127 for NaN).  Products >= 2^31
-// (only possible for non-finite inputs) follow the x86 conversion and give -127.
-__device__ __forceinline__ float quantize_clamped(float x, float qm) {
-  const float v = x * qm;
-  const float c = __builtin_amdgcn_fmed3f(v, -127.0f, 127.0f);
-  return (v >= 2147483648.0f) ? -127.0f : c;
-}
-
 // Four clamped products -> four int8 in one word.  Adding 1.5 * 2^23 rounds to nearest-even and
 // leaves the integer in the low byte of the sum; the SDWA form of the add writes that low byte
 // straight into byte 0..3 of the destination, so no byte shuffles are needed afterwards.
@@ -57,19 +38,19 @@ __device__ __forceinline__ uint32_t round_pack4(float c0, float c1, float c2, fl
   return q;
 }
 
-// Fast form for the usual case (finite quantMult): every product lies within
-// [-127.0001, 127.0001], so the out-of-range check of quantize_clamped can never fire (med3
-// still maps a NaN among the values to -127).
-__device__ __forceinline__ uint32_t quantize_pack4_finite(v4f x, float qm) {
+// q = clamp(rne(fl32(x * qm)), -127, 127); products that are NaN or outside int32 give -127 (x86 cvtps2dq integer-indefinite followed
+// by saturating packs and max(-127)).  Clamping first commutes with the rounding (the bounds are integers), and med3 returns -127
+// for NaN.  With a finite quantMult every product lies within [-127.0001, 127.0001]: finite values are at most the abs-max in
+// magnitude, and an infinite value makes the quantMult 0 and its product NaN.  An abs-max of zero, or one below 127 / FLT_MAX, gives an
+// infinite quantMult, and then products that are infinite or NaN: all -127, so NaN stands in for such a multiplier (a second path
+// for it was half of the quantizing code of a launch, which fetches what it passes over).
+__device__ __forceinline__ float quantizer(float qm) { return qm < __builtin_inff() ? qm : __builtin_nanf(""); }
+// qm: a quantizer's
+__device__ __forceinline__ uint32_t quantize_pack4(v4f x, float qm) {
   return round_pack4(__builtin_amdgcn_fmed3f(x.x * qm, -127.0f, 127.0f),
                      __builtin_amdgcn_fmed3f(x.y * qm, -127.0f, 127.0f),
                      __builtin_amdgcn_fmed3f(x.z * qm, -127.0f, 127.0f),
                      __builtin_amdgcn_fmed3f(x.w * qm, -127.0f, 127.0f));
-}
-
-__device__ __forceinline__ uint32_t quantize_pack4(v4f x, float qm) {
-  return round_pack4(quantize_clamped(x.x, qm), quantize_clamped(x.y, qm), quantize_clamped(x.z, qm),
-                     quantize_clamped(x.w, qm));
 }
 
 __device__ __forceinline__ float abs4max(v4f x, float m) {

@@ -47,15 +47,15 @@ __global__ __launch_bounds__(kSingleBlockThreads) void prepare_a_single_block_ke
     for(int u = 0; u < 8; ++u) m = abs4max(v[u], m);
   }
   m = block_max<kSingleBlockThreads / kWave>(m, red);
-  const float qm = quant_mult_from_maxabs(m);
+  const float qm = quant_mult_from_maxabs(m), by = quantizer(qm);
   uint4* o16 = reinterpret_cast<uint4*>(out);
   for(int i = threadIdx.x; i < n16; i += kSingleBlockThreads) {
     v4f a = x4[4 * i], b = x4[4 * i + 1], c = x4[4 * i + 2], d = x4[4 * i + 3];
     uint4 q;
-    q.x = quantize_pack4(a, qm);
-    q.y = quantize_pack4(b, qm);
-    q.z = quantize_pack4(c, qm);
-    q.w = quantize_pack4(d, qm);
+    q.x = quantize_pack4(a, by);
+    q.y = quantize_pack4(b, by);
+    q.z = quantize_pack4(c, by);
+    q.w = quantize_pack4(d, by);
     o16[i] = q;
   }
   if(threadIdx.x == 0) *reinterpret_cast<float*>(out + (size_t)n16 * 16) = qm;
@@ -107,8 +107,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
   if(G > 1)
     amax = onepass_exchange((int)blockIdx.x, m, nonce, gen, words, gen_word, polls, G, &shared_max,
                                   [&] { return onepass_scan<1024>(x, (size_t)n16 * 4, red); });
-  const float qm = quant_mult_from_maxabs(amax);
-  const bool finite = qm < __builtin_inff();
+  const float qm = quant_mult_from_maxabs(amax), by = quantizer(qm);
 #pragma unroll
   for(int j = 0; j < SETS; ++j) {
     if(!live[j]) continue;
@@ -118,7 +117,7 @@ __global__ __launch_bounds__(1024) void prepare_a_onepass_kernel(const float* __
     // output i, so that a wave stores 1 KB of contiguous bytes, 16 per lane.
 #pragma unroll
     for(int e = 0; e < 4; ++e)
-      turn[(quad * 4 + e) * 4 + qlane] = finite ? quantize_pack4_finite(vals[j][e], qm) : quantize_pack4(vals[j][e], qm);
+      turn[(quad * 4 + e) * 4 + qlane] = quantize_pack4(vals[j][e], by);
     const uint4 w = *reinterpret_cast<const uint4*>(&turn[(quad * 4 + qlane) * 4]);
     *reinterpret_cast<uint4*>(reinterpret_cast<char*>(out) + (size_t)q * 64 + qlane * 16) = w;
   }
@@ -157,8 +156,7 @@ __global__ __launch_bounds__(THREADS) void quantize_a_wide_kernel(const float* _
 #pragma unroll
   for(int i = 0; i < kAbsmaxSlots / THREADS; ++i) m = fmaxf(m, pm[i]);
   m = block_max<THREADS / kWave>(m, red);
-  const float qm = quant_mult_from_maxabs(m);
-  const bool finite = qm < __builtin_inff();
+  const float qm = quant_mult_from_maxabs(m), by = quantizer(qm);
   for(; set < n_sets; set += blocks) {
     v4f cur[4];
 #pragma unroll
@@ -169,7 +167,7 @@ __global__ __launch_bounds__(THREADS) void quantize_a_wide_kernel(const float* _
       // (the four lanes of a quad sit in one wave, whose LDS operations execute in order)
 #pragma unroll
       for(int e = 0; e < 4; ++e)
-        turn[(quad * 4 + e) * 4 + qlane] = finite ? quantize_pack4_finite(cur[e], qm) : quantize_pack4(cur[e], qm);
+        turn[(quad * 4 + e) * 4 + qlane] = quantize_pack4(cur[e], by);
       const uint4 w = *reinterpret_cast<const uint4*>(&turn[(quad * 4 + qlane) * 4]);
       *reinterpret_cast<uint4*>(reinterpret_cast<char*>(out) + (size_t)q * 64 + qlane * 16) = w;
     }
@@ -193,9 +191,10 @@ __device__ __forceinline__ void load_b_tile(const float* __restrict__ W, int K, 
 __device__ __forceinline__ void store_b_tile(const float (&v)[16], float qm, uint32_t (*tile)[17], int K, int N, int n0, int k0,
                                              int thread, bool live, int8_t* __restrict__ out) {
   const int tn = thread % 64, tk = thread / 64;
+  const float by = quantizer(qm);
 #pragma unroll
   for(int g = 0; g < 4; ++g)   // four consecutive k of column n: one packed dword
-    tile[tn][tk * 4 + g] = quantize_pack4(v4f{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}, qm);
+    tile[tn][tk * 4 + g] = quantize_pack4(v4f{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}, by);
   __syncthreads();
   // 64 columns (n) x four 16-byte chunks (k): two neighbouring threads write the two halves of a
   // column's sub-step, a wave 32 columns of one sub-step (1 KB of consecutive memory)
