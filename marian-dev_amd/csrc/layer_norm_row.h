@@ -45,29 +45,46 @@ __device__ __forceinline__ float normalize_row(v4f (&v)[VECS], const v4f (&t)[VE
     if(j * kWave + lane < cols4) sum += (v[j].x + v[j].y) + (v[j].z + v[j].w);
   }
   const float mean = wave_sum(sum) / (float)cols;
-  float sq = 0.0f;
+  float sq = 0.0f, least = kQuotientMost;
 #pragma unroll
   for(int j = 0; j < VECS; ++j) {
+    v[j] = v4f{v[j].x - mean, v[j].y - mean, v[j].z - mean, v[j].w - mean};
     if(j * kWave + lane < cols4) {
-      const float d0 = v[j].x - mean, d1 = v[j].y - mean, d2 = v[j].z - mean, d3 = v[j].w - mean;
-      sq += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
+      sq += (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w);
+      least = fminf(fminf(fminf(least, fabsf(v[j].x)), fminf(fabsf(v[j].y), fabsf(v[j].z))), fabsf(v[j].w));
     }
   }
   const float sigma = sqrtf(wave_sum(sq) / (float)cols + eps);
+  // Quotients by a shared reciprocal, a few operations each where a division takes eleven, unless a step could under- or overflow (no
+  // quotient is above sqrt(cols)).  The division stands in a loop, not unrolled: what a launch runs once it also fetches, and with a second copy of
+  // the code steps of 6 layers were no faster (128 x 1024 374.5 us before, 368.9 so; 64 x 64 words through an encoder of 1024 957 and 951).
+  if(__builtin_expect(__all(least >= kQuotientLeast) && sigma >= kDivisorLeast && sigma <= kDivisorMost, 1)) {
+    const float reciprocal = 1.0f / sigma;
+#pragma unroll
+    for(int j = 0; j < VECS; ++j)
+#pragma unroll
+      for(int e = 0; e < 4; ++e) v[j][e] = shared_quotient(v[j][e], sigma, reciprocal);
+  } else {
+#pragma unroll 1
+    for(int i = 0; i < 4 * VECS; ++i) {   // (the first value is divided and goes to the end)
+      const float q = v[0][0] / sigma;
+#pragma unroll
+      for(int k = 0; k < 4 * VECS - 1; ++k) v[k / 4][k % 4] = v[(k + 1) / 4][(k + 1) % 4];
+      v[VECS - 1][3] = q;
+    }
+  }
   float omax = 0.0f;
 #pragma unroll
   for(int j = 0; j < VECS; ++j) {
     if(j * kWave + lane < cols4) {
-      float r[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
       const float g[4] = {gm[j].x, gm[j].y, gm[j].z, gm[j].w}, b[4] = {bt[j].x, bt[j].y, bt[j].z, bt[j].w};
 #pragma unroll
       for(int e = 0; e < 4; ++e) {
-        float o = g[e] * ((r[e] - mean) / sigma);
+        float o = g[e] * v[j][e];
         if(has_beta) o = o + b[e];
-        r[e] = o;
+        v[j][e] = o;
         omax = fmaxf(omax, fabsf(o));
       }
-      v[j] = v4f{r[0], r[1], r[2], r[3]};
     }
   }
   return omax;
