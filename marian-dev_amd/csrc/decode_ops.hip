@@ -293,7 +293,7 @@ __global__ __launch_bounds__(THREADS < 256 ? 256 : THREADS) void softmax_kernel(
 // runs between the two reductions, when the THREADS / 64 wave maxima are in red[0 ...]; they stay
 // there.
 struct NoAfterMax {
-  __device__ void operator()(float, const float*) const {}
+  __device__ void operator()(float, const float*, float) const {}
 };
 template <bool LOG, int THREADS, int VPT, typename AfterMax = NoAfterMax>
 __device__ __forceinline__ float softmax_wide_row(const v4f* x, const v4f* mk, int cols4, v4f (&v)[VPT], float* red,
@@ -317,13 +317,14 @@ __device__ __forceinline__ float softmax_wide_row(const v4f* x, const v4f* mk, i
   for(int j = 0; j < VPT; ++j) {
     const int i = j * THREADS + t;
     if(i < cols4) {
-      const float a = v[j].x > v[j].y ? v[j].x : v[j].y, b = v[j].z > v[j].w ? v[j].z : v[j].w;
-      const float c = a > b ? a : b;
-      mx = c > mx ? c : mx;
+      // (one instruction for two values; a NaN, which it lets through, makes all results NaN by way of the sum as well)
+      mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, v[j].x), v[j].y);
+      mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, v[j].z), v[j].w);
     }
   }
+  const float own = mx;
   mx = row_reduce_fresh<THREADS, true>(mx, red);
-  after_max(mx, red);
+  after_max(mx, red, own);
   float sum = 0.0f;
 #pragma unroll
   for(int j = 0; j < VPT; ++j) {
@@ -1523,7 +1524,7 @@ __device__ __forceinline__ bool nbest_before(float v, unsigned i, float w, unsig
 }
 
 struct NbestShared {
-  float val[16];
+  alignas(16) float val[16];
   unsigned idx[16];
   int who[16];
   int winner;
@@ -1633,47 +1634,37 @@ __device__ __forceinline__ void nbest_wave_draw(const float* lv, const unsigned*
 // called once for r = 0 .. N-1 (best first) by one thread each; index is the position within x.
 // scan(f) calls f(value, index) for every element this thread owns (each element of the row is
 // owned by exactly one thread of the workgroup; the order does not matter).
-// The N-th largest of 16 values in LDS (equal values in index order), the same in every thread:
-// lane l % 16 ranks value l % 16, the one of rank N - 1 is it (the cost does not grow with N).
+// The N-th largest of 16 values in LDS (equal values in index order), the same in every thread: the four lanes l % 16 = c of a wave
+// compare value c with four of them each, the lane whose rank is N - 1 has it (the cost does not grow with N; every wave of a
+// workgroup of sixteen does this, and a lane to all sixteen comparisons took 1200 clocks of the launch more).
 __device__ __forceinline__ float nth_largest_of_16(const float* w16, int N) {
-  const int c = threadIdx.x % 16;
+  const int c = threadIdx.x % 16, row = threadIdx.x % 64 / 16;
   const float cvv = w16[c];
-  int rank = 0;
+  const v4f four = reinterpret_cast<const v4f*>(w16)[row];
+  unsigned rank = 0;
 #pragma unroll
-  for(int w = 0; w < 16; ++w) rank += (w16[w] > cvv || (w16[w] == cvv && w < c)) ? 1 : 0;
-  const unsigned long long holders = __ballot(rank == N - 1) & 0xFFFFull;
-  return __shfl(cvv, __ffsll((long long)holders) - 1, 64);   // (ranks 0..15 are all taken: one holder)
+  for(int w = 0; w < 4; ++w) rank += (four[w] > cvv || (four[w] == cvv && 4 * row + w < c)) ? 1u : 0u;
+  v2u_rows s = __builtin_amdgcn_permlane16_swap(rank, rank, false, false);   // (the sum over the four rows of sixteen lanes)
+  s = __builtin_amdgcn_permlane32_swap(s.x + s.y, s.x + s.y, false, false);
+  rank = s.x + s.y;
+  const unsigned long long holders = __ballot(rank == (unsigned)(N - 1)) & 0xFFFFull;
+  const int holder = holders ? __builtin_ctzll(holders) : 0;   // (ranks 0 .. 15 are all taken, but for NaN among the values)
+  return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(cvv), holder));
 }
 
-// Steps 2 and 3: tv is a bound that at least N elements of the row reach (or -inf).
-// count_is_zero: sh.count has been zero since a workgroup barrier that every thread has passed.
+// Step 3, all threads: the N best of what has been collected, or of all that scan goes over where that was too much.
 template <int KEEP, typename Scan, typename Emit>
-__device__ __forceinline__ void nbest_from_bound(Scan scan, int N, NbestShared& sh, Emit emit, float tv,
-                                                 bool count_is_zero) {
+__device__ __forceinline__ void nbest_of_collected(Scan scan, int N, NbestShared& sh, Emit emit) {
   const int tid = threadIdx.x;
   const float ninf = -__builtin_inff();
   const unsigned none = 0xFFFFFFFFu;
-
-  // 2. collect what is >= the bound
-  if(!count_is_zero) {
-    if(tid == 0) sh.count = 0;
-    __syncthreads();
-  }
-  scan([&](float v, unsigned i) {
-    if(v >= tv) {
-      const int slot = atomicAdd(&sh.count, 1);
-      if(slot < 1024) {
-        sh.cand_val[slot] = v; sh.cand_idx[slot] = i;
-      }
-    }
-  });
   __syncthreads();
   const int count = sh.count;
 
-  if(count <= 1024) {
+  if(__builtin_expect(count <= 1024, 1)) {   // (the draws stand here, what follows them behind: a launch fetches its code)
     // 3. the N best of the collected elements, drawn by wave 0: up to 64, one per lane; more,
     //    sixteen per lane
-    if(count <= 64) {
+    if(__builtin_expect(count <= 64, 1)) {
       if(tid < 64) {   // (no candidates - a row of NaN -: lane 0 emits fillers)
         const int e = max(min(tid, count - 1), 0);
         nbest_small_draw(sh.cand_val[e], sh.cand_idx[e], count, N, emit);
@@ -1730,6 +1721,23 @@ __device__ __forceinline__ void nbest_from_bound(Scan scan, int N, NbestShared& 
   }
 }
 
+// Steps 2 and 3: tv is a bound that at least N elements of the row reach (or -inf).
+template <int KEEP, typename Scan, typename Emit>
+__device__ __forceinline__ void nbest_from_bound(Scan scan, int N, NbestShared& sh, Emit emit, float tv) {
+  // 2. collect what is >= the bound
+  if(threadIdx.x == 0) sh.count = 0;
+  __syncthreads();
+  scan([&](float v, unsigned i) {
+    if(v >= tv) {
+      const int slot = atomicAdd(&sh.count, 1);
+      if(slot < 1024) {
+        sh.cand_val[slot] = v; sh.cand_idx[slot] = i;
+      }
+    }
+  });
+  nbest_of_collected<KEEP>(scan, N, sh, emit);
+}
+
 template <int KEEP, typename Scan, typename Emit>
 __device__ __forceinline__ void nbest_core(Scan scan, int N, NbestShared& sh, Emit emit) {
   const int tid = threadIdx.x;
@@ -1744,7 +1752,7 @@ __device__ __forceinline__ void nbest_core(Scan scan, int N, NbestShared& sh, Em
   if(tid % 64 == 0) sh.val[tid / 64] = wv;
   __syncthreads();
   const float tv = nth_largest_of_16(sh.val, N);
-  nbest_from_bound<KEEP>(scan, N, sh, emit, tv, false);
+  nbest_from_bound<KEEP>(scan, N, sh, emit, tv);
 }
 
 // The row in memory.  (Every scan keeps eight 16-byte loads in flight per thread; the last round
@@ -2025,7 +2033,7 @@ __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __r
                                                                 unsigned* __restrict__ outKeys) {
   __shared__ NbestShared sh;
   __shared__ int is_last;
-  __shared__ float red[32];
+  __shared__ __attribute__((aligned(16))) float red[32];
   const int k = blockIdx.x, t = threadIdx.x;
   const long long b = blockIdx.y;
   const size_t row = (size_t)k * dimBatch + b;
@@ -2035,20 +2043,21 @@ __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __r
   // The selection's bound comes out of the softmax's own maximum: the N-th largest of the 16 wave
   // maxima of the logits (at least N logits reach it), taken through the same operations as every
   // element below, which are monotonic, so at least N scores reach the result.
-  float bound_logit = -__builtin_inff(), row_max = 0.0f;
+  float bound_logit = -__builtin_inff(), row_max = 0.0f, own_max = 0.0f;
   const float log_sum = softmax_wide_row<true, 1024, VPT>(
-      reinterpret_cast<const v4f*>(in + row * vocab), nullptr, cols4, v, red, [&](float mx, const float* wave_max) {
+      reinterpret_cast<const v4f*>(in + row * vocab), nullptr, cols4, v, red, [&](float mx, const float* wave_max, float own) {
         row_max = mx;
+        own_max = own;
         bound_logit = nth_largest_of_16(wave_max, N);
       });
-  const float add = rowAdd ? rowAdd[row] : 0.0f;
-  float tv = (bound_logit - row_max) - log_sum;
-  if(rowAdd) tv = tv + add;
+  const float add = rowAdd ? rowAdd[row] : -0.0f;   // (the number that changes none)
+  auto score = [&](float x) __attribute__((always_inline)) { return (x - log_sum) + add; };
+  const float tv = score(bound_logit - row_max);
+  if(lpOut) {
 #pragma unroll
-  for(int j = 0; j < VPT; ++j) {
-    v[j] = v4f{v[j].x - log_sum, v[j].y - log_sum, v[j].z - log_sum, v[j].w - log_sum};
-    if(lpOut && j * 1024 + t < cols4) reinterpret_cast<v4f*>(lpOut + row * vocab)[j * 1024 + t] = v[j];
-    if(rowAdd) v[j] = v4f{v[j].x + add, v[j].y + add, v[j].z + add, v[j].w + add};
+    for(int j = 0; j < VPT; ++j)
+      if(j * 1024 + t < cols4)
+        reinterpret_cast<v4f*>(lpOut + row * vocab)[j * 1024 + t] = v4f{v[j].x - log_sum, v[j].y - log_sum, v[j].z - log_sum, v[j].w - log_sum};
   }
   auto scan = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
@@ -2056,17 +2065,48 @@ __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __r
       const int i4 = j * 1024 + t;
       if(i4 < cols4) {
         const unsigned e = 4u * (unsigned)i4;
-        f(v[j].x, e); f(v[j].y, e + 1); f(v[j].z, e + 2); f(v[j].w, e + 3);
+        f(score(v[j].x), e); f(score(v[j].y), e + 1); f(score(v[j].z), e + 2); f(score(v[j].w), e + 3);
       }
     }
   };
+  // What reaches the bound lies in few threads, those whose largest score does (of N waves, but for equal scores).  Such a thread's values
+  // take a turn through LDS to a lane each of its wave, which appends those that reach it; more than can be collected are of no use.
+  // (An append in place, for each of a thread's values, with a branch around it: 3000 clocks of a launch of 6 rows of 32000 values, 14 600 in all; now 1600
+  // of 12 400.  128 rows 19 200 and 16 700, 65 rows 17 700 and 15 600, with what is rarely run moved behind the rest.)
+  __shared__ __attribute__((aligned(16))) float turn[16][4 * VPT];
+  static_assert(4 * VPT <= 64, "a lane for each of a thread's values");
+  for(unsigned long long todo = __ballot(score(own_max - row_max) >= tv); todo; todo &= todo - 1) {   // (whole waves)
+    const int from = __builtin_ctzll(todo), lane = t % 64, i = min(lane, 4 * VPT - 1);
+    if(lane == from) {
+#pragma unroll
+      for(int j = 0; j < VPT; ++j) reinterpret_cast<v4f*>(turn[t / 64])[j] = v[j];
+    }
+    // (a wave's LDS operations keep their order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float sv = score(turn[t / 64][i]);
+    const int i4 = i / 4 * 1024 + t - lane + from;
+    const unsigned long long reached = __ballot(lane == i && i4 < cols4 && sv >= tv);
+    int slot = 0;
+    if(lane == 0) slot = atomicAdd(&sh.count, (int)__popcll(reached));
+    slot = __builtin_amdgcn_readfirstlane(slot);
+    if(slot > 1024) break;
+    if(reached >> lane & 1) {
+      slot += (int)__builtin_amdgcn_mbcnt_hi((unsigned)(reached >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)reached, 0u));
+      if(slot < 1024) {
+        sh.cand_val[slot] = sv; sh.cand_idx[slot] = 4u * (unsigned)i4 + (unsigned)i % 4u;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
   float* cv = candVal + ((size_t)b * parts + k) * N;
   unsigned* ci = candIdx + ((size_t)b * parts + k) * N;
   const unsigned base = (unsigned)k * (unsigned)vocab;
-  nbest_from_bound<KEEP>(scan, N, sh, [&](int r, float val, unsigned i) {
+  nbest_of_collected<KEEP>(scan, N, sh, [&](int r, float val, unsigned i) {
     __hip_atomic_store(cv + r, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(ci + r, base + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }, tv, true);
+  });
   nbest_hand_over<FENCED>(sh, &is_last, b, parts, N, (long long)parts * vocab, candVal, candIdx, counters, outScores, outKeys);
 }
 
