@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
   // ---- everything this workgroup will need is requested now, in the order of its use (a wave's
   //      loads complete in the order of their issue): abs-max slots, the input rows, weights, the
   //      mask value, the quantization multipliers of the weights, bias ----
-  float pm[NORM ? 1 : kAbsmaxSlots / kProjThreads];
+  [[maybe_unused]] PartialMaxima<kProjThreads> pm;
   // a quad of lanes takes four consecutive 16-value groups of one row: 64 contiguous bytes per load
   const int grp = (tid / 4) * 4, qlane = tid % 4;
   const int r_in = grp / (2 * S), c16 = grp % (2 * S);
@@ -1234,8 +1234,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     nr.load(p.A, aux, p.norm, M, K);
     __builtin_amdgcn_sched_barrier(0);
   } else {
-#pragma unroll
-    for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) pm[i] = p.partials[min(tid + i * kProjThreads, p.n_partials - 1)];
+    pm.load(p.partials, p.n_partials);
     const int m = min(row_of(min(r_in, R - 1)), M - 1);
     const float* src = p.A + (size_t)m * (size_t)K + (size_t)c16 * 16 + qlane * 4;
 #pragma unroll
@@ -1337,8 +1336,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
   if constexpr(NORM) {
     amax = nr.normalize(p.norm, K);
   } else {
-#pragma unroll
-    for(int i = 0; i < kAbsmaxSlots / kProjThreads; ++i) amax = fmaxf(amax, pm[i]);
+    amax = pm.max();
   }
   amax = block_max<kProjThreads / 64>(amax, red);
   if constexpr(STAGED && NORM) load_stage();

@@ -71,6 +71,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
   constexpr int CHUNK = rows_chunk_bytes<ROWS>(), LOADS = ROWS / 4;   // of four rows a load
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
   __shared__ float red[kRowsWaves + 1];
+  __shared__ __attribute__((aligned(16))) float bias_lds[32];
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int li = lane % 32, lg = lane / 32;
@@ -83,20 +84,10 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
   // The order of the loads: see gemm_stream32_kernel (ids first, then what is needed first, all unconditional).
   const int n0 = bx * 32;
   int wsrc = stream32_lane_column(n0, li, args.n_out);
-  const int bias_n = min(n0 + 4 * (lane % 8), args.n_out - 4);   // n_out % 8 == 0: four valid columns
-  uint32_t bias_at[4];
-#pragma unroll
-  for(int e = 0; e < 4; ++e) bias_at[e] = (uint32_t)(bias_n + e);
-  if(flags & 1) {   // through a shortlist
-    if(args.bias) {
-#pragma unroll
-      for(int e = 0; e < 4; ++e) bias_at[e] = args.idx[bias_at[e]];
-    }
-    wsrc = (int)args.idx[wsrc];
-  }
+  if(flags & 1) wsrc = (int)args.idx[wsrc];   // through a shortlist
   asm volatile("" : "+v"(wsrc));
   const float bqm = tail_quant_mult(args.Bq, (size_t)K * (size_t)args.N);
-  float pm[kAbsmaxSlots / kRowsThreads];
+  [[maybe_unused]] PartialMaxima<kRowsThreads> pm;
   v4f share[kRowsShareVecs];
   const int block = tile.by * args.blocks_x + tile.bx, blocks = args.blocks_x * args.blocks_y;
   if constexpr(EXCHANGE) {
@@ -104,8 +95,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
 #pragma unroll
     for(int i = 0; i < kRowsShareVecs; ++i) share[i] = reinterpret_cast<const v4f*>(A)[rows_share_vec(block, each, i, tid, kRowsThreads, n4)];
   } else {
-#pragma unroll
-    for(int i = 0; i < kAbsmaxSlots / kRowsThreads; ++i) pm[i] = partials[min(tid + i * kRowsThreads, n_partials - 1)];
+    pm.load(partials, n_partials);
   }
 
   // lane: value group v (four values) of row 4 j + lane / 16 of load j
@@ -122,7 +112,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
   int8_t* const mine = lds + wave * 4 * CHUNK;
   int8_t* const put = mine + (v / 4) * CHUNK + (lane / 16) * 16 + (v % 4) * 4;
   const int8_t* const get = mine + lg * CHUNK + (li % ROWS) * 16;   // (rows past ROWS: others again, their outputs are not stored)
-  float bias_s[4], unquant = 0.0f;
+  float bias_v = 0.0f, unquant = 0.0f;   // (bias_v: of the column that this lane loads)
   v16i_s acc;
   // The whole of a wave's share of K, for T steps: straight-line code, because a load behind a branch would be waited for at
   // once.  WRITE_AQ: the quantized activations leave as well (rows past M: the last one again, to the same place).
@@ -142,8 +132,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for(int d = 0; d < D; ++d) load(d, d);
-#pragma unroll
-    for(int e = 0; e < 4; ++e) bias_s[e] = bias_src[bias_at[e]];
+    bias_v = bias_src[wsrc];
     __builtin_amdgcn_sched_barrier(0);
     float amax = 0.0f;
     if constexpr(EXCHANGE) {
@@ -154,9 +143,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
         amax = onepass_exchange(block, amax, absmax.nonce, 0u, absmax.words, nullptr, absmax.polls, blocks, &red[kRowsWaves],
                                 [&] { return onepass_scan<kRowsThreads>(A, (size_t)M * K / 4, red); });
     } else {
-#pragma unroll
-      for(int i = 0; i < kAbsmaxSlots / kRowsThreads; ++i) amax = fmaxf(amax, pm[i]);
-      amax = block_max<kRowsWaves>(amax, red);
+      amax = block_max<kRowsWaves>(pm.max(), red);
     }
     const float aqm = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(quant_mult_from_maxabs(amax))));
     unquant = unquant_mult(aqm, bqm, args.scale);
@@ -204,6 +191,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
   // ---- partial sums: every wave drops its ROWS x 32 NT tile into LDS (row-major, the 16-byte pieces of a row permuted by
   //      the row number) and finishes an eighth of the rows, as in gemm_stream32_kernel ----
   constexpr int kTileBytes = ROWS * 128;
+  if(tid < 32) bias_lds[tid] = bias_v;
   __syncthreads();   // (the tiles lie over the staging of other waves)
   if(li < ROWS) {
 #pragma unroll
@@ -219,11 +207,12 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     v4i sum = *reinterpret_cast<const v4i*>(src);
 #pragma unroll
     for(int k = 1; k < kRowsWaves; ++k) sum += *reinterpret_cast<const v4i*>(src + k * kTileBytes);
+    const v4f bias4 = reinterpret_cast<const v4f*>(bias_lds)[lane % 8];
     float y[4];
 #pragma unroll
     for(int e = 0; e < 4; ++e) {   // y = float(acc) * unquant (+ bias); relu: y > 0 ? y : 0; multiply and add round separately
       y[e] = (float)sum[e] * unquant;
-      if(args.bias) y[e] = y[e] + bias_s[e];
+      if(args.bias) y[e] = y[e] + bias4[e];
       if(args.relu) y[e] = y[e] > 0.0f ? y[e] : 0.0f;
       omax = fmaxf(omax, fabsf(y[e]));
     }

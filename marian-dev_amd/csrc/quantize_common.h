@@ -102,6 +102,33 @@ __device__ __forceinline__ float block_max(float m, float* red) {
   return row16_max(r);
 }
 
+// The abs-max partials a launch starts from, n of them, 1 .. kAbsmaxSlots: up to four a load (a load takes the CU's address unit
+// sixteen clocks whatever its width, and four of them a wave were a third of what a call of few rows asks for).
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+template <int THREADS>
+struct PartialMaxima {
+  static_assert(kAbsmaxSlots % (4 * THREADS) == 0, "whole vectors a thread");
+  static constexpr int kVecs = kAbsmaxSlots / (4 * THREADS);
+  v4f v[kVecs];
+  __device__ __forceinline__ void load(const float* partials, int n) {
+    if(__builtin_expect(n % 4 == 0, 1)) {
+#pragma unroll
+      for(int i = 0; i < kVecs; ++i) v[i] = *reinterpret_cast<const v4f_any*>(partials + 4 * min((int)threadIdx.x + i * THREADS, n / 4 - 1));
+    } else {
+#pragma unroll
+      for(int i = 0; i < kVecs; ++i)
+#pragma unroll
+        for(int e = 0; e < 4; ++e) v[i][e] = partials[min(4 * ((int)threadIdx.x + i * THREADS) + e, n - 1)];
+    }
+  }
+  __device__ __forceinline__ float max() const {   // (of this thread's, at least 0)
+    float m = 0.0f;
+#pragma unroll
+    for(int i = 0; i < kVecs; ++i) m = fmaxf(fmaxf(fmaxf(m, v[i].x), fmaxf(v[i].y, v[i].z)), v[i].w);
+    return m;
+  }
+};
+
 // quantMult = 127.0f / maxabs as one correctly rounded fp32 division (via double).
 __device__ __forceinline__ float quant_mult_from_maxabs(float maxabs) {
   return (float)(127.0 / (double)maxabs);
