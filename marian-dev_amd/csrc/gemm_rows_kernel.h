@@ -116,6 +116,11 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
   v16i_s acc;
   // The whole of a wave's share of K, for T steps: straight-line code, because a load behind a branch would be waited for at
   // once.  WRITE_AQ: the quantized activations leave as well (rows past M: the last one again, to the same place).
+  constexpr bool EARLY = STEPS > 2;   // of the abs-max that is in slots
+  auto exchange_of = [&]() __attribute__((always_inline)) {
+    if constexpr(EXCHANGE) return OnepassExchange(block, absmax.nonce, 0u, absmax.words, blocks);
+    else return 0;
+  };
   auto run = [&](auto steps_tag, auto write_tag) __attribute__((always_inline)) {
     constexpr int T = decltype(steps_tag)::value, D = T < rows_depth(ROWS) ? T : rows_depth(ROWS);
     constexpr bool WRITE_AQ = decltype(write_tag)::value;
@@ -130,19 +135,30 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
       __builtin_amdgcn_sched_barrier(0);
     };
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for(int d = 0; d < D; ++d) load(d, d);
-    bias_v = bias_src[wsrc];
-    __builtin_amdgcn_sched_barrier(0);
+    // The abs-max comes between the first pair's loads and the others': a wave goes on only when its loads have been accepted, and those of the later
+    // four waves stand behind all of the earlier ones', 3000 clocks of a launch of 14 000 before anyone knew it or sent its share of it.  All loads
+    // first: 64 x 512 x 2048 and back 10.19 us, now 9.78, 256 x 1024 x 1000 of a shortlist with its four best words 11.03 and 10.13, a step of 65 x 512
+    // 299.9 and 298.9; none first: 9.90 and 10.21.  (Two pairs and fewer are all on their way together.)
     float amax = 0.0f;
+    [[maybe_unused]] const auto exchange = exchange_of();
+    if(D > 0) load(0, 0);
     if constexpr(EXCHANGE) {
 #pragma unroll
       for(int i = 0; i < kRowsShareVecs; ++i) amax = abs4max(share[i], amax);
       amax = block_max<kRowsWaves>(amax, red);
+      if(blocks > 1) exchange.publish(amax);
+    } else if constexpr(EARLY) {
+      amax = block_max<kRowsWaves>(pm.max(), red);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for(int d = 1; d < D; ++d) load(d, d);
+    bias_v = bias_src[wsrc];
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr(EXCHANGE) {
       if(blocks > 1)
-        amax = onepass_exchange(block, amax, absmax.nonce, 0u, absmax.words, nullptr, absmax.polls, blocks, &red[kRowsWaves],
-                                [&] { return onepass_scan<kRowsThreads>(A, (size_t)M * K / 4, red); });
-    } else {
+        amax = exchange.collect(amax, 0u, nullptr, absmax.polls, &red[kRowsWaves], [&] { return onepass_scan<kRowsThreads>(A, (size_t)M * K / 4, red); });
+    } else if constexpr(!EARLY) {
       amax = block_max<kRowsWaves>(pm.max(), red);
     }
     const float aqm = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(quant_mult_from_maxabs(amax))));

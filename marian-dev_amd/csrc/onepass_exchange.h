@@ -28,51 +28,70 @@ namespace marian_hip {
 __device__ __forceinline__ unsigned long long onepass_word(unsigned tag, float v) {
   return ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v);
 }
-// g: this workgroup of G <= 256, m: the abs-max of its values (in every thread), nonce: this launch's; gen: the generation
-// word as it was (0 without one).  scan: the abs-max of the whole input, by this workgroup alone.
+// In two parts, between which a workgroup may ask for what it needs next.  g: this workgroup of G <= 256, m: the abs-max of its values (in
+// every thread), nonce: this launch's; gen: the generation word as it was (0 without one).
+struct OnepassExchange {
+  unsigned long long* words;
+  unsigned tag;
+  int g, G;
+  __device__ __forceinline__ OnepassExchange(int g, unsigned nonce, unsigned gen, unsigned long long* words, int G)
+      : words(words), tag((nonce + gen) | 0x80000000u), g(g), G(G) {}   // (the tag is never 0: a cleared word does not match)
+  __device__ __forceinline__ int shift() const { return G > 16 ? 28 - __builtin_clz(G - 1) : 0; }   // 1 << shift lines of 16 words: the fewest that hold G
+  __device__ __forceinline__ unsigned long long* place() const {   // (lanes below kOnePassCopies)
+    return words + ((int)threadIdx.x % kOnePassCopies) * kOnePassMaxGroups + ((g & ((1 << shift()) - 1)) * 16 + (g >> shift()));
+  }
+  __device__ __forceinline__ void publish(float m) const {
+    if(threadIdx.x < kOnePassCopies) __hip_atomic_store(place(), onepass_word(tag, m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // scan: the abs-max of the whole input, by this workgroup alone.
+  template <class Scan>
+  __device__ __forceinline__ float collect(float m, unsigned gen, unsigned long long* gen_word, int polls, float* shared_max, Scan scan) const {
+    const int tid = threadIdx.x;
+    static_assert(kOnePassMaxGroups == 4 * kWave, "four words a lane");
+    int polls_left = polls;   // (of the whole workgroup: only its first wave waits)
+    if(tid < kWave) {
+      const unsigned long long own = onepass_word(tag, m);
+      const int lines = shift();
+      const unsigned long long* const get = words + (g % kOnePassCopies) * kOnePassMaxGroups;
+      auto word = [&](int i) __attribute__((always_inline)) {
+        const int at = i * kWave + tid, from = (at % 16 << lines) + at / 16;   // (lanes past the words: one of theirs again)
+        return i * kWave < 16 << lines ? __hip_atomic_load(get + (from < G && at < 16 << lines ? at : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : own;
+      };
+      auto tag_of = [](unsigned long long w) { return (unsigned)(w >> 32); };
+      auto value_of = [](unsigned long long w) { return __uint_as_float((unsigned)w); };
+      float v = 0.0f;
+      bool found = false;
+      for(; onepass_patience(polls_left); onepass_polled(polls_left)) {
+        const unsigned long long w0 = word(0), w1 = word(1), w2 = word(2), w3 = word(3);
+        v = fmaxf(fmaxf(value_of(w0), value_of(w1)), fmaxf(value_of(w2), value_of(w3)));
+        found = __all(tag_of(w0) == tag && tag_of(w1) == tag && tag_of(w2) == tag && tag_of(w3) == tag);
+        if(found) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      v = wave_max(v);
+      if(gen_word) {
+        // Words that went out behind the generation's end carry the next replay's tag.  Their workgroup never finds those of
+        // workgroup 0, which ended before it read the generation, so it comes here without an answer and takes them back.
+        if(!found && tid < kOnePassCopies) __hip_atomic_store(place(), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the next replay expects another tag; every workgroup of this one has read the generation by now, or will find its
+        // words unanswered and help itself
+        if(g == 0 && tid == 0) __hip_atomic_store(gen_word, (unsigned long long)(gen + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if(tid == 0) *shared_max = found ? v : -1.0f;
+    }
+    __syncthreads();
+    const float all = *shared_max;
+    return all >= 0.0f ? all : scan();
+  }
+};
+// Both, with the pause between them.
 template <class Scan>
 __device__ __forceinline__ float onepass_exchange(int g, float m, unsigned nonce, unsigned gen, unsigned long long* words,
                                                   unsigned long long* gen_word, int polls, int G, float* shared_max, Scan scan) {
-  const int tid = threadIdx.x;
-  static_assert(kOnePassMaxGroups == 4 * kWave, "four words a lane");
-  int polls_left = polls;   // (of the whole workgroup: only its first wave waits)
-  if(tid < kWave) {
-    const unsigned tag = (nonce + gen) | 0x80000000u;   // never 0: a cleared word does not match
-    const unsigned long long own = onepass_word(tag, m);
-    const int shift = G > 16 ? 28 - __builtin_clz(G - 1) : 0;   // 1 << shift lines of 16 words: the fewest that hold G
-    unsigned long long* const put = words + (tid % kOnePassCopies) * kOnePassMaxGroups + ((g & ((1 << shift) - 1)) * 16 + (g >> shift));
-    const unsigned long long* const get = words + (g % kOnePassCopies) * kOnePassMaxGroups;
-    if(tid < kOnePassCopies) __hip_atomic_store(put, own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    auto word = [&](int i) __attribute__((always_inline)) {
-      const int at = i * kWave + tid, from = (at % 16 << shift) + at / 16;   // (lanes past the words: one of theirs again)
-      return i * kWave < 16 << shift ? __hip_atomic_load(get + (from < G && at < 16 << shift ? at : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : own;
-    };
-    auto tag_of = [](unsigned long long w) { return (unsigned)(w >> 32); };
-    auto value_of = [](unsigned long long w) { return __uint_as_float((unsigned)w); };
-    float v = 0.0f;
-    bool found = false;
-    __builtin_amdgcn_s_sleep(16);   // (1024 clocks, see above)
-    for(; onepass_patience(polls_left); onepass_polled(polls_left)) {
-      const unsigned long long w0 = word(0), w1 = word(1), w2 = word(2), w3 = word(3);
-      v = fmaxf(fmaxf(value_of(w0), value_of(w1)), fmaxf(value_of(w2), value_of(w3)));
-      found = __all(tag_of(w0) == tag && tag_of(w1) == tag && tag_of(w2) == tag && tag_of(w3) == tag);
-      if(found) break;
-      __builtin_amdgcn_s_sleep(1);
-    }
-    v = wave_max(v);
-    if(gen_word) {
-      // Words that went out behind the generation's end carry the next replay's tag.  Their workgroup never finds those of
-      // workgroup 0, which ended before it read the generation, so it comes here without an answer and takes them back.
-      if(!found && tid < kOnePassCopies) __hip_atomic_store(put, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      // the next replay expects another tag; every workgroup of this one has read the generation by now, or will find its
-      // words unanswered and help itself
-      if(g == 0 && tid == 0) __hip_atomic_store(gen_word, (unsigned long long)(gen + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if(tid == 0) *shared_max = found ? v : -1.0f;
-  }
-  __syncthreads();
-  const float all = *shared_max;
-  return all >= 0.0f ? all : scan();
+  const OnepassExchange exchange(g, nonce, gen, words, G);
+  exchange.publish(m);
+  if(threadIdx.x < kWave) __builtin_amdgcn_s_sleep(16);   // (1024 clocks, see above)
+  return exchange.collect(m, gen, gen_word, polls, shared_max, scan);
 }
 // Abs-max of n4 vectors by one workgroup (the way out of a wait that ran out).
 template <int THREADS>
