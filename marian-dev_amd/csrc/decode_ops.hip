@@ -1243,14 +1243,43 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
   v4i w[NPROJ][PW];
   const unsigned w_off = stream32_lane_offset(h * 64 + wn * 32 + li, lg), w_step = 32u * (unsigned)N;
   // (asked for in the order the multiplication takes them: sub-step by sub-step, all projections; as buffers: no vector arithmetic)
+  auto load_weights = [&](int from, int to) __attribute__((always_inline)) {
 #pragma unroll
-  for(int pp = 0; pp < PW; ++pp) {
-    const unsigned at = (unsigned)stream32_clamped_substep(kw * steps + pp, S) * w_step;
+    for(int pp = from; pp < to; ++pp) {
+      const unsigned at = (unsigned)stream32_clamped_substep(kw * steps + pp, S) * w_step;
 #pragma unroll
-    for(int g = 0; g < NPROJ; ++g) {
-      const auto w_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.Bq[g]), 0, (int)((unsigned)K * (unsigned)N), kRawBuffer);
-      w[g][pp] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w_buf, w_off, at, 0));
+      for(int g = 0; g < NPROJ; ++g) {
+        const auto w_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.Bq[g]), 0, (int)((unsigned)K * (unsigned)N), kRawBuffer);
+        w[g][pp] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w_buf, w_off, at, 0));
+      }
     }
+  };
+  float aqm = 0.0f;
+  constexpr int kFirstSubsteps = NORM ? PW : PW / 2;
+  load_weights(0, kFirstSubsteps);
+  if constexpr(!NORM) {
+    // ---- 1, 2: abs-max, quantize into LDS, behind half of the weights' loads: a wave goes on only when its loads have been accepted, and behind
+    //      all of them that was 5000 - 9000 clocks after the input had come (a step of 65 x 512 298.9 -> 293.2 us; 128 x 1024, which is bound by what a
+    //      CU can fetch, the same with half or a quarter) ----
+    __builtin_amdgcn_sched_barrier(0);
+    aqm = quant_mult_from_maxabs(block_max<kProjThreads / 64>(pm.max(), red));
+    const float by = quantizer(aqm);
+    if(has_in) {
+      uint32_t q[4];
+#pragma unroll
+      for(int e = 0; e < 4; ++e) q[e] = quantize_pack4(in[e], by);
+      const int slot0 = (c16 / 2) * 64, x = r_in ^ proj_row_key(c16);
+      const int m = row_of(min(r_in, R - 1));
+#pragma unroll
+      for(int e = 0; e < 4; ++e) {
+        const int sw = slot0 + (e / 2) * 64 + (e % 2) * 32 + (x ^ e);
+        *reinterpret_cast<uint32_t*>(a_lds + sw * 16 + qlane * 4) = q[e];
+        if(p.aq_out && h == 0 && m < M)
+          *reinterpret_cast<uint32_t*>(p.aq_out + (size_t)m * (size_t)K + (size_t)(c16 + e) * 16 + qlane * 4) = q[e];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load_weights(kFirstSubsteps, PW);
   }
   // keys and values of the workgroup's sentences: sixteen threads per position, 32 positions per pass
   constexpr int kStageSegs = STAGED ? SEGS : 1, kStagePasses = STAGED ? PASSES : 1;
@@ -1331,32 +1360,10 @@ __global__ __launch_bounds__(kProjThreads) void proj_attention_kernel(const floa
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // ---- 1, 2: abs-max, quantize into LDS ----
-  float amax = 0.0f;
-  if constexpr(NORM) {
-    amax = nr.normalize(p.norm, K);
-  } else {
-    amax = pm.max();
-  }
-  amax = block_max<kProjThreads / 64>(amax, red);
-  if constexpr(STAGED && NORM) load_stage();
-  const float aqm = quant_mult_from_maxabs(amax);
-  const float by = quantizer(aqm);
-  if(has_in) {
-    uint32_t q[4];
-#pragma unroll
-    for(int e = 0; e < 4; ++e) q[e] = quantize_pack4(in[e], by);
-    const int slot0 = (c16 / 2) * 64, x = r_in ^ proj_row_key(c16);
-    const int m = row_of(min(r_in, R - 1));
-#pragma unroll
-    for(int e = 0; e < 4; ++e) {
-      const int sw = slot0 + (e / 2) * 64 + (e % 2) * 32 + (x ^ e);
-      *reinterpret_cast<uint32_t*>(a_lds + sw * 16 + qlane * 4) = q[e];
-      if(p.aq_out && h == 0 && m < M)
-        *reinterpret_cast<uint32_t*>(p.aq_out + (size_t)m * (size_t)K + (size_t)(c16 + e) * 16 + qlane * 4) = q[e];
-    }
-  }
-  if constexpr(NORM) {   // wave w holds row w: quantized where this workgroup multiplies it, written out by one workgroup
+  if constexpr(NORM) {   // 1, 2: wave w holds row w, quantized where this workgroup multiplies it, written out by one workgroup
+    const float amax = block_max<kProjThreads / 64>(nr.normalize(p.norm, K), red);
+    if constexpr(STAGED) load_stage();
+    aqm = quant_mult_from_maxabs(amax);
     const int row = wave;
     if(row < M) {
       if(norm_at >= 0) nr.quantize(a_lds, norm_at, K, aqm, proj_row_key);
