@@ -76,6 +76,7 @@ struct Stream32Rest {
   NORMED norm;
 };
 
+struct NoPartials {};
 // Dynamic LDS: one chunk (kStageBytes), for kFusedAll all of K (32 * MT32 * K bytes) if that is
 // more; at least kReduceBytes.  aux: n_partials (1..2048) abs-max values (kFusedTiled), what is added to A (kFusedNorm), the
 // bias (kFusedAll: one address fewer to wait for ahead of the weights; in a graph 4 x 1024 x 2360 3.38 us with it in args and 3.32 now,
@@ -119,6 +120,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
   constexpr bool TILED = MODE == kFusedTiled;
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
   __shared__ float red[kStream32Waves];
+  __shared__ __attribute__((aligned(16))) float bias_lds[kStream32Waves][32];
 
   long long tp[6] = {0, 0, 0, 0, 0, 0}, wall0 = 0;
   if(MH_PROF(args)) {
@@ -143,21 +145,10 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
   // are clamped and the values replaced afterwards), so the activations are waited for with
   // exactly the weight and bias loads still in flight.
 
-  // ---- weight row of this lane and where the bias of the four columns this lane will write
-  //      sits (see the epilogue), both through the shortlist ids when there are any ----
+  // ---- weight row of this lane, through the shortlist ids when there are any; it loads that column's bias too, which the epilogue finds in LDS ----
   const int n0 = (bx * WN + wn) * 32;
   int wsrc = stream32_lane_column(n0, li, args.n_out);
-  const int bias_n = min(n0 + 4 * (lane % 8), args.n_out - 4);   // n_out % 8 == 0: four valid columns
-  uint32_t bias_at[4];
-#pragma unroll
-  for(int e = 0; e < 4; ++e) bias_at[e] = (uint32_t)(bias_n + e);
-  if(shortlist) {
-    if(args.bias) {
-#pragma unroll
-      for(int e = 0; e < 4; ++e) bias_at[e] = args.idx[bias_at[e]];
-    }
-    wsrc = (int)args.idx[wsrc];
-  }
+  if(shortlist) wsrc = (int)args.idx[wsrc];
   // (pins the wait for the ids here, where nothing else is in flight; left to itself the compiler
   // computes the weight address, and waits, after the activation loads)
   asm volatile("" : "+v"(wsrc));
@@ -165,14 +156,8 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
   float aqm_pre = 0.0f;
   if(MODE == kPrequant) aqm_pre = tail_quant_mult(args.Aq, (size_t)M * (size_t)K);
   float amax = 0.0f;
-  if(TILED) {   // a few (clamped) abs-max partials per thread cover all kAbsmaxSlots
-    float pm[kAbsmaxSlots / kStream32Threads];
-#pragma unroll
-    for(int i = 0; i < kAbsmaxSlots / kStream32Threads; ++i)
-      pm[i] = partials[min(tid + i * kStream32Threads, n_partials - 1)];
-#pragma unroll
-    for(int i = 0; i < kAbsmaxSlots / kStream32Threads; ++i) amax = fmaxf(amax, pm[i]);
-  }
+  [[maybe_unused]] typename std::conditional<TILED_, PartialMaxima<TILED_ ? kStream32Threads : 512>, NoPartials>::type pm;
+  if constexpr(TILED_) pm.load(partials, n_partials);
   // this lane's 16 bytes of K sub-step 0; a sub-step further is w_step bytes further for every column
   const int8_t* wrow = args.Bq + stream32_lane_offset(wsrc, lg);
   const size_t w_step = 32u * (size_t)args.N;
@@ -330,16 +315,14 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
   __builtin_amdgcn_sched_barrier(0);
   // (unconditional as well: without a bias the weights stand in - 4 * N readable bytes - and the
   // values are dropped in the epilogue)
-  float bias_s[4];
   const float* bias_src = args.bias ? args.bias : reinterpret_cast<const float*>(args.Bq);
-#pragma unroll
-  for(int e = 0; e < 4; ++e) bias_s[e] = bias_src[bias_at[e]];
+  const float bias_v = bias_src[wsrc];
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- activations into LDS, operand order: slot (sub-step, m-tile, lane) of 16 bytes holds
   //      Aq[mt*32 + lane%32][(s0+step)*32 + (lane/32)*16 .. +15]
-  if(TILED) {
-    amax = block_max<kStream32Waves>(amax, red);
+  if constexpr(TILED_) {
+    amax = block_max<kStream32Waves>(pm.max(), red);
     aqm = quant_mult_from_maxabs(amax);
     unquant = unquant_mult(aqm, bqm, args.scale);
     by = quantizer(aqm);
@@ -492,6 +475,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
             v4i{acc[mt][4 * q], acc[mt][4 * q + 1], acc[mt][4 * q + 2], acc[mt][4 * q + 3]};
       }
   }
+  if(lane < 32) bias_lds[wave][lane] = bias_v;
   __syncthreads();
 
   if(MH_PROF(args)) tp[4] = MH_CLOCK();
@@ -501,11 +485,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
     const bool has_bias = args.bias != nullptr;
     const int n = n0 + 4 * (lane % 8);
     const int8_t* tiles = lds + (size_t)(wn * KW) * kTileBytes;
-    // Use the bias values once ahead of the stores, so that the compiler waits for their loads here
-    // (they arrived long ago).  Otherwise it waits inside the loop, behind the branches, for all
-    // vector memory operations before each use - and every store then waits for the one before.
-#pragma unroll
-    for(int e = 0; e < 4; ++e) asm volatile("" ::"v"(bias_s[e]));
+    const v4f bias4 = reinterpret_cast<const v4f*>(bias_lds[wave])[lane % 8];
 #pragma unroll
     for(int it = 0; it < (kPieces + 63) / 64; ++it) {
       const int pc = it * 64 + lane;
@@ -527,7 +507,7 @@ __global__ __launch_bounds__(WN * KW * kWave) void gemm_stream32_kernel(const fl
 #pragma unroll
       for(int e = 0; e < 4; ++e) {
         y[e] = (float)sum[e] * unquant;
-        if(has_bias) y[e] = y[e] + bias_s[e];
+        if(has_bias) y[e] = y[e] + bias4[e];
         if(args.relu) y[e] = y[e] > 0.0f ? y[e] : 0.0f;
         omax = fmaxf(omax, fabsf(y[e]));
       }
