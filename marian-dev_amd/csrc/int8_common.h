@@ -10,6 +10,7 @@ namespace marian_hip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));   // (where only its elements are aligned)
 
 constexpr int kWave = 64;        // CDNA wavefront
 constexpr int kRawBuffer = 0x00020000;   // a buffer descriptor's last word: 32-bit data, no swizzle

@@ -104,7 +104,6 @@ __device__ __forceinline__ float block_max(float m, float* red) {
 
 // The abs-max partials a launch starts from, n of them, 1 .. kAbsmaxSlots: up to four a load (a load takes the CU's address unit
 // sixteen clocks whatever its width, and four of them a wave were a third of what a call of few rows asks for).
-typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 template <int THREADS>
 struct PartialMaxima {
   static_assert(kAbsmaxSlots % (4 * THREADS) == 0, "whole vectors a thread");
