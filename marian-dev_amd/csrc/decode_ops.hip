@@ -829,6 +829,8 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
 // and the whole 24 100.  In the smaller forms K = 512 asks for the sub-steps it has (PW: eight with repeats before), and rows are worked
 // out without a division (the launch has a dimension for sentence groups and one for hypothesis chunks): 6 rows x 8 heads over 12
 // positions 19 800 -> 15 600 clocks, their context over 23 positions 18 100 -> 14 100; 65 rows over 34 positions 19 300 -> 17 900.
+// Then (attention_row64_short, the input quantized behind half of the weights' loads, requests and code that are not needed left out) launches of 6 rows
+// 8.9 -> 7.6 us and 8.1 -> 6.2 (context), of 65 rows over 34 positions 10.5 -> 8.9 and over 47 of the source 7.6 -> 6.3, of 128 rows 13.4 -> 12.4 and 11.5 -> 9.6.
 // Tried and dropped: barriers that put every wave's small requests in front of any wave's large ones; the
 // workgroups of a head starting at different sub-steps of K, so that they would not all miss L2 on
 // the same lines of the weights at the same time (+5 us per step).
