@@ -12,6 +12,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));   // (where only its elements are aligned)
 
+typedef unsigned v4u_raw __attribute__((ext_vector_type(4)));
+
 constexpr int kWave = 64;        // CDNA wavefront
 constexpr int kRawBuffer = 0x00020000;   // a buffer descriptor's last word: 32-bit data, no swizzle
 constexpr int kFragBytes = 1024; // one MFMA 16x16x64 i8 operand: 64 lanes x 16 bytes

@@ -110,19 +110,21 @@ struct NormRow {
   v4f v[VECS], t[VECS], gm[VECS], bt[VECS];
   // Wave w loads row w (rows past M: a copy of the last one).  All loads unconditional, so that waits count them exactly.
   __device__ __forceinline__ void load(const float* A, const float* add, const NormInput& n, int M, int K) {
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, cols4 = K / 4;
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const size_t row = (size_t)min(wave, M - 1) * K;
+    auto load_buffer = [&](const float* p, int j) __attribute__((always_inline)) {   // (past the row: zeros)
+      return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, K * 4, kRawBuffer), lane * 16 + j * 1024, 0, 0));
+    };
 #pragma unroll
     for(int j = 0; j < VECS; ++j) {
-      const int i = min(j * kWave + lane, cols4 - 1);
-      v[j] = reinterpret_cast<const v4f*>(A + row)[i];
-      t[j] = reinterpret_cast<const v4f*>(add + row)[i];
+      v[j] = load_buffer(A + row, j);
+      t[j] = load_buffer(add + row, j);
     }
 #pragma unroll
     for(int j = 0; j < VECS; ++j) {
-      const int i = min(j * kWave + lane, cols4 - 1);
-      gm[j] = reinterpret_cast<const v4f*>(n.gamma)[i];
-      bt[j] = reinterpret_cast<const v4f*>(n.beta)[i];
+      gm[j] = load_buffer(n.gamma, j);
+      bt[j] = load_buffer(n.beta, j);
     }
   }
   __device__ __forceinline__ float normalize(const NormInput& n, int K) {

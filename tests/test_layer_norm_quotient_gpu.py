@@ -38,5 +38,10 @@ def test_bits_of_the_division(rows, cols):
                 other = (x == -lost[:, None]).argmax(1)
                 x[np.arange(rows), np.arange(rows) % cols], x[np.arange(rows), other] = f32(0.0), f32(-0.0)
             eps = 1e-6 if exponent > -40 else 1e-30
+            want = expected(x, gamma, beta, eps)
             got = ops.layerNorm(dev(x), dev(gamma), dev(beta), eps=eps)
-            assert np.array_equal(got.cpu().numpy(), expected(x, gamma, beta, eps)), (exponent, zero)
+            assert np.array_equal(got.cpu().numpy(), want), (exponent, zero)
+            # with a skip input (all loads as buffers), in whole numbers as well; nothing is written past the rows
+            part = rng.integers(-15, 16, (rows, cols)).astype(f32) * f32(2.0) ** f32(exponent)
+            got = ops.layerNorm(dev(x - part), dev(gamma), dev(beta), eps=eps, add=dev(part))
+            assert np.array_equal(got.cpu().numpy(), want), (exponent, zero, "skip")
