@@ -1753,12 +1753,9 @@ __device__ __forceinline__ void nbest_of_collected(Scan scan, int N, NbestShared
   }
 }
 
-// Steps 2 and 3: tv is a bound that at least N elements of the row reach (or -inf).
-template <int KEEP, typename Scan, typename Emit>
-__device__ __forceinline__ void nbest_from_bound(Scan scan, int N, NbestShared& sh, Emit emit, float tv) {
-  // 2. collect what is >= the bound
-  if(threadIdx.x == 0) sh.count = 0;
-  __syncthreads();
+// Step 2: what reaches tv, a bound that at least N elements of the row reach (or -inf).  sh.count has been zero since a workgroup barrier.
+template <typename Scan>
+__device__ __forceinline__ void nbest_collect(Scan scan, NbestShared& sh, float tv) {
   scan([&](float v, unsigned i) {
     if(v >= tv) {
       const int slot = atomicAdd(&sh.count, 1);
@@ -1767,6 +1764,14 @@ __device__ __forceinline__ void nbest_from_bound(Scan scan, int N, NbestShared& 
       }
     }
   });
+}
+
+// Steps 2 and 3.
+template <int KEEP, typename Scan, typename Emit>
+__device__ __forceinline__ void nbest_from_bound(Scan scan, int N, NbestShared& sh, Emit emit, float tv) {
+  if(threadIdx.x == 0) sh.count = 0;
+  __syncthreads();
+  nbest_collect(scan, sh, tv);
   nbest_of_collected<KEEP>(scan, N, sh, emit);
 }
 
@@ -2101,14 +2106,19 @@ __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __r
       }
     }
   };
-  // What reaches the bound lies in few threads, those whose largest score does (of N waves, but for equal scores).  Such a thread's values
-  // take a turn through LDS to a lane each of its wave, which appends those that reach it; more than can be collected are of no use.
-  // (An append in place, for each of a thread's values, with a branch around it: 3000 clocks of a launch of 6 rows of 32000 values, 14 600 in all; now 1600
-  // of 12 400.  128 rows 19 200 and 16 700, 65 rows 17 700 and 15 600, with what is rarely run moved behind the rest.)
+  // What reaches the bound lies in few threads, those whose largest score does (of N waves, but for equal scores).  Where it is one of a
+  // wave, its values take a turn through LDS to a lane each, which appends those that reach it; of several, every thread goes through its own.
+  // (Times of recorded launches, N best of so many rows and words: every thread of all waves through its own, a turn for each of a wave's threads, and
+  // so: 128 x 32000, N = 1 8.7, 7.1, 7.1 us; 4 8.7, 7.7, 7.9; 6 8.9, 8.2, 8.2; 12 10.4, 11.1, 9.7; 16 19.3, 23.9, 18.5.  6 x 32000, N = 1 8.2, 6.7, 6.6; 16
+  // 14.9, 17.2, 14.0.  65 x 8000 with every eighth word the best, N = 1 8.7, 37.4, 8.0; 6 13.5, 42.7, 12.7: turns follow one another, 2000 clocks each
+  // where all sixteen waves have some.)
   __shared__ __attribute__((aligned(16))) float turn[16][4 * VPT];
   static_assert(4 * VPT <= 64, "a lane for each of a thread's values");
-  for(unsigned long long todo = __ballot(score(own_max - row_max) >= tv); todo; todo &= todo - 1) {   // (whole waves)
-    const int from = __builtin_ctzll(todo), lane = t % 64, i = min(lane, 4 * VPT - 1);
+  const unsigned long long reaching = __ballot(score(own_max - row_max) >= tv);   // (whole waves)
+  if(__builtin_expect((reaching & (reaching - 1)) != 0, 0)) {
+    nbest_collect(scan, sh, tv);
+  } else if(reaching) {
+    const int from = __builtin_ctzll(reaching), lane = t % 64, i = min(lane, 4 * VPT - 1);
     if(lane == from) {
 #pragma unroll
       for(int j = 0; j < VPT; ++j) reinterpret_cast<v4f*>(turn[t / 64])[j] = v[j];
@@ -2122,15 +2132,10 @@ __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __r
     const unsigned long long reached = __ballot(lane == i && i4 < cols4 && sv >= tv);
     int slot = 0;
     if(lane == 0) slot = atomicAdd(&sh.count, (int)__popcll(reached));
-    slot = __builtin_amdgcn_readfirstlane(slot);
-    if(slot > 1024) break;
-    if(reached >> lane & 1) {
-      slot += (int)__builtin_amdgcn_mbcnt_hi((unsigned)(reached >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)reached, 0u));
-      if(slot < 1024) {
-        sh.cand_val[slot] = sv; sh.cand_idx[slot] = 4u * (unsigned)i4 + (unsigned)i % 4u;
-      }
+    slot = __builtin_amdgcn_readfirstlane(slot) + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(reached >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)reached, 0u));
+    if((reached >> lane & 1) && slot < 1024) {
+      sh.cand_val[slot] = sv; sh.cand_idx[slot] = 4u * (unsigned)i4 + (unsigned)i % 4u;
     }
-    __builtin_amdgcn_wave_barrier();
   }
   float* cv = candVal + ((size_t)b * parts + k) * N;
   unsigned* ci = candIdx + ((size_t)b * parts + k) * N;
