@@ -16,6 +16,7 @@
 
 #include "../../include/marian_hip_int8.h"
 #include "abi_common.h"
+#include "attention_plan.h"
 #include "attention_rows_kernel.h"
 #include "int8_common.h"
 #include "layer_norm_row.h"
@@ -2570,13 +2571,10 @@ int marian_hip_attention_rows(const float* q, const int64_t* q_strides, const fl
   if(groups > row_blocks) groups = row_blocks;
   if(batchQ * groups > kMaxElemsOps / 256) return MARIAN_HIP_ERR_RANGE;
   if(absmax_out && batchQ * groups * 4 > kAbsmaxSlots) return MARIAN_HIP_ERR_RANGE;
-  // A wave to 16 query rows where that deal leaves some CUs two workgroups: 144 heads of 64 x 64 7.7 -> 6.8 us, of 23 x 23 5.2 -> 4.6,
-  // of 80 x 80 13.1 -> 11.2; 128 of 64 x 64 stay at 6.2 (6.7), 64 of 128 x 128 at 8.8 (10.4).  Not where its workgroups have one block
-  // each (80 heads of 64 x 64 5.6, 6.7 us) unless a head has two blocks at the most.
-  if(batchQ * groups > 256 && (groups < row_blocks || row_blocks <= 2) && len <= 128) {
-    const int tiles = len <= 32 ? 2 : len <= 48 ? 3 : len <= 64 ? 4 : len <= 80 ? 5 : len <= 96 ? 6 : 8;
-    const int waves = tiles == 2 ? 2 : tiles % 4 == 0 ? 4 : 3;
-    const int64_t wgs = (row_blocks + waves - 1) / waves;   // of a head
+  const AttentionHeadsPlan plan = attention_heads_plan(batchQ, groups, row_blocks, len);
+  if(plan.workgroups) {   // a wave to 16 query rows
+    const int tiles = plan.tiles, waves = plan.waves;
+    const int64_t wgs = plan.workgroups;   // of a head
     // (its buffers hold a head each, offsets past the last row included, and end behind the last row of 64 values)
     auto fits = [](int64_t row, int64_t positions) { return row <= (1 << 29) / (positions + 128); };
     if(fits(q_strides[2], m) && fits(k_strides[2], len) && fits(v_strides[2], len) && fits(out_strides[2], m) && k_strides[2] >= 64 && v_strides[2] >= 64 &&
