@@ -13,8 +13,8 @@ namespace marian_hip {
 
 // a / s from r = 1.0f / s, s positive: three operations where a division takes eleven.  The residual correction with a correctly rounded
 // reciprocal gives the correctly rounded quotient (P. Markstein, "Computation of elementary functions on the IBM RISC
-// System/6000 processor", 1990), so the bits are the division's (tests/test_shared_quotient.py: the pairs of significands, of odd divisors, whose
-// quotient lies close to a rounding edge).  The callers keep to magnitudes in which no step under- or overflows.  A zero keeps its
+// System/6000 processor", 1990), so the bits are the division's (tests/test_shared_quotient.py, for odd divisors, and
+// tests/test_shared_quotient_even.py: every pair of significands whose quotient lies close to a rounding edge).  The callers keep to magnitudes in which no step under- or overflows.  A zero keeps its
 // sign: what is added to it is the remainder, which is +0, times -r (tests/test_quotients_of_zero.py).
 constexpr float kQuotientLeast = 0x1p-60f, kQuotientMost = 0x1p60f;  // magnitudes of dividends that are not zero
 constexpr float kDivisorLeast = 0x1p-40f, kDivisorMost = 0x1p40f;
