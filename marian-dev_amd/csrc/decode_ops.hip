@@ -2107,35 +2107,38 @@ __global__ __launch_bounds__(1024) void logsoftmax_nbest_kernel(const float* __r
       }
     }
   };
-  // What reaches the bound lies in few threads, those whose largest score does (of N waves, but for equal scores).  Where it is one of a
-  // wave, its values take a turn through LDS to a lane each, which appends those that reach it; of several, every thread goes through its own.
+  // What reaches the bound lies in few threads, those whose largest score does (of N waves, but for equal scores).  Where it is one or two of a
+  // wave, each one's values take a turn through LDS to a lane each, which appends those that reach it; of more, every thread goes through its own.
   // (Times of recorded launches, N best of so many rows and words: every thread of all waves through its own, a turn for each of a wave's threads, and
-  // so: 128 x 32000, N = 1 8.7, 7.1, 7.1 us; 4 8.7, 7.7, 7.9; 6 8.9, 8.2, 8.2; 12 10.4, 11.1, 9.7; 16 19.3, 23.9, 18.5.  6 x 32000, N = 1 8.2, 6.7, 6.6; 16
-  // 14.9, 17.2, 14.0.  65 x 8000 with every eighth word the best, N = 1 8.7, 37.4, 8.0; 6 13.5, 42.7, 12.7: turns follow one another, 2000 clocks each
-  // where all sixteen waves have some.)
+  // so: 128 x 32000, N = 1 8.7, 7.1, 7.1 us; 4 8.7, 7.7, 7.8; 6 9.0, 8.3, 8.2; 12 10.4, 11.0, 9.8; 16 19.3, 23.9, 18.5.  6 x 32000, N = 1 8.2, 6.7, 6.7; 16 15.0, 17.2, 14.1.  65 x 8000 with every eighth
+  // word the best, N = 1 8.8, 37.4, 7.9; 6 13.5, 42.7, 12.7: turns follow one another, 2000 clocks each where all sixteen waves have some.  One turn at the most is 0 - 3 % ahead of
+  // two there and behind them where other launches ran before and the code is cold: in a step of 6 hypotheses 10.5 and 9.5 us, of 65 11.1 and 10.3.)
   __shared__ __attribute__((aligned(16))) float turn[16][4 * VPT];
   static_assert(4 * VPT <= 64, "a lane for each of a thread's values");
   const unsigned long long reaching = __ballot(score(own_max - row_max) >= tv);   // (whole waves)
-  if(__builtin_expect((reaching & (reaching - 1)) != 0, 0)) {
+  if(__builtin_expect(__popcll(reaching) > 2, 0)) {
     nbest_collect(scan, sh, tv);
-  } else if(reaching) {
-    const int from = __builtin_ctzll(reaching), lane = t % 64, i = min(lane, 4 * VPT - 1);
-    if(lane == from) {
+  } else {
+    for(unsigned long long todo = reaching; todo; todo &= todo - 1) {
+      const int from = __builtin_ctzll(todo), lane = t % 64, i = min(lane, 4 * VPT - 1);
+      if(lane == from) {
 #pragma unroll
-      for(int j = 0; j < VPT; ++j) reinterpret_cast<v4f*>(turn[t / 64])[j] = v[j];
-    }
-    // (a wave's LDS operations keep their order)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const float sv = score(turn[t / 64][i]);
-    const int i4 = i / 4 * 1024 + t - lane + from;
-    const unsigned long long reached = __ballot(lane == i && i4 < cols4 && sv >= tv);
-    int slot = 0;
-    if(lane == 0) slot = atomicAdd(&sh.count, (int)__popcll(reached));
-    slot = __builtin_amdgcn_readfirstlane(slot) + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(reached >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)reached, 0u));
-    if((reached >> lane & 1) && slot < 1024) {
-      sh.cand_val[slot] = sv; sh.cand_idx[slot] = 4u * (unsigned)i4 + (unsigned)i % 4u;
+        for(int j = 0; j < VPT; ++j) reinterpret_cast<v4f*>(turn[t / 64])[j] = v[j];
+      }
+      // (a wave's LDS operations keep their order)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const float sv = score(turn[t / 64][i]);
+      const int i4 = i / 4 * 1024 + t - lane + from;
+      const unsigned long long reached = __ballot(lane == i && i4 < cols4 && sv >= tv);
+      int slot = 0;
+      if(lane == 0) slot = atomicAdd(&sh.count, (int)__popcll(reached));
+      slot = __builtin_amdgcn_readfirstlane(slot) + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(reached >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)reached, 0u));
+      if((reached >> lane & 1) && slot < 1024) {
+        sh.cand_val[slot] = sv; sh.cand_idx[slot] = 4u * (unsigned)i4 + (unsigned)i % 4u;
+      }
+      __builtin_amdgcn_wave_barrier();
     }
   }
   float* cv = candVal + ((size_t)b * parts + k) * N;
