@@ -58,31 +58,38 @@ __device__ __forceinline__ float normalize_row(v4f (&v)[VECS], const v4f (&t)[VE
   // Quotients by a shared reciprocal, a few operations each where a division takes eleven, unless a step could under- or overflow (no
   // quotient is above sqrt(cols)).  The division stands in a loop, not unrolled: what a launch runs once it also fetches, and with a second copy of
   // the code steps of 6 layers were no faster (128 x 1024 374.5 us before, 368.9 so; 64 x 64 words through an encoder of 1024 957 and 951).
-  // Values equal to the mean (rows of padding) are zeros here, for which the reciprocal will do; a wave that has some looks once more (a launch of 6 x 512
-  // zeros 3.2 us by division, 4.1 in the loop, 3.0 so, of 4096 x 1024 9.6, 11.6 and 9.8, without a skip input 7.7, 9.8 and 7.2; other rows the same).
-  bool quotients = sigma >= kDivisorLeast && sigma <= kDivisorMost;
-  if(__builtin_expect(!__all(least >= kQuotientLeast), 0)) {
+  // Values equal to the mean (rows of padding) are zeros here, for which the reciprocal will do as well; a wave that has some finds that out off the
+  // others' way (a launch of 6 x 512 zeros 3.2 us by division, 4.1 in the loop, 3.0 so, of 4096 x 1024 9.7, 11.5 and 9.8, without a skip input 7.7, 9.9
+  // and 7.4; other rows the same.  With one copy of the quotients behind the second look a step of 6 hypotheses took 0.9 % longer).
+  const bool in_range = sigma >= kDivisorLeast && sigma <= kDivisorMost;
+  auto by_reciprocal = [&](float sigma) __attribute__((always_inline)) {
+    const float reciprocal = 1.0f / sigma;
+#pragma unroll
+    for(int j = 0; j < VECS; ++j)
+#pragma unroll
+      for(int e = 0; e < 4; ++e) v[j][e] = shared_quotient(v[j][e], sigma, reciprocal);
+  };
+  if(__builtin_expect(__all(least >= kQuotientLeast) && in_range, 1)) {
+    by_reciprocal(sigma);
+  } else {
     unsigned order = ~0u;
 #pragma unroll
     for(int j = 0; j < VECS; ++j)
       if(j * kWave + lane < cols4)
 #pragma unroll
         for(int e = 0; e < 4; ++e) order = min(order, dividend_order(v[j][e]));
-    quotients = quotients && __all(order >= kDividendLeast);
-  }
-  if(__builtin_expect(quotients, 1)) {
-    const float reciprocal = 1.0f / sigma;
-#pragma unroll
-    for(int j = 0; j < VECS; ++j)
-#pragma unroll
-      for(int e = 0; e < 4; ++e) v[j][e] = shared_quotient(v[j][e], sigma, reciprocal);
-  } else {
+    if(__all(order >= kDividendLeast) && in_range) {
+      float same = sigma;
+      asm volatile("" : "+v"(same));   // (or else the compiler has one copy of this for both, behind everything)
+      by_reciprocal(same);
+    } else {
 #pragma unroll 1
-    for(int i = 0; i < 4 * VECS; ++i) {   // (the first value is divided and goes to the end)
-      const float q = v[0][0] / sigma;
+      for(int i = 0; i < 4 * VECS; ++i) {   // (the first value is divided and goes to the end)
+        const float q = v[0][0] / sigma;
 #pragma unroll
-      for(int k = 0; k < 4 * VECS - 1; ++k) v[k / 4][k % 4] = v[(k + 1) / 4][(k + 1) % 4];
-      v[VECS - 1][3] = q;
+        for(int k = 0; k < 4 * VECS - 1; ++k) v[k / 4][k % 4] = v[(k + 1) / 4][(k + 1) % 4];
+        v[VECS - 1][3] = q;
+      }
     }
   }
   float omax = 0.0f;
