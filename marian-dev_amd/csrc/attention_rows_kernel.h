@@ -254,8 +254,9 @@ __device__ __forceinline__ float rows4_sum(float v) {
 // four waves to every 16 x 64 scores.  Loads run past the ends into nothing (buffers) instead of having their rows clamped, divisions share
 // their divisor's reciprocal.
 // Measured (masks included, the form above and this): 1024 heads of 64 x 64 21.8 -> 18.8 us, 256 of them 9.2 -> 7.1; 1024 of 23 x 23 10.0 -> 7.6;
-// 512 of 48 x 48 9.6 -> 8.6; 512 of 70 x 70 23.0 -> 20.0; 384 of 128 x 128 28.5 -> 26.0.  The least number of blocks
-// of keys is a kernel of its own: four for 37 keys 14.8 us, three 12.7.
+// 512 of 48 x 48 9.6 -> 8.6; 512 of 70 x 70 23.0 -> 20.0; 384 of 128 x 128 28.5 -> 26.0.  Which heads take it:
+// attention_plan.h.  The least number of blocks of keys is a kernel of its own (four for 37 keys 14.8 us, three 12.7), but for seven, which run as eight
+// without the products of the last block's values.
 // TILES: blocks of 16 keys; WAVES: 16-row blocks of queries of a workgroup.
 template <int TILES, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, 4) void attention_heads_kernel(AttentionRowsArgs p) {
@@ -269,7 +270,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void attention_heads_kernel(Attentio
   const unsigned ekv = entry < p.batchKV ? entry : entry % p.batchKV;
   const unsigned k_row = (unsigned)p.ks.row * 4u, v_row = (unsigned)p.vs.row * 4u, q_row = (unsigned)p.qs.row * 4u;   // bytes
   const int row0 = (group * kWaves + wave) * 16, row = row0 + c;
-  // (as buffers that end behind their last row: rows past it read as zeros, without a check)
+  // (as buffers that end behind their last row: rows past it read as zeros, without a check.  The hardware holds the sum of the lane's and the scalar
+  // offset against the buffer's end, also where the latter alone lies behind it: looked at for 45 of both, within an allocation that goes on)
   const auto k_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.k + p.ks.entry(ekv, p.heads)), 0, (int)((unsigned)(p.len - 1) * k_row + 256u), kRawBuffer);
   const auto v_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.v + p.vs.entry(ekv, p.heads)), 0, (int)((unsigned)(p.len - 1) * v_row + 256u), kRawBuffer);
   const auto q_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.q + p.qs.entry(entry, p.heads)), 0, (int)((unsigned)(p.m - 1) * q_row + 256u), kRawBuffer);

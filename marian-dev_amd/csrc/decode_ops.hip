@@ -204,7 +204,7 @@ __global__ __launch_bounds__(MANY ? 256 : 64) void layer_norm_wave_kernel(const 
 #pragma unroll
     for(int j = 0; j < VPL; ++j) r[j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(buf, lane * 16 + j * 1024, 0, 0));
   };
-  // all loads at once, positions past the row clamped and dropped afterwards
+  // all loads at once; positions past the row (zeros of a buffer, or the last values again) are dropped afterwards
   auto load_row = [&](size_t row, v4f (&v)[VPL], v4f (&t)[VPL]) __attribute__((always_inline)) {
     if constexpr(PLAIN) {
       load_buffer(in + row * cols, v);
@@ -911,9 +911,9 @@ __device__ __forceinline__ int proj_row_key(int c16) { return (c16 ^ (c16 >> 2))
 // One query row of 64 values by one wave: attention_kernel's path for that head size (sixteen lanes
 // cover a key or value row, four consecutive positions per load, up to 64 positions in flight), the
 // same operations in the same order, so the result has the same bits.  q, k_last, v_last may lie
-// in LDS.  sc: len4 floats of this wave, part: 256 floats behind them.  Returns |out| of this lane.
+// in LDS.  sc: len4 floats of this wave (len rounded up to four), part: the 256 floats behind them.  Returns |out| of this lane.
 // ANC: kb and vb are the whole caches, and cached position p lies in the entry of hypothesis anc.row[p], as in
-// attention_kernel's form of that name; anc.first: row[min(4 u + lane / 16, len - 1)], requested by the caller.
+// attention_kernel's form of that name; anc.first: row[4 u + lane / 16], requested by the caller (past the newest position: not looked at).
 constexpr int kAttU = 16;
 struct Ancestors {
   const uint32_t* row;
@@ -1004,7 +1004,7 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
   sum = wave_sum(sum);
   for(int pos = lane; pos < len; pos += 64) sc[pos] = (pos == lane ? e_first : expf(sc[pos] - mx)) / sum;
   v4f o4 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-  for(int base = 0; base < len; base += 4 * kAttU) {   // (rows in hand: once)
+  for(int base = 0; base < len; base += 4 * kAttU) {
     if(base > 0) load_rows(vb, v_last, base, vr);
 #pragma unroll
     for(int u0 = 0; u0 < kAttU; u0 += 4) {
@@ -1037,6 +1037,8 @@ __device__ __forceinline__ float attention_row64(const float* q, const float* kb
 // 34 and 47 315.9 -> 307.7, 128 x 1024 over 21 and 60 392.0 -> 378.4.
 // keys(r), values(r): rows 4 u + lane / 16 (those past the last one: it again), four values from 4 (lane % 16) on.
 // Positions past len within four weigh nothing, fours past it are not added.
+// sc and part lie one behind the other (len4 + 256 floats in all, 16 BLOCKS or more): scores and weights of all 16 BLOCKS positions, zeros past len, fill sc and
+// the beginning of part, which is written when the weights have been read.
 template <int BLOCKS, class Keys, class Values>
 __device__ __forceinline__ float attention_row64_short(const float* q, Keys keys, Values values, const float* mk, float mk0, int len,
                                                        float scale, float* sc, float* part, float* out_row, int lane) {
@@ -1130,7 +1132,7 @@ struct StagedRows {
 // sentence, for one head - read the same entry).  Workgroup (e, y) takes rows e + (4 y + w) batchKV
 // for its waves w = 0 .. 3, reads entry e's keys and values once (sixteen threads per position,
 // PASSES passes of sixteen positions; positions past the end repeat the last one) into LDS, and each
-// wave then runs attention_row64 on them: the operations of attention_kernel's 64-wide path in the
+// wave then runs attention_row64_short on them: the operations of attention_kernel's 64-wide path in the
 // same order, so the same bits, with a quarter (for four hypotheses) of the bytes through the
 // CU's memory path and out of L2.  One position per query row, head size 64, len <= 16 * PASSES.
 constexpr int kSharedAttLen = 96;

@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemm_rows_kernel(const float* A,
     // The abs-max comes between the first pair's loads and the others': a wave goes on only when its loads have been accepted, and those of the later
     // four waves stand behind all of the earlier ones', 3000 clocks of a launch of 14 000 before anyone knew it or sent its share of it.  All loads
     // first: 64 x 512 x 2048 and back 10.19 us, now 9.78, 256 x 1024 x 1000 of a shortlist with its four best words 11.03 and 10.13, a step of 65 x 512
-    // 299.9 and 298.9; none first: 9.90 and 10.21.  (Two pairs and fewer are all on their way together.)
+    // 300.8 and 298.9; none first: 9.90 and 10.21.  (Two pairs and fewer are all on their way together.)
     float amax = 0.0f;
     [[maybe_unused]] const auto exchange = exchange_of();
     if(D > 0) load(0, 0);

@@ -31,8 +31,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 constexpr int kNormVecs = 4;   // float4 per lane: rows of up to 1024 values, cols % 4 == 0 (half as many: up to 512)
 
-// Value j of a lane is float4 number j * 64 + lane of the row; positions past the row are clamped by the
-// loader and dropped here.  v: the row, becomes its normalization (clamped positions: anything); t: what is added to
+// Value j of a lane is float4 number j * 64 + lane of the row; positions past the row hold whatever the loader gives there (zeros of a
+// buffer, or the row's last values again) and are dropped here.  v: the row, becomes its normalization (those positions: anything); t: what is added to
 // it first (has_add).  Returns the largest magnitude of this lane's values.
 template <int VECS>
 __device__ __forceinline__ float normalize_row(v4f (&v)[VECS], const v4f (&t)[VECS], bool has_add, const v4f (&gm)[VECS],

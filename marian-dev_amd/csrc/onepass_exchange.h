@@ -18,7 +18,9 @@ namespace marian_hip {
 // (without the pause, with 512, 1024, 1536 and 2048 clocks of it: 64 x 1024 x 1024 through gemm_rows_kernel 5.7, 5.7, 5.4, 5.6, 5.7 us,
 // 256 x 1024 x 1000 7.1, 6.9, 6.5, 6.8, 7.0, prepareA of 4096 x 1024 7.2, 7.0, 6.3, 6.2, 6.4; a wave of its own for the polls, without
 // loads in front of them, is no better).  The form before had four trips, groups of 16 whose first workgroup answered for them: 6.6, 7.8 and
-// 7.5 us.  gemm_rows_kernel, which now asks for the bulk of its operands between its words and the first poll, has no pause.  Copies, a launch that does nothing else, without the pause: 1, 2, 4, 8 and 16 of them 3.8, 3.6, 3.4, 3.4 and 3.5 us, 4.5 in four trips.
+// 7.5 us.  These are of gemm_rows_kernel as it asked for all its operands first; it asks for their bulk between its words and the first poll now, which
+// takes the pause's place (the launches alone, under the profiler: 5.6 and 8.1 us with the pause, 5.4 and 7.1 so).  Copies, a launch that does nothing else,
+// without the pause: 1, 2, 4, 8 and 16 of them 3.8, 3.6, 3.4, 3.4 and 3.5 us, 4.5 in four trips.
 // The tag is a host nonce, another for every launch; words left by an earlier launch never match, whatever the workspace
 // held before its first use.  A launch that is recorded into a graph repeats its nonce with every replay, so there a generation word that
 // lives in the workspace and that workgroup 0 advances at the end of every replay is added to it (0.2 us: gen_word is null elsewhere).
